@@ -695,6 +695,35 @@ def test_gemm_w4_exact_layout(gpu):
   assert torch.equal(h, want)
 
 
+@pytest.mark.parametrize("rows", [128, 160, 192, 224, 256, 0])
+def test_gemm_w4_row_heights_exact(gpu, rows):
+  """Every row height of the four-wave tile (0: the launcher's rule) bit for bit on integer operands: one row, the edges of
+  a 128-row tile, several tiles with a remainder; one k stage pair, uneven K splits, the residual in place, SiLU pairs."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  from xotorch_support_jetson_amd.ops.weights_layout import shuffle_for_stream
+  g = torch.Generator(device="cpu").manual_seed(11)
+  N, code = 512, rows * 10000 + 4256
+  for M, Kd in ((1, 128), (127, 640), (128, 128), (129, 384), (481, 1152), (700, 512)):
+    x = torch.randint(-3, 4, (M, Kd), generator=g).to(torch.bfloat16).to(gpu)
+    w = torch.randint(-3, 4, (N, Kd), generator=g).to(torch.bfloat16).to(gpu)
+    ref, ws = x.float() @ w.float().t(), shuffle_for_stream(w)
+    y = torch.zeros(M, N, device=gpu, dtype=torch.float32)
+    require().gemm_big(x, ws, y, None, None, None, 0, code, 1)
+    assert torch.equal(y, ref), (M, Kd)
+    S = min(3, Kd // 64)
+    require().gemm_big(x, ws, y.zero_(), None, None, torch.empty(S * M * N, device=gpu), 0, code, S)
+    assert torch.equal(y, ref), (M, Kd, S)
+    h = torch.randint(-3, 4, (M, N), generator=g).to(torch.bfloat16).to(gpu)
+    want = (h.float() + ref).to(torch.bfloat16)
+    require().gemm_big(x, ws, h, None, h, None, 1, code, 1)
+    assert torch.equal(h, want), (M, Kd)
+    f = ref.view(M, N // 32, 2, 16)
+    act = torch.empty(M, N // 2, device=gpu, dtype=torch.float32)
+    require().gemm_big(x, ws, act, None, None, None, K.EPI["silu"], code, 1)
+    # fp32 throughout: the exponential and the quotient differ by a few units in the last place
+    torch.testing.assert_close(act, (torch.nn.functional.silu(f[:, :, 0]) * f[:, :, 1]).reshape(M, N // 2), rtol=2e-6, atol=1e-4)
+
+
 def test_gemm_big_exact_layout(gpu):
   """Integer-valued operands (exact in bf16 and fp32): every output element must match bit for bit,
   which pins the fragment maps, the LDS swizzle and the shuffled-layout k order."""

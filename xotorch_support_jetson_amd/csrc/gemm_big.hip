@@ -546,8 +546,9 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
   // 10000 x BM for row tiles below 256 (160 / 192 / 224: M = 320 / 384 / 448 in two tiles without padding rows;
   // 2256 only with 192)
   const int bm = bn / 10000 ? bn / 10000 : 256, code = bn % 10000;
-  if (code == 4256 && bm == 256) {  // four-wave 256 x 256 tile (gemm_w4.hip)
-    const int rc = launch_gemm_w4(X, ldx, W, bias, R, ldr, Y, ldy, F32, EPI, ws, M, N, K, S, big_group_m(), epi_arg, st);
+  if (code == 4256) {  // four-wave tile, 256 columns, rows by its own rule or as given (gemm_w4.hip)
+    const int rc = launch_gemm_w4(X, ldx, W, bias, R, ldr, Y, ldy, F32, EPI, ws, M, N, K, S, bn / 10000 ? bm : 0, big_group_m(),
+                                  epi_arg, st);
     if (rc != 0 || S == 1 || !reduce) return rc;
     const int ncol = epi_is_glu(EPI) ? N / 2 : N;
     const long chunks = (long)M * (ncol / 8);

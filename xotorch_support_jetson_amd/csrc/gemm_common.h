@@ -36,7 +36,13 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// the same for a wave-uniform runtime count 0 <= n <= N (a chain of scalar compares; n clamped to N)
+// wait until at most N of this wave's LDS (and scalar) operations are in flight (the counter holds at most 15)
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// the same for vector-memory operations and a wave-uniform runtime count 0 <= n <= N (a chain of scalar compares; n clamped to N)
 template <int N>
 __device__ __forceinline__ void wait_vm_upto(int n) {
   if constexpr (N == 0) {

@@ -1,4 +1,5 @@
 // Four-wave 256 x 256 x 64 GEMM on the pre-shuffled weight layout (tile code 4256):  Y[M,N] = X[M,K] . W[N,K]^T
+// (described for 256 rows; the row tile is 32 MI, MI = 4 .. 8, see gemm_w4_mi)
 //
 // The large-M shapes of prefill and training (M >= 1024: a dozen k stages or more per tile) run gemm_big's
 // eight-wave ping-pong at ~1.55 us per 64-deep k step and 18 us of fixed cost per tile; hipBLASLt's
@@ -94,9 +95,9 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {  // f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
   static_for_<0, N>(f);
 }
-constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int A_EL = BM * BK, STAGE = (BM + BN) * BK;  // bf16 elements per stage buffer (64 KB)
-constexpr int SMEM = 2 * STAGE * 2;                     // two stage buffers, 128 KB
+constexpr int BN = 256, BK = 64;
+constexpr int least(int a, int b) { return a < b ? a : b; }
+constexpr int smem_bytes(int mi) { return 2 * (32 * mi + BN) * BK * 2; }  // two stage buffers (MI = 8: 128 KB)
 }  // namespace w4
 
 // TN (the weight-gradient GEMM dW = dY^T . X on the step's token-major tensors, no dY^T / shuffle(X^T) images in
@@ -105,7 +106,9 @@ constexpr int SMEM = 2 * STAGE * 2;                     // two stage buffers, 12
 // XOR-swizzled by tn_swz(k row) through the source offsets) and every fragment (8 consecutive k of one row or
 // column) is two ds_read_b64_tr_b16; the fragment rows are in natural order (no PERM), so the epilogue stores 8 B
 // per lane and tile.  The reads are compiler-visible (the explicit read waits below assume one read per fragment).
-template <int EPI, bool OUT_F32, bool SPLIT, bool TN = false>
+// MI (4 .. 8): token tiles of 16 rows per wave, i.e. row tiles of 32 MI rows.  The schedule keeps its proportions: 16 MI
+// MFMAs a stage, MI + 8 fragment reads per k half, MI + 8 LDS-DMA issues; launch_gemm_w4 picks the height.
+template <int EPI, bool OUT_F32, bool SPLIT, bool TN = false, int MI = 8>
 __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restrict__ X, int ldx,
                                                          const uint16_t* __restrict__ W,
                                                          const uint16_t* __restrict__ bias,
@@ -114,6 +117,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
                                                          int M, int N, int K, int S, int group_m, int ldw,
                                                          float epi_arg) {
   using namespace w4;
+  constexpr int BM = 32 * MI, A_EL = BM * BK, STAGE = (BM + BN) * BK;  // bf16 elements per stage buffer
+  constexpr int H = 8 * MI, NR = MI + 8;  // MFMAs of a k half; fragment reads of a k half = LDS-DMA issues of a stage
+  static_assert(MI >= 4 && MI <= 8 && (!TN || MI == 8), "row tiles of 128 .. 256 rows");
   static_assert(!TN || (!SPLIT && !epi_is_glu(EPI)), "TN: weight gradients (plain or residual epilogue)");
   constexpr bool PERM = !epi_is_glu(EPI) && !TN;
   constexpr bool ASMRD = W4_ASMRD && !TN;
@@ -156,9 +162,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   // per stage -- cost 20 % of the k loop: profiles/r5/gemm_w4/lab_ablation.log.)  Byte offsets are 32-bit: the
   // launcher requires X and this tile's weight rows below 4 GB.
   //   X image: 256 rows x 128 B, 16-B slot (lane % 8) of row r holds logical slot (lane % 8) ^ ((r >> 1) & 7) (gemm_big's
-  //   BK = 64 map); instruction d < 8 copies rows 8 (8 wave + d) .. +7, so the swizzle of lane's row is
-  //   ((lane >> 4) + 4 (d & 1)) & 7.  Rows past M re-read the last; their outputs are masked.
-  //   W image: (16-row group, k32 block) 1-KB blocks in order (group * 2 + block); instruction 8 + i copies block
+  //   BK = 64 map); instruction d < MI copies rows 8 (MI wave + d) .. +7, so the swizzle of lane's row is
+  //   ((lane >> 4) + 4 ((MI wave + d) & 1)) & 7.  Rows past M re-read the last; their outputs are masked.
+  //   W image: (16-row group, k32 block) 1-KB blocks in order (group * 2 + block); instruction MI + i copies block
   //   i & 1 of group 4 wave + i / 2.  PERM: lane l of a block loads granule (kq = l >> 4, row (l & 15) ^ 4 (kq & 1)).
   auto aswz = [](int row) -> int { return (row >> 1) & 7; };
   const int swave = __builtin_amdgcn_readfirstlane(wave);
@@ -180,17 +186,18 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     }
     wvo = 0;
   } else {
-    const int xr0 = 64 * wave + (lane >> 3);
-    const int xslot[2] = {((lane & 7) ^ ((lane >> 4) & 7)) * 8, ((lane & 7) ^ (((lane >> 4) + 4) & 7)) * 8};
+    const int xr0 = 8 * MI * wave + (lane >> 3);
 #pragma unroll
-    for (int d = 0; d < 8; ++d)
-      xvo[d] = (int)(((unsigned)min(m0 + xr0 + 8 * d, M - 1) * (unsigned)ldx + xslot[d & 1]) * 2u);
+    for (int d = 0; d < MI; ++d) {
+      const int slot = ((lane & 7) ^ (((lane >> 4) + 4 * ((MI * wave + d) & 1)) & 7)) * 8;
+      xvo[d] = (int)(((unsigned)min(m0 + xr0 + 8 * d, M - 1) * (unsigned)ldx + slot) * 2u);
+    }
     wvo = (PERM ? (((lane >> 4) * 16 + ((lane & 15) ^ (4 * ((lane >> 4) & 1)))) * 8) : lane * 8) * 2;
 #pragma unroll
     for (int d = 0; d < 8; ++d) tvo[d] = 0;
   }
   const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc((void*)W, (short)0, -1, 0x00020000);
-  auto issue = [&](int t, int buf, int d) {  // LDS-DMA instruction d (0..15) of this wave for k stage t
+  auto issue = [&](int t, int buf, int d) {  // LDS-DMA instruction d (0 .. NR - 1) of this wave for k stage t
     typedef __attribute__((address_space(3))) void* lds_t;
     uint16_t* As = smem + buf * STAGE;
     if constexpr (TN) {
@@ -202,11 +209,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
                                                  t * (BK * 2) * ldw, 0, W4_WAUX);
       return;
     }
-    if (d < 8) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_t)(As + (8 * swave + d) * 512), 16, xvo[d], t * (BK * 2), 0,
+    if (d < MI) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_t)(As + (MI * swave + d) * 512), 16, xvo[d], t * (BK * 2), 0,
                                                W4_XAUX);
     } else {
-      const int i = d - 8;  // group 4 wave + i / 2, block i & 1
+      const int i = d - MI;  // group 4 wave + i / 2, block i & 1
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_t)(As + A_EL + (8 * swave + i) * 512), 16, wvo,
                                                t * 2048 + (i >> 1) * (K / 128) * 4096 + (i & 1) * 1024, 0, W4_WAUX);
     }
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   // ((16 i + c) >> 1) & 7 = (c >> 1) & 7 does not depend on i.  Weight tile j: pair base (j & 1) + 2048 (j >> 1).
   int xo[2], wo[2][2];
   {
-    const int row = wm * 128 + c;
+    const int row = wm * (16 * MI) + c;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) xo[s2] = row * BK + (((4 * s2 + g) ^ aswz(row)) * 8);
   }
@@ -235,12 +242,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     for (int s2 = 0; s2 < 2; ++s2) wo[jj][s2] = A_EL + (grp * 2 + s2) * 512 + pos * 8;
   }
 
-  f32x4 acc[8][8];
+  f32x4 acc[MI][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  s16x8 wf[2][8], xf[2][8];
+  s16x8 wf[2][8], xf[2][MI];
 
   // The k loop's waits as the s_waitcnt builtin, not inline asm: the compiler's wait-count model then sees them.
   // With an opaque asm lgkmcnt(0) it still counted half 1's 16 reads as in flight at the loop top, more than the
@@ -252,9 +259,9 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     __builtin_amdgcn_s_waitcnt(0xC07F);
     asm volatile("" ::: "memory");
   };
-  auto vm16 = []() {  // vmcnt(16): this wave's older stage landed, the 16 refill DMAs stay in flight
+  auto vm_refill = []() {  // vmcnt(NR): this wave's older stage landed, the NR refill DMAs stay in flight
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((16 & 15) | (7 << 4) | (15 << 8) | ((16 >> 4) << 14));
+    __builtin_amdgcn_s_waitcnt((NR & 15) | (7 << 4) | (15 << 8) | ((NR >> 4) << 14));
     asm volatile("" ::: "memory");
   };
   auto bar = []() {  // raw barrier: LDS-DMA stays in flight; the asm statements fence the compiler
@@ -262,15 +269,15 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  // MFMA u (0..63) of k half h: weight tile j = u / 8 against token tile i = u % 8.  Inline asm with the accumulator
+  // MFMA u (0 .. H - 1) of k half h: weight tile j = u / MI against token tile i = u % MI.  Inline asm with the accumulator
   // tied to its AGPR quad: with the builtin the compiler kept moving the 256 accumulators between AGPRs and VGPRs
   // inside the k loop (~500 v_accvgpr moves per stage).  The asm is invisible to the hazard recognizer: the
   // epilogue waits for the last MFMAs explicitly.
   auto mma = [&](int h, int u) {
-    const int j = u >> 3, i = u & 7;
+    const int j = u / MI, i = u % MI;
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(wf[h][j]), "v"(xf[h][i]));
   };
-  // Keep the 16 fragments of k half h alive up to this point.  The MFMAs are inline asm, so the hazard recognizer
+  // Keep the fragments of k half h alive up to this point.  The MFMAs are inline asm, so the hazard recognizer
   // does not know they read their A / B registers over several cycles: a VALU write to a fragment register right
   // after the MFMA that last read it (the compiler reused dead fragment registers for address arithmetic one MFMA
   // later) corrupted the product.  Fragment registers stay allocated for a whole phase, and the loop end pads the
@@ -278,10 +285,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   auto keep = [&](int h) {
     asm volatile("" ::"v"(wf[h][0]), "v"(wf[h][1]), "v"(wf[h][2]), "v"(wf[h][3]), "v"(wf[h][4]), "v"(wf[h][5]),
                  "v"(wf[h][6]), "v"(wf[h][7]), "v"(xf[h][0]), "v"(xf[h][1]), "v"(xf[h][2]), "v"(xf[h][3]),
-                 "v"(xf[h][4]), "v"(xf[h][5]), "v"(xf[h][6]), "v"(xf[h][7]));
+                 "v"(xf[h][least(4, MI - 1)]), "v"(xf[h][least(5, MI - 1)]), "v"(xf[h][least(6, MI - 1)]),
+                 "v"(xf[h][MI - 1]));
   };
-  // fragment read f (0..15) of k half h, in the order the MFMAs consume them (weight tile 0, token tiles 0..7,
-  // weight tiles 1..7): the first MFMA of a half waits for 2 reads (counted lgkmcnt), not for all 16
+  // fragment read f (0 .. NR - 1) of k half h, in the order the MFMAs consume them (weight tile 0, token tiles
+  // 0 .. MI - 1, weight tiles 1 .. 7): the first MFMA of a half waits for 2 reads (counted lgkmcnt), not for all
 #if W4_ASMRD
   // Fragment reads as inline asm with explicit counted waits (before MFMAs 0..8 and 16 of a stage): the
   // compiler's wait-count model, merging the prologue's and the previous stage's read-ahead at the loop header,
@@ -290,8 +298,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)smem;
   auto rd_asm = [&](int buf, int h, int f) {
     const uint32_t bo = lds0 + (uint32_t)buf * (STAGE * 2);
-    if (f == 0 || f > 8) {
-      const int j = f == 0 ? 0 : f - 8;
+    if (f == 0 || f > MI) {
+      const int j = f == 0 ? 0 : f - MI;
       const uint32_t a = bo + (uint32_t)wo[j & 1][h] * 2;
       switch (j >> 1) {  // immediate offset 4096 (j / 2) bytes
         case 0: asm volatile("ds_read_b128 %0, %1" : "=v"(wf[h][j]) : "v"(a)); break;
@@ -317,7 +325,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
 #endif
   auto rd_c = [&](int buf, int h, int f) {
     const uint16_t* Ls = smem + buf * STAGE;
-    const int j = f == 0 ? 0 : (f <= 8 ? -1 : f - 8);
+    const int j = f == 0 ? 0 : (f <= MI ? -1 : f - MI);
     if (j >= 0) wf[h][j] = ld16(Ls + wo[j & 1][h] + 2048 * (j >> 1));
     else xf[h][f - 1] = ld16(Ls + xo[h] + 1024 * (f - 1));
   };
@@ -366,13 +374,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
 
   {  // T >= 1 (S <= K / 64).  Prologue without branches: stage 1 (stage 0 again when T == 1) into buffer 1
 #pragma unroll
-    for (int d = 0; d < 16; ++d) issue(t_beg, 0, d);
+    for (int d = 0; d < NR; ++d) issue(t_beg, 0, d);
 #pragma unroll
-    for (int d = 0; d < 16; ++d) issue(t_beg + min(1, T - 1), 1, d);
-    wait_vm<16>();
+    for (int d = 0; d < NR; ++d) issue(t_beg + min(1, T - 1), 1, d);
+    wait_vm<NR>();
     bar();
 #pragma unroll
-    for (int f = 0; f < 16; ++f) {  // in consumption order, as in the loop
+    for (int f = 0; f < NR; ++f) {  // in consumption order, as in the loop
       rd(0, 0, f);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -380,30 +388,34 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     // one 64-deep stage.  Every stage refills and reads ahead unconditionally -- past the end stage T - 1 again,
     // into a buffer no later stage reads -- so the k loop is straight-line code: a branch inside it made the
     // register allocator shuffle the 256 accumulators between AGPR quads at the join.
-    // Global MFMA index v = 0..127 of a stage (half v / 64, MFMA v % 64).  Half 1's 16 fragment reads go under the
-    // first 16; after MFMA B1 - 1 every wave has them (lgkmcnt(0) + barrier) and this buffer is free; the 16 refill
-    // DMAs of stage t + 2 spread evenly over MFMAs B1 .. 64 + B2 - 1; after MFMA 64 + B2 - 1 stage t + 1 has landed
-    // for this wave (vmcnt(16): the refill stays in flight) and for every wave (barrier), and its half-0 fragments
-    // are read under the next 16 MFMAs, in the order the next stage consumes them.
-    constexpr int B1 = W4_B1, B2 = W4_B2, SPAN = 64 - B1 + B2, DGAP = W4_DGAP, RSP = W4_RSP;
-    static_assert(16 * RSP <= B1 && B2 + 16 * RSP <= 64, "fragment reads between the barriers");
-    static_assert(DGAP == 0 || B1 + DGAP * 15 < 64 + B2, "refill DMAs before barrier 2");
-    static_assert(B1 >= 17 && B1 <= 64 && B2 >= 8 && B2 <= 48, "schedule positions");
+    // Global MFMA index v = 0 .. 2 H - 1 of a stage (half v / H, MFMA v % H).  Half 1's NR fragment reads go under the
+    // first NR; after MFMA B1 - 1 every wave has them (lgkmcnt(0) + barrier) and this buffer is free; the NR refill
+    // DMAs of stage t + 2 spread evenly over MFMAs B1 .. H + B2 - 1; after MFMA H + B2 - 1 stage t + 1 has landed
+    // for this wave (vmcnt(NR): the refill stays in flight) and for every wave (barrier), and its half-0 fragments
+    // are read under the next NR MFMAs, in the order the next stage consumes them.
+    constexpr int B1 = W4_B1 * MI / 8, B2 = W4_B2 * MI / 8, SPAN = H - B1 + B2, DGAP = W4_DGAP, RSP = W4_RSP;
+    static_assert(NR * RSP <= B1 && B2 + NR * RSP <= H, "fragment reads between the barriers");
+    static_assert(DGAP == 0 || B1 + DGAP * (NR - 1) < H + B2, "refill DMAs before barrier 2");
+    static_assert(B1 >= NR && B1 <= H && B2 >= 4 && B2 <= 48, "schedule positions");
     static_assert(!W4_ASMRD || RSP == 1, "the explicit read waits assume one read per MFMA");
     auto body = [&](int t) {
       const int buf = t & 1;
       const int tr = t_beg + min(t + 2, T - 1);
       W4_MARK(0);
-      static_for<128>([&](auto vc) {  // compile-time v: every condition below folds away
+      static_for<2 * H>([&](auto vc) {  // compile-time v: every condition below folds away
         constexpr int v = decltype(vc)::value;
-        constexpr int h = v >> 6, u = v & 63;
+        constexpr int h = v / H, u = v % H;
 #if W4_ASMRD
         if constexpr (ASMRD) {
-        // the read-ahead (16 reads, consumption order) and the v half-1 reads issued since: MFMA v <= 8 needs
-        // read-ahead v + 1 (w0 + x_v, then w1) -> at most 14 younger reads in flight; from MFMA 16 on (w2..w7)
-        // the whole read-ahead -> 15 (stricter than needed, the counter's maximum)
-        if constexpr (v <= 8) asm volatile("s_waitcnt lgkmcnt(14)" ::: "memory");
-        if constexpr (v == 16) asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
+        // the read-ahead (NR reads, consumption order) and the v half-1 reads issued since: MFMA v <= MI needs
+        // read-ahead v + 1 (w0 + x_v, then w1) -> at most NR + v - (v + 2) = MI + 6 younger reads in flight; w2 at MFMA
+        // 2 MI: NR + 2 MI issued, at most 15 in flight leaves 3 MI - 7 >= MI + 3 done (MI >= 5; 128 rows: the exact
+        // count 12); from MFMA NR on 15 in flight means 2 NR - 15 done, which covers w3 .. up to barrier 1's
+        // lgkmcnt(0) where the tile is 256 rows high (all 16), and each w_j at j MI needs MI + 1 + j reads: counted
+        // again at 3 MI for the short tiles, whose half-1 reads end at MFMA NR
+        if constexpr (v <= MI) wait_lgkm<MI + 6>();
+        if constexpr (v == 2 * MI) wait_lgkm<least(15, least(v, NR) + NR - (MI + 3))>();
+        if constexpr (v == 3 * MI && v < B1) wait_lgkm<least(15, least(v, NR) + NR - (MI + 4))>();
         }
 #endif
         // TN: 32 read-ahead reads (two per fragment, consumption order) then two half-1 reads per MFMA from MFMA 0:
@@ -412,13 +424,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
         // and, at 16, all 32 read-ahead reads
         if constexpr (TN && v <= 16) asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
         mma(h, u);
-        if constexpr (!(W4_ABL & 4) && v % RSP == 0 && v < 16 * RSP) rd(buf, 1, v / RSP);
-        if constexpr (!(W4_ABL & 4) && v >= 64 + B2 && (v - 64 - B2) % RSP == 0 && v < 64 + B2 + 16 * RSP)
-          rd(buf ^ 1, 0, (v - 64 - B2) / RSP);
-        if constexpr (!(W4_ABL & 1) && v >= B1 && v < 64 + B2) {
-          static_for<16>([&](auto kc) {  // refill DMA k after MFMA B1 + ((k + 1) SPAN) / 16 - 1
+        if constexpr (!(W4_ABL & 4) && v % RSP == 0 && v < NR * RSP) rd(buf, 1, v / RSP);
+        if constexpr (!(W4_ABL & 4) && v >= H + B2 && (v - H - B2) % RSP == 0 && v < H + B2 + NR * RSP)
+          rd(buf ^ 1, 0, (v - H - B2) / RSP);
+        if constexpr (!(W4_ABL & 1) && v >= B1 && v < H + B2) {
+          static_for<NR>([&](auto kc) {  // refill DMA k after MFMA B1 + ((k + 1) SPAN) / 16 - 1
             constexpr int k = decltype(kc)::value;
-            if constexpr ((DGAP ? B1 + DGAP * k : B1 + ((k + 1) * SPAN) / 16 - 1) == v) issue(tr, buf, k);
+            if constexpr ((DGAP ? B1 + DGAP * k : B1 + ((k + 1) * SPAN) / NR - 1) == v) issue(tr, buf, k);
           });
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -427,12 +439,12 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
           if constexpr (!(W4_ABL & 16)) bar();
           W4_MARK(1);
         }
-        if constexpr (!(W4_ABL & 2) && v == 64 + B2 - 1) {
-          if constexpr (!(W4_ABL & 32)) vm16();
+        if constexpr (!(W4_ABL & 2) && v == H + B2 - 1) {
+          if constexpr (!(W4_ABL & 32)) vm_refill();
           if constexpr (!(W4_ABL & 64)) bar();
           W4_MARK(2);
         }
-        if constexpr (v == 63) keep(0);
+        if constexpr (v == H - 1) keep(0);
       });
       keep(1);
       __builtin_amdgcn_sched_barrier(0);
@@ -455,14 +467,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   asm volatile("s_nop 7\n s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- epilogue.  Lane (g, c): token row trow(i) = m0 + 128 wm + 16 i + c; PERM: columns 32 J + 8 g .. +8 of the
+  // ---- epilogue.  Lane (g, c): token row trow(i) = m0 + 16 MI wm + 16 i + c; PERM: columns 32 J + 8 g .. +8 of the
   // wave's 128 from tiles (2J, 2J + 1); SiLU: output columns 16 J + 4 g .. +4 (gate tile 2J, up tile 2J + 1).
-  const int rbase = m0 + wm * 128 + c;
+  const int rbase = m0 + wm * (16 * MI) + c;
   const int cbase = n0 + wn * 128;
   if constexpr (SPLIT) {  // raw fp32 partial slabs, in the natural or permuted column order of the lane
     float* slab = ws + (size_t)split * M * N;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int m = rbase + 16 * i;
       if (m >= M) continue;
       float* row = slab + (size_t)m * N + cbase;
@@ -480,7 +492,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   } else if constexpr (TN) {  // natural column order: lane (g, c) holds columns cbase + 16 j + 4 g .. +4 of token row
     typedef short s16x4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int m = rbase + 16 * i;
       if (m >= M) continue;
 #pragma unroll
@@ -511,7 +523,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
       for (int J = 0; J < 4; ++J) bv[J] = ld16(bias + cbase + 32 * J + 8 * g);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int m = rbase + 16 * i;
       s16x8 rv[4];
       if constexpr (EPI == EPI_RESID) {
@@ -557,7 +569,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   } else {  // SiLU: natural rows, gate tile 2J / up tile 2J + 1 -> 4 output columns per lane
     const int obase = cbase / 2;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MI; ++i) {
       const int m = rbase + 16 * i;
       if (m >= M) continue;
 #pragma unroll
@@ -589,16 +601,33 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   }
 }
 
+template <int EPI, bool F32, bool SPLIT, int MI>
+static void w4_launch_rows(const uint16_t* X, int ldx, const uint16_t* W, const uint16_t* bias, const uint16_t* R, int ldr,
+                           void* Y, int ldy, float* ws, int M, int N, int K, int S, int group_m, hipStream_t st,
+                           float epi_arg) {
+  auto kern = gemm_w4_kernel<EPI, F32, SPLIT, false, MI>;
+  constexpr int SMEM = w4::smem_bytes(MI);
+  static bool attr =
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) == hipSuccess;
+  (void)attr;
+  const int nwg = ((M + 32 * MI - 1) / (32 * MI)) * (N / 256) * S;
+  kern<<<nwg, 256, SMEM, st>>>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, 0, epi_arg);
+}
+
 template <int EPI, bool F32, bool SPLIT>
 static void w4_launch(const uint16_t* X, int ldx, const uint16_t* W, const uint16_t* bias, const uint16_t* R, int ldr,
-                      void* Y, int ldy, float* ws, int M, int N, int K, int S, int group_m, hipStream_t st,
+                      void* Y, int ldy, float* ws, int M, int N, int K, int S, int mi, int group_m, hipStream_t st,
                       float epi_arg = 0.f) {
-  auto kern = gemm_w4_kernel<EPI, F32, SPLIT>;
-  static bool attr =
-      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, w4::SMEM) == hipSuccess;
-  (void)attr;
-  const int nwg = ((M + 255) / 256) * (N / 256) * S;
-  kern<<<nwg, 256, w4::SMEM, st>>>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, 0, epi_arg);
+#define XOT_W4(MI_) \
+  w4_launch_rows<EPI, F32, SPLIT, MI_>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, st, epi_arg)
+  switch (mi) {
+    case 4: XOT_W4(4); break;
+    case 5: XOT_W4(5); break;
+    case 6: XOT_W4(6); break;
+    case 7: XOT_W4(7); break;
+    default: XOT_W4(8); break;
+  }
+#undef XOT_W4
 }
 
 template <int EPI, bool F32>
@@ -606,9 +635,9 @@ static void w4_tn_launch(const uint16_t* Xt, int ldx, const uint16_t* Wt, int ld
                          int ldy, int M, int N, int K, int group_m, hipStream_t st) {
   auto kern = gemm_w4_kernel<EPI, F32, false, true>;
   static bool attr =
-      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, w4::SMEM) == hipSuccess;
+      hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, w4::smem_bytes(8)) == hipSuccess;
   (void)attr;
-  kern<<<(M / 256) * (N / 256), 256, w4::SMEM, st>>>(Xt, ldx, Wt, nullptr, R, ldr, Y, ldy, nullptr, M, N, K, 1,
+  kern<<<(M / 256) * (N / 256), 256, w4::smem_bytes(8), st>>>(Xt, ldx, Wt, nullptr, R, ldr, Y, ldy, nullptr, M, N, K, 1,
                                                        group_m, ldw, 0.f);
 }
 
@@ -631,32 +660,55 @@ int launch_gemm_w4_tn(const uint16_t* Xt, int ldx, const uint16_t* Wt, int ldw, 
   return 0;
 }
 
-// Tile code 4256 of launch_gemm_big.  S > 1 writes fp32 slabs (reduced by the caller's reduce kernel).
+// Row tile (in units of 32 rows) of the four-wave kernel: the height whose rounds of workgroups over the 256 CUs cost
+// least.  A 64-deep stage of a 32 mi x 256 tile takes 0.59 + 0.091 mi us (M 2048, N 4096, K 28672: 427 / 459 / 497 / 546 /
+// 589 us for 128 .. 256 rows, one round each -- the weights' fragment reads, barriers and refills do not shrink with the
+// rows), so a round costs 2 mi + 13 and a lower tile pays where it saves a round or fills one: 256 -> chosen height, us,
+//   2230 x 4096 x 14336  315 -> 226 (160 rows: 224 workgroups instead of 144)   3000 x 8192 x 8192   334 -> 297 (192)
+//   2048 x 4096 x 4096    82 -> 58 (128: 256 instead of 128)                   12900 x 2048 x 5632   275 -> 247 (224)
+// and 256 rows stay where their rounds are full (8192^3 740, 900 or more with any lower tile).
+int gemm_w4_mi(int M, int N, int S) {
+  int best = 8;
+  long cost = -1;
+  for (int mi = 8; mi >= 4; --mi) {
+    const long tiles = (long)((M + 32 * mi - 1) / (32 * mi)) * (N / 256) * S;
+    const long c = ((tiles + 255) / 256) * (2 * mi + 13);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = mi;
+    }
+  }
+  return best;
+}
+
+// Tile code 4256 of launch_gemm_big (+ 10000 x rows for a fixed height).  S > 1 writes fp32 slabs (reduced by the caller's reduce kernel).
 int launch_gemm_w4(const uint16_t* X, int ldx, const uint16_t* W, const uint16_t* bias, const uint16_t* R, int ldr,
-                   void* Y, int ldy, bool out_f32, int epi, float* ws, int M, int N, int K, int S, int group_m,
+                   void* Y, int ldy, bool out_f32, int epi, float* ws, int M, int N, int K, int S, int rows, int group_m,
                    float epi_arg, hipStream_t st) {
   if (M <= 0) return 0;
   if (N % 256 != 0 || K % 128 != 0 || S < 1 || S > K / 64) return -1;
   if ((size_t)M * ldx * 2 >= (1ull << 32)) return -1;  // 32-bit byte offsets of the LDS-DMA buffer loads
+  if (rows != 0 && (rows % 32 != 0 || rows < 128 || rows > 256)) return -1;
+  const int mi = rows ? rows / 32 : gemm_w4_mi(M, N, S);
   if (S > 1) {
     if (ws == nullptr) return -1;
-    if (epi_is_glu(epi)) w4_launch<EPI_SILU, true, true>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, st);
-    else w4_launch<EPI_NONE, true, true>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, st);
+    if (epi_is_glu(epi)) w4_launch<EPI_SILU, true, true>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, mi, group_m, st);
+    else w4_launch<EPI_NONE, true, true>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, mi, group_m, st);
     return 0;
   }
   if (epi == EPI_CLAMP_GLU || epi == EPI_RELU2) {
     if (out_f32) return -1;
-    if (epi == EPI_RELU2) w4_launch<EPI_RELU2, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
-    else w4_launch<EPI_CLAMP_GLU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st, epi_arg);
+    if (epi == EPI_RELU2) w4_launch<EPI_RELU2, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
+    else w4_launch<EPI_CLAMP_GLU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st, epi_arg);
   } else if (epi == EPI_SILU) {
-    if (out_f32) w4_launch<EPI_SILU, true, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
-    else w4_launch<EPI_SILU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
+    if (out_f32) w4_launch<EPI_SILU, true, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
+    else w4_launch<EPI_SILU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
   } else if (epi == EPI_RESID) {
     if (out_f32) return -1;
-    w4_launch<EPI_RESID, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
+    w4_launch<EPI_RESID, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
   } else {
-    if (out_f32) w4_launch<EPI_NONE, true, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
-    else w4_launch<EPI_NONE, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, group_m, st);
+    if (out_f32) w4_launch<EPI_NONE, true, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
+    else w4_launch<EPI_NONE, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
   }
   return 0;
 }

@@ -372,8 +372,15 @@ class GemmPolicy:
       # tuned candidates below)
       # tall GEMMs (prefill chunks, training): the four-wave tile at S = 1 won every tuned tall shape this round
       # (profiles/r5/headline/bench_r5o_tunelog.log), so it is taken without the cold-timing pass, which cost
-      # ~0.5 s inside the first prefill chunk of every fresh process
-      got = ("big", 4256, 1)
+      # ~0.5 s inside the first prefill chunk of every fresh process.  (Its row height follows M inside the kernel's
+      # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long: the fp32
+      # slabs cost ~65 us at 2048 x 4096, half the k loop saves more from K ~ 24576 (28672: 369 us against 427 with
+      # 128-row tiles; 14336: about level; 4096: 74 against 58).
+      got = ("big", 4256, 2 if Kd >= 24576 and -(-M // 256) * (N // 256) <= 128 and M <= 2048 else 1)
+      if got[2] > 1:
+        if self._no_tuning():
+          return ("big", 4256, 1)  # (the slabs are sized outside a capture)
+        scratch.splitk(x.device, _ws_elems(got, M, N))
       self._store(key, got)
       return got
     cands = []
