@@ -1,0 +1,96 @@
+"""linear_recurrence in chunks of 16 tokens (csrc/recurrence_chunk.hip) against the recurrence token by token in float64: every
+rule it takes, ends of chunks and of the ring of chunks in flight, decays at their extremes, channels and slots left alone."""
+import pytest
+import torch
+
+from xotorch_support_jetson_amd.ops import kernels as K
+
+F64 = torch.float64
+# rule -> (decay per key channel, delta rule, input scale, normaliser channel)
+RULES = {"delta": (False, True, False, False), "channel_delta": (True, True, False, False), "channel": (True, False, False, False),
+         "head": (False, False, False, False), "scaled": (False, False, True, False), "normaliser": (False, False, True, True)}
+
+
+def token_by_token(q, k, v, decay, beta, q_scale, S, rule, H):
+  """One sequence in float64: q, k [n, G, d], v [n, H, dvin], decay [n, H, d | 1], S [H, dv, d] -> (out [n, H, dv], S)."""
+  _, delta, scaled, norm = RULES[rule]
+  rep, out = H // q.shape[1], []
+  for t in range(q.shape[0]):
+    qt, kt = ((x[t].to(F64)).repeat_interleave(rep, 0) for x in (q, k))
+    vt = v[t].to(F64)
+    if norm:
+      vt = torch.cat([vt, torch.ones(H, 1, dtype=F64)], 1)
+    S = S * decay[t].to(F64)[:, None, :]
+    if delta:
+      vt = vt - torch.einsum("hvd,hd->hv", S, kt)
+    if delta or scaled:
+      vt = vt * beta[t].to(F64)[:, None]
+    S = S + vt[:, :, None] * kt[:, None, :]
+    out.append(torch.einsum("hvd,hd->hv", S, qt) * q_scale)
+  return torch.stack(out), S
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule", list(RULES))
+@pytest.mark.parametrize("d,dv,G", [(64, 40, 4), (128, 64, 2), (128, 17, 4)])
+@pytest.mark.parametrize("decays", ["near one", "wide", "zero and above one"])
+def test_chunks_match_token_by_token(gpu, rule, d, dv, G, decays):
+  channel, delta, scaled, norm = RULES[rule]
+  H, q_scale = 4, 0.7
+  G = H if channel and not delta else G
+  lens = [1, 15, 16, 17, 33, 100, 47]
+  T, B, dvs = sum(lens), len(lens), dv + norm
+  g = torch.Generator().manual_seed(d + dv + len(rule))
+  rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+  q, k, v = rn(T, G, d), rn(T, G, d), rn(T, H, dv)
+  q, k = q / q.norm(dim=-1, keepdim=True), k / k.norm(dim=-1, keepdim=True)
+  a = rn(T, H, d if channel else 1)
+  if decays == "near one":
+    a = torch.sigmoid(3 + a) ** (1 / 16)
+  elif decays == "wide":
+    a = torch.exp(-3 * torch.nn.functional.softplus(3 * a))
+  else:
+    a = torch.where(a > 1, torch.zeros_like(a), torch.where(a < -1.5, torch.full_like(a, 1.1), torch.sigmoid(a + 2)))
+  beta = torch.sigmoid(rn(T, H)) if delta else torch.rand(T, H, generator=g) * 2 if scaled else None
+  state = rn(B + 2, H, dvs, d)
+  slots = torch.tensor([3, -1, 5, 0, 8, 1, 6], dtype=torch.int32)
+  cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+  S, out = state.to(gpu), torch.full((T, H * dvs), 7.0, device=gpu)
+  # (q and k as column slices of wider rows)
+  wide = torch.zeros(T, 2 * G * d + 8)
+  wide[:, 4:4 + G * d], wide[:, 4 + G * d:4 + 2 * G * d] = q.reshape(T, -1), k.reshape(T, -1)
+  wide = wide.to(gpu)
+  K.linear_recurrence(wide[:, 4:4 + G * d], wide[:, 4 + G * d:4 + 2 * G * d], v.reshape(T, -1).to(gpu), a.reshape(T, -1).to(gpu),
+                      None if beta is None else beta.to(gpu), q_scale, S, slots.to(gpu), cu.to(gpu), out, plain=scaled and not norm, max_qlen=100)
+  S, out = S.cpu(), out.cpu().view(T, H, dvs)
+  kept = [s for s in range(B + 2) if s not in slots.tolist()]
+  assert torch.equal(S[kept], state[kept])
+  for b in range(B):
+    t0, t1, slot = int(cu[b]), int(cu[b + 1]), int(slots[b])
+    if slot < 0:
+      assert (out[t0:t1] == 7.0).all()
+      continue
+    want, last = token_by_token(q[t0:t1], k[t0:t1], v[t0:t1], a[t0:t1], None if beta is None else beta[t0:t1], q_scale,
+                                state[slot].to(F64), rule, H)
+    # fp32 products and sums throughout: dot products of d and of 16 terms and a chain of at most 100 decays and writes, a
+    # few units of 6e-8 each (the token-by-token kernel: 1e-7 to 3e-7)
+    for got, ref in ((out[t0:t1], want), (S[slot], last)):
+      assert ((got.to(F64) - ref).norm() / ref.norm()) < 1e-6, (b, lens[b])
+
+
+@pytest.mark.gpu
+def test_chunk_rule_keeps_what_it_cannot_take(gpu):
+  """Rows off 16 bytes, key dims it has no tiles for and short steps run token by token, with the same results."""
+  g = torch.Generator(device=gpu).manual_seed(3)
+  T, H, dv = 130, 2, 24
+  cu, slots = torch.tensor([0, T], dtype=torch.int32, device=gpu), torch.zeros(1, dtype=torch.int32, device=gpu)
+  for d, off in ((64, 0), (64, 1), (48, 0)):
+    x = torch.randn(T, 2 * H * d + off, device=gpu, generator=g) / d ** 0.5
+    v, a, b = torch.randn(T, H * dv, device=gpu, generator=g), torch.rand(T, H, device=gpu, generator=g), torch.rand(T, H, device=gpu, generator=g)
+    got = []
+    for longest in (1, T):
+      S, out = torch.zeros(1, H, dv, d, device=gpu), torch.empty(T, H * dv, device=gpu)
+      K.linear_recurrence(x[:, off:off + H * d], x[:, off + H * d:], v, a, b, 1.0, S, slots, cu, out, max_qlen=longest)
+      got.append((out, S))
+    for one, other in zip(*got):
+      torch.testing.assert_close(one, other, rtol=0, atol=float(2e-6 * one.abs().max()))

@@ -11,12 +11,14 @@
 //   delta_prep         short causal convolutions + SiLU, unit-norm q / k, sigmoid write strength, scalar decay
 //   conv_state_update  the last taps-1 convolution inputs of every sequence -> its state slot
 //   gla_prep           per-key-channel decay sigmoid(low-rank z)^(1/tau)
-//   linear_recurrence  S <- decay * S, delta-rule or outer-product write, o = S^T q; fp32 state per slot
+//   linear_recurrence  S <- decay * S, delta-rule or outer-product write, o = S^T q; fp32 state per slot (token by token here;
+//                      prompts in chunks of 16 tokens: recurrence_chunk.hip)
 //   gated_rmsnorm      per-head RMS norm of o, weight, SiLU gate
 //
 // A fused projection's output P is fp32 [T, ldp]; "column offset" arguments address its slices.  Activations that
 // feed the next GEMM (AT) are bf16 or fp32; everything that enters a norm, a score or a recurrence is fp32.
 #include "mixer_util.h"
+#include "recurrence_chunk.h"
 
 namespace xot {
 namespace {
@@ -1105,7 +1107,7 @@ void launch_rec(int KR, dim3 grid, const float* q, int ldq, const float* k, int 
 // rows contiguous).
 void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& decay,
                        const c10::optional<at::Tensor>& beta, double q_scale, at::Tensor& state, const at::Tensor& state_slots,
-                       const at::Tensor& cu_q, at::Tensor& out, bool plain) {
+                       const at::Tensor& cu_q, at::Tensor& out, bool plain, int64_t max_qlen) {
   const int ldq = ld_of(q, "q"), ldk = ld_of(k, "k"), ldv = ld_of(v, "v");
   f32c(decay, "decay");
   f32c(state, "state");
@@ -1134,6 +1136,24 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   // one decay per head (and token: [T, H]; or fixed: a 1-D [H]), q / k shared by H / G heads
   const bool fixed = !beta.has_value() && decay.dim() == 1 && decay.numel() == H;
   const bool scalar = !beta.has_value() && (fixed || decay.numel() == T * H);
+  const float* bp = beta.has_value() ? beta->data_ptr<float>() : nullptr;
+  auto on16 = [](const at::Tensor& t, int ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
+  const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
+  // Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
+  // its 1.4 us a chunk (2.2 with channel decays) beat 0.2 us a token, whatever the other sequences of the step do.  us before / after,
+  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 191, 8 of 961 .. 2431 1018 / 419, 30 single tokens and one
+  // prompt of 500 131 / 92, one of 33 11 / 15; channel decays 498 / 299, 1124 / 565, 229 / 122, 14 / 20.
+  // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
+  const int64_t widest = std::max(std::max<int64_t>(ldq, ldk), std::max<int64_t>(std::max<int64_t>(ldv, H * dv), H * d));
+  if ((d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && on16(q, ldq) &&
+      on16(k, ldk) && on16(state, 0) && (!per_channel || on16(decay, 0))) {
+    auto ws = at::empty({chunk_recurrence_ws(T, B, H)}, q.options());
+    chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, ldk, ldv,
+                      fixed ? 0 : (int)H, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(),
+                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, per_channel, delta, ws.data_ptr<float>(),
+                      out.data_ptr<float>()});
+    return;
+  }
   int DP = 16;
   while (DP < d) DP *= 2;
   MCHECK(DP <= 256, "linear_recurrence: key dim above 256");
@@ -1144,7 +1164,6 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool two = (chan || inscale) && dv > 16 && REC_COLS != 1 && (REC_COLS == 2 || (T >= 16 * B && B * H * ((dv + 31) / 32) >= 512));
   const int cols = 256 / RS * (two ? 2 : 1);
   const dim3 grid((unsigned)B, (unsigned)H, (unsigned)((dv + cols - 1) / cols));
-  const float* bp = beta.has_value() ? beta->data_ptr<float>() : nullptr;
 #define REC_GO(R, D, N)                                                                                                       \
   launch_rec<R, D, N>(DP / R, grid, q.data_ptr<float>(), ldq, k.data_ptr<float>(), ldk, v.data_ptr<float>(), ldv,              \
                    decay.data_ptr<float>(), bp, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(),        \

@@ -1,0 +1,22 @@
+// linear_recurrence over chunks of 16 tokens (recurrence_chunk.hip); arguments checked by linear_recurrence (mixers.hip).
+#pragma once
+#include <cstdint>
+
+namespace xot {
+
+struct ChunkRecurrence {
+  const float *q, *k, *v, *decay, *beta;  // beta: the delta rule's write strength, or (not delta) an input scale, may be null
+  int ldq, ldk, ldv, dstride;             // dstride: decays of consecutive tokens (0: one fixed decay per head)
+  float q_scale;
+  float* state;
+  const int *state_slots, *cu_q;
+  int T, B, H, G, d, dv, dvin;
+  bool chan, delta;  // a decay per key channel; the delta rule
+  float *ws, *out;
+};
+
+// takes d 64 or 128, rows of q, k, the decays (chan) and the state on 16-byte boundaries
+void chunk_recurrence(const ChunkRecurrence& a);
+int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H);  // floats
+
+}  // namespace xot

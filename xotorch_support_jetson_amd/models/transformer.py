@@ -503,13 +503,13 @@ class ShardModel:
       K.delta_prep(P, lw.cols["rq"][0], lw.cols["rb"][0], lw.cols["ra"][0], lw.conv_w, st.conv[j], inp.state_slots,
                    inp.cu_q, lw.A_log, lw.dt_bias, H, G, d, dv, qkv, beta, decay)
       K.linear_recurrence(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], decay, beta, 1.0, st.S[j],
-                          inp.state_slots, inp.cu_q, o)
+                          inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     else:
       decay = torch.empty(T, H * d, dtype=torch.float32, device=dev)
       K.gla_prep(P, lw.cols["ra1"][0], lw.a2_w, lw.a2_b, r.tau, decay)
       (qo, qn), (ko, kn), (vo, vn) = lw.cols["rq"], lw.cols["rk"], lw.cols["rv"]
       K.linear_recurrence(P[:, qo:qo + qn], P[:, ko:ko + kn], P[:, vo:vo + vn], decay, None, d ** -0.5, st.S[j],
-                          inp.state_slots, inp.cu_q, o)
+                          inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     off, n = lw.mix_cols["rec"]
     K.gated_rmsnorm(o, lw.rec_norm, P, lw.cols["rg"][0], self.c.rms_norm_eps, lw.spec.rec_scale, mix[:, off:off + n])
 
@@ -632,7 +632,7 @@ class ShardModel:
     o = torch.empty(T, H * (r.vdim + 1), dtype=torch.float32, device=dev)
     (qo, qn), (ko, kn), (vo, vn) = lw.cols["rq"], lw.cols["rk"], lw.cols["rv"]
     K.linear_recurrence(P[:, qo:qo + qn], P[:, ko:ko + kn], P[:, vo:vo + vn], decay, inscale, r.dim ** -0.5, st.S[j],
-                        inp.state_slots, inp.cu_q, o)
+                        inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     K.gated_group_norm(o, m, lw.rec_norm, P, lw.cols["rg"][0], H, self.c.rms_norm_eps, mix)
 
   def _lightning(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor) -> None:
@@ -645,7 +645,7 @@ class ShardModel:
     K.silu_cols(P, lw.cols["rq"][0], 2 * nq + nv, qkv)  # (q | k | v are neighbours in the fused projection)
     o = torch.empty(T, nv, dtype=torch.float32, device=dev)
     K.linear_recurrence(qkv[:, :nq], qkv[:, nq:2 * nq], qkv[:, 2 * nq:], lw.decay, None, 1.0,
-                        st.S[j], inp.state_slots, inp.cu_q, o)
+                        st.S[j], inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     K.gated_group_norm(o, None, lw.rec_norm, P, lw.cols["rg"][0], 1, self.c.rms_norm_eps, mix)
 
   def _ssd(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor) -> None:
@@ -662,7 +662,7 @@ class ShardModel:
     K.ssd_prep(P, i0 + inner, i0 + 2 * inner + 2 * gn, lw.conv_w, lw.conv_b, st.conv[j], inp.state_slots, inp.cu_q,
                lw.A_log, lw.dt_bias, m.heads, m.vdim, xbc, v, decay)
     K.linear_recurrence(xbc[:, inner + gn:], xbc[:, inner:inner + gn], v, decay, None, 1.0, st.S[j], inp.state_slots,
-                        inp.cu_q, o)
+                        inp.cu_q, o, max_qlen=inp.max_qlen)
     K.ssd_gate_norm(o, xbc, lw.skip_d, P, i0, lw.ssd_norm, m.norm_groups, self.c.rms_norm_eps, mix)
 
   def _conv(self, P: torch.Tensor, off: int, lw, j: int, inp: StepInputs, **gates) -> torch.Tensor:
@@ -696,7 +696,7 @@ class ShardModel:
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
                        gates=(lw.cols["rb"][0], beta, a0, lw.a2_w, lw.dt_bias, lw.A_log, decay, g0, lw.g2_w, gate))
     o = torch.empty(T, nv, dtype=torch.float32, device=dev)
-    K.linear_recurrence(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], decay, beta, 1.0, st.S[j], inp.state_slots, inp.cu_q, o)
+    K.linear_recurrence(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], decay, beta, 1.0, st.S[j], inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     K.gated_group_norm(o, None, lw.rec_norm, gate, 0, H, self.c.rms_norm_eps, mix)
 
   def _ssd_conv(self, P: torch.Tensor, x: torch.Tensor, dt: torch.Tensor, decay: torch.Tensor, lw, j: int, inp: StepInputs,
@@ -707,7 +707,7 @@ class ShardModel:
     T, inner, gn = mix.shape[0], m.inner, m.groups * m.state
     o = torch.empty(T, inner, dtype=torch.float32, device=dev)
     K.linear_recurrence(x[:, inner + gn:inner + 2 * gn], x[:, inner:inner + gn], x[:, :inner], decay, dt, 1.0, st.S[j],
-                        inp.state_slots, inp.cu_q, o, plain=True)
+                        inp.state_slots, inp.cu_q, o, plain=True, max_qlen=inp.max_qlen)
     K.ssd_gate_norm(o, x, lw.skip_d, P, lw.cols["z"][0], lw.ssd_norm, m.norm_groups, self.c.rms_norm_eps, mix)
 
   def _relu2_moe(self, hn: torch.Tensor, P: torch.Tensor, lw, rows) -> torch.Tensor:

@@ -530,15 +530,21 @@ def ssd_steps(P, dt_off: int, dt_bias, A_log, dt, decay) -> None:
   _mix("ssd_steps", _gpu(P))(P, int(dt_off), dt_bias, A_log, dt, decay)
 
 
-def linear_recurrence(q, k, v, decay, beta, q_scale: float, state, state_slots, cu_q, out, plain: bool = False) -> None:
+def linear_recurrence(q, k, v, decay, beta, q_scale: float, state, state_slots, cu_q, out, plain: bool = False,
+                      max_qlen: int = 0) -> None:
   """Per sequence and value head, token by token on the fp32 state, stored S^T [slots, H, dv, d] (updated in place):
   beta given (delta rule, decay [T, H], or [T, H d] per key channel):  S *= g; u = beta (v - S^T k); S += k u^T; o = S^T q
   (plain: beta scales the input of the plain write instead, S = g S + k (beta v)^T)
   else (decay [T, H d] per key channel, [T, H] per head, or a 1-D [H]: fixed per head):  S = diag(a) S + k v^T; o = S^T q.
   q is scaled by q_scale.
   A state with one value channel more than v has (decay [T, H], beta [T, H] an input scale): S = g S + k (beta [v | 1])^T,
-  the last channel being a normaliser n = g n + beta k; out [T, H (dv + 1)] then ends each head with n . q."""
-  _mix("linear_recurrence", _gpu(q))(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, out, bool(plain))
+  the last channel being a normaliser n = g n + beta k; out [T, H (dv + 1)] then ends each head with n . q.
+  max_qlen: tokens of the step's longest sequence (0: not known); long ones run in chunks on the GPU, where a value that is no
+  number reaches the outputs of its whole chunk of 16 tokens."""
+  if _gpu(q):
+    require().linear_recurrence(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, out, bool(plain), int(max_qlen))
+  else:
+    ref.linear_recurrence(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, out, bool(plain))
 
 
 def gated_rmsnorm(o, w, P, g_off: int, eps: float, out_scale: float, out) -> None:
