@@ -1,0 +1,128 @@
+"""The whole-K decode GEMM (csrc/gemm_wave.hip): every epilogue, column width and prologue at the edges of its range."""
+import pytest
+import torch
+
+from xotorch_support_jetson_amd.ops import kernels as K
+from xotorch_support_jetson_amd.ops import linear as L
+from xotorch_support_jetson_amd.ops.weights_layout import shuffle_for_stream
+
+
+def integers(gen, *shape):
+  return torch.randint(-3, 4, shape, generator=gen).to(torch.bfloat16)
+
+
+def test_candidates_cover_their_range_only():
+  """Up to WAVE_MAX_M rows, whole column tiles, gate / up pairs inside a workgroup, one width for rotation pairs."""
+  cands = L.GemmPolicy._wave_cands
+  assert cands(1, 48, 128, "none", False) == [("wave", 1, 1)]
+  assert cands(L.WAVE_MAX_M, 64, 128, "none", False) == [("wave", 1, 1), ("wave", 2, 1), ("wave", 4, 1)]
+  assert cands(3, 64, 256, "silu", False) == [("wave", 2, 1), ("wave", 4, 1)]
+  assert cands(3, 64, 256, "none", True) == [("wave", 2, 1)]
+  assert cands(L.WAVE_MAX_M + 1, 64, 128, "none", False) == [] and cands(1, 64, 96, "none", False) == []
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 15, 16])
+@pytest.mark.parametrize("N,Kd", [(64, 128), (192, 256), (320, 1408), (128, 4096)])
+def test_epilogues_exact(gpu, M, N, Kd):
+  """Integer operands: sums bit for bit (waves without a k block, uneven shares, a last stage that is not full), fp32 and bf16,
+  bias, residual in place, relu^2, gated pairs, rows of a wider buffer."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  g = torch.Generator().manual_seed(M + N + Kd)
+  x, w, b, r = integers(g, M, Kd), integers(g, N, Kd), integers(g, N), integers(g, M, N)
+  full = x.float() @ w.float().t()
+  ws, bd, C = shuffle_for_stream(w.to(gpu)), b.to(gpu), require()
+  wide = torch.zeros(M, Kd + 16, dtype=torch.bfloat16, device=gpu)
+  wide[:, 8:8 + Kd] = x.to(gpu)
+  xd = wide[:, 8:8 + Kd]
+  for nt in (1, 2, 4):
+    y = torch.zeros(M, N, device=gpu)
+    C.gemm_wave(xd, ws, y, bd, None, K.EPI["none"], nt)
+    assert torch.equal(y.cpu(), full + b.float()), nt
+    h = r.to(gpu)
+    C.gemm_wave(xd, ws, h, None, h, K.EPI["resid"], nt)
+    assert torch.equal(h.cpu(), (full + r.float()).to(torch.bfloat16)), nt
+    a = torch.zeros(M, N, dtype=torch.bfloat16, device=gpu)
+    C.gemm_wave(xd, ws, a, None, None, K.EPI["relu2"], nt)
+    assert torch.equal(a.cpu(), full.clamp(min=0).square().to(torch.bfloat16)), nt
+    if nt == 1:
+      continue
+    f = (full + b.float()).view(M, N // 32, 2, 16)
+    want = {"silu": torch.nn.functional.silu(f[:, :, 0]) * f[:, :, 1],
+            "clamp_glu": (lambda u, v: u * torch.sigmoid(1.702 * u) * (v + 1))(f[:, :, 0].clamp(max=7.0), f[:, :, 1].clamp(-7.0, 7.0))}
+    for epi, ref in want.items():
+      act = torch.zeros(M, N // 2, dtype=torch.bfloat16, device=gpu)
+      C.gemm_wave(xd, ws, act, bd, None, K.EPI[epi], nt, 7.0)
+      # one bf16 rounding (2^-9 of the value) behind fp32 arithmetic that differs in its last places
+      torch.testing.assert_close(act.cpu().float(), ref.reshape(M, N // 2), rtol=4e-3, atol=1e-3)
+  with pytest.raises(RuntimeError):
+    C.gemm_wave(xd, ws, torch.zeros(M, N // 2, dtype=torch.bfloat16, device=gpu), None, None, K.EPI["silu"], 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,H,Hkv,Dh", [(1, 8, 2, 64), (5, 4, 4, 128), (16, 6, 2, 96), (3, 2, 1, 32)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_rope_and_cache_write(gpu, M, H, Hkv, Dh, bias):
+  """q, K and V as the slab reduce with RoPE writes them: rotated in fp32 from the whole sums, padding rows (slot -1) and slots
+  past the pool left alone, positions clamped to the table."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  g = torch.Generator().manual_seed(Dh + M)
+  N, Kd, pages = (H + 2 * Hkv) * Dh, 256, 4
+  x, w = integers(g, M, Kd).to(gpu), integers(g, N, Kd).to(gpu)
+  b = integers(g, N).to(gpu) if bias else None
+  tab = torch.randn(50, Dh, generator=g).to(gpu)
+  pos = torch.randint(0, 60, (M,), generator=g, dtype=torch.int32).to(gpu)
+  slots = torch.randperm(pages * 64, generator=g)[:M]
+  slots[0] = -1 if M > 1 else slots[0]
+  slots[-1] = pages * 64 + 3 if M > 4 else slots[-1]
+  slots = slots.to(gpu)
+  got = []
+  for own in (True, False):
+    q = torch.zeros(M, H, Dh, dtype=torch.bfloat16, device=gpu)
+    kc, vc = torch.zeros(pages, Hkv, 64, Dh, dtype=torch.bfloat16, device=gpu), torch.zeros(pages, Hkv, Dh, 64, dtype=torch.bfloat16, device=gpu)
+    if own:
+      require().gemm_wave(x, shuffle_for_stream(w), None, b, None, 0, 2, pos=pos, cos_sin=tab, slots=slots, q_out=q, k_cache=kc, v_cache=vc, H=H, Hkv=Hkv)
+    else:  # (integer sums: both add up the same numbers)
+      require().splitk_rope_kv_write((x.float() @ w.float().t()).contiguous(), 1, b, pos, tab, slots, q, kc, vc, H, Hkv)
+    got.append((q, kc, vc))
+  for one, other in zip(*got):
+    torch.testing.assert_close(one, other, rtol=8e-3, atol=1e-2)  # the last bf16 place (products contracted differently)
+    assert torch.equal(one == 0, other == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,S", [(128, 1), (2048, 3), (2176, 8), (4096, 4), (8192, 5)])
+def test_norm_prologue_is_the_unfused_row(gpu, D, S):
+  """One row whose residual add and RMS norm run in the prologue: the residual and the product bit for bit those of the slab
+  reduce followed by the plain kernel, with and without the gated epilogue and the rotation."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  g = torch.Generator(device=gpu).manual_seed(D)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  h, lnw, slabs = rn(1, D).to(torch.bfloat16), (1 + 0.1 * rn(D)).to(torch.bfloat16), rn(S, 1, D)
+  H, Hkv, Dh = 4, 2, 64
+  N = (H + 2 * Hkv) * Dh
+  w = shuffle_for_stream((rn(N, D) / D ** 0.5).to(torch.bfloat16))
+  w.xot_layout = "stream"
+  p = L.PendingNorm(h, torch.zeros_like(h), slabs, S, None, lnw, 1e-5)
+  xn = L.PendingNorm(h, torch.zeros_like(h), slabs, S, None, lnw, 1e-5).materialize()
+  C = require()
+  for epi, nt, n in (("none", 1, N), ("none", 4, N), ("silu", 2, N // 2)):
+    y, z = (torch.zeros(1, n, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    p.run_wave(w, y, None, epi, nt)
+    C.gemm_wave(xn, w, z, None, None, K.EPI[epi], nt)
+    assert torch.equal(y, z), (epi, nt)
+  m = h.clone()
+  C.splitk_resid_rmsnorm(slabs, S, None, m, lnw, torch.empty_like(m), 1e-5)
+  assert torch.equal(p.dst, m)
+  tab, pos, slots = rn(16, Dh), torch.tensor([5], dtype=torch.int32, device=gpu), torch.tensor([9], device=gpu)
+  got = []
+  for fused in (True, False):
+    kw = dict(pos=pos, cos_sin=tab, slots=slots, q_out=torch.zeros(1, H, Dh, dtype=torch.bfloat16, device=gpu),
+              k_cache=torch.zeros(1, Hkv, 64, Dh, dtype=torch.bfloat16, device=gpu),
+              v_cache=torch.zeros(1, Hkv, Dh, 64, dtype=torch.bfloat16, device=gpu), H=H, Hkv=Hkv)
+    if fused:
+      p.run_wave(w, None, None, "none", 2, **kw)
+    else:
+      C.gemm_wave(xn, w, None, None, None, 0, 2, **kw)
+    got.append([kw[k] for k in ("q_out", "k_cache", "v_cache")])
+  assert all(torch.equal(a, b) for a, b in zip(*got))

@@ -336,6 +336,98 @@ void gemm_stream_norm(const at::Tensor& w, at::Tensor& y, const c10::optional<at
          " s_in=", s_in);
 }
 
+// Decode GEMM on whole K sums (gemm_wave.hip).  x [M, K], or (norm row) none and h .. eps as in gemm_stream_norm; y as in
+// gemm_stream, or (rope) none and pos .. Hkv as in splitk_rope_kv_write.
+void gemm_wave(const c10::optional<at::Tensor>& x, const at::Tensor& w, const c10::optional<at::Tensor>& y,
+               const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& res, int64_t epi, int64_t nt, double epi_arg,
+               const c10::optional<at::Tensor>& h, const c10::optional<at::Tensor>& ws_in, int64_t s_in,
+               const c10::optional<at::Tensor>& bias_in, const c10::optional<at::Tensor>& lnw, const c10::optional<at::Tensor>& hout,
+               double eps, const c10::optional<at::Tensor>& pos, const c10::optional<at::Tensor>& cos_sin,
+               const c10::optional<at::Tensor>& slots, const c10::optional<at::Tensor>& q_out, const c10::optional<at::Tensor>& k_cache,
+               const c10::optional<at::Tensor>& v_cache, int64_t H, int64_t Hkv) {
+  CHECK_BF16(w);
+  XCHECK(w.dim() == 2 && w.is_contiguous(), "gemm_wave: w");
+  XCHECK(x.has_value() != h.has_value(), "gemm_wave: x, or the norm row");
+  XCHECK(y.has_value() != q_out.has_value(), "gemm_wave: y, or the rotated outputs");
+  const int64_t N = w.size(0), K = w.size(1);
+  xot::WaveGemm a{};
+  a.W = bf(w);
+  a.N = (int)N;
+  a.K = (int)K;
+  a.epi_arg = (float)epi_arg;
+  if (x.has_value()) {
+    CHECK_BF16((*x));
+    XCHECK(x->dim() == 2 && x->size(1) == K && x->stride(1) == 1 && x->stride(0) % 8 == 0 &&
+               (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15) == 0,
+           "gemm_wave: x rows must be contiguous and 16-B aligned");
+    a.X = bf(*x);
+    a.ldx = (int)x->stride(0);
+    a.M = (int)x->size(0);
+  } else {
+    CHECK_BF16((*h));
+    XCHECK(lnw.has_value() && hout.has_value(), "gemm_wave: the norm row needs its weight and output");
+    CHECK_BF16((*lnw));
+    CHECK_BF16((*hout));
+    XCHECK(h->dim() == 2 && h->size(0) == 1 && h->size(1) == K && h->is_contiguous() && hout->sizes() == h->sizes() &&
+               hout->is_contiguous() && hout->data_ptr() != h->data_ptr() && lnw->numel() == K && lnw->is_contiguous(),
+           "gemm_wave: h, hout must be distinct [1, K] rows, lnw [K]");
+    if (bias_in.has_value()) {
+      CHECK_BF16((*bias_in));
+      XCHECK(bias_in->numel() == K && bias_in->is_contiguous(), "gemm_wave: bias_in");
+    }
+    a.np = xot::NormPro{bf(*h), nullptr, (long)K, (int)s_in, bf_opt(bias_in), bf(*lnw), bf(*hout), (float)eps, (int)K};
+    if (s_in > 0) {
+      XCHECK(ws_in.has_value(), "gemm_wave: ws_in");
+      CHECK_GPU((*ws_in));
+      CHECK_DT((*ws_in), at::kFloat);
+      XCHECK(ws_in->is_contiguous() && ws_in->numel() >= s_in * K, "gemm_wave: ws_in holds s_in slabs of K");
+      a.np.ws = ws_in->data_ptr<float>();
+    }
+    a.M = 1;
+  }
+  if (bias.has_value()) {
+    CHECK_BF16((*bias));
+    XCHECK(bias->numel() == N && bias->is_contiguous(), "gemm_wave: bias");
+    a.bias = bf(*bias);
+  }
+  bool f32 = false;
+  if (y.has_value()) {
+    CHECK_GPU((*y));
+    f32 = y->scalar_type() == at::kFloat;
+    XCHECK((f32 || y->scalar_type() == at::kBFloat16) && y->dim() == 2 && y->size(0) == a.M &&
+               y->size(1) == (epi == 2 || epi == 3 ? N / 2 : N) && y->stride(1) == 1,
+           "gemm_wave: y");
+    a.Y = y->data_ptr();
+    a.ldy = (int)y->stride(0);
+    if (epi == 1) {
+      XCHECK(res.has_value(), "gemm_wave: residual epilogue needs res");
+      CHECK_BF16((*res));
+      XCHECK(res->dim() == 2 && res->size(0) == a.M && res->size(1) == N && res->stride(1) == 1, "gemm_wave: res");
+      a.R = bf(*res);
+      a.ldr = (int)res->stride(0);
+    }
+  } else {
+    XCHECK(pos.has_value() && cos_sin.has_value() && slots.has_value() && k_cache.has_value() && v_cache.has_value(), "gemm_wave: rope arguments");
+    CHECK_BF16((*q_out));
+    CHECK_BF16((*k_cache));
+    CHECK_BF16((*v_cache));
+    CHECK_DT((*pos), at::kInt);
+    CHECK_DT((*slots), at::kLong);
+    CHECK_DT((*cos_sin), at::kFloat);
+    XCHECK(all_contig_gpu(*pos, *cos_sin, *slots, *q_out), "gemm_wave: non-contiguous");
+    XCHECK(k_cache->is_contiguous() && v_cache->is_contiguous() && k_cache->dim() == 4 && v_cache->dim() == 4, "gemm_wave: caches must be contiguous 4-D");
+    const int64_t Dh = k_cache->size(3), BS = k_cache->size(2), nb = k_cache->size(0);
+    XCHECK(k_cache->size(1) == Hkv && v_cache->size(0) == nb && v_cache->size(1) == Hkv && v_cache->size(2) == Dh && v_cache->size(3) == BS,
+           "gemm_wave: cache layout must be K[nb,Hkv,BS,Dh], V[nb,Hkv,Dh,BS]");
+    XCHECK(pos->numel() == a.M && slots->numel() == a.M && q_out->numel() == a.M * H * Dh, "gemm_wave: q_out / pos / slots shape");
+    XCHECK(cos_sin->dim() == 2 && cos_sin->size(1) == Dh, "gemm_wave: cos_sin must be [max_pos, Dh]");
+    a.ro = xot::RopeOut{bf(*q_out), bf(*k_cache), bf(*v_cache), pos->data_ptr<int32_t>(), cos_sin->data_ptr<float>(),
+                        slots->data_ptr<int64_t>(), (int)H, (int)Hkv, (int)Dh, (int)BS, (int)cos_sin->size(0), nb * BS};
+  }
+  const int rc = xot::launch_gemm_wave(a, f32, (int)epi, (int)nt, cur_stream());
+  XCHECK(rc == 0, "gemm_wave: unsupported M=", a.M, " N=", N, " K=", K, " epi=", epi, " nt=", nt, " s_in=", s_in);
+}
+
 // Decode GEMM on FP8 (e4m3) pre-shuffled weights w8 [N, K] uint8 with per-row fp32 scales (y = x . (w8 * s)^T).
 void gemm_stream8(const at::Tensor& x, const at::Tensor& w8, const at::Tensor& wscale, at::Tensor& y,
                   const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& res,
@@ -1049,6 +1141,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_tn", &gemm_tn, py::arg("dy"), py::arg("x"), py::arg("y"), py::arg("resid"));
   m.def("gemm_batched", &gemm_batched, py::arg("x"), py::arg("xbat"), py::arg("K"), py::arg("w"), py::arg("y"),
         py::arg("ybat"), py::arg("ldy"), py::arg("M"));
+  m.def("gemm_wave", &gemm_wave, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("bias"), py::arg("res"), py::arg("epi"),
+        py::arg("nt"), py::arg("epi_arg") = 0.0, py::arg("h") = py::none(), py::arg("ws_in") = py::none(), py::arg("s_in") = 0,
+        py::arg("bias_in") = py::none(), py::arg("lnw") = py::none(), py::arg("hout") = py::none(), py::arg("eps") = 0.0,
+        py::arg("pos") = py::none(), py::arg("cos_sin") = py::none(), py::arg("slots") = py::none(), py::arg("q_out") = py::none(),
+        py::arg("k_cache") = py::none(), py::arg("v_cache") = py::none(), py::arg("H") = 0, py::arg("Hkv") = 0);
   m.def("gemm_big", &gemm_big, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("bias"), py::arg("res"),
         py::arg("ws"), py::arg("epi"), py::arg("bn"), py::arg("splits"), py::arg("reduce") = true,
         py::arg("epi_arg") = 0.0);

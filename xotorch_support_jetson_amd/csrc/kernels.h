@@ -63,6 +63,28 @@ void launch_attn_decode_merge(const float* ws_o, const float* ws_ml, const int32
 int launch_gemm_stream_norm(const uint16_t* W, const uint16_t* bias, void* Y, int ldy, int epi, float* ws,
                             long ws_elems, int N, int K, int ntw, int S, bool reduce, const NormPro& np,
                             hipStream_t s);
+// decode GEMM whose workgroups hold whole K sums (gemm_wave.hip): M <= 16, N % (16 nt) == 0, K % 128 == 0, pre-shuffled W.
+// np.h: one row, its norm prologue; ro.q: the QKV projection, rotated and written to q and the paged caches (nt 2)
+struct RopeOut {
+  uint16_t *q, *kc, *vc;
+  const int32_t* pos;
+  const float* cos_sin;
+  const int64_t* slots;
+  int H, Hkv, Dh, BS, max_pos;
+  int64_t nslots;
+};
+struct WaveGemm {
+  const uint16_t* X;
+  int ldx;
+  const uint16_t *W, *bias, *R;
+  int ldr;
+  void* Y;
+  int ldy, M, N, K;
+  float epi_arg;
+  NormPro np;
+  RopeOut ro;
+};
+int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream_t st);
 // decode GEMM with weight-only FP8 (e4m3 pre-shuffled tiles + per-row fp32 scale), bf16 activations
 int launch_gemm_stream8(const uint16_t* X, int ldx, const uint8_t* W, const float* wscale, const uint16_t* bias,
                         const uint16_t* R, int ldr, void* Y, int ldy, bool out_f32, int epi, float* ws, long ws_elems,

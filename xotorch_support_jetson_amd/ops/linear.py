@@ -1,11 +1,13 @@
 """Projection dispatch for the transformer: y = x @ W.T with a fused epilogue.
 
 GPU weights are stored PRE-SHUFFLED (ops.weights_layout.shuffle_for_stream; tagged
-`w.xot_layout == "stream"`): 16-row x 32-k MFMA B-fragment blocks, 1 KB each.  Two library kernels
-consume that layout, both with the epilogue fused (bias / residual add / SiLU*mul):
+`w.xot_layout == "stream"`): 16-row x 32-k MFMA B-fragment blocks, 1 KB each.  Three library
+kernels consume that layout, all with the epilogue fused (bias / residual add / SiLU*mul):
 
   gemm_stream  decode-shaped M: weight-streaming MFMA GEMM (1 KB coalesced weight loads per wave
                instruction straight to registers, X shared through swizzled LDS, optional split-K).
+  gemm_wave    up to 16 rows: a workgroup holds its columns for the whole of K (its waves split K among themselves), so no
+               slabs and no reduce launch; also with RoPE and the paged KV write in the epilogue.
   gemm_big     compute-bound M (large decode batches, prefill chunks): 256 x {256,128} x 64 tiles,
                both operands staged by LDS-DMA, 8 waves, XCD-aware tile order, optional split-K.
 No vendor GEMM runs on a shuffled weight: at prefill sizes gemm_big matches hipBLASLt once the weight
@@ -48,6 +50,9 @@ TALL_FIXED = True
 BLAS_CAND = os.environ.get("XOT_GEMM_BLAS", "0") == "1"
 # largest M for which the stream GEMM is a candidate (above it only gemm_big is timed)
 STREAM_MAX_M = int(os.environ.get("XOT_STREAM_MAX_M", "512"))
+# largest M for which the whole-K decode GEMM (csrc/gemm_wave.hip) is a candidate: no slabs, no reduce launch (its X traffic
+# grows with the rows: at 24 and more the K split of the stream GEMM won every timed shape)
+WAVE_MAX_M = 16
 # smallest M for which gemm_big is a candidate
 BIG_MIN_M = int(os.environ.get("XOT_BIG_MIN_M", "65"))
 
@@ -358,11 +363,21 @@ class GemmPolicy:
         cands.append(("big", bn, S))
     return cands
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype) -> Tuple:
-    """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket."""
+  @staticmethod
+  def _wave_cands(M, N, Kd, epi, rope):
+    """Whole-K decode GEMM: 16, 32 or 64 columns a workgroup (gated pairs from 32; rotation pairs of column tiles: 32)."""
+    if M > WAVE_MAX_M or Kd % 128:
+      return []
+    return [("wave", nt, 1) for nt in ((2,) if rope else (2, 4) if epi in K.GLU_EPI else (1, 2, 4)) if N % (16 * nt) == 0]
+
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "") -> Tuple:
+    """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
+    GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
+    reduce, timed with them, stands for the launch that does it there)."""
     M, Kd = x.shape
     N = w.shape[0]
-    key = ("sh", _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
+    wave = wave if M <= WAVE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
+    key = ("sh" + wave, _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
     got = self._lookup(key)
     if got is not None:
       return got
@@ -386,6 +401,8 @@ class GemmPolicy:
     cands = []
     if M <= STREAM_MAX_M:
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
+    if wave:
+      cands += self._wave_cands(M, N, Kd, epi, wave == "rope")
     if M >= BIG_MIN_M and Kd % 128 == 0:
       big = self._big_cands(M, N, Kd)
       cands += [c for c in big if c[1] in (2256, 128, 4256)] if epi in ("clamp_glu", "relu2") else big  # (the tiles built with them)
@@ -516,6 +533,9 @@ def _linear8(x, w, bias, residual, epi, out, dt):
 def _shuffled_call(x, w, bias, residual, epi, out, cfg, epi_arg: float = 0.0):
   if cfg[0] == "stream":
     return _stream_call(x, w, bias, residual, epi, out, cfg[1:], epi_arg=epi_arg)
+  if cfg[0] == "wave":
+    require().gemm_wave(x, w, out, bias, residual, K.EPI[epi], cfg[1], epi_arg)
+    return out
   _, bn, S = cfg
   M, N = x.shape[0], w.shape[0]
   ws = scratch.splitk(x.device, S * M * N) if S > 1 else None
@@ -605,18 +625,24 @@ class PendingNorm:
     require().splitk_resid_rmsnorm(self.ws, self.S, self.bias, self.dst, self.ln_w, out, self.eps)
     return out
 
+  def run_wave(self, w: torch.Tensor, y, bias, epi: str, nt: int, **rope) -> None:
+    require().gemm_wave(None, w, y, bias, None, K.EPI[epi], nt, 0.0, self.src, self.ws, self.S, self.bias, self.ln_w, self.dst,
+                        self.eps, **rope)
+
   def run(self, w: torch.Tensor, y: torch.Tensor, bias, epi: str, ntw: int, S: int, reduce: bool) -> None:
     ws = scratch.splitk(y.device, S * w.shape[0]) if S > 1 else None
     require().gemm_stream_norm(w, y, bias, ws, K.EPI[epi], ntw, S, reduce, self.src, self.ws, self.S, self.bias,
                                self.ln_w, self.dst, self.eps)
 
 
-def _pending_cfg(p: PendingNorm, w: torch.Tensor, bias, epi: str):
+def _pending_cfg(p: PendingNorm, w: torch.Tensor, bias, epi: str, wave: str = "y"):
   """The stream configuration the consumer GEMM of a pending norm runs (tuned on the unfused kernel with the
   residual row as a stand-in input), or None when the fused kernel does not cover it."""
   if layout_of(w) != "stream" or epi not in ("none", "silu") or w.shape[1] != p.src.shape[1]:
     return None
-  cfg = policy.shuffled_cfg(p.src, w, bias, None, epi, torch.bfloat16)
+  cfg = policy.shuffled_cfg(p.src, w, bias, None, epi, torch.bfloat16, wave=wave)
+  if cfg[0] == "wave" and w.shape[1] <= 8192:
+    return cfg
   if cfg[0] != "stream" or w.shape[1] % (cfg[2] * 128) or (w.shape[1] // cfg[2]) * 2 > 65536:
     return None
   return cfg
@@ -635,7 +661,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, r
       if out is None:
         out = torch.empty(1, w.shape[0] // 2 if epi == "silu" else w.shape[0], dtype=torch.bfloat16,
                           device=x.src.device)
-      x.run(w, out, bias, epi, cfg[1], cfg[2], True)
+      if cfg[0] == "wave":
+        x.run_wave(w, out, bias, epi, cfg[1])
+      else:
+        x.run(w, out, bias, epi, cfg[1], cfg[2], True)
       return out
   if not x.is_cuda:
     return K.gemm(x, to_rowmajor(w), bias=bias, residual=residual, epi=epi, out=out, out_dtype=out_dtype)
@@ -650,7 +679,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, r
     out = torch.empty(M, N // 2 if epi in K.GLU_EPI else N, dtype=dt, device=x.device)
   if x.stride(1) != 1 or x.stride(0) % 8:
     x = x.contiguous()
-  cfg = policy.shuffled_cfg(x, w, bias, residual, epi, dt)
+  cfg = policy.shuffled_cfg(x, w, bias, residual, epi, dt, wave="y")
   _shuffled_call(x, w, bias, residual, epi, out, cfg, epi_arg)
   return out
 
@@ -662,7 +691,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32)
+    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y")
     S = cfg[2]
     if S > 1:
       ws = scratch.splitk(x.device, S * M * N)
@@ -742,15 +771,24 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
   When the QKV projection runs split-K on the pre-shuffled layout, its fp32 slabs go straight to one
   kernel that sums them, rotates and writes q / the caches (no bf16 qkv round trip, one launch less).
   x may be a PendingNorm: the projection then computes its input row in its prologue."""
+  Dh = k_cache.shape[-1]
+  wave = "rope" if Dh % 32 == 0 and k_cache.dtype == torch.bfloat16 and w.shape[0] == (H + 2 * Hkv) * Dh else ""
+
+  def rope(M):  # the outputs of the GEMM that rotates and writes by itself
+    q = torch.empty(M, H, Dh, dtype=torch.bfloat16, device=k_cache.device)
+    return q, dict(pos=pos, cos_sin=cos_sin, slots=slots, q_out=q, k_cache=k_cache, v_cache=v_cache, H=int(H), Hkv=int(Hkv))
   if isinstance(x, PendingNorm):
-    cfg = _pending_cfg(x, w, bias, "none")
+    cfg = _pending_cfg(x, w, bias, "none", wave)
+    if cfg is not None and cfg[0] == "wave":
+      q, kw = rope(1)
+      x.run_wave(w, None, bias, "none", 2, **kw)
+      return q
     if cfg is None or cfg[2] < 2:
       x = x.materialize()
     else:
       S, N = cfg[2], w.shape[0]
       y = torch.empty(1, N, dtype=torch.bfloat16, device=x.src.device)  # shape carrier only
       x.run(w, y, None, "none", cfg[1], S, False)
-      Dh = k_cache.shape[-1]
       q = torch.empty(1, H, Dh, dtype=torch.bfloat16, device=y.device)
       ws = scratch.splitk(y.device, S * N)
       require().splitk_rope_kv_write(ws, S, bias, pos, cos_sin, slots, q, k_cache, v_cache, int(H), int(Hkv))
@@ -759,7 +797,11 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, bias, None, "none", x.dtype)
+    cfg = policy.shuffled_cfg(x, w, bias, None, "none", x.dtype, wave=wave)
+    if cfg[0] == "wave":
+      q, kw = rope(M)
+      require().gemm_wave(x, w, None, bias, None, K.EPI["none"], 2, **kw)
+      return q
     if cfg[0] in ("stream", "big") and cfg[2] > 1:
       S = cfg[2]
       ws = scratch.splitk(x.device, S * M * N)
@@ -769,7 +811,6 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
         C.gemm_stream(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, True, False)
       else:
         C.gemm_big(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, False)
-      Dh = k_cache.shape[-1]
       q = torch.empty(M, H, Dh, dtype=x.dtype, device=x.device)
       C.splitk_rope_kv_write(ws, S, bias, pos, cos_sin, slots, q, k_cache, v_cache, int(H), int(Hkv))
       return q
