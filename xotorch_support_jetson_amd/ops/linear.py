@@ -41,9 +41,11 @@ PP2 = os.environ.get("XOT_GEMM_PP2", "1") == "1"
 # XOT_GEMM_W4=0: leave the four-wave 256 x 256 tile (code 4256) out of the candidates
 W4 = os.environ.get("XOT_GEMM_W4", "1") == "1"
 # rows from which the four-wave tile is preferred over the two-phase ping-pong within TIE (tall prefill / training
-# GEMMs: it reads a third less LDS per FLOP and has ~6 us less fixed cost per tile, profiles/r5/gemm_w4/); below
-# it the ping-pong tile, the measured in-step winner at the decode batches, keeps the preference
-W4_PREF_M = int(os.environ.get("XOT_GEMM_W4_PREF_M", "2048"))
+# GEMMs: it reads a third less LDS per FLOP and has ~6 us less fixed cost per tile, profiles/r5/gemm_w4/), and from which it
+# is taken untimed: with row heights of its own (csrc/gemm_w4.hip gemm_w4_mi) it also leads where 256-row tiles fill the
+# last round badly (1999 x 28672 x 4096 SiLU 365 us on the ping-pong tile, 322 here; 1999 x 4096 x 4096 72 / 60).  Below it
+# the ping-pong tile, the measured in-step winner at the decode batches, keeps the preference
+W4_PREF_M = int(os.environ.get("XOT_GEMM_W4_PREF_M", "1024"))
 # tall GEMMs take the four-wave tile without a timing pass (see shuffled_cfg; tests switch it off)
 TALL_FIXED = True
 # XOT_GEMM_BLAS=1: time hipBLASLt among the candidates for row-major weights (off: the kernel library only)
@@ -388,10 +390,11 @@ class GemmPolicy:
       # tall GEMMs (prefill chunks, training): the four-wave tile at S = 1 won every tuned tall shape this round
       # (profiles/r5/headline/bench_r5o_tunelog.log), so it is taken without the cold-timing pass, which cost
       # ~0.5 s inside the first prefill chunk of every fresh process.  (Its row height follows M inside the kernel's
-      # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long: the fp32
-      # slabs cost ~65 us at 2048 x 4096, half the k loop saves more from K ~ 24576 (28672: 369 us against 427 with
-      # 128-row tiles; 14336: about level; 4096: 74 against 58).
-      got = ("big", 4256, 2 if Kd >= 24576 and -(-M // 256) * (N // 256) <= 128 and M <= 2048 else 1)
+      # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long enough to pay for
+      # the fp32 slabs: ~65 us at 2048 x 4096 with a reduce launch, from K ~ 24576 (28672: 369 us against 427 with 128-row
+      # tiles; 14336: about level; 4096: 74 against 58); ~30 where the residual norm that follows sums them, from K ~ 8192.
+      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576)
+      got = ("big", 4256, 2 if half else 1)
       if got[2] > 1:
         if self._no_tuning():
           return ("big", 4256, 1)  # (the slabs are sized outside a capture)
