@@ -126,3 +126,20 @@ def test_norm_prologue_is_the_unfused_row(gpu, D, S):
       C.gemm_wave(xn, w, None, None, None, 0, 2, **kw)
     got.append([kw[k] for k in ("q_out", "k_cache", "v_cache")])
   assert all(torch.equal(a, b) for a, b in zip(*got))
+
+def test_wave_entries_of_the_tuning_table():
+  """A saved choice is taken as it stands; a caller that cannot run the whole-K GEMM passes over its entry; residual products
+  keep a table entry of their own where another caller sums the slabs."""
+  pol = L.GemmPolicy()
+  x, w = torch.zeros(8, 256, dtype=torch.bfloat16), torch.zeros(512, 256, dtype=torch.bfloat16)
+  tail = (L._m_bucket(8), 512, 256, "none", False, str(torch.float32))
+  cfg = lambda wave, epi="none": pol.shuffled_cfg(x, w, None, None, epi, torch.float32, wave=wave)  # noqa: E731
+  pol.table[("sh",) + tail] = ("stream", 1, 4)
+  assert cfg("y") == ("stream", 1, 4) and cfg("") == ("stream", 1, 4)
+  pol.table[("sh",) + tail] = ("wave", 2, 1)
+  pol.table[("shn",) + tail] = ("stream", 2, 1)
+  assert cfg("y") == ("wave", 2, 1) and cfg("") == ("stream", 2, 1)
+  rtail = (L._m_bucket(8), 512, 256, "resid", False, str(torch.bfloat16))
+  pol.table[("sh",) + rtail], pol.table[("shy",) + rtail] = ("stream", 1, 2), ("wave", 1, 1)
+  got = [pol.shuffled_cfg(x, w, None, x, "resid", torch.bfloat16, wave=wave) for wave in ("", "y")]
+  assert got == [("stream", 1, 2), ("wave", 1, 1)]

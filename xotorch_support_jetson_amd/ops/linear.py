@@ -379,8 +379,14 @@ class GemmPolicy:
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WAVE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
-    key = ("sh" + wave, _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
+    # (a residual product's plain entry belongs to linear_resid_norm, which sums the slabs itself; a caller that does not
+    # take the whole-K GEMM passes over such an entry)
+    kind = "sh" + wave if wave == "rope" or epi == "resid" else "sh"
+    key = (kind, _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
     got = self._lookup(key)
+    if got is not None and got[0] == "wave" and not wave:
+      key = ("shn",) + key[1:]
+      got = self._lookup(key)
     if got is not None:
       return got
     if (TALL_FIXED and W4 and M >= W4_PREF_M and N % 256 == 0 and Kd % 128 == 0 and (N > 256 or -(-M // 256) >= 256)
