@@ -1,0 +1,75 @@
+"""gelu_tanh(gate) * up in the epilogue of the dense projections, every kernel configuration the policy would try."""
+import pytest
+import torch
+
+from xotorch_support_jetson_amd.models.weights import interleave_gate_up
+
+F64 = torch.float64
+
+
+def want_of(x, g, u):
+  z = x.double() @ g.double().T
+  gelu = 0.5 * z * (1 + torch.tanh((2 / torch.pi) ** 0.5 * (z + 0.044715 * z ** 3)))
+  return gelu * (x.double() @ u.double().T), z
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [65, 130, 520, 1024, 2100])
+@pytest.mark.parametrize("N,D", [(256, 128), (512, 384), (768, 1024)])
+def test_gelu_glu_epilogue(M, N, D):
+  from xotorch_support_jetson_amd.ops import linear as L
+  gen = torch.Generator().manual_seed(M + N)
+  x = torch.randn(M, D, generator=gen).bfloat16()
+  w = (torch.randn(N, D, generator=gen) * (3 * D ** -0.5)).bfloat16()  # gates of +-10: both tails of the tanh
+  want, z = want_of(x, w[:N // 2], w[N // 2:])
+  xd, ws = x.cuda(), L.to_stream_layout(interleave_gate_up(w[:N // 2], w[N // 2:]).contiguous().cuda())
+  cands = [c for c in L.policy._big_cands(M, N, D) if c[1] in (2256, 128, 4256)]
+  assert cands
+  for cfg in cands + ["as chosen"]:
+    out = torch.full((M, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+    if cfg == "as chosen":
+      L.linear(xd, ws, epi="gelu_glu", out=out)
+    else:
+      L._shuffled_call(xd, ws, None, None, "gelu_glu", out, cfg)
+    # half a bf16 step of the result, and the fp32 sums' error (products of magnitude |x||w|, sqrt(D) of them at random
+    # signs, so within 2^-24 D of the operands' scale) through the gate's slope (at most 1.13) and the other factor
+    err = (out.double().cpu() - want).abs()
+    lim = want.abs() * 2.0 ** -8 + 2.0 ** -24 * D * 9 * (1 + z.abs()) * 4
+    assert bool((err <= lim).all()), (cfg, float((err / lim).max()))
+
+
+@pytest.mark.gpu
+def test_gelu_glu_epilogue_extremes():
+  """Huge gates give the activation's limits, zero gates (the padding rows) 0."""
+  from xotorch_support_jetson_amd.ops import linear as L
+  vals = [0.0, -0.0, 3e38, -3e38]
+  for M in (65, 300):
+    x = torch.zeros(M, 128, dtype=torch.bfloat16)
+    w = torch.zeros(256, 128, dtype=torch.bfloat16)
+    w[:128, 0] = 1.0
+    w[128:, 1] = 1.0
+    x[:, 1] = 2.0
+    for i in range(M):
+      x[i, 0] = vals[i % 4]
+    ws = L.to_stream_layout(interleave_gate_up(w[:128], w[128:]).contiguous().cuda())
+    out = L.linear(x.cuda(), ws, epi="gelu_glu").float().cpu()
+    for i in range(M):
+      v = vals[i % 4]
+      # (0 * anything stays 0 in the sums: 3e38 and 2 are the only terms of their columns; 6e38 overflows to infinity)
+      assert bool((out[i] == (float("inf") if v > 1e38 else 0.0)).all()), (M, v, out[i, :2])
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("T,F,off,pad", [(1, 16, 0, 0), (5, 40, 12, 0), (7, 100, 64, 28), (3, 33, 5, 3)])
+def test_gelu_mul_of_tiles(dev, T, F, off, pad):
+  """Gate and up columns in alternating tiles of 16, whole vectors or not, against the two-run form (bit for bit)."""
+  from xotorch_support_jetson_amd.ops import kernels as K
+  n = -(-F // 16) * 16
+  gu = torch.randn(T, 2, n, generator=torch.Generator().manual_seed(F))
+  P = torch.zeros(T, off + 2 * n + pad)
+  P[:, off:off + 2 * n] = gu.reshape(T, 2, n // 16, 16).transpose(1, 2).reshape(T, 2 * n)
+  for dt in (torch.float32, torch.bfloat16):
+    got, want = (torch.zeros(T, n + 4, dtype=dt, device=dev) for _ in range(2))
+    K.gelu_mul(P.to(dev), off, -1, F, got)
+    K.gelu_mul(gu.reshape(T, 2 * n).to(dev), 0, n, F, want)
+    assert torch.equal(got, want)

@@ -30,6 +30,8 @@ bool all_contig_gpu(const Ts&... ts) {
   return ((ts.is_contiguous() && ts.is_cuda()) && ...);
 }
 
+// epilogues that turn interleaved (gate, up) columns into half as many: silu, clamp_glu, gelu_glu (gemm_common.h)
+inline bool glu(int64_t epi) { return epi == 2 || epi == 3 || epi == 5; }
 inline hipStream_t cur_stream() { return at::hip::getCurrentHIPStream().stream(); }
 inline uint16_t* bf(const at::Tensor& t) { return reinterpret_cast<uint16_t*>(t.data_ptr()); }
 inline uint16_t* bf_opt(const c10::optional<at::Tensor>& t) {
@@ -252,7 +254,7 @@ void gemm_stream(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const 
   XCHECK(w.size(1) == K, "gemm_stream: K mismatch");
   const bool f32 = y.scalar_type() == at::kFloat;
   XCHECK(f32 || y.scalar_type() == at::kBFloat16, "gemm_stream: y must be bf16 or fp32");
-  XCHECK(y.size(0) == M && y.size(1) == (epi == 2 || epi == 3 ? N / 2 : N), "gemm_stream: y shape mismatch");
+  XCHECK(y.size(0) == M && y.size(1) == (glu(epi) ? N / 2 : N), "gemm_stream: y shape mismatch");
   XCHECK(M <= 65536, "gemm_stream: M must be <= 65536");
   if (bias.has_value()) {
     CHECK_BF16((*bias));
@@ -395,7 +397,7 @@ void gemm_wave(const c10::optional<at::Tensor>& x, const at::Tensor& w, const c1
     CHECK_GPU((*y));
     f32 = y->scalar_type() == at::kFloat;
     XCHECK((f32 || y->scalar_type() == at::kBFloat16) && y->dim() == 2 && y->size(0) == a.M &&
-               y->size(1) == (epi == 2 || epi == 3 ? N / 2 : N) && y->stride(1) == 1,
+               y->size(1) == (glu(epi) ? N / 2 : N) && y->stride(1) == 1,
            "gemm_wave: y");
     a.Y = y->data_ptr();
     a.ldy = (int)y->stride(0);
@@ -484,7 +486,7 @@ void gemm_big(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const c10
   XCHECK(w.size(1) == K, "gemm_big: K mismatch");
   const bool f32 = y.scalar_type() == at::kFloat;
   XCHECK(f32 || y.scalar_type() == at::kBFloat16, "gemm_big: y must be bf16 or fp32");
-  XCHECK(y.size(0) == M && y.size(1) == (epi == 2 || epi == 3 ? N / 2 : N), "gemm_big: y shape mismatch");
+  XCHECK(y.size(0) == M && y.size(1) == (glu(epi) ? N / 2 : N), "gemm_big: y shape mismatch");
   XCHECK(M <= (1 << 24), "gemm_big: M too large");
   if (bias.has_value()) {
     CHECK_BF16((*bias));

@@ -814,7 +814,7 @@ int launch_gemm_moe(const uint16_t* X, int ldx, const uint16_t* W, void* Y, int 
                     long ysplit, float epi_arg, hipStream_t s) {
   if (max_rows <= 0) return 0;
   if (N % 128 != 0 || S < 1 || K % (128 * S) != 0) return -1;
-  if (epi != EPI_NONE && !epi_is_glu(epi)) return -1;
+  if (epi != EPI_NONE && epi != EPI_SILU && epi != EPI_CLAMP_GLU) return -1;
   if (epi_is_glu(epi) && out_f32) return -1;
   if (S > 1 && (epi != EPI_NONE || !out_f32)) return -1;  // K slices write fp32 partial slabs
 #define XOT_MOE(EPIV, F32V)                                                                                     \
@@ -958,6 +958,7 @@ int launch_gemm_stream(const uint16_t* X, int ldx, const uint16_t* W, int ldw, c
                        int M, int N, int K, int ntw, int S, bool wshuf, bool reduce,
                        float epi_arg, hipStream_t s) {
   if (M <= 0) return 0;
+  if (epi == EPI_GELU_GLU) return -1;  // (built for the tall tiles alone)
   if (epi == EPI_CLAMP_GLU)
     return out_f32 ? -1 : stream_dispatch<EPI_CLAMP_GLU, false>(X, ldx, W, ldw, bias, R, ldr, Y, ldy, ws, ws_elems, M, N, K, ntw, S, wshuf, reduce, s, epi_arg);
   if (epi == EPI_RELU2)

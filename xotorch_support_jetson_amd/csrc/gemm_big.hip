@@ -560,7 +560,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
 #define XOT_BIG(BM_, BN_, WM_, NBUF_, ...)                                                                        \
   big_launch<BM_, BN_, WM_, 8 / WM_, 64, NBUF_, EPI, F32, ##__VA_ARGS__>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, \
                                                                          S, reduce, st, epi_arg)
-  if constexpr (EPI == EPI_CLAMP_GLU || EPI == EPI_RELU2) {  // (built for the tiles that win: two-phase 256, 128 columns)
+  if constexpr (EPI == EPI_CLAMP_GLU || EPI == EPI_RELU2 || EPI == EPI_GELU_GLU) {  // (built for the tiles that win: two-phase 256, 128 columns)
     if (bm != 256) return -1;
     if (code == 2256) XOT_BIG(256, 256, 2, 2, 2);
     else if (code == 128) XOT_BIG(256, 128, 4, 3);
@@ -602,6 +602,8 @@ int launch_gemm_big(const uint16_t* X, int ldx, const uint16_t* W, const uint16_
   if (epi_is_glu(epi) && N % 32 != 0) return -1;
   if (epi == EPI_CLAMP_GLU)
     return out_f32 ? -1 : big_dispatch<EPI_CLAMP_GLU, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, ws_elems, M, N, K, bn, S, reduce, s, epi_arg);
+  if (epi == EPI_GELU_GLU)
+    return out_f32 ? -1 : big_dispatch<EPI_GELU_GLU, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, ws_elems, M, N, K, bn, S, reduce, s);
   if (epi == EPI_RELU2)
     return out_f32 ? -1 : big_dispatch<EPI_RELU2, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, ws_elems, M, N, K, bn, S, reduce, s);
   if (epi == EPI_SILU)
@@ -702,7 +704,7 @@ int launch_gemm_moe_big(const uint16_t* X, int ldx, const uint16_t* W, void* Y, 
       K % 128 != 0 || S < 1 ||
       S > K / 64)
     return -1;
-  if (epi != EPI_NONE && !epi_is_glu(epi)) return -1;
+  if (epi != EPI_NONE && epi != EPI_SILU && epi != EPI_CLAMP_GLU) return -1;
   if (epi_is_glu(epi) && out_f32) return -1;
   if (S > 1 && (epi != EPI_NONE || !out_f32)) return -1;  // K slices write fp32 partial slabs
   if (epi == EPI_SILU)

@@ -4,18 +4,21 @@
 
 namespace xot {
 
-enum { EPI_NONE = 0, EPI_RESID = 1, EPI_SILU = 2, EPI_CLAMP_GLU = 3, EPI_RELU2 = 4 };
+enum { EPI_NONE = 0, EPI_RESID = 1, EPI_SILU = 2, EPI_CLAMP_GLU = 3, EPI_RELU2 = 4, EPI_GELU_GLU = 5 };
 
 // epilogues that turn a (gate, up) column pair into one output column
-constexpr bool epi_is_glu(int epi) { return epi == EPI_SILU || epi == EPI_CLAMP_GLU; }
+constexpr bool epi_is_glu(int epi) { return epi == EPI_SILU || epi == EPI_CLAMP_GLU || epi == EPI_GELU_GLU; }
 
-// silu(g) u, or the clamped form: g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clamp(u, -limit, limit)
+// silu(g) u, gelu_tanh(g) u, or the clamped form: g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clamp(u, -limit, limit)
 template <int EPI>
 __device__ __forceinline__ float glu_pair(float g, float u, float limit) {
   if constexpr (EPI == EPI_CLAMP_GLU) {
     g = fminf(g, limit);
     u = fminf(fmaxf(u, -limit), limit);
     return g / (1.0f + __expf(-1.702f * g)) * (u + 1.0f);
+  } else if constexpr (EPI == EPI_GELU_GLU) {
+    // (1 + tanh z) / 2 = 1 / (1 + e^-2z): no cancellation where tanh z nears -1
+    return g / (1.0f + __expf(-1.5957691216057308f * (g + 0.044715f * g * g * g))) * u;
   } else {
     return silu(g) * u;
   }

@@ -696,9 +696,10 @@ int launch_gemm_w4(const uint16_t* X, int ldx, const uint16_t* W, const uint16_t
     else w4_launch<EPI_NONE, true, true>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, mi, group_m, st);
     return 0;
   }
-  if (epi == EPI_CLAMP_GLU || epi == EPI_RELU2) {
+  if (epi == EPI_CLAMP_GLU || epi == EPI_RELU2 || epi == EPI_GELU_GLU) {
     if (out_f32) return -1;
     if (epi == EPI_RELU2) w4_launch<EPI_RELU2, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
+    else if (epi == EPI_GELU_GLU) w4_launch<EPI_GELU_GLU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);
     else w4_launch<EPI_CLAMP_GLU, false, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st, epi_arg);
   } else if (epi == EPI_SILU) {
     if (out_f32) w4_launch<EPI_SILU, true, false>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, 1, mi, group_m, st);

@@ -51,16 +51,34 @@ __global__ void resid_scale_norm_k(float* __restrict__ x, const float* __restric
 }
 
 // ------------------------------------------------------------------ gelu_tanh(gate) * up
-template <typename AT>
-__global__ void gelu_mul_k(const float* __restrict__ P, int ldp, int gate_off, int up_off, int F, AT* __restrict__ out,
-                           int ldo, int64_t total) {
+// up_off < 0: gate and up columns alternate in tiles of 16 from gate_off on.  W columns per thread: memory-bound, so float4
+// where the rows allow it.
+template <typename AT, int W>
+__global__ __launch_bounds__(256) void gelu_mul_k(const float* __restrict__ P, int ldp, int gate_off, int up_off, int F,
+                                                  AT* __restrict__ out, int ldo, int64_t total) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= total) return;
-  const int64_t t = idx / F;
-  const int i = (int)(idx - t * F);
-  const float z = P[t * ldp + gate_off + i], u = P[t * ldp + up_off + i];
-  const float g = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-  stf(out + t * ldo + i, g * u);
+  const int nw = F / W;
+  const int64_t t = idx / nw;
+  const int i = (int)(idx - t * nw) * W;
+  const float* gp = P + t * ldp + gate_off + (up_off < 0 ? 32 * (i >> 4) + (i & 15) : i);
+  const float* up = up_off < 0 ? gp + 16 : P + t * ldp + up_off + i;
+  float z[W], u[W], y[W];
+  if constexpr (W == 4) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(gp), b = *reinterpret_cast<const f32x4*>(up);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z[k] = a[k], u[k] = b[k];
+  } else {
+    z[0] = gp[0];
+    u[0] = up[0];
+  }
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    const float g = 0.5f * z[k] * (1.0f + tanhf(0.7978845608028654f * (z[k] + 0.044715f * z[k] * z[k] * z[k])));
+    y[k] = g * u[k];
+  }
+  if constexpr (W == 4) st4(out + t * ldo + i, f32x4{y[0], y[1], y[2], y[3]});
+  else stf(out + t * ldo + i, y[0]);
 }
 
 // gelu_tanh(gate) * the token's slice of a table: out[t, i] = gelu(P[t, off + i]) * table[ids[t], col0 + i]; W columns per
@@ -846,17 +864,23 @@ void gelu_mul(const at::Tensor& P, int64_t gate_off, int64_t up_off, int64_t F, 
   MCHECK(out.is_cuda() && is_act(out) && out.dim() == 2 && out.size(0) == T && out.size(1) >= F && out.stride(1) == 1,
          "out must be [T, >= F] rows");
   const int ldo = (int)out.stride(0);
-  cols_ok(P, gate_off, F, "gate");
-  cols_ok(P, up_off, F, "up");
-  const int64_t total = T * F;
-  if (total == 0) return;
+  const bool tiles = up_off < 0;
+  cols_ok(P, gate_off, tiles ? (F + 15) / 16 * 32 : F, "gate");
+  if (!tiles) cols_ok(P, up_off, F, "up");
+  if (T * F == 0) return;
+  const bool vec = (ldp | gate_off | F | ldo | (tiles ? 0 : up_off)) % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(P.data_ptr()) | reinterpret_cast<uintptr_t>(out.data_ptr())) & 15) == 0;
+  const int64_t total = T * F / (vec ? 4 : 1);
   const int blocks = (int)((total + 255) / 256);
-  if (out.scalar_type() == at::kBFloat16)
-    gelu_mul_k<uint16_t><<<blocks, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)gate_off, (int)up_off, (int)F,
-                                                       (uint16_t*)out.data_ptr(), ldo, total);
-  else
-    gelu_mul_k<float><<<blocks, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)gate_off, (int)up_off, (int)F,
-                                                    out.data_ptr<float>(), ldo, total);
+#define GM_GO(AT, W)                                                                                                        \
+  gelu_mul_k<AT, W><<<blocks, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)gate_off, (int)up_off, (int)F,             \
+                                                  (AT*)out.data_ptr(), ldo, total)
+  if (out.scalar_type() == at::kBFloat16) {
+    if (vec) GM_GO(uint16_t, 4); else GM_GO(uint16_t, 1);
+  } else {
+    if (vec) GM_GO(float, 4); else GM_GO(float, 1);
+  }
+#undef GM_GO
 }
 
 void gelu_gather_mul(const at::Tensor& P, int64_t off, const at::Tensor& table, const at::Tensor& ids, int64_t col0, int64_t n,

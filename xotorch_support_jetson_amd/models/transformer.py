@@ -29,7 +29,7 @@ from ..inference.shard import Shard
 from ..ops import kernels as K
 from ..ops._ext import require
 from ..ops.linear import (FUSE_MERGE, FUSE_NORM, PendingNorm, layout_of, linear, linear_resid_norm, linear_rope_kv,
-                          linear_slabs, scratch)
+                          linear_slabs, scratch, stream_rows)
 from ..ops.rope import longrope_window, rope_shift, rope_table
 from .config import ModelConfig
 from .weights import ShardWeights, expert
@@ -43,6 +43,11 @@ MOE_DN_SPLITS = int(os.environ.get("XOT_MOE_DN_SPLITS", "0"))  # force the group
 MOE_PP2 = os.environ.get("XOT_MOE_PP2", "1") == "1"  # 256-row expert tiles on the two-phase ping-pong schedule
 PAGE = 64
 # tokens of a step from which the second projections of low-rank gates run as GEMMs (below: inside the gate kernel, in fp32)
+# a parallel block's gate / up rows in a GEMM of their own, which ends in the gated activation: from 1024 tokens (the row count of
+# the four-wave tile) and 2^23 gate / up results on.  Against one GEMM and a pass over its fp32 result: 1024 x (8960 | 11264)
+# x 2048 91 us / 100, 2048 rows 168 / 179, 7000 rows 875 / 1130; 768 rows 82 / 70, 48 rows 35 / 25 and 2048 x (512 | 1024) x
+# 512 26 / 20, where the second launch costs more than the pass
+GELU_EPI_ROWS, GELU_EPI_SIZE = 1024, 1 << 23
 LOW_RANK_GEMM_ROWS = int(os.environ.get("XOT_LOW_RANK_GEMM_ROWS", "256"))
 
 
@@ -465,6 +470,23 @@ class ShardModel:
     K.glu_act(torch.cat([t[:, :, 0].reshape(-1, n), t[:, :, 1].reshape(-1, n)], 1), 0, n, n, clamped, limit, out)
     return out
 
+  def _in_and_act(self, hn: torch.Tensor, lw, rows):
+    """A parallel block's input projections P and its gated activation (None without a feed-forward)."""
+    ff = lw.spec.ff
+    n0, n = lw.cols.get("gate_up", (0, 0))
+    if (n and hn.is_cuda and layout_of(lw.in_w) == "stream" and hn.shape[0] >= GELU_EPI_ROWS
+        and hn.shape[0] * n >= GELU_EPI_SIZE):
+      return self._proj(hn, stream_rows(lw.in_w, 0, n0)), linear(hn, stream_rows(lw.in_w, n0, n0 + n), epi="gelu_glu")
+    P = self._proj(hn, lw.in_w)
+    if not ff:
+      return P, None
+    act = rows("act", ff, lw.down_w.shape[1])
+    if n:
+      K.gelu_mul(P, n0, -1, ff, act)
+    else:
+      K.gelu_mul(P, lw.cols["gate"][0], lw.cols["up"][0], ff, act)
+    return P, act
+
   def _router(self, hn: torch.Tensor, w: torch.Tensor, E: int) -> torch.Tensor:
     """fp32 router logits [T, E] of a projection whose first E rows are the router."""
     if hn.is_cuda and hn.dtype == torch.bfloat16 and layout_of(w) == "rowmajor" and (
@@ -516,7 +538,8 @@ class ShardModel:
   def _forward_mixed(self, x: torch.Tensor, inp: StepInputs) -> torch.Tensor:
     """Layers of config.layer_specs on an fp32 residual stream h:
       hn = h / rms(h) * g                       one scalar gain per norm (fused into the previous layer's residual add)
-      P  = hn @ in_w^T                          every projection of the layer in one GEMM, fp32 result
+      P  = hn @ in_w^T                          every projection of the layer in one GEMM, fp32 result (long
+                                                steps: gate | up in one that ends in the gated activation)
       mix = [attn_scale * attention | rec_scale * recurrence]    both mixers read hn; outputs side by side along K
       h += ls1 * (mix @ out_w^T) + ls2 * (gelu_tanh(gate) * up) @ down_w^T
     Returns h (non-last shard) or logit_scale * head(norm(h rows inp.last_idx))."""
@@ -554,7 +577,7 @@ class ShardModel:
     for j, li in enumerate(self.layer_ids):
       lw = w.layers[li]
       s = lw.spec
-      P = self._proj(hn, lw.in_w)
+      P, act = self._in_and_act(hn, lw, rows)
       live = sum(sz for _, sz in lw.mix_cols.values())
       mix = rows("mix", live, lw.out_w.shape[1])
       if s.attn is not None:
@@ -564,8 +587,6 @@ class ShardModel:
       y1 = self._proj(mix, lw.out_w)
       y2 = None
       if s.ff:
-        act = rows("act", s.ff, lw.down_w.shape[1])
-        K.gelu_mul(P, lw.cols["gate"][0], lw.cols["up"][0], s.ff, act)
         y2 = self._proj(act, lw.down_w)
       nxt = w.layers[self.layer_ids[j + 1]].norm_g if j + 1 < n else None
       K.resid_scale_norm(h, y1, lw.ls1, y2, lw.ls2 if y2 is not None else None, gain=nxt, eps=c.rms_norm_eps,

@@ -14,8 +14,8 @@ import torch
 from . import reference as ref
 from ._ext import require
 
-EPI = {"none": 0, "resid": 1, "silu": 2, "clamp_glu": 3, "relu2": 4}
-GLU_EPI = ("silu", "clamp_glu")  # epilogues that turn interleaved (gate, up) columns into half as many
+EPI = {"none": 0, "resid": 1, "silu": 2, "clamp_glu": 3, "relu2": 4, "gelu_glu": 5}
+GLU_EPI = ("silu", "clamp_glu", "gelu_glu")  # epilogues that turn interleaved (gate, up) columns into half as many
 PAGE = 64
 
 
@@ -452,7 +452,8 @@ def resid_scale_norm(x, y1=None, s1=None, y2=None, s2=None, gain=None, eps: floa
 
 
 def gelu_mul(P, gate_off: int, up_off: int, F: int, out) -> None:
-  """out[:, :F] = gelu_tanh(P[:, gate_off : +F]) * P[:, up_off : +F]  (out rows may be wider: K padding)."""
+  """out[:, :F] = gelu_tanh(P[:, gate_off : +F]) * P[:, up_off : +F]  (out rows may be wider: K padding).  up_off < 0: gate and
+  up columns alternate in tiles of 16 from gate_off on."""
   _mix("gelu_mul", _gpu(P))(P, int(gate_off), int(up_off), int(F), out)
 
 

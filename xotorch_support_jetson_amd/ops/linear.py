@@ -100,6 +100,14 @@ def to_stream_layout(w: torch.Tensor) -> torch.Tensor:
   return s
 
 
+def stream_rows(w: torch.Tensor, n0: int, n1: int) -> torch.Tensor:
+  """Rows n0 .. n1 (multiples of 16) of a pre-shuffled weight: its blocks of 16 rows lie one after the other."""
+  assert layout_of(w) == "stream" and n0 % 16 == 0 and n1 % 16 == 0
+  s = w[n0:n1]
+  s.xot_layout = "stream"
+  return s
+
+
 def to_stream8_layout(w: torch.Tensor) -> torch.Tensor:
   """Weight-only FP8 copy of a row-major [N, K] GPU weight: shuffled e4m3 bytes tagged "stream8", the
   per-row fp32 scales in `.xot_scale`."""
@@ -408,13 +416,13 @@ class GemmPolicy:
       self._store(key, got)
       return got
     cands = []
-    if M <= STREAM_MAX_M:
+    if M <= STREAM_MAX_M and epi != "gelu_glu":
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
-    if wave:
+    if wave and epi != "gelu_glu":
       cands += self._wave_cands(M, N, Kd, epi, wave == "rope")
     if M >= BIG_MIN_M and Kd % 128 == 0:
       big = self._big_cands(M, N, Kd)
-      cands += [c for c in big if c[1] in (2256, 128, 4256)] if epi in ("clamp_glu", "relu2") else big  # (the tiles built with them)
+      cands += [c for c in big if c[1] in (2256, 128, 4256)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
     if not cands:
       raise RuntimeError(f"no GEMM configuration for pre-shuffled N={N} K={Kd} M={M}")
     if self._no_tuning():
@@ -660,7 +668,8 @@ def _pending_cfg(p: PendingNorm, w: torch.Tensor, bias, epi: str, wave: str = "y
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, residual: torch.Tensor | None = None,
            epi: str = "none", out: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
            epi_arg: float = 0.0) -> torch.Tensor:
-  """epi "clamp_glu" (limit: epi_arg) and "relu2" run on pre-shuffled GPU weights with bf16 output only."""
+  """epi "clamp_glu" (limit: epi_arg), "gelu_glu" (from BIG_MIN_M rows) and "relu2" run on pre-shuffled GPU weights with bf16
+  output only."""
   if isinstance(x, PendingNorm):
     cfg = None if (residual is not None or (out_dtype not in (None, torch.bfloat16))
                    or (out is not None and out.dtype != torch.bfloat16)) else _pending_cfg(x, w, bias, epi)

@@ -247,7 +247,12 @@ def resid_scale_norm(x, y1, s1, y2, s2, gain, eps, out):
 
 
 def gelu_mul(P, gate_off, up_off, Fd, out):
-  z, u = P[:, gate_off:gate_off + Fd].float(), P[:, up_off:up_off + Fd].float()
+  if up_off < 0:
+    n = -(-Fd // 16)
+    t = P[:, gate_off:gate_off + 32 * n].float().reshape(-1, n, 2, 16)
+    z, u = t[:, :, 0].reshape(-1, 16 * n)[:, :Fd], t[:, :, 1].reshape(-1, 16 * n)[:, :Fd]
+  else:
+    z, u = P[:, gate_off:gate_off + Fd].float(), P[:, up_off:up_off + Fd].float()
   out[:, :Fd] = (0.5 * z * (1 + torch.tanh(0.7978845608028654 * (z + 0.044715 * z ** 3))) * u).to(out.dtype)
 
 
