@@ -57,6 +57,13 @@ __device__ __forceinline__ void ld8(const uint16_t* p, float* o) {
   for (int i = 0; i < 8; ++i) o[i] = bf2f(a[i]);
 }
 
+__device__ __forceinline__ void st2(float* p, float a, float b) {
+  typedef float f32x2_s __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<f32x2_s*>(p) = f32x2_s{a, b};
+}
+__device__ __forceinline__ void st2(uint16_t* p, float a, float b) {
+  *reinterpret_cast<uint32_t*>(p) = (uint32_t)f2bf(a) | (uint32_t)f2bf(b) << 16;
+}
 __device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ void st4(uint16_t* p, f32x4 v) {
   *reinterpret_cast<s16x4*>(p) = s16x4{(short)f2bf(v[0]), (short)f2bf(v[1]), (short)f2bf(v[2]), (short)f2bf(v[3])};

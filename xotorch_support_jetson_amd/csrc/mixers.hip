@@ -3,13 +3,9 @@
 //   resid_scale_norm   x += s1 * y1 (+ s2 * y2) on the fp32 residual stream, then RMS norm with one scalar gain
 //   gelu_mul           gelu_tanh(gate) * up out of a fused projection's columns
 //   gelu_gather_mul    gelu_tanh(gate) * the token's slice of a table (per-layer side inputs)
-//   rope_kv_store      partial rotate-half RoPE on q and k, paged write of the rotated key and of the value
-//                      (the value may be the un-rotated key)
 //   attn_gated_chunk   chunk-local attention with sigmoid(score + bias[head]) weights, no normalisation: an MFMA
 //                      kernel for prompt portions (bf16), a (token, kv head, key split) kernel for single tokens
 //                      and fp32, a wave per (token, head) for groups above 8 query heads
-//   delta_prep         short causal convolutions + SiLU, unit-norm q / k, sigmoid write strength, scalar decay
-//   conv_state_update  the last taps-1 convolution inputs of every sequence -> its state slot
 //   gla_prep           per-key-channel decay sigmoid(low-rank z)^(1/tau)
 //   linear_recurrence  S <- decay * S, delta-rule or outer-product write, o = S^T q; fp32 state per slot (token by token here;
 //                      prompts in chunks of 16 tokens: recurrence_chunk.hip)
@@ -25,20 +21,26 @@ namespace {
 using namespace mix;
 
 // ------------------------------------------------------------------ residual + scalar-gain RMS norm
+// x += s1 * y1 (+ s2 * y2); y1 / y2 may still be split-K slabs of their projections, summed here in slab order.
+struct Branch {
+  const float* y;  // null: none
+  const float* s;
+  int ld, S;
+  int64_t ss;
+};
+
 template <typename AT>
-__global__ void resid_scale_norm_k(float* __restrict__ x, const float* __restrict__ y1, const float* __restrict__ s1,
-                                   const float* __restrict__ y2, const float* __restrict__ s2,
-                                   const float* __restrict__ gain, float eps, AT* __restrict__ out, int D, int ld1,
-                                   int ld2, int ldo) {
+__global__ void resid_scale_norm_k(float* __restrict__ x, Branch b1, Branch b2, const float* __restrict__ gain, float eps,
+                                   AT* __restrict__ out, int D, int ldo) {
   __shared__ float red[16];
   const int64_t r = blockIdx.x;
   float* xr = x + r * D;
   float ss = 0.0f;
   for (int i = threadIdx.x; i < D; i += blockDim.x) {
     float v = xr[i];
-    if (y1) {
-      float a = s1[i] * y1[r * ld1 + i];
-      if (y2) a += s2[i] * y2[r * ld2 + i];
+    if (b1.y) {
+      float a = b1.s[i] * slab1(b1.y + r * b1.ld + i, b1.S, b1.ss);
+      if (b2.y) a += b2.s[i] * slab1(b2.y + r * b2.ld + i, b2.S, b2.ss);
       v += a;
       xr[i] = v;
     }
@@ -48,6 +50,44 @@ __global__ void resid_scale_norm_k(float* __restrict__ x, const float* __restric
   ss = block_sum(ss, red);
   const float k = gain[0] / sqrtf(ss / (float)D + eps);
   for (int i = threadIdx.x; i < D; i += blockDim.x) stf(out + r * ldo + i, xr[i] * k);
+}
+
+// Rows of at most 1024 R numbers in whole vectors of four: the row stays in registers between the sum of squares and the
+// write.  Memory-bound on long steps (12807 x 2048, two branches: 127 us with scalar loads and a second pass over x, 74 here);
+// on short ones it saves the slab reduces of both branches' projections, 4.7 us each.
+template <typename AT, int R>
+__global__ __launch_bounds__(256) void resid_scale_norm_reg_k(float* __restrict__ x, Branch b1, Branch b2,
+                                                              const float* __restrict__ gain, float eps, AT* __restrict__ out,
+                                                              int D, int ldo) {
+  __shared__ float red[16];
+  const int64_t r = blockIdx.x;
+  float* xr = x + r * D;
+  auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
+  f32x4 v[R];
+  float ss = 0.0f;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = 4 * (threadIdx.x + 256 * j);
+    v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i >= D) continue;
+    v[j] = ld(xr + i);
+    if (b1.y) {
+      f32x4 a = ld(b1.s + i) * slab4(b1.y + r * b1.ld + i, b1.S, b1.ss);
+      if (b2.y) a += ld(b2.s + i) * slab4(b2.y + r * b2.ld + i, b2.S, b2.ss);
+      v[j] += a;
+      st4(xr + i, v[j]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
+  }
+  if (!out) return;
+  ss = block_sum(ss, red);
+  const float k = gain[0] / sqrtf(ss / (float)D + eps);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = 4 * (threadIdx.x + 256 * j);
+    if (i < D) st4(out + r * ldo + i, v[j] * k);
+  }
 }
 
 // ------------------------------------------------------------------ gelu_tanh(gate) * up
@@ -108,42 +148,6 @@ __global__ __launch_bounds__(256) void gelu_gather_mul_k(const float* __restrict
     y[k] = 0.5f * z[k] * (1.0f + tanhf(0.7978845608028654f * (z[k] + 0.044715f * z[k] * z[k] * z[k]))) * ldf(e + k);
   if constexpr (W == 4) st4(out + t * ldo + i, f32x4{y[0], y[1], y[2], y[3]});
   else stf(out + t * ldo + i, y[0]);
-}
-
-// ------------------------------------------------------------------ RoPE + paged key / value write
-// cos_sin [rows, R]: row p = [cos(p f_0 .. f_{R/2-1}) | sin(...)].  Pair (i, i + R/2), i < R/2; dims >= R pass.
-template <typename AT>
-__global__ void rope_kv_store_k(const float* __restrict__ P, int ldp, int q_off, int k_off, int v_off, int H, int G, int d,
-                                int R, const int* __restrict__ pos, const float* __restrict__ cos_sin,
-                                const int64_t* __restrict__ slots, AT* __restrict__ q_out, AT* __restrict__ k_cache,
-                                AT* __restrict__ v_cache) {
-  const int t = blockIdx.x;
-  const float* row = P + (int64_t)t * ldp;
-  const float* cs = cos_sin + (int64_t)pos[t] * R;
-  const int half = R >> 1;
-  const int64_t slot = slots[t];
-  const int n = (H + G) * d;
-  for (int e = threadIdx.x; e < n; e += blockDim.x) {
-    const int head = e / d, i = e - head * d;
-    const bool isq = head < H;
-    const float* x = row + (isq ? q_off + head * d : k_off + (head - H) * d);
-    float v = x[i];
-    const float raw = v;
-    if (i < half) {
-      v = x[i] * cs[i] - x[i + half] * cs[half + i];
-    } else if (i < R) {
-      const int j = i - half;
-      v = x[i] * cs[j] + x[j] * cs[half + j];
-    }
-    if (isq) {
-      stf(q_out + ((int64_t)t * H + head) * d + i, v);
-    } else if (slot >= 0) {
-      const int g = head - H;
-      const int64_t pg = (slot / PAGE_TOK) * G + g;
-      stf(k_cache + (pg * PAGE_TOK + (slot % PAGE_TOK)) * d + i, v);
-      stf(v_cache + (pg * d + i) * PAGE_TOK + (slot % PAGE_TOK), v_off >= 0 ? row[v_off + g * d + i] : raw);
-    }
-  }
 }
 
 // ------------------------------------------------------------------ chunk-local gated attention
@@ -484,116 +488,45 @@ __global__ __launch_bounds__(256) void attn_gated_chunk_mfma_k(
   }
 }
 
-// ------------------------------------------------------------------ delta-rule inputs
-// Channels [q: G d | k: G d | v: H dv] at P[:, x_off ...]; conv_w [C, taps] (last column: the current token);
-// conv_state [slots, taps - 1, C] holds the inputs before this step (zeros for a new sequence).
-// qkv [T, C]: q = unit(silu(conv q)) * d^-1/2, k = unit(silu(conv k)), v = silu(conv v);
-// beta [T, H] = sigmoid(P[b_off + h]); decay [T, H] = exp(-exp(A_log[h]) softplus(P[a_off + h] + dt_bias[h])).
-__global__ void delta_prep_k(const float* __restrict__ P, int ldp, int x_off, int b_off, int a_off,
-                             const float* __restrict__ conv_w, int taps, const float* __restrict__ conv_state,
-                             const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B,
-                             const float* __restrict__ A_log, const float* __restrict__ dt_bias, int H, int G, int d, int dv,
-                             float* __restrict__ qkv, float* __restrict__ beta, float* __restrict__ decay, int T, int tpb) {
-  // workgroup = (tpb <= 8 consecutive tokens, unit): units 0 .. G-1 the q heads, G .. 2G-1 the k heads, then H value
-  // heads, then the gates.  A thread owns one channel of the unit for all the tokens: their convolution inputs are
-  // loaded together and the tokens' sums of squares are reduced in one pass.  tpb is 1 for decode steps.
-  constexpr int TPB = 8;
-  __shared__ float red[TPB][4];
-  const int unit = blockIdx.y;
-  const int C = 2 * G * d + H * dv;
-  const int tbase = blockIdx.x * tpb;
-  if (unit == 2 * G + H) {
-    for (int e = threadIdx.x; e < tpb * H; e += blockDim.x) {
-      const int t = tbase + e / H, h = e % H;
-      if (t >= T || state_slots[seq_of(cu_q, B, t)] < 0) continue;
-      const float* row = P + (int64_t)t * ldp;
-      beta[(int64_t)t * H + h] = sigmoidf_(row[b_off + h]);
-      decay[(int64_t)t * H + h] = expf(-expf(A_log[h]) * softplusf_(row[a_off + h] + dt_bias[h]));
-    }
-    return;
-  }
-  const bool qk = unit < 2 * G;
-  const int c0 = qk ? unit * d : 2 * G * d + (unit - 2 * G) * dv, n = qk ? d : dv;
-  const int i = threadIdx.x;  // the launch gives a thread per channel of the widest unit (n <= blockDim.x <= 256)
-  const int c = c0 + i;
-  float y[TPB];
-  bool ok[TPB];
-#pragma unroll
-  for (int tt = 0; tt < TPB; ++tt) {
-    const int t = tbase + tt;
-    y[tt] = 0.0f;
-    ok[tt] = false;
-    if (tt >= tpb || t >= T) continue;
-    const int b = seq_of(cu_q, B, t);
-    const int slot = state_slots[b];
-    if (slot < 0) continue;
-    ok[tt] = true;
-    if (i >= n) continue;
-    const int local = t - cu_q[b], tstart = cu_q[b];
-    const float* st = conv_state + (int64_t)slot * (taps - 1) * C;
-    float acc = 0.0f;
-    for (int j = 0; j < taps; ++j) {
-      const int sidx = local - (taps - 1 - j);
-      const float x = sidx >= 0 ? P[(int64_t)(tstart + sidx) * ldp + x_off + c] : st[(int64_t)(taps - 1 + sidx) * C + c];
-      acc += conv_w[c * taps + j] * x;
-    }
-    y[tt] = siluf_(acc);
-  }
-  if (qk) {
-    const int wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-    for (int tt = 0; tt < TPB; ++tt) {
-      const float ss = wave_sum(y[tt] * y[tt]);
-      if ((threadIdx.x & 63) == 0) red[tt][wave] = ss;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int tt = 0; tt < TPB; ++tt) {
-      float ss = 0.0f;
-      for (int w = 0; w < nw; ++w) ss += red[tt][w];
-      float kn = 1.0f / sqrtf(ss + 1e-6f);
-      if (unit < G) kn *= 1.0f / sqrtf((float)d);
-      y[tt] *= kn;
-    }
-  }
-  if (i < n) {
-#pragma unroll
-    for (int tt = 0; tt < TPB; ++tt)
-      if (ok[tt]) qkv[(int64_t)(tbase + tt) * C + c] = y[tt];
-  }
-}
-
-__global__ void conv_state_update_k(const float* __restrict__ P, int ldp, int x_off, int C, int taps,
-                                    float* __restrict__ conv_state, const int* __restrict__ state_slots,
-                                    const int* __restrict__ cu_q) {
-  const int b = blockIdx.x;
-  const int slot = state_slots[b];
-  const int n = cu_q[b + 1] - cu_q[b];
-  if (slot < 0 || n <= 0) return;
-  float* st = conv_state + (int64_t)slot * (taps - 1) * C;
-  for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < C; c += gridDim.y * blockDim.x) {
-    // ascending: entry idx takes the old entry idx + n (> idx) or a token of this step
-    for (int idx = 0; idx < taps - 1; ++idx) {
-      const int s = n - (taps - 1) + idx;
-      st[(int64_t)idx * C + c] = s >= 0 ? P[(int64_t)(cu_q[b] + s) * ldp + x_off + c] : st[(int64_t)(idx + n) * C + c];
-    }
-  }
-}
-
 // ------------------------------------------------------------------ GLA decay
 // decay [T, HD] = exp(logsigmoid(z) / tau), z[c] = a2_b[c] + sum_r a2[c, r] P[t, a1_off + r]
-__global__ void gla_prep_k(const float* __restrict__ P, int ldp, int a1_off, int rank, const float* __restrict__ a2,
-                           const float* __restrict__ a2_b, float inv_tau, int HD, float* __restrict__ decay) {
-  extern __shared__ float ys[];  // [rank]
-  const int t = blockIdx.x;
-  for (int r = threadIdx.x; r < rank; r += blockDim.x) ys[r] = P[(int64_t)t * ldp + a1_off + r];
-  __syncthreads();
-  for (int c = threadIdx.x; c < HD; c += blockDim.x) {
-    float z = 0.0f;
-    for (int r = 0; r < rank; ++r) z += a2[(int64_t)c * rank + r] * ys[r];
-    z += a2_b[c];
-    decay[(int64_t)t * HD + c] = expf(logsigmoidf_(z) * inv_tau);
+// Workgroup = (TOK tokens, 256 channels): a thread reads its channel's weight row once for all the tokens; the tokens' rank
+// rows are the same for every lane (scalar loads, so neither LDS nor a barrier).  Bound by the exponentials and by latency:
+// 12807 tokens x 1024 channels, rank 16: 50 us, 62 with a workgroup per token and its rank row in LDS; eight tokens a
+// workgroup from 512 on, two below, where too few workgroups would be left.
+template <int TOK>
+__global__ __launch_bounds__(256) void gla_prep_k(const float* __restrict__ P, int ldp, int a1_off, int rank,
+                                                  const float* __restrict__ a2, const float* __restrict__ a2_b, float inv_tau,
+                                                  int HD, float* __restrict__ decay, int T) {
+  const int t0 = blockIdx.x * TOK, c = blockIdx.y * 256 + threadIdx.x;
+  if (c >= HD) return;
+  const float* w = a2 + (int64_t)c * rank;
+  const float b = a2_b[c];
+  const float* p[TOK];
+#pragma unroll
+  for (int i = 0; i < TOK; ++i) p[i] = P + (int64_t)min(t0 + i, T - 1) * ldp + a1_off;
+  float z[TOK];
+#pragma unroll
+  for (int i = 0; i < TOK; ++i) z[i] = 0.0f;
+  int r = 0;
+  if (rank % 4 == 0 && (reinterpret_cast<uintptr_t>(a2) & 15) == 0) {
+#pragma unroll 4
+    for (; r < rank; r += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(w + r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) z[i] += v[e] * p[i][r + e];
+    }
   }
+  for (; r < rank; ++r) {
+    const float v = w[r];
+#pragma unroll
+    for (int i = 0; i < TOK; ++i) z[i] += v * p[i][r];
+  }
+#pragma unroll
+  for (int i = 0; i < TOK; ++i)
+    if (t0 + i < T) decay[(int64_t)(t0 + i) * HD + c] = expf(logsigmoidf_(z[i] + b) * inv_tau);
 }
 
 // ------------------------------------------------------------------ the recurrence
@@ -803,18 +736,45 @@ __global__ __launch_bounds__(256) void linear_recurrence_k(
 }
 
 // ------------------------------------------------------------------ per-head RMS norm * weight * silu(gate)
-template <typename AT>
-__global__ void gated_rmsnorm_k(const float* __restrict__ o, const float* __restrict__ w, const float* __restrict__ P, int ldp,
-                                int g_off, float eps, float out_scale, AT* __restrict__ out, int ldo, int H, int dv) {
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+// A wave per (token, head), four heads a workgroup; W values a lane and load (12807 x 16 heads of 128: 90 us one value at a
+// time in workgroups of one wave, 64 here).
+template <typename AT, int W>
+__global__ __launch_bounds__(256) void gated_rmsnorm_k(const float* __restrict__ o, const float* __restrict__ w,
+                                                       const float* __restrict__ P, int ldp, int g_off, float eps,
+                                                       float out_scale, AT* __restrict__ out, int ldo, int H, int dv) {
+  const int t = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (h >= H) return;  // (wave-uniform; no workgroup barrier below)
+  typedef float vec __attribute__((ext_vector_type(W)));
   const float* x = o + ((int64_t)t * H + h) * dv;
+  const float* gp = P + (int64_t)t * ldp + g_off + h * dv;
+  AT* op = out + (int64_t)t * ldo + h * dv;
+  const int i0 = lane * W;
+  vec v = {}, g = {};
+  if (i0 < dv) {  // (the first 64 W values stay in registers: every head of at most 64 W)
+    v = *reinterpret_cast<const vec*>(x + i0);
+    g = *reinterpret_cast<const vec*>(gp + i0);
+  }
   float ss = 0.0f;
-  for (int i = lane; i < dv; i += 64) ss += x[i] * x[i];
+#pragma unroll
+  for (int e = 0; e < W; ++e) ss += v[e] * v[e];
+  for (int i = i0 + 64 * W; i < dv; i += 64 * W) {
+    const vec u = *reinterpret_cast<const vec*>(x + i);
+#pragma unroll
+    for (int e = 0; e < W; ++e) ss += u[e] * u[e];
+  }
   ss = wave_sum(ss);
   const float k = out_scale / sqrtf(ss / (float)dv + eps);
-  for (int i = lane; i < dv; i += 64) {
-    const float gate = P[(int64_t)t * ldp + g_off + h * dv + i];
-    stf(out + (int64_t)t * ldo + h * dv + i, x[i] * k * w[i] * siluf_(gate));
+  for (int i = i0; i < dv; i += 64 * W) {
+    if (i != i0) {
+      v = *reinterpret_cast<const vec*>(x + i);
+      g = *reinterpret_cast<const vec*>(gp + i);
+    }
+    const vec wv = *reinterpret_cast<const vec*>(w + i);
+#pragma unroll
+    for (int e = 0; e < W; ++e) v[e] = v[e] * k * wv[e] * siluf_(g[e]);
+    if constexpr (W == 4) st4(op + i, f32x4{v[0], v[1], v[2], v[3]});
+    else if constexpr (W == 2) st2(op + i, v[0], v[1]);
+    else stf(op + i, v[0]);
   }
 }
 
@@ -826,36 +786,53 @@ void resid_scale_norm(at::Tensor& x, const c10::optional<at::Tensor>& y1, const 
   MCHECK(x.dim() == 2, "x must be [T, D]");
   const int64_t T = x.size(0), D = x.size(1);
   if (T == 0) return;
-  auto chk = [&](const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& s) {
-    if (!y.has_value()) return;
-    MCHECK(ld_of(*y, "y") >= D && y->size(0) == T && y->size(1) >= D, "residual branch must be fp32 [T, >= D] rows");
+  auto al = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
+  bool vec = D % 4 == 0 && al(x);
+  auto branch = [&](const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& s) {
+    Branch b{};
+    if (!y.has_value()) return b;
+    const Slabs p = slabs_of(*y, "residual branch");
+    MCHECK(p.ld >= D && p.T == T && p.n >= D, "residual branch must be fp32 [T, >= D] rows");
     MCHECK(s.has_value(), "a residual branch needs its scale");
     f32c(*s, "scale");
     MCHECK(s->numel() == D, "residual branch scale must hold D numbers");
+    b.y = p.p;
+    b.s = s->data_ptr<float>();
+    b.ld = p.ld;
+    b.S = p.S;
+    b.ss = p.ss;
+    vec = vec && p.vec && al(*s);
+    return b;
   };
-  chk(y1, s1);
-  chk(y2, s2);
+  const Branch b1 = branch(y1, s1), b2 = branch(y2, s2);
   MCHECK(y1.has_value() || !y2.has_value(), "y2 without y1");
+  int ldo = 0;
   if (out.has_value()) {
     MCHECK(gain.has_value(), "a normed output needs the gain");
     f32c(*gain, "gain");
     MCHECK(gain->numel() == 1, "gain must hold one number");
     MCHECK(out->is_cuda() && is_act(*out) && out->dim() == 2 && out->size(0) == T && out->size(1) >= D && out->stride(1) == 1,
            "out must be [T, >= D] rows");
+    ldo = (int)out->stride(0);
+    vec = vec && ldo % 4 == 0 && al(*out);
   }
-  const int ld1 = y1.has_value() ? (int)y1->stride(0) : 0, ld2 = y2.has_value() ? (int)y2->stride(0) : 0;
-  const int ldo = out.has_value() ? (int)out->stride(0) : 0;
-  const float* p1 = y1.has_value() ? y1->data_ptr<float>() : nullptr;
-  const float* q1 = y1.has_value() ? s1->data_ptr<float>() : nullptr;
-  const float* p2 = y2.has_value() ? y2->data_ptr<float>() : nullptr;
-  const float* q2 = y2.has_value() ? s2->data_ptr<float>() : nullptr;
   const float* g = out.has_value() ? gain->data_ptr<float>() : nullptr;
-  if (out.has_value() && out->scalar_type() == at::kBFloat16)
-    resid_scale_norm_k<uint16_t><<<T, 256, 0, stream()>>>(x.data_ptr<float>(), p1, q1, p2, q2, g, (float)eps,
-                                                          (uint16_t*)out->data_ptr(), (int)D, ld1, ld2, ldo);
-  else
-    resid_scale_norm_k<float><<<T, 256, 0, stream()>>>(x.data_ptr<float>(), p1, q1, p2, q2, g, (float)eps,
-                                                       out.has_value() ? out->data_ptr<float>() : nullptr, (int)D, ld1, ld2, ldo);
+#define RSN_GO(AT, ...)                                                                                     \
+  __VA_ARGS__<<<T, 256, 0, stream()>>>(x.data_ptr<float>(), b1, b2, g, (float)eps,                          \
+                                       out.has_value() ? (AT*)out->data_ptr() : nullptr, (int)D, ldo)
+#define RSN_PICK(AT)                                                       \
+  if (vec && D <= 1024) RSN_GO(AT, resid_scale_norm_reg_k<AT, 1>);         \
+  else if (vec && D <= 2048) RSN_GO(AT, resid_scale_norm_reg_k<AT, 2>);    \
+  else if (vec && D <= 4096) RSN_GO(AT, resid_scale_norm_reg_k<AT, 4>);    \
+  else if (vec && D <= 8192) RSN_GO(AT, resid_scale_norm_reg_k<AT, 8>);    \
+  else RSN_GO(AT, resid_scale_norm_k<AT>)
+  if (out.has_value() && out->scalar_type() == at::kBFloat16) {
+    RSN_PICK(uint16_t);
+  } else {
+    RSN_PICK(float);
+  }
+#undef RSN_PICK
+#undef RSN_GO
 }
 
 void gelu_mul(const at::Tensor& P, int64_t gate_off, int64_t up_off, int64_t F, at::Tensor& out) {
@@ -908,41 +885,6 @@ void gelu_gather_mul(const at::Tensor& P, int64_t off, const at::Tensor& table, 
     if (vec) GGM_GO(float, 4); else GGM_GO(float, 1);
   }
 #undef GGM_GO
-}
-
-void rope_kv_store(const at::Tensor& P, int64_t q_off, int64_t k_off, int64_t v_off, int64_t H, int64_t G, int64_t d,
-                   int64_t R, const at::Tensor& pos, const at::Tensor& cos_sin, const at::Tensor& slots, at::Tensor& q_out,
-                   at::Tensor& k_cache, at::Tensor& v_cache) {
-  const int ldp = ld_of(P, "P");
-  const int64_t T = P.size(0);
-  if (T == 0) return;
-  i32c(pos, "pos");
-  f32c(cos_sin, "cos_sin");
-  MCHECK(slots.is_cuda() && slots.scalar_type() == at::kLong && slots.is_contiguous() && slots.numel() == T && pos.numel() == T,
-         "pos / slots must hold one entry per token");
-  MCHECK(R % 2 == 0 && R >= 0 && R <= d && (R == 0 || (cos_sin.dim() == 2 && cos_sin.size(1) == R)), "bad rotary dims");
-  cols_ok(P, q_off, H * d, "q");
-  cols_ok(P, k_off, G * d, "k");
-  if (v_off >= 0) cols_ok(P, v_off, G * d, "v");
-  MCHECK(q_out.is_cuda() && is_act(q_out) && q_out.is_contiguous() && q_out.numel() == T * H * d, "q_out must be [T, H, d]");
-  MCHECK(k_cache.is_cuda() && k_cache.scalar_type() == q_out.scalar_type() && k_cache.is_contiguous() && k_cache.dim() == 4 &&
-             k_cache.size(1) == G && k_cache.size(2) == PAGE_TOK && k_cache.size(3) == d,
-         "k_cache must be [pages, G, 64, d] of q_out's dtype");
-  MCHECK(v_cache.is_cuda() && v_cache.scalar_type() == q_out.scalar_type() && v_cache.is_contiguous() && v_cache.dim() == 4 &&
-             v_cache.size(0) == k_cache.size(0) && v_cache.size(1) == G && v_cache.size(2) == d && v_cache.size(3) == PAGE_TOK,
-         "v_cache must be [pages, G, d, 64] of q_out's dtype");
-  // positions and slots are checked on the host by their producer (the block manager hands out slots < pages * 64
-  // and the runner bounds positions by the table's rows)
-  if (q_out.scalar_type() == at::kBFloat16)
-    rope_kv_store_k<uint16_t><<<T, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)q_off, (int)k_off, (int)v_off, (int)H,
-                                                       (int)G, (int)d, (int)R, pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
-                                                       slots.data_ptr<int64_t>(), (uint16_t*)q_out.data_ptr(),
-                                                       (uint16_t*)k_cache.data_ptr(), (uint16_t*)v_cache.data_ptr());
-  else
-    rope_kv_store_k<float><<<T, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)q_off, (int)k_off, (int)v_off, (int)H, (int)G,
-                                                    (int)d, (int)R, pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
-                                                    slots.data_ptr<int64_t>(), q_out.data_ptr<float>(),
-                                                    k_cache.data_ptr<float>(), v_cache.data_ptr<float>());
 }
 
 template <int NK>
@@ -1043,47 +985,6 @@ void attn_gated_chunk(const at::Tensor& q, const at::Tensor& k_cache, const at::
         (int)chunk, (float)out_scale, out.data_ptr<float>(), ldo, (int)H, (int)G, (int)d);
 }
 
-void delta_prep(const at::Tensor& P, int64_t x_off, int64_t b_off, int64_t a_off, const at::Tensor& conv_w,
-                at::Tensor& conv_state, const at::Tensor& state_slots, const at::Tensor& cu_q, const at::Tensor& A_log,
-                const at::Tensor& dt_bias, int64_t H, int64_t G, int64_t d, int64_t dv, at::Tensor& qkv, at::Tensor& beta,
-                at::Tensor& decay) {
-  const int ldp = ld_of(P, "P");
-  const int64_t T = P.size(0), C = 2 * G * d + H * dv;
-  if (T == 0) return;
-  f32c(conv_w, "conv_w");
-  f32c(conv_state, "conv_state");
-  f32c(A_log, "A_log");
-  f32c(dt_bias, "dt_bias");
-  f32c(qkv, "qkv");
-  f32c(beta, "beta");
-  f32c(decay, "decay");
-  i32c(state_slots, "state_slots");
-  i32c(cu_q, "cu_q");
-  MCHECK(conv_w.dim() == 2 && conv_w.size(0) == C, "conv_w must be [C, taps]");
-  const int64_t taps = conv_w.size(1), B = state_slots.numel();
-  MCHECK(taps >= 1 && conv_state.dim() == 3 && conv_state.size(1) == taps - 1 && conv_state.size(2) == C,
-         "conv_state must be [slots, taps - 1, C]");
-  MCHECK(cu_q.numel() == B + 1 && A_log.numel() == H && dt_bias.numel() == H && H % G == 0, "delta_prep: shape mismatch");
-  MCHECK(qkv.numel() == T * C && beta.numel() == T * H && decay.numel() == T * H, "delta_prep: output shape mismatch");
-  cols_ok(P, x_off, C, "conv inputs");
-  cols_ok(P, b_off, H, "beta");
-  cols_ok(P, a_off, H, "decay");
-  MCHECK(d <= 256 && dv <= 256, "delta_prep: head sizes above 256");
-  const int bs = (int)(((std::max(d, dv) + 63) / 64) * 64);
-  const int tpb = T > 256 ? 8 : 1;
-  delta_prep_k<<<dim3((unsigned)((T + tpb - 1) / tpb), (unsigned)(2 * G + H + 1)), bs, 0, stream()>>>(
-      P.data_ptr<float>(), ldp, (int)x_off, (int)b_off, (int)a_off, conv_w.data_ptr<float>(), (int)taps,
-      conv_state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(), (int)B, A_log.data_ptr<float>(),
-      dt_bias.data_ptr<float>(), (int)H, (int)G, (int)d, (int)dv, qkv.data_ptr<float>(), beta.data_ptr<float>(),
-      decay.data_ptr<float>(), (int)T, tpb);
-  if (taps > 1) {
-    const dim3 grid((unsigned)B, (unsigned)((C + 255) / 256));
-    conv_state_update_k<<<grid, 256, 0, stream()>>>(P.data_ptr<float>(), ldp, (int)x_off, (int)C, (int)taps,
-                                                    conv_state.data_ptr<float>(), state_slots.data_ptr<int>(),
-                                                    cu_q.data_ptr<int>());
-  }
-}
-
 void gla_prep(const at::Tensor& P, int64_t a1_off, const at::Tensor& a2, const at::Tensor& a2_b, double tau, at::Tensor& decay) {
   const int ldp = ld_of(P, "P");
   const int64_t T = P.size(0);
@@ -1095,9 +996,13 @@ void gla_prep(const at::Tensor& P, int64_t a1_off, const at::Tensor& a2, const a
   const int64_t HD = a2.size(0), rank = a2.size(1);
   MCHECK(a2_b.numel() == HD && decay.numel() == T * HD && tau > 0, "gla_prep: shape mismatch");
   cols_ok(P, a1_off, rank, "decay projection");
-  gla_prep_k<<<T, 256, rank * sizeof(float), stream()>>>(P.data_ptr<float>(), ldp, (int)a1_off, (int)rank, a2.data_ptr<float>(),
-                                                         a2_b.data_ptr<float>(), (float)(1.0 / tau), (int)HD,
-                                                         decay.data_ptr<float>());
+#define GLA_GO(TOK)                                                                                                        \
+  gla_prep_k<TOK><<<dim3((unsigned)((T + TOK - 1) / TOK), (unsigned)((HD + 255) / 256)), 256, 0, stream()>>>(              \
+      P.data_ptr<float>(), ldp, (int)a1_off, (int)rank, a2.data_ptr<float>(), a2_b.data_ptr<float>(), (float)(1.0 / tau),  \
+      (int)HD, decay.data_ptr<float>(), (int)T)
+  if (T >= 512) GLA_GO(8);
+  else GLA_GO(2);
+#undef GLA_GO
 }
 
 // XOT_REC_COLS=1 / 2 forces the recurrences' channels per thread (A/B runs)
@@ -1215,15 +1120,25 @@ void gated_rmsnorm(const at::Tensor& o, const at::Tensor& w, const at::Tensor& P
   const int64_t H = o.numel() / (T * dv);
   cols_ok(P, g_off, H * dv, "gate");
   const int ldo = act_ld(out, T, H * dv, "out");
-  const dim3 grid((unsigned)T, (unsigned)H);
-  if (out.scalar_type() == at::kBFloat16)
-    gated_rmsnorm_k<uint16_t><<<grid, 64, 0, stream()>>>(o.data_ptr<float>(), w.data_ptr<float>(), P.data_ptr<float>(), ldp,
-                                                         (int)g_off, (float)eps, (float)out_scale, (uint16_t*)out.data_ptr(),
-                                                         ldo, (int)H, (int)dv);
-  else
-    gated_rmsnorm_k<float><<<grid, 64, 0, stream()>>>(o.data_ptr<float>(), w.data_ptr<float>(), P.data_ptr<float>(), ldp,
-                                                      (int)g_off, (float)eps, (float)out_scale, out.data_ptr<float>(), ldo,
-                                                      (int)H, (int)dv);
+  const dim3 grid((unsigned)T, (unsigned)((H + 3) / 4));
+  const uintptr_t al = reinterpret_cast<uintptr_t>(o.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr()) |
+                       reinterpret_cast<uintptr_t>(P.data_ptr()) | reinterpret_cast<uintptr_t>(out.data_ptr());
+  const int64_t st = ldp | ldo | g_off | dv;
+  const int W = dv > 128 && st % 4 == 0 && al % 16 == 0 ? 4 : dv > 64 && st % 2 == 0 && al % 8 == 0 ? 2 : 1;
+#define GR_GO(AT, W)                                                                                                       \
+  gated_rmsnorm_k<AT, W><<<grid, 256, 0, stream()>>>(o.data_ptr<float>(), w.data_ptr<float>(), P.data_ptr<float>(), ldp,   \
+                                                     (int)g_off, (float)eps, (float)out_scale, (AT*)out.data_ptr(), ldo,   \
+                                                     (int)H, (int)dv)
+  if (out.scalar_type() == at::kBFloat16) {
+    if (W == 4) GR_GO(uint16_t, 4);
+    else if (W == 2) GR_GO(uint16_t, 2);
+    else GR_GO(uint16_t, 1);
+  } else {
+    if (W == 4) GR_GO(float, 4);
+    else if (W == 2) GR_GO(float, 2);
+    else GR_GO(float, 1);
+  }
+#undef GR_GO
 }
 
 }  // namespace
@@ -1232,9 +1147,7 @@ void bind_mixers(pybind11::module& m) {
   m.def("resid_scale_norm", &resid_scale_norm);
   m.def("gelu_mul", &gelu_mul);
   m.def("gelu_gather_mul", &gelu_gather_mul);
-  m.def("rope_kv_store", &rope_kv_store);
   m.def("attn_gated_chunk", &attn_gated_chunk);
-  m.def("delta_prep", &delta_prep);
   m.def("gla_prep", &gla_prep);
   m.def("linear_recurrence", &linear_recurrence);
   m.def("gated_rmsnorm", &gated_rmsnorm);

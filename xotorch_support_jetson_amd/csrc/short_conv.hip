@@ -4,6 +4,7 @@
 //                      SiLU and a unit length or a weighted RMS norm; the per-request state of last inputs
 //   recurrence_gates   step sizes, low-rank channel decays and low-rank output gates of the channel-decay delta rule
 //   ssd_steps          step sizes and decays of an SSD mixer
+//   delta_gates        write strengths and decays (one per head) of the scalar-decay delta rule
 //
 // P is a fused projection's fp32 output [T, ldp]; "column offset" arguments address its slices.  Everything here is fp32.
 #include "mixer_util.h"
@@ -445,13 +446,14 @@ struct StepArgs {
   const float *dt_bias, *A_log;
   int H, total;
   float *dt, *decay;
+  int b_off;  // >= 0 (delta_gates): dt takes sigmoid(P[:, b_off : +H]) instead of the step size
 };
 
 __device__ __forceinline__ void steps_body(const StepArgs& a, int e) {
   if (e >= a.total) return;
   const int t = e / a.H, h = e - t * a.H;
   const float s = softplusf_(slab1(a.P + (int64_t)t * a.ldp + a.dt_off + h, a.S, a.ss) + a.dt_bias[h]);
-  a.dt[e] = s;
+  a.dt[e] = a.b_off >= 0 ? sigmoidf_(slab1(a.P + (int64_t)t * a.ldp + a.b_off + h, a.S, a.ss)) : s;
   a.decay[e] = expf(-expf(a.A_log[h]) * s);
 }
 
@@ -578,7 +580,8 @@ GateArgs gate_args(const Slabs& p, int64_t b_off, at::Tensor& beta, int64_t a1_o
 inline unsigned gate_jobs(const GateArgs& a) { return (unsigned)(1 + (a.H * a.d + 63) / 64 + (a.ng + 63) / 64); }
 inline size_t gate_lds(const GateArgs& a) { return (size_t)GTOK * std::max(a.ra, a.rg) * sizeof(float); }
 
-StepArgs step_args(const Slabs& p, int64_t dt_off, const at::Tensor& dt_bias, const at::Tensor& A_log, at::Tensor& dt, at::Tensor& decay) {
+StepArgs step_args(const Slabs& p, int64_t dt_off, const at::Tensor& dt_bias, const at::Tensor& A_log, at::Tensor& dt, at::Tensor& decay,
+                   int64_t b_off = -1) {
   const int64_t T = p.T, H = A_log.numel();
   f32c(dt_bias, "dt_bias");
   f32c(A_log, "A_log");
@@ -586,7 +589,9 @@ StepArgs step_args(const Slabs& p, int64_t dt_off, const at::Tensor& dt_bias, co
   f32c(decay, "decay");
   MCHECK(dt_bias.numel() == H && dt.numel() == T * H && decay.numel() == T * H, "ssd_steps: shape mismatch");
   cols_ok(p, dt_off, H, "dt");
+  if (b_off >= 0) cols_ok(p, b_off, H, "write strengths");
   StepArgs a{};
+  a.b_off = (int)b_off;
   a.P = p.p;
   a.ldp = p.ld;
   a.S = p.S;
@@ -635,7 +640,8 @@ void conv_prep(const at::Tensor& P, int64_t x_off, const at::Tensor& conv_w, con
         a.P, a.ldp, a.S, a.ss, a.x_off, a.C, a.taps, a.conv_state, a.state_slots, a.cu);
 }
 
-// A step of single tokens (T == B): conv_prep together with recurrence_gates (beta given) or ssd_steps (dt given).
+// A step of single tokens (T == B): conv_prep together with recurrence_gates (beta and a2 given), delta_gates (beta alone, the
+// decay's columns at dt_off) or ssd_steps (dt given).
 void conv_prep_gates(const at::Tensor& P, int64_t x_off, const at::Tensor& conv_w, const OptT& conv_b, const at::Tensor& units,
                      const OptT& norm_w, at::Tensor& conv_state, const at::Tensor& state_slots, const at::Tensor& cu_q, double eps,
                      at::Tensor& out, int64_t width, int64_t b_off, const OptT& beta, int64_t a1_off, const OptT& a2,
@@ -652,7 +658,12 @@ void conv_prep_gates(const at::Tensor& P, int64_t x_off, const at::Tensor& conv_
   bool bf = false;
   int n_gate = 0, gate_x = 1, n_step = 0;
   size_t lds = 0;
-  if (beta.has_value()) {
+  if (beta.has_value() && !a2.has_value()) {
+    at::Tensor bt = *beta;
+    MCHECK(b_off >= 0, "conv_prep_gates: write strengths");
+    s = step_args(p, dt_off, dt_bias, A_log, bt, decay, b_off);
+    n_step = (s.total + 255) / 256;
+  } else if (beta.has_value()) {
     at::Tensor bt = *beta;
     g = gate_args(p, b_off, bt, a1_off, a2, dt_bias, A_log, decay, g1_off, g2, gate, &bf);
     gate_x = (a.T + GTOK - 1) / GTOK;
@@ -719,6 +730,15 @@ void ssd_steps(const at::Tensor& P, int64_t dt_off, const at::Tensor& dt_bias, c
   ssd_steps_k<<<(unsigned)((a.total + 255) / 256), 256, 0, stream()>>>(a);
 }
 
+void delta_gates(const at::Tensor& P, int64_t b_off, int64_t a_off, const at::Tensor& dt_bias, const at::Tensor& A_log,
+                 at::Tensor& beta, at::Tensor& decay) {
+  const Slabs p = slabs_of(P, "P");
+  if (p.T == 0) return;
+  MCHECK(b_off >= 0, "delta_gates: write strengths");
+  const StepArgs a = step_args(p, a_off, dt_bias, A_log, beta, decay, b_off);
+  ssd_steps_k<<<(unsigned)((a.total + 255) / 256), 256, 0, stream()>>>(a);
+}
+
 }  // namespace
 
 void bind_short_conv(pybind11::module& m) {
@@ -726,6 +746,7 @@ void bind_short_conv(pybind11::module& m) {
   m.def("conv_prep_gates", &conv_prep_gates);
   m.def("recurrence_gates", &recurrence_gates);
   m.def("ssd_steps", &ssd_steps);
+  m.def("delta_gates", &delta_gates);
 }
 
 }  // namespace xot

@@ -45,7 +45,7 @@ PAGE = 64
 # tokens of a step from which the second projections of low-rank gates run as GEMMs (below: inside the gate kernel, in fp32)
 # a parallel block's gate / up rows in a GEMM of their own, which ends in the gated activation: from 1024 tokens (the row count of
 # the four-wave tile) and 2^23 gate / up results on.  Against one GEMM and a pass over its fp32 result: 1024 x (8960 | 11264)
-# x 2048 91 us / 100, 2048 rows 168 / 179, 7000 rows 875 / 1130; 768 rows 82 / 70, 48 rows 35 / 25 and 2048 x (512 | 1024) x
+# x 2048 91 us / 100, 2048 rows 168 / 179, 12807 rows 875 / 1130; 768 rows 82 / 70, 48 rows 35 / 25 and 2048 x (512 | 1024) x
 # 512 26 / 20, where the second launch costs more than the pass
 GELU_EPI_ROWS, GELU_EPI_SIZE = 1024, 1 << 23
 LOW_RANK_GEMM_ROWS = int(os.environ.get("XOT_LOW_RANK_GEMM_ROWS", "256"))
@@ -196,10 +196,16 @@ class StatePool:
                        if sd is not None and sd[4] else None)
       self.aux.append(torch.zeros(slots, sd[0], sd[5], device=device, dtype=torch.float32) if sd is not None and sd[0] and sd[5] else None)
 
-  def clear(self, slot: int) -> None:
+  def clear(self, slots) -> None:
+    """Clear some slots: one fill per tensor and run of neighbouring slots (48 requests admitted together: 12 fills of 4 layers'
+    states, not 288 of 2 us each)."""
+    order = sorted(slots)
+    starts = [i for i, s in enumerate(order) if i == 0 or s != order[i - 1] + 1]
+    runs = [(order[a], order[b - 1] + 1) for a, b in zip(starts, starts[1:] + [len(order)])]
     for t in self.S + self.conv + self.aux:
       if t is not None:
-        t[slot].zero_()
+        for a, b in runs:
+          t[a:b].zero_()
 
   def nbytes(self) -> int:
     return sum(t.numel() * 4 for t in self.S + self.conv + self.aux if t is not None)
@@ -449,11 +455,12 @@ class ShardModel:
     return linear(x, w, out_dtype=torch.float32)
 
   @staticmethod
-  def _proj_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """The same for a consumer that sums unreduced split-K slabs itself (and runs before the next GEMM): [T, n] or [S, T, n]."""
+  def _proj_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0) -> torch.Tensor:
+    """The same for a consumer that sums unreduced split-K slabs itself (and runs before the next GEMM of its scratch slot):
+    [T, n] or [S, T, n]."""
     if x.dtype == torch.float32 or not x.is_cuda:
       return ShardModel._proj(x, w)
-    return linear_slabs(x, w)
+    return linear_slabs(x, w, slot)
 
   @staticmethod
   def _fused_act(x: torch.Tensor, w: torch.Tensor, epi: str, limit: float = 0.0) -> Optional[torch.Tensor]:
@@ -504,7 +511,7 @@ class ShardModel:
     tab = self.rope_tabs.get((a.rot_dims, a.rot_base))
     K.rope_kv_store(P, lw.cols["aq"][0], lw.cols["ak"][0], -1 if a.values_are_keys else lw.cols["av"][0], a.heads,
                     a.kv_heads, a.dim, a.rot_dims if tab is not None else 0,
-                    inp.positions, tab if tab is not None else torch.zeros(1, 0, device=P.device), inp.slots, q,
+                    inp.positions, tab if tab is not None else lw.attn_pb.new_empty(1, 0), inp.slots, q,
                     self.kv.k[j], self.kv.v[j])
     off, n = lw.mix_cols["attn"]
     K.attn_gated_chunk(q, self.kv.k[j], self.kv.v[j], inp.block_tables, inp.cu_q, inp.ctx_lens, lw.attn_pb, a.scale,
@@ -518,12 +525,10 @@ class ShardModel:
     H, G, d, dv = r.heads, r.kv_heads, r.dim, r.vdim
     o = torch.empty(T, H * dv, dtype=torch.float32, device=dev)
     if r.rule == "delta":
-      C = 2 * G * d + H * dv
-      qkv = torch.empty(T, C, dtype=torch.float32, device=dev)
       beta = torch.empty(T, H, dtype=torch.float32, device=dev)
       decay = torch.empty(T, H, dtype=torch.float32, device=dev)
-      K.delta_prep(P, lw.cols["rq"][0], lw.cols["rb"][0], lw.cols["ra"][0], lw.conv_w, st.conv[j], inp.state_slots,
-                   inp.cu_q, lw.A_log, lw.dt_bias, H, G, d, dv, qkv, beta, decay)
+      qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
+                       delta=(lw.cols["rb"][0], lw.cols["ra"][0], lw.dt_bias, lw.A_log, beta, decay))
       K.linear_recurrence(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], decay, beta, 1.0, st.S[j],
                           inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
     else:
@@ -584,10 +589,10 @@ class ShardModel:
         self._gated_attn(P, lw, j, inp, mix)
       if s.rec is not None:
         self._recurrence(P, lw, j, inp, mix)
-      y1 = self._proj(mix, lw.out_w)
-      y2 = None
-      if s.ff:
-        y2 = self._proj(act, lw.down_w)
+      # (the sum below reduces split-K slabs of both: the second branch's lie in a scratch of their own, and its GEMM comes
+      # first, so that choosing a kernel for the other does not write over them)
+      y2 = self._proj_slabs(act, lw.down_w, slot=1) if s.ff else None
+      y1 = self._proj_slabs(mix, lw.out_w)
       nxt = w.layers[self.layer_ids[j + 1]].norm_g if j + 1 < n else None
       K.resid_scale_norm(h, y1, lw.ls1, y2, lw.ls2 if y2 is not None else None, gain=nxt, eps=c.rms_norm_eps,
                          out=hn if nxt is not None else None)

@@ -796,6 +796,7 @@ def mixed_layer_names(spec, p: str) -> Dict[str, list]:
 
 def build_mixed_layer(spec, get, p: str, D: int, device, dtype) -> MixedLayerWeights:
   """Assemble one layer from `get(name) -> fp32 CPU tensor` (a checkpoint reader or a random generator)."""
+  from ..ops.reference import conv_units, delta_units
   names = mixed_layer_names(spec, p)
   blocks = [(n, get(t)) for n, t in names["in"]]
   # bf16: the gate and up rows come last and interleave, so that a prompt's GEMM over them ends in the gated activation
@@ -807,8 +808,8 @@ def build_mixed_layer(spec, get, p: str, D: int, device, dtype) -> MixedLayerWei
     cols[n] = (off, w.shape[0])
     off += w.shape[0]
   Dp = _up(D, 128)
-  # whole 256-row tiles where that costs at most 5 % of zero rows: the four-wave GEMM takes no others (7000 x 20032 x 2048,
-  # fp32: 942 us on the ping-pong tile and a pass of 190 for the activation; 7000 x 8960 380 and 7000 x 11264 495 on the
+  # whole 256-row tiles where that costs at most 5 % of zero rows: the four-wave GEMM takes no others (12807 x 20032 x 2048,
+  # fp32: 942 us on the ping-pong tile and a pass of 190 for the activation; 12807 x 8960 380 and 12807 x 11264 495 on the
   # four-wave one, activation included)
   Np = _up(off, 256) if dtype == torch.bfloat16 and 20 * _up(off, 256) <= 21 * off else _up(off, 64)
   Fp = _up(spec.ff, 128)
@@ -839,6 +840,9 @@ def build_mixed_layer(spec, get, p: str, D: int, device, dtype) -> MixedLayerWei
   if "conv" in names:
     lw.conv_w = dev(torch.cat([get(n) for n in names["conv"]], 0))
     lw.A_log, lw.dt_bias = dev(get(names["A_log"])), dev(get(names["dt_bias"]))
+    r = spec.rec
+    u, lw.conv_width = conv_units(delta_units(r.heads, r.kv_heads, r.dim, r.vdim), lw.conv_w.shape[0])
+    lw.conv_units = u.to(device)
   if "a2" in names:
     lw.a2_w, lw.a2_b = dev(get(names["a2"])), dev(get(names["a2_b"]))
   lw.rec_norm = dev(get(names["rec_norm"]))

@@ -462,8 +462,8 @@ def rope_kv_store(P, q_off: int, k_off: int, v_off: int, H: int, G: int, d: int,
   """Rotate-half RoPE on the first R dims of every q / k head (pairs (i, i + R/2)); q -> q_out [T, H, d], the
   rotated key -> k_cache [pages, G, 64, d], the value (v_off < 0: the key before rotation) -> v_cache [pages, G, d, 64],
   both at `slots`."""
-  _mix("rope_kv_store", _gpu(P))(P, int(q_off), int(k_off), int(v_off), int(H), int(G), int(d), int(R), pos, cos_sin,
-                                 slots, q_out, k_cache, v_cache)
+  qk_norm_rope_store(P, None, q_off, k_off, k_off if v_off < 0 else v_off, H, G, d, d, R, pos, cos_sin, slots, 0.0, False, q_out,
+                     k_cache, v_cache)
 
 
 def attn_gated_chunk(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, scale: float, chunk: int, out_scale: float,
@@ -479,9 +479,12 @@ def attn_gated_chunk(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, scal
 
 def delta_prep(P, x_off: int, b_off: int, a_off: int, conv_w, conv_state, state_slots, cu_q, A_log, dt_bias, H: int,
                G: int, d: int, dv: int, qkv, beta, decay) -> None:
-  """Delta-rule inputs of a step and the convolution state's update (see csrc/mixers.hip delta_prep)."""
-  _mix("delta_prep", _gpu(P))(P, int(x_off), int(b_off), int(a_off), conv_w, conv_state, state_slots, cu_q, A_log, dt_bias,
-                              int(H), int(G), int(d), int(dv), qkv, beta, decay)
+  """Delta-rule inputs of a step and the convolution state's update: channels [q: G d | k: G d | v: H dv] at P[:, x_off ...];
+  q = unit(silu(conv q)) d^-1/2, k = unit(silu(conv k)), v = silu(conv v) -> qkv [T, C]; beta and decay: delta_gates.  (A model
+  step calls conv_prep with the units that its weights hold on the device.)"""
+  units, width = ref.conv_units(ref.delta_units(H, G, d, dv), conv_w.shape[0])
+  conv_prep(P, x_off, conv_w, None, units.to(P.device), None, conv_state, state_slots, cu_q, 0.0, qkv.view(P.shape[-2], -1),
+            width=width, delta=(b_off, a_off, dt_bias, A_log, beta, decay))
 
 
 def gla_prep(P, a1_off: int, a2, a2_b, tau: float, decay) -> None:
@@ -493,15 +496,19 @@ conv_units = ref.conv_units
 
 
 def conv_prep(P, x_off: int, conv_w, conv_b, units, norm_w, conv_state, state_slots, cu_q, eps: float, out, max_qlen: int = 0,
-              width: int = 256, gates: tuple | None = None, steps: tuple | None = None) -> None:
+              width: int = 256, gates: tuple | None = None, steps: tuple | None = None, delta: tuple | None = None) -> None:
   """Causal convolutions over time of the channels P[:, x_off : +C] (conv_w [C, taps], last column the current token; conv_b
   [C] or None) -> out [T, C] fp32, then per unit (conv_units) SiLU and a unit length or a weighted RMS norm (norm_w).  The
   inputs before the step come from conv_state [slots, taps - 1, C], which takes the step's last ones.  max_qlen 1: every
   sequence has one new token (the state is updated in the same launch).  width: the most channels of a unit.  P may be [T, n]
-  or unreduced split-K slabs [S, T, n] (also below).  gates / steps: the arguments behind P of recurrence_gates or ssd_steps,
-  which read the same projection: done as well, for single tokens in the same launch."""
-  if _gpu(P) and max_qlen == 1 and P.shape[-2] == state_slots.numel() and (gates is not None) != (steps is not None):
-    if gates is not None:
+  or unreduced split-K slabs [S, T, n] (also below).  gates / steps / delta: the arguments behind P of recurrence_gates,
+  ssd_steps or delta_gates, which read the same projection: done as well, for single tokens in the same launch."""
+  if _gpu(P) and max_qlen == 1 and P.shape[-2] == state_slots.numel() and sum(g is not None for g in (gates, steps, delta)) == 1:
+    if delta is not None:
+      b_off, dt_off, dt_bias, A_log, beta, decay = delta
+      a1_off = g1_off = 0
+      a2 = g2 = gate = dt = None
+    elif gates is not None:
       b_off, beta, a1_off, a2, dt_bias, A_log, decay, g1_off, g2, gate = gates
       dt_off, dt = 0, None
     else:
@@ -517,6 +524,13 @@ def conv_prep(P, x_off: int, conv_w, conv_b, units, norm_w, conv_state, state_sl
     recurrence_gates(P, *gates)
   if steps is not None:
     ssd_steps(P, *steps)
+  if delta is not None:
+    delta_gates(P, *delta)
+
+
+def delta_gates(P, b_off: int, a_off: int, dt_bias, A_log, beta, decay) -> None:
+  """beta [T, H] = sigmoid(P[:, b_off : +H]), decay [T, H] = exp(-exp(A_log) softplus(P[:, a_off : +H] + dt_bias))."""
+  _mix("delta_gates", _gpu(P))(P, int(b_off), int(a_off), dt_bias, A_log, beta, decay)
 
 
 def recurrence_gates(P, b_off: int, beta, a1_off: int, a2, dt_bias, A_log, decay, g1_off: int, g2, gate, za=None) -> None:

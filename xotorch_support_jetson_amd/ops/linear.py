@@ -139,7 +139,8 @@ class _Scratch:
 
   def splitk(self, device, n: int, slot: int = 0) -> torch.Tensor:
     """slot 1 holds the slabs of a residual projection whose reduce is deferred into the next GEMM (PendingNorm),
-    which writes its own slabs to slot 0 while it still reads slot 1."""
+    which writes its own slabs to slot 0 while it still reads slot 1, or those of the second of two projections whose
+    slabs one kernel sums."""
     key = (device.index or 0, slot)
     t = self.ws.get(key)
     if t is None or t.numel() < n:
@@ -702,9 +703,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, r
   return out
 
 
-def linear_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def linear_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0) -> torch.Tensor:
   """fp32 x @ w.T for a consumer that sums split-K slabs itself: [M, N], or [S, M, N] when the projection runs split over K
-  (a view of the shared scratch: valid until the next split-K GEMM)."""
+  (a view of the shared scratch: valid until the next split-K GEMM of its slot, where choosing a configuration counts as one
+  of slot 0)."""
   if x.is_cuda and layout_of(w) == "stream":
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
@@ -712,7 +714,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y")
     S = cfg[2]
     if S > 1:
-      ws = scratch.splitk(x.device, S * M * N)
+      ws = scratch.splitk(x.device, S * M * N, slot)
       y = torch.empty(M, N, dtype=torch.float32, device=x.device)  # shape carrier only: the slabs are not reduced
       if cfg[0] == "stream":
         require().gemm_stream(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, True, False)

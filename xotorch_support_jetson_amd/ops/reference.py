@@ -256,27 +256,6 @@ def gelu_mul(P, gate_off, up_off, Fd, out):
   out[:, :Fd] = (0.5 * z * (1 + torch.tanh(0.7978845608028654 * (z + 0.044715 * z ** 3))) * u).to(out.dtype)
 
 
-def rope_kv_store(P, q_off, k_off, v_off, H, G, d, R, pos, cos_sin, slots, q_out, k_cache, v_cache):
-  T = P.shape[0]
-  q = P[:, q_off:q_off + H * d].float().reshape(T, H, d)
-  k = P[:, k_off:k_off + G * d].float().reshape(T, G, d)
-  v = k if v_off < 0 else P[:, v_off:v_off + G * d].float().reshape(T, G, d)
-  half = R // 2
-
-  def rot(x):
-    if R == 0:
-      return x
-    cs = cos_sin[pos.long()]
-    c, s = cs[:, None, :half], cs[:, None, half:]
-    a, b = x[..., :half], x[..., half:R]
-    return torch.cat([a * c - b * s, b * c + a * s, x[..., R:]], -1)
-  q_out.copy_(rot(q).to(q_out.dtype))
-  ok = slots >= 0
-  s = slots[ok].long()
-  k_cache[s // PAGE, :, s % PAGE] = rot(k)[ok].to(k_cache.dtype)
-  v_cache[s // PAGE, :, :, s % PAGE] = v[ok].to(v_cache.dtype)
-
-
 def attn_gated_chunk(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, scale, chunk, out_scale, out, max_qlen=0):
   T, H, d = q.shape
   G = k_cache.shape[1]
@@ -297,23 +276,10 @@ def attn_gated_chunk(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, scal
     out[t0:t1] = o.reshape(t1 - t0, H * d).to(out.dtype)
 
 
-def delta_prep(P, x_off, b_off, a_off, conv_w, conv_state, state_slots, cu_q, A_log, dt_bias, H, G, d, dv, qkv, beta, decay):
-  C = 2 * G * d + H * dv
-  taps = conv_w.shape[1]
-  for b in range(state_slots.numel()):
-    t0, t1, slot = int(cu_q[b]), int(cu_q[b + 1]), int(state_slots[b])
-    if slot < 0 or t1 == t0:
-      continue
-    x = torch.cat([conv_state[slot], P[t0:t1, x_off:x_off + C].float()], 0)  # [taps - 1 + n, C]
-    y = sum(conv_w[:, j].float() * x[j:j + t1 - t0] for j in range(taps))
-    y = F.silu(y)
-    qk = y[:, :2 * G * d].reshape(t1 - t0, 2 * G, d)
-    qk = qk / torch.sqrt(qk.pow(2).sum(-1, keepdim=True) + 1e-6)
-    qk[:, :G] *= d ** -0.5
-    qkv[t0:t1] = torch.cat([qk.reshape(t1 - t0, -1), y[:, 2 * G * d:]], 1)
-    conv_state[slot] = x[x.shape[0] - (taps - 1):]
-    beta[t0:t1] = torch.sigmoid(P[t0:t1, b_off:b_off + H].float())
-    decay[t0:t1] = torch.exp(-torch.exp(A_log.float()) * F.softplus(P[t0:t1, a_off:a_off + H].float() + dt_bias.float()))
+def delta_gates(P, b_off, a_off, dt_bias, A_log, beta, decay):
+  H = A_log.numel()
+  beta.copy_(torch.sigmoid(P[:, b_off:b_off + H].float()))
+  decay.copy_(torch.exp(-torch.exp(A_log.float()) * F.softplus(P[:, a_off:a_off + H].float() + dt_bias.float())))
 
 
 def gla_prep(P, a1_off, a2, a2_b, tau, decay):
@@ -346,6 +312,11 @@ def conv_units(parts, C: int):
   if c0 != C:
     raise ValueError(f"the units cover {c0} of {C} channels")
   return torch.tensor(rows, dtype=torch.int32), width
+
+
+def delta_units(H, G, d, dv):
+  """conv_units of the scalar-decay delta rule's channels [q: G heads of d | k: G heads of d | v: H heads of dv]."""
+  return [(d, CONV_SILU | CONV_UNIT_SCALED)] * G + [(d, CONV_SILU | CONV_UNIT)] * G + [(H * dv, CONV_SILU)]
 
 
 def conv_prep(P, x_off, conv_w, conv_b, units, norm_w, conv_state, state_slots, cu_q, eps, out, max_qlen=0, width=CONV_MAX):

@@ -211,15 +211,22 @@ class ShardRunner:
       return False
     return self.bm.can_append(rid, n_new) and self.num_tokens(rid) + n_new <= self.max_ctx
 
-  def _state_slot(self, rid: str) -> int:
-    """The request's state slot; a request seen for the first time gets a cleared one."""
-    if self.sm.has(rid):
-      return self.sm.slot(rid)
-    if self.bm.has(rid) and self.bm.num_tokens(rid) > 0:
-      raise RuntimeError(f"request {rid} holds cached tokens but no recurrent state")
-    s = self.sm.acquire(rid)
-    self.state.clear(s)
-    return s
+  def _state_slots(self, rids: Sequence[str]) -> List[int]:
+    """The requests' state slots; requests seen for the first time get cleared ones."""
+    out, new = [], []
+    try:
+      for rid in rids:
+        if self.sm.has(rid):
+          out.append(self.sm.slot(rid))
+          continue
+        if self.bm.has(rid) and self.bm.num_tokens(rid) > 0:
+          raise RuntimeError(f"request {rid} holds cached tokens but no recurrent state")
+        out.append(self.sm.acquire(rid))
+        new.append(out[-1])
+    finally:  # (also where a later request is refused: those before it keep their slots)
+      if new:
+        self.state.clear(new)
+    return out
 
   def truncate(self, rid: str, n: int) -> None:
     if self.sm is not None and n != self.num_tokens(rid):
@@ -234,7 +241,7 @@ class ShardRunner:
     pos: List[int] = []
     slots: List[int] = []
     cu = [0]
-    sslots = [self._state_slot(rid) for rid in rids] if self.sm is not None else None
+    sslots = self._state_slots(rids) if self.sm is not None else None
     for rid, n in zip(rids, qlens):
       start = self.num_tokens(rid)
       if start + n > self.max_ctx:
@@ -308,7 +315,7 @@ class ShardRunner:
     self._reuse_staging()
     pos, slots = [], []
     most = 0
-    sslots = [self._state_slot(rid) for rid in rids] if self.sm is not None else None
+    sslots = self._state_slots(rids) if self.sm is not None else None
     for rid in rids:
       start = self.num_tokens(rid)
       if start + 1 > self.max_ctx:
