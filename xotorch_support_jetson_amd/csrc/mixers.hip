@@ -1,6 +1,7 @@
 // Token mixers beside softmax attention, and the fp32-residual layer plumbing around them (gfx950).
 //
 //   resid_scale_norm   x += s1 * y1 (+ s2 * y2) on the fp32 residual stream, then RMS norm with one scalar gain
+//   embed_rows         rows of an fp32 embedding table, ids clamped to it
 //   gelu_mul           gelu_tanh(gate) * up out of a fused projection's columns
 //   gelu_gather_mul    gelu_tanh(gate) * the token's slice of a table (per-layer side inputs)
 //   attn_gated_chunk   chunk-local attention with sigmoid(score + bias[head]) weights, no normalisation: an MFMA
@@ -88,6 +89,21 @@ __global__ __launch_bounds__(256) void resid_scale_norm_reg_k(float* __restrict_
     const int i = 4 * (threadIdx.x + 256 * j);
     if (i < D) st4(out + r * ldo + i, v[j] * k);
   }
+}
+
+// ------------------------------------------------------------------ embedding rows
+// out [T, D] = table[ids] (ids clamped to the table), ids_out [T] (or null) the clamped ids.  A step of single tokens is bound by
+// launches: one, where clamp, conversions and gather were four of 2 to 5 us.
+template <typename IT, int W>
+__global__ __launch_bounds__(256) void embed_rows_k(const IT* __restrict__ ids, const float* __restrict__ table, int D, int64_t V,
+                                                    float* __restrict__ out, int* __restrict__ ids_out) {
+  const int64_t t = blockIdx.x;
+  const int64_t id = min(max((int64_t)ids[t], (int64_t)0), V - 1);
+  if (ids_out && threadIdx.x == 0) ids_out[t] = (int)id;
+  typedef float vec __attribute__((ext_vector_type(W)));
+  const vec* src = reinterpret_cast<const vec*>(table + id * D);
+  vec* dst = reinterpret_cast<vec*>(out + t * D);
+  for (int i = threadIdx.x; i < D / W; i += 256) dst[i] = src[i];
 }
 
 // ------------------------------------------------------------------ gelu_tanh(gate) * up
@@ -835,6 +851,34 @@ void resid_scale_norm(at::Tensor& x, const c10::optional<at::Tensor>& y1, const 
 #undef RSN_GO
 }
 
+void embed_rows(const at::Tensor& ids, const at::Tensor& table, at::Tensor& out, const c10::optional<at::Tensor>& ids_out) {
+  f32c(table, "table");
+  f32c(out, "out");
+  const bool wide = ids.scalar_type() == at::kLong;
+  MCHECK(ids.is_cuda() && ids.is_contiguous() && (wide || ids.scalar_type() == at::kInt), "ids must be contiguous int32 / int64");
+  const int64_t T = ids.numel();
+  MCHECK(table.dim() == 2 && table.size(0) >= 1 && table.size(0) < (int64_t(1) << 31) && out.numel() == T * table.size(1),
+         "embed_rows: shape mismatch");
+  int* io = nullptr;
+  if (ids_out.has_value()) {
+    i32c(*ids_out, "ids_out");
+    MCHECK(ids_out->numel() == T, "ids_out must hold one id per token");
+    io = ids_out->data_ptr<int>();
+  }
+  const int64_t D = table.size(1);
+  if (T * D == 0) return;
+  const bool vec = D % 4 == 0 && ((reinterpret_cast<uintptr_t>(table.data_ptr()) | reinterpret_cast<uintptr_t>(out.data_ptr())) & 15) == 0;
+#define EMB_GO(IT, W)                                                                                                   \
+  embed_rows_k<IT, W><<<(unsigned)T, 256, 0, stream()>>>((const IT*)ids.data_ptr(), table.data_ptr<float>(), (int)D,    \
+                                                         table.size(0), out.data_ptr<float>(), io)
+  if (wide) {
+    if (vec) EMB_GO(int64_t, 4); else EMB_GO(int64_t, 1);
+  } else {
+    if (vec) EMB_GO(int, 4); else EMB_GO(int, 1);
+  }
+#undef EMB_GO
+}
+
 void gelu_mul(const at::Tensor& P, int64_t gate_off, int64_t up_off, int64_t F, at::Tensor& out) {
   const int ldp = ld_of(P, "P");
   const int64_t T = P.size(0);
@@ -1145,6 +1189,7 @@ void gated_rmsnorm(const at::Tensor& o, const at::Tensor& w, const at::Tensor& P
 
 void bind_mixers(pybind11::module& m) {
   m.def("resid_scale_norm", &resid_scale_norm);
+  m.def("embed_rows", &embed_rows);
   m.def("gelu_mul", &gelu_mul);
   m.def("gelu_gather_mul", &gelu_gather_mul);
   m.def("attn_gated_chunk", &attn_gated_chunk);

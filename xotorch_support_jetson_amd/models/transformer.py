@@ -84,6 +84,7 @@ class StepInputs:
   image_embeds: Optional[torch.Tensor] = None  # LLaVA: [n image-token rows, D], in token order (first shard)
   # models with recurrent layers: [B] int32 state slot of each sequence (-1: padding row, nothing is read or written)
   state_slots: Optional[torch.Tensor] = None
+  all_rows: bool = False  # last_idx is 0 .. T - 1 (a decode step): the rows need no gather
 
   @property
   def num_tokens(self) -> int:
@@ -477,6 +478,15 @@ class ShardModel:
     K.glu_act(torch.cat([t[:, :, 0].reshape(-1, n), t[:, :, 1].reshape(-1, n)], 1), 0, n, n, clamped, limit, out)
     return out
 
+  @staticmethod
+  def _last_rows(h: torch.Tensor, inp: StepInputs, hn: torch.Tensor):
+    """The stream's rows the logits are asked of and a row buffer for their final norm (K padding zero): the step's own
+    where these are all of them."""
+    if inp.all_rows:
+      return h, hn
+    hl = h.index_select(0, inp.last_idx)
+    return hl, torch.zeros(hl.shape[0], hn.shape[1], dtype=hn.dtype, device=h.device)
+
   def _in_and_act(self, hn: torch.Tensor, lw, rows):
     """A parallel block's input projections P and its gated activation (None without a feed-forward)."""
     ff = lw.spec.ff
@@ -553,9 +563,7 @@ class ShardModel:
       raise RuntimeError("a model with recurrent layers needs a state pool and the step's state slots")
     ids = None  # (token ids, for layers with side inputs: shards after the first find them in the hidden state's last column)
     if self.shard.is_first_layer():
-      ids = x.view(-1).long().clamp(0, w.embed.shape[0] - 1)
-      h = w.embed.index_select(0, ids)
-      ids = ids.to(torch.int32)
+      h, ids = K.embed_rows(x.view(-1), w.embed, want_ids=bool(c.side_dim))
     else:
       if c.side_dim:
         ids = x[:, c.hidden_size].to(torch.int32)
@@ -598,11 +606,10 @@ class ShardModel:
                          out=hn if nxt is not None else None)
     if not last:
       return h
-    hl = h.index_select(0, inp.last_idx)
-    xn = torch.zeros(hl.shape[0], hn.shape[1], dtype=adt, device=h.device)
+    hl, xn = self._last_rows(h, inp, hn)
     K.resid_scale_norm(hl, gain=w.norm, eps=c.rms_norm_eps, out=xn)
     logits = self._proj(xn, w.lm_head)[:, :c.vocab_size]
-    return logits * c.logit_scale
+    return logits * c.logit_scale if c.logit_scale != 1.0 else logits
 
   # ------------------------------------------------------------------ post-norm blocks (window attention / SSD, MoE)
   def _window_attn(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor) -> None:
@@ -849,8 +856,7 @@ class ShardModel:
       K.gated_postnorm(h, y, P, lw.ff_cols["gate"][0], lw.gate2_b, c.postln_alpha, lw.norm2, c.rms_norm_eps, hn)
     if not self.shard.is_last_layer():
       return h
-    hl = h.index_select(0, inp.last_idx)
-    xn = torch.zeros(hl.shape[0], Dp, dtype=adt, device=h.device)
+    hl, xn = self._last_rows(h, inp, hn)
     K.gated_postnorm(hl, None, None, 0, None, 1.0, w.norm, c.rms_norm_eps, xn)
     return self._proj(xn, w.lm_head)[:, :c.vocab_size]
 
@@ -1076,8 +1082,7 @@ class ShardModel:
       fresh = nl is None
     if not self.shard.is_last_layer():
       return torch.cat([h, ids.to(torch.float32)[:, None]], 1) if c.side_dim else h
-    hl = h.index_select(0, inp.last_idx)
-    xn = torch.zeros(hl.shape[0], Dp, dtype=adt, device=h.device)
+    hl, xn = self._last_rows(h, inp, hn)
     K.sandwich_add_norm(hl, None, None, w.norm, eps, xn, bn=w.norm_b, layer=ln)
     logits = self._proj(xn, w.lm_head)[:, :c.vocab_size]
     if c.logit_softcap > 0:

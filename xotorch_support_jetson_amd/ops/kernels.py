@@ -451,6 +451,17 @@ def resid_scale_norm(x, y1=None, s1=None, y2=None, s2=None, gain=None, eps: floa
   _mix("resid_scale_norm", _gpu(x))(x, y1, s1, y2, s2, gain, float(eps), out)
 
 
+def embed_rows(ids, table, want_ids: bool = False):
+  """(rows of the fp32 table [V, D] at ids [T] clamped to it, the clamped ids as int32 or None)."""
+  if not (_gpu(table) and table.dtype == torch.float32 and ids.dtype in (torch.int32, torch.int64)):
+    ids = ids.long().clamp(0, table.shape[0] - 1)
+    return table.index_select(0, ids), ids.to(torch.int32) if want_ids else None
+  h = torch.empty(ids.numel(), table.shape[1], dtype=table.dtype, device=table.device)
+  ids32 = torch.empty(ids.numel(), dtype=torch.int32, device=table.device) if want_ids else None
+  require().embed_rows(ids.contiguous(), table, h, ids32)
+  return h, ids32
+
+
 def gelu_mul(P, gate_off: int, up_off: int, F: int, out) -> None:
   """out[:, :F] = gelu_tanh(P[:, gate_off : +F]) * P[:, up_off : +F]  (out rows may be wider: K padding).  up_off < 0: gate and
   up columns alternate in tiles of 16 from gate_off on."""

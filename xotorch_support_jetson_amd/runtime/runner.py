@@ -81,6 +81,29 @@ def _bucket(n: int) -> int:
   return n
 
 
+def _pack_layout(Bp: int, w: int):
+  """Byte offsets of a decode step's inputs in one buffer: ({name: (offset, dtype, shape)}, bytes)."""
+  out, at = {}, 0
+  for name, dt, shape in (("slots", torch.int64, (Bp,)), ("pos", torch.int32, (Bp,)), ("ctx", torch.int32, (Bp,)),
+                          ("sslots", torch.int32, (Bp,)), ("tables", torch.int32, (Bp, w))):
+    out[name] = (at, dt, shape)
+    n = 8 if dt == torch.int64 else 4
+    for s in shape:
+      n *= s
+    at = -(-(at + n) // 16) * 16
+  return out, at
+
+
+def _unpack(buf: torch.Tensor, Bp: int, w: int) -> Dict[str, torch.Tensor]:
+  out = {}
+  for name, (at, dt, shape) in _pack_layout(Bp, w)[0].items():
+    n = 8 if dt == torch.int64 else 4
+    for s in shape:
+      n *= s
+    out[name] = buf[at:at + n].view(dt).view(shape)
+  return out
+
+
 class ShardRunner:
   def __init__(self, config: ModelConfig, shard: Shard, device: torch.device | str = "cpu",
                weights: Optional[ShardWeights] = None, num_pages: Optional[int] = None, max_batch: int = 128,
@@ -154,14 +177,13 @@ class ShardRunner:
     for _ in range(2):
       st = {"tables": torch.zeros(max_batch, self.width, dtype=torch.int32),
             "ctx": torch.zeros(max_batch, dtype=torch.int32),
-            "pos": torch.zeros(bmax, dtype=torch.int32),  # decode-step positions / slots (graph inputs)
-            "slots": torch.zeros(bmax, dtype=torch.int64),
-            "sslots": torch.zeros(bmax, dtype=torch.int32)}  # state slots (recurrent layers)
+            # a decode step's inputs as its graph holds them, one copy for all (each copy costs the step 3 to 5 us)
+            "pack": torch.zeros(_pack_layout(bmax, self.width)[1], dtype=torch.uint8)}
       if self.device.type == "cuda":
         # pinned: an async copy out of pageable memory may wait for the stream to drain, i.e. for the step
         # already running, which would forbid queueing the next decode step behind it
         st = {k: v.pin_memory() for k, v in st.items()}
-      st["cls"] = {}  # narrower block tables per width class
+      st["views"] = {}  # of the pack, per captured (batch bucket, table width)
       st["event"] = None  # completion of the last async H2D copy out of this set
       self._sets.append(st)
     self._set_idx = 1
@@ -170,9 +192,7 @@ class ShardRunner:
   def _use_set(self, i: int) -> None:
     st = self._sets[i]
     self._set_idx = i
-    self._tables_host, self._ctx_host, self._pos_host, self._slots_host = st["tables"], st["ctx"], st["pos"], st["slots"]
-    self._sslots_host = st["sslots"]
-    self._tables_cls = st["cls"]
+    self._tables_host, self._ctx_host, self._pack_host = st["tables"], st["ctx"], st["pack"]
 
   def _reuse_staging(self) -> None:
     """Switch to the other staging set; wait only if ITS last async copy (two steps back) is still running."""
@@ -266,6 +286,7 @@ class ShardRunner:
       max_qlen=max(qlens),
       decode=all(q == 1 for q in qlens),
       state_slots=None if sslots is None else torch.tensor(sslots, dtype=torch.int32).to(dev, non_blocking=nb),
+      all_rows=logit_rows is None and all(q == 1 for q in qlens),
     )
     self._mark_staged()
     return inp
@@ -297,16 +318,14 @@ class ShardRunner:
       return image_features(self.config, self.weights.vision, pixels.to(self.device))
 
   # ------------------------------------------------------------------ graphs
-  def _tables_staging(self, w: int) -> torch.Tensor:
-    if w == self.width:
-      return self._tables_host
-    t = self._tables_cls.get(w)
-    if t is None:
-      t = torch.zeros(self.max_batch, w, dtype=torch.int32)
-      if self.device.type == "cuda":
-        t = t.pin_memory()
-      self._tables_cls[w] = t
-    return t
+  def _pack_views(self, Bp: int, w: int) -> dict:
+    """numpy views of the current staging set's pack as the graph (Bp, w) lays it out, and its length in bytes."""
+    views = self._sets[self._set_idx]["views"]
+    v = views.get((Bp, w))
+    if v is None:
+      v = views[(Bp, w)] = {k: t.numpy() for k, t in _unpack(self._pack_host, Bp, w).items()}
+      v["bytes"] = _pack_layout(Bp, w)[1]
+    return v
 
   def _decode_graph(self, rids: Sequence[str], x: torch.Tensor) -> torch.Tensor:
     B = len(rids)
@@ -328,23 +347,17 @@ class ShardRunner:
     g = self._graphs.get((Bp, w))
     if g is None:
       g = self._capture(Bp, w)
-    tables = self._tables_staging(w)
-    self.bm.fill_batch(list(rids), tables[:B].numpy(), self._ctx_host[:B].numpy())
-    pad = Bp - B
-    self._pos_host[:Bp] = torch.tensor(pos + [0] * pad, dtype=torch.int32)
-    self._slots_host[:Bp] = torch.tensor(slots + [-1] * pad, dtype=torch.int64)
-    g["pos"].copy_(self._pos_host[:Bp], non_blocking=True)
-    g["slots"].copy_(self._slots_host[:Bp], non_blocking=True)
-    if sslots is not None:
-      self._sslots_host[:Bp] = torch.tensor(sslots + [-1] * pad, dtype=torch.int32)
-      g["sslots"].copy_(self._sslots_host[:Bp], non_blocking=True)
-    self._ctx_host[B:Bp] = 0
-    g["tables"].copy_(tables[:Bp], non_blocking=True)
-    g["ctx"].copy_(self._ctx_host[:Bp], non_blocking=True)
+    v = self._pack_views(Bp, w)
+    self.bm.fill_batch(list(rids), v["tables"][:B], v["ctx"][:B])
+    v["pos"][:B], v["slots"][:B] = pos, slots
+    v["sslots"][:B] = -1 if sslots is None else sslots
+    # (padding rows: no context, no KV or state slot)
+    v["tables"][B:], v["ctx"][B:], v["pos"][B:], v["slots"][B:], v["sslots"][B:] = 0, 0, 0, -1, -1
+    g["pack"].copy_(self._pack_host[:v["bytes"]], non_blocking=True)
     self._mark_staged()
     if self.shard.is_first_layer():
-      g["x"][:B].copy_(x.view(-1).to(torch.int32))
-      if pad:
+      g["x"][:B].copy_(x.view(-1))
+      if Bp > B:
         g["x"][B:].zero_()
     else:
       g["x"][:B].copy_(x)
@@ -381,11 +394,9 @@ class ShardRunner:
     dev = self.device
     c = self.config
     w = w or self.width
+    pack = torch.zeros(_pack_layout(Bp, w)[1], dtype=torch.uint8, device=dev)
     g = {
-      "pos": torch.zeros(Bp, dtype=torch.int32, device=dev),
-      "slots": torch.full((Bp,), -1, dtype=torch.int64, device=dev),
-      "tables": torch.zeros(Bp, w, dtype=torch.int32, device=dev),
-      "ctx": torch.zeros(Bp, dtype=torch.int32, device=dev),
+      "pack": pack, **_unpack(pack, Bp, w),
       "cu": torch.arange(Bp + 1, dtype=torch.int32, device=dev),
       "last": torch.arange(Bp, dtype=torch.int64, device=dev),
     }
@@ -393,10 +404,11 @@ class ShardRunner:
       g["x"] = torch.zeros(Bp, dtype=torch.int32, device=dev)
     else:
       g["x"] = torch.zeros(Bp, c.hidden_width, dtype=self.hidden_dtype, device=dev)
-    inp = StepInputs(g["pos"], g["slots"], g["tables"], g["ctx"], g["cu"], g["last"], 1, True)
+    # warm-up and capture run on padding rows only (state slot -1, no KV slot): no request's state is touched
+    g["slots"].fill_(-1)
+    g["sslots"].fill_(-1)
+    inp = StepInputs(g["pos"], g["slots"], g["tables"], g["ctx"], g["cu"], g["last"], 1, True, all_rows=True)
     if self.sm is not None:
-      # warm-up and capture run on padding rows only (state slot -1, no KV slot): no request's state is touched
-      g["sslots"] = torch.full((Bp,), -1, dtype=torch.int32, device=dev)
       inp.state_slots = g["sslots"]
     # warm up eagerly (also settles the GEMM policy for these shapes) on a side stream
     s = torch.cuda.Stream(dev)
