@@ -222,18 +222,20 @@ __global__ __launch_bounds__(DH) void attn_decode_reduce_kernel(const float* __r
 // so that this works with contiguous V^T reads: tile t = 2kk + h, row c = 4q + r holds key
 // 32kk + 8q + 4h + r, hence lane group g of the P^T operand owns keys 32kk + 8g .. +8 and reads one
 // 16-byte run of the transposed V page.  No LDS.
-// PF 1: prefetch the next page's K / V into a second register set under the current page's math (378
-//       registers: one wave per SIMD).
 // PF 2: ONE register set, each half refilled as soon as it is consumed -- the next page's K right after the
 //       S^T MFMAs, its V right after the P.V MFMAs -- so a page's loads fly under the other half's math and,
 //       at under 256 registers, two waves per SIMD keep twice the pages in flight per CU (algo 5 / 6).
-// NT: K / V pages loaded non-temporal (read once per step; algo 3 / 6)
-template <int DH, int PF, bool NT>
+// NT: K / V pages loaded non-temporal (read once per step; algo 3 / 6; the workgroup form of algo 2 / 3 follows)
+// NW > 1 (PF 2): the NW waves of a workgroup share the unit, wave w takes pages w, w + NW, ..., and they meet in LDS (sm:
+//       [NW][G][DH + 4] partial sums, then [NW][G][2] maxima and sums)
+template <int DH, int PF, bool NT, int NW = 1>
 __device__ __forceinline__ void decode_wave_unit(
     const int unit, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx_lens,
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int B, int H, int Hkv,
-    int pages_per_part, int nparts, float scale_log2, int num_pages, int* __restrict__ tickets, bool vtail) {
+    int pages_per_part, int nparts, float scale_log2, int num_pages, int* __restrict__ tickets, bool vtail,
+    float* sm = nullptr) {
+  static_assert(NW == 1 || PF == 2, "waves that share a unit run the single-set pipeline");
   constexpr int KS = DH / 32;   // k-steps of S^T over the head dim
   constexpr int NDT = DH / 16;  // 16-row d tiles of O^T
   const int lane = threadIdx.x & 63;
@@ -242,8 +244,9 @@ __device__ __forceinline__ void decode_wave_unit(
   const int G = H / Hkv;
   const int ctx = min(max(ctx_lens[b], 0), max_blocks * PAGE);
   const int npages = (ctx + PAGE - 1) / PAGE;
-  const int p_begin = part * pages_per_part;
-  const int p_end = min(npages, p_begin + pages_per_part);
+  const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p_begin = part * pages_per_part + wave;
+  const int p_end = min(npages, part * pages_per_part + pages_per_part);
 
   // Q^T (B operand): column c = query head kvh*G + c; k-step s, lane group g: d 32s + 8g .. +8
   // (natural MFMA order, so each K load instruction below reads 64 contiguous bytes of 16 rows).
@@ -358,27 +361,15 @@ __device__ __forceinline__ void decode_wave_unit(
   if constexpr (PF == 2) {
     s16x8 kf[4][KS], vf[NDT][2];
     if (p_begin < p_end) load(p_begin, kf, vf);
-    for (int p = p_begin; p < p_end; ++p) {
-      const bool more = p + 1 < p_end;
-      const long nxt = more ? page_of(p + 1) : 0;  // scalar block-table read, ahead of the loads that need it
+    for (int p = p_begin; p < p_end; p += NW) {
+      const bool more = p + NW < p_end;
+      const long nxt = more ? page_of(p + NW) : 0;  // scalar block-table read, ahead of the loads that need it
       f32x4 st[4];
       scores(kf, st);
-      if (more) load_k(p + 1, nxt, kf);  // K registers are free once the S^T MFMAs have read them
+      if (more) load_k(p + NW, nxt, kf);  // K registers are free once the S^T MFMAs have read them
       pv(p, st, vf);
-      if (more) load_v(p + 1, nxt, vf);
+      if (more) load_v(p + NW, nxt, vf);
     }
-  } else if constexpr (PF == 1) {
-    s16x8 ka[4][KS], kb2[4][KS];
-    s16x8 va[NDT][2], vb2[NDT][2];
-    int p = p_begin;
-    if (p < p_end) load(p, ka, va);
-    for (; p + 1 < p_end; p += 2) {
-      load(p + 1, kb2, vb2);
-      compute(p, ka, va);
-      if (p + 2 < p_end) load(p + 2, ka, va);
-      compute(p + 1, kb2, vb2);
-    }
-    if (p < p_end) compute(p, ka, va);
   } else {
     for (int p = p_begin; p < p_end; ++p) {
       s16x8 kf[4][KS], vf[NDT][2];
@@ -391,6 +382,44 @@ __device__ __forceinline__ void decode_wave_unit(
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
   const int h = kvh * G + c;
+  if constexpr (NW > 1) {
+    constexpr int LD = DH + 4;
+    float* ml = sm + NW * G * LD;
+    if (c < G) {
+      float* so = sm + (wave * G + c) * LD + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4*>(so + 16 * dt) = o[dt];
+      if (g == 0) {
+        ml[(wave * G + c) * 2] = m;
+        ml[(wave * G + c) * 2 + 1] = l;
+      }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < G * DH; e += NW * 64) {
+      const int hq = e / DH, d = e - hq * DH;
+      float M = NEG_BIG;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[(w * G + hq) * 2]);
+      float L = 0.f, O = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {  // (a wave without pages: m = NEG_BIG, l = 0, o = 0)
+        const float f = exp2f(ml[(w * G + hq) * 2] - M);
+        L += ml[(w * G + hq) * 2 + 1] * f;
+        O += sm[(w * G + hq) * LD + d] * f;
+      }
+      const size_t row = (size_t)b * H + kvh * G + hq;
+      if (nparts == 1) {
+        out[row * DH + d] = f2bf(L > 0.f ? O / L : 0.f);
+      } else {
+        ws_o[(row * nparts + part) * DH + d] = O;
+        if (d == 0) {
+          ws_ml[(row * nparts + part) * 2] = M;
+          ws_ml[(row * nparts + part) * 2 + 1] = L;
+        }
+      }
+    }
+    return;
+  }
   if (nparts == 1) {
     if (c >= G) return;
     const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -432,6 +461,24 @@ __global__ __launch_bounds__(PF == 2 ? 512 : 256, PF == 2 ? 2 : 1) void attn_dec
                                pages_per_part, nparts, scale_log2, num_pages, tickets, vtail != 0);
 }
 
+// The NW waves of a workgroup share one (sequence, KV head, partition): a short context's pages are in flight together and the
+// waves meet in LDS, not in a reduce launch.  A lone wave per unit walked its pages one behind the other (~3 us each) and needed
+// partitions, and their merge launch, to shorten that.  Llama-3-8B heads, ragged contexts, us per layer with the merge, before /
+// now: 24 sequences up to 1407 tokens 24.1 / 21.3, 64 up to 393 18.7 / 15.8, 128 up to 1900 113.5 / 67.4, 64 up to 8000
+// 180 / 159; 256 even ones of 1900 307 / 301 (6.6 TB/s).  Four waves measured ahead of eight (two workgroups a CU overlap one's
+// start with the other's pages); two where a table of 8 pages leaves most waves of four without one and there are enough units
+// to fill the chip (512 sequences of 33 .. 189 tokens: 50.7 before, 51.4 with four waves, 44.0 with two).
+template <int DH, bool NT, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_decode_group_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx_lens,
+    uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int B, int H, int Hkv,
+    int pages_per_part, int nparts, float scale_log2, int num_pages) {
+  extern __shared__ __attribute__((aligned(16))) float gsm[];
+  decode_wave_unit<DH, 2, NT, NW>(blockIdx.x, q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, ws_ml, B, H, Hkv,
+                                  pages_per_part, nparts, scale_log2, num_pages, nullptr, true, gsm);
+}
+
 int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                        int max_blocks, const int32_t* ctx_lens, uint16_t* out, float* ws_o, float* ws_ml, int B,
                        int H, int Hkv, int Dh, int pages_per_part, int nparts, float scale, int num_pages, int algo,
@@ -445,6 +492,28 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
   if (H % Hkv != 0 || H / Hkv > 16) return -1;
   dim3 grid(nparts, Hkv, B);
   const float sl = scale * LOG2E;
+  if (algo == 2 || algo == 3) {  // NW waves per (sequence, KV head, partition); 3: nt loads
+    const int units = B * Hkv * nparts, G = H / Hkv;
+    const bool pair = max_blocks <= 8 && units >= 1024;
+    const size_t lds = (size_t)(pair ? 2 : 4) * G * (Dh + 6) * sizeof(float);  // at most 34 KB
+#define XOT_GROUP(DHV, NTV, NWV)                                                                                \
+  attn_decode_group_kernel<DHV, NTV, NWV><<<units, 64 * NWV, lds, s>>>(q, kc, vc, block_tables, max_blocks,     \
+                                                        ctx_lens, out, ws_o, ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages)
+#define XOT_GROUP_DH(DHV)                                                                                       \
+  do {                                                                                                          \
+    if (pair && algo == 3) XOT_GROUP(DHV, true, 2);                                                             \
+    else if (pair) XOT_GROUP(DHV, false, 2);                                                                    \
+    else if (algo == 3) XOT_GROUP(DHV, true, 4);                                                                \
+    else XOT_GROUP(DHV, false, 4);                                                                              \
+    if (reduce) attn_decode_reduce_kernel<DHV><<<B * H, DHV, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part); \
+  } while (0)
+    if (Dh == 128) XOT_GROUP_DH(128);
+    else if (Dh == 64) XOT_GROUP_DH(64);
+    else return -1;
+#undef XOT_GROUP_DH
+#undef XOT_GROUP
+    return 0;
+  }
   if (algo != 0) {  // wave per (sequence, KV head, partition)
     // algo 5 / 6: 8-wave workgroups (two waves per SIMD)
     const int units = B * Hkv * nparts, wpg = algo >= 5 ? 8 : 4;
@@ -452,14 +521,12 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
 #define XOT_WAVE(DHV, PFV, NTV)                                                                                  \
   attn_decode_wave_kernel<DHV, PFV, NTV><<<wgs, 64 * wpg, 0, s>>>(q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, \
                                                         ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages, tickets, 1)
-    // algo 1: no prefetch; 2 / 3: double register set (3: nt loads); 5 / 6: one set refilled per half (6: nt)
+    // algo 1: no prefetch; 5 / 6: one register set refilled per half (6: nt loads)
     if (Dh == 128) {
-      if (algo == 3) XOT_WAVE(128, 1, true); else if (algo == 2) XOT_WAVE(128, 1, false);
-      else if (algo == 5) XOT_WAVE(128, 2, false); else if (algo == 6) XOT_WAVE(128, 2, true); else XOT_WAVE(128, 0, false);
+      if (algo == 5) XOT_WAVE(128, 2, false); else if (algo == 6) XOT_WAVE(128, 2, true); else XOT_WAVE(128, 0, false);
       if (reduce) attn_decode_reduce_kernel<128><<<B * H, 128, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
     } else if (Dh == 64) {
-      if (algo == 3) XOT_WAVE(64, 1, true); else if (algo == 2) XOT_WAVE(64, 1, false);
-      else if (algo == 5) XOT_WAVE(64, 2, false); else if (algo == 6) XOT_WAVE(64, 2, true); else XOT_WAVE(64, 0, false);
+      if (algo == 5) XOT_WAVE(64, 2, false); else if (algo == 6) XOT_WAVE(64, 2, true); else XOT_WAVE(64, 0, false);
       if (reduce) attn_decode_reduce_kernel<64><<<B * H, 64, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
     } else {
       return -1;

@@ -147,20 +147,14 @@ def rope_apply(x: torch.Tensor, pos: torch.Tensor, cos_sin: torch.Tensor, nh: in
 
 
 # ------------------------------------------------------------------ attention
-# 0: workgroup per (sequence, KV head, partition), waves split pages + LDS combine
-# 1 / 2: wave per (sequence, KV head, partition), transposed S^T (lane = query head), no LDS;
-#        2 prefetches the next page under the current one
-# 3: 2 with non-temporal K / V loads (neutral in round 3, profiles/r3/s3/; on the chunk-major V cache of round 6
-#        the KV stream runs 5-13 % faster in isolation -- B 512: 183.9 vs 193.7 us per layer, B 256 / ctx 1040:
-#        166.6 vs 185.1, B 128 / ctx 2048: 156.2 vs 177.3 -- and the 70B headline step 74.6-74.7 vs 75.4-75.7 ms,
-#        profiles/r6/headline/attn_nt/)
-# -1 (default): 0 below 64 (sequence, KV head) pairs -- few long sequences, where the workgroup
-#        kernel's 4-wave page split needs fewer partitions; else 3 once a layer's K / V pages (batch x block-table
-#        width) outgrow the 256 MB last-level cache, 2 below (B 16 / ctx 530: 15.1 vs 13.5 us, B 64 / ctx 530: 29.3 vs
-#        24.8 with nt; B 16 / ctx 8192: 85.7 vs 97.1, B 64 / ctx 2048: 85.1 vs 97.2; tools/bench_attn_small.py,
-#        profiles/r6/headline/attn_nt/attn_small.log)
-# (4, an 8-wave workgroup over one partition for short tables at small batch, measured 1 % slower at 8B batch 1 --
-#  3.55 vs 3.52 ms, profiles/r3/s3/ -- and was removed in round 6)
+# 0: workgroup per (sequence, KV head, partition), waves split pages + LDS combine (scores by rows, P through LDS)
+# 1: wave per (sequence, KV head, partition), transposed S^T (lane = query head), no LDS; 5 / 6: the same with the next page's
+#    loads under the current one (6: non-temporal)
+# 2 / 3: four (or two) waves per (sequence, KV head, partition), each as in 5, meeting in LDS; 3 with non-temporal K / V loads
+# -1 (default): 0 below 16 (sequence, KV head) pairs, where the partitions of a single sequence are merged by the output
+#    projection's prologue; else 3 once a layer's K / V pages (batch x block-table width) outgrow the 256 MB last-level cache
+#    (256 sequences of 1900 tokens: 301 us, 331 with plain loads), 2 below (24 up to 1407 tokens: 21.3 us, 23.5 with nt).
+#    From 16 pairs on 2 also leads 0: 2 sequences x 8 heads of 130 tokens 6.3 us / 9.1, of 8000 21.0 / 29.8; 6 of 2000 15.0 / 18.8
 DECODE_ALGO = int(os.environ.get("XOT_ATTN_DECODE", "-1"))
 
 
@@ -170,10 +164,18 @@ NT_MIN_KV_BYTES = 256 << 20  # K / V bytes per layer from which the page loads g
 def resolve_decode_algo(batch: int, Hkv: int, algo: int | None = None, kv_bytes: int | None = None) -> int:
   algo = DECODE_ALGO if algo is None else algo
   if algo < 0:
-    if batch * Hkv < 64:
+    if batch * Hkv < 16:
       return 0
     return 3 if kv_bytes is None or kv_bytes >= NT_MIN_KV_BYTES else 2
   return algo
+
+
+def group_parts(batch: int, Hkv: int, pages: int) -> int:
+  """Most partitions of a context of `pages` pages for algo 2 / 3 (grows with pages)."""
+  pairs = max(batch * Hkv, 1)
+  if pages <= 8:
+    return 1
+  return min(max(round(256 / pairs), 2 if pages > 64 and pairs < 384 else 1), -(-pages // 4))
 
 
 def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None = None) -> int:
@@ -185,6 +187,12 @@ def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None =
       if batch * Hkv * -(-pages // ppp) >= 1024:
         return ppp
     return 4
+  if algo in (2, 3):
+    # four waves per unit (csrc/attention.hip attn_decode_group_kernel): a context of 8 pages is two pages a wave and best left
+    # whole; longer ones are cut until the units cover the CUs, in partitions of at least 4 pages (8 sequences x 8 heads, up to
+    # 1900 tokens: 20.4 us whole, 13.9 in 4; 16: 21.7, 18.0 in 2, 19.5 in 4; 24: 21.3 whole, 23.0 in 2), and very long ones
+    # once more, since the longest workgroup ends the launch (32 sequences up to 7800 tokens: 100 us whole, 87 in 2)
+    return -(-pages // group_parts(batch, Hkv, pages))
   # one wave per unit: ~1024 waves (4 per CU), partitions of 2..32 pages (tools/bench_attn_small.py,
   # profiles/bench_attn_small_r1.json: 2048 waves of shorter partitions lose to the extra merge work)
   nparts = max(1, min(max(pages // 2, 1), -(-1024 // max(batch * Hkv, 1))))
@@ -207,6 +215,9 @@ class DecodeWorkspace:
     worst = 1
     for b in range(1, max_batch + 1):
       for hkv in (1, 2, 4, 8, 16):
+        if pages_per_part is None and resolve_decode_algo(b, hkv, self.algo) in (2, 3):
+          worst = max(worst, b * group_parts(b, hkv, pages))  # (narrower tables have no more partitions)
+          continue
         ppp = pages_per_part or choose_pages_per_part(b, hkv, max_ctx, self.algo)
         worst = max(worst, b * -(-pages // ppp))
     self.units = worst  # max over batch of batch * nparts
