@@ -808,10 +808,7 @@ def build_mixed_layer(spec, get, p: str, D: int, device, dtype) -> MixedLayerWei
     cols[n] = (off, w.shape[0])
     off += w.shape[0]
   Dp = _up(D, 128)
-  # whole 256-row tiles where that costs at most 5 % of zero rows: the four-wave GEMM takes no others (12807 x 20032 x 2048,
-  # fp32: 942 us on the ping-pong tile and a pass of 190 for the activation; 12807 x 8960 380 and 12807 x 11264 495 on the
-  # four-wave one, activation included)
-  Np = _up(off, 256) if dtype == torch.bfloat16 and 20 * _up(off, 256) <= 21 * off else _up(off, 64)
+  Np = _up(off, _row_mult(off, dtype))
   Fp = _up(spec.ff, 128)
   in_w = torch.zeros(Np + (2 * Fp if tiles else 0), Dp)
   in_w[:off, :D] = torch.cat([w for _, w in blocks], 0)
@@ -847,6 +844,13 @@ def build_mixed_layer(spec, get, p: str, D: int, device, dtype) -> MixedLayerWei
     lw.a2_w, lw.a2_b = dev(get(names["a2"])), dev(get(names["a2_b"]))
   lw.rec_norm = dev(get(names["rec_norm"]))
   return lw
+
+
+def _row_mult(rows: int, dtype) -> int:
+  """Row padding of a fused projection: whole 256-row tiles where that costs at most 5 % of zero rows, since the four-wave GEMM
+  takes no others (12807 x 20032 x 2048, fp32: 942 us on the ping-pong tile and a pass of 190 for the activation; 12807 x 8960
+  380 and 12807 x 11264 495 on the four-wave one, activation included)."""
+  return 256 if dtype == torch.bfloat16 and 20 * _up(rows, 256) <= 21 * rows else 64
 
 
 def _fused_rows(blocks, D: int, row_mult: int = 64):
@@ -1175,7 +1179,7 @@ def build_conv_sandwich_layer(spec, get, p: str, D: int, device, dtype) -> Mixed
       conv_b = torch.cat([conv_b, get(n + "conv.b")])
       units = units + [(C, CONV_SILU)]
       out2 = get(n + "o")
-  in_w, cols = _fused_rows(blocks, D)
+  in_w, cols = _fused_rows(blocks, D, _row_mult(sum(w.shape[0] for _, w in blocks), dtype))
   lw = MixedLayerWeights(spec, dev(in_w, dtype), cols, dev(_pad2(out, _up(D, 64), _up(out.shape[1], 128)), dtype),
                          {"mix": (0, out.shape[1])})
   for n in ("norm1", "norm1b") + (("norm2", "norm2b") if f is not None else ()):
