@@ -78,18 +78,26 @@ __device__ __forceinline__ void splitk_out8(const float* __restrict__ wsrow, siz
     float gs[8], us[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) gs[e] = us[e] = 0.f;
-    for (int s = 0; s < S; ++s) {
-      const float* row = wsrow + s * sstride;
-      const f32x4 g0 = *reinterpret_cast<const f32x4*>(row + 32 * j + w);
-      const f32x4 g1 = *reinterpret_cast<const f32x4*>(row + 32 * j + w + 4);
-      const f32x4 u0 = *reinterpret_cast<const f32x4*>(row + 32 * j + 16 + w);
-      const f32x4 u1 = *reinterpret_cast<const f32x4*>(row + 32 * j + 16 + w + 4);
+    for (int s0 = 0; s0 < S; s0 += 4) {  // four slabs' loads in flight (past the last: it again, not added)
+      f32x4 g[4][2], u[4][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        gs[e] += g0[e];
-        gs[e + 4] += g1[e];
-        us[e] += u0[e];
-        us[e + 4] += u1[e];
+      for (int k = 0; k < 4; ++k) {
+        const float* row = wsrow + (s0 + k < S ? s0 + k : S - 1) * sstride + 32 * j + w;
+        g[k][0] = *reinterpret_cast<const f32x4*>(row);
+        g[k][1] = *reinterpret_cast<const f32x4*>(row + 4);
+        u[k][0] = *reinterpret_cast<const f32x4*>(row + 16);
+        u[k][1] = *reinterpret_cast<const f32x4*>(row + 20);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (s0 + k >= S) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          gs[e] += g[k][0][e];
+          gs[e + 4] += g[k][1][e];
+          us[e] += u[k][0][e];
+          us[e + 4] += u[k][1][e];
+        }
       }
     }
 #pragma unroll
@@ -100,13 +108,22 @@ __device__ __forceinline__ void splitk_out8(const float* __restrict__ wsrow, siz
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    for (int s = 0; s < S; ++s) {
-      const float* row = wsrow + s * sstride + o;
-      const f32x4 a = *reinterpret_cast<const f32x4*>(row), b = *reinterpret_cast<const f32x4*>(row + 4);
+    for (int s0 = 0; s0 < S; s0 += 4) {
+      f32x4 a[4][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[e] += a[e];
-        v[e + 4] += b[e];
+      for (int k = 0; k < 4; ++k) {
+        const float* row = wsrow + (s0 + k < S ? s0 + k : S - 1) * sstride + o;
+        a[k][0] = *reinterpret_cast<const f32x4*>(row);
+        a[k][1] = *reinterpret_cast<const f32x4*>(row + 4);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (s0 + k >= S) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] += a[k][0][e];
+          v[e + 4] += a[k][1][e];
+        }
       }
     }
     if (bias != nullptr) {

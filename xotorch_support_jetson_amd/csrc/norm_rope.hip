@@ -81,7 +81,7 @@ void launch_rmsnorm(const uint16_t* x, const uint16_t* res, const uint16_t* w, u
 // One workgroup per row: h = bf16(h + bias + sum_s ws[s][row]) (in place), out = rmsnorm(h) * w.  Replaces
 // the split-K reduce kernel of a residual projection (o_proj / down_proj) and the RMSNorm that follows it.
 // SS > 0: exactly SS slabs, loads unrolled and issued together (a runtime slab loop waits for each load
-// in turn: one row at decode batch 1 took 6.9 us); SS = 0: any S.
+// in turn: one row at decode batch 1 took 6.9 us); SS = 0: any S, four slabs at a time.
 // NTH threads per row: 1024 for wide rows (D = 8192 at decode batch 512: 512 workgroups of 256 threads left 8 waves
 // per CU and each thread's four chunks x (h + S slabs) loads partly serialised; 16 waves per row keep one chunk each)
 template <int MAXC, int SS, int NTH = 256>
@@ -124,12 +124,22 @@ __global__ __launch_bounds__(NTH) void splitk_resid_rmsnorm_kernel(const float* 
             acc[4 + j] += p[sl][1][j];
           }
       } else {
-        for (int sl = 0; sl < S; ++sl, sp += sstride) {
-          const f32x4 p0 = *reinterpret_cast<const f32x4*>(sp), p1 = *reinterpret_cast<const f32x4*>(sp + 4);
+        for (int s0 = 0; s0 < S; s0 += 4) {  // four slabs' loads in flight (past the last: it again, not added)
+          f32x4 p[4][2];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            acc[j] += p0[j];
-            acc[4 + j] += p1[j];
+          for (int k = 0; k < 4; ++k) {
+            const float* q = sp + (size_t)min(s0 + k, S - 1) * sstride;
+            p[k][0] = *reinterpret_cast<const f32x4*>(q);
+            p[k][1] = *reinterpret_cast<const f32x4*>(q + 4);
+          }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            if (s0 + k >= S) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              acc[j] += p[k][0][j];
+              acc[4 + j] += p[k][1][j];
+            }
           }
         }
       }
