@@ -253,6 +253,106 @@ __global__ __launch_bounds__(1024) void moe_slots_kernel(const int32_t* __restri
   }
 }
 
+// The same for few tokens (at most MOE_SMALL_T), at most 64 experts and no group choice, in one workgroup and one launch: a wave
+// per token, lane = expert; then the counts' scan and the slots in LDS.  The k rounds take the largest choice as an ordered
+// integer by six register-to-register (DPP) steps and the lowest lane that holds it by a ballot: 90 instructions a token, where
+// argmax rounds over ds_bpermute are a chain of 12 k LDS round trips, and ranks counted over 64 broadcasts 450 instructions
+// that one CU has to issue (12.2 us).  37 tokens, 64 experts, top 6: 6.8 us, 8.8 + 4.6 in two launches.
+// Scores, ties and rows that are not numbers as in moe_topk_ds_kernel, bit for bit.
+constexpr int MOE_SMALL_T = 128;
+constexpr int MOE_SMALL_K = 16;
+
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_umax(unsigned x) {
+  return max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false));
+}
+// the largest of the wave's values, in every lane
+__device__ __forceinline__ unsigned wave_umax(unsigned x) {
+  x = dpp_umax<0x111>(x);  // row_shr 1, 2, 4, 8: lane 15 of a row has its row's
+  x = dpp_umax<0x112>(x);
+  x = dpp_umax<0x114>(x);
+  x = dpp_umax<0x118>(x);
+  x = dpp_umax<0x142>(x);  // row_bcast 15, 31: lane 63 has all of them
+  x = dpp_umax<0x143>(x);
+  return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+__global__ __launch_bounds__(1024) void moe_route_small_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
+                                                               int T, int E, int k, int sigmoid, int norm, float scale,
+                                                               float* __restrict__ topw, int32_t* __restrict__ topi,
+                                                               int32_t* __restrict__ slot_of, int32_t* __restrict__ sorted_tok,
+                                                               int32_t* __restrict__ off) {
+  constexpr int TPW = MOE_SMALL_T / 16;  // tokens of a wave
+  __shared__ int cnt[64], base[64], chosen[MOE_SMALL_T * MOE_SMALL_K];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid < 64) cnt[tid] = 0;
+  __syncthreads();
+  float lg[TPW];
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {  // every token's logits are on their way before the first is used
+    const int t = wave + 16 * i;
+    lg[i] = t < T && lane < E ? logits[(size_t)t * E + lane] : -INFINITY;
+  }
+  const float b = bias != nullptr && lane < E ? bias[lane] : 0.f;
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    const int t = wave + 16 * i;
+    if (t >= T) break;  // (wave-uniform; no workgroup barrier inside)
+    float sc;
+    if (sigmoid) {
+      sc = lane < E ? 1.f / (1.f + expf(-lg[i])) : 0.f;
+    } else {
+      const float mx = wave_max(lg[i]);
+      sc = lane < E ? __expf(lg[i] - mx) : 0.f;
+      sc /= wave_sum(sc);
+    }
+    const float ch = lane < E ? sc + b + 0.0f : -INFINITY;  // (+ 0.0: equal zeros have equal bits)
+    // bits in the order of the numbers; 0 for what cannot win: no expert, minus infinity, not a number
+    const unsigned bits = __float_as_uint(ch);
+    unsigned key = bits ^ (bits >> 31 ? 0xffffffffu : 0x80000000u);
+    if ((bits & 0x7fffffffu) > 0x7f800000u || bits == 0xff800000u) key = 0;
+    float wsum = 0.f, w_mine = 0.f;
+    int e_mine = 0;
+    for (int j = 0; j < k; ++j) {
+      const unsigned top = wave_umax(key);
+      const int id = top ? __ffsll((unsigned long long)__ballot(key == top)) - 1 : j;  // (no winner left: expert j)
+      const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), id));
+      wsum += w;
+      if (lane == j) {
+        w_mine = w;
+        e_mine = id;
+      }
+      if (lane == id) key = 0;
+    }
+    if (lane < k) {
+      topw[(size_t)t * k + lane] = w_mine * (norm ? scale / (wsum + 1e-20f) : scale);
+      topi[(size_t)t * k + lane] = e_mine;
+      chosen[t * k + lane] = e_mine;
+      atomicAdd(cnt + e_mine, 1);
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int c = cnt[lane];
+    int sum = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(sum, o, 64);
+      sum += lane >= o ? v : 0;
+    }
+    base[lane] = sum - c;
+    if (lane < E) off[lane] = sum - c;
+    if (lane == 63) off[E] = sum;
+    cnt[lane] = 0;
+  }
+  __syncthreads();
+  for (int q = tid; q < T * k; q += 1024) {
+    const int e = chosen[q], pos = base[e] + atomicAdd(cnt + e, 1);
+    slot_of[q] = pos;
+    sorted_tok[pos] = q / k;
+  }
+}
+
 int launch_moe_route_ds(const float* logits, const float* bias, int T, int E, int k, int n_group, int topk_group,
                         int method, bool sigmoid, bool norm, float scale, int* cnt, float* topw, int32_t* topi,
                         int32_t* slot_of, int32_t* sorted_tok, int32_t* off, hipStream_t s) {
@@ -260,6 +360,11 @@ int launch_moe_route_ds(const float* logits, const float* bias, int T, int E, in
       topk_group < 1 || topk_group > n_group || k > (E / n_group) * topk_group)
     return -1;
   if (T <= 0) return 0;
+  if (T <= MOE_SMALL_T && E <= 64 && k <= MOE_SMALL_K && topk_group == n_group) {
+    moe_route_small_kernel<<<1, 1024, 0, s>>>(logits, bias, T, E, k, sigmoid ? 1 : 0, norm ? 1 : 0, scale, topw, topi, slot_of,
+                                              sorted_tok, off);
+    return 0;
+  }
   moe_topk_ds_kernel<<<std::min((T + 3) / 4, 512), 256, 0, s>>>(logits, bias, T, E, k, n_group, topk_group, method, sigmoid ? 1 : 0,
                                                  norm ? 1 : 0, scale, topw, topi, cnt);
   moe_slots_kernel<<<1, 1024, 0, s>>>(topi, T, E, k, cnt, slot_of, sorted_tok, off);
@@ -417,19 +522,20 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint16_t* __re
 // expert tile's row (B fragment, same map) from global / L2, U steps at a time with every load issued before
 // the MFMAs; the NW partial 16 x E tiles are summed in LDS in wave order (deterministic).  Rows past T
 // re-read row T - 1 and are not stored.  Requires D % (128 NW) == 0.
-template <int ET, int NW>
+// Few tokens: a workgroup takes one of the expert tiles (ETW 1, grid.y of them) and 8 k steps at a time, so that a 2048-wide row
+// is one round of loads (37 tokens, 64 experts: 5.2 us, 10.4 with all tiles in a workgroup; the sums keep their order).
+template <int ETW, int NW, int U>
 __global__ __launch_bounds__(NW * 64) void router_logits_mfma_kernel(const uint16_t* __restrict__ x,
                                                                      const uint16_t* __restrict__ w,
-                                                                     float* __restrict__ out, int T, int D) {
-  constexpr int E = 16 * ET;
-  constexpr int U = ET <= 4 ? 4 : (ET <= 8 ? 2 : 1);  // k steps in flight per iteration (register budget)
+                                                                     float* __restrict__ out, int T, int D, int E_all) {
+  constexpr int ET = ETW, E = 16 * ET;  // of this workgroup: experts 16 ET blockIdx.y .. + E
   extern __shared__ float red[];                      // [NW][16][E] partial logits
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int t0 = blockIdx.x * 16;
   const int kq = D / NW, kb = wave * kq;
   const uint16_t* xr = x + (size_t)min(t0 + c, T - 1) * D + kb + 8 * g;
-  const uint16_t* wr = w + (size_t)c * D + kb + 8 * g;  // + 16 j D for tile j
+  const uint16_t* wr = w + (size_t)(blockIdx.y * E + c) * D + kb + 8 * g;  // + 16 j D for tile j
   f32x4 acc[ET];
 #pragma unroll
   for (int j = 0; j < ET; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -456,13 +562,20 @@ __global__ __launch_bounds__(NW * 64) void router_logits_mfma_kernel(const uint1
 #pragma unroll
     for (int q = 0; q < NW; ++q) v += red[q * 16 * E + i];
     const int t = t0 + i / E;
-    if (t < T) out[(size_t)t * E + i % E] = v;
+    if (t < T) out[(size_t)t * E_all + blockIdx.y * E + i % E] = v;
   }
 }
 
 template <int ET, int NW>
 static void router_mfma_launch(const uint16_t* x, const uint16_t* w, float* out, int T, int D, hipStream_t s) {
-  router_logits_mfma_kernel<ET, NW><<<(T + 15) / 16, NW * 64, NW * 16 * 16 * ET * 4, s>>>(x, w, out, T, D);
+  constexpr int U = ET <= 4 ? 4 : (ET <= 8 ? 2 : 1);  // k steps in flight per iteration (register budget)
+  const int mt = (T + 15) / 16;
+  if (mt * ET <= 256 && D % (256 * NW) == 0)  // one workgroup a CU at most
+    router_logits_mfma_kernel<1, NW, 8><<<dim3(mt, ET), NW * 64, NW * 16 * 16 * 4, s>>>(x, w, out, T, D, 16 * ET);
+  else if (mt * ET <= 256)
+    router_logits_mfma_kernel<1, NW, 4><<<dim3(mt, ET), NW * 64, NW * 16 * 16 * 4, s>>>(x, w, out, T, D, 16 * ET);
+  else
+    router_logits_mfma_kernel<ET, NW, U><<<mt, NW * 64, NW * 16 * 16 * ET * 4, s>>>(x, w, out, T, D, 16 * ET);
 }
 
 int launch_router_logits(const uint16_t* x, const uint16_t* w, float* out, int T, int E, int D, hipStream_t s) {
