@@ -744,6 +744,33 @@ void mla_prep(const at::Tensor& ckv, const at::Tensor& kv_ln, at::Tensor& q, int
                        cur_stream());
 }
 
+// the same from the fused projection's fp32 result P [T, N] or split-K slabs [S, T, N]; q [T, >= H dn + H DR] takes the queries
+void mla_prep_slabs(const at::Tensor& P, int64_t nope, const at::Tensor& kv_ln, at::Tensor& q, int64_t H, const at::Tensor& pos,
+                    const at::Tensor& cos_sin, const at::Tensor& slots, at::Tensor& cache, double eps) {
+  CHECK_GPU(P);
+  CHECK_DT(P, at::kFloat);
+  CHECK_BF16(kv_ln);
+  CHECK_BF16(q);
+  CHECK_BF16(cache);
+  CHECK_DT(pos, at::kInt);
+  CHECK_DT(cos_sin, at::kFloat);
+  CHECK_DT(slots, at::kLong);
+  XCHECK(all_contig_gpu(P, kv_ln, pos, cos_sin, slots, cache) && (P.dim() == 2 || P.dim() == 3), "mla_prep_slabs: contiguous GPU tensors");
+  const int64_t S = P.dim() == 3 ? P.size(0) : 1, T = P.size(-2), N = P.size(-1), DL = kv_ln.numel(), DR = cos_sin.size(1);
+  XCHECK(cache.dim() == 3 && cache.size(1) == 64 && cache.size(2) == DL + DR, "mla_prep_slabs: cache [pages, 64, DL + DR]");
+  XCHECK(N >= nope + H * DR + DL + DR && nope >= 0 && H >= 1, "mla_prep_slabs: projection columns");
+  XCHECK(q.dim() == 2 && q.stride(1) == 1 && q.size(0) == T && q.size(1) >= nope + H * DR && pos.numel() == T && slots.numel() == T,
+         "mla_prep_slabs: shapes");
+  XCHECK(reinterpret_cast<uintptr_t>(P.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0 &&
+             reinterpret_cast<uintptr_t>(cache.data_ptr()) % 16 == 0 && (DL + DR) % 8 == 0,
+         "mla_prep_slabs: 16-byte rows");
+  const int rc = xot::launch_mla_prep_slabs(P.data_ptr<float>(), (int)S, (long)(T * N), (int)N, (int)nope, bf(kv_ln), bf(q),
+                                            (long)q.stride(0), pos.data_ptr<int>(), cos_sin.data_ptr<float>(),
+                                            slots.data_ptr<int64_t>(), bf(cache), (int)T, (int)H, (int)DL, (int)DR,
+                                            (int)cos_sin.size(0), (long)(cache.size(0) * 64), (float)eps, cur_stream());
+  XCHECK(rc == 0, "mla_prep_slabs: unsupported dims");
+}
+
 // q_lat / out [H, T, DL]; q_pe rows of q (row stride ldqpe = q_pe.stride(0)) as [T, H * DR]
 void mla_attn(const at::Tensor& q_lat, const at::Tensor& q_pe, const at::Tensor& cache, const at::Tensor& block_tables,
               const at::Tensor& cu_q, const at::Tensor& ctx_lens, at::Tensor& out, at::Tensor& ws_o, at::Tensor& ws_ml,
@@ -1158,6 +1185,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_route", &moe_route);
   m.def("moe_route_ds", &moe_route_ds);
   m.def("mla_prep", &mla_prep);
+  m.def("mla_prep_slabs", &mla_prep_slabs);
   m.def("mla_attn", &mla_attn, py::arg("q_lat"), py::arg("q_pe"), py::arg("cache"), py::arg("block_tables"),
         py::arg("cu_q"), py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
         py::arg("nparts"), py::arg("scale"), py::arg("wide") = 0);

@@ -137,6 +137,9 @@ int launch_moe_route_ds(const float* logits, const float* bias, int T, int E, in
                         int method, bool sigmoid, bool norm, float scale, int* cnt, float* topw, int32_t* topi,
                         int32_t* slot_of, int32_t* sorted_tok, int32_t* off, hipStream_t s);
 // DeepSeek MLA: latent norm + rope + latent cache write (q_pe rotated in place), and the absorbed attention
+int launch_mla_prep_slabs(const float* P, int S, long ss, int N, int nope, const uint16_t* kv_ln, uint16_t* q, long ldq,
+                          const int32_t* pos, const float* cos_sin, const int64_t* slots, uint16_t* cache, int T, int H, int DL,
+                          int DR, int max_pos, long nslots, float eps, hipStream_t s);
 void launch_mla_prep(const uint16_t* ckv, long ldc, const uint16_t* kv_ln, uint16_t* q, long ldq, long qpe_off,
                      const int32_t* pos, const float* cos_sin, const int64_t* slots, uint16_t* cache, int T, int H,
                      int DL, int DR, int max_pos, long nslots, float eps, hipStream_t s);

@@ -120,6 +120,136 @@ void launch_mla_prep(const uint16_t* ckv, long ldc, const uint16_t* kv_ln, uint1
                                     nslots, eps);
 }
 
+// The same on the split-K slabs of the fused projection [q_nope: H dn | q_pe: H DR | latent: DL | key part: DR] (S slabs ss
+// floats apart, rows of N): sums in slab order, rounded to bf16 as the reduce kernel rounds them, the queries to q [T, ldq].
+// Workgroup = (token, role): 0 the latent and the shared key, then 2048 unrotated query columns each, then the rotated parts.
+// Launch-bound at decode batches: it takes the place of a reduce launch and the kernel above (37 tokens of DeepSeek-V2-Lite, 8
+// slabs: 5.0 us, 4.9 + 4.9 before).
+constexpr int MLA_SLAB_COLS = 2048;
+
+// eight columns at each of NP places
+template <int NP>
+__device__ __forceinline__ void slab8(const float* const (&p)[NP], int S, long ss, float (&v)[NP][8]) {
+#pragma unroll
+  for (int n = 0; n < NP; ++n)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[n][e] = 0.f;
+  for (int s0 = 0; s0 < S; s0 += 8) {  // eight slabs' loads in flight (past the last: it again, not added)
+    f32x4 a[8][NP][2];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        const float* q = p[n] + (long)min(s0 + k, S - 1) * ss;
+        a[k][n][0] = *reinterpret_cast<const f32x4*>(q);
+        a[k][n][1] = *reinterpret_cast<const f32x4*>(q + 4);
+      }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (s0 + k >= S) continue;
+#pragma unroll
+      for (int n = 0; n < NP; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[n][e] += a[k][n][0][e];
+          v[n][e + 4] += a[k][n][1][e];
+        }
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NP; ++n)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[n][e] = bf2f(f2bf(v[n][e]));
+}
+
+__global__ __launch_bounds__(256) void mla_prep_slabs_kernel(const float* __restrict__ P, int S, long ss, int N, int nope,
+                                                             const uint16_t* __restrict__ kv_ln, uint16_t* __restrict__ q,
+                                                             long ldq, const int32_t* __restrict__ pos,
+                                                             const float* __restrict__ cos_sin,
+                                                             const int64_t* __restrict__ slots, uint16_t* __restrict__ cache,
+                                                             int H, int DL, int DR, int max_pos, long nslots, float eps) {
+  __shared__ float red[4];
+  const int t = blockIdx.x, tid = threadIdx.x, role = blockIdx.y, half = DR >> 1;
+  const float* row = P + (size_t)t * N;
+  const int p = min(max(pos[t], 0), max_pos - 1);
+  const float* cs = cos_sin + (size_t)p * DR;
+  // eight rotation pairs (i .. i + 7, half + i ..) of the DR columns at src
+  auto rotate = [&](const float* src, int i, uint16_t* dst) {
+    const float* at[2] = {src + i, src + half + i};
+    float v[2][8];
+    slab8<2>(at, S, ss, v);
+    const float(&a)[8] = v[0];
+    const float(&b)[8] = v[1];
+    s16x8 y0, y1;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float c = cs[i + e], s = cs[half + i + e];
+      y0[e] = (short)f2bf(a[e] * c - b[e] * s);
+      y1[e] = (short)f2bf(b[e] * c + a[e] * s);
+    }
+    st16(dst + i, y0);
+    st16(dst + half + i, y1);
+  };
+  if (role == 0) {
+    const int64_t slot = slots[t] < nslots ? slots[t] : -1;
+    const float* lat = row + nope + H * DR;
+    const int nch = DL >> 3;
+    float v[1][8];
+    float sq = 0.f;
+    if (tid >= 192 && tid < 192 + half / 8 && slot >= 0) rotate(lat + DL, 8 * (tid - 192), cache + (size_t)slot * (DL + DR) + DL);
+    if (tid < nch) {
+      const float* at[1] = {lat + 8 * tid};
+      slab8<1>(at, S, ss, v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sq += v[0][e] * v[0][e];
+    }
+    sq = wave_sum(sq);
+    if ((tid & 63) == 0) red[tid >> 6] = sq;
+    __syncthreads();
+    const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)DL + eps);
+    if (slot < 0) return;
+    uint16_t* out = cache + (size_t)slot * (DL + DR);
+    if (tid < nch) {
+      const s16x8 w = ld16(kv_ln + tid * 8);
+      s16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(bf2f(f2bf(v[0][e] * inv)) * bf2f(w[e]));
+      st16(out + tid * 8, o);
+    }
+    return;
+  }
+  uint16_t* qr = q + (size_t)t * ldq;
+  if (role < (int)gridDim.y - 1) {
+    const int c = (role - 1) * MLA_SLAB_COLS + 8 * tid;
+    if (c >= nope) return;
+    const float* at[1] = {row + c};
+    float v[1][8];
+    slab8<1>(at, S, ss, v);
+    s16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(v[0][e]);
+    st16(qr + c, o);
+    return;
+  }
+  const int per = half / 8;
+  for (int w = tid; w < H * per; w += 256) {
+    const int h = w / per;
+    rotate(row + nope + h * DR, 8 * (w - h * per), qr + nope + h * DR);
+  }
+}
+
+int launch_mla_prep_slabs(const float* P, int S, long ss, int N, int nope, const uint16_t* kv_ln, uint16_t* q, long ldq,
+                          const int32_t* pos, const float* cos_sin, const int64_t* slots, uint16_t* cache, int T, int H, int DL,
+                          int DR, int max_pos, long nslots, float eps, hipStream_t s) {
+  if (T <= 0) return 0;
+  // (16-byte loads and stores: rows, slabs, parts and pairs in whole eights)
+  if (N % 8 || ss % 4 || nope % 8 || DL % 8 || DL > 2048 || DR % 16 || DR > 1024 || ldq % 8) return -1;
+  const dim3 grid((unsigned)T, (unsigned)(2 + (nope + MLA_SLAB_COLS - 1) / MLA_SLAB_COLS));
+  mla_prep_slabs_kernel<<<grid, 256, 0, s>>>(P, S, ss, N, nope, kv_ln, q, ldq, pos, cos_sin, slots, cache, H, DL, DR, max_pos,
+                                             nslots, eps);
+  return 0;
+}
+
 // ------------------------------------------------------------------------------------------ attention
 template <int DL>
 __global__ __launch_bounds__(256, 1) void mla_attn_kernel(

@@ -284,16 +284,32 @@ class ShardModel:
     c = self.c
     T = xn.shape[0]
     H, dn, dr, dv, L = c.num_heads, c.qk_nope_head_dim, c.qk_rope_head_dim, c.v_head_dim, c.kv_lora_rank
-    A = linear(xn, lw.qkv_w)
     nq = c.q_lora_rank or H * (dn + dr)
+    cache = self.kv.k[li]
+    # single tokens without a query latent: the norm + rope kernel sums the projection's split-K slabs itself (at more rows the
+    # fp32 slabs cost more than the launch they save)
+    slabs = (not c.q_lora_rank and inp.decode and T <= 128 and not isinstance(xn, PendingNorm) and xn.is_cuda
+             and layout_of(lw.qkv_w) == "stream" and (H * dn) % 8 == 0 and dr % 16 == 0 and L % 8 == 0 and L <= 2048)
+    if slabs:
+      q = torch.empty(T, nq, device=xn.device, dtype=xn.dtype)
+      require().mla_prep_slabs(linear_slabs(xn, lw.qkv_w), H * dn, lw.kv_ln, q, H, inp.positions, self.cos_sin, inp.slots, cache,
+                               float(c.rms_norm_eps))
+      return self._mla_tail(xn, q, lw, li, inp)
+    A = linear(xn, lw.qkv_w)
     if c.q_lora_rank:
       qa, _ = K.rmsnorm(A[:, :nq].contiguous(), lw.q_ln, c.rms_norm_eps)
       q = linear(qa, lw.qb_w)  # [T, H dn | H dr]
     else:
       q = A  # q = A[:, :nq], rows of stride A.shape[1]
     ckv = A[:, nq:]
-    cache = self.kv.k[li]
     K.mla_prep(ckv, lw.kv_ln, q, H * dn, H, inp.positions, self.cos_sin, inp.slots, cache, c.rms_norm_eps)
+    return self._mla_tail(xn, q, lw, li, inp)
+
+  def _mla_tail(self, xn: torch.Tensor, q: torch.Tensor, lw, li: int, inp: StepInputs) -> torch.Tensor:
+    """The absorbed queries, the attention and the values out of the latent (q: rows of [q_nope | rotated q_pe])."""
+    c = self.c
+    T, cache = xn.shape[0], self.kv.k[li]
+    H, dn, dv, L = c.num_heads, c.qk_nope_head_dim, c.v_head_dim, c.kv_lora_rank
     dt = q.dtype
     q_pe = q[:, H * dn:]
     if getattr(lw.wuk, "xot_layout", "rowmajor") == "stream_t":
