@@ -465,7 +465,8 @@ __global__ __launch_bounds__(PF == 2 ? 512 : 256, PF == 2 ? 2 : 1) void attn_dec
 // waves meet in LDS, not in a reduce launch.  A lone wave per unit walked its pages one behind the other (~3 us each) and needed
 // partitions, and their merge launch, to shorten that.  Llama-3-8B heads, ragged contexts, us per layer with the merge, before /
 // now: 24 sequences up to 1407 tokens 24.1 / 21.3, 64 up to 393 18.7 / 15.8, 128 up to 1900 113.5 / 67.4, 64 up to 8000
-// 180 / 159; 256 even ones of 1900 307 / 301 (6.6 TB/s).  Four waves measured ahead of eight (two workgroups a CU overlap one's
+// 180 / 159; 256 even ones of 1900 307 / 301 (6.6 TB/s).  Even batches whose waves fill the chip exactly were the lone wave's
+// best case and are level to 3 % slower (70B heads, 523 tokens: 512 sequences 183 / 183, 256 93 / 94, 128 47.7 / 49.1).  Four waves measured ahead of eight (two workgroups a CU overlap one's
 // start with the other's pages); two where a table of 8 pages leaves most waves of four without one and there are enough units
 // to fill the chip (512 sequences of 33 .. 189 tokens: 50.7 before, 51.4 with four waves, 44.0 with two).
 template <int DH, bool NT, int NW>

@@ -407,7 +407,7 @@ class GemmPolicy:
         and not (epi == "resid" and out_dtype == torch.float32) and M * x.stride(0) * 2 < (1 << 32)):
       # (one column of tiles that leaves CUs idle is tuned like the small shapes; the last term: the tile's LDS-DMA loads take 32-bit byte offsets into X; taller / wider X take the
       # tuned candidates below)
-      # tall GEMMs (prefill chunks, training): the four-wave tile at S = 1 won every tuned tall shape this round
+      # tall GEMMs (prefill chunks, training): the four-wave tile at S = 1 won every tuned tall shape
       # (profiles/r5/headline/bench_r5o_tunelog.log), so it is taken without the cold-timing pass, which cost
       # ~0.5 s inside the first prefill chunk of every fresh process.  (Its row height follows M inside the kernel's
       # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long enough to pay for
