@@ -1,4 +1,4 @@
-"""Decode attention at small batches (latency regime): workgroup kernel (algo 0) vs wave kernel
+"""Decode attention at small batches (latency regime): workgroup kernel (algo 0) vs groups of waves
 (algo 2, and 3 with non-temporal page loads) over partition sizes, each timed as 20 calls replayed from one HIP graph.
 
   python tools/bench_attn_small.py [--json out.json]
