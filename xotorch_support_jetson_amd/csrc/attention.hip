@@ -222,10 +222,12 @@ __global__ __launch_bounds__(DH) void attn_decode_reduce_kernel(const float* __r
 // so that this works with contiguous V^T reads: tile t = 2kk + h, row c = 4q + r holds key
 // 32kk + 8q + 4h + r, hence lane group g of the P^T operand owns keys 32kk + 8g .. +8 and reads one
 // 16-byte run of the transposed V page.  No LDS.
+// PF 1: the next page's K / V go to a second register set under the current page's math (378 registers: one wave per SIMD;
+//       algo 7, and 8 with NT).
 // PF 2: ONE register set, each half refilled as soon as it is consumed -- the next page's K right after the
 //       S^T MFMAs, its V right after the P.V MFMAs -- so a page's loads fly under the other half's math and,
 //       at under 256 registers, two waves per SIMD keep twice the pages in flight per CU (algo 5 / 6).
-// NT: K / V pages loaded non-temporal (read once per step; algo 3 / 6; the workgroup form of algo 2 / 3 follows)
+// NT: K / V pages loaded non-temporal (read once per step; algo 3 / 6 / 8; the workgroup form of algo 2 / 3 follows)
 // NW > 1 (PF 2): the NW waves of a workgroup share the unit, wave w takes pages w, w + NW, ..., and they meet in LDS (sm:
 //       [NW][G][DH + 4] partial sums, then [NW][G][2] maxima and sums)
 template <int DH, int PF, bool NT, int NW = 1>
@@ -370,6 +372,18 @@ __device__ __forceinline__ void decode_wave_unit(
       pv(p, st, vf);
       if (more) load_v(p + NW, nxt, vf);
     }
+  } else if constexpr (PF == 1) {
+    s16x8 ka[4][KS], kb2[4][KS];
+    s16x8 va[NDT][2], vb2[NDT][2];
+    int p = p_begin;
+    if (p < p_end) load(p, ka, va);
+    for (; p + 1 < p_end; p += 2) {
+      load(p + 1, kb2, vb2);
+      compute(p, ka, va);
+      if (p + 2 < p_end) load(p + 2, ka, va);
+      compute(p + 1, kb2, vb2);
+    }
+    if (p < p_end) compute(p, ka, va);
   } else {
     for (int p = p_begin; p < p_end; ++p) {
       s16x8 kf[4][KS], vf[NDT][2];
@@ -517,17 +531,19 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
   }
   if (algo != 0) {  // wave per (sequence, KV head, partition)
     // algo 5 / 6: 8-wave workgroups (two waves per SIMD)
-    const int units = B * Hkv * nparts, wpg = algo >= 5 ? 8 : 4;
+    const int units = B * Hkv * nparts, wpg = algo == 5 || algo == 6 ? 8 : 4;
     const int wgs = (units + wpg - 1) / wpg;
 #define XOT_WAVE(DHV, PFV, NTV)                                                                                  \
   attn_decode_wave_kernel<DHV, PFV, NTV><<<wgs, 64 * wpg, 0, s>>>(q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, \
                                                         ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages, tickets, 1)
-    // algo 1: no prefetch; 5 / 6: one register set refilled per half (6: nt loads)
+    // algo 1: no prefetch; 5 / 6: one register set refilled per half (6: nt loads); 7 / 8: two register sets (8: nt loads)
     if (Dh == 128) {
-      if (algo == 5) XOT_WAVE(128, 2, false); else if (algo == 6) XOT_WAVE(128, 2, true); else XOT_WAVE(128, 0, false);
+      if (algo == 5) XOT_WAVE(128, 2, false); else if (algo == 6) XOT_WAVE(128, 2, true);
+      else if (algo == 7) XOT_WAVE(128, 1, false); else if (algo == 8) XOT_WAVE(128, 1, true); else XOT_WAVE(128, 0, false);
       if (reduce) attn_decode_reduce_kernel<128><<<B * H, 128, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
     } else if (Dh == 64) {
-      if (algo == 5) XOT_WAVE(64, 2, false); else if (algo == 6) XOT_WAVE(64, 2, true); else XOT_WAVE(64, 0, false);
+      if (algo == 5) XOT_WAVE(64, 2, false); else if (algo == 6) XOT_WAVE(64, 2, true);
+      else if (algo == 7) XOT_WAVE(64, 1, false); else if (algo == 8) XOT_WAVE(64, 1, true); else XOT_WAVE(64, 0, false);
       if (reduce) attn_decode_reduce_kernel<64><<<B * H, 64, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
     } else {
       return -1;

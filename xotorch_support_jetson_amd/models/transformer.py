@@ -254,7 +254,7 @@ class ShardModel:
       if c.is_mla:
         self.ws = K.MLAWorkspace(max_batch, c.num_heads, c.kv_lora_rank, max_ctx, self.device)
       else:
-        self.ws = K.DecodeWorkspace(max_batch, c.num_heads, c.head_dim, max_ctx, self.device)
+        self.ws = K.DecodeWorkspace(max_batch, c.num_heads, c.head_dim, max_ctx, self.device, routed=c.num_experts > 0)
     if c.is_mla:
       self.scale = c.attn_scale()
     # last shard with the LM head split across two ring stages: logits of vocab rows [0, head_rows) only,

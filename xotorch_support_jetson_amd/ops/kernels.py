@@ -155,18 +155,24 @@ def rope_apply(x: torch.Tensor, pos: torch.Tensor, cos_sin: torch.Tensor, nh: in
 #    projection's prologue; else 3 once a layer's K / V pages (batch x block-table width) outgrow the 256 MB last-level cache
 #    (256 sequences of 1900 tokens: 301 us, 331 with plain loads), 2 below (24 up to 1407 tokens: 21.3 us, 23.5 with nt).
 #    From 16 pairs on 2 also leads 0: 2 sequences x 8 heads of 130 tokens 6.3 us / 9.1, of 8000 21.0 / 29.8; 6 of 2000 15.0 / 18.8
+# 7 / 8: as 5 / 6 with two register sets, one wave a SIMD.  With routed experts (DecodeWorkspace.routed) -1 is 0 below 64 pairs
+#    and 7 or 8 above: those sum a partition page by page and merge the partitions in order.  2 / 3 deal a context's pages to
+#    waves, sums in another order, no less exact; but a token whose experts are almost tied turns on the last bits, and its whole
+#    row with it.  So routed models keep the order they have always been served with (64 sequences x 8 heads up to 393 tokens:
+#    18.7 us in 8 with its merge, 15.8 in 2)
 DECODE_ALGO = int(os.environ.get("XOT_ATTN_DECODE", "-1"))
 
 
 NT_MIN_KV_BYTES = 256 << 20  # K / V bytes per layer from which the page loads go non-temporal (algo 3)
 
 
-def resolve_decode_algo(batch: int, Hkv: int, algo: int | None = None, kv_bytes: int | None = None) -> int:
+def resolve_decode_algo(batch: int, Hkv: int, algo: int | None = None, kv_bytes: int | None = None,
+                        routed: bool = False) -> int:
   algo = DECODE_ALGO if algo is None else algo
   if algo < 0:
-    if batch * Hkv < 16:
+    if batch * Hkv < (64 if routed else 16):
       return 0
-    return 3 if kv_bytes is None or kv_bytes >= NT_MIN_KV_BYTES else 2
+    return (7 if routed else 2) + int(kv_bytes is None or kv_bytes >= NT_MIN_KV_BYTES)
   return algo
 
 
@@ -202,11 +208,13 @@ def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None =
 
 class DecodeWorkspace:
   """Split-KV scratch for attn_decode, sized for every batch up to max_batch at this context bound.
-  The partitioning is chosen per call from the actual batch (static per captured graph)."""
+  The partitioning is chosen per call from the actual batch (static per captured graph).  routed: the model has routed
+  experts (see DECODE_ALGO)."""
 
   def __init__(self, max_batch: int, H: int, Dh: int, max_ctx: int, device, pages_per_part: int | None = None,
-               algo: int | None = None):
+               algo: int | None = None, routed: bool = False):
     self.algo = DECODE_ALGO if algo is None else algo
+    self.routed = routed
     self.max_ctx = max_ctx
     self.Hkv_hint = None
     self.Dh = Dh
@@ -215,10 +223,11 @@ class DecodeWorkspace:
     worst = 1
     for b in range(1, max_batch + 1):
       for hkv in (1, 2, 4, 8, 16):
-        if pages_per_part is None and resolve_decode_algo(b, hkv, self.algo) in (2, 3):
+        kind = resolve_decode_algo(b, hkv, self.algo, routed=routed)
+        if pages_per_part is None and kind in (2, 3):
           worst = max(worst, b * group_parts(b, hkv, pages))  # (narrower tables have no more partitions)
           continue
-        ppp = pages_per_part or choose_pages_per_part(b, hkv, max_ctx, self.algo)
+        ppp = pages_per_part or choose_pages_per_part(b, hkv, max_ctx, kind)
         worst = max(worst, b * -(-pages // ppp))
     self.units = worst  # max over batch of batch * nparts
     self.o = torch.empty(worst * H * Dh, dtype=torch.float32, device=device)
@@ -226,7 +235,7 @@ class DecodeWorkspace:
 
   def partition(self, batch: int, Hkv: int, width_pages: int):
     """(pages per partition, partitions, kernel) for this call."""
-    algo = resolve_decode_algo(batch, Hkv, self.algo, kv_bytes=batch * Hkv * width_pages * PAGE * self.Dh * 4)
+    algo = resolve_decode_algo(batch, Hkv, self.algo, batch * Hkv * width_pages * PAGE * self.Dh * 4, self.routed)
     ppp = self.fixed_ppp or choose_pages_per_part(batch, Hkv, width_pages * PAGE, algo)
     nparts = max(1, -(-width_pages // ppp))
     if batch * nparts > self.units:
