@@ -1,5 +1,5 @@
 """Decode attention by the waves of a workgroup together (algo 2 / 3): edges of pages, waves without a page, empty contexts,
-partitions, two and four waves, every group size."""
+partitions, one and four waves, every group size."""
 import math
 
 import pytest
@@ -26,7 +26,7 @@ def test_group_kernel(H, Hkv, Dh, width, ppp):
   g = torch.Generator(device="cuda").manual_seed(H + width)
   full = width * 64
   ctx = sorted({1, 63, 64, 65, 128, 129, 255, 257, 511, min(full, 1300), full - 1, full} & set(range(1, full + 1))) + [0]
-  # a step that fills the chip with units (two waves each over short tables), and one that does not
+  # a step that fills the chip with units (one wave each over short tables), and one that does not
   for rep in (1, 1 + 1024 // (Hkv * len(ctx))) if width == 8 and ppp is None else (1,):
     lens = ctx * rep
     B = len(lens)
@@ -50,3 +50,23 @@ def test_group_kernel(H, Hkv, Dh, width, ppp):
       assert float((out[:n1] - want).abs().max()) < 2e-2 * float(want.abs().max()), (algo, rep)
       assert float(out[n1].abs().max()) == 0.0 and bool(torch.isfinite(out).all())
       assert torch.equal(K.attn_decode(q, kc, vc, bt, cl, 1 / math.sqrt(Dh), ws).float(), out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hkv,Dh", [(32, 8, 64), (64, 8, 128), (16, 1, 128)])
+@pytest.mark.parametrize("width", [1, 3, 8])
+def test_short_tables_of_large_batches_take_one_wave_a_unit(H, Hkv, Dh, width):
+  """1024 and more units over at most 8 pages: bit for bit the lone wave without a prefetch (algo 1)."""
+  g = torch.Generator(device="cuda").manual_seed(width)
+  B = 1024 // Hkv
+  cl = torch.randint(0, width * 64 + 1, (B,), generator=g, device="cuda", dtype=torch.int32)
+  pages = 40
+  kc = torch.randn(pages, Hkv, 64, Dh, generator=g, device="cuda").bfloat16()
+  vc = torch.randn(pages, Hkv, Dh, 64, generator=g, device="cuda").bfloat16()
+  bt = torch.randint(0, pages, (B, width), generator=g, device="cuda", dtype=torch.int32)
+  q = torch.randn(B, H, Dh, generator=g, device="cuda").bfloat16()
+  one = K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, K.DecodeWorkspace(B, H, Dh, width * 64, q.device, pages_per_part=width, algo=1))
+  for algo in (2, 3):
+    ws = K.DecodeWorkspace(B, H, Dh, width * 64, q.device, algo=algo)
+    assert ws.partition(B, Hkv, width)[1] == 1
+    assert torch.equal(K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, ws), one)

@@ -476,13 +476,18 @@ __global__ __launch_bounds__(PF == 2 ? 512 : 256, PF == 2 ? 2 : 1) void attn_dec
 }
 
 // The NW waves of a workgroup share one (sequence, KV head, partition): a short context's pages are in flight together and the
-// waves meet in LDS, not in a reduce launch.  A lone wave per unit walked its pages one behind the other (~3 us each) and needed
-// partitions, and their merge launch, to shorten that.  Llama-3-8B heads, ragged contexts, us per layer with the merge, before /
-// now: 24 sequences up to 1407 tokens 24.1 / 21.3, 64 up to 393 18.7 / 15.8, 128 up to 1900 113.5 / 67.4, 64 up to 8000
-// 180 / 159; 256 even ones of 1900 307 / 301 (6.6 TB/s).  Even batches whose waves fill the chip exactly were the lone wave's
-// best case and are level to 3 % slower (70B heads, 523 tokens: 512 sequences 183 / 183, 256 93 / 94, 128 47.7 / 49.1).  Four waves measured ahead of eight (two workgroups a CU overlap one's
-// start with the other's pages); two where a table of 8 pages leaves most waves of four without one and there are enough units
-// to fill the chip (512 sequences of 33 .. 189 tokens: 50.7 before, 51.4 with four waves, 44.0 with two).
+// waves meet in LDS, not in a reduce launch.  A lone wave per unit (algo 7 / 8) walks its pages one behind the other (~3 us each)
+// and needs partitions, and their merge launch, to shorten that.  Bound by the longest context where units are few (one CU takes
+// ~50 GB/s), by HBM where they fill the chip.  Llama-3-8B heads, ragged contexts, us per layer with the merge, lone wave / here:
+// 24 sequences up to 1407 tokens 24.1 / 21.3, 64 up to 393 18.7 / 15.8, 128 up to 1900 114 / 74, 64 up to 8000 180 / 159.
+// Four waves measured ahead of eight (two workgroups a CU overlap one's start with the other's pages).
+// NW 1: tables of at most 8 pages with units enough to fill the chip (1024 and more).  Sharing so few pages leaves waves idle
+// (3 pages are two rounds of two waves), and a workgroup of one wave still frees its place as soon as its context ends.  Lone
+// wave / four / two / one here: 256 sequences x 8 heads of 64, 60 tokens each 9.1 / 12.0 / 9.9 / 8.5 us, 190 19.2 / 20.0 / 21.1
+// / 19.0, 320 29.8 / 32.2 / 33.1 / 31.3; 512 x 8 of 128, 60 tokens 32.8 / 40.0 / 33.5 / 27.6, 33 .. 190 48.4 / 51.3 / 45.0 /
+// 41.6, 448 163 / 165 / 165 / 161.  Longer tables stay at four: even contexts whose units fill the chip exactly are the lone
+// wave's best case and level within the runs (70B heads, 523 tokens: 512 sequences 188 / 190, 256 95.5 / 92.6, 128 48.3 / 48.3;
+// 1000: 512 339 / 341), and ragged ones gain (512 up to 900 tokens 163 / 142, 256 94 / 77; one wave 149, 77).
 template <int DH, bool NT, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attn_decode_group_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
@@ -509,15 +514,15 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
   const float sl = scale * LOG2E;
   if (algo == 2 || algo == 3) {  // NW waves per (sequence, KV head, partition); 3: nt loads
     const int units = B * Hkv * nparts, G = H / Hkv;
-    const bool pair = max_blocks <= 8 && units >= 1024;
-    const size_t lds = (size_t)(pair ? 2 : 4) * G * (Dh + 6) * sizeof(float);  // at most 34 KB
+    const bool lone = max_blocks <= 8 && units >= 1024;
+    const size_t lds = lone ? 0 : (size_t)4 * G * (Dh + 6) * sizeof(float);  // at most 34 KB
 #define XOT_GROUP(DHV, NTV, NWV)                                                                                \
   attn_decode_group_kernel<DHV, NTV, NWV><<<units, 64 * NWV, lds, s>>>(q, kc, vc, block_tables, max_blocks,     \
                                                         ctx_lens, out, ws_o, ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages)
 #define XOT_GROUP_DH(DHV)                                                                                       \
   do {                                                                                                          \
-    if (pair && algo == 3) XOT_GROUP(DHV, true, 2);                                                             \
-    else if (pair) XOT_GROUP(DHV, false, 2);                                                                    \
+    if (lone && algo == 3) XOT_GROUP(DHV, true, 1);                                                             \
+    else if (lone) XOT_GROUP(DHV, false, 1);                                                                    \
     else if (algo == 3) XOT_GROUP(DHV, true, 4);                                                                \
     else XOT_GROUP(DHV, false, 4);                                                                              \
     if (reduce) attn_decode_reduce_kernel<DHV><<<B * H, DHV, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part); \

@@ -150,7 +150,8 @@ def rope_apply(x: torch.Tensor, pos: torch.Tensor, cos_sin: torch.Tensor, nh: in
 # 0: workgroup per (sequence, KV head, partition), waves split pages + LDS combine (scores by rows, P through LDS)
 # 1: wave per (sequence, KV head, partition), transposed S^T (lane = query head), no LDS; 5 / 6: the same with the next page's
 #    loads under the current one (6: non-temporal)
-# 2 / 3: four (or two) waves per (sequence, KV head, partition), each as in 5, meeting in LDS; 3 with non-temporal K / V loads
+# 2 / 3: four waves per (sequence, KV head, partition), each as in 5, meeting in LDS (one over short tables at large batches); 3
+#    with non-temporal K / V loads
 # -1 (default): 0 below 16 (sequence, KV head) pairs, where the partitions of a single sequence are merged by the output
 #    projection's prologue; else 3 once a layer's K / V pages (batch x block-table width) outgrow the 256 MB last-level cache
 #    (256 sequences of 1900 tokens: 301 us, 331 with plain loads), 2 below (24 up to 1407 tokens: 21.3 us, 23.5 with nt).
