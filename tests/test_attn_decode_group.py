@@ -70,3 +70,13 @@ def test_short_tables_of_large_batches_take_one_wave_a_unit(H, Hkv, Dh, width):
     ws = K.DecodeWorkspace(B, H, Dh, width * 64, q.device, algo=algo)
     assert ws.partition(B, Hkv, width)[1] == 1
     assert torch.equal(K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, ws), one)
+
+
+def test_partitions_leave_at_most_one_unit_a_cu():
+  """Contexts of up to 64 pages are cut only while (sequence, KV head, partition) units do not outnumber the 256 CUs."""
+  for batch in range(1, 128):
+    for hkv in (1, 2, 3, 8, 16):
+      for pages in (1, 8, 9, 16, 32, 64):
+        parts = K.group_parts(batch, hkv, pages)
+        assert parts == 1 or batch * hkv * parts <= 256
+        assert parts <= -(-pages // 4)

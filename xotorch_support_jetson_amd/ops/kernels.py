@@ -182,7 +182,7 @@ def group_parts(batch: int, Hkv: int, pages: int) -> int:
   pairs = max(batch * Hkv, 1)
   if pages <= 8:
     return 1
-  return min(max(round(256 / pairs), 2 if pages > 64 and pairs < 384 else 1), -(-pages // 4))
+  return min(max(256 // pairs, 2 if pages > 64 and pairs < 384 else 1), -(-pages // 4))
 
 
 def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None = None) -> int:
@@ -196,9 +196,10 @@ def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None =
     return 4
   if algo in (2, 3):
     # four waves per unit (csrc/attention.hip attn_decode_group_kernel): a context of 8 pages is two pages a wave and best left
-    # whole; longer ones are cut until the units cover the CUs, in partitions of at least 4 pages (8 sequences x 8 heads, up to
-    # 1900 tokens: 20.4 us whole, 13.9 in 4; 16: 21.7, 18.0 in 2, 19.5 in 4; 24: 21.3 whole, 23.0 in 2), and very long ones
-    # once more, since the longest workgroup ends the launch (32 sequences up to 7800 tokens: 100 us whole, 87 in 2)
+    # whole; longer ones are cut while the units stay within one a CU, in partitions of at least 4 pages (8 sequences x 8 heads, up
+    # to 1900 tokens: 20.4 us whole, 13.9 in 4; 16: 21.7, 18.0 in 2, 19.5 in 4; 24: 21.3 whole, 23.0 in 2; more units than CUs
+    # share some CUs, and those end the launch: 12 of 900 tokens 19.1 in 3, 15.2 in 2; 20 of 523 20.6 in 2, 13.7 whole), and very
+    # long ones once more, since the longest workgroup ends the launch (32 sequences up to 7800 tokens: 100 us whole, 87 in 2)
     return -(-pages // group_parts(batch, Hkv, pages))
   # one wave per unit: ~1024 waves (4 per CU), partitions of 2..32 pages (tools/bench_attn_small.py,
   # profiles/bench_attn_small_r1.json: 2048 waves of shorter partitions lose to the extra merge work)
