@@ -94,3 +94,44 @@ def test_chunk_rule_keeps_what_it_cannot_take(gpu):
       got.append((out, S))
     for one, other in zip(*got):
       torch.testing.assert_close(one, other, rtol=0, atol=float(2e-6 * one.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule", list(RULES))
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "decay", "beta"])
+def test_a_value_that_is_no_number_reaches_no_earlier_token(gpu, rule, value, where):
+  """Outputs before the token that holds it are those without it, and later ones are numbers wherever the recurrence token by
+  token gives numbers (other channels, other heads, the other sequence)."""
+  channel, delta, scaled, norm = RULES[rule]
+  if where == "beta" and not (delta or scaled):
+    pytest.skip("the rule has no input scale")
+  g = torch.Generator().manual_seed(len(rule) + len(where))
+  rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+  H, d, dv, lens = 2, 64, 40, [117, 100]
+  T, dvs, t = sum(lens), dv + norm, 44  # token 12 of the first sequence's third chunk
+  q, k, v, a = rn(T, H, d), rn(T, H, d), rn(T, H, dv), torch.rand(T, H, d if channel else 1, generator=g) * 0.2 + 0.8
+  k = k / k.norm(dim=-1, keepdim=True)
+  beta = torch.rand(T, H, generator=g) if delta or scaled else None
+  bad = {"q": q, "k": k, "v": v, "decay": a, "beta": beta}
+  one = {n: None if x is None else x.clone() for n, x in bad.items()}
+  one[where][t, 1, ...] = value if where == "beta" else one[where][t, 1]
+  if where != "beta":
+    one[where][t, 1, 0] = value
+
+  def run(x):
+    S, out = torch.zeros(2, H, dvs, d, device=gpu), torch.empty(T, H * dvs, device=gpu)
+    K.linear_recurrence(*(x[n].reshape(T, -1).to(gpu) for n in ("q", "k", "v", "decay")),
+                        None if beta is None else x["beta"].to(gpu), 0.7, S, torch.tensor([0, 1], dtype=torch.int32, device=gpu),
+                        torch.tensor([0, lens[0], T], dtype=torch.int32, device=gpu), out, plain=scaled and not norm, max_qlen=117)
+    return out.cpu().view(T, H, dvs)
+  clean, got = run(bad), run(one)
+  torch.testing.assert_close(got[:t], clean[:t], rtol=0, atol=float(2e-6 * clean[:t].abs().max()))
+  assert torch.equal(got[:, 0], clean[:, 0]) and torch.equal(got[lens[0]:], clean[lens[0]:])
+  want, _ = token_by_token(*(one[n][:lens[0]] for n in ("q", "k", "v", "decay")), None if beta is None else one["beta"][:lens[0]],
+                           0.7, torch.zeros(H, dvs, d, dtype=F64), rule, H)
+  number = torch.isfinite(want)
+  assert not number[t].all()
+  diff = torch.where(number, got[:lens[0]].to(F64) - want, torch.zeros((), dtype=F64)).abs().max()
+  assert diff < 1e-5 * want[number].abs().max()
+  assert not torch.isfinite(got[:lens[0]][~number]).any()

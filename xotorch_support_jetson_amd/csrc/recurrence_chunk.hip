@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
   }
 #pragma unroll
   for (int row = 0; row < CT; ++row)
-    if ((row >> 2) == g) M[row * CT + i] = x[row] * bi;
+    if ((row >> 2) == g) M[row * CT + i] = row >= i ? x[row] * bi : 0.0f;  // (selected: bi may be no number)
 }
 
 // buffer over `bytes` from p on: loads past the end give 0, stores past it are dropped
@@ -338,6 +338,29 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
+  // c + L b, L lower triangular (lane: row i of L, tokens 4 g + r; row r of b and c: token 4 g + r).  The products with the zeros
+  // above its diagonal would carry an infinity or a NaN of b back to earlier tokens: such a chunk sums what is below alone
+  // (all lanes of the wave; no memory operation, so that the loads in flight are waited for as without it).
+  auto lower = [&](f32x4 l, f32x4 b, f32x4 c) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) top = max(top, __float_as_uint(b[r]) & 0x7fffffffu);
+    if (__builtin_expect(__any(top >= 0x7f800000u), 0)) {
+#pragma unroll
+      for (int m = 0; m < CT; ++m) {
+        const float bm = __shfl(b[m & 3], (m >> 2) * 16 + i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float lm = __shfl(l[m & 3], (m >> 2) * 16 + 4 * g + r);
+          c[r] = m <= 4 * g + r ? c[r] + lm * bm : c[r];
+        }
+      }
+      return c;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c = mfma4(l[r], b[r], c);
+    return c;
+  };
   Share sh[RING];
   Wave wv[RING];
 #pragma unroll
@@ -388,16 +411,13 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
       f32x4 R;
 #pragma unroll
       for (int r = 0; r < 4; ++r) R[r] = U[r] - (CHAN ? X[r] : cur.p[r] * X[r]);
-      U = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int r = 0; r < 4; ++r) U = mfma4(cur.m[r], R[r], U);
+      U = lower(cur.m, R, f32x4{0.f, 0.f, 0.f, 0.f});
     }
     if (!CHAN) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) Y[r] *= cur.p[r];
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) Y = mfma4(cur.nn[r], U[r], Y);
+    Y = lower(cur.nn, U, Y);
     f32x4 E = U;
     if (!CHAN) {
 #pragma unroll
