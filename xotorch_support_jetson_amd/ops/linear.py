@@ -20,9 +20,11 @@ eagerly first, so the timed choice is normally cached).  Row-major GPU weights u
 """
 from __future__ import annotations
 
+import contextlib
 import json
 import os
 import sys
+import threading
 from typing import Dict, Tuple
 
 import torch
@@ -134,14 +136,26 @@ class _Scratch:
   bucket 1, then grew the slabs for bucket 64, faulted exactly that way)."""
 
   def __init__(self):
-    self.ws: Dict[int, torch.Tensor] = {}
+    self.ws: Dict[Tuple, torch.Tensor] = {}
     self.retired: list = []
+    self._own = threading.local()
+
+  @contextlib.contextmanager
+  def apart(self, name: str):
+    """The calling thread's GEMMs inside take slabs of their own: work on a side stream, which nothing orders between another
+    stream's GEMM and the reduce of its slabs."""
+    old = getattr(self._own, "name", "")
+    self._own.name = name
+    try:
+      yield
+    finally:
+      self._own.name = old
 
   def splitk(self, device, n: int, slot: int = 0) -> torch.Tensor:
     """slot 1 holds the slabs of a residual projection whose reduce is deferred into the next GEMM (PendingNorm),
     which writes its own slabs to slot 0 while it still reads slot 1, or those of the second of two projections whose
     slabs one kernel sums."""
-    key = (device.index or 0, slot)
+    key = (device.index or 0, slot, getattr(self._own, "name", ""))
     t = self.ws.get(key)
     if t is None or t.numel() < n:
       if torch.cuda.is_current_stream_capturing():

@@ -459,7 +459,8 @@ def own_dw(dy: torch.Tensor, x: torch.Tensor, acc: "GradAcc", cb: bool = True) -
     return
   side = _dw_stream(dy.device)
   side.wait_stream(torch.cuda.current_stream(dy.device))  # dy and x are ready
-  with torch.cuda.stream(side):
+  from ..ops.linear import scratch
+  with torch.cuda.stream(side), scratch.apart("dw"):
     _dw(dy, x, acc)
   dy.record_stream(side)  # allocated on the main stream, read by the side stream: no reuse before it ran
   x.record_stream(side)
