@@ -113,6 +113,34 @@ def test_tall_gemms_take_the_four_wave_tile_untimed(monkeypatch):
   assert pol2.shuffled_cfg(x, w, None, None, "none", torch.bfloat16)[0] == "big"
 
 
+def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
+  """Two K halves where 256-row tiles fill at most half the CUs, whatever M of the bucket came before: from K 8192 for a caller
+  whose residual norm sums the slabs, from 24576 for those that pay a reduce launch."""
+  monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: False)
+  sized = []
+  monkeypatch.setattr(L.scratch, "splitk", lambda dev, n, slot=0: sized.append(n))
+
+  def splits(pol, M, N, Kd, epi="none", **kw):
+    x, w = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta"), torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
+    kind, code, S = pol.shuffled_cfg(x, w, None, None, epi, torch.bfloat16, **kw)
+    assert (kind, code) == ("big", 4256)
+    return S
+  for N, last in ((4096, 2048), (5120, 1536), (6144, 1280)):
+    for Ms in ((1100, 2048), (2048, 1100)):
+      pol = L.GemmPolicy()
+      for M in Ms:
+        half = M <= last
+        assert splits(pol, M, N, 14336, "resid", norm=True) == (2 if half else 1)
+        assert splits(pol, M, N, 14336, "resid") == 1
+        for epi in ("none", "resid"):
+          assert splits(pol, M, N, 24576, epi) == (2 if half else 1)
+        assert splits(pol, M, N, 4096, "resid", norm=True) == 1
+      assert not any(k[0].startswith("sh") and k[1] == 2048 and k[2] == N for k in pol.table)
+  assert sized and max(sized) == 2 * 2048 * 4096
+  monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: True)  # under capture: nothing to size
+  assert splits(L.GemmPolicy(), 2048, 4096, 28672) == 1
+
+
 def test_seed_table_parses_and_loads_under_the_box_table(tmp_path):
   """ops/gemm_seed_mi355x.json: comment keys skipped, the headline decode picks load, and a key the box tuned itself
   keeps the box's choice (the seed only fills gaps)."""

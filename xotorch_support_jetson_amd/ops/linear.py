@@ -400,10 +400,10 @@ class GemmPolicy:
       return []
     return [("wave", nt, 1) for nt in ((2,) if rope else (2, 4) if epi in K.GLU_EPI else (1, 2, 4)) if N % (16 * nt) == 0]
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "") -> Tuple:
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", norm: bool = False) -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
-    reduce, timed with them, stands for the launch that does it there)."""
+    reduce, timed with them, stands for the launch that does it there).  norm: the caller's residual norm sums the slabs."""
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WAVE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
@@ -419,22 +419,20 @@ class GemmPolicy:
       return got
     if (TALL_FIXED and W4 and M >= W4_PREF_M and N % 256 == 0 and Kd % 128 == 0 and (N > 256 or -(-M // 256) >= 256)
         and not (epi == "resid" and out_dtype == torch.float32) and M * x.stride(0) * 2 < (1 << 32)):
-      # (one column of tiles that leaves CUs idle is tuned like the small shapes; the last term: the tile's LDS-DMA loads take 32-bit byte offsets into X; taller / wider X take the
-      # tuned candidates below)
+      # (one column of tiles that leaves CUs idle is tuned like the small shapes; the last term: the tile's LDS-DMA loads take
+      # 32-bit byte offsets into X; taller / wider X take the tuned candidates below)
       # tall GEMMs (prefill chunks, training): the four-wave tile at S = 1 won every tuned tall shape
       # (profiles/r5/headline/bench_r5o_tunelog.log), so it is taken without the cold-timing pass, which cost
       # ~0.5 s inside the first prefill chunk of every fresh process.  (Its row height follows M inside the kernel's
       # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long enough to pay for
       # the fp32 slabs: ~65 us at 2048 x 4096 with a reduce launch, from K ~ 24576 (28672: 369 us against 427 with 128-row
       # tiles; 14336: about level; 4096: 74 against 58); ~30 where the residual norm that follows sums them, from K ~ 8192.
-      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576)
-      got = ("big", 4256, 2 if half else 1)
-      if got[2] > 1:
-        if self._no_tuning():
-          return ("big", 4256, 1)  # (the slabs are sized outside a capture)
-        scratch.splitk(x.device, _ws_elems(got, M, N))
-      self._store(key, got)
-      return got
+      # Not stored: the halves follow this M, a table entry would answer for its whole bucket.
+      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if norm else 24576)
+      if half and not self._no_tuning():  # (the slabs are sized outside a capture)
+        scratch.splitk(x.device, 2 * M * N)
+        return ("big", 4256, 2)
+      return ("big", 4256, 1)
     cands = []
     if M <= STREAM_MAX_M and epi != "gelu_glu":
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
@@ -778,14 +776,14 @@ def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: t
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype)
+    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype, norm=h.is_contiguous())
     if (defer_to is not None and FUSE_NORM and M == 1 and cfg[0] == "stream" and 1 < cfg[2] <= 8 and N <= DEFER_MAX_D
         and out is None and h.is_contiguous() and h.dtype == torch.bfloat16):
       S = cfg[2]
       ws = scratch.splitk(x.device, S * M * N, slot=1)
       require().gemm_stream(x, w, h, None, h, ws, K.EPI["resid"], cfg[1], S, True, False)
       return PendingNorm(h, defer_to, ws, S, bias, ln_w, eps)
-    if cfg[0] in ("stream", "big") and cfg[2] > 1:
+    if cfg[0] in ("stream", "big") and cfg[2] > 1 and (M < W4_PREF_M or h.is_contiguous()):
       S = cfg[2]
       ws = scratch.splitk(x.device, S * M * N)
       C = require()
