@@ -141,6 +141,17 @@ def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
   assert splits(L.GemmPolicy(), 2048, 4096, 28672) == 1
 
 
+def test_untuned_choice_without_stream_candidates(monkeypatch):
+  """The GELU pair epilogue is built for the tall tiles alone: a choice without a timing pass takes one of them at any row count."""
+  monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: True)
+  w = torch.empty(512, 256, dtype=torch.bfloat16)
+  for M in (L.BIG_MIN_M, 100, 128, 129, 700):
+    x = torch.empty(M, 256, dtype=torch.bfloat16)
+    got = L.GemmPolicy().shuffled_cfg(x, w, None, None, "gelu_glu", torch.bfloat16)
+    assert got[0] == "big" and got[1] in (2256, 128, 4256)
+    assert L.GemmPolicy().shuffled_cfg(x, w, None, None, "none", torch.bfloat16)[0] == ("stream" if M <= 128 else "big")
+
+
 def test_seed_table_parses_and_loads_under_the_box_table(tmp_path):
   """ops/gemm_seed_mi355x.json: comment keys skipped, the headline decode picks load, and a key the box tuned itself
   keeps the box's choice (the seed only fills gaps)."""

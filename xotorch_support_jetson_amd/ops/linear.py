@@ -464,7 +464,8 @@ class GemmPolicy:
   def _heuristic(M, N, cands):
     if not any(c[0] in ("big", "stream") for c in cands):
       return cands[0]
-    if M <= 128 or not any(c[0] == "big" for c in cands):
+    kinds = {c[0] for c in cands}
+    if "stream" in kinds and (M <= 128 or "big" not in kinds):
       best = None  # stream GEMM: enough workgroups to cover 256 CUs a few times
       for c in cands:
         if c[0] != "stream":
