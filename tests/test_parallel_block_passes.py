@@ -107,3 +107,14 @@ def test_slots_are_cleared_in_runs():
   Pool(ts).clear([7, 2, 3, 0, 8])
   for t in ts:
     assert [int(r.abs().sum() > 0) for r in t] == [0, 1, 0, 0, 1, 1, 1, 0, 0]
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_delta_rule_inputs_of_an_empty_step(dev):
+  H, G, d, dv, taps = 2, 1, 8, 16, 3
+  C = 2 * G * d + H * dv
+  e = lambda *s: torch.empty(*s, device=dev)  # noqa: E731
+  state = torch.ones(1, taps - 1, C, device=dev)
+  K.delta_prep(e(0, C + 2 * H), 0, C, C + H, e(C, taps), state, torch.empty(0, dtype=torch.int32, device=dev),
+               torch.zeros(1, dtype=torch.int32, device=dev), e(H), e(H), H, G, d, dv, e(0, C), e(0, H), e(0, H))
+  assert bool((state == 1).all())

@@ -516,7 +516,7 @@ def delta_prep(P, x_off: int, b_off: int, a_off: int, conv_w, conv_state, state_
   q = unit(silu(conv q)) d^-1/2, k = unit(silu(conv k)), v = silu(conv v) -> qkv [T, C]; beta and decay: delta_gates.  (A model
   step calls conv_prep with the units that its weights hold on the device.)"""
   units, width = ref.conv_units(ref.delta_units(H, G, d, dv), conv_w.shape[0])
-  conv_prep(P, x_off, conv_w, None, units.to(P.device), None, conv_state, state_slots, cu_q, 0.0, qkv.view(P.shape[-2], -1),
+  conv_prep(P, x_off, conv_w, None, units.to(P.device), None, conv_state, state_slots, cu_q, 0.0, qkv.view(P.shape[-2], conv_w.shape[0]),
             width=width, delta=(b_off, a_off, dt_bias, A_log, beta, decay))
 
 
