@@ -73,3 +73,13 @@ def test_gelu_mul_of_tiles(dev, T, F, off, pad):
     K.gelu_mul(P.to(dev), off, -1, F, got)
     K.gelu_mul(gu.reshape(T, 2 * n).to(dev), 0, n, F, want)
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_gelu_mul_refuses_columns_outside_the_projection():
+  from xotorch_support_jetson_amd.ops import kernels as K
+  P, out = torch.zeros(2, 64, device="cuda"), torch.zeros(2, 16, device="cuda")
+  for gate, up in ((0, -2), (0, -16), (-1, 16), (0, 49), (33, -1)):
+    with pytest.raises(RuntimeError):
+      K.gelu_mul(P, gate, up, 16, out)
+  K.gelu_mul(P, 32, -1, 16, out)

@@ -123,7 +123,7 @@ __global__ __launch_bounds__(256) void embed_rows_k(const IT* __restrict__ ids, 
 }
 
 // ------------------------------------------------------------------ gelu_tanh(gate) * up
-// up_off < 0: gate and up columns alternate in tiles of 16 from gate_off on.  W columns per thread: memory-bound, so float4
+// up_off -1: gate and up columns alternate in tiles of 16 from gate_off on.  W columns per thread: memory-bound, so float4
 // where the rows allow it.
 template <typename AT, int W>
 __global__ __launch_bounds__(256) void gelu_mul_k(const float* __restrict__ P, int ldp, int gate_off, int up_off, int F,
@@ -898,7 +898,7 @@ void gelu_mul(const at::Tensor& P, int64_t gate_off, int64_t up_off, int64_t F, 
   MCHECK(out.is_cuda() && is_act(out) && out.dim() == 2 && out.size(0) == T && out.size(1) >= F && out.stride(1) == 1,
          "out must be [T, >= F] rows");
   const int ldo = (int)out.stride(0);
-  const bool tiles = up_off < 0;
+  const bool tiles = up_off == -1;
   cols_ok(P, gate_off, tiles ? (F + 15) / 16 * 32 : F, "gate");
   if (!tiles) cols_ok(P, up_off, F, "up");
   if (T * F == 0) return;

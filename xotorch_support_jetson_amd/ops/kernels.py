@@ -485,7 +485,7 @@ def embed_rows(ids, table, want_ids: bool = False):
 
 
 def gelu_mul(P, gate_off: int, up_off: int, F: int, out) -> None:
-  """out[:, :F] = gelu_tanh(P[:, gate_off : +F]) * P[:, up_off : +F]  (out rows may be wider: K padding).  up_off < 0: gate and
+  """out[:, :F] = gelu_tanh(P[:, gate_off : +F]) * P[:, up_off : +F]  (out rows may be wider: K padding).  up_off -1: gate and
   up columns alternate in tiles of 16 from gate_off on."""
   _mix("gelu_mul", _gpu(P))(P, int(gate_off), int(up_off), int(F), out)
 

@@ -247,7 +247,7 @@ def resid_scale_norm(x, y1, s1, y2, s2, gain, eps, out):
 
 
 def gelu_mul(P, gate_off, up_off, Fd, out):
-  if up_off < 0:
+  if up_off == -1:
     n = -(-Fd // 16)
     t = P[:, gate_off:gate_off + 32 * n].float().reshape(-1, n, 2, 16)
     z, u = t[:, :, 0].reshape(-1, 16 * n)[:, :Fd], t[:, :, 1].reshape(-1, 16 * n)[:, :Fd]
