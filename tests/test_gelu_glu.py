@@ -83,3 +83,39 @@ def test_gelu_mul_refuses_columns_outside_the_projection():
     with pytest.raises(RuntimeError):
       K.gelu_mul(P, gate, up, 16, out)
   K.gelu_mul(P, 32, -1, 16, out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ff", [192, 130, 640])
+@pytest.mark.parametrize("T", [65, 300, 1030])
+def test_parallel_block_in_two_products(ff, T, monkeypatch):
+  """The gate / up rows at the end of a parallel block's fused projection in a GEMM of their own (long steps), and one GEMM with
+  the pass over its result, against float64: the other columns, the activation, its zero K padding."""
+  import types
+
+  from xotorch_support_jetson_amd.models import config, transformer, weights
+  from xotorch_support_jetson_amd.ops import linear as L
+  c = config.from_hf_config(dict(config.TINY_TAREPEL, layers=[dict(config.TINY_TAREPEL["layers"][0], mlp={"kind": "dense", "ff": ff})]))
+  get = {k: v.bfloat16().float() for k, v in weights.random_mixed_tensors(c, ff).items()}.__getitem__
+  lw = weights.build_mixed_layer(c.layer_specs[0], get, "l0.", 128, "cuda", torch.bfloat16)
+  lw.in_w = L.to_stream_layout(lw.in_w)
+  assert L.layout_of(lw.in_w) == "stream"
+  x = torch.randn(T, 128, generator=torch.Generator().manual_seed(T)).bfloat16()
+  epis, real = [], transformer.linear
+  monkeypatch.setattr(transformer, "linear", lambda *a, **k: (epis.append(k.get("epi")), real(*a, **k))[1])
+  z, u = (x.double() @ get(f"l0.mlp.{n}").double().T for n in ("gate", "up"))
+  want = 0.5 * z * (1 + torch.tanh(0.7978845608028654 * (z + 0.044715 * z ** 3))) * u
+  for split in (True, False):
+    monkeypatch.setattr(transformer, "GELU_EPI_ROWS", 1 if split else T + 1)
+    monkeypatch.setattr(transformer, "GELU_EPI_SIZE", 1)
+    P, act = transformer.ShardModel._in_and_act(
+      types.SimpleNamespace(_proj=transformer.ShardModel._proj), x.cuda(), lw,
+      lambda name, live, padded: torch.zeros(T, padded, dtype=torch.bfloat16, device="cuda"))
+    P, act = P.cpu().double(), act.cpu().double()
+    assert epis.count("gelu_glu") == 1
+    assert act.shape[1] == lw.down_w.shape[1] >= ff and bool((act[:, ff:] == 0).all())
+    # half a bf16 step (2^-9) of the value, and fp32 sums of 128 products in front of it
+    assert bool(((act[:, :ff] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max()).all())
+    for name, w in weights.mixed_layer_names(c.layer_specs[0], "l0.")["in"]:
+      (o, n), ref = lw.cols[name], x.double() @ get(w).double().T
+      assert o + n <= lw.cols["gate_up"][0] and bool(((P[:, o:o + n] - ref).abs() <= 1e-5 * ref.abs().max()).all())
