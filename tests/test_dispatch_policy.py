@@ -10,16 +10,16 @@ def test_decode_partition_defaults():
   ws = K.DecodeWorkspace(512, 64, 128, 8192, torch.device("cpu"), algo=-1)
   # few (sequence, KV head) pairs: 4-wave workgroups over 4-page partitions, merged by the reduce launch
   assert ws.partition(1, 8, 32) == (4, 8, 0)
-  # many pairs: one wave per unit with page prefetch
+  # many pairs: the waves of a workgroup share a unit
   ppp, nparts, algo = ws.partition(512, 8, 9)
-  assert algo == 3 and ppp * nparts >= 9  # one wave per unit, page prefetch, non-temporal page loads
+  assert algo == 3 and ppp * nparts >= 9  # non-temporal page loads
 
 
 
 def test_decode_partition_small_batch():
   ws = K.DecodeWorkspace(8, 32, 128, 4096, torch.device("cpu"), algo=-1)
   assert ws.partition(1, 8, 16)[2] == 0 and ws.partition(1, 8, 32)[2] == 0  # the workgroup kernel, split
-  assert ws.partition(8, 8, 8)[2] == 2  # 64 pairs: the wave kernel (cache-resident pages: plain loads)
+  assert ws.partition(8, 8, 8)[2] == 2  # 64 pairs: shared units (cache-resident pages: plain loads)
   assert K.DecodeWorkspace(64, 32, 128, 8192, torch.device("cpu"), algo=-1).partition(64, 8, 128)[2] == 3  # 2 GB: nt
   fixed = K.DecodeWorkspace(8, 32, 128, 4096, torch.device("cpu"), pages_per_part=4, algo=-1)
   assert fixed.partition(1, 8, 16)[2] == 0  # an explicit partition size is honoured
@@ -101,7 +101,8 @@ def test_tuner_prefers_four_wave_tile_on_tall_gemms(monkeypatch):
 
 
 def test_tall_gemms_take_the_four_wave_tile_untimed(monkeypatch):
-  """M >= W4_PREF_M: ('big', 4256, 1) straight away (no cold-timing pass inside the first prefill chunk), except a
+  """M >= W4_PREF_M: ('big', 4256, 1) straight away (no cold-timing pass inside the first prefill chunk; two K halves of a
+  long K: below), except a
   residual epilogue into fp32 (the tile has none); XOT_GEMM_TALL_TUNE=1 times them again."""
   pol = L.GemmPolicy()
   x, w = torch.empty(4096, 1024, dtype=torch.bfloat16), torch.empty(2048, 1024, dtype=torch.bfloat16)

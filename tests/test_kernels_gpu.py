@@ -218,8 +218,8 @@ def test_attn_decode(gpu, H, Hkv, Dh, ctx):
   q = torch.randn(B, H, Dh, device=gpu, dtype=torch.bfloat16)
   scale = 1 / math.sqrt(Dh)
   ref = R.attn_decode(q, kc, vc, bt, cl, scale)
-  for algo in (0, 1, 2, 3, 5, 6):  # workgroup kernel; wave kernel without / with page prefetch (2 / 3: double
-    # register set, 5 / 6: one set refilled per half), + nt loads
+  for algo in (0, 1, 2, 3, 5, 6, 7, 8):  # workgroup kernel; wave kernel without / with page prefetch (5 / 6: one register set
+    # refilled per half, 7 / 8: two); 2 / 3: four waves of 5 sharing a unit's pages; 3, 6, 8: nt loads
     for ppp in (1, 3, 4, 8, None):  # None: per-call choice from the batch
       if algo == 0 and ppp in (1, 3):
         continue
@@ -233,7 +233,7 @@ def test_attn_decode(gpu, H, Hkv, Dh, ctx):
 @pytest.mark.parametrize("H,Hkv,Dh", [(32, 8, 128), (32, 8, 64), (14, 2, 64)])
 @pytest.mark.parametrize("ctx", [[700, 65, 1, 1024], [1], [512, 3]])
 def test_attn_decode_auto_short_table(gpu, H, Hkv, Dh, ctx):
-  """The default choice at small batch over a short block table (the workgroup kernel below 64 (sequence, KV head)
+  """The default choice at small batch over a short block table (the workgroup kernel below 16 (sequence, KV head)
   pairs) against the fp32 reference."""
   torch.manual_seed(1)
   B, maxb = len(ctx), 16

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
         // the read-ahead (NR reads, consumption order) and the v half-1 reads issued since: MFMA v <= MI needs
         // read-ahead v + 1 (w0 + x_v, then w1) -> at most NR + v - (v + 2) = MI + 6 younger reads in flight; w2 at MFMA
         // 2 MI: NR + 2 MI issued, at most 15 in flight leaves 3 MI - 7 >= MI + 3 done (MI >= 5; 128 rows: the exact
-        // count 12); from MFMA NR on 15 in flight means 2 NR - 15 done, which covers w3 .. up to barrier 1's
+        // count 13); from MFMA NR on 15 in flight means 2 NR - 15 done, which covers w3 .. up to barrier 1's
         // lgkmcnt(0) where the tile is 256 rows high (all 16), and each w_j at j MI needs MI + 1 + j reads: counted
         // again at 3 MI for the short tiles, whose half-1 reads end at MFMA NR
         if constexpr (v <= MI) wait_lgkm<MI + 6>();
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
         if constexpr (!(W4_ABL & 4) && v >= H + B2 && (v - H - B2) % RSP == 0 && v < H + B2 + NR * RSP)
           rd(buf ^ 1, 0, (v - H - B2) / RSP);
         if constexpr (!(W4_ABL & 1) && v >= B1 && v < H + B2) {
-          static_for<NR>([&](auto kc) {  // refill DMA k after MFMA B1 + ((k + 1) SPAN) / 16 - 1
+          static_for<NR>([&](auto kc) {  // refill DMA k after MFMA B1 + ((k + 1) SPAN) / NR - 1
             constexpr int k = decltype(kc)::value;
             if constexpr ((DGAP ? B1 + DGAP * k : B1 + ((k + 1) * SPAN) / NR - 1) == v) issue(tr, buf, k);
           });

@@ -1127,8 +1127,8 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
   // Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
   // its 1.4 us a chunk (2.2 with channel decays) beat 0.2 us a token, whatever the other sequences of the step do.  us before / after,
-  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 191, 8 of 961 .. 2431 1018 / 419, 30 single tokens and one
-  // prompt of 500 131 / 92, one of 33 11 / 15; channel decays 498 / 299, 1124 / 565, 229 / 122, 14 / 20.
+  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 196, 8 of 961 .. 2431 1018 / 425, 30 single tokens and one
+  // prompt of 500 131 / 95, one of 33 11 / 15; channel decays 498 / 308, 1124 / 574, 229 / 132, 14 / 20.
   // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
   const int64_t widest = std::max(std::max<int64_t>(ldq, ldk), std::max<int64_t>(std::max<int64_t>(ldv, H * dv), H * d));
   if ((d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && on16(q, ldq) &&

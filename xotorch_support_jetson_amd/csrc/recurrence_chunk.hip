@@ -18,11 +18,11 @@
 //     pass LDS once per workgroup, two chunks ahead in registers.
 // Bound by that chain: about 1.4 us a chunk at D 128 where 56 MFMAs of 32 cycles are 0.75 (the rest: two barriers, LDS
 // reads and the four-step products with M and N between them).  Tarepel-design prompts (8 of 961 .. 2431 tokens, 16 heads
-// of 128 x 128): 1018 -> 419 us, delta rule with channel decays 1124 -> 565.
+// of 128 x 128): 1018 -> 425 us, delta rule with channel decays 1124 -> 574.
 // v_mfma_f32_16x16x4_f32 multiplies and accumulates in fp32 as the vector units do; no operand is rounded.
 //
-// Decays per key channel: q P and k / P stay within 2^+-100 or the chunk takes exact pairwise products instead (a decay of 0,
-// above 1 or not a number is among those), so no ratio of vanishing products is formed.
+// Decays per key channel: where a prefix product P leaves 2^-100 .. 2^100 (a decay of 0, or a value that is no number, among
+// others) the chunk takes exact pairwise products instead, so no ratio of vanishing products is formed.
 #include "mixer_util.h"
 #include "recurrence_chunk.h"
 

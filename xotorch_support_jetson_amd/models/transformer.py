@@ -42,12 +42,12 @@ MOE_BM = int(os.environ.get("XOT_MOE_BM", "0"))  # force the grouped gemm_big ti
 MOE_DN_SPLITS = int(os.environ.get("XOT_MOE_DN_SPLITS", "0"))  # force the grouped down GEMM's K split on gemm_big tiles
 MOE_PP2 = os.environ.get("XOT_MOE_PP2", "1") == "1"  # 256-row expert tiles on the two-phase ping-pong schedule
 PAGE = 64
-# tokens of a step from which the second projections of low-rank gates run as GEMMs (below: inside the gate kernel, in fp32)
 # a parallel block's gate / up rows in a GEMM of their own, which ends in the gated activation: from 1024 tokens (the row count of
 # the four-wave tile) and 2^23 gate / up results on.  Against one GEMM and a pass over its fp32 result: 1024 x (8960 | 11264)
 # x 2048 91 us / 100, 2048 rows 168 / 179, 12807 rows 875 / 1130; 768 rows 82 / 70, 48 rows 35 / 25 and 2048 x (512 | 1024) x
 # 512 26 / 20, where the second launch costs more than the pass
 GELU_EPI_ROWS, GELU_EPI_SIZE = 1024, 1 << 23
+# tokens of a step from which the second projections of low-rank gates run as GEMMs (below: inside the gate kernel, in fp32)
 LOW_RANK_GEMM_ROWS = int(os.environ.get("XOT_LOW_RANK_GEMM_ROWS", "256"))
 
 

@@ -376,7 +376,7 @@ class GemmPolicy:
       return cands
     # 1256 / 2256: the 256 x 256 tile on the two-group ping-pong schedule in four / two phases per stage
     codes = [256, 1256, 2256, 128] if PP2 else [256, 1256, 128]
-    if W4 and N % 256 == 0:  # four-wave 256 x 256 tile (csrc/gemm_w4.hip): 256-row tiles only
+    if W4 and N % 256 == 0:  # four-wave tile of 256 columns (csrc/gemm_w4.hip): its launcher picks the rows (gemm_w4_mi)
       codes.append(4256)
     if N % 224 == 0:  # 7 row groups per wave: whole rounds where 256-wide tiles leave a half round (8B gate/up)
       codes.append(224)
