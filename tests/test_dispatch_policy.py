@@ -115,15 +115,15 @@ def test_tall_gemms_take_the_four_wave_tile_untimed(monkeypatch):
 
 
 def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
-  """Two K halves where 256-row tiles fill at most half the CUs, whatever M of the bucket came before: from K 8192 for a caller
-  whose residual norm sums the slabs, from 24576 for those that pay a reduce launch."""
+  """Two K halves where 256-row tiles fill at most half the CUs, whatever M of the bucket came before: from K 8192 for residual
+  products, from 24576 for plain ones."""
   monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: False)
   sized = []
   monkeypatch.setattr(L.scratch, "splitk", lambda dev, n, slot=0: sized.append(n))
 
-  def splits(pol, M, N, Kd, epi="none", **kw):
+  def splits(pol, M, N, Kd, epi="none"):
     x, w = torch.empty(M, Kd, dtype=torch.bfloat16, device="meta"), torch.empty(N, Kd, dtype=torch.bfloat16, device="meta")
-    kind, code, S = pol.shuffled_cfg(x, w, None, None, epi, torch.bfloat16, **kw)
+    kind, code, S = pol.shuffled_cfg(x, w, None, None, epi, torch.bfloat16)
     assert (kind, code) == ("big", 4256)
     return S
   for N, last in ((4096, 2048), (5120, 1536), (6144, 1280)):
@@ -131,11 +131,11 @@ def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
       pol = L.GemmPolicy()
       for M in Ms:
         half = M <= last
-        assert splits(pol, M, N, 14336, "resid", norm=True) == (2 if half else 1)
-        assert splits(pol, M, N, 14336, "resid") == 1
+        assert splits(pol, M, N, 14336, "resid") == (2 if half else 1)
+        assert splits(pol, M, N, 14336) == 1
         for epi in ("none", "resid"):
           assert splits(pol, M, N, 24576, epi) == (2 if half else 1)
-        assert splits(pol, M, N, 4096, "resid", norm=True) == 1
+        assert splits(pol, M, N, 4096, "resid") == 1
       assert not any(k[0].startswith("sh") and k[1] == 2048 and k[2] == N for k in pol.table)
   assert sized and max(sized) == 2 * 2048 * 4096
   monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: True)  # under capture: nothing to size

@@ -400,10 +400,10 @@ class GemmPolicy:
       return []
     return [("wave", nt, 1) for nt in ((2,) if rope else (2, 4) if epi in K.GLU_EPI else (1, 2, 4)) if N % (16 * nt) == 0]
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", norm: bool = False) -> Tuple:
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "") -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
-    reduce, timed with them, stands for the launch that does it there).  norm: the caller's residual norm sums the slabs."""
+    reduce, timed with them, stands for the launch that does it there)."""
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WAVE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
@@ -425,10 +425,12 @@ class GemmPolicy:
       # (profiles/r5/headline/bench_r5o_tunelog.log), so it is taken without the cold-timing pass, which cost
       # ~0.5 s inside the first prefill chunk of every fresh process.  (Its row height follows M inside the kernel's
       # launcher, gemm_w4_mi.)  Two K halves where 256-row tiles fill at most half the CUs and K is long enough to pay for
-      # the fp32 slabs: ~65 us at 2048 x 4096 with a reduce launch, from K ~ 24576 (28672: 369 us against 427 with 128-row
-      # tiles; 14336: about level; 4096: 74 against 58); ~30 where the residual norm that follows sums them, from K ~ 8192.
+      # the fp32 slabs.  Residual products from K 8192 on, us in one pass / in halves with the reduce / one pass and the norm /
+      # halves summed by the norm: 1024 x 4096 x 8192 124 / 89 / 129 / 82, x 14336 185 / 121 / 190 / 122; 1500 x 4096 x 14336
+      # 186 / 150 / 193 / 150; 2048 x 4096 x 8192 131 / 116 / 138 / 118, x 11008 144 / 149 / 156 / 149, x 14336 204 / 202 / 210
+      # / 199; K 4096: 58 / 74.  Plain ones from K ~ 24576 (2048 x 4096 x 28672 427 / 369).
       # Not stored: the halves follow this M, a table entry would answer for its whole bucket.
-      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if norm else 24576)
+      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576)
       if half and not self._no_tuning():  # (the slabs are sized outside a capture)
         scratch.splitk(x.device, 2 * M * N)
         return ("big", 4256, 2)
@@ -777,7 +779,7 @@ def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: t
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype, norm=h.is_contiguous())
+    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype)
     if (defer_to is not None and FUSE_NORM and M == 1 and cfg[0] == "stream" and 1 < cfg[2] <= 8 and N <= DEFER_MAX_D
         and out is None and h.is_contiguous() and h.dtype == torch.bfloat16):
       S = cfg[2]
