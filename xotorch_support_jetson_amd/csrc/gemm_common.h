@@ -1,5 +1,7 @@
 // Shared pieces of the GEMM kernels: epilogue kinds and the split-K slab reduction.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace xot {
@@ -66,6 +68,21 @@ __device__ __forceinline__ float epi_elem(float v) {
   return v;
 }
 
+// f(s0, integral_constant<int, n>) for n slabs from s0 on until all S are taken: four at a time, then two, then one, so that the
+// loads of a call are in flight together and no slab is read twice.  GEMM and reduce, us, slab by slab / four loads a round with
+// the last slab again / here: 55 x 16384 x 2048 SiLU in 2 slabs 23.8 / 24.3 / 23.8, 1 row 20.4 / 20.8 / 20.2; 55 x 2048 x 8192 in
+// 8 16.5 / 15.8 / 15.6.
+template <class F>
+__device__ __forceinline__ void for_slabs(int S, F&& f) {
+  int s0 = 0;
+  for (; s0 + 4 <= S; s0 += 4) f(s0, std::integral_constant<int, 4>{});
+  if (S & 2) {
+    f(s0, std::integral_constant<int, 2>{});
+    s0 += 2;
+  }
+  if (S & 1) f(s0, std::integral_constant<int, 1>{});
+}
+
 // Sum the S fp32 slabs of one output row at 8 output columns [o, o+8) and apply the epilogue.
 // wsrow = slab 0 of this row (slabs are sstride floats apart); rrow / yrow = this row of R / Y.
 template <int EPI, bool OUT_F32>
@@ -78,19 +95,19 @@ __device__ __forceinline__ void splitk_out8(const float* __restrict__ wsrow, siz
     float gs[8], us[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) gs[e] = us[e] = 0.f;
-    for (int s0 = 0; s0 < S; s0 += 4) {  // four slabs' loads in flight (past the last: it again, not added)
-      f32x4 g[4][2], u[4][2];
+    for_slabs(S, [&](int s0, auto n) {
+      constexpr int NS = decltype(n)::value;
+      f32x4 g[NS][2], u[NS][2];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float* row = wsrow + (s0 + k < S ? s0 + k : S - 1) * sstride + 32 * j + w;
+      for (int k = 0; k < NS; ++k) {
+        const float* row = wsrow + (s0 + k) * sstride + 32 * j + w;
         g[k][0] = *reinterpret_cast<const f32x4*>(row);
         g[k][1] = *reinterpret_cast<const f32x4*>(row + 4);
         u[k][0] = *reinterpret_cast<const f32x4*>(row + 16);
         u[k][1] = *reinterpret_cast<const f32x4*>(row + 20);
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (s0 + k >= S) continue;
+      for (int k = 0; k < NS; ++k)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           gs[e] += g[k][0][e];
@@ -98,8 +115,7 @@ __device__ __forceinline__ void splitk_out8(const float* __restrict__ wsrow, siz
           us[e] += u[k][0][e];
           us[e + 4] += u[k][1][e];
         }
-      }
-    }
+    });
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float bg = bias ? bf2f(bias[32 * j + w + e]) : 0.f, bu = bias ? bf2f(bias[32 * j + 16 + w + e]) : 0.f;
@@ -108,24 +124,23 @@ __device__ __forceinline__ void splitk_out8(const float* __restrict__ wsrow, siz
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    for (int s0 = 0; s0 < S; s0 += 4) {
-      f32x4 a[4][2];
+    for_slabs(S, [&](int s0, auto n) {
+      constexpr int NS = decltype(n)::value;
+      f32x4 a[NS][2];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float* row = wsrow + (s0 + k < S ? s0 + k : S - 1) * sstride + o;
+      for (int k = 0; k < NS; ++k) {
+        const float* row = wsrow + (s0 + k) * sstride + o;
         a[k][0] = *reinterpret_cast<const f32x4*>(row);
         a[k][1] = *reinterpret_cast<const f32x4*>(row + 4);
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (s0 + k >= S) continue;
+      for (int k = 0; k < NS; ++k)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           v[e] += a[k][0][e];
           v[e + 4] += a[k][1][e];
         }
-      }
-    }
+    });
     if (bias != nullptr) {
       const s16x8 bb = ld16(bias + o);
 #pragma unroll
