@@ -129,6 +129,10 @@ def to_rowmajor(w: torch.Tensor) -> torch.Tensor:
 
 
 # ------------------------------------------------------------------ per-device scratch
+class _Owner(threading.local):
+  name = ""
+
+
 class _Scratch:
   """Per-device split-K slabs shared by every GEMM call.  A buffer that has to grow is replaced, but the old one is
   kept alive: HIP graphs captured earlier (decode graphs of other batch buckets) hold its address, and replaying
@@ -138,13 +142,13 @@ class _Scratch:
   def __init__(self):
     self.ws: Dict[Tuple, torch.Tensor] = {}
     self.retired: list = []
-    self._own = threading.local()
+    self._own = _Owner()
 
   @contextlib.contextmanager
   def apart(self, name: str):
     """The calling thread's GEMMs inside take slabs of their own: work on a side stream, which nothing orders between another
     stream's GEMM and the reduce of its slabs."""
-    old = getattr(self._own, "name", "")
+    old = self._own.name
     self._own.name = name
     try:
       yield
@@ -155,7 +159,7 @@ class _Scratch:
     """slot 1 holds the slabs of a residual projection whose reduce is deferred into the next GEMM (PendingNorm),
     which writes its own slabs to slot 0 while it still reads slot 1, or those of the second of two projections whose
     slabs one kernel sums."""
-    key = (device.index or 0, slot, getattr(self._own, "name", ""))
+    key = (device.index or 0, slot, self._own.name)
     t = self.ws.get(key)
     if t is None or t.numel() < n:
       if torch.cuda.is_current_stream_capturing():
@@ -812,7 +816,8 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
   kernel that sums them, rotates and writes q / the caches (no bf16 qkv round trip, one launch less).
   x may be a PendingNorm: the projection then computes its input row in its prologue."""
   Dh = k_cache.shape[-1]
-  wave = "rope" if Dh % 32 == 0 and k_cache.dtype == torch.bfloat16 and w.shape[0] == (H + 2 * Hkv) * Dh else ""
+  few = isinstance(x, PendingNorm) or x.shape[0] <= WAVE_MAX_M
+  wave = "rope" if few and Dh % 32 == 0 and k_cache.dtype == torch.bfloat16 and w.shape[0] == (H + 2 * Hkv) * Dh else ""
 
   def rope(M):  # the outputs of the GEMM that rotates and writes by itself
     q = torch.empty(M, H, Dh, dtype=torch.bfloat16, device=k_cache.device)
