@@ -143,3 +143,80 @@ def test_wave_entries_of_the_tuning_table():
   pol.table[("sh",) + rtail], pol.table[("shy",) + rtail] = ("stream", 1, 2), ("wave", 1, 1)
   got = [pol.shuffled_cfg(x, w, None, x, "resid", torch.bfloat16, wave=wave) for wave in ("", "y")]
   assert got == [("stream", 1, 2), ("wave", 1, 1)]
+
+
+def test_wide_candidates_leave_no_cu_idle():
+  """17 to 64 rows: widths whose busiest CU has at most 1.4 times an even share of the column tiles, as many tiles as the
+  bucket of row counts has row tiles at least (a wave copies at most eight pieces of X), pairs inside a workgroup."""
+  cands = lambda *a: [c[1] for c in L.GemmPolicy._wide_cands(*a)]  # noqa: E731
+  assert cands(16, 4096, 128, "none", False) == [] == cands(65, 4096, 128, "none", False) == cands(48, 4096, 96, "none", False)
+  assert cands(48, 20224, 2048, "none", False) == [5, 6] == cands(33, 20224, 2048, "none", False) and cands(64, 28672, 4096, "silu", False) == [8, 4]
+  assert cands(64, 6144, 4096, "none", True) == []
+  for M, N, epi, rope in ((17, 256 * 16, "none", False), (64, 28672, "silu", False), (33, 6144, "none", True), (49, 11264, "clamp_glu", False)):
+    for nt in cands(M, N, 256, epi, rope):
+      assert L._m_bucket(M) // 16 <= nt <= 8 and (nt % 2 == 0 or not (rope or epi in K.GLU_EPI))
+      assert -(-(-(-N // 16 // nt)) // 256) * nt * 256 <= 1.4 * (N // 16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,Kd", [(96, 128), (224, 1408), (128, 2176)])
+def test_more_row_tiles_exact(gpu, M, N, Kd):
+  """Two to four row tiles on integer operands, bit for bit: a last workgroup with fewer tiles, chunks without a block for every
+  wave, a last chunk that is not full, rows past M, every epilogue, rows of a wider buffer; rotation
+  and cache write against float64."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  g = torch.Generator().manual_seed(M + N + Kd)
+  x, w, b, r = integers(g, M, Kd), integers(g, N, Kd), integers(g, N), integers(g, M, N)
+  full = x.float() @ w.float().t()
+  ws, bd, C = shuffle_for_stream(w.to(gpu)), b.to(gpu), require()
+  wide = torch.zeros(M, Kd + 16, dtype=torch.bfloat16, device=gpu)
+  wide[:, 8:8 + Kd] = x.to(gpu)
+  xd = wide[:, 8:8 + Kd]
+  f = (full + b.float()).view(M, N // 32, 2, 16)
+  want = {"silu": torch.nn.functional.silu(f[:, :, 0]) * f[:, :, 1],
+          "clamp_glu": (lambda u, v: u * torch.sigmoid(1.702 * u) * (v + 1))(f[:, :, 0].clamp(max=7.0), f[:, :, 1].clamp(-7.0, 7.0))}
+  for nt in range(1, 9):
+    y = torch.full((M + 1, N), 5.0, device=gpu)
+    if nt < -(-M // 16):
+      with pytest.raises(RuntimeError):
+        C.gemm_wave(xd, ws, y[:M], bd, None, K.EPI["none"], nt)
+      continue
+    C.gemm_wave(xd, ws, y[:M], bd, None, K.EPI["none"], nt)
+    assert torch.equal(y[:M].cpu(), full + b.float()) and bool((y[M] == 5.0).all()), nt
+    h = r.to(gpu)
+    C.gemm_wave(xd, ws, h, None, h, K.EPI["resid"], nt)
+    assert torch.equal(h.cpu(), (full + r.float()).to(torch.bfloat16)), nt
+    a = torch.zeros(M, N, dtype=torch.bfloat16, device=gpu)
+    C.gemm_wave(xd, ws, a, None, None, K.EPI["relu2"], nt)
+    assert torch.equal(a.cpu(), full.clamp(min=0).square().to(torch.bfloat16)), nt
+    for epi, ref in want.items():
+      act = torch.zeros(M, N // 2, dtype=torch.bfloat16, device=gpu)
+      if nt % 2:
+        with pytest.raises(RuntimeError):
+          C.gemm_wave(xd, ws, act, bd, None, K.EPI[epi], nt, 7.0)
+        continue
+      C.gemm_wave(xd, ws, act, bd, None, K.EPI[epi], nt, 7.0)
+      # one bf16 rounding (2^-9 of the value) behind fp32 arithmetic that differs in its last places
+      torch.testing.assert_close(act.cpu().float(), ref.reshape(M, N // 2), rtol=4e-3, atol=1e-3)
+  H, Hkv, Dh, pages = N // 32 - 2, 1, 32, 2
+  tab = torch.randn(70, Dh, generator=g)
+  c, sn = tab[:M, None, :16].double(), tab[:M, None, 16:].double()
+  lo, hi = (t.double() for t in full.view(M, H + 2, 2, 16).unbind(2))
+  rot = torch.cat([lo * c - hi * sn, hi * c + lo * sn], -1)
+  slots = torch.randperm(pages * 64, generator=g)[:M]
+  slots[M // 2] = -1
+  live = slots >= 0
+  for nt in (n for n in (2, 4, 6, 8) if n >= -(-M // 16)):
+    q = torch.zeros(M, H, Dh, dtype=torch.bfloat16, device=gpu)
+    kc, vc = torch.zeros(pages, Hkv, 64, Dh, dtype=torch.bfloat16, device=gpu), torch.zeros(pages, Hkv, Dh, 64, dtype=torch.bfloat16, device=gpu)
+    C.gemm_wave(xd, ws, None, None, None, 0, nt, pos=torch.arange(M, dtype=torch.int32, device=gpu), cos_sin=tab.to(gpu),
+                slots=slots.to(gpu), q_out=q, k_cache=kc, v_cache=vc, H=H, Hkv=Hkv)
+    # one bf16 rounding of two products of whole numbers (below 2^14, so exact to 2^-10 in fp32)
+    torch.testing.assert_close(q.cpu().double(), rot[:, :H], rtol=4e-3, atol=2e-3)
+    torch.testing.assert_close(kc.cpu().double().view(-1, Dh)[slots[live]], rot[live, H], rtol=4e-3, atol=2e-3)
+    # (a page of V: 8 chunks of 8 keys, [Dh][8] each)
+    values = vc.cpu().view(pages, 8, Dh, 8).transpose(2, 3).reshape(-1, Dh)
+    assert torch.equal(values[slots[live]], full.view(M, H + 2, Dh)[live, H + 1].to(torch.bfloat16))
+    untouched = torch.ones(pages * 64, dtype=torch.bool).index_fill_(0, slots[live], False)
+    assert not kc.cpu().view(-1, Dh)[untouched].any() and not values[untouched].any()

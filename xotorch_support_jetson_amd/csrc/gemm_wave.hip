@@ -1,19 +1,22 @@
-// Decode GEMM whose workgroups own their output columns for the whole of K:  Y[M, N] = X[M, K] . W[N, K]^T, M <= 16, on the
-// pre-shuffled layout ([N/16][K/32] blocks of 16 rows x 32 k, 1 KB).
+// Decode GEMM whose waves own whole column tiles:  Y[M, N] = X[M, K] . W[N, K]^T, M <= 64, on the pre-shuffled layout
+// ([N/16][K/32] blocks of 16 rows x 32 k, 1 KB).
 //
-// gemm_stream puts 64 or more columns on a workgroup's four waves, so a projection of a few thousand columns needs K split
-// over workgroups to cover the 256 CUs: fp32 slabs and a second launch of 4.5 to 6 us to add them, whatever their size.  Here
-// eight waves split K among themselves over 16, 32 or 64 columns: every wave streams its own 1-KB weight blocks (two stages of
-// eight in flight) and the matching k columns of X, and the eight partial tiles meet in LDS.  So the epilogue has the whole
-// sum -- bias, residual, gated pairs, or RoPE and the paged KV write (ROPE: a workgroup's two column tiles are the rotation
-// partners i and i + Dh/2 of one head) -- and the second launch is gone.
-// Cold-cache us, best split of gemm_stream with its reduce -> here, 1 / 6 rows: 3072 x 2048 10.4 -> 7.8 / 10.3 -> 8.4,
-// 16384 x 2048 SiLU 20.5 -> 17.3 / 21.0 -> 18.3, 2048 x 5632 15.5 -> 10.3 / 15.6 -> 12.0; bound by the ramp of one wave's
-// loads and the LDS exchange at these sizes (2 - 4 TB/s), by the loads of X beyond: every workgroup reads all of it, and from 24
-// rows on the split wins again (4096 x 14336 at 24 rows 28.0 -> 38.7), which is why one row tile is all there is.  Shapes
-// with columns enough for one pass of gemm_stream stay there, too (28672 x 4096 42 against 48): ops.linear times both.
-// NORM (batch-1 decode): the input row is rmsnorm(residual + the previous projection's slabs), computed by the first
-// four waves in splitk_resid_rmsnorm's order while all eight have their first weight blocks in flight.
+// A workgroup has nt column tiles, KW waves each: a wave streams its own part of ONE tile's K, eight consecutive blocks (8 KB) a
+// stage, two stages in flight.  What bounds a decode product is the weight stream, and the stream is fastest when every CU has
+// the same share of it and each wave reads long runs: 28672 x 4096 in pieces of 2 x 4 KB from two tiles 47 us, in 8 KB runs of
+// one 41, which is what a plain read of the same bytes takes.  So the rows of X, which all waves need, must not cost loads of
+// their own between the weights' (gathered per block as MFMA operands they were a third of the time at 16 rows): the workgroup
+// copies them chunk by chunk (a chunk: the KW parts' next eight blocks) through a swizzled LDS double buffer.
+// The KW partial tiles meet in LDS, so the epilogue has the whole sum -- bias, residual, gated pairs, or RoPE and the paged KV
+// write (ROPE: neighbouring tiles hold the rotation partners i and i + Dh/2 of one head) -- and no slabs, no reduce launch.
+// Cold weights in a graph, us, the eight-way K split of 16 / 32 columns with gathered rows that stood here before / here: 1 row
+// 16384 x 2048 SiLU 15.8 / 12.3 (a plain read: 12.6), 6 rows 11264 x 2048 clamped 13.9 / 10.9, 6144 x 2048 8.4 / 7.0, 12 rows
+// 128256 x 2048 94 (gemm_stream) / 86.  Beyond 16 rows, gemm_stream / here: 48 x 20224 x 2048 23.3 / 19.6, 37 x 21888 x 2048 SiLU
+// 25.9 / 20.6, 24 x 28672 x 4096 SiLU 47.2 / 45.2, 24 x 6144 x 4096 with RoPE 16.3 / 15.2.
+// NORM (batch-1 decode): the input row is rmsnorm(residual + the previous projection's slabs), computed by the first four waves
+// in splitk_resid_rmsnorm's order while all have their first weight blocks in flight.
+#include <algorithm>
+
 #include "common.h"
 #include "gemm_common.h"
 #include "kernels.h"
@@ -21,94 +24,158 @@
 namespace xot {
 namespace {
 
-constexpr int KW = 8, NTH = 64 * KW;  // waves of a workgroup, splitting K
+constexpr int U = 8;  // k blocks a stage
 
 __device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, int voff, int soff, bool nt) {
   return __builtin_bit_cast(s16x8, nt ? __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 2)
                                       : __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
-template <int NT, int EPI, bool F32, int NORM, int SM, bool ROPE>
-__global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restrict__ X, int ldx,
-                                                        const uint16_t* __restrict__ W, const uint16_t* __restrict__ bias,
-                                                        const uint16_t* __restrict__ R, int ldr, void* __restrict__ Yv, int ldy,
-                                                        int M, int K, float epi_arg, NormPro np, RopeOut ro) {
-  static_assert(!ROPE || NT == 2, "a rotation pair of column tiles");
-  static_assert(!epi_is_glu(EPI) || NT % 2 == 0, "gate / up tile pairs");
-  constexpr int U = 8 / NT;  // k blocks a stage
+// MT: 16-row tiles of X.  XL: X pieces (1 KB) a wave copies per chunk.  rw: rows of X kept in LDS (a power of two >= M up to 16,
+// whole tiles beyond; MFMA rows past it repeat them)
+template <int MT, int KW, int XL, int EPI, bool F32, int NORM, int SM, bool ROPE>
+__global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE ? 4 : 2) void gemm_wave_kernel(const uint16_t* __restrict__ X, int ldx, const uint16_t* __restrict__ W,
+                                                        const uint16_t* __restrict__ bias, const uint16_t* __restrict__ R,
+                                                        int ldr, void* __restrict__ Yv, int ldy, int M, int N, int K, int rw,
+                                                        float epi_arg, NormPro np, RopeOut ro) {
+  static_assert(NORM == 0 || MT == 1, "the norm prologue has one row");
+  constexpr int CB = U * KW, SL = CB * 4;  // k blocks of a chunk, 16-byte slots of a row's chunk
+  constexpr bool PAIR = ROPE || epi_is_glu(EPI);
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  f32x4(*red)[NT][64] = reinterpret_cast<f32x4(*)[NT][64]>(smem);                      // [KW]
-  uint16_t* x1 = reinterpret_cast<uint16_t*>(smem + sizeof(f32x4) * KW * NT * 64);     // NORM: the row [K]
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nb = K >> 5, b0 = wave * nb / KW, b1 = (wave + 1) * nb / KW;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6, nt = nw / KW;
+  const int t = wave / KW, p = wave - t * KW;
+  const int ntiles = N >> 4, nb = K >> 5, nch = (nb + CB - 1) / CB;
 
-  int tile[NT];  // 16-row groups of W
-  int head = 0, ra = 0;
-  if constexpr (ROPE) {
-    const int per = ro.Dh >> 5;
-    head = blockIdx.x / per;
-    ra = (blockIdx.x - head * per) * 16;
-    tile[0] = (head * ro.Dh + ra) >> 4;
-    tile[1] = tile[0] + (ro.Dh >> 5);
-  } else {
-#pragma unroll
-    for (int j = 0; j < NT; ++j) tile[j] = blockIdx.x * NT + j;
-  }
-  __amdgpu_buffer_rsrc_t wr[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-    wr[j] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W + (size_t)tile[j] * nb * 512), (short)0, nb * 1024, 0x00020000);
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X), (short)0, -1, 0x00020000);
-  const int xo = (min(c, M - 1) * ldx + 8 * g) * 2;  // the lane's row (past M the last again; not written)
+  // 16-row group of W that tile t of this workgroup is (ROPE: tiles 2 i and 2 i + 1 hold dims ra .. and Dh/2 + ra .. of a head)
+  auto tile_of = [&](int t) {
+    const int n = blockIdx.x * nt + t;
+    if constexpr (!ROPE) return n;
+    const int per = ro.Dh >> 5, pr = n >> 1, head = pr / per;
+    return (head * ro.Dh >> 4) + pr - head * per + (n & 1) * per;
+  };
+  // (a last workgroup's waves without a tile read the last one and write nothing)
+  const int tile = tile_of(min(t, ntiles - 1 - (int)blockIdx.x * nt));
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W + (size_t)tile * nb * 512), (short)0, nb * 1024, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X), (short)0, NORM ? 0 : ((M - 1) * ldx + K) * 2, 0x00020000);
 
   struct Stage {
-    s16x8 w[U][NT], x[NORM ? 1 : U];
+    s16x8 w[U];
   };
-  auto load = [&](Stage& s, int it) {  // k blocks b0 + it U .. (past the wave's range: its last block again, not used)
+  auto load = [&](Stage& s, int ch) {  // the wave's blocks of chunk ch (past K: zeros, not used)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int b = max(min(b0 + it * U + u, b1 - 1), 0);
+    for (int u = 0; u < U; ++u) s.w[u] = buf16(wr, lane * 16 + u * 1024, (ch * CB + p * U) * 1024, true);
+  };
+  // piece l of a chunk's rows of X: 64 consecutive slots of one row (or of 64 / SL rows)
+  constexpr int LR = SL >= 64 ? SL / 64 : 1, RL = SL >= 64 ? 1 : 64 / SL;
+  const int npc = (M * LR + RL - 1) / RL;
+  s16x8 xv[XL];
+  auto xload = [&](int ch) {
 #pragma unroll
-      for (int j = 0; j < NT; ++j) s.w[u][j] = buf16(wr[j], lane * 16, b * 1024, true);
-      if constexpr (!NORM) s.x[u] = buf16(xr, xo, b * 64, false);
+    for (int i = 0; i < XL; ++i) {
+      const int l = min(wave + i * nw, npc - 1);
+      if constexpr (RL > 1) xv[i] = buf16(xr, min(l * RL + lane / SL, M - 1) * ldx * 2 + (lane % SL) * 16, ch * CB * 64, false);
+      else xv[i] = buf16(xr, lane * 16, (l / LR) * ldx * 2 + (l % LR) * 1024 + ch * CB * 64, false);
     }
   };
-  f32x4 acc[NT];
+  const int half = rw * SL * 16;  // bytes of one of the two buffers
+  auto xstore = [&](int buf) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto one = [&](const Stage& s, int it, int u) {
-    s16x8 a;
-    if constexpr (NORM) a = ld16(x1 + (b0 + it * U + u) * 32 + 8 * g);  // (every MFMA row the same: row 0 is written)
-    else a = s.x[u];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[j] = mfma16(a, s.w[u][j], acc[j]);
-  };
-  auto whole = [&](const Stage& s, int it) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) one(s, it, u);
-  };
-  auto part = [&](const Stage& s, int it) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (b0 + it * U + u < b1) one(s, it, u);
-  };
-  Stage sa, sb;
-  s16x8 ha[NORM ? NORM : 1], la[NORM ? NORM : 1];
-  f32x4 p[NORM ? NORM : 1][NORM ? SM : 1][2];
-  const int nchunk = np.D >> 3;
-  // SM slabs from s0 on of the thread's chunks (past the last: the last again, not added)
-  auto slabs = [&](int s0) {
-#pragma unroll
-    for (int i = 0; i < (NORM ? NORM : 0); ++i)
-#pragma unroll
-      for (int sl = 0; sl < SM; ++sl) {
-        const float* sp = np.ws + min(s0 + sl, np.S - 1) * np.sstride + min((tid & 255) + 256 * i, nchunk - 1) * 8;
-        p[i][sl][0] = *reinterpret_cast<const f32x4*>(sp);
-        p[i][sl][1] = *reinterpret_cast<const f32x4*>(sp + 4);
+    for (int i = 0; i < XL; ++i) {
+      const int l = wave + i * nw;
+      if (l < npc) {
+        const int row = RL > 1 ? l * RL + lane / SL : l / LR, slot = RL > 1 ? lane % SL : (l % LR) * 64 + lane;
+        if (RL == 1 || row < M) *reinterpret_cast<s16x8*>(smem + buf * half + (row * SL + (slot ^ (row & 15))) * 16) = xv[i];
       }
+    }
   };
-  if constexpr (NORM > 0) {  // (asked for before the weights: loads return in order, and the row's chain is the longer one)
+  // LDS offsets of the A fragments: slot 4 u + g of the wave's part; the swizzle reaches the slot's low four bits only
+  int fo[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = MT > 1 ? c : c & (rw - 1);
+    fo[j] = (row * SL + p * U * 4 + ((4 * j + g) ^ row)) * 16;
+  }
+  f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto frag = [&](int q, int base) {  // q = u MT + i
+    const int u = q / MT, i = q % MT;
+    return *reinterpret_cast<const s16x8*>(smem + base + fo[u & 3] + (u >> 2) * 256 + i * 16 * SL * 16);
+  };
+  auto compute = [&](const Stage& s, int ch) {
+    const int base = NORM ? ch * SL * 16 : (ch & 1) * half;
+    if (ch * CB + p * U + U <= nb) {
+      constexpr int PF = MT == 1 ? 2 : 4;  // fragments read ahead of their MFMA
+      s16x8 a[PF];
+#pragma unroll
+      for (int q = 0; q < PF; ++q) a[q] = frag(q, base);
+#pragma unroll
+      for (int q = 0; q < U * MT; ++q) {
+        const s16x8 cur = a[q % PF];
+        if (q + PF < U * MT) a[q % PF] = frag(q + PF, base);
+        acc[q % MT] = mfma16(cur, s.w[q / MT], acc[q % MT]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (ch * CB + p * U + u < nb) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[i] = mfma16(frag(u * MT + i, base), s.w[u], acc[i]);
+        }
+    }
+  };
+
+  // ROPE: unit q (a pair of tiles and a row tile) of the epilogue, its rows' slots and table entries.  The wave's first unit asks for
+  // them here, or two dependent loads would stand between the sums and the stores
+  const int have = min(nt, ntiles - (int)blockIdx.x * nt);  // tiles of this workgroup
+  struct Rot {
+    int pos[4];
+    int64_t slot[4];
+    float c[4], s[4];
+  } rot;
+  auto rope_rows = [&](int q) {
+    const int i = q % MT;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = min(16 * i + 4 * g + r, M - 1);
+      rot.pos[r] = ro.pos[m];
+      rot.slot[r] = ro.slots[m];
+    }
+  };
+  auto rope_table = [&](int q) {
+    const int per = ro.Dh >> 5, n = (blockIdx.x * nt >> 1) + q / MT, d = n % per * 16 + c;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* cs = ro.cos_sin + (size_t)min(max(rot.pos[r], 0), ro.max_pos - 1) * ro.Dh + d;
+      rot.c[r] = cs[0];
+      rot.s[r] = cs[ro.Dh >> 1];
+    }
+  };
+  const int units = (have >> 1) * MT;
+  const bool rope_here = ROPE && wave < units;
+  if (rope_here) rope_rows(wave);
+
+  Stage sa, sb;
+  if constexpr (NORM > 0) {
+    s16x8 ha[NORM], la[NORM];
+    f32x4 pv[NORM][SM][2];
+    const int nchunk = np.D >> 3;
+    // SM slabs from s0 on of the thread's chunks (past the last: the last again, not added)
+    auto slabs = [&](int s0) {
+#pragma unroll
+      for (int i = 0; i < NORM; ++i)
+#pragma unroll
+        for (int sl = 0; sl < SM; ++sl) {
+          const float* sp = np.ws + min(s0 + sl, np.S - 1) * np.sstride + min((tid & 255) + 256 * i, nchunk - 1) * 8;
+          pv[i][sl][0] = *reinterpret_cast<const f32x4*>(sp);
+          pv[i][sl][1] = *reinterpret_cast<const f32x4*>(sp + 4);
+        }
+    };
+    // (asked for before the weights: loads return in order, and the row's chain is the longer one)
 #pragma unroll
     for (int i = 0; i < NORM; ++i) {
       const int cc = min((tid & 255) + 256 * i, nchunk - 1);
@@ -117,12 +184,12 @@ __global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restri
     }
     if (np.S > 0) slabs(0);
     __builtin_amdgcn_sched_barrier(0);
-  }
-  load(sa, 0);
-  load(sb, 1);
-  if constexpr (NORM > 0) {
+    load(sa, 0);
+    load(sb, 1);
     __builtin_amdgcn_sched_barrier(0);
-    // one row: residual + bias + slabs -> bf16 residual (stored by workgroup 0), its RMS norm times the weight -> x1.  256
+    if (rope_here) rope_table(wave);
+    __builtin_amdgcn_sched_barrier(0);
+    // one row: residual + bias + slabs -> bf16 residual (stored by workgroup 0), its RMS norm times the weight -> LDS.  256
     // threads, 8 consecutive elements each per round, in the order of splitk_resid_rmsnorm_kernel<*, *, 256>
     __shared__ float nred[4];
     if (wave < 4) {
@@ -147,8 +214,8 @@ __global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restri
             if (s0 + sl < np.S) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                v[i][e] += p[i][sl][0][e];
-                v[i][4 + e] += p[i][sl][1][e];
+                v[i][e] += pv[i][sl][0][e];
+                v[i][4 + e] += pv[i][sl][1][e];
               }
             }
       }
@@ -180,32 +247,67 @@ __global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restri
         s16x8 o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(bf2f(ha[i][e]) * inv * bf2f(la[i][e]));
-        st16(x1 + cc * 8, o);
+        *reinterpret_cast<s16x8*>(smem + cc * 16) = o;
       }
     }
     __syncthreads();
-  }
-  {
-    const int nfull = (b1 - b0) / U, nit = (b1 - b0 + U - 1) / U;
-    int it = 0;
-    for (; it + 2 <= nfull; it += 2) {
-      whole(sa, it);
-      load(sa, it + 2);
-      whole(sb, it + 1);
-      load(sb, it + 3);
+    int ch = 0;
+    for (; ch + 2 < nch; ch += 2) {
+      compute(sa, ch);
+      load(sa, ch + 2);
+      compute(sb, ch + 1);
+      load(sb, ch + 3);
     }
-    if (it < nit) part(sa, it);
-    if (it + 1 < nit) part(sb, it + 1);
+    compute(sa, ch);
+    if (ch + 1 < nch) compute(sb, ch + 1);
+  } else {
+    // (X first: loads return in order, and its way through LDS is the longer one)
+    xload(0);
+    load(sa, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(sb, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (rope_here) rope_table(wave);
+    __builtin_amdgcn_sched_barrier(0);
+    xstore(0);
+    __builtin_amdgcn_sched_barrier(0);
+    xload(1);
+    __syncthreads();
+    int ch = 0;
+    for (; ch + 2 < nch; ch += 2) {  // (a chunk's rows go where the chunk before last was read: one barrier a chunk)
+      compute(sa, ch);
+      xstore(1);
+      __syncthreads();
+      xload(ch + 2);
+      load(sa, ch + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(sb, ch + 1);
+      xstore(0);
+      __syncthreads();
+      xload(ch + 3);
+      load(sb, ch + 3);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    compute(sa, ch);
+    if (ch + 1 < nch) {
+      xstore(1);
+      __syncthreads();
+      compute(sb, ch + 1);
+    }
   }
-#pragma unroll
-  for (int j = 0; j < NT; ++j) red[wave][j][lane] = acc[j];
-  __syncthreads();
 
-  // the waves' partial tiles in wave order; lane (g, c) of tile j: tokens 4 g + r, column c of the tile
-  auto total = [&](int t, int l) {
-    f32x4 v = red[0][t][l];
+  // partial tiles of a tile's waves in K order; lane (g, c): tokens 16 i + 4 g + r, column c of the tile
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [nw][MT][64]
+  if constexpr (KW > 1 || PAIR) {
+    __syncthreads();
 #pragma unroll
-    for (int w = 1; w < KW; ++w) v += red[w][t][l];
+    for (int i = 0; i < MT; ++i) red[(wave * MT + i) * 64 + lane] = acc[i];
+    __syncthreads();
+  }
+  auto total = [&](int t, int i) {
+    f32x4 v = red[(t * KW * MT + i) * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < KW; ++q) v += red[((t * KW + q) * MT + i) * 64 + lane];
     return v;
   };
   auto put = [&](int m, int col, float v) {
@@ -213,26 +315,30 @@ __global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restri
     else reinterpret_cast<uint16_t*>(Yv)[(size_t)m * ldy + col] = f2bf(v);
   };
   if constexpr (ROPE) {
-    const int half = ro.Dh >> 1;
-    if (tid < 64) {
-      const int l = tid, d = ra + (l & 15);
-      f32x4 lo = total(0, l), hi = total(1, l);
+    const int hd = ro.Dh >> 1, per = ro.Dh >> 5;
+    for (int q = wave; q < units; q += nw) {
+      if (q != wave) {
+        rope_rows(q);
+        rope_table(q);
+      }
+      const int pr = q / MT, i = q - pr * MT, n = (blockIdx.x * nt >> 1) + pr, head = n / per, d = (n - head * per) * 16 + c;
+      f32x4 lo = total(2 * pr, i), hi = total(2 * pr + 1, i);
       if (bias != nullptr) {
         lo += bf2f(bias[head * ro.Dh + d]);
-        hi += bf2f(bias[head * ro.Dh + half + d]);
+        hi += bf2f(bias[head * ro.Dh + hd + d]);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = 4 * (l >> 4) + r;
+        const int m = 16 * i + 4 * g + r;
         if (m >= M) continue;
-        const int64_t slot = ro.slots[m] < ro.nslots ? ro.slots[m] : -1;
+        const int64_t slot = rot.slot[r] < ro.nslots ? rot.slot[r] : -1;
         const int64_t page = slot >= 0 ? slot / ro.BS : 0;
         const int off = slot >= 0 ? (int)(slot % ro.BS) : 0;
         if (head >= ro.H + ro.Hkv) {
           if (slot < 0) continue;
           uint16_t* dst = ro.vc + ((size_t)page * ro.Hkv + (head - ro.H - ro.Hkv)) * ro.Dh * ro.BS;
           dst[v_page_off(off, d, ro.Dh)] = f2bf(lo[r]);
-          dst[v_page_off(off, half + d, ro.Dh)] = f2bf(hi[r]);
+          dst[v_page_off(off, hd + d, ro.Dh)] = f2bf(hi[r]);
           continue;
         }
         uint16_t* dst;
@@ -242,67 +348,92 @@ __global__ __launch_bounds__(NTH) void gemm_wave_kernel(const uint16_t* __restri
           if (slot < 0) continue;
           dst = ro.kc + (((size_t)page * ro.Hkv + (head - ro.H)) * ro.BS + off) * ro.Dh;
         }
-        const float* cs = ro.cos_sin + (size_t)min(max(ro.pos[m], 0), ro.max_pos - 1) * ro.Dh;
-        dst[d] = f2bf(lo[r] * cs[d] - hi[r] * cs[half + d]);
-        dst[half + d] = f2bf(hi[r] * cs[d] + lo[r] * cs[half + d]);
+        dst[d] = f2bf(lo[r] * rot.c[r] - hi[r] * rot.s[r]);
+        dst[hd + d] = f2bf(hi[r] * rot.c[r] + lo[r] * rot.s[r]);
       }
     }
   } else if constexpr (epi_is_glu(EPI)) {
-    if (tid < 32 * NT) {
-      const int p = tid >> 6, l = tid & 63;
-      f32x4 gv = total(2 * p, l), uv = total(2 * p + 1, l);
-      const int n = tile[0] * 16 + 32 * p + (l & 15);  // gate row of W; its up row is 16 further
+    for (int q = wave; q < units; q += nw) {
+      const int pr = q / MT, i = q - pr * MT, n0 = (blockIdx.x * nt + 2 * pr) * 16;  // gate rows of W; the up rows follow
+      f32x4 gv = total(2 * pr, i), uv = total(2 * pr + 1, i);
       if (bias != nullptr) {
-        gv += bf2f(bias[n]);
-        uv += bf2f(bias[n + 16]);
+        gv += bf2f(bias[n0 + c]);
+        uv += bf2f(bias[n0 + 16 + c]);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = 4 * (l >> 4) + r;
-        if (m < M) put(m, tile[0] * 8 + 16 * p + (l & 15), glu_pair<EPI>(gv[r], uv[r], epi_arg));
+        const int m = 16 * i + 4 * g + r;
+        if (m < M) put(m, n0 / 2 + c, glu_pair<EPI>(gv[r], uv[r], epi_arg));
       }
     }
   } else {
-    if (tid < 64 * NT) {
-      const int t = tid >> 6, l = tid & 63, n = tile[0] * 16 + 16 * t + (l & 15);
-      f32x4 v = total(t, l);
+    auto out = [&](int t, int i, f32x4 v) {
+      const int n = (blockIdx.x * nt + t) * 16 + c;
       if (bias != nullptr) v += bf2f(bias[n]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = 4 * (l >> 4) + r;
+        const int m = 16 * i + 4 * g + r;
         if (m >= M) continue;
         if constexpr (EPI == EPI_RESID) v[r] += bf2f(R[(size_t)m * ldr + n]);
         put(m, n, epi_elem<EPI>(v[r]));
       }
+    };
+    if constexpr (KW == 1) {
+      if (t < have) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) out(t, i, acc[i]);
+      }
+    } else {
+      for (int q = wave; q < have * MT; q += nw) out(q / MT, q % MT, total(q / MT, q % MT));
     }
   }
 }
 
-template <int NT, int EPI, bool F32, int NORM, int SM, bool ROPE>
-void go(const WaveGemm& a, hipStream_t st) {
-  const size_t smem = sizeof(f32x4) * KW * NT * 64 + (NORM ? a.K * 2 : 0);  // at most 32 + 16 KB
-  gemm_wave_kernel<NT, EPI, F32, NORM, SM, ROPE><<<a.N / (16 * NT), NTH, smem, st>>>(a.X, a.ldx, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy,
-                                                                                 a.M, a.K, a.epi_arg, a.np, a.ro);
+template <int MT, int KW, int XL, int EPI, bool F32, int NORM, int SM, bool ROPE>
+int go(const WaveGemm& a, int nt, hipStream_t st) {
+  constexpr int CB = U * KW;
+  int rw = 16 * MT;
+  if (MT == 1)
+    while (rw / 2 >= a.M) rw /= 2;
+  const int nw = nt * KW, nb = a.K / 32;
+  const size_t xbytes = NORM ? (size_t)(nb + CB - 1) / CB * CB * 64 : (size_t)2 * rw * CB * 64;
+  const size_t smem = std::max(xbytes, KW > 1 || ROPE || epi_is_glu(EPI) ? (size_t)nw * MT * 1024 : 0);
+  auto kern = gemm_wave_kernel<MT, KW, XL, EPI, F32, NORM, SM, ROPE>;
+  static_assert(2 * 16 * MT * CB * 64 <= 65536 && 8 * MT * 1024 <= 65536, "LDS a launch takes without asking");
+  kern<<<(a.N / 16 + nt - 1) / nt, 64 * nw, smem, st>>>(a.X, a.ldx, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy, a.M, a.N, a.K, rw, a.epi_arg,
+                                                        a.np, a.ro);
+  return 0;
 }
 
-template <int EPI, bool F32, int NORM, int SM>
-int columns(const WaveGemm& a, int nt, hipStream_t st) {
+// Waves per tile (cold weights in a graph, us).  One row tile: eight waves in all, but never more than four a tile: 3072 x 2048 at
+// 1 row by single tiles, 4 / 8 waves 5.0 / 5.2, 6144 x 2048 at 6 rows 8.0 / 10.2; 11264 x 2048 by fours, 1 / 2 waves 12.2 / 10.9.
+// More rows: the chunk's X takes the LDS that more parts would need, and the waves' stages are enough in flight: 20224 x 2048 at
+// 48 rows by threes, 1 / 2 waves 20.8 / 24.1; two only beside a lone pair (6144 x 4096 at 24 rows 16.4 / 14.7).
+template <int EPI, bool F32, int NORM, int SM, bool ROPE>
+int one_row_tile(const WaveGemm& a, int nt, hipStream_t st) {
+  constexpr bool LONE = !ROPE && !epi_is_glu(EPI);
   if (nt == 1) {
-    if constexpr (epi_is_glu(EPI)) return -1;
-    else go<1, EPI, F32, NORM, SM, false>(a, st);
-  } else if (nt == 2) {
-    go<2, EPI, F32, NORM, SM, false>(a, st);
-  } else {
-    go<4, EPI, F32, NORM, SM, false>(a, st);
+    if constexpr (LONE) return go<1, 4, NORM ? 4 : 8, EPI, F32, NORM, SM, ROPE>(a, nt, st);  // (half the waves copy X)
+    else return -1;
   }
-  return 0;
+  if (nt == 2) return go<1, 4, 4, EPI, F32, NORM, SM, ROPE>(a, nt, st);
+  return nt <= 4 ? go<1, 2, 4, EPI, F32, NORM, SM, ROPE>(a, nt, st) : -1;
+}
+
+template <int EPI, bool F32, bool ROPE>
+int by_rows(const WaveGemm& a, int nt, hipStream_t st) {
+  const int mt = (a.M + 15) / 16;
+  if (mt == 1) return one_row_tile<EPI, F32, 0, 1, ROPE>(a, nt, st);
+  if (nt < mt) return -1;  // (a wave copies at most eight pieces of a chunk)
+  if (mt == 2) return nt == 2 ? go<2, 2, 8, EPI, F32, 0, 1, ROPE>(a, nt, st) : go<2, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st);
+  return mt == 3 ? go<3, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st) : go<4, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st);
 }
 
 template <int NORM, int SM>
 int normed(const WaveGemm& a, int epi, int nt, hipStream_t st) {
-  if (a.ro.q == nullptr) return epi == EPI_SILU ? columns<EPI_SILU, false, NORM, SM>(a, nt, st) : columns<EPI_NONE, false, NORM, SM>(a, nt, st);
-  go<2, EPI_NONE, false, NORM, SM, true>(a, st);
-  return 0;
+  if (a.ro.q != nullptr) return one_row_tile<EPI_NONE, false, NORM, SM, true>(a, nt, st);
+  return epi == EPI_SILU ? one_row_tile<EPI_SILU, false, NORM, SM, false>(a, nt, st)
+                         : one_row_tile<EPI_NONE, false, NORM, SM, false>(a, nt, st);
 }
 
 }  // namespace
@@ -310,10 +441,11 @@ int normed(const WaveGemm& a, int epi, int nt, hipStream_t st) {
 int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream_t st) {
   if (a.M <= 0) return 0;
   const bool rope = a.ro.q != nullptr, norm = a.np.h != nullptr;
-  if (a.M > 16 || a.K % 128 != 0 || a.K <= 0 || (nt != 1 && nt != 2 && nt != 4) || a.N % (16 * nt) != 0) return -1;
+  if (a.M > 64 || a.K % 128 != 0 || a.K <= 0 || nt < 1 || nt > 8 || a.N % 16 != 0) return -1;
+  if ((int64_t)a.K * 32 >= (int64_t(1) << 31)) return -1;  // (32-bit byte offsets into a tile)
   if (!norm && (a.ldx % 8 != 0 || (int64_t)a.M * a.ldx * 2 >= (int64_t(1) << 31))) return -1;
-  if (epi_is_glu(epi) && nt == 1) return -1;
-  if (rope && (nt != 2 || epi != EPI_NONE || out_f32 || a.ro.Dh % 32 != 0 || a.N != (a.ro.H + 2 * a.ro.Hkv) * a.ro.Dh || a.ro.max_pos < 1)) return -1;
+  if ((rope || epi_is_glu(epi)) && (nt % 2 != 0 || a.N % 32 != 0)) return -1;
+  if (rope && (epi != EPI_NONE || out_f32 || a.ro.Dh % 32 != 0 || a.N != (a.ro.H + 2 * a.ro.Hkv) * a.ro.Dh || a.ro.max_pos < 1)) return -1;
   if (norm) {
     if (a.M != 1 || out_f32 || (epi != EPI_NONE && epi != EPI_SILU) || a.np.D != a.K || a.K > 8192 || a.np.S < 0 ||
         a.np.lnw == nullptr || a.np.hout == nullptr || (a.np.S > 0 && (a.np.ws == nullptr || a.np.sstride < a.K)))
@@ -322,16 +454,13 @@ int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream
     if (a.K <= 2048) return a.np.S > 4 ? normed<1, 8>(a, epi, nt, st) : normed<1, 4>(a, epi, nt, st);
     return a.K <= 4096 ? normed<2, 4>(a, epi, nt, st) : normed<4, 2>(a, epi, nt, st);
   }
-  if (rope) {
-    go<2, EPI_NONE, false, 0, 1, true>(a, st);
-    return 0;
-  }
+  if (rope) return by_rows<EPI_NONE, false, true>(a, nt, st);
   switch (epi) {
-    case EPI_NONE: return out_f32 ? columns<EPI_NONE, true, 0, 1>(a, nt, st) : columns<EPI_NONE, false, 0, 1>(a, nt, st);
-    case EPI_RESID: return out_f32 ? -1 : columns<EPI_RESID, false, 0, 1>(a, nt, st);
-    case EPI_SILU: return out_f32 ? -1 : columns<EPI_SILU, false, 0, 1>(a, nt, st);
-    case EPI_CLAMP_GLU: return out_f32 ? -1 : columns<EPI_CLAMP_GLU, false, 0, 1>(a, nt, st);
-    case EPI_RELU2: return out_f32 ? -1 : columns<EPI_RELU2, false, 0, 1>(a, nt, st);
+    case EPI_NONE: return out_f32 ? by_rows<EPI_NONE, true, false>(a, nt, st) : by_rows<EPI_NONE, false, false>(a, nt, st);
+    case EPI_RESID: return out_f32 ? -1 : by_rows<EPI_RESID, false, false>(a, nt, st);
+    case EPI_SILU: return out_f32 ? -1 : by_rows<EPI_SILU, false, false>(a, nt, st);
+    case EPI_CLAMP_GLU: return out_f32 ? -1 : by_rows<EPI_CLAMP_GLU, false, false>(a, nt, st);
+    case EPI_RELU2: return out_f32 ? -1 : by_rows<EPI_RELU2, false, false>(a, nt, st);
   }
   return -1;
 }

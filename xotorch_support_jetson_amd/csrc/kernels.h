@@ -63,8 +63,9 @@ void launch_attn_decode_merge(const float* ws_o, const float* ws_ml, const int32
 int launch_gemm_stream_norm(const uint16_t* W, const uint16_t* bias, void* Y, int ldy, int epi, float* ws,
                             long ws_elems, int N, int K, int ntw, int S, bool reduce, const NormPro& np,
                             hipStream_t s);
-// decode GEMM whose workgroups hold whole K sums (gemm_wave.hip): M <= 16, N % (16 nt) == 0, K % 128 == 0, pre-shuffled W.
-// np.h: one row, its norm prologue; ro.q: the QKV projection, rotated and written to q and the paged caches (nt 2)
+// decode GEMM whose workgroups hold whole K sums (gemm_wave.hip): M <= 64, N % 16 == 0, K % 128 == 0, pre-shuffled W; nt column tiles a
+// workgroup (1 .. 4 up to 16 rows; ceil(M / 16) .. 8 beyond; even for gated pairs and rope).  np.h: one row, its norm prologue; ro.q:
+// the QKV projection, rotated and written to q and the paged caches
 struct RopeOut {
   uint16_t *q, *kc, *vc;
   const int32_t* pos;

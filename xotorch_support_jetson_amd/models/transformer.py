@@ -1137,7 +1137,7 @@ class ShardModel:
       else:
         # QKV projection + RoPE + paged KV write (split-K slabs reduced inside the RoPE kernel)
         q = linear_rope_kv(xn, lw.qkv_w, lw.qkv_b, inp.positions, self.cos_sin, inp.slots, self.kv.k[j],
-                           self.kv.v[j], c.num_heads, c.num_kv_heads)
+                           self.kv.v[j], c.num_heads, c.num_kv_heads, wide=not c.num_experts)
         if isinstance(xn, PendingNorm):
           h = xn.dst
         a = self._attention(q, j, inp, defer_merge=fuse and FUSE_MERGE and lw.router is None)

@@ -6,8 +6,8 @@ kernels consume that layout, all with the epilogue fused (bias / residual add / 
 
   gemm_stream  decode-shaped M: weight-streaming MFMA GEMM (1 KB coalesced weight loads per wave
                instruction straight to registers, X shared through swizzled LDS, optional split-K).
-  gemm_wave    up to 16 rows: a workgroup holds its columns for the whole of K (its waves split K among themselves), so no
-               slabs and no reduce launch; also with RoPE and the paged KV write in the epilogue.
+  gemm_wave    up to 64 rows: a wave owns a column tile (or a part of its K), so no slabs and no reduce launch; also with RoPE
+               and the paged KV write in the epilogue.
   gemm_big     compute-bound M (large decode batches, prefill chunks): 256 x {256,128} x 64 tiles,
                both operands staged by LDS-DMA, 8 waves, XCD-aware tile order, optional split-K.
 No vendor GEMM runs on a shuffled weight: at prefill sizes gemm_big matches hipBLASLt once the weight
@@ -54,9 +54,11 @@ TALL_FIXED = True
 BLAS_CAND = os.environ.get("XOT_GEMM_BLAS", "0") == "1"
 # largest M for which the stream GEMM is a candidate (above it only gemm_big is timed)
 STREAM_MAX_M = int(os.environ.get("XOT_STREAM_MAX_M", "512"))
-# largest M for which the whole-K decode GEMM (csrc/gemm_wave.hip) is a candidate: no slabs, no reduce launch (its X traffic
-# grows with the rows: at 24 and more the K split of the stream GEMM won every timed shape)
+# largest M for which the whole-K decode GEMM (csrc/gemm_wave.hip) is a candidate with any width of its workgroups: no slabs, no
+# reduce launch.  Beyond it every workgroup's copy of X counts, and only widths that leave no CU idle are timed (_wide_cands)
 WAVE_MAX_M = 16
+# ... and at all (its row tiles; a chunk of X for more would not fit beside a second workgroup's)
+WIDE_MAX_M = 64
 # smallest M for which gemm_big is a candidate
 BIG_MIN_M = int(os.environ.get("XOT_BIG_MIN_M", "65"))
 
@@ -404,13 +406,30 @@ class GemmPolicy:
       return []
     return [("wave", nt, 1) for nt in ((2,) if rope else (2, 4) if epi in K.GLU_EPI else (1, 2, 4)) if N % (16 * nt) == 0]
 
+  @staticmethod
+  def _wide_cands(M, N, Kd, epi, rope):
+    """The same at 17 to 64 rows: the (at most three) workgroup widths whose busiest CU has the fewest columns, as long as that is at
+    most 1.4 times an even share.  The time follows that share: 48 x 20224 x 2048, nt 3 .. 8: 20.8, 23.1, 19.6, 20.2, 21.3, 23.2 us
+    for 6, 8, 5, 6, 7, 8 tiles (an even share is 4.9; the stream GEMM 23.3); 64 x 28672 x 4096 48.7 at nt 8 (7 of 8 tiles), 65.6 at
+    nt 6 (7 of 12; stream 50.5); 24 x 6144 x 4096 14.7 (1.5 of 2; stream in slabs with the reduce 15.6), at 64 rows 23.6 (1.5 of
+    4; stream 19.0).  A choice holds for its
+    whole bucket of row counts, so nt has a tile for each of the bucket's row tiles."""
+    if not WAVE_MAX_M < M <= WIDE_MAX_M or Kd % 128 or N % 16:
+      return []
+    tiles, pairs = N // 16, rope or epi in K.GLU_EPI
+    if pairs and N % 32:
+      return []
+    busiest = {nt: -(-(-(-tiles // nt)) // 256) * nt for nt in range(_m_bucket(M) // 16, 9) if not (pairs and nt % 2)}
+    top = sorted(busiest, key=lambda nt: (busiest[nt], -nt))[:3]
+    return [("wave", nt, 1) for nt in top if busiest[nt] * 256 <= 1.4 * tiles]
+
   def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "") -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
     reduce, timed with them, stands for the launch that does it there)."""
     M, Kd = x.shape
     N = w.shape[0]
-    wave = wave if M <= WAVE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
+    wave = wave if M <= WIDE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
     # (a residual product's plain entry belongs to linear_resid_norm, which sums the slabs itself; a caller that does not
     # take the whole-K GEMM passes over such an entry)
     kind = "sh" + wave if wave == "rope" or epi == "resid" else "sh"
@@ -443,7 +462,7 @@ class GemmPolicy:
     if M <= STREAM_MAX_M and epi != "gelu_glu":
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
     if wave and epi != "gelu_glu":
-      cands += self._wave_cands(M, N, Kd, epi, wave == "rope")
+      cands += self._wave_cands(M, N, Kd, epi, wave == "rope") or self._wide_cands(M, N, Kd, epi, wave == "rope")
     if M >= BIG_MIN_M and Kd % 128 == 0:
       big = self._big_cands(M, N, Kd)
       cands += [c for c in big if c[1] in (2256, 128, 4256)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
@@ -671,7 +690,11 @@ class PendingNorm:
     require().gemm_wave(None, w, y, bias, None, K.EPI[epi], nt, 0.0, self.src, self.ws, self.S, self.bias, self.ln_w, self.dst,
                         self.eps, **rope)
 
-  def run(self, w: torch.Tensor, y: torch.Tensor, bias, epi: str, ntw: int, S: int, reduce: bool) -> None:
+  def run(self, w: torch.Tensor, y, bias, epi: str, cfg: Tuple, reduce: bool = True, **rope) -> None:
+    """The consumer GEMM in the configuration _pending_cfg gave (rope: outputs of the whole-K form that rotates and writes)."""
+    if cfg[0] == "wave":
+      return self.run_wave(w, y, bias, epi, cfg[1], **rope)
+    _, ntw, S = cfg
     ws = scratch.splitk(y.device, S * w.shape[0]) if S > 1 else None
     require().gemm_stream_norm(w, y, bias, ws, K.EPI[epi], ntw, S, reduce, self.src, self.ws, self.S, self.bias,
                                self.ln_w, self.dst, self.eps)
@@ -704,10 +727,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, r
       if out is None:
         out = torch.empty(1, w.shape[0] // 2 if epi == "silu" else w.shape[0], dtype=torch.bfloat16,
                           device=x.src.device)
-      if cfg[0] == "wave":
-        x.run_wave(w, out, bias, epi, cfg[1])
-      else:
-        x.run(w, out, bias, epi, cfg[1], cfg[2], True)
+      x.run(w, out, bias, epi, cfg)
       return out
   if not x.is_cuda:
     return K.gemm(x, to_rowmajor(w), bias=bias, residual=residual, epi=epi, out=out, out_dtype=out_dtype)
@@ -809,14 +829,15 @@ def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: t
 
 def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, pos: torch.Tensor,
                    cos_sin: torch.Tensor, slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, H: int,
-                   Hkv: int) -> torch.Tensor:
+                   Hkv: int, wide: bool = True) -> torch.Tensor:
   """qkv = x @ w.T (+ bias); returns rope(q) [T, H, Dh] and writes rope(k), v into the paged caches.
 
   When the QKV projection runs split-K on the pre-shuffled layout, its fp32 slabs go straight to one
   kernel that sums them, rotates and writes q / the caches (no bf16 qkv round trip, one launch less).
-  x may be a PendingNorm: the projection then computes its input row in its prologue."""
+  x may be a PendingNorm: the projection then computes its input row in its prologue.
+  wide=False: from 17 rows on never the whole-K GEMM, whose K order is another one than the slabs'."""
   Dh = k_cache.shape[-1]
-  few = isinstance(x, PendingNorm) or x.shape[0] <= WAVE_MAX_M
+  few = isinstance(x, PendingNorm) or x.shape[0] <= (WIDE_MAX_M if wide else WAVE_MAX_M)
   wave = "rope" if few and Dh % 32 == 0 and k_cache.dtype == torch.bfloat16 and w.shape[0] == (H + 2 * Hkv) * Dh else ""
 
   def rope(M):  # the outputs of the GEMM that rotates and writes by itself
@@ -826,14 +847,14 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
     cfg = _pending_cfg(x, w, bias, "none", wave)
     if cfg is not None and cfg[0] == "wave":
       q, kw = rope(1)
-      x.run_wave(w, None, bias, "none", 2, **kw)
+      x.run(w, None, bias, "none", cfg, **kw)
       return q
     if cfg is None or cfg[2] < 2:
       x = x.materialize()
     else:
       S, N = cfg[2], w.shape[0]
       y = torch.empty(1, N, dtype=torch.bfloat16, device=x.src.device)  # shape carrier only
-      x.run(w, y, None, "none", cfg[1], S, False)
+      x.run(w, y, None, "none", cfg, reduce=False)
       q = torch.empty(1, H, Dh, dtype=torch.bfloat16, device=y.device)
       ws = scratch.splitk(y.device, S * N)
       require().splitk_rope_kv_write(ws, S, bias, pos, cos_sin, slots, q, k_cache, v_cache, int(H), int(Hkv))
@@ -845,7 +866,7 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
     cfg = policy.shuffled_cfg(x, w, bias, None, "none", x.dtype, wave=wave)
     if cfg[0] == "wave":
       q, kw = rope(M)
-      require().gemm_wave(x, w, None, bias, None, K.EPI["none"], 2, **kw)
+      require().gemm_wave(x, w, None, bias, None, K.EPI["none"], cfg[1], **kw)
       return q
     if cfg[0] in ("stream", "big") and cfg[2] > 1:
       S = cfg[2]
