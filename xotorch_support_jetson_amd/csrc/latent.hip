@@ -566,26 +566,37 @@ __global__ __launch_bounds__(256) void latent_attn_merge_k(const float* __restri
   }
 }
 
-// The same for rows of at most 1024 R numbers (a multiple of four): a thread keeps R groups of four values of y and of x in
+// The same for rows of at most 4 NT R numbers (a multiple of four): a thread keeps R groups of four values of y and of x in
 // registers, so each row is read once (the sums run over registers; the variance still after the mean, as the mean of the
-// squared deviations).  y may be S split-K slabs.
-template <typename AT, int R>
-__global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict__ x, const float* __restrict__ y, int ldy,
-                                                               const float* __restrict__ wb, const float* __restrict__ bb,
-                                                               const float* __restrict__ wn, const float* __restrict__ bn,
-                                                               const float* __restrict__ yb, float mult, float eps,
-                                                               AT* __restrict__ out, int ldo, int D, int S, int64_t ss_,
-                                                               int layer) {
+// squared deviations).  y may be S split-K slabs.  Of few rows everything they need is asked for at once: the norm weights, asked
+// for behind each sum, cost a memory latency each, and slabs four at a time one per round (6 x 2048 cold in a graph, one slab 3.9 ->
+// 3.5 us, 11 slabs 6.3 -> 4.5; 4593 rows 29 -> 27.5).
+template <typename AT, int R, int F, int NT>
+__global__ __launch_bounds__(NT) void sandwich_add_norm_reg_k(float* __restrict__ x, const float* __restrict__ y, int ldy,
+                                                              const float* __restrict__ wb, const float* __restrict__ bb,
+                                                              const float* __restrict__ wn, const float* __restrict__ bn,
+                                                              const float* __restrict__ yb, float mult, float eps,
+                                                              AT* __restrict__ out, int ldo, int D, int S, int64_t ss_,
+                                                              int layer) {
   __shared__ float red[8];
   const int64_t t = blockIdx.x;
   float* xr = x + t * D;
+  const float* yr = y ? y + t * ldy : nullptr;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
-  f32x4 xv[R];
+  f32x4 xv[R], wbv[R], wnv[R];
+  Slab4<F> ys[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int i = 4 * (threadIdx.x + 256 * r);
-    xv[r] = i < D ? ld(xr + i) : zero;
+    const int i = 4 * (threadIdx.x + NT * r);
+    xv[r] = wbv[r] = wnv[r] = zero;
+    if (i >= D) continue;
+    xv[r] = ld(xr + i);
+    if (y) {
+      ys[r].ask(yr + i, S, ss_);
+      wbv[r] = ld(wb + i);
+    }
+    if (wn) wnv[r] = ld(wn + i);
   }
   // (shift, scale) of a row held in registers
   auto stats = [&](const f32x4* v, bool center, float* mu, float* rs) {
@@ -599,7 +610,7 @@ __global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict
     float ss = 0.0f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if (4 * (threadIdx.x + 256 * r) >= D) continue;
+      if (4 * (threadIdx.x + NT * r) >= D) continue;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float c = v[r][e] - mean;
@@ -611,14 +622,13 @@ __global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict
     *rs = 1.0f / sqrtf(ss / D + eps);
   };
   if (y) {
-    const float* yr = y + t * ldy;
     f32x4 yv[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int i = 4 * (threadIdx.x + 256 * r);
+      const int i = 4 * (threadIdx.x + NT * r);
       yv[r] = zero;
       if (i < D) {
-        yv[r] = slab4(yr + i, S, ss_);
+        yv[r] = ys[r].sum(yr + i, S, ss_);
         if (yb) yv[r] += ld(yb + i);
       }
     }
@@ -626,9 +636,9 @@ __global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict
     stats(yv, layer || bb, &mu, &rs);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int i = 4 * (threadIdx.x + 256 * r);
+      const int i = 4 * (threadIdx.x + NT * r);
       if (i < D) {
-        f32x4 a = (yv[r] - mu) * rs * ld(wb + i);
+        f32x4 a = (yv[r] - mu) * rs * wbv[r];
         if (bb) a += ld(bb + i);
         xv[r] += mult * a;
         *reinterpret_cast<f32x4*>(xr + i) = xv[r];
@@ -640,9 +650,9 @@ __global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict
     stats(xv, layer || bn, &mu, &rs);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int i = 4 * (threadIdx.x + 256 * r);
+      const int i = 4 * (threadIdx.x + NT * r);
       if (i < D) {
-        f32x4 a = (xv[r] - mu) * rs * ld(wn + i);
+        f32x4 a = (xv[r] - mu) * rs * wnv[r];
         if (bn) a += ld(bn + i);
         st4(out + t * ldo + i, a);
       }
@@ -650,7 +660,7 @@ __global__ __launch_bounds__(256) void sandwich_add_norm_reg_k(float* __restrict
   } else if (out) {  // the stream itself, in the operand dtype
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int i = 4 * (threadIdx.x + 256 * r);
+      const int i = 4 * (threadIdx.x + NT * r);
       if (i < D) st4(out + t * ldo + i, xv[r]);
     }
   }
@@ -715,15 +725,19 @@ void sandwich_add_norm(at::Tensor& x, const c10::optional<at::Tensor>& y, const 
   }
   if (!yp && !op) return;
   for (const float* p : {(const float*)x.data_ptr<float>(), bp, np, bbp, bnp, ybp, (const float*)op}) al(p);
-#define SAN_GO(KERNEL, AT)                                                                                              \
-  KERNEL<<<T, 256, 0, stream()>>>(x.data_ptr<float>(), yp, ldy, bp, bbp, np, bnp, ybp, (float)mult, (float)eps, (AT*)op, ldo, \
-                                  (int)D, S, ss, (int)layer)
-#define SAN_PICK(AT)                                                     \
-  if (vec && D <= 1024) SAN_GO((sandwich_add_norm_reg_k<AT, 1>), AT);      \
-  else if (vec && D <= 2048) SAN_GO((sandwich_add_norm_reg_k<AT, 2>), AT); \
-  else if (vec && D <= 4096) SAN_GO((sandwich_add_norm_reg_k<AT, 4>), AT); \
-  else if (vec && D <= 8192) SAN_GO((sandwich_add_norm_reg_k<AT, 8>), AT); \
-  else SAN_GO(sandwich_add_norm_k<AT>, AT)
+#define SAN_GO(KERNEL, AT, NT)                                                                                          \
+  KERNEL<<<T, NT, 0, stream()>>>(x.data_ptr<float>(), yp, ldy, bp, bbp, np, bnp, ybp, (float)mult, (float)eps, (AT*)op, ldo, \
+                                 (int)D, S, ss, (int)layer)
+#define SAN_PICK(AT)                                                                                           \
+  if (vec && few && S > 1 && D <= 2048) SAN_GO((sandwich_add_norm_reg_k<AT, 1, SLABS_ASKED, 512>), AT, 512);     \
+  else if (vec && few && S > 1 && D <= 4096) SAN_GO((sandwich_add_norm_reg_k<AT, 2, SLABS_ASKED, 512>), AT, 512); \
+  else if (vec && few && D <= 2048) SAN_GO((sandwich_add_norm_reg_k<AT, 1, 1, 512>), AT, 512);                   \
+  else if (vec && D <= 1024) SAN_GO((sandwich_add_norm_reg_k<AT, 1, 1, 256>), AT, 256);                          \
+  else if (vec && D <= 2048) SAN_GO((sandwich_add_norm_reg_k<AT, 2, 1, 256>), AT, 256);                          \
+  else if (vec && D <= 4096) SAN_GO((sandwich_add_norm_reg_k<AT, 4, 1, 256>), AT, 256);                          \
+  else if (vec && D <= 8192) SAN_GO((sandwich_add_norm_reg_k<AT, 8, 1, 256>), AT, 256);                          \
+  else SAN_GO(sandwich_add_norm_k<AT>, AT, 256)
+  const bool few = few_rows(T);
   if (bf) {
     SAN_PICK(uint16_t);
   } else {

@@ -94,6 +94,39 @@ __device__ __forceinline__ f32x4 slab4(const float* p, int S, int64_t ss) {
   return v;
 }
 
+// The same in two halves, so that the loads of up to F slabs are in flight together with whatever else a row needs: a pass over a
+// few rows is a chain of load latencies (most of its data was written by other XCDs a moment ago), not of bytes.  The order of
+// the sum is slab4's.
+template <int F>
+struct Slab4 {
+  f32x4 a[F];
+  __device__ __forceinline__ void ask(const float* p, int S, int64_t ss) {
+    a[0] = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+    for (int i = 1; i < F; ++i)
+      if (i < S) a[i] = *reinterpret_cast<const f32x4*>(p + i * ss);
+  }
+  __device__ __forceinline__ f32x4 sum(const float* p, int S, int64_t ss) const {
+    f32x4 v = a[0];
+#pragma unroll
+    for (int i = 1; i < F; ++i)
+      if (i < S) v += a[i];
+    for (int s0 = F; s0 < S; s0 += 4) {  // (the rest as slab4 takes them)
+      f32x4 b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = *reinterpret_cast<const f32x4*>(p + min(s0 + i, S - 1) * ss);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (s0 + i < S) v += b[i];
+    }
+    return v;
+  }
+};
+constexpr int SLABS_ASKED = 12;  // of a row pass that sums split-K slabs (48 registers a vector of four)
+// A row pass of few rows is its chain of latencies: 512 threads a row, every slab asked for at once.  At 200 rows the bytes of the
+// slabs count already (a step of 200 tokens lost 0.7 % with that form), so the line lies where the decode steps end
+inline bool few_rows(int64_t T) { return T <= 64; }
+
 // ------------------------------------------------------------------ host side
 #define MCHECK(cond, ...) TORCH_CHECK(cond, "xot mixers: ", __VA_ARGS__)
 

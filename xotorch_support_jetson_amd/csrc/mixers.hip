@@ -69,28 +69,44 @@ __global__ void resid_scale_norm_k(float* __restrict__ x, Branch b1, Branch b2, 
   for (int i = threadIdx.x; i < D; i += blockDim.x) stf(out + r * ldo + i, xr[i] * k);
 }
 
-// Rows of at most 1024 R numbers in whole vectors of four: the row stays in registers between the sum of squares and the
+// Rows of at most 4 NT R numbers in whole vectors of four: the row stays in registers between the sum of squares and the
 // write.  Memory-bound on long steps (12807 x 2048, two branches: 127 us with scalar loads and a second pass over x, 74 here);
-// on short ones it saves the slab reduces of both branches' projections, 4.7 us each.
-template <typename AT, int R>
-__global__ __launch_bounds__(256) void resid_scale_norm_reg_k(float* __restrict__ x, Branch b1, Branch b2,
-                                                              const float* __restrict__ gain, float eps, AT* __restrict__ out,
-                                                              int D, int ldo) {
+// on short ones it saves the slab reduces of both branches' projections, 4.7 us each, and is bound by its chain of loads: 48 x
+// 2048 with branches in 8 and 11 slabs 8.0 us four slabs at a time, 5.5 with every load of the row asked for at once.
+template <typename AT, int R, int F, int NT>
+__global__ __launch_bounds__(NT) void resid_scale_norm_reg_k(float* __restrict__ x, Branch b1, Branch b2,
+                                                             const float* __restrict__ gain, float eps, AT* __restrict__ out,
+                                                             int D, int ldo) {
   __shared__ float red[16];
   const int64_t r = blockIdx.x;
   float* xr = x + r * D;
   auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
-  f32x4 v[R];
-  float ss = 0.0f;
+  const float gn = out ? gain[0] : 0.0f;
+  f32x4 v[R], s1[R], s2[R];
+  Slab4<F> y1[R], y2[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int i = 4 * (threadIdx.x + 256 * j);
+    const int i = 4 * (threadIdx.x + NT * j);
     v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (i >= D) continue;
     v[j] = ld(xr + i);
     if (b1.y) {
-      f32x4 a = ld(b1.s + i) * slab4(b1.y + r * b1.ld + i, b1.S, b1.ss);
-      if (b2.y) a += ld(b2.s + i) * slab4(b2.y + r * b2.ld + i, b2.S, b2.ss);
+      y1[j].ask(b1.y + r * b1.ld + i, b1.S, b1.ss);
+      s1[j] = ld(b1.s + i);
+      if (b2.y) {
+        y2[j].ask(b2.y + r * b2.ld + i, b2.S, b2.ss);
+        s2[j] = ld(b2.s + i);
+      }
+    }
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = 4 * (threadIdx.x + NT * j);
+    if (i >= D) continue;
+    if (b1.y) {
+      f32x4 a = s1[j] * y1[j].sum(b1.y + r * b1.ld + i, b1.S, b1.ss);
+      if (b2.y) a += s2[j] * y2[j].sum(b2.y + r * b2.ld + i, b2.S, b2.ss);
       v[j] += a;
       st4(xr + i, v[j]);
     }
@@ -99,10 +115,10 @@ __global__ __launch_bounds__(256) void resid_scale_norm_reg_k(float* __restrict_
   }
   if (!out) return;
   ss = block_sum(ss, red);
-  const float k = gain[0] / sqrtf(ss / (float)D + eps);
+  const float k = gn / sqrtf(ss / (float)D + eps);
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int i = 4 * (threadIdx.x + 256 * j);
+    const int i = 4 * (threadIdx.x + NT * j);
     if (i < D) st4(out + r * ldo + i, v[j] * k);
   }
 }
@@ -846,15 +862,19 @@ void resid_scale_norm(at::Tensor& x, const c10::optional<at::Tensor>& y1, const 
     vec = vec && ldo % 4 == 0 && al(*out);
   }
   const float* g = out.has_value() ? gain->data_ptr<float>() : nullptr;
-#define RSN_GO(AT, ...)                                                                                     \
-  __VA_ARGS__<<<T, 256, 0, stream()>>>(x.data_ptr<float>(), b1, b2, g, (float)eps,                          \
-                                       out.has_value() ? (AT*)out->data_ptr() : nullptr, (int)D, ldo)
-#define RSN_PICK(AT)                                                       \
-  if (vec && D <= 1024) RSN_GO(AT, resid_scale_norm_reg_k<AT, 1>);         \
-  else if (vec && D <= 2048) RSN_GO(AT, resid_scale_norm_reg_k<AT, 2>);    \
-  else if (vec && D <= 4096) RSN_GO(AT, resid_scale_norm_reg_k<AT, 4>);    \
-  else if (vec && D <= 8192) RSN_GO(AT, resid_scale_norm_reg_k<AT, 8>);    \
-  else RSN_GO(AT, resid_scale_norm_k<AT>)
+#define RSN_GO(AT, NT, ...)                                                                                 \
+  __VA_ARGS__<<<T, NT, 0, stream()>>>(x.data_ptr<float>(), b1, b2, g, (float)eps,                           \
+                                      out.has_value() ? (AT*)out->data_ptr() : nullptr, (int)D, ldo)
+#define RSN_PICK(AT)                                                                                          \
+  if (vec && few && slabs && D <= 2048) RSN_GO(AT, 512, resid_scale_norm_reg_k<AT, 1, SLABS_ASKED, 512>);      \
+  else if (vec && few && slabs && D <= 4096) RSN_GO(AT, 512, resid_scale_norm_reg_k<AT, 2, SLABS_ASKED, 512>); \
+  else if (vec && few && D <= 2048) RSN_GO(AT, 512, resid_scale_norm_reg_k<AT, 1, 1, 512>);                    \
+  else if (vec && D <= 1024) RSN_GO(AT, 256, resid_scale_norm_reg_k<AT, 1, 1, 256>);                           \
+  else if (vec && D <= 2048) RSN_GO(AT, 256, resid_scale_norm_reg_k<AT, 2, 1, 256>);                           \
+  else if (vec && D <= 4096) RSN_GO(AT, 256, resid_scale_norm_reg_k<AT, 4, 1, 256>);                           \
+  else if (vec && D <= 8192) RSN_GO(AT, 256, resid_scale_norm_reg_k<AT, 8, 1, 256>);                           \
+  else RSN_GO(AT, 256, resid_scale_norm_k<AT>)
+  const bool few = few_rows(T), slabs = b1.S > 1 || b2.S > 1;
   if (out.has_value() && out->scalar_type() == at::kBFloat16) {
     RSN_PICK(uint16_t);
   } else {

@@ -94,12 +94,14 @@ __global__ __launch_bounds__(NTH) void splitk_resid_rmsnorm_kernel(const float* 
   const int row = blockIdx.x, tid = threadIdx.x, nchunk = D >> 3;
   const size_t base = (size_t)row * D;
   float v[MAXC][8];
+  s16x8 wv[MAXC];  // (asked for with the row: behind the sum it is one more memory latency)
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int c = tid + i * NTH;
     if (c < nchunk) {
       const s16x8 a = ld16(h + base + c * 8);
+      wv[i] = ld16(w + c * 8);
       float acc[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] = bf2f(a[j]);
@@ -164,9 +166,9 @@ __global__ __launch_bounds__(NTH) void splitk_resid_rmsnorm_kernel(const float* 
   for (int i = 0; i < MAXC; ++i) {
     const int c = tid + i * NTH;
     if (c < nchunk) {
-      s16x8 wv = ld16(w + c * 8), o;
+      s16x8 o;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (short)f2bf(v[i][j] * inv * bf2f(wv[j]));
+      for (int j = 0; j < 8; ++j) o[j] = (short)f2bf(v[i][j] * inv * bf2f(wv[i][j]));
       st16(out + base + c * 8, o);
     }
   }

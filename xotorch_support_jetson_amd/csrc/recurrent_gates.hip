@@ -169,23 +169,32 @@ __global__ __launch_bounds__(256) void pair_norm_mean_k(const float* __restrict_
   for (int i = threadIdx.x; i < D; i += blockDim.x) out[t * D + i] = a[i] * ka * w[i] + slab1(b + i, S, ss) * kb * w[D + i];
 }
 
-// Rows of at most 1024 R numbers in whole vectors of four: both rows stay in registers between the sums and the write.
-template <int R>
-__global__ __launch_bounds__(256) void pair_norm_mean_reg_k(const float* __restrict__ y1, int ld1, const float* __restrict__ y2,
-                                                            int ld2, int S, int64_t ss, const float* __restrict__ w, float eps,
-                                                            float* __restrict__ out, int D) {
+// Rows of at most 4 NT R numbers in whole vectors of four: both rows stay in registers between the sums and the write, and
+// every load of a row is asked for before the first is used.
+template <int R, int F, int NT>
+__global__ __launch_bounds__(NT) void pair_norm_mean_reg_k(const float* __restrict__ y1, int ld1, const float* __restrict__ y2,
+                                                           int ld2, int S, int64_t ss, const float* __restrict__ w, float eps,
+                                                           float* __restrict__ out, int D) {
   __shared__ float red[16];
   const int64_t t = blockIdx.x;
   auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
-  f32x4 a[R], b[R];
+  f32x4 a[R], b[R], wa[R], wb[R];
+  Slab4<F> ys[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = 4 * (threadIdx.x + NT * r);
+    if (i >= D) continue;
+    a[r] = ld(y1 + t * ld1 + i);
+    ys[r].ask(y2 + t * ld2 + i, S, ss);
+    wa[r] = ld(w + i);
+    wb[r] = ld(w + D + i);
+  }
   float sa = 0.0f, sb = 0.0f;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int i = 4 * (threadIdx.x + 256 * r);
-    a[r] = b[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int i = 4 * (threadIdx.x + NT * r);
     if (i >= D) continue;
-    a[r] = ld(y1 + t * ld1 + i);
-    b[r] = slab4(y2 + t * ld2 + i, S, ss);
+    b[r] = ys[r].sum(y2 + t * ld2 + i, S, ss);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       sa += a[r][e] * a[r][e];
@@ -197,8 +206,8 @@ __global__ __launch_bounds__(256) void pair_norm_mean_reg_k(const float* __restr
   const float ka = 0.5f / sqrtf(sa / (float)D + eps), kb = 0.5f / sqrtf(sb / (float)D + eps);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const int i = 4 * (threadIdx.x + 256 * r);
-    if (i < D) *reinterpret_cast<f32x4*>(out + t * D + i) = a[r] * ka * ld(w + i) + b[r] * kb * ld(w + D + i);
+    const int i = 4 * (threadIdx.x + NT * r);
+    if (i < D) *reinterpret_cast<f32x4*>(out + t * D + i) = a[r] * ka * wa[r] + b[r] * kb * wb[r];
   }
 }
 
@@ -338,13 +347,17 @@ void pair_norm_mean(const at::Tensor& y1, const at::Tensor& y2, const at::Tensor
   if (T == 0) return;
   MCHECK(y1.size(0) == T && p2.T == T && y1.size(1) >= D && p2.n >= D && w.numel() == 2 * D, "pair_norm_mean: shape mismatch");
   auto al = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
-#define PNM_GO(KERNEL)                                                                                                  \
-  KERNEL<<<T, 256, 0, stream()>>>(y1.data_ptr<float>(), ld1, p2.p, p2.ld, p2.S, p2.ss, w.data_ptr<float>(), (float)eps, \
-                                  out.data_ptr<float>(), (int)D)
+#define PNM_GO(NT, KERNEL)                                                                                             \
+  KERNEL<<<T, NT, 0, stream()>>>(y1.data_ptr<float>(), ld1, p2.p, p2.ld, p2.S, p2.ss, w.data_ptr<float>(), (float)eps, \
+                                 out.data_ptr<float>(), (int)D)
   const bool vec = p2.vec && D % 4 == 0 && ld1 % 4 == 0 && al(y1) && al(w) && al(out);
-  if (vec && D <= 2048) PNM_GO(pair_norm_mean_reg_k<2>);
-  else if (vec && D <= 4096) PNM_GO(pair_norm_mean_reg_k<4>);
-  else PNM_GO(pair_norm_mean_k);
+  const bool few = few_rows(T);
+  if (vec && few && p2.S > 1 && D <= 2048) PNM_GO(512, (pair_norm_mean_reg_k<1, SLABS_ASKED, 512>));
+  else if (vec && few && p2.S > 1 && D <= 4096) PNM_GO(512, (pair_norm_mean_reg_k<2, SLABS_ASKED, 512>));
+  else if (vec && few && D <= 2048) PNM_GO(512, (pair_norm_mean_reg_k<1, 1, 512>));
+  else if (vec && D <= 2048) PNM_GO(256, (pair_norm_mean_reg_k<2, 1, 256>));
+  else if (vec && D <= 4096) PNM_GO(256, (pair_norm_mean_reg_k<4, 1, 256>));
+  else PNM_GO(256, pair_norm_mean_k);
 #undef PNM_GO
 }
 

@@ -335,7 +335,11 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
       p[j] = P + (int64_t)(t0 + min(i, nt - 1)) * ldp + off + e - i * rank;
       v[j] = 0.0f;
     }
-    for (int k0 = 0; k0 < S; k0 += 8) {
+    if (S == 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = *p[j];
+    }
+    for (int k0 = 0; S > 1 && k0 < S; k0 += 8) {
       float a[8][4];
 #pragma unroll
       for (int k = 0; k < 8; ++k)

@@ -472,12 +472,12 @@ class ShardModel:
     return linear(x, w, out_dtype=torch.float32)
 
   @staticmethod
-  def _proj_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0) -> torch.Tensor:
-    """The same for a consumer that sums unreduced split-K slabs itself (and runs before the next GEMM of its scratch slot):
-    [T, n] or [S, T, n]."""
+  def _proj_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0, once: bool = True) -> torch.Tensor:
+    """The same for consumers that sum unreduced split-K slabs themselves (and run before the next GEMM of their scratch slot):
+    [T, n] or [S, T, n].  once: one pass over rows reads them."""
     if x.dtype == torch.float32 or not x.is_cuda:
       return ShardModel._proj(x, w)
-    return linear_slabs(x, w, slot)
+    return linear_slabs(x, w, slot, once)
 
   @staticmethod
   def _fused_act(x: torch.Tensor, w: torch.Tensor, epi: str, limit: float = 0.0) -> Optional[torch.Tensor]:
@@ -617,13 +617,14 @@ class ShardModel:
       # first, so that choosing a kernel for the other does not write over them)
       y2 = self._proj_slabs(act, lw.down_w, slot=1) if s.ff else None
       y1 = self._proj_slabs(mix, lw.out_w)
-      nxt = w.layers[self.layer_ids[j + 1]].norm_g if j + 1 < n else None
+      nxt = w.layers[self.layer_ids[j + 1]].norm_g if j + 1 < n else w.norm if last and inp.all_rows else None
       K.resid_scale_norm(h, y1, lw.ls1, y2, lw.ls2 if y2 is not None else None, gain=nxt, eps=c.rms_norm_eps,
                          out=hn if nxt is not None else None)
     if not last:
       return h
     hl, xn = self._last_rows(h, inp, hn)
-    K.resid_scale_norm(hl, gain=w.norm, eps=c.rms_norm_eps, out=xn)
+    if not (n and inp.all_rows):  # (a step whose rows all ask for logits: the last layer's pass normed them)
+      K.resid_scale_norm(hl, gain=w.norm, eps=c.rms_norm_eps, out=xn)
     logits = self._proj(xn, w.lm_head)[:, :c.vocab_size]
     return logits * c.logit_scale if c.logit_scale != 1.0 else logits
 
@@ -1015,6 +1016,9 @@ class ShardModel:
     eps, mult = c.rms_norm_eps, c.residual_mult
     ln = c.norm_kind == "layer"
     fresh = True  # hn does not hold this run's normed input yet
+    # the head's norm is the last run's next norm, where every row asks for logits and nothing else still reads the stream
+    ends_here = (self.shard.is_last_layer() and inp.all_rows and bool(runs) and w.norm is not None
+                 and w.layers[runs[-1][0]].side_norm is None)
     for j, (li, t) in enumerate(runs):
       lw = w.layers[li]
       s = lw.spec
@@ -1033,7 +1037,7 @@ class ShardModel:
       # (projections whose readers sum split-K slabs themselves, all of them before the next GEMM: window attention alone,
       # and everything behind short convolutions)
       sums = s.wattn is not None and s.wattn.gate == "none" and not pair or lw.conv_units is not None
-      P = (self._proj_slabs if sums else self._proj)(hn, lw.in_w)
+      P = self._proj_slabs(hn, lw.in_w, once=False) if sums else self._proj(hn, lw.in_w)
       mix = rows("mix", lw.mix_cols["mix"][1], lw.out_w.shape[1])
       if s.lattn is not None:
         self._latent_attn(P, lw, j, inp, mix, rows)
@@ -1064,7 +1068,10 @@ class ShardModel:
       # the norm that follows this run: the next run's input norm unless a pass starts there
       nl = w.layers[runs[j + 1][0]] if j + 1 < len(runs) and runs[j + 1][1] < 0 else None
       nxt, nxt_b = (nl.norm1, nl.norm1_b) if nl is not None else (None, None)
-      hn_nxt = hn if nl is not None else None
+      ends = ends_here and j + 1 == len(runs)
+      if ends:
+        nxt, nxt_b = w.norm, w.norm_b
+      hn_nxt = hn if nl is not None or ends else None
       after = (lw.side_norm is not None, f is not None)  # what still reads hn in this layer: the side input, the feed-forward
       if f is None:
         K.sandwich_add_norm(h, y, lw.norm1b, nxt, eps, hn if after[0] else hn_nxt, bb=lw.norm1b_b, bn=nxt_b, mult=mult,
@@ -1099,7 +1106,8 @@ class ShardModel:
     if not self.shard.is_last_layer():
       return torch.cat([h, ids.to(torch.float32)[:, None]], 1) if c.side_dim else h
     hl, xn = self._last_rows(h, inp, hn)
-    K.sandwich_add_norm(hl, None, None, w.norm, eps, xn, bn=w.norm_b, layer=ln)
+    if not ends_here:
+      K.sandwich_add_norm(hl, None, None, w.norm, eps, xn, bn=w.norm_b, layer=ln)
     logits = self._proj(xn, w.lm_head)[:, :c.vocab_size]
     if c.logit_softcap > 0:
       logits = torch.tanh(logits / c.logit_softcap) * c.logit_softcap

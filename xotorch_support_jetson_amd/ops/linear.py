@@ -423,16 +423,17 @@ class GemmPolicy:
     top = sorted(busiest, key=lambda nt: (busiest[nt], -nt))[:3]
     return [("wave", nt, 1) for nt in top if busiest[nt] * 256 <= 1.4 * tiles]
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "") -> Tuple:
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", slabs: bool = False) -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
-    reduce, timed with them, stands for the launch that does it there)."""
+    reduce, timed with them, stands for the launch that does it there).  slabs: the caller's consumer reads split-K slabs
+    itself, so a split is timed without their reduce (2048 x 5632 at 6 rows: 9.1 us whole, 6.4 in 11 slabs, 10.2 with the reduce)."""
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WIDE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
     # (a residual product's plain entry belongs to linear_resid_norm, which sums the slabs itself; a caller that does not
     # take the whole-K GEMM passes over such an entry)
-    kind = "sh" + wave if wave == "rope" or epi == "resid" else "sh"
+    kind = "sl" if slabs else "sh" + wave if wave == "rope" or epi == "resid" else "sh"
     key = (kind, _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
     got = self._lookup(key)
     if got is not None and got[0] == "wave" and not wave:
@@ -475,7 +476,8 @@ class GemmPolicy:
     times = {}
     for cfg in cands:
       try:
-        times[cfg] = self._time(lambda: _shuffled_call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
+        call = _slab_call if slabs and cfg[2] > 1 else _shuffled_call
+        times[cfg] = self._time(lambda: call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
       except RuntimeError:
         pass
     got = _tie_break(times, M) if times else cands[0]
@@ -602,6 +604,17 @@ def _shuffled_call(x, w, bias, residual, epi, out, cfg, epi_arg: float = 0.0):
   ws = scratch.splitk(x.device, S * M * N) if S > 1 else None
   require().gemm_big(x, w, out, bias, residual, ws, K.EPI[epi], bn, S, True, epi_arg)
   return out
+
+
+def _slab_call(x, w, bias, residual, epi, out, cfg, slot: int = 0):
+  """The split-K slabs of x @ w.T (cfg[2] > 1), left unreduced in the scratch slot; out: fp32 [M, N], a shape carrier only."""
+  kind, tile, S = cfg
+  ws = scratch.splitk(x.device, S * out.numel(), slot)
+  if kind == "stream":
+    require().gemm_stream(x, w, out, None, None, ws, K.EPI["none"], tile, S, True, False)
+  else:
+    require().gemm_big(x, w, out, None, None, ws, K.EPI["none"], tile, S, False)
+  return ws[:S * out.numel()].view(S, *out.shape)
 
 
 def _run_rowmajor(impl, x, w, bias, residual, epi, out, out_dtype):
@@ -747,24 +760,18 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, r
   return out
 
 
-def linear_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0) -> torch.Tensor:
+def linear_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0, once: bool = True) -> torch.Tensor:
   """fp32 x @ w.T for a consumer that sums split-K slabs itself: [M, N], or [S, M, N] when the projection runs split over K
   (a view of the shared scratch: valid until the next split-K GEMM of its slot, where choosing a configuration counts as one
-  of slot 0)."""
+  of slot 0).  once: one pass over rows reads the slabs, of few rows as cheaply as one result; otherwise (several kernels, one that
+  reads a row many times, or rows whose slabs are the bytes that count: 200 x 2048 lost 1 % of a step) a split is chosen as if it
+  had to be reduced first."""
   if x.is_cuda and layout_of(w) == "stream":
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
-    M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y")
-    S = cfg[2]
-    if S > 1:
-      ws = scratch.splitk(x.device, S * M * N, slot)
-      y = torch.empty(M, N, dtype=torch.float32, device=x.device)  # shape carrier only: the slabs are not reduced
-      if cfg[0] == "stream":
-        require().gemm_stream(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, True, False)
-      else:
-        require().gemm_big(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, False)
-      return ws[:S * M * N].view(S, M, N)
+    y = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y", slabs=once and x.shape[0] <= WIDE_MAX_M)
+    return _slab_call(x, w, None, None, "none", y, cfg, slot) if cfg[2] > 1 else _shuffled_call(x, w, None, None, "none", y, cfg)
   return linear(x, w, out_dtype=torch.float32)
 
 
