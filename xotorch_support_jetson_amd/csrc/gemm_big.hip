@@ -29,9 +29,9 @@ namespace xot {
 
 
 // AUXA / AUXB: cache-policy bits of the X / W LDS-DMA loads (sc0 = 1, nt = 2, sc1 = 16)
-// MOE = 1 / 2: grouped GEMM over experts (blockIdx.y = expert e, weight W[e], rows moe_off[e] ..
+// MOE = 1 / 2: grouped GEMM over group_m experts (a 1-D grid; expert e: weight W[e], rows moe_off[e] ..
 // moe_off[e+1] of the expert-sorted slot order; MOE 2 gathers X row moe_gather[slot]); M is the
-// worst-case rows per expert (row tiles past an expert's count exit at once, so the grid is fixed and
+// worst-case rows per expert (workgroups past an expert's row tiles exit at once, so the grid is fixed and
 // graph-capturable).  A K split writes fp32 partial slabs ysplit elements apart (summed by the consumer).
 // MOE = 4: K-grouped GEMM (the weight gradients of grouped experts): blockIdx.y = group e multiplies the k
 // range [moe_off[e], moe_off[e+1]) (multiples of BK) of the shared operands X [M, K] and W [N, K] into
@@ -86,10 +86,30 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
   const int wm = wave / WN, wn = wave % WN;
 
   // ---- tile of this workgroup (bijective XCD remap, then split-major / column / row order, grouped when tall)
-  const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;  // N % BN != 0: a masked last column tile
+  // Grouped over E = group_m experts (grid: the tiles of max_rows rows of each): the workgroups past an expert's own tiles leave at
+  // once, and they are its last: between the working ones, every second or fourth workgroup, they kept half or more of the shader
+  // engines, which workgroups go to in turn, without work.  Where one row of tiles fills those evenly, expert follows expert
+  // (8 experts of 28672 x 4096 at 150 tokens 418 -> 325 us, at 400 811 -> 368); smaller experts (turns) advance side by side, position p
+  // of all before position p + 1 of any, or the leaving ones of one come between the tiles of two (64 of 2048 x 1408 at 850 tokens
+  // 232 -> 90).  Their rotation spreads each over the XCDs, positions p and p + 8 on one (E a multiple of 8).
+  const int ntiles = (N + BN - 1) / BN;  // N % BN != 0: a masked last column tile
+  const bool turns = (MOE == 1 || MOE == 2) && ntiles * S < 32;
+  int row0 = 0, Mv = M, expert = 0, pos = 0;  // first output row (slot) and valid rows of this launch's row range
+  if constexpr (MOE == 1 || MOE == 2) {
+    const int E = group_m, per = gridDim.x / E;
+    pos = turns ? blockIdx.x / E : blockIdx.x % per;
+    expert = turns ? (blockIdx.x - pos * E + pos) % E : blockIdx.x / per;
+    row0 = moe_off[expert];
+    Mv = moe_off[expert + 1] - row0;
+  }
+  const int mtiles = (min(M, Mv) + BM - 1) / BM;
   const int nwg = mtiles * ntiles * S;
   int b = blockIdx.x;
-  {
+  if constexpr (MOE == 1 || MOE == 2) {
+    b = pos;
+    if (b >= nwg) return;  // uniform over the workgroup, before any barrier
+  }
+  if (!turns) {
     const int xcd = b & 7, q = nwg >> 3, r = nwg & 7;
     b = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (b >> 3);
   }
@@ -103,7 +123,11 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
     const int tiles = mtiles * ntiles;
     split = b / tiles;
     const int bt = b - split * tiles;
-    if ((MOE == 0 || MOE == 4) && group_m > 1 && mtiles >= 2 * group_m) {
+    if (turns) {  // the row tiles of a column 8 positions apart: its weights from one L2
+      const int per = 8 * mtiles, q = bt / per, rem = bt - q * per, w = min(8, ntiles - 8 * q);
+      mt = rem / w;
+      nt = 8 * q + rem % w;
+    } else if ((MOE == 0 || MOE == 4) && group_m > 1 && mtiles >= 2 * group_m) {
       const int per = group_m * ntiles, grp = bt / per, first = grp * group_m;
       const int gm = min(mtiles - first, group_m), rr = bt - grp * per;
       mt = first + rr % gm;
@@ -114,13 +138,8 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
     }
   }
   const int m0 = mt * BM, n0 = nt * BN;
-  int row0 = 0, Mv = M;  // first output row (slot) and valid rows of this launch's row range
   if constexpr (MOE == 1 || MOE == 2) {
-    const int e = blockIdx.y;
-    row0 = moe_off[e];
-    Mv = moe_off[e + 1] - row0;
-    W += (size_t)e * N * K;
-    if (m0 >= Mv) return;  // uniform over the workgroup, before any barrier
+    W += (size_t)expert * N * K;
     if (ysplit != 0) Yv = reinterpret_cast<float*>(Yv) + (size_t)split * ysplit;
   }
   const int T_all = K / BK;
@@ -663,9 +682,9 @@ static void big_moe_launch(const uint16_t* X, int ldx, const uint16_t* W, void* 
   static bool attr = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) ==
                      hipSuccess;
   (void)attr;
-  dim3 grid(((max_rows + BM - 1) / BM) * (N / BN) * S, E);
+  const dim3 grid((unsigned)E * ((max_rows + BM - 1) / BM) * (N / BN) * S);
   kern<<<grid, 512, SMEM, st>>>(X, ldx, W, nullptr, nullptr, 0, Y, ldy, nullptr, max_rows, N, K, S, off, gather,
-                                S > 1 ? ysplit : 0L, 4, epi_arg);
+                                S > 1 ? ysplit : 0L, E, epi_arg);
 }
 
 // bm = row tile (128 / 192 / 256) + 1000 x pipeline variant: 0 = two 64-deep LDS stages (one in flight under
