@@ -656,9 +656,18 @@ void gemm_moe(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const at:
                                   off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, (int)splits,
                                   (long)(slots * y.size(1)), (int)big_bm, (float)epi_arg, cur_stream());
   } else {
-    rc = xot::launch_gemm_moe(bf(x), (int)x.stride(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,
-                              off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, wshuf, (int)splits,
-                              (long)(slots * y.size(1)), (float)epi_arg, cur_stream());
+    // many small experts, or more tokens than the streaming kernel's 64-row tile: gemm_group, which works through the rows an
+    // expert has.  gate/up + down, us, gemm_stream / gemm_group: 64 experts of 1408 x 2048 at 4 tokens 41 + 31 / 40 + 26, 37
+    // 133 + 59 / 123 + 58, 130 213 + 117 / 130 + 66; 8 of 14336 x 4096 at 64 tokens 311 + 143 / 316 + 148, at 90 365 + 156 / 318 + 151
+    rc = -1;
+    if (wshuf && (E > 16 || max_rows > 64))
+      rc = xot::launch_gemm_group(bf(x), (int)x.stride(0), (int)x.size(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,
+                                  off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, (int)splits,
+                                  (long)(slots * y.size(1)), (float)epi_arg, cur_stream());
+    if (rc != 0)
+      rc = xot::launch_gemm_moe(bf(x), (int)x.stride(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,
+                                off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, wshuf, (int)splits,
+                                (long)(slots * y.size(1)), (float)epi_arg, cur_stream());
   }
   XCHECK(rc == 0, "gemm_moe: unsupported shape N=", N, " K=", K, " epi=", epi, " splits=", splits);
 }

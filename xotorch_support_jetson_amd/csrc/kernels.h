@@ -119,6 +119,9 @@ void launch_splitk_resid_rmsnorm(const float* ws, int S, const uint16_t* bias, u
 int launch_gemm_moe_big(const uint16_t* X, int ldx, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi,
                         const int* off, const int* gather, int E, int max_rows, int N, int K, int S, long ysplit,
                         int bm, float epi_arg, hipStream_t s);
+// grouped decode GEMM of routed experts on pre-shuffled weights (gemm_group.hip); X has xrows rows
+int launch_gemm_group(const uint16_t* X, int ldx, int xrows, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi, const int* off,
+                      const int* gather, int E, int max_rows, int N, int K, int S, long ysplit, float epi_arg, hipStream_t st);
 // grouped GEMM over experts: rows of expert e are off[e]..off[e+1] (slot order), W is [E][N][K]
 int launch_gemm_moe(const uint16_t* X, int ldx, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi,
                     const int* off, const int* gather, int E, int max_rows, int N, int K, bool wshuf, int S,

@@ -34,8 +34,8 @@ from ..ops.rope import longrope_window, rope_shift, rope_table
 from .config import ModelConfig
 from .weights import ShardWeights, expert
 
-# average rows per expert above which the grouped expert GEMMs run on gemm_big tiles
-MOE_BIG_MIN_ROWS = float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", "24"))
+# average rows per expert from which the grouped expert GEMMs run on gemm_big tiles: at most 16 experts, more
+MOE_TILE_ROWS = (16, 32)
 # K splits of the grouped gate/up GEMM for decode-sized batches (1: fused SiLU epilogue, no slabs)
 MOE_GU_SPLITS = int(os.environ.get("XOT_MOE_GU_SPLITS", "4"))
 MOE_BM = int(os.environ.get("XOT_MOE_BM", "0"))  # force the grouped gemm_big tile code (tests, A/B)
@@ -51,20 +51,20 @@ GELU_EPI_ROWS, GELU_EPI_SIZE = 1024, 1 << 23
 LOW_RANK_GEMM_ROWS = int(os.environ.get("XOT_LOW_RANK_GEMM_ROWS", "256"))
 
 
-def moe_tiles(rows: float, E: int) -> Tuple[int, int, int]:
-  """(gate/up tile code, down tile code, down K split) of the grouped expert GEMMs on gemm_big tiles at `rows`
-  average rows per expert.  Tile code = row tile + 1000 for the deeper LDS pipeline (three 64-deep stages for
-  128 rows: more expert-weight bytes in flight, which is what the HBM-bound small groups need).  Measured at
-  Mixtral shapes (tools/bench_moe.py, profiles/r3/moe_tiles/): ~32 rows gate/up 315 us (1128) vs 356 (128),
-  down 144 (1128, S 2) vs 166; ~64 rows gate/up 441 (1128) vs 566 (128), down 178 (256, S 2) vs 288 (128, S 2);
-  ~128 rows 192-row tiles (gate/up 439 us, down 254 at S 4).  Many small experts (DeepSeek-V2-Lite, 64 x ~24
-  rows) keep 256-row tiles (11.0 vs 12.6 ms per step with 128)."""
-  if rows <= 96 and E > 16:
-    return 256, 256, 2
-  if rows <= 48:
-    return 1128, 1128, 2
+def moe_tiles(T: int, k: int, E: int) -> Tuple[int, int, int]:
+  """(gate/up tile code, down tile code, down K split) of the grouped expert GEMMs of T tokens with k of E experts each on
+  gemm_big tiles, or (0, 0, 0): the weight-streaming kernels (csrc/gemm_group.hip, gemm.hip), which are bound by the expert weights
+  as long as few rows meet them.  Tile code = row tile, + 1000 with a deeper LDS pipeline, + 2000 on the two-phase ping-pong
+  schedule.  gate/up + down, us, at rows = T k / E; all of them sum in the same order.  Many small experts (64 of 1408 x 2048):
+  24 rows 133 + 71 streamed, 136 + 72 (2128), 182 + 85 (2256); 48 rows 150 + 81, 139 + 76, 170 + 86; 94 rows 296 + 155, 152 + 88,
+  186 + 92; 192 rows 292 + 171 (2128), 209 + 118 (2256).  Few large ones (8 of 14336 x 4096): 16 rows (up to 64 tokens) 311 + 143
+  streamed, 22 rows 365 + 156 streamed, 330 + 142 (1128); 64 rows 343 + 148 (1128), 419 + 184 (2256), 375 + 157 (2192); 128 rows
+  485 + 248, 448 + 190, 404 + 172."""
+  rows = T * k / E
+  if rows < MOE_TILE_ROWS[E > 16] or (E <= 16 and T <= 64 and rows < 24):
+    return 0, 0, 0
   if rows <= 96:
-    return 1128, 256, 2
+    return (2128, 2128, 2) if E > 16 else (1128, 1128, 2)
   if rows <= 160:
     return 192, 192, 4
   return 256, 256, 2
@@ -429,8 +429,7 @@ class ShardModel:
     shuffled = layout_of(lw.gu_w) == "stream" and layout_of(lw.down_w) == "stream"
     # rows per expert decide the kernel: the weight-streaming GEMM for decode-sized groups, gemm_big
     # tiles (128 or 256 rows) once the groups are compute-bound
-    rows = T * k / E
-    bm, bm_dn, S_dn = (0, 0, 0) if not shuffled or rows < MOE_BIG_MIN_ROWS else moe_tiles(rows, E)
+    bm, bm_dn, S_dn = moe_tiles(T, k, E) if shuffled and F % 128 == 0 and D % 256 == 0 else (0, 0, 0)
     if MOE_PP2:  # 256- / 192-row expert tiles on the two-phase ping-pong schedule (csrc/gemm_big.hip 2256 / 2192)
       bm, bm_dn = ({256: 2256, 192: 2192}.get(b, b) for b in (bm, bm_dn))
     if MOE_BM and bm:
@@ -799,12 +798,10 @@ class ShardModel:
       # for decode-sized groups (down projection split over K), gemm_big tiles once the groups are compute-bound
       C = require()
       sh_up, sh_dn = layout_of(lw.ex_up_w) == "stream", layout_of(lw.ex_down_w) == "stream"
-      per_expert = T * k / E
-      big = sh_up and sh_dn and per_expert >= MOE_BIG_MIN_ROWS and Fp % 256 == 0 and Dq % 256 == 0
-      bm, bm_dn, S_dn = moe_tiles(per_expert, E) if big else (0, 0, 0)
+      bm, bm_dn, S_dn = moe_tiles(T, k, E) if sh_up and sh_dn and Fp % 256 == 0 and Dq % 256 == 0 else (0, 0, 0)
       if MOE_PP2:
         bm, bm_dn = ({256: 2256, 192: 2192}.get(t, t) for t in (bm, bm_dn))
-      S = S_dn if big else (4 if T * k <= 64 else 2)
+      S = S_dn if bm else (4 if T * k <= 64 else 2)
       if Fp % (256 * S):
         S = 1
       up = torch.empty(T * k, Fp, dtype=torch.float32, device=dev)
@@ -938,12 +935,10 @@ class ShardModel:
     if hn.dtype == torch.bfloat16 and hn.is_cuda:
       C = require()
       sh_up, sh_dn = layout_of(lw.ex_up_w) == "stream", layout_of(lw.ex_down_w) == "stream"
-      per_expert = T * k / E
-      big = sh_up and sh_dn and per_expert >= MOE_BIG_MIN_ROWS and Fp % 256 == 0 and Dq % 256 == 0
-      bm, bm_dn, S_dn = moe_tiles(per_expert, E) if big else (0, 0, 0)
+      bm, bm_dn, S_dn = moe_tiles(T, k, E) if sh_up and sh_dn and Fp % 256 == 0 and Dq % 256 == 0 else (0, 0, 0)
       if MOE_PP2:
         bm, bm_dn = ({256: 2256, 192: 2192}.get(t, t) for t in (bm, bm_dn))
-      S = S_dn if big else (4 if T * k <= 64 else 2)
+      S = S_dn if bm else (4 if T * k <= 64 else 2)
       if Fp % (256 * S):
         S = 1
       act = torch.empty(T * k, Fp, dtype=torch.bfloat16, device=dev)  # the gated activation in the GEMM's epilogue
