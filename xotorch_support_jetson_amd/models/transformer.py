@@ -547,23 +547,20 @@ class ShardModel:
     per-head gated RMS norm, scaled into the mixers' output row."""
     r, st, dev = lw.spec.rec, self.state, P.device
     T = P.shape[0]
-    H, G, d, dv = r.heads, r.kv_heads, r.dim, r.vdim
-    o = torch.empty(T, H * dv, dtype=torch.float32, device=dev)
+    H, G, d = r.heads, r.kv_heads, r.dim
+    (go, gn), (off, n) = lw.cols["rg"], lw.mix_cols["rec"]
+    norm = (lw.rec_norm, P[:, go:go + gn], False, self.c.rms_norm_eps, lw.spec.rec_scale, mix[:, off:off + n])
     if r.rule == "delta":
       beta = torch.empty(T, H, dtype=torch.float32, device=dev)
       decay = torch.empty(T, H, dtype=torch.float32, device=dev)
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
                        delta=(lw.cols["rb"][0], lw.cols["ra"][0], lw.dt_bias, lw.A_log, beta, decay))
-      K.linear_recurrence(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], decay, beta, 1.0, st.S[j],
-                          inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
+      K.recurrence_norm(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], decay, beta, 1.0, st.S[j],
+                        inp.state_slots, inp.cu_q, *norm, max_qlen=inp.max_qlen)
     else:
-      decay = torch.empty(T, H * d, dtype=torch.float32, device=dev)
-      K.gla_prep(P, lw.cols["ra1"][0], lw.a2_w, lw.a2_b, r.tau, decay)
       (qo, qn), (ko, kn), (vo, vn) = lw.cols["rq"], lw.cols["rk"], lw.cols["rv"]
-      K.linear_recurrence(P[:, qo:qo + qn], P[:, ko:ko + kn], P[:, vo:vo + vn], decay, None, d ** -0.5, st.S[j],
-                          inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
-    off, n = lw.mix_cols["rec"]
-    K.gated_rmsnorm(o, lw.rec_norm, P, lw.cols["rg"][0], self.c.rms_norm_eps, lw.spec.rec_scale, mix[:, off:off + n])
+      K.recurrence_norm(P[:, qo:qo + qn], P[:, ko:ko + kn], P[:, vo:vo + vn], None, None, d ** -0.5, st.S[j], inp.state_slots,
+                        inp.cu_q, *norm, gla=(P, lw.cols["ra1"][0], lw.a2_w, lw.a2_b, r.tau), max_qlen=inp.max_qlen)
 
   def _forward_mixed(self, x: torch.Tensor, inp: StepInputs) -> torch.Tensor:
     """Layers of config.layer_specs on an fp32 residual stream h:
@@ -744,9 +741,8 @@ class ShardModel:
       gate = torch.empty(T, nv, dtype=torch.float32, device=dev)
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
                        gates=(lw.cols["rb"][0], beta, a0, lw.a2_w, lw.dt_bias, lw.A_log, decay, g0, lw.g2_w, gate))
-    o = torch.empty(T, nv, dtype=torch.float32, device=dev)
-    K.linear_recurrence(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], decay, beta, 1.0, st.S[j], inp.state_slots, inp.cu_q, o, max_qlen=inp.max_qlen)
-    K.gated_group_norm(o, None, lw.rec_norm, gate, 0, H, self.c.rms_norm_eps, mix)
+    K.recurrence_norm(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], decay, beta, 1.0, st.S[j], inp.state_slots, inp.cu_q,
+                      lw.rec_norm, gate, True, self.c.rms_norm_eps, 1.0, mix, max_qlen=inp.max_qlen)
 
   def _ssd_conv(self, P: torch.Tensor, x: torch.Tensor, dt: torch.Tensor, decay: torch.Tensor, lw, j: int, inp: StepInputs,
                 mix: torch.Tensor) -> None:

@@ -599,6 +599,28 @@ def gated_rmsnorm(o, w, P, g_off: int, eps: float, out_scale: float, out) -> Non
   _mix("gated_rmsnorm", _gpu(o))(o, w, P, int(g_off), float(eps), float(out_scale), out)
 
 
+def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu_q, w, gate, sigmoid: bool, eps: float, scale: float,
+                    out, gla=None, max_qlen: int = 0) -> None:
+  """linear_recurrence, then each head's RMS norm times w ([dv], or one per head [H dv]), gate [T, H dv]'s silu (or its logistic
+  function) and scale -> out [T, >= H dv].  gla: (P, first column, a2, a2_b, tau) of gla_prep, which then makes the decays.  A step
+  of single tokens is one launch on the GPU (csrc/recurrence_step.hip) where that covers the sizes."""
+  if max_qlen == 1 and _gpu(q):
+    a1, a2, a2_b, tau = (gla[0][:, gla[1]:gla[1] + gla[2].shape[1]], *gla[2:]) if gla is not None else (None, None, None, 0.0)
+    if require().recurrence_step(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, a1, a2, a2_b, float(tau), w, gate,
+                                 bool(sigmoid), float(eps), float(scale), out):
+      return
+  T, H, dv, d = q.shape[0], state.shape[1], state.shape[2], state.shape[3]
+  if gla is not None:
+    decay = torch.empty(T, H * d, dtype=torch.float32, device=q.device)
+    gla_prep(*gla, decay)
+  o = torch.empty(T, H * dv, dtype=torch.float32, device=q.device)
+  linear_recurrence(q, k, v, decay, beta, q_scale, state, state_slots, cu_q, o, max_qlen=max_qlen)
+  if sigmoid:
+    gated_group_norm(o, None, w, gate, 0, H, eps, out)
+  else:
+    gated_rmsnorm(o, w, gate, 0, eps, scale, out[:, :H * dv])
+
+
 # ------------------------------------------------------------------ post-norm blocks (csrc/hybrid.hip)
 pool_dims = ref.pool_dims
 
