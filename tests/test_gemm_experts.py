@@ -74,3 +74,44 @@ def test_group_epilogues(gpu, E):
   C.gemm_moe(x, ws, a, off, tok, K.EPI["clamp_glu"], T, True, 1, 0, 7.0)
   gc, uc = gate.clamp(max=7.0), up.clamp(-7.0, 7.0)
   torch.testing.assert_close(a.cpu().double(), gc * torch.sigmoid(1.702 * gc) * (uc + 1), rtol=2 ** -7, atol=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 16, 64, 65, 150])
+@pytest.mark.parametrize("n", [1, 2])
+@pytest.mark.parametrize("N,Kd,S", [(256, 128, 1), (128, 1408, 1), (384, 1024, 4)])
+def test_shared_experts_exact(gpu, T, n, N, Kd, S):
+  """Shared experts of every token behind the routed ones: matrices of n N rows and of n K columns, bit for bit on integers, and
+  their rows in the combine (bf16 of an fp32 sum: one rounding)."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  C = require()
+  g = torch.Generator().manual_seed(T + n + N)
+  E, k = 17, 2
+  x, w, wr, wc = integers(g, T, Kd), integers(g, E, N, Kd), integers(g, n * N, Kd), integers(g, N, n * Kd)
+  topi = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)])
+  order = torch.argsort(topi.reshape(-1), stable=True)
+  off = torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(topi.reshape(-1), minlength=E).cumsum(0)]).int()
+  tok, routed, slots = (order // k).int(), T * k, T * (k + n)
+  ws = torch.stack([shuffle_for_stream(m.to(gpu)) for m in w])
+  shr, shc = shuffle_for_stream(wr.to(gpu)), shuffle_for_stream(wc.to(gpu))
+  full = torch.cat([x[tok[off[e]:off[e + 1]].long()].float() @ w[e].float().t() for e in range(E)])
+  y = torch.full((S * slots, N), 7.0, device=gpu)
+  C.gemm_moe(x.to(gpu), ws, y, off.to(gpu), tok.to(gpu), K.EPI["none"], T, True, S, 0, w_sh=shr)
+  got = y.view(S, slots, N).sum(0).cpu()
+  assert torch.equal(got[:routed], full)
+  assert torch.equal(got[routed:], torch.cat([x.float() @ wr[j * N:(j + 1) * N].float().t() for j in range(n)]))
+  xs = torch.cat([x[tok.long()], integers(g, n * T, Kd)])
+  C.gemm_moe(xs.to(gpu), ws, y, off.to(gpu), None, K.EPI["none"], T, True, S, 0, w_sh=shc)
+  sh = torch.cat([xs[routed + j * T:routed + (j + 1) * T].float() @ wc[:, j * Kd:(j + 1) * Kd].float().t() for j in range(n)])
+  got = y.view(S, slots, N).sum(0).cpu()
+  assert torch.equal(got[:routed], full) and torch.equal(got[routed:], sh)
+  topw, h = torch.rand(T * k, generator=g), torch.randn(T, N, generator=g).to(torch.bfloat16)
+  slot_of = torch.empty(T * k, dtype=torch.int32)
+  slot_of[order] = torch.arange(T * k, dtype=torch.int32)
+  want = h.double() + sum(sh.double().view(n, T, N)) + (topw.double()[:, None] * full.double()[slot_of.long()]).view(T, k, N).sum(1)
+  out = h.to(gpu)
+  C.moe_combine(y, slot_of.to(gpu), topw.to(gpu), out, S)
+  torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8, atol=1e-3)
+  h2, normed = h.to(gpu), torch.empty(T, N, dtype=torch.bfloat16, device=gpu)
+  C.moe_combine_norm(y, slot_of.to(gpu), topw.to(gpu), h2, S, torch.ones(N, dtype=torch.bfloat16, device=gpu), normed, 1e-5)
+  assert torch.equal(h2, out)

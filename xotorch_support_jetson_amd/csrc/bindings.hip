@@ -623,7 +623,7 @@ void splitk_resid_rmsnorm(const at::Tensor& ws, int64_t splits, const c10::optio
 // big_bm = 128 / 256: gemm_big tiles (pre-shuffled weights), else the weight-streaming kernel
 void gemm_moe(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const at::Tensor& off,
               const c10::optional<at::Tensor>& gather, int64_t epi, int64_t max_rows, bool wshuf, int64_t splits,
-              int64_t big_bm, double epi_arg) {
+              int64_t big_bm, double epi_arg, const c10::optional<at::Tensor>& w_sh) {
   CHECK_BF16(x);
   CHECK_BF16(w);
   CHECK_GPU(y);
@@ -641,11 +641,23 @@ void gemm_moe(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const at:
   XCHECK(splits >= 1 && y.size(0) % splits == 0, "gemm_moe: y rows must be splits * slots");
   const int64_t slots = y.size(0) / splits;
   XCHECK(max_rows >= 0 && max_rows <= slots, "gemm_moe: max_rows must be <= slots");
+  // shared experts of all max_rows tokens: [n N, K], or [N, n K] (an expert a block of columns); their slots are the last n max_rows
+  int64_t nsh = 0;
+  bool sh_cols = false;
+  if (w_sh.has_value()) {
+    CHECK_BF16((*w_sh));
+    sh_cols = w_sh->size(1) != K;
+    XCHECK(w_sh->dim() == 2 && w_sh->is_contiguous() && (sh_cols ? w_sh->size(0) == N && w_sh->size(1) % K == 0 : w_sh->size(0) % N == 0),
+           "gemm_moe: shared experts must be [n N, K] or [N, n K]");
+    nsh = w_sh->numel() / (N * K);
+    XCHECK(nsh * max_rows <= slots && wshuf && big_bm == 0, "gemm_moe: shared experts: slots, pre-shuffled weights, no tiles");
+    XCHECK(!gather.has_value() || x.size(0) == max_rows, "gemm_moe: shared experts read every row of x");
+  }
   const int* gp = nullptr;
   if (gather.has_value()) {
     CHECK_GPU((*gather));
     CHECK_DT((*gather), at::kInt);
-    XCHECK(gather->is_contiguous() && gather->numel() == slots, "gemm_moe: gather must have one entry per slot");
+    XCHECK(gather->is_contiguous() && gather->numel() == slots - nsh * max_rows, "gemm_moe: gather must have one entry per routed slot");
     gp = gather->data_ptr<int>();
   } else {
     XCHECK(x.size(0) == slots, "gemm_moe: without gather, x rows are slots");
@@ -661,11 +673,12 @@ void gemm_moe(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const at:
     // expert has.  gate/up + down, us, gemm_stream / gemm_group: 64 experts of 1408 x 2048 at 4 tokens 41 + 31 / 40 + 26, 37
     // 133 + 59 / 123 + 58, 130 213 + 117 / 130 + 66; 8 of 14336 x 4096 at 64 tokens 311 + 143 / 316 + 148, at 90 365 + 156 / 318 + 151
     rc = -1;
-    if (wshuf && (E > 16 || max_rows > 64))
+    if (wshuf && (E > 16 || max_rows > 64 || nsh > 0))
       rc = xot::launch_gemm_group(bf(x), (int)x.stride(0), (int)x.size(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,
                                   off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, (int)splits,
-                                  (long)(slots * y.size(1)), (float)epi_arg, cur_stream());
-    if (rc != 0)
+                                  (long)(slots * y.size(1)), (float)epi_arg, nsh > 0 ? bf(*w_sh) : nullptr, (int)nsh, sh_cols,
+                                  (int)(slots - nsh * max_rows), cur_stream());
+    if (rc != 0 && nsh == 0)
       rc = xot::launch_gemm_moe(bf(x), (int)x.stride(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,
                                 off.data_ptr<int>(), gp, (int)E, (int)max_rows, (int)N, (int)K, wshuf, (int)splits,
                                 (long)(slots * y.size(1)), (float)epi_arg, cur_stream());
@@ -818,10 +831,11 @@ void moe_combine(const at::Tensor& y, const at::Tensor& slot_of, const at::Tenso
   CHECK_BF16(h);
   XCHECK(all_contig_gpu(y, slot_of, topw, h), "moe_combine: tensors must be contiguous GPU");
   const int64_t T = h.size(0), D = h.size(1), k = slot_of.numel() / T;
-  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) == splits * T * k && topw.numel() == T * k,
-         "moe_combine: shapes");
+  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) % (splits * T) == 0 && y.size(0) >= splits * T * k &&
+             topw.numel() == T * k, "moe_combine: shapes");
+  const int64_t nsh = y.size(0) / (splits * T) - k;  // shared experts
   xot::launch_moe_combine(y.data_ptr<float>(), slot_of.data_ptr<int>(), topw.data_ptr<float>(), bf(h), (int)T, (int)k,
-                          (int)D, (int)splits, (long)(T * k * D), cur_stream());
+                          (int)nsh, (int)D, (int)splits, (long)(T * (k + nsh) * D), cur_stream());
 }
 
 void splitk_silu(const at::Tensor& ws, int64_t S, at::Tensor& y) {
@@ -841,12 +855,13 @@ void moe_combine_norm(const at::Tensor& y, const at::Tensor& slot_of, const at::
   CHECK_BF16(out);
   XCHECK(all_contig_gpu(y, slot_of, topw, h, ln_w, out), "moe_combine_norm: tensors must be contiguous GPU");
   const int64_t T = h.size(0), D = h.size(1), k = slot_of.numel() / T;
-  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) == splits * T * k && topw.numel() == T * k &&
-             ln_w.numel() == D && out.sizes() == h.sizes(),
+  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) % (splits * T) == 0 && y.size(0) >= splits * T * k &&
+             topw.numel() == T * k && ln_w.numel() == D && out.sizes() == h.sizes(),
          "moe_combine_norm: shapes");
+  const int64_t nsh = y.size(0) / (splits * T) - k;  // shared experts
   const int rc = xot::launch_moe_combine_norm(y.data_ptr<float>(), slot_of.data_ptr<int>(), topw.data_ptr<float>(),
-                                              bf(h), bf(ln_w), bf(out), (int)T, (int)k, (int)D, (int)splits,
-                                              (long)(T * k * D), (float)eps, cur_stream());
+                                              bf(h), bf(ln_w), bf(out), (int)T, (int)k, (int)nsh, (int)D, (int)splits,
+                                              (long)(T * (k + nsh) * D), (float)eps, cur_stream());
   XCHECK(rc == 0, "moe_combine_norm: unsupported D=", D);
 }
 
@@ -1192,7 +1207,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("splitk_resid_rmsnorm", &splitk_resid_rmsnorm);
   m.def("gemm_moe", &gemm_moe, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("off"), py::arg("gather"),
         py::arg("epi"), py::arg("max_rows"), py::arg("wshuf"), py::arg("splits") = 1, py::arg("big_bm") = 0,
-        py::arg("epi_arg") = 0.0);
+        py::arg("epi_arg") = 0.0, py::arg("w_sh") = py::none());
   m.def("moe_route", &moe_route);
   m.def("moe_route_ds", &moe_route_ds);
   m.def("mla_prep", &mla_prep);

@@ -7,6 +7,7 @@
 // tiles is taken from the offsets: an expert with three rows copies, reads and multiplies one tile, where a launch sized for
 // the step's tokens would work through four or eight.  Weights are asked for before the gathered rows (their indices are the only
 // thing a workgroup waits for first).  A tile's sum runs through K in one order whatever the number of rows.
+// Experts that every token passes (shared ones) are a few tiles more of the same launches instead of two products of their own.
 #include "common.h"
 #include "gemm_common.h"
 #include "kernels.h"
@@ -155,69 +156,73 @@ __device__ __forceinline__ void group_rows(char* smem, __amdgpu_buffer_rsrc_t wr
   }
 }
 
-// blockIdx: (column group and row block, K slice, expert).  Row block mb of mblocks takes the expert's rows in blocks of 64: mb,
-// mb + mblocks, ...; those of one column group have ids 8 apart, i.e. run together on one XCD, whose L2 then has the weights.
+// Shared experts of every token, behind the routed ones: n matrices like theirs (a column tile's blocks
+// `stride` apart), whose slots follow the routed ones, T tokens each.  A block of 64 tokens has workgroups of its own.
+struct Shared {
+  const uint16_t* W;
+  int n, T, blocks, slot0;  // blocks of 64 tokens
+  long expert, stride;      // 1 KB blocks between shared experts, and between column tiles
+};
+
+// blockIdx: (column group, K slice, shared expert and block of tokens | expert).  An expert's rows are taken 64 at a time.
 template <int EPI, bool F32>
 __global__ __launch_bounds__(64 * TW, 4) void gemm_group_kernel(const uint16_t* __restrict__ X, int ldx, int xrows,
                                                                 const uint16_t* __restrict__ W, void* __restrict__ Yv, int ldy,
                                                                 const int* __restrict__ off, const int* __restrict__ gather, int N,
-                                                                int K, int mblocks, long ysplit, float epi_arg) {
+                                                                int K, long ysplit, float epi_arg, Shared sh) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int e = blockIdx.z, ngrp = N >> 7;
-  const int first = off[e], count = off[e + 1] - first;
-  int bt = blockIdx.x, mb = 0;
-  if (mblocks > 1) {
-    if ((ngrp & 7) == 0) {
-      const int per = 8 * mblocks, q = bt / per, rem = bt % per;
-      mb = rem >> 3;
-      bt = 8 * q + (rem & 7);
-    } else {
-      mb = bt % mblocks;
-      bt /= mblocks;
-    }
-  }
-  if (mb * ROWS >= count) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nb = (K >> 5) / gridDim.y, kb = blockIdx.y * nb;
-  const uint16_t* wt = W + (((size_t)e * (N >> 4) + bt * TW + wave) * (K >> 5) + kb) * 512;
+  const int nb = (K >> 5) / gridDim.y, kb = blockIdx.y * nb, tile = blockIdx.x * TW + wave;
+  int e = (int)blockIdx.z - sh.n * sh.blocks, first, count, x0;  // slots, and without gather their rows of X
+  const uint16_t* wt;
+  if (e >= 0) {
+    first = off[e], count = off[e + 1] - first, x0 = first;
+    wt = W + (((size_t)e * (N >> 4) + tile) * (K >> 5) + kb) * 512;
+  } else {  // (first: their work does not hang on the routing, and a block is a full one)
+    const int j = blockIdx.z / sh.blocks, t0 = (blockIdx.z - j * sh.blocks) * ROWS;
+    first = sh.slot0 + j * sh.T + t0, count = min(ROWS, sh.T - t0), x0 = gather != nullptr ? t0 : first;
+    wt = sh.W + (j * sh.expert + tile * sh.stride + kb) * 512;
+  }
+  if (count <= 0) return;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wt), (short)0, nb * 1024, 0x00020000);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X + kb * 32), (short)0,
                                                                       ((xrows - 1) * ldx + K - kb * 32) * 2, 0x00020000);
   if constexpr (F32) Yv = reinterpret_cast<float*>(Yv) + blockIdx.y * ysplit;
-  for (; mb * ROWS < count; mb += mblocks) {
-    const int r0 = first + mb * ROWS, M = min(ROWS, count - mb * ROWS);
-    void* y = F32 ? (void*)(reinterpret_cast<float*>(Yv) + (size_t)r0 * ldy) : (void*)(reinterpret_cast<uint16_t*>(Yv) + (size_t)r0 * ldy);
-    const int* rows = gather != nullptr ? gather + r0 : nullptr;
-    if (M <= 16) group_rows<1, EPI, F32>(smem, wr, xr, rows, r0, ldx, nb, M, y, ldy, bt * 128, epi_arg);
-    else if (M <= 32) group_rows<2, EPI, F32>(smem, wr, xr, rows, r0, ldx, nb, M, y, ldy, bt * 128, epi_arg);
-    else if (M <= 48) group_rows<3, EPI, F32>(smem, wr, xr, rows, r0, ldx, nb, M, y, ldy, bt * 128, epi_arg);
-    else group_rows<4, EPI, F32>(smem, wr, xr, rows, r0, ldx, nb, M, y, ldy, bt * 128, epi_arg);
+  for (int r0 = 0; r0 < count; r0 += ROWS) {
+    const int M = min(ROWS, count - r0);
+    const size_t yo = (size_t)(first + r0) * ldy;
+    void* y = F32 ? (void*)(reinterpret_cast<float*>(Yv) + yo) : (void*)(reinterpret_cast<uint16_t*>(Yv) + yo);
+    const int* rows = gather != nullptr && e >= 0 ? gather + first + r0 : nullptr;
+    const int n0 = blockIdx.x * TW * 16;
+    if (M <= 16) group_rows<1, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
+    else if (M <= 32) group_rows<2, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
+    else if (M <= 48) group_rows<3, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
+    else group_rows<4, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
     __syncthreads();  // the next block's rows overwrite what this one reads
   }
-}
-
-template <int EPI, bool F32>
-int go(const uint16_t* X, int ldx, int xrows, const uint16_t* W, void* Y, int ldy, const int* off, const int* gather, int E, int max_rows,
-       int N, int K, int S, long ysplit, float epi_arg, hipStream_t st) {
-  const int mblocks = 1;
-  gemm_group_kernel<EPI, F32><<<dim3(N / 128 * mblocks, S, E), 64 * TW, 2 * HALF, st>>>(X, ldx, xrows, W, Y, ldy, off, gather, N, K, mblocks,
-                                                                                       S > 1 ? ysplit : 0L, epi_arg);
-  return 0;
 }
 
 }  // namespace
 
 int launch_gemm_group(const uint16_t* X, int ldx, int xrows, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi, const int* off,
-                      const int* gather, int E, int max_rows, int N, int K, int S, long ysplit, float epi_arg, hipStream_t st) {
+                      const int* gather, int E, int max_rows, int N, int K, int S, long ysplit, float epi_arg, const uint16_t* Wsh,
+                      int nsh, bool sh_cols, int slot0, hipStream_t st) {
   if (max_rows <= 0) return 0;
   if (N % 128 != 0 || S < 1 || K % (128 * S) != 0 || ldx % 8 != 0 || xrows < 1) return -1;
   if (((int64_t)xrows * ldx + K) * 2 >= (int64_t(1) << 31) || (int64_t)K * 32 >= (int64_t(1) << 31)) return -1;  // 32-bit byte offsets
   if (S > 1 && (epi != EPI_NONE || !out_f32)) return -1;
-  if (epi == EPI_SILU && !out_f32) return go<EPI_SILU, false>(X, ldx, xrows, W, Y, ldy, off, gather, E, max_rows, N, K, S, ysplit, epi_arg, st);
-  if (epi == EPI_CLAMP_GLU && !out_f32) return go<EPI_CLAMP_GLU, false>(X, ldx, xrows, W, Y, ldy, off, gather, E, max_rows, N, K, S, ysplit, epi_arg, st);
-  if (epi != EPI_NONE) return -1;
-  return out_f32 ? go<EPI_NONE, true>(X, ldx, xrows, W, Y, ldy, off, gather, E, max_rows, N, K, S, ysplit, epi_arg, st)
-                 : go<EPI_NONE, false>(X, ldx, xrows, W, Y, ldy, off, gather, E, max_rows, N, K, S, ysplit, epi_arg, st);
+  if (epi != EPI_NONE && (out_f32 || (epi != EPI_SILU && epi != EPI_CLAMP_GLU))) return -1;
+  const long kbl = K / 32;
+  const Shared sh{Wsh, nsh, max_rows, (max_rows + ROWS - 1) / ROWS, slot0, sh_cols ? kbl : N / 16 * kbl, sh_cols ? nsh * kbl : kbl};
+  const dim3 grid(N / 128, S, E + nsh * sh.blocks);
+  auto go = [&](auto kern) {
+    kern<<<grid, 64 * TW, 2 * HALF, st>>>(X, ldx, xrows, W, Y, ldy, off, gather, N, K, S > 1 ? ysplit : 0L, epi_arg, sh);
+  };
+  if (epi == EPI_SILU) go(gemm_group_kernel<EPI_SILU, false>);
+  else if (epi == EPI_CLAMP_GLU) go(gemm_group_kernel<EPI_CLAMP_GLU, false>);
+  else if (out_f32) go(gemm_group_kernel<EPI_NONE, true>);
+  else go(gemm_group_kernel<EPI_NONE, false>);
+  return 0;
 }
 
 }  // namespace xot

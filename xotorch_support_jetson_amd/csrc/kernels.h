@@ -119,22 +119,24 @@ void launch_splitk_resid_rmsnorm(const float* ws, int S, const uint16_t* bias, u
 int launch_gemm_moe_big(const uint16_t* X, int ldx, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi,
                         const int* off, const int* gather, int E, int max_rows, int N, int K, int S, long ysplit,
                         int bm, float epi_arg, hipStream_t s);
-// grouped decode GEMM of routed experts on pre-shuffled weights (gemm_group.hip); X has xrows rows
+// grouped decode GEMM of routed experts on pre-shuffled weights (gemm_group.hip); X has xrows rows.  Wsh: nsh shared experts of all
+// max_rows tokens, one matrix [nsh N, K], or (sh_cols) [N, nsh K]; their slots are slot0 ...
 int launch_gemm_group(const uint16_t* X, int ldx, int xrows, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi, const int* off,
-                      const int* gather, int E, int max_rows, int N, int K, int S, long ysplit, float epi_arg, hipStream_t st);
+                      const int* gather, int E, int max_rows, int N, int K, int S, long ysplit, float epi_arg, const uint16_t* Wsh,
+                      int nsh, bool sh_cols, int slot0, hipStream_t st);
 // grouped GEMM over experts: rows of expert e are off[e]..off[e+1] (slot order), W is [E][N][K]
 int launch_gemm_moe(const uint16_t* X, int ldx, const uint16_t* W, void* Y, int ldy, bool out_f32, int epi,
                     const int* off, const int* gather, int E, int max_rows, int N, int K, bool wshuf, int S,
                     long ysplit, float epi_arg, hipStream_t s);
 void launch_splitk_silu(const float* ws, int S, int M, int N, uint16_t* y, hipStream_t s);
 int launch_moe_combine_norm(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h,
-                            const uint16_t* lnw, uint16_t* out, int T, int k, int D, int S, long ysplit, float eps,
+                            const uint16_t* lnw, uint16_t* out, int T, int k, int nsh, int D, int S, long ysplit, float eps,
                             hipStream_t s);
 int launch_router_logits(const uint16_t* x, const uint16_t* w, float* out, int T, int E, int D, hipStream_t s);
 void launch_moe_route(const float* logits, int T, int E, int k, float* topw, int32_t* topi, int32_t* slot_of,
                       int32_t* sorted_tok, int32_t* off, hipStream_t s);
-void launch_moe_combine(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h, int T, int k, int D,
-                        int S, long ysplit, hipStream_t s);
+void launch_moe_combine(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h, int T, int k, int nsh,
+                        int D, int S, long ysplit, hipStream_t s);
 // DeepSeekMoE routing: method 0 greedy, 1 group max (V2 group_limited_greedy), 2 group top-2 sum (V3 noaux_tc)
 // cnt: [E] int32 counters, zero on entry and left zero on exit
 int launch_moe_route_ds(const float* logits, const float* bias, int T, int E, int k, int n_group, int topk_group,

@@ -5,7 +5,7 @@
 // (token, j) gets a slot in the expert-sorted order.  Slot order inside an expert is arbitrary: the
 // grouped GEMM treats rows independently and the combine sums each token's k slots in j order, so
 // results do not depend on it.  Everything stays on the device (graph-capturable).
-// moe_combine: h[t] += sum_j w[t, j] * y[slot_of[t, j]] with the expert outputs y in fp32.
+// moe_combine: h[t] += sum_j w[t, j] * y[slot_of[t, j]] (+ the shared experts' rows) with the expert outputs y in fp32.
 #include <algorithm>
 #include "common.h"
 #include "kernels.h"
@@ -375,7 +375,7 @@ int launch_moe_route_ds(const float* logits, const float* bias, int T, int E, in
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ y,
                                                           const int32_t* __restrict__ slot_of,
                                                           const float* __restrict__ topw, uint16_t* __restrict__ h,
-                                                          int T, int k, int D, int S, long ysplit) {
+                                                          int T, int k, int nsh, int D, int S, long ysplit) {
   const long total = (long)T * (D / 8);
   for (long q = blockIdx.x * 256L + threadIdx.x; q < total; q += (long)gridDim.x * 256) {
     const int t = (int)(q / (D / 8));
@@ -384,9 +384,9 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = bf2f(hv[e]);
-    for (int j = 0; j < k; ++j) {
-      const float w = topw[(size_t)t * k + j];
-      const float* yr = y + (size_t)slot_of[(size_t)t * k + j] * D + d;
+    for (int j = 0; j < k + nsh; ++j) {  // (shared experts' slots follow the routed ones, T each)
+      const float w = j < k ? topw[(size_t)t * k + j] : 1.f;
+      const float* yr = y + (j < k ? (size_t)slot_of[(size_t)t * k + j] : (size_t)T * j + t) * D + d;
       for (int sl = 0; sl < S; ++sl, yr += ysplit) {  // K-slice partial slabs of the grouped down GEMM
         const f32x4 a = *reinterpret_cast<const f32x4*>(yr);
         const f32x4 b = *reinterpret_cast<const f32x4*>(yr + 4);
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(const float* __re
                                                                const int32_t* __restrict__ slot_of,
                                                                const float* __restrict__ topw, uint16_t* __restrict__ h,
                                                                const uint16_t* __restrict__ lnw,
-                                                               uint16_t* __restrict__ out, int k, int D, int S,
+                                                               uint16_t* __restrict__ out, int k, int nsh, int D, int S,
                                                                long ysplit, float eps) {
   __shared__ float red[4];
   const int t = blockIdx.x, tid = threadIdx.x, nchunk = D >> 3;
@@ -427,9 +427,9 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(const float* __re
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = bf2f(hv[e]);
-    for (int j = 0; j < k; ++j) {
-      const float w = topw[(size_t)t * k + j];
-      const float* yr = y + (size_t)slot_of[(size_t)t * k + j] * D + d;
+    for (int j = 0; j < k + nsh; ++j) {
+      const float w = j < k ? topw[(size_t)t * k + j] : 1.f;
+      const float* yr = y + (j < k ? (size_t)slot_of[(size_t)t * k + j] : (size_t)gridDim.x * j + t) * D + d;
       for (int sl = 0; sl < S; ++sl, yr += ysplit) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(yr);
         const f32x4 b = *reinterpret_cast<const f32x4*>(yr + 4);
@@ -466,12 +466,12 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(const float* __re
 }
 
 int launch_moe_combine_norm(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h,
-                            const uint16_t* lnw, uint16_t* out, int T, int k, int D, int S, long ysplit, float eps,
+                            const uint16_t* lnw, uint16_t* out, int T, int k, int nsh, int D, int S, long ysplit, float eps,
                             hipStream_t s) {
   if (T <= 0) return 0;
   const int nchunk = D / 8;
   if (D % 8 != 0 || nchunk > 8 * 256) return -1;
-#define XOT_MCN(MC) moe_combine_norm_kernel<MC><<<T, 256, 0, s>>>(y, slot_of, topw, h, lnw, out, k, D, S, ysplit, eps)
+#define XOT_MCN(MC) moe_combine_norm_kernel<MC><<<T, 256, 0, s>>>(y, slot_of, topw, h, lnw, out, k, nsh, D, S, ysplit, eps)
   if (nchunk <= 256) XOT_MCN(1);
   else if (nchunk <= 512) XOT_MCN(2);
   else if (nchunk <= 1024) XOT_MCN(4);
@@ -612,13 +612,13 @@ void launch_moe_route(const float* logits, int T, int E, int k, float* topw, int
   moe_route_kernel<<<1, 1024, 0, s>>>(logits, T, E, k, topw, topi, slot_of, sorted_tok, off);
 }
 
-void launch_moe_combine(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h, int T, int k, int D,
-                        int S, long ysplit, hipStream_t s) {
+void launch_moe_combine(const float* y, const int32_t* slot_of, const float* topw, uint16_t* h, int T, int k, int nsh,
+                        int D, int S, long ysplit, hipStream_t s) {
   const long chunks = (long)T * (D / 8);
   int blocks = (int)((chunks + 255) / 256);
   if (blocks > 4096) blocks = 4096;
   if (blocks < 1) return;
-  moe_combine_kernel<<<blocks, 256, 0, s>>>(y, slot_of, topw, h, T, k, D, S, ysplit);
+  moe_combine_kernel<<<blocks, 256, 0, s>>>(y, slot_of, topw, h, T, k, nsh, D, S, ysplit);
 }
 
 }  // namespace xot

@@ -370,7 +370,8 @@ class ShardModel:
     experts (DeepSeek) added as a dense SwiGLU, tokens grouped per expert, expert GEMMs on the kernel library
     (gate/up with fused SiLU epilogue), weighted scatter-add back into h."""
     c = self.c
-    if lw.sh_gu_w is not None:  # shared experts: h += down(silu(gate) * up) of every token
+    shared = xn.is_cuda and self._shared_grouped(xn.shape[0], lw)
+    if lw.sh_gu_w is not None and not shared:  # shared experts: h += down(silu(gate) * up) of every token
       linear(linear(xn, lw.sh_gu_w, epi="silu"), lw.sh_down_w, residual=h, epi="resid", out=h)
     if xn.is_cuda and (c.num_experts in (4, 8, 16) or (c.num_experts in (32, 64, 128, 160, 256)
                                                        and c.hidden_size % 512 == 0)) and layout_of(lw.router) == "rowmajor":
@@ -380,7 +381,7 @@ class ShardModel:
     else:
       logits = linear(xn, lw.router, out_dtype=torch.float32)  # [T, E]
     if xn.is_cuda:
-      return self._moe_gpu(xn, lw, h, logits, next_norm)
+      return self._moe_gpu(xn, lw, h, logits, next_norm, shared)
     if self._ds_route:
       topw, topi = K.moe_route_ds(logits, lw.router_bias, *self._route_args())
     else:
@@ -407,8 +408,20 @@ class ShardModel:
     h += out.to(h.dtype)
     return None
 
+  def _shared_grouped(self, T: int, lw) -> bool:
+    """Shared experts in the routed ones' launches, as experts that every token passes: where those stream their weights
+    (csrc/gemm_group.hip) and the widths are whole experts.  37 tokens, two shared experts of 1408 x 2048: gate/up + down of their own
+    8.7 + 4.6 (slab reduce) + 5.6 + 4.9 us in launches of their own; a decode step of 9 such layers 2574 us, 2464 here."""
+    c = self.c
+    if lw.sh_gu_w is None or c.num_experts <= 16 or moe_tiles(T, c.num_experts_per_tok, c.num_experts)[0]:
+      return False
+    F, D = c.expert_dim, c.hidden_size
+    sh = (lw.sh_gu_w, lw.sh_down_w)
+    return (all(layout_of(w) == "stream" and w.dtype == torch.bfloat16 and w.is_contiguous() for w in (*sh, lw.gu_w, lw.down_w)) and
+            F % 128 == 0 and D % 128 == 0 and sh[0].shape[0] % (2 * F) == 0 and tuple(sh[1].shape) == (D, sh[0].shape[0] // 2))
+
   def _moe_gpu(self, xn: torch.Tensor, lw, h: torch.Tensor, logits: torch.Tensor,
-               next_norm: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+               next_norm: Optional[torch.Tensor] = None, shared: bool = False) -> Optional[torch.Tensor]:
     """Device-only MoE (graph-capturable): routing kernel (softmax top-k, per-expert slot order),
     grouped gate/up GEMM gathering token rows with the SiLU*mul epilogue, grouped down GEMM into fp32
     slots, combine kernel adding sum_j w_j * y_slot(j) into the residual stream."""
@@ -436,24 +449,26 @@ class ShardModel:
       bm = bm_dn = MOE_BM
     if MOE_DN_SPLITS and bm:
       S_dn = MOE_DN_SPLITS
-    act = torch.empty(T * k, F, dtype=torch.bfloat16, device=dev)
+    w_sh, n_sh = ((lw.sh_gu_w, lw.sh_down_w), lw.sh_down_w.shape[1] // F) if shared else ((None, None), 0)
+    slots = T * (k + n_sh)
+    act = torch.empty(slots, F, dtype=torch.bfloat16, device=dev)
     Sg = MOE_GU_SPLITS if (bm == 0 and T * k <= 32 and D % (256 * MOE_GU_SPLITS) == 0) else 1
     if Sg > 1:
       # decode-sized groups: the weight-streaming gate/up split over K into fp32 slabs (k experts x N/128
       # column blocks alone leave the last wave of workgroups short, e.g. 448 on 512 slots at batch 1),
       # SiLU*mul applied by the slab reduce
-      ys = torch.empty(Sg * T * k, 2 * F, dtype=torch.float32, device=dev)
-      C.gemm_moe(xn, lw.gu_w, ys, off, sorted_tok, K.EPI["none"], T, layout_of(lw.gu_w) == "stream", Sg, 0)
+      ys = torch.empty(Sg * slots, 2 * F, dtype=torch.float32, device=dev)
+      C.gemm_moe(xn, lw.gu_w, ys, off, sorted_tok, K.EPI["none"], T, layout_of(lw.gu_w) == "stream", Sg, 0, w_sh=w_sh[0])
       C.splitk_silu(ys, Sg, act)
     else:
-      C.gemm_moe(xn, lw.gu_w, act, off, sorted_tok, K.EPI["silu"], T, layout_of(lw.gu_w) == "stream", 1, bm)
+      C.gemm_moe(xn, lw.gu_w, act, off, sorted_tok, K.EPI["silu"], T, layout_of(lw.gu_w) == "stream", 1, bm, w_sh=w_sh[0])
     # down projection split over K (fp32 partial slabs summed by the combine): the grouped GEMM only has
     # (experts hit) x N/tile workgroups with work, too few to stream the expert weights at full HBM rate
     S = (4 if T * k <= 64 else 2) if bm == 0 else S_dn
     if F % (256 * S):
       S = 1
-    y = torch.empty(S * T * k, D, dtype=torch.float32, device=dev)
-    C.gemm_moe(act, lw.down_w, y, off, None, K.EPI["none"], T, layout_of(lw.down_w) == "stream", S, bm_dn)
+    y = torch.empty(S * slots, D, dtype=torch.float32, device=dev)
+    C.gemm_moe(act, lw.down_w, y, off, None, K.EPI["none"], T, layout_of(lw.down_w) == "stream", S, bm_dn, w_sh=w_sh[1])
     if next_norm is not None:  # combine + the following RMSNorm in one kernel
       out = torch.empty_like(h)
       C.moe_combine_norm(y, slot_of, topw, h, S, next_norm, out, float(c.rms_norm_eps))
