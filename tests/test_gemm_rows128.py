@@ -1,0 +1,48 @@
+"""The 128-row tiles of the large-M GEMM (csrc/gemm_big.hip codes 1280128 and 1280256): partial row and column tiles, fewer stages
+than the pipeline holds, K splits, every epilogue; and where the policy offers them."""
+import pytest
+import torch
+
+from xotorch_support_jetson_amd.ops import kernels as K
+from xotorch_support_jetson_amd.ops import linear as L
+from xotorch_support_jetson_amd.ops.weights_layout import shuffle_for_stream
+
+
+def test_candidates():
+  """128-row tiles where they hold all rows, 128 x 128 up to 256 rows; no preference for half-empty 256-row tiles."""
+  codes = lambda M: {c[1] for c in L.GemmPolicy._big_cands(M, 8192, 4096)}  # noqa: E731
+  assert {1280128, 1280256} <= codes(65) and {1280128, 1280256} <= codes(128)
+  assert 1280128 in codes(129) and 1280128 in codes(256) and 1280256 not in codes(129)
+  assert 1280128 not in codes(257) and 1280128 not in codes(512)
+  times = {("big", 1280256, 1): 1.0, ("big", 2256, 1): 1.04}
+  assert L._tie_break(times, 128) == ("big", 1280256, 1) and L._tie_break(times, 200) == ("big", 2256, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("code", [1280128, 1280256])
+@pytest.mark.parametrize("M", [1, 65, 128, 129, 256])
+@pytest.mark.parametrize("N,Kd,S", [(256, 128, 1), (400, 128, 1), (512, 1408, 1), (272, 1024, 3), (512, 512, 4)])
+def test_exact(gpu, code, M, N, Kd, S):
+  """Integer operands: sums bit for bit, fp32 and bf16, with bias and residual; gated pairs within one rounding (2^-8)."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  C = require()
+  g = torch.Generator().manual_seed(M + N + Kd)
+  rn = lambda *s: torch.randint(-3, 4, s, generator=g).to(torch.bfloat16)  # noqa: E731
+  x, w, b, r = rn(M, Kd), rn(N, Kd), rn(N), rn(M, N)
+  full = x.float() @ w.float().t()
+  xd, ws, ws_buf = x.to(gpu), shuffle_for_stream(w.to(gpu)), torch.empty(S * M * N, device=gpu)
+  y = torch.empty(M, N, device=gpu)
+  C.gemm_big(xd, ws, y, None, None, ws_buf, K.EPI["none"], code, S, True)
+  assert torch.equal(y.cpu(), full)
+  y = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+  C.gemm_big(xd, ws, y, b.to(gpu), r.to(gpu), ws_buf, K.EPI["resid"], code, S, True)
+  assert torch.equal(y.cpu(), (full + b.float() + r.float()).to(torch.bfloat16))
+  if N % 32 == 0:
+    gate, up = (full.double().view(M, N // 32, 2, 16)[:, :, i].reshape(M, -1) for i in (0, 1))
+    for epi, want in (("silu", gate * torch.sigmoid(gate) * up),
+                      ("clamp_glu", gate.clamp(max=7) * torch.sigmoid(1.702 * gate.clamp(max=7)) * (up.clamp(-7, 7) + 1))):
+      if epi == "clamp_glu" and code == 1280256:
+        continue  # (built with 128 columns)
+      a = torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu)
+      C.gemm_big(xd, ws, a, None, None, ws_buf, K.EPI[epi], code, S, True, 7.0)
+      torch.testing.assert_close(a.cpu().double(), want, rtol=2 ** -7, atol=1e-6)

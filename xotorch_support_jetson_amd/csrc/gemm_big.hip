@@ -563,7 +563,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
                         bool reduce, hipStream_t st, float epi_arg = 0.f) {
   // bn = tile code: BN (256 / 128 / 224), 1256 / 2256 (256 x 256 on the four- / two-phase ping-pong), plus
   // 10000 x BM for row tiles below 256 (160 / 192 / 224: M = 320 / 384 / 448 in two tiles without padding rows;
-  // 2256 only with 192)
+  // 2256 only with 192; 128 with a deeper pipeline: four 64-deep stages of 128 x 128, three of 128 x 256)
   const int bm = bn / 10000 ? bn / 10000 : 256, code = bn % 10000;
   if (code == 4256) {  // four-wave tile, 256 columns, rows by its own rule or as given (gemm_w4.hip)
     const int rc = launch_gemm_w4(X, ldx, W, bias, R, ldr, Y, ldy, F32, EPI, ws, M, N, K, S, bn / 10000 ? bm : 0, big_group_m(),
@@ -580,8 +580,9 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
   big_launch<BM_, BN_, WM_, 8 / WM_, 64, NBUF_, EPI, F32, ##__VA_ARGS__>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, \
                                                                          S, reduce, st, epi_arg)
   if constexpr (EPI == EPI_CLAMP_GLU || EPI == EPI_RELU2 || EPI == EPI_GELU_GLU) {  // (built for the tiles that win: two-phase 256, 128 columns)
-    if (bm != 256) return -1;
-    if (code == 2256) XOT_BIG(256, 256, 2, 2, 2);
+    if (bm == 128 && code == 128) XOT_BIG(128, 128, 2, 4);
+    else if (bm != 256) return -1;
+    else if (code == 2256) XOT_BIG(256, 256, 2, 2, 2);
     else if (code == 128) XOT_BIG(256, 128, 4, 3);
     else return -1;
     return 0;
@@ -596,6 +597,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
     if (bm == 224) XOT_BIG(224, 256, 2, 2);
     else if (bm == 192) XOT_BIG(192, 256, 2, 2);
     else if (bm == 160) XOT_BIG(160, 256, 2, 2);
+    else if (bm == 128) XOT_BIG(128, 256, 2, 3);
     else return -1;
   } else if (code == 2256) {
     if (bm == 192) XOT_BIG(192, 256, 2, 2, 2);  // two-phase ping-pong on 192-row tiles (three row tiles per A half)
@@ -604,6 +606,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
     if (bm == 224) XOT_BIG(224, 128, 2, 3);
     else if (bm == 192) XOT_BIG(192, 128, 2, 3);
     else if (bm == 160) XOT_BIG(160, 128, 2, 3);
+    else if (bm == 128) XOT_BIG(128, 128, 2, 4);
     else return -1;
   } else {
     return -1;

@@ -386,9 +386,14 @@ class GemmPolicy:
       codes.append(4256)
     if N % 224 == 0:  # 7 row groups per wave: whole rounds where 256-wide tiles leave a half round (8B gate/up)
       codes.append(224)
-    bm = big_row_tile(M)
+    bm = 128 if M <= 128 else big_row_tile(M)
     if bm < 256:  # rows that would leave >= 32 padding rows in 256-row tiles: shorter row tiles (two-phase: 192 only)
       codes += [bm * 10000 + 256, bm * 10000 + 128] + ([bm * 10000 + 2256] if PP2 and bm == 192 else [])
+    # 128 x 128 tiles keep four 64-deep stages in LDS, so more weight bytes are in flight, and fill the CUs where 256 rows leave
+    # half of them idle: 28672 x 4096 at 128 rows 62 -> 47 us, 16384 x 2048 at 256 35 -> 26.  Beyond 256 rows the products of a
+    # step run at the power limit, where their extra LDS reads cost what they gain alone (a Llama-3-8B step of 400 rows 2700 us, 2810)
+    if 128 < M <= 256:
+      codes.append(1280128)
     for bn in codes:
       if N % tile_width(bn) and N < tile_width(bn):  # a partial last column tile is masked; skip tiles wider than N
         continue
@@ -466,7 +471,7 @@ class GemmPolicy:
       cands += self._wave_cands(M, N, Kd, epi, wave == "rope") or self._wide_cands(M, N, Kd, epi, wave == "rope")
     if M >= BIG_MIN_M and Kd % 128 == 0:
       big = self._big_cands(M, N, Kd)
-      cands += [c for c in big if c[1] in (2256, 128, 4256)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
+      cands += [c for c in big if c[1] in (2256, 128, 4256, 1280128)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
     if not cands:
       raise RuntimeError(f"no GEMM configuration for pre-shuffled N={N} K={Kd} M={M}")
     if self._no_tuning():
@@ -532,7 +537,7 @@ _BIG_PREF_TALL = {4256: 0, 2256: 1, 1256: 2, 256: 3, 224: 4, 128: 5}
 def _tie_break(times: Dict, M: int = 0) -> Tuple:
   best = min(times, key=times.get)
   code = lambda c: c[1] % 10000  # noqa: E731 - the schedule, whatever the row tile
-  if best[0] != "big" or code(best) not in _BIG_PREF or TIE <= 0:
+  if best[0] != "big" or code(best) not in _BIG_PREF or TIE <= 0 or 0 < M <= 128:  # (256-row tiles at 128 rows: half of them padding)
     return best
   pref = _BIG_PREF_TALL if M >= W4_PREF_M else _BIG_PREF
   top = min(pref, key=pref.get)
