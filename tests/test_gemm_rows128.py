@@ -1,4 +1,4 @@
-"""The 128-row tiles of the large-M GEMM (csrc/gemm_big.hip codes 1280128 and 1280256): partial row and column tiles, fewer stages
+"""The 128- and 64-row tiles of the large-M GEMM (csrc/gemm_big.hip codes 1280128, 1280256, 640128 and 640256): partial row and column tiles, fewer stages
 than the pipeline holds, K splits, every epilogue; and where the policy offers them."""
 import pytest
 import torch
@@ -14,13 +14,16 @@ def test_candidates():
   assert {1280128, 1280256} <= codes(65) and {1280128, 1280256} <= codes(128)
   assert 1280128 in codes(129) and 1280128 in codes(256) and 1280256 not in codes(129)
   assert 1280128 not in codes(257) and 1280128 not in codes(512)
+  rows64 = L.GemmPolicy._rows64_cands
+  assert {("big", 640128, 1), ("big", 640256, 8)} <= set(rows64(17, 8192, 4096)) and rows64(64, 128, 128) == [("big", 640128, 1)]
+  assert rows64(16, 8192, 4096) == [] and rows64(65, 8192, 4096) == [] and rows64(64, 8200, 4096) == []
   times = {("big", 1280256, 1): 1.0, ("big", 2256, 1): 1.04}
   assert L._tie_break(times, 128) == ("big", 1280256, 1) and L._tie_break(times, 200) == ("big", 2256, 1)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("code", [1280128, 1280256])
-@pytest.mark.parametrize("M", [1, 65, 128, 129, 256])
+@pytest.mark.parametrize("code,M", [(c, m) for c, ms in ((1280128, (1, 65, 128, 129, 256)), (1280256, (1, 65, 128, 129)),
+                                                         (640128, (1, 17, 63, 64, 65)), (640256, (1, 17, 63, 64, 65))) for m in ms])
 @pytest.mark.parametrize("N,Kd,S", [(256, 128, 1), (400, 128, 1), (512, 1408, 1), (272, 1024, 3), (512, 512, 4)])
 def test_exact(gpu, code, M, N, Kd, S):
   """Integer operands: sums bit for bit, fp32 and bf16, with bias and residual; gated pairs within one rounding (2^-8)."""
@@ -41,8 +44,8 @@ def test_exact(gpu, code, M, N, Kd, S):
     gate, up = (full.double().view(M, N // 32, 2, 16)[:, :, i].reshape(M, -1) for i in (0, 1))
     for epi, want in (("silu", gate * torch.sigmoid(gate) * up),
                       ("clamp_glu", gate.clamp(max=7) * torch.sigmoid(1.702 * gate.clamp(max=7)) * (up.clamp(-7, 7) + 1))):
-      if epi == "clamp_glu" and code == 1280256:
-        continue  # (built with 128 columns)
+      if epi == "clamp_glu" and code != 1280128:
+        continue  # (the one it is built with)
       a = torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu)
       C.gemm_big(xd, ws, a, None, None, ws_buf, K.EPI[epi], code, S, True, 7.0)
       torch.testing.assert_close(a.cpu().double(), want, rtol=2 ** -7, atol=1e-6)

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
                                                           long ysplit = 0, int group_m = 4, float epi_arg = 0.f) {
   static_assert(WM * WN == 8, "8 waves");
   static_assert(BK == 32 || BK == 64, "k stage of 32 or 64");
-  static_assert(BM % (16 * WM) == 0 && BM >= 128 && BM <= 512, "row tile of 128 .. 512 rows");
+  static_assert(BM % (16 * WM) == 0 && BM >= 64 && BM <= 512, "row tile of 64 .. 512 rows");
   static_assert(PP == 0 || PP == 1 || PP == 2, "schedules: base (0), ping-pong in 4 phases (1) or 2 phases (2)");
   static_assert(MOE == 0 || MOE == 4 || (!SPLIT && EPI != EPI_RESID), "grouped GEMM: no slab reduce, no residual");
   static_assert(MOE != 4 || !SPLIT, "K-grouped GEMM: no K split");
@@ -563,7 +563,8 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
                         bool reduce, hipStream_t st, float epi_arg = 0.f) {
   // bn = tile code: BN (256 / 128 / 224), 1256 / 2256 (256 x 256 on the four- / two-phase ping-pong), plus
   // 10000 x BM for row tiles below 256 (160 / 192 / 224: M = 320 / 384 / 448 in two tiles without padding rows;
-  // 2256 only with 192; 128 with a deeper pipeline: four 64-deep stages of 128 x 128, three of 128 x 256)
+  // 2256 only with 192; 128 with a deeper pipeline: four 64-deep stages of 128 x 128, three of
+  // 128 x 256; 64 for 17 .. 64 rows, six of 64 x 128, four of 64 x 256)
   const int bm = bn / 10000 ? bn / 10000 : 256, code = bn % 10000;
   if (code == 4256) {  // four-wave tile, 256 columns, rows by its own rule or as given (gemm_w4.hip)
     const int rc = launch_gemm_w4(X, ldx, W, bias, R, ldr, Y, ldy, F32, EPI, ws, M, N, K, S, bn / 10000 ? bm : 0, big_group_m(),
@@ -598,6 +599,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
     else if (bm == 192) XOT_BIG(192, 256, 2, 2);
     else if (bm == 160) XOT_BIG(160, 256, 2, 2);
     else if (bm == 128) XOT_BIG(128, 256, 2, 3);
+    else if (bm == 64) XOT_BIG(64, 256, 2, 4);
     else return -1;
   } else if (code == 2256) {
     if (bm == 192) XOT_BIG(192, 256, 2, 2, 2);  // two-phase ping-pong on 192-row tiles (three row tiles per A half)
@@ -607,6 +609,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
     else if (bm == 192) XOT_BIG(192, 128, 2, 3);
     else if (bm == 160) XOT_BIG(160, 128, 2, 3);
     else if (bm == 128) XOT_BIG(128, 128, 2, 4);
+    else if (bm == 64) XOT_BIG(64, 128, 2, 6);
     else return -1;
   } else {
     return -1;

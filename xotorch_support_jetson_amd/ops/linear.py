@@ -405,6 +405,17 @@ class GemmPolicy:
     return cands
 
   @staticmethod
+  def _rows64_cands(M, N, Kd):
+    """64-row tiles of gemm_big: 17 to 64 rows of X arrive once a workgroup by LDS-DMA (128 or 256 columns, six or four 64-deep
+    stages in LDS), where the stream GEMM passes them through registers.  us, the best other / here: 24 x 28672 x 4096 44.3 / 41.5,
+    64 x 57344 x 8192 155 / 146, 64 x 128256 x 8192 367 / 353, 64 x 102400 x 2048 93 / 84; the K slices of 2048 x 2048 stay with
+    the stream GEMM (10.7 / 12.3).  At 16 rows and fewer X is no load to speak of."""
+    if not WAVE_MAX_M < M <= 64 or N % 16:
+      return []
+    return [("big", 640000 + bn, S) for bn in (128, 256) for S in (1, 2, 3, 4, 6, 8)
+            if N >= bn and (S == 1 or (-(-N // bn) < 256 and -(-N // bn) * S <= 1024 and Kd // 64 >= 2 * S))]
+
+  @staticmethod
   def _wave_cands(M, N, Kd, epi, rope):
     """Whole-K decode GEMM: 16, 32 or 64 columns a workgroup (gated pairs from 32; rotation pairs of column tiles: 32)."""
     if M > WAVE_MAX_M or Kd % 128:
@@ -469,6 +480,8 @@ class GemmPolicy:
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
     if wave and epi != "gelu_glu":
       cands += self._wave_cands(M, N, Kd, epi, wave == "rope") or self._wide_cands(M, N, Kd, epi, wave == "rope")
+    if epi not in ("clamp_glu", "relu2", "gelu_glu") and Kd % 128 == 0:
+      cands += self._rows64_cands(M, N, Kd)
     if M >= BIG_MIN_M and Kd % 128 == 0:
       big = self._big_cands(M, N, Kd)
       cands += [c for c in big if c[1] in (2256, 128, 4256, 1280128)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
