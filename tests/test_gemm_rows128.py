@@ -1,4 +1,4 @@
-"""The 128- and 64-row tiles of the large-M GEMM (csrc/gemm_big.hip codes 1280128, 1280256, 640128 and 640256): partial row and column tiles, fewer stages
+"""The 128- and 64-row tiles (and the 160 x 256 one) of the large-M GEMM (csrc/gemm_big.hip codes 1280128, 1280256, 640128, 640256): partial row and column tiles, fewer stages
 than the pipeline holds, K splits, every epilogue; and where the policy offers them."""
 import pytest
 import torch
@@ -23,7 +23,7 @@ def test_candidates():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("code,M", [(c, m) for c, ms in ((1280128, (1, 65, 128, 129, 256)), (1280256, (1, 65, 128, 129)),
-                                                         (640128, (1, 17, 63, 64, 65)), (640256, (1, 17, 63, 64, 65))) for m in ms])
+                                                         (640128, (1, 17, 63, 64, 65)), (640256, (1, 17, 63, 64, 65)), (1600256, (1, 160, 161, 320))) for m in ms])
 @pytest.mark.parametrize("N,Kd,S", [(256, 128, 1), (400, 128, 1), (512, 1408, 1), (272, 1024, 3), (512, 512, 4)])
 def test_exact(gpu, code, M, N, Kd, S):
   """Integer operands: sums bit for bit, fp32 and bf16, with bias and residual; gated pairs within one rounding (2^-8)."""

@@ -597,7 +597,7 @@ static int big_dispatch(const uint16_t* X, int ldx, const uint16_t* W, const uin
   } else if (code == 256) {
     if (bm == 224) XOT_BIG(224, 256, 2, 2);
     else if (bm == 192) XOT_BIG(192, 256, 2, 2);
-    else if (bm == 160) XOT_BIG(160, 256, 2, 2);
+    else if (bm == 160) XOT_BIG(160, 256, 2, 3);  // (a third stage: a Llama-3-8B step of 300 rows 2216 -> 2132 us; 192 rows have no room for one)
     else if (bm == 128) XOT_BIG(128, 256, 2, 3);
     else if (bm == 64) XOT_BIG(64, 256, 2, 4);
     else return -1;
