@@ -49,3 +49,21 @@ def test_exact(gpu, code, M, N, Kd, S):
       a = torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu)
       C.gemm_big(xd, ws, a, None, None, ws_buf, K.EPI[epi], code, S, True, 7.0)
       torch.testing.assert_close(a.cpu().double(), want, rtol=2 ** -7, atol=1e-6)
+
+
+def test_routed_models_keep_their_sums(monkeypatch):
+  """Attention weights of models with routed experts: the candidates of 17 to 256 rows are those without the tiles above, under keys
+  of their own."""
+  seen = {}
+  monkeypatch.setattr(L.policy, "_lookup", lambda key: None)
+  monkeypatch.setattr(L.policy, "_no_tuning", lambda: True)
+  monkeypatch.setattr(L.policy, "_heuristic", lambda M, N, cands: seen.setdefault("cands", cands) and cands[0])
+  for M in (17, 64, 100, 200):
+    for kept in (False, True):
+      w = torch.empty(6144, 4096, dtype=torch.bfloat16, device="meta")
+      if kept:
+        L.keep_order(w)
+      seen.clear()
+      L.policy.shuffled_cfg(torch.empty(M, 4096, dtype=torch.bfloat16, device="meta"), w, None, None, "none", torch.bfloat16, "rope")
+      new = [c for c in seen["cands"] if c[0] == "wave" or (c[0] == "big" and L.tile_rows(c[1]) in (64, 128))]
+      assert bool(new) != kept

@@ -28,7 +28,7 @@ import torch
 from ..inference.shard import Shard
 from ..ops import kernels as K
 from ..ops._ext import require
-from ..ops.linear import (FUSE_MERGE, FUSE_NORM, PendingNorm, layout_of, linear, linear_resid_norm, linear_rope_kv,
+from ..ops.linear import (FUSE_MERGE, FUSE_NORM, PendingNorm, keep_order, layout_of, linear, linear_resid_norm, linear_rope_kv,
                           linear_slabs, scratch, stream_rows)
 from ..ops.rope import longrope_window, rope_shift, rope_table
 from .config import ModelConfig
@@ -257,6 +257,10 @@ class ShardModel:
         self.ws = K.DecodeWorkspace(max_batch, c.num_heads, c.head_dim, max_ctx, self.device, routed=c.num_experts > 0)
     if c.is_mla:
       self.scale = c.attn_scale()
+    if c.num_experts > 0:
+      for lw in weights.layers.values():
+        for w in (lw.qkv_w, lw.o_w, getattr(lw, "qb_w", None)):
+          keep_order(w)
     # last shard with the LM head split across two ring stages: logits of vocab rows [0, head_rows) only,
     # and forward returns (logits, normed hidden)
     self.head_rows: Optional[int] = None

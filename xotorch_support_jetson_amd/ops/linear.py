@@ -25,7 +25,7 @@ import json
 import os
 import sys
 import threading
-from typing import Dict, Tuple
+from typing import Dict, Optional, Tuple
 
 import torch
 
@@ -93,6 +93,14 @@ def tile_rows(code: int) -> int:
 
 def layout_of(w: torch.Tensor) -> str:
   return getattr(w, "xot_layout", "rowmajor")
+
+
+def keep_order(w: Optional[torch.Tensor]) -> None:
+  """Products of w at 17 to 256 rows choose among the kernels they always had, so their K splits, and with them the order of their
+  sums, stay: the attention of models with routed experts.  A token whose experts are almost tied turns on the last bits, and its
+  whole row with it (64 sequences of Mixtral: rel 0.021, single logits 0.7 of their size, either way round)."""
+  if isinstance(w, torch.Tensor):
+    w.xot_keep_order = True
 
 
 def to_stream_layout(w: torch.Tensor) -> torch.Tensor:
@@ -376,7 +384,7 @@ class GemmPolicy:
 
   # ---------------------------------------------------------------- shuffled weights
   @staticmethod
-  def _big_cands(M, N, Kd):
+  def _big_cands(M, N, Kd, rows128=True):
     cands = []
     if N % 16:
       return cands
@@ -386,13 +394,13 @@ class GemmPolicy:
       codes.append(4256)
     if N % 224 == 0:  # 7 row groups per wave: whole rounds where 256-wide tiles leave a half round (8B gate/up)
       codes.append(224)
-    bm = 128 if M <= 128 else big_row_tile(M)
+    bm = 128 if M <= 128 and rows128 else big_row_tile(M)
     if bm < 256:  # rows that would leave >= 32 padding rows in 256-row tiles: shorter row tiles (two-phase: 192 only)
       codes += [bm * 10000 + 256, bm * 10000 + 128] + ([bm * 10000 + 2256] if PP2 and bm == 192 else [])
     # 128 x 128 tiles keep four 64-deep stages in LDS, so more weight bytes are in flight, and fill the CUs where 256 rows leave
     # half of them idle: 28672 x 4096 at 128 rows 62 -> 47 us, 16384 x 2048 at 256 35 -> 26.  Beyond 256 rows the products of a
     # step run at the power limit, where their extra LDS reads cost what they gain alone (a Llama-3-8B step of 400 rows 2700 us, 2810)
-    if 128 < M <= 256:
+    if 128 < M <= 256 and rows128:
       codes.append(1280128)
     for bn in codes:
       if N % tile_width(bn) and N < tile_width(bn):  # a partial last column tile is masked; skip tiles wider than N
@@ -450,6 +458,9 @@ class GemmPolicy:
     # (a residual product's plain entry belongs to linear_resid_norm, which sums the slabs itself; a caller that does not
     # take the whole-K GEMM passes over such an entry)
     kind = "sl" if slabs else "sh" + wave if wave == "rope" or epi == "resid" else "sh"
+    kept = getattr(w, "xot_keep_order", False)
+    if kept and WAVE_MAX_M < M <= 256:
+      kind += "o"
     key = (kind, _m_bucket(M), N, Kd, epi, bias is not None, str(out_dtype))
     got = self._lookup(key)
     if got is not None and got[0] == "wave" and not wave:
@@ -478,12 +489,12 @@ class GemmPolicy:
     cands = []
     if M <= STREAM_MAX_M and epi != "gelu_glu":
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
-    if wave and epi != "gelu_glu":
+    if wave and epi != "gelu_glu" and not (kept and M > WAVE_MAX_M):
       cands += self._wave_cands(M, N, Kd, epi, wave == "rope") or self._wide_cands(M, N, Kd, epi, wave == "rope")
-    if epi not in ("clamp_glu", "relu2", "gelu_glu") and Kd % 128 == 0:
+    if epi not in ("clamp_glu", "relu2", "gelu_glu") and Kd % 128 == 0 and not kept:
       cands += self._rows64_cands(M, N, Kd)
     if M >= BIG_MIN_M and Kd % 128 == 0:
-      big = self._big_cands(M, N, Kd)
+      big = self._big_cands(M, N, Kd, not kept)
       cands += [c for c in big if c[1] in (2256, 128, 4256, 1280128)] if epi in ("clamp_glu", "relu2", "gelu_glu") else big  # (the tiles built with them)
     if not cands:
       raise RuntimeError(f"no GEMM configuration for pre-shuffled N={N} K={Kd} M={M}")
@@ -498,7 +509,7 @@ class GemmPolicy:
         times[cfg] = self._time(lambda: call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
       except RuntimeError:
         pass
-    got = _tie_break(times, M) if times else cands[0]
+    got = _tie_break(times, 0 if kept and M <= 128 else M) if times else cands[0]
     if TUNE_LOG:
       print(f"[gemm tune] {key} -> {got}: " + ", ".join(f"{c}={t * 1e3:.1f}us" for c, t in sorted(times.items(), key=lambda i: i[1])),
             file=sys.stderr, flush=True)
