@@ -46,3 +46,27 @@ def test_against_the_plain_form(gpu, mode, H, G, d, dv, B, dtype):
   rtol = 2 ** -8 if dtype == torch.bfloat16 else 1e-4
   torch.testing.assert_close(got[:, :H * dv].cpu().float()[live], out[live], rtol=rtol, atol=1e-4)
   assert not got[:, H * dv:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,d", [("delta", 128), ("gla", 64), ("gla", 32)])
+@pytest.mark.parametrize("F,tiles", [(48, True), (4, False), (200, False), (50, False), (1040, True)])
+@pytest.mark.parametrize("B", [1, 37])
+def test_activation_along_with_it(gpu, mode, d, F, tiles, B):
+  """gelu(gate) * up in the same launch (columns apart, or alternating in tiles of 16; widths that are no multiple of four and
+  uncovered key dims take a launch of its own): exactly gelu_mul's rows, and the recurrence's as without it."""
+  H, dv = 2, 32
+  a = inputs(mode, B, H, H, d, dv, B + F)
+  dev = {n: t.to(gpu) if torch.is_tensor(t) else t for n, t in a.items()}
+  if a["gla"]:
+    dev["gla"] = tuple(t.to(gpu) if torch.is_tensor(t) else t for t in a["gla"])
+  P = torch.randn(B, 8 + 2 * F + 32, device=gpu)
+  args = (P, 8, -1, F) if tiles else (P, 8, 8 + F, F)
+  want = torch.zeros(B, F + 8, dtype=torch.bfloat16, device=gpu)
+  K.gelu_mul(*args, want)
+  act, state = torch.zeros_like(want), dev["state"].clone()
+  live = dev["state_slots"] >= 0  # (rows without a slot are not written)
+  out, plain = (torch.zeros(B, H * dv, device=gpu) for _ in range(2))
+  K.recurrence_norm(**dev, out=plain)
+  K.recurrence_norm(**dict(dev, state=state), out=out, gelu=(*args, act))
+  assert torch.equal(act, want) and torch.equal(out[live], plain[live]) and torch.equal(state, dev["state"])

@@ -161,10 +161,7 @@ __global__ __launch_bounds__(256) void gelu_mul_k(const float* __restrict__ P, i
     u[0] = up[0];
   }
 #pragma unroll
-  for (int k = 0; k < W; ++k) {
-    const float g = 0.5f * z[k] * (1.0f + tanhf(0.7978845608028654f * (z[k] + 0.044715f * z[k] * z[k] * z[k])));
-    y[k] = g * u[k];
-  }
+  for (int k = 0; k < W; ++k) y[k] = gelu_tanhf_(z[k]) * u[k];
   if constexpr (W == 4) st4(out + t * ldo + i, f32x4{y[0], y[1], y[2], y[3]});
   else stf(out + t * ldo + i, y[0]);
 }

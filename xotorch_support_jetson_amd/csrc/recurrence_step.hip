@@ -5,7 +5,8 @@
 // it is the state, read and written once (48 sequences x 16 heads x 128 x 128 fp32: 101 MB): every load of it is asked for at once,
 // in whole 256-byte runs, next to k, q and the decays, which come straight from memory (one token: nothing to stage).  The general
 // kernel (mixers.hip linear_recurrence_k) has 8 KB of state a workgroup behind a pass through LDS, and the norm and the decays of
-// gated linear attention were launches of their own; here a head's outputs meet in LDS.  us, before / here: delta rule as above
+// gated linear attention were launches of their own; here a head's outputs meet in LDS, and a parallel block's gated activation, 4.9 us
+// on its own, fills in behind the heads.  us, before / here: delta rule as above
 // 26.2 + 4.7 (norm) / 17.5 (5.8 TB/s), gated linear attention 64 x 128 4.7 (decays) + 15.4 + 4.7 / 11.3; 6 sequences, channel decays
 // 5.7 + 3.9 / 6.1.
 // MODE 0: gated linear attention, S = diag(a) S + k v^T with a = exp(logsigmoid(a2 . P[a1 ...] + b) / tau) made here.  MODE 1:
@@ -49,14 +50,42 @@ struct StepArgs {
   int ldo;
 };
 
+// A parallel block's gated activation gelu(gate) * up, which only needs the projections as well (workgroups behind the heads')
+struct GeluArgs {
+  const float* P;
+  int ld, gate, up, F;  // up < 0: gate and up columns alternate in tiles of 16
+  void* out;
+  int ldo;
+  bool bf;
+  int total;  // groups of four columns
+};
+
+__device__ __forceinline__ void gelu_part(const GeluArgs& a, int idx) {
+  if (idx >= a.total) return;
+  const int nw = a.F / 4, t = idx / nw, i = (idx - t * nw) * 4;
+  const float* gp = a.P + (int64_t)t * a.ld + a.gate + (a.up < 0 ? 32 * (i >> 4) + (i & 15) : i);
+  const float* up = a.up < 0 ? gp + 16 : a.P + (int64_t)t * a.ld + a.up + i;
+  const f32x4 z = *reinterpret_cast<const f32x4*>(gp), u = *reinterpret_cast<const f32x4*>(up);
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = gelu_tanhf_(z[e]) * u[e];
+  if (a.bf) st4(static_cast<uint16_t*>(a.out) + (int64_t)t * a.ldo + i, y);
+  else st4(static_cast<float*>(a.out) + (int64_t)t * a.ldo + i, y);
+}
+
 constexpr int CW = 32;
 
 template <int D, int MODE, int NC>
-__global__ __launch_bounds__(512) void recurrence_step_k(StepArgs a) {
+__global__ __launch_bounds__(512) void recurrence_step_k(StepArgs a, int heads, GeluArgs ge) {
   constexpr int KJ = D / 64, dv = CW * NC;  // float4s of key rows a thread has
   __shared__ float so[dv];
   __shared__ __attribute__((aligned(16))) float sd[MODE == 0 ? D : 4];
-  const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, rg = tid & 15, cl = tid >> 4;
+  const int tid = threadIdx.x, rg = tid & 15, cl = tid >> 4;
+  if ((int)blockIdx.x >= heads) {  // (heads: sequences x value heads)
+    gelu_part(ge, ((int)blockIdx.x - heads) * 512 + tid);
+    return;
+  }
+  const int b = blockIdx.x / a.H, h = blockIdx.x - b * a.H;
   const int slot = a.slots[b], t = a.cu[b];
   if (slot < 0 || a.cu[b + 1] <= t) return;  // (the same for all threads)
   const int hk = h / (a.H / a.G);
@@ -140,12 +169,14 @@ __global__ __launch_bounds__(512) void recurrence_step_k(StepArgs a) {
 
 // The whole of it for T = B single tokens where it is covered: key dims of 64 and 128, value dims of 32, 64 and 128, rows on 16 bytes.
 // Arguments as in linear_recurrence (delta rules alone; gla: (a1 [T, rank] rows, a2, a2_b, tau), a decay per key channel),
-// then the norm's weight ([dv], or one per head [H dv]), the gate's rows, whether its function is the logistic one, eps, out's scale.
+// then the norm's weight ([dv], or one per head [H dv]), the gate's rows, whether its function is the logistic one, eps, out's scale;
+// with gelu_P the arguments of gelu_mul, whose work joins the launch.
 bool recurrence_step(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const c10::optional<at::Tensor>& decay,
                      const c10::optional<at::Tensor>& beta, double q_scale, at::Tensor& state, const at::Tensor& state_slots,
                      const at::Tensor& cu_q, const c10::optional<at::Tensor>& a1, const c10::optional<at::Tensor>& a2,
                      const c10::optional<at::Tensor>& a2_b, double tau, const at::Tensor& w, const at::Tensor& gate, bool sig, double eps,
-                     double scale, at::Tensor& out) {
+                     double scale, at::Tensor& out, const c10::optional<at::Tensor>& gelu_P, int64_t gate_off, int64_t up_off, int64_t F,
+                     const c10::optional<at::Tensor>& act) {
   StepArgs a{};
   a.ldq = ld_of(q, "q"), a.ldk = ld_of(k, "k"), a.ldv = ld_of(v, "v");
   f32c(state, "state");
@@ -198,12 +229,29 @@ bool recurrence_step(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   a.out = out.data_ptr();
   a.sig = sig, a.bf = out.scalar_type() == at::kBFloat16;
   a.eps = (float)eps, a.scale = (float)scale;
-  const dim3 grid((unsigned)B, (unsigned)H);
+  GeluArgs ge{};
+  if (gelu_P.has_value()) {
+    ge.ld = ld_of(*gelu_P, "P");
+    MCHECK(act.has_value() && gelu_P->size(0) == T, "the activation's rows");
+    ge.ldo = act_ld_min(*act, T, F, "activation");
+    cols_ok(*gelu_P, gate_off, up_off == -1 ? (F + 15) / 16 * 32 : F, "gate");
+    if (up_off != -1) cols_ok(*gelu_P, up_off, F, "up");
+    if ((ge.ld | gate_off | F | ge.ldo | (up_off == -1 ? 0 : up_off)) % 4 != 0 || T * F >= (int64_t(1) << 31) ||
+        ((reinterpret_cast<uintptr_t>(gelu_P->data_ptr()) | reinterpret_cast<uintptr_t>(act->data_ptr())) & 15) != 0)
+      return false;
+    ge.P = gelu_P->data_ptr<float>();
+    ge.gate = (int)gate_off, ge.up = (int)up_off, ge.F = (int)F;
+    ge.out = act->data_ptr();
+    ge.bf = act->scalar_type() == at::kBFloat16;
+    ge.total = (int)(T * F / 4);
+  }
+  MCHECK(B * H < (int64_t(1) << 30), "recurrence_step: too many heads");
+  const int heads = (int)(B * H), grid = heads + (ge.total + 511) / 512;
   auto go = [&](auto D, auto MODE) {
     constexpr int D_ = decltype(D)::value, M_ = decltype(MODE)::value;
-    if (dv == 32) recurrence_step_k<D_, M_, 1><<<grid, 512, 0, stream()>>>(a);
-    else if (dv == 64) recurrence_step_k<D_, M_, 2><<<grid, 512, 0, stream()>>>(a);
-    else recurrence_step_k<D_, M_, 4><<<grid, 512, 0, stream()>>>(a);
+    if (dv == 32) recurrence_step_k<D_, M_, 1><<<grid, 512, 0, stream()>>>(a, heads, ge);
+    else if (dv == 64) recurrence_step_k<D_, M_, 2><<<grid, 512, 0, stream()>>>(a, heads, ge);
+    else recurrence_step_k<D_, M_, 4><<<grid, 512, 0, stream()>>>(a, heads, ge);
   };
   auto by_mode = [&](auto D) {
     if (mode == 0) go(D, std::integral_constant<int, 0>());

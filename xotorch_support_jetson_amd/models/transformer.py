@@ -522,21 +522,18 @@ class ShardModel:
     return hl, torch.zeros(hl.shape[0], hn.shape[1], dtype=hn.dtype, device=h.device)
 
   def _in_and_act(self, hn: torch.Tensor, lw, rows):
-    """A parallel block's input projections P and its gated activation (None without a feed-forward)."""
+    """A parallel block's input projections P, its gated activation (None without a feed-forward) and the arguments of the gelu_mul
+    that still has to write it, or None."""
     ff = lw.spec.ff
     n0, n = lw.cols.get("gate_up", (0, 0))
     if (n and hn.is_cuda and layout_of(lw.in_w) == "stream" and hn.shape[0] >= GELU_EPI_ROWS
         and hn.shape[0] * n >= GELU_EPI_SIZE):
-      return self._proj(hn, stream_rows(lw.in_w, 0, n0)), linear(hn, stream_rows(lw.in_w, n0, n0 + n), epi="gelu_glu")
+      return self._proj(hn, stream_rows(lw.in_w, 0, n0)), linear(hn, stream_rows(lw.in_w, n0, n0 + n), epi="gelu_glu"), None
     P = self._proj(hn, lw.in_w)
     if not ff:
-      return P, None
+      return P, None, None
     act = rows("act", ff, lw.down_w.shape[1])
-    if n:
-      K.gelu_mul(P, n0, -1, ff, act)
-    else:
-      K.gelu_mul(P, lw.cols["gate"][0], lw.cols["up"][0], ff, act)
-    return P, act
+    return P, act, (P, n0, -1, ff, act) if n else (P, lw.cols["gate"][0], lw.cols["up"][0], ff, act)
 
   def _router(self, hn: torch.Tensor, w: torch.Tensor, E: int) -> torch.Tensor:
     """fp32 router logits [T, E] of a projection whose first E rows are the router."""
@@ -561,9 +558,9 @@ class ShardModel:
     K.attn_gated_chunk(q, self.kv.k[j], self.kv.v[j], inp.block_tables, inp.cu_q, inp.ctx_lens, lw.attn_pb, a.scale,
                        a.chunk, lw.spec.attn_scale, mix[:, off:off + n], max_qlen=inp.max_qlen)
 
-  def _recurrence(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor) -> None:
+  def _recurrence(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor, gelu=None) -> None:
     """Linear-attention recurrence over each sequence's state slot (delta rule or per-channel decay), then the
-    per-head gated RMS norm, scaled into the mixers' output row."""
+    per-head gated RMS norm, scaled into the mixers' output row; gelu: the feed-forward's activation, made along with it."""
     r, st, dev = lw.spec.rec, self.state, P.device
     T = P.shape[0]
     H, G, d = r.heads, r.kv_heads, r.dim
@@ -575,11 +572,12 @@ class ShardModel:
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
                        delta=(lw.cols["rb"][0], lw.cols["ra"][0], lw.dt_bias, lw.A_log, beta, decay))
       K.recurrence_norm(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], decay, beta, 1.0, st.S[j],
-                        inp.state_slots, inp.cu_q, *norm, max_qlen=inp.max_qlen)
+                        inp.state_slots, inp.cu_q, *norm, max_qlen=inp.max_qlen, gelu=gelu)
     else:
       (qo, qn), (ko, kn), (vo, vn) = lw.cols["rq"], lw.cols["rk"], lw.cols["rv"]
       K.recurrence_norm(P[:, qo:qo + qn], P[:, ko:ko + kn], P[:, vo:vo + vn], None, None, d ** -0.5, st.S[j], inp.state_slots,
-                        inp.cu_q, *norm, gla=(P, lw.cols["ra1"][0], lw.a2_w, lw.a2_b, r.tau), max_qlen=inp.max_qlen)
+                        inp.cu_q, *norm, gla=(P, lw.cols["ra1"][0], lw.a2_w, lw.a2_b, r.tau), max_qlen=inp.max_qlen,
+                        gelu=gelu)
 
   def _forward_mixed(self, x: torch.Tensor, inp: StepInputs) -> torch.Tensor:
     """Layers of config.layer_specs on an fp32 residual stream h:
@@ -621,13 +619,15 @@ class ShardModel:
     for j, li in enumerate(self.layer_ids):
       lw = w.layers[li]
       s = lw.spec
-      P, act = self._in_and_act(hn, lw, rows)
+      P, act, gelu = self._in_and_act(hn, lw, rows)
       live = sum(sz for _, sz in lw.mix_cols.values())
       mix = rows("mix", live, lw.out_w.shape[1])
       if s.attn is not None:
         self._gated_attn(P, lw, j, inp, mix)
       if s.rec is not None:
-        self._recurrence(P, lw, j, inp, mix)
+        self._recurrence(P, lw, j, inp, mix, gelu)
+      elif gelu is not None:
+        K.gelu_mul(*gelu)
       # (the sum below reduces split-K slabs of both: the second branch's lie in a scratch of their own, and its GEMM comes
       # first, so that choosing a kernel for the other does not write over them)
       y2 = self._proj_slabs(act, lw.down_w, slot=1) if s.ff else None

@@ -600,15 +600,21 @@ def gated_rmsnorm(o, w, P, g_off: int, eps: float, out_scale: float, out) -> Non
 
 
 def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu_q, w, gate, sigmoid: bool, eps: float, scale: float,
-                    out, gla=None, max_qlen: int = 0) -> None:
+                    out, gla=None, max_qlen: int = 0, gelu=None) -> None:
   """linear_recurrence, then each head's RMS norm times w ([dv], or one per head [H dv]), gate [T, H dv]'s silu (or its logistic
-  function) and scale -> out [T, >= H dv].  gla: (P, first column, a2, a2_b, tau) of gla_prep, which then makes the decays.  A step
-  of single tokens is one launch on the GPU (csrc/recurrence_step.hip) where that covers the sizes."""
+  function) and scale -> out [T, >= H dv].  gla: (P, first column, a2, a2_b, tau) of gla_prep, which then makes the decays.  gelu:
+  arguments of a gelu_mul that is done along with it.  A step of single tokens is one launch on the GPU (csrc/recurrence_step.hip)
+  where that covers the sizes."""
   if max_qlen == 1 and _gpu(q):
     a1, a2, a2_b, tau = (gla[0][:, gla[1]:gla[1] + gla[2].shape[1]], *gla[2:]) if gla is not None else (None, None, None, 0.0)
-    if require().recurrence_step(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, a1, a2, a2_b, float(tau), w, gate,
-                                 bool(sigmoid), float(eps), float(scale), out):
-      return
+    for g in ((gelu, None) if gelu is not None else (None,)):  # (an activation it cannot take along has a launch of its own)
+      if require().recurrence_step(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, a1, a2, a2_b, float(tau), w, gate,
+                                   bool(sigmoid), float(eps), float(scale), out, *(g or (None, 0, 0, 0, None))):
+        if gelu is not None and g is None:
+          gelu_mul(*gelu)
+        return
+  if gelu is not None:
+    gelu_mul(*gelu)
   T, H, dv, d = q.shape[0], state.shape[1], state.shape[2], state.shape[3]
   if gla is not None:
     decay = torch.empty(T, H * d, dtype=torch.float32, device=q.device)
