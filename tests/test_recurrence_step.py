@@ -11,7 +11,7 @@ def inputs(mode, B, H, G, d, dv, seed):
   g = torch.Generator().manual_seed(seed)
   rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
   P = rn(B, 2 * G * d + 2 * H * dv + 24)
-  q, k, v, gate, a1 = P.split([G * d, G * d, H * dv, H * dv, 24], 1)
+  q, k, v, gate = P.split([G * d, G * d, H * dv, H * dv + 24], 1)  # (a gate's rows may be wider)
   k = torch.nn.functional.normalize(k.reshape(B, G, d), dim=-1).reshape(B, G * d)
   slots = torch.randperm(B + 2, generator=g)[:B].int()
   if B > 2:

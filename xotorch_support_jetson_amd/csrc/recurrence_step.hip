@@ -223,7 +223,7 @@ bool recurrence_step(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   a.w = w.data_ptr<float>();
   a.wh = w.numel() == dv ? 0 : (int)dv;
   a.ldg = ld_of(gate, "gate");
-  MCHECK(gate.size(0) == T && gate.size(1) == H * dv, "the gate must be [T, H dv]");
+  MCHECK(gate.size(0) == T && gate.size(1) >= H * dv, "the gate must be [T, >= H dv]");
   a.gate = gate.data_ptr<float>();
   a.ldo = act_ld_min(out, T, H * dv, "out");
   a.out = out.data_ptr();

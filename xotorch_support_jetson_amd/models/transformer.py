@@ -35,7 +35,7 @@ from .config import ModelConfig
 from .weights import ShardWeights, expert
 
 # average rows per expert from which the grouped expert GEMMs run on gemm_big tiles: at most 16 experts, more
-MOE_TILE_ROWS = (16, 32)
+MOE_TILE_ROWS = (float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", "16")), float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", "32")))
 # K splits of the grouped gate/up GEMM for decode-sized batches (1: fused SiLU epilogue, no slabs)
 MOE_GU_SPLITS = int(os.environ.get("XOT_MOE_GU_SPLITS", "4"))
 MOE_BM = int(os.environ.get("XOT_MOE_BM", "0"))  # force the grouped gemm_big tile code (tests, A/B)
@@ -521,19 +521,24 @@ class ShardModel:
     hl = h.index_select(0, inp.last_idx)
     return hl, torch.zeros(hl.shape[0], hn.shape[1], dtype=hn.dtype, device=h.device)
 
-  def _in_and_act(self, hn: torch.Tensor, lw, rows):
-    """A parallel block's input projections P, its gated activation (None without a feed-forward) and the arguments of the gelu_mul
-    that still has to write it, or None."""
+  def _in_and_act(self, hn: torch.Tensor, lw, rows, later: Optional[list] = None):
+    """A parallel block's input projections P and its gated activation (None without a feed-forward).  later: takes the arguments
+    of the gelu_mul that writes the activation, where it is not the GEMM's epilogue, instead of running it."""
     ff = lw.spec.ff
     n0, n = lw.cols.get("gate_up", (0, 0))
     if (n and hn.is_cuda and layout_of(lw.in_w) == "stream" and hn.shape[0] >= GELU_EPI_ROWS
         and hn.shape[0] * n >= GELU_EPI_SIZE):
-      return self._proj(hn, stream_rows(lw.in_w, 0, n0)), linear(hn, stream_rows(lw.in_w, n0, n0 + n), epi="gelu_glu"), None
+      return self._proj(hn, stream_rows(lw.in_w, 0, n0)), linear(hn, stream_rows(lw.in_w, n0, n0 + n), epi="gelu_glu")
     P = self._proj(hn, lw.in_w)
     if not ff:
-      return P, None, None
+      return P, None
     act = rows("act", ff, lw.down_w.shape[1])
-    return P, act, (P, n0, -1, ff, act) if n else (P, lw.cols["gate"][0], lw.cols["up"][0], ff, act)
+    args = (P, n0, -1, ff, act) if n else (P, lw.cols["gate"][0], lw.cols["up"][0], ff, act)
+    if later is None:
+      K.gelu_mul(*args)
+    else:
+      later.append(args)
+    return P, act
 
   def _router(self, hn: torch.Tensor, w: torch.Tensor, E: int) -> torch.Tensor:
     """fp32 router logits [T, E] of a projection whose first E rows are the router."""
@@ -619,15 +624,14 @@ class ShardModel:
     for j, li in enumerate(self.layer_ids):
       lw = w.layers[li]
       s = lw.spec
-      P, act, gelu = self._in_and_act(hn, lw, rows)
+      gelu = [] if s.rec is not None else None  # (the recurrence takes the activation along)
+      P, act = self._in_and_act(hn, lw, rows, gelu)
       live = sum(sz for _, sz in lw.mix_cols.values())
       mix = rows("mix", live, lw.out_w.shape[1])
       if s.attn is not None:
         self._gated_attn(P, lw, j, inp, mix)
       if s.rec is not None:
-        self._recurrence(P, lw, j, inp, mix, gelu)
-      elif gelu is not None:
-        K.gelu_mul(*gelu)
+        self._recurrence(P, lw, j, inp, mix, gelu[0] if gelu else None)
       # (the sum below reduces split-K slabs of both: the second branch's lie in a scratch of their own, and its GEMM comes
       # first, so that choosing a kernel for the other does not write over them)
       y2 = self._proj_slabs(act, lw.down_w, slot=1) if s.ff else None
