@@ -128,6 +128,45 @@ constexpr int SLABS_ASKED = 12;  // of a row pass that sums split-K slabs (48 re
 // slabs count already (a step of 200 tokens lost 0.7 % with that form), so the line lies where the decode steps end
 inline bool few_rows(int64_t T) { return T <= 64; }
 
+// Per-head norm and gate of prompts: out = o / rms(o) * w * gate * scale for heads of at most 128 values in whole vectors of four.
+// What bounds it is the bytes: o and the gate once in fp32.  Half a wave has a head of TOK tokens and asks for o and the gate of all of
+// them before the first is used, 16 bytes a lane (a wave per head with 4 or 8 bytes a lane kept too little in flight).  Cold, before and
+// now, heads of 128: 4593 tokens x 32 heads logistic gate 89 us, 67 and silu gate 75, 67; 12807 x 16 117, 87 and 88, 87; heads of 68,
+// 4593 x 16 36, 22 and 29, 22.  w: head h's weights from h wh on.
+template <typename AT, bool SIG, int TOK>
+__global__ __launch_bounds__(256) void gated_norm_half_k(const float* __restrict__ o, const float* __restrict__ w, int wh,
+                                                         const float* __restrict__ P, int ldp, int g_off, float eps, float scale,
+                                                         AT* __restrict__ out, int ldo, int T, int H, int dv) {
+  const int t0 = blockIdx.x * TOK, h = blockIdx.y * 8 + (threadIdx.x >> 5), i = 4 * (threadIdx.x & 31);
+  const bool in = h < H && i < dv;
+  const int hc = min(h, H - 1), ic = in ? i : 0;  // (idle lanes read a valid place and write nothing)
+  auto ld = [](const float* p) { return *reinterpret_cast<const f32x4*>(p); };
+  f32x4 v[TOK], g[TOK];
+#pragma unroll
+  for (int r = 0; r < TOK; ++r) {
+    const int64_t t = min(t0 + r, T - 1);
+    v[r] = ld(o + (t * H + hc) * dv + ic);
+    g[r] = ld(P + t * ldp + g_off + hc * dv + ic);
+  }
+  const f32x4 wv = ld(w + hc * wh + ic);
+#pragma unroll
+  for (int r = 0; r < TOK; ++r) {
+    float ss = in ? (v[r][0] * v[r][0] + v[r][1] * v[r][1]) + (v[r][2] * v[r][2] + v[r][3] * v[r][3]) : 0.0f;
+#pragma unroll
+    for (int m = 16; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    const float k = scale / sqrtf(ss / (float)dv + eps);
+    if (!in || t0 + r >= T) continue;
+    f32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = v[r][e] * k * wv[e] * (SIG ? sigmoidf_(g[r][e]) : siluf_(g[r][e]));
+    st4(out + (int64_t)(t0 + r) * ldo + h * dv + i, y);
+  }
+}
+// the forms it takes; each caller adds the size from which it is the faster one
+inline bool gated_norm_half_ok(int64_t dv, int64_t strides, uintptr_t pointers) {
+  return dv >= 68 && dv <= 128 && dv % 4 == 0 && strides % 4 == 0 && pointers % 16 == 0;
+}
+
 // ------------------------------------------------------------------ host side
 #define MCHECK(cond, ...) TORCH_CHECK(cond, "xot mixers: ", __VA_ARGS__)
 

@@ -1198,6 +1198,19 @@ void gated_rmsnorm(const at::Tensor& o, const at::Tensor& w, const at::Tensor& P
   const uintptr_t al = reinterpret_cast<uintptr_t>(o.data_ptr()) | reinterpret_cast<uintptr_t>(w.data_ptr()) |
                        reinterpret_cast<uintptr_t>(P.data_ptr()) | reinterpret_cast<uintptr_t>(out.data_ptr());
   const int64_t st = ldp | ldo | g_off | dv;
+  // (from 2 M values: 4593 tokens x 4 heads of 128 13.0 -> 12.7 us, 512 x 16 lost, 8.1 -> 8.5)
+  if (T * H * dv >= 1 << 21 && gated_norm_half_ok(dv, st, al)) {
+    constexpr int TOK = 2;
+    const dim3 half((unsigned)((T + TOK - 1) / TOK), (unsigned)((H + 7) / 8));
+#define GH_GO(AT)                                                                                                          \
+  gated_norm_half_k<AT, false, TOK><<<half, 256, 0, stream()>>>(o.data_ptr<float>(), w.data_ptr<float>(), 0, P.data_ptr<float>(), ldp, \
+                                                                (int)g_off, (float)eps, (float)out_scale, (AT*)out.data_ptr(), ldo,   \
+                                                                (int)T, (int)H, (int)dv)
+    if (out.scalar_type() == at::kBFloat16) GH_GO(uint16_t);
+    else GH_GO(float);
+#undef GH_GO
+    return;
+  }
   const int W = dv > 128 && st % 4 == 0 && al % 16 == 0 ? 4 : dv > 64 && st % 2 == 0 && al % 8 == 0 ? 2 : 1;
 #define GR_GO(AT, W)                                                                                                       \
   gated_rmsnorm_k<AT, W><<<grid, 256, 0, stream()>>>(o.data_ptr<float>(), w.data_ptr<float>(), P.data_ptr<float>(), ldp,   \
