@@ -132,7 +132,7 @@ inline bool few_rows(int64_t T) { return T <= 64; }
 // What bounds it is the bytes: o and the gate once in fp32.  Half a wave has a head of TOK tokens and asks for o and the gate of all of
 // them before the first is used, 16 bytes a lane (a wave per head with 4 or 8 bytes a lane kept too little in flight).  Cold, before and
 // now, heads of 128: 4593 tokens x 32 heads logistic gate 89 us, 67 and silu gate 75, 67; 12807 x 16 117, 87 and 88, 87; heads of 68,
-// 4593 x 16 36, 22 and 29, 22.  w: head h's weights from h wh on.
+// 4593 x 16 36, 22 and 29, 22; behind the kernels that write its inputs 12807 x 16 silu 69, 47 and 4593 x 16 logistic 37, 18.  w: head h's weights from h wh on.
 template <typename AT, bool SIG, int TOK>
 __global__ __launch_bounds__(256) void gated_norm_half_k(const float* __restrict__ o, const float* __restrict__ w, int wh,
                                                          const float* __restrict__ P, int ldp, int g_off, float eps, float scale,
