@@ -1,4 +1,7 @@
 """The whole-K decode GEMM (csrc/gemm_wave.hip): every epilogue, column width and prologue at the edges of its range."""
+import pathlib
+import re
+
 import pytest
 import torch
 
@@ -220,3 +223,15 @@ def test_more_row_tiles_exact(gpu, M, N, Kd):
     assert torch.equal(values[slots[live]], full.view(M, H + 2, Dh)[live, H + 1].to(torch.bfloat16))
     untouched = torch.ones(pages * 64, dtype=torch.bool).index_fill_(0, slots[live], False)
     assert not kc.cpu().view(-1, Dh)[untouched].any() and not values[untouched].any()
+
+
+def test_loads_past_an_operand_are_bounds_checked():
+  """A buffer load's scalar offset is no part of its bounds check, so a load that may pass the end of its operand (a chunk past K,
+  a stage past the last one) carries its place in the vector offset.  The exceptions are named: `inside` is within the operand
+  for all lanes, and loads to LDS go stage by stage through whole tiles."""
+  csrc = pathlib.Path(L.__file__).parents[1] / "csrc"
+  calls = [(f.name, a) for f in sorted(csrc.glob("*.hip")) for a in re.findall(r"amdgcn_raw_buffer_load_b\d+\(([^()]*(?:\([^()]*\)[^()]*)*)\)", f.read_text())]
+  assert {"gemm_wave.hip", "gemm_group.hip", "recurrence_chunk.hip"} <= {f for f, _ in calls}
+  assert not [(f, a) for f, a in calls if a.split(",")[-2].strip() not in ("0", "inside")]
+  group = (csrc / "gemm_group.hip").read_text()  # its weights: the slice's last block at most
+  assert re.findall(r"buf16nt\(wr,.*\)", group) == ["buf16nt(wr, lane * 16, min(ch * U + u, nb - 1) * 1024)"]

@@ -18,11 +18,14 @@ namespace {
 constexpr int U = 8, TW = 8, SL = 4 * U;  // k blocks a stage; waves = column tiles of a workgroup; 16-byte slots of a row's chunk
 constexpr int ROWS = 64, HALF = ROWS * SL * 16;
 
-__device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(s16x8, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+// 16 bytes a lane, zeros past the end of r: all of the offset is in the lane's register, for the scalar offset of a buffer load is no
+// part of its bounds check
+__device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(s16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
-__device__ __forceinline__ s16x8 buf16nt(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(s16x8, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 2));
+// (inside: a scalar offset behind which all lanes' bytes lie within r)
+__device__ __forceinline__ s16x8 buf16nt(__amdgpu_buffer_rsrc_t r, int off, int inside) {
+  return __builtin_bit_cast(s16x8, __builtin_amdgcn_raw_buffer_load_b128(r, off, inside, 2));
 }
 
 struct Stage {
@@ -54,7 +57,7 @@ __device__ __forceinline__ void group_rows(char* smem, __amdgpu_buffer_rsrc_t wr
   s16x8 xv[MT];
   auto xload = [&](int ch) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xv[i] = buf16(xr, xo[i], min(ch, nch - 1) * SL * 16);
+    for (int i = 0; i < MT; ++i) xv[i] = buf16(xr, xo[i] + min(ch, nch - 1) * SL * 16);  // (a last chunk may pass X's end)
   };
   auto xstore = [&](int buf) {
 #pragma unroll

@@ -26,9 +26,11 @@ namespace {
 
 constexpr int U = 8;  // k blocks a stage
 
-__device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, int voff, int soff, bool nt) {
-  return __builtin_bit_cast(s16x8, nt ? __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 2)
-                                      : __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+// 16 bytes a lane, zeros past the end of r: all of the offset is in the lane's register, for the scalar offset of a buffer load is no
+// part of its bounds check
+__device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, unsigned off, bool nt) {
+  return __builtin_bit_cast(s16x8, nt ? __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 2)
+                                      : __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
 }
 
 // MT: 16-row tiles of X.  XL: X pieces (1 KB) a wave copies per chunk.  rw: rows of X kept in LDS (a power of two >= M up to 16,
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE 
   };
   auto load = [&](Stage& s, int ch) {  // the wave's blocks of chunk ch (past K: zeros, not used)
 #pragma unroll
-    for (int u = 0; u < U; ++u) s.w[u] = buf16(wr, lane * 16 + u * 1024, (ch * CB + p * U) * 1024, true);
+    for (int u = 0; u < U; ++u) s.w[u] = buf16(wr, lane * 16u + (ch * CB + p * U + u) * 1024u, true);
   };
   // piece l of a chunk's rows of X: 64 consecutive slots of one row (or of 64 / SL rows)
   constexpr int LR = SL >= 64 ? SL / 64 : 1, RL = SL >= 64 ? 1 : 64 / SL;
@@ -76,8 +78,9 @@ __global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE 
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
       const int l = min(wave + i * nw, npc - 1);
-      if constexpr (RL > 1) xv[i] = buf16(xr, min(l * RL + lane / SL, M - 1) * ldx * 2 + (lane % SL) * 16, ch * CB * 64, false);
-      else xv[i] = buf16(xr, lane * 16, (l / LR) * ldx * 2 + (l % LR) * 1024 + ch * CB * 64, false);
+      // (a chunk past K: the next row's numbers or, behind the last row, zeros; not used)
+      if constexpr (RL > 1) xv[i] = buf16(xr, min(l * RL + lane / SL, M - 1) * ldx * 2u + (lane % SL) * 16u + ch * CB * 64u, false);
+      else xv[i] = buf16(xr, lane * 16u + (l / LR) * ldx * 2u + (l % LR) * 1024u + ch * CB * 64u, false);
     }
   };
   const int half = rw * SL * 16;  // bytes of one of the two buffers
