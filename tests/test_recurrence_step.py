@@ -70,3 +70,61 @@ def test_activation_along_with_it(gpu, mode, d, F, tiles, B):
   K.recurrence_norm(**dev, out=plain)
   K.recurrence_norm(**dict(dev, state=state), out=out, gelu=(*args, act))
   assert torch.equal(act, want) and torch.equal(out[live], plain[live]) and torch.equal(state, dev["state"])
+
+
+def float64_rows(a):
+  """recurrence_norm's definition in float64, token by token (inputs' single tokens), and the rows that have a slot."""
+  B, (_, H, dv, d) = a["q"].shape[0], a["state"].shape
+  G = a["q"].shape[1] // d
+  q, k, v, w, gate = (a[n].double() for n in ("q", "k", "v", "w", "gate"))
+  heads = lambda t: t.reshape(B, G, d).repeat_interleave(H // G, 1)  # noqa: E731
+  q, k, v = heads(q) * a["q_scale"], heads(k), v.reshape(B, H, dv)
+  S = a["state"].double()[a["state_slots"].clamp(min=0).long()]
+  if a["beta"] is None:
+    P, c0, a2, b, tau = a["gla"]
+    decay = torch.exp(torch.nn.functional.logsigmoid(P[:, c0:c0 + a2.shape[1]].double() @ a2.double().t() + b.double()) / tau)
+  else:
+    decay = a["decay"].double()
+  S = S * decay.reshape(B, H, 1, -1)
+  u = v if a["beta"] is None else a["beta"].double()[..., None] * (v - torch.einsum("bhvd,bhd->bhv", S, k))
+  o = torch.einsum("bhvd,bhd->bhv", S + u[..., None] * k[:, :, None], q)
+  gate = gate[:, :H * dv].reshape(B, H, dv)
+  o = o / torch.sqrt(o.square().mean(-1, keepdim=True) + a["eps"]) * (w.view(H, dv) if w.numel() == H * dv else w)
+  o = o * (torch.sigmoid(gate) if a["sigmoid"] else torch.nn.functional.silu(gate)) * a["scale"]
+  return o.reshape(B, H * dv), a["state_slots"] >= 0
+
+
+def norm_forms(mode, sigmoid, per_head, d, B=5):
+  H, G, dv = 4, 4 if mode == "gla" else 2, 64
+  a = inputs(mode, B, H, G, d, dv, d + 7)
+  w = torch.randn(H * dv if per_head else dv, generator=torch.Generator().manual_seed(3))
+  return dict(a, sigmoid=sigmoid, scale=0.7, w=w), torch.zeros(B, H * dv)
+
+
+@pytest.mark.parametrize("mode", ["delta", "channel", "gla"])
+@pytest.mark.parametrize("sigmoid", [False, True])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_every_norm_form_means_the_same(mode, sigmoid, per_head):
+  """Both gates with both weights and a scale, by the passes behind each other."""
+  a, out = norm_forms(mode, sigmoid, per_head, 64)
+  want, live = float64_rows(a)
+  K.recurrence_norm(**a, out=out)
+  torch.testing.assert_close(out[live].double(), want[live], rtol=1e-4, atol=1e-4)  # (bound: test_against_the_plain_form)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["delta", "channel", "gla"])
+@pytest.mark.parametrize("sigmoid", [False, True])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("d,max_qlen", [(64, 1), (64, 0), (32, 1)])
+def test_every_norm_form_on_every_route(gpu, mode, sigmoid, per_head, d, max_qlen):
+  """The same on the GPU: in one launch, and by general kernels where the step's longest sequence is not known or the key
+  dims are not covered."""
+  a, out = norm_forms(mode, sigmoid, per_head, d)
+  want, live = float64_rows(a)
+  dev = {n: t.to(gpu) if torch.is_tensor(t) else t for n, t in a.items()}
+  if a["gla"]:
+    dev["gla"] = tuple(t.to(gpu) if torch.is_tensor(t) else t for t in a["gla"])
+  out = out.to(gpu)
+  K.recurrence_norm(**dict(dev, max_qlen=max_qlen), out=out)
+  torch.testing.assert_close(out.cpu()[live].double(), want[live], rtol=1e-4, atol=1e-4)

@@ -621,10 +621,15 @@ def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu
     gla_prep(*gla, decay)
   o = torch.empty(T, H * dv, dtype=torch.float32, device=q.device)
   linear_recurrence(q, k, v, decay, beta, q_scale, state, state_slots, cu_q, o, max_qlen=max_qlen)
-  if sigmoid:
-    gated_group_norm(o, None, w, gate, 0, H, eps, out)
-  else:
+  if sigmoid:  # (that pass has a weight per head and no scale)
+    wh = w if w.numel() == H * dv else w.repeat(H)
+    gated_group_norm(o, None, wh if scale == 1.0 else wh * scale, gate, 0, H, eps, out)
+  elif w.numel() == dv:
     gated_rmsnorm(o, w, gate, 0, eps, scale, out[:, :H * dv])
+  else:  # (that one has a weight for all heads)
+    y = torch.empty_like(o)
+    gated_rmsnorm(o, torch.ones_like(w[:dv]), gate, 0, eps, scale, y)
+    out[:, :H * dv].copy_(y * w)
 
 
 # ------------------------------------------------------------------ post-norm blocks (csrc/hybrid.hip)
