@@ -110,8 +110,28 @@ def test_shared_experts_exact(gpu, T, n, N, Kd, S):
   slot_of[order] = torch.arange(T * k, dtype=torch.int32)
   want = h.double() + sum(sh.double().view(n, T, N)) + (topw.double()[:, None] * full.double()[slot_of.long()]).view(T, k, N).sum(1)
   out = h.to(gpu)
-  C.moe_combine(y, slot_of.to(gpu), topw.to(gpu), out, S)
+  C.moe_combine(y, slot_of.to(gpu), topw.to(gpu), out, S, n)
   torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8, atol=1e-3)
   h2, normed = h.to(gpu), torch.empty(T, N, dtype=torch.bfloat16, device=gpu)
-  C.moe_combine_norm(y, slot_of.to(gpu), topw.to(gpu), h2, S, torch.ones(N, dtype=torch.bfloat16, device=gpu), normed, 1e-5)
+  C.moe_combine_norm(y, slot_of.to(gpu), topw.to(gpu), h2, S, torch.ones(N, dtype=torch.bfloat16, device=gpu), normed, 1e-5, n)
   assert torch.equal(h2, out)
+
+
+@pytest.mark.gpu
+def test_combine_takes_exactly_the_rows_it_was_told_of(gpu):
+  """Rows beyond splits x tokens x (choices + shared experts) are refused, not taken for shared experts: two K slices given as
+  one, a shared expert that was not announced, and the other way round."""
+  from xotorch_support_jetson_amd.ops._ext import require
+  C, T, k, D = require(), 3, 2, 64
+  slot_of, topw = torch.arange(T * k, dtype=torch.int32, device=gpu), torch.ones(T, k, device=gpu)
+  h, lnw = torch.zeros(T, D, dtype=torch.bfloat16, device=gpu), torch.ones(D, dtype=torch.bfloat16, device=gpu)
+  for rows, splits, shared, ok in ((T * k, 1, 0, True), (2 * T * k, 2, 0, True), (2 * T * (k + 1), 2, 1, True), (2 * T * k, 1, 0, False),
+                                   (T * (k + 1), 1, 0, False), (T * k, 1, 1, False), (T * k, 1, -1, False), (2 * T * k, 1, 1, False)):
+    y = torch.zeros(rows, D, device=gpu)
+    for call in (lambda: C.moe_combine(y, slot_of, topw, h, splits, shared),
+                 lambda: C.moe_combine_norm(y, slot_of, topw, h, splits, lnw, torch.empty_like(h), 1e-5, shared)):
+      if ok:
+        call()
+      else:
+        with pytest.raises(RuntimeError):
+          call()

@@ -824,16 +824,16 @@ void mla_attn(const at::Tensor& q_lat, const at::Tensor& q_pe, const at::Tensor&
   XCHECK(rc == 0, "mla_attn: unsupported DL=", DL, " DR=", DR);
 }
 
+// splits: K slices of the expert rows y, [splits, T (k + nsh), D]; nsh: shared experts, whose rows follow the routed ones
 void moe_combine(const at::Tensor& y, const at::Tensor& slot_of, const at::Tensor& topw, at::Tensor& h,
-                 int64_t splits) {
+                 int64_t splits, int64_t nsh) {
   CHECK_GPU(y);
   CHECK_DT(y, at::kFloat);
   CHECK_BF16(h);
   XCHECK(all_contig_gpu(y, slot_of, topw, h), "moe_combine: tensors must be contiguous GPU");
   const int64_t T = h.size(0), D = h.size(1), k = slot_of.numel() / T;
-  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) % (splits * T) == 0 && y.size(0) >= splits * T * k &&
-             topw.numel() == T * k, "moe_combine: shapes");
-  const int64_t nsh = y.size(0) / (splits * T) - k;  // shared experts
+  XCHECK(splits >= 1 && nsh >= 0 && D % 8 == 0 && y.size(1) == D && y.size(0) == splits * T * (k + nsh) && topw.numel() == T * k,
+         "moe_combine: shapes");
   xot::launch_moe_combine(y.data_ptr<float>(), slot_of.data_ptr<int>(), topw.data_ptr<float>(), bf(h), (int)T, (int)k,
                           (int)nsh, (int)D, (int)splits, (long)(T * (k + nsh) * D), cur_stream());
 }
@@ -848,17 +848,16 @@ void splitk_silu(const at::Tensor& ws, int64_t S, at::Tensor& y) {
 }
 
 void moe_combine_norm(const at::Tensor& y, const at::Tensor& slot_of, const at::Tensor& topw, at::Tensor& h,
-                      int64_t splits, const at::Tensor& ln_w, at::Tensor& out, double eps) {
+                      int64_t splits, const at::Tensor& ln_w, at::Tensor& out, double eps, int64_t nsh) {
   CHECK_DT(y, at::kFloat);
   CHECK_BF16(h);
   CHECK_BF16(ln_w);
   CHECK_BF16(out);
   XCHECK(all_contig_gpu(y, slot_of, topw, h, ln_w, out), "moe_combine_norm: tensors must be contiguous GPU");
   const int64_t T = h.size(0), D = h.size(1), k = slot_of.numel() / T;
-  XCHECK(splits >= 1 && D % 8 == 0 && y.size(1) == D && y.size(0) % (splits * T) == 0 && y.size(0) >= splits * T * k &&
+  XCHECK(splits >= 1 && nsh >= 0 && D % 8 == 0 && y.size(1) == D && y.size(0) == splits * T * (k + nsh) &&
              topw.numel() == T * k && ln_w.numel() == D && out.sizes() == h.sizes(),
          "moe_combine_norm: shapes");
-  const int64_t nsh = y.size(0) / (splits * T) - k;  // shared experts
   const int rc = xot::launch_moe_combine_norm(y.data_ptr<float>(), slot_of.data_ptr<int>(), topw.data_ptr<float>(),
                                               bf(h), bf(ln_w), bf(out), (int)T, (int)k, (int)nsh, (int)D, (int)splits,
                                               (long)(T * (k + nsh) * D), (float)eps, cur_stream());
@@ -1216,7 +1215,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("cu_q"), py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
         py::arg("nparts"), py::arg("scale"), py::arg("wide") = 0);
   m.def("moe_combine", &moe_combine, py::arg("y"), py::arg("slot_of"), py::arg("topw"), py::arg("h"),
-        py::arg("splits") = 1);
+        py::arg("splits") = 1, py::arg("n_shared") = 0);
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
         py::arg("nparts"), py::arg("scale"), py::arg("algo") = 2, py::arg("merge") = true);
@@ -1228,7 +1227,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("cu_q"), py::arg("ctx_lens"), py::arg("out"), py::arg("max_qlen"), py::arg("scale"), py::arg("algo") = 2);
   m.def("router_logits", &router_logits);
-  m.def("moe_combine_norm", &moe_combine_norm);
+  m.def("moe_combine_norm", &moe_combine_norm, py::arg("y"), py::arg("slot_of"), py::arg("topw"), py::arg("h"), py::arg("splits"),
+        py::arg("ln_w"), py::arg("out"), py::arg("eps"), py::arg("n_shared") = 0);
   m.def("splitk_silu", &splitk_silu);
   m.def("splitk_rope_kv_write", &splitk_rope_kv_write);
   m.def("attn_train_transpose", &attn_train_transpose);

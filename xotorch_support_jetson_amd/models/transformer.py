@@ -475,9 +475,9 @@ class ShardModel:
     C.gemm_moe(act, lw.down_w, y, off, None, K.EPI["none"], T, layout_of(lw.down_w) == "stream", S, bm_dn, w_sh=w_sh[1])
     if next_norm is not None:  # combine + the following RMSNorm in one kernel
       out = torch.empty_like(h)
-      C.moe_combine_norm(y, slot_of, topw, h, S, next_norm, out, float(c.rms_norm_eps))
+      C.moe_combine_norm(y, slot_of, topw, h, S, next_norm, out, float(c.rms_norm_eps), n_sh)
       return out
-    C.moe_combine(y, slot_of, topw, h, S)
+    C.moe_combine(y, slot_of, topw, h, S, n_sh)
     return None
 
   # ------------------------------------------------------------------ layers of differing mixers
