@@ -171,7 +171,13 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
   // X: instruction i of wave w covers rows (1024 / (2*BK)) * (A_INSTR*w + i) .. ; lane -> row +lane/SPR,
   // physical slot lane%SPR holding logical slot (lane%SPR) ^ aswz(row).
   const uint16_t* asrc[A_INSTR];
-  auto aq = [&](int i) { return A_UNEVEN ? 8 * i + wave : A_INSTR * wave + i; };
+  // PP 2: a row half is copied by the waves that read it (wl of four); its first quarter's MT instructions (row tiles of A half 0)
+  // by their instructions below a_lead, the second's by the others, which are issued a phase later (issue_tail)
+  const int wl = wave & 3, a_lead = MT / 4 + (wl < MT % 4 ? 1 : 0);
+  auto aq = [&](int i) {
+    if constexpr (PP == 2) return wm * 2 * MT + (i < a_lead ? wl + 4 * i : MT + 3 - wl + 4 * (i - a_lead));
+    return A_UNEVEN ? 8 * i + wave : A_INSTR * wave + i;
+  };
 #pragma unroll
   for (int i = 0; i < A_INSTR; ++i) {
     const int row = (64 / SPR) * min(aq(i), NAI - 1) + lane / SPR;
@@ -195,7 +201,30 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int ni_w = NI - (A_UNEVEN && wave_u >= NAI % 8 ? 1 : 0) - (B_UNEVEN && wave_u >= NBI % 8 ? 1 : 0);
 
+  // PP 2: the X rows of A half 1 of stage t, and everything else of it
+  constexpr int TAIL_MIN = PP == 2 ? A_INSTR - MT / 4 - (MT % 4 ? 1 : 0) : 0;  // the fewest instructions of a wave's tail
+  const int lead_u = __builtin_amdgcn_readfirstlane(a_lead);
+  auto issue_tail = [&](int t, int buf) {
+#pragma unroll
+    for (int i = MT / 4; i < A_INSTR; ++i)
+      if (MT % 4 == 0 || i >= lead_u) glds16<AUXA>(asrc[i] + t * BK, smem + buf * STAGE + aq(i) * 512);
+  };
+  auto issue_lead = [&](int t, int buf) {
+    uint16_t* As = smem + buf * STAGE;
+    const int k0 = t * BK;
+    const size_t woff = (size_t)(k0 >> 7) * 2048 + ((k0 & 127) >> 5) * 512;
+#pragma unroll
+    for (int i = 0; i < MT / 4 + (MT % 4 ? 1 : 0); ++i)
+      if (MT % 4 == 0 || i < lead_u) glds16<AUXA>(asrc[i] + k0, As + aq(i) * 512);
+#pragma unroll
+    for (int i = 0; i < B_INSTR; ++i) glds16<AUXB>(bsrc[i] + woff, As + A_ELEMS + bq(i) * 512);
+  };
   auto issue = [&](int t, int buf) {  // stage t (absolute k step) -> LDS buffer buf
+    if constexpr (PP == 2) {
+      issue_lead(t, buf);
+      issue_tail(t, buf);
+      return;
+    }
     uint16_t* As = smem + buf * STAGE;
     uint16_t* Bs = As + A_ELEMS;
     const int k0 = t * BK;
@@ -318,29 +347,38 @@ __global__ __launch_bounds__(512, 1) void gemm_big_kernel(const uint16_t* __rest
       if (half == 1) bar();  // row-half 1 runs one barrier behind
       if constexpr (PP == 2) {
       for (int t = 0; t < T; ++t) {
-        // two phases of 32 MFMAs: {A half 0, both B halves} -> quads (0,0), (0,1); {A half 1, refill with stage
-        // t+2, retire stage t+1} -> quads (1,1), (1,0).  Four barriers per stage instead of eight.
+        // two phases of 32 MFMAs: {A half 0, both B halves} -> quads (0,0), (0,1); {A half 1} -> quads (1,1), (1,0).  Four
+        // barriers per stage instead of eight.  A wave's LDS-DMA issue inside its MFMA phase costs more than the whole schedule
+        // gains (profiles/r4/pp2/), so refills go into the read phases, each into rows whose readers have passed a barrier since:
+        // stage t+2's B and A half 0 behind barrier 2 (A half 0: this row half's MFMAs have waited for it; B: the other half, a
+        // barrier behind, has waited for its reads in front of its barrier 1), its A half 1 in the next stage's first phase.  Both
+        // vmcnt waits leave one stage's instructions in flight.  us, the whole refill in the second phase, where a stalled
+        // wave's reads could have come behind it / here: 4096 x 28672 x 4096 SiLU 757 / 739, 1000 x 11264 x 2048 52.2 / 49.9, 192 rows
+        // 384 x 28672 x 4096 90 / 91, 64 experts of 1408 x 2048 at 700 tokens 154 / 153.
         const int buf = t & 1;
-        read_a(buf, 0);
         read_b(buf, 0);
         read_b(buf, 1);
+        asm volatile("" ::: "memory");
+        read_a(buf, 0);
+        if (t > 0) {
+          if (t + 1 < T) {
+            issue_tail(t_beg + t + 1, buf ^ 1);
+            wait_vm<NI>();  // this stage's A half 1
+          } else {
+            wait_vm<0>();
+          }
+        }
+        wait_lgkm<2 * MQ>();  // (W's reads, which come first)
         bar();
         quad(0, 0);
         quad(0, 1);
         bar();
-        read_a(buf, 1);  // last read of this stage by this wave
-        // Refill with stage t+2 here, in the read phase: a wave's LDS-DMA issue inside its MFMA phase costs more
-        // than the whole schedule gains (measured: refill after the barrier, or only the A rows the group is
-        // still reading moved there, ran slower than the four-phase schedule, profiles/r4/pp2/).  The refill
-        // lands >= one L2 round trip after issue, while the reads it could overtake -- the group's own A rows
-        // here, issued at the start of this phase, and the other group's B reads, issued before the previous
-        // barrier -- complete within one LDS round trip (the same margin the four-phase schedule relies on).
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        read_a(buf, 1);
         if (t + 2 < T) {
-          issue(t_beg + t + 2, buf);
-          wait_vm<NI>();
-        } else {
-          wait_vm<0>();
+          issue_lead(t_beg + t + 2, buf);
+          wait_vm<NI>();  // the next stage but for its A half 1
+        } else if (t + 1 < T) {
+          wait_vm<TAIL_MIN>();
         }
         bar();
         quad(1, 1);
