@@ -1,5 +1,9 @@
 """Grouped expert GEMMs (csrc/gemm_group.hip and the grouped order of csrc/gemm_big.hip): experts without rows, row counts at the
 edges of every row tile, K slices, gathered rows, and the rule that picks a kernel."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -39,6 +43,15 @@ def test_rule():
   assert moe_tiles(65, 2, 8) == moe_tiles(384, 2, 8) == moe_tiles(48, 2, 4) == (1128, 1128, 2)
   assert moe_tiles(342, 6, 64) == moe_tiles(1024, 6, 64) == (2128, 2128, 2)
   assert moe_tiles(385, 2, 8) == (192, 192, 4) and moe_tiles(8192, 6, 64) == (256, 256, 2)
+
+
+@pytest.mark.parametrize("rows,tiled", [("8", [True] * 4), ("60", [False] * 3 + [True])])
+def test_switch_moves_every_line(rows, tiled):
+  """XOT_MOE_BIG_MIN_ROWS: one line for few and for many experts, steps of up to 64 tokens included (8, 12, 16 and 64 rows)."""
+  code = ("from xotorch_support_jetson_amd.models.transformer import moe_tiles\n"
+          "print([moe_tiles(*a)[0] > 0 for a in ((32, 2, 8), (128, 6, 64), (64, 2, 8), (256, 2, 8))])")
+  got = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, XOT_MOE_BIG_MIN_ROWS=rows), capture_output=True, text=True, check=True)
+  assert got.stdout.strip() == str(tiled)
 
 
 @pytest.mark.gpu

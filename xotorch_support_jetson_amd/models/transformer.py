@@ -34,8 +34,9 @@ from ..ops.rope import longrope_window, rope_shift, rope_table
 from .config import ModelConfig
 from .weights import ShardWeights, expert
 
-# average rows per expert from which the grouped expert GEMMs run on gemm_big tiles: at most 16 experts, more
-MOE_TILE_ROWS = (float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", "16")), float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", "32")))
+# average rows per expert from which the grouped expert GEMMs run on gemm_big tiles: at most 16 experts, more, and at most 16 in a step
+# of up to 64 tokens (XOT_MOE_BIG_MIN_ROWS: one line for all)
+MOE_TILE_ROWS = tuple(float(os.environ.get("XOT_MOE_BIG_MIN_ROWS", rows)) for rows in ("16", "32", "24"))
 # K splits of the grouped gate/up GEMM for decode-sized batches (1: fused SiLU epilogue, no slabs)
 MOE_GU_SPLITS = int(os.environ.get("XOT_MOE_GU_SPLITS", "4"))
 MOE_BM = int(os.environ.get("XOT_MOE_BM", "0"))  # force the grouped gemm_big tile code (tests, A/B)
@@ -61,7 +62,7 @@ def moe_tiles(T: int, k: int, E: int) -> Tuple[int, int, int]:
   streamed, 22 rows 365 + 156 streamed, 330 + 142 (1128); 64 rows 343 + 148 (1128), 419 + 184 (2256), 375 + 157 (2192); 128 rows
   485 + 248, 448 + 190, 404 + 172."""
   rows = T * k / E
-  if rows < MOE_TILE_ROWS[E > 16] or (E <= 16 and T <= 64 and rows < 24):
+  if rows < MOE_TILE_ROWS[1 if E > 16 else 2 if T <= 64 else 0]:
     return 0, 0, 0
   if rows <= 96:
     return (2128, 2128, 2) if E > 16 else (1128, 1128, 2)
