@@ -1,5 +1,9 @@
 """The 128- and 64-row tiles (and the 160 x 256 one) of the large-M GEMM (csrc/gemm_big.hip codes 1280128, 1280256, 640128, 640256): partial row and column tiles, fewer stages
 than the pipeline holds, K splits, every epilogue; and where the policy offers them."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -19,6 +23,18 @@ def test_candidates():
   assert rows64(16, 8192, 4096) == [] and rows64(65, 8192, 4096) == [] and rows64(64, 8200, 4096) == []
   times = {("big", 1280256, 1): 1.0, ("big", 2256, 1): 1.04}
   assert L._tie_break(times, 128) == ("big", 1280256, 1) and L._tie_break(times, 200) == ("big", 2256, 1)
+
+
+@pytest.mark.parametrize("least,offered", [("129", [False] * 3), ("40", [False, True, True]), (None, [True] * 3)])
+def test_switch_keeps_the_kernel_out(least, offered):
+  """XOT_BIG_MIN_M holds for the 64-row tiles as well: rows 24, 40 and 64."""
+  code = ("from xotorch_support_jetson_amd.ops import linear as L\n"
+          "print([bool(L.GemmPolicy._rows64_cands(M, 8192, 4096)) for M in (24, 40, 64)])")
+  env = {k: v for k, v in os.environ.items() if k != "XOT_BIG_MIN_M"}
+  if least:
+    env["XOT_BIG_MIN_M"] = least
+  got = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True)
+  assert got.stdout.strip() == str(offered)
 
 
 @pytest.mark.gpu

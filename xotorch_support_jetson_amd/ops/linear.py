@@ -59,8 +59,8 @@ STREAM_MAX_M = int(os.environ.get("XOT_STREAM_MAX_M", "512"))
 WAVE_MAX_M = 16
 # ... and at all (its row tiles; a chunk of X for more would not fit beside a second workgroup's)
 WIDE_MAX_M = 64
-# smallest M for which gemm_big is a candidate
-BIG_MIN_M = int(os.environ.get("XOT_BIG_MIN_M", "65"))
+# smallest M for which gemm_big is a candidate, and for which its 64-row tiles are (XOT_BIG_MIN_M: no gemm_big below that)
+BIG_MIN_M, ROWS64_MIN_M = (int(os.environ.get("XOT_BIG_MIN_M", m)) for m in ("65", "17"))
 
 
 def _m_bucket(M: int) -> int:
@@ -198,7 +198,7 @@ def _default_table_path():
     dev = torch.cuda.get_device_name(torch.cuda.current_device()).replace(" ", "_").replace("/", "_")
     from ..helpers import xot_home
     # settings that change the candidate sets are part of the name, so a table never answers for another
-    tag = (f"{os.environ.get('XOT_GEMM', 'auto')}-{STREAM_MAX_M}-{BIG_MIN_M}-{SLAB_TBPS:g}"
+    tag = (f"{os.environ.get('XOT_GEMM', 'auto')}-{STREAM_MAX_M}-{BIG_MIN_M}-{ROWS64_MIN_M}-{SLAB_TBPS:g}"
            f"{'-blas' if BLAS_CAND else ''}-t{TIE:g}-x{TIE_X:g}{'' if PP2 else '-nopp2'}")
     return str(xot_home() / "gemm" / f"{dev}-{st.st_size:x}-{int(st.st_mtime):x}-{tag}.json")
   except Exception:  # noqa: BLE001 - no table then; tuning still works in memory
@@ -418,7 +418,7 @@ class GemmPolicy:
     stages in LDS), where the stream GEMM passes them through registers.  us, the best other / here: 24 x 28672 x 4096 44.3 / 41.5,
     64 x 57344 x 8192 155 / 146, 64 x 128256 x 8192 367 / 353, 64 x 102400 x 2048 93 / 84; the K slices of 2048 x 2048 stay with
     the stream GEMM (10.7 / 12.3).  At 16 rows and fewer X is no load to speak of."""
-    if not WAVE_MAX_M < M <= 64 or N % 16:
+    if not max(WAVE_MAX_M + 1, ROWS64_MIN_M) <= M <= 64 or N % 16:
       return []
     return [("big", 640000 + bn, S) for bn in (128, 256) for S in (1, 2, 3, 4, 6, 8)
             if N >= bn and (S == 1 or (-(-N // bn) < 256 and -(-N // bn) * S <= 1024 and Kd // 64 >= 2 * S))]
