@@ -32,7 +32,8 @@ struct Stage {
   s16x8 w[U];
 };
 
-// One block of M <= 16 MT rows.  wr: the wave's tile and K slice; xr: X from the slice's first column on, to
+// One block of M <= 16 MT rows (its registers: one and two row tiles fit the 128 of four waves a SIMD, three spill a dozen, four a
+// hundred, 116 to 140 bytes a lane).  wr: the wave's tile and K slice; xr: X from the slice's first column on, to
 // the end of its last row; rows: gather entries of the block's slots, or null with the slots' rows from row0 on.
 template <int MT, int EPI, bool F32>
 __device__ __forceinline__ void group_rows(char* smem, __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, const int* rows, int row0,
@@ -167,42 +168,67 @@ struct Shared {
   long expert, stride;      // 1 KB blocks between shared experts, and between column tiles
 };
 
-// blockIdx: (column group, K slice, shared expert and block of tokens | expert).  An expert's rows are taken 64 at a time.
+// Rows 64 .. of an expert with more, as blocks of their own: the q-th such block of all experts (one wave's search through the
+// offsets; the result is uniform), or -1
+__device__ __forceinline__ int more_rows(const int* __restrict__ off, int E, int q, int* r0) {
+  const int lane = threadIdx.x & 63;
+  for (int b = 0; b < E; b += 64) {
+    const int i = min(b + lane, E - 1), n = b + lane < E ? max(off[i + 1] - off[i] - 1, 0) / ROWS : 0;
+    int sum = n;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+      const int v = __shfl_up(sum, m, 64);
+      if (lane >= m) sum += v;
+    }
+    const unsigned long long behind = __ballot(sum > q);
+    if (behind != 0) {
+      const int l = __builtin_ctzll(behind);
+      *r0 = (q - __builtin_amdgcn_readlane(sum - n, l) + 1) * ROWS;
+      return b + l;
+    }
+    q -= __builtin_amdgcn_readlane(sum, 63);
+  }
+  return -1;
+}
+
+// blockIdx: (column group, K slice, shared expert and block of tokens | expert | further blocks of experts with more than 64 rows).
+// Those last ones are as many as the slots can make and mostly leave at once, all at the launch's end; one workgroup through all of an
+// expert's blocks streamed its weights once a block, one after the other (64 experts of 1408 x 2048, 340 tokens that all
+// want the same six: gate/up + down 184 + 139 us, here 82 + 42; evenly spread 138 + 72, here 131 + 69).
 template <int EPI, bool F32>
 __global__ __launch_bounds__(64 * TW, 4) void gemm_group_kernel(const uint16_t* __restrict__ X, int ldx, int xrows,
                                                                 const uint16_t* __restrict__ W, void* __restrict__ Yv, int ldy,
-                                                                const int* __restrict__ off, const int* __restrict__ gather, int N,
+                                                                const int* __restrict__ off, const int* __restrict__ gather, int E, int N,
                                                                 int K, long ysplit, float epi_arg, Shared sh) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nb = (K >> 5) / gridDim.y, kb = blockIdx.y * nb, tile = blockIdx.x * TW + wave;
-  int e = (int)blockIdx.z - sh.n * sh.blocks, first, count, x0;  // slots, and without gather their rows of X
+  int e = (int)blockIdx.z - sh.n * sh.blocks, first, M, x0;  // slots, and without gather their rows of X
   const uint16_t* wt;
   if (e >= 0) {
-    first = off[e], count = off[e + 1] - first, x0 = first;
+    int r0 = 0;
+    if (e >= E) e = more_rows(off, E, e - E, &r0);
+    if (e < 0) return;
+    x0 = first = off[e] + r0, M = min(ROWS, off[e + 1] - first);
     wt = W + (((size_t)e * (N >> 4) + tile) * (K >> 5) + kb) * 512;
   } else {  // (first: their work does not hang on the routing, and a block is a full one)
     const int j = blockIdx.z / sh.blocks, t0 = (blockIdx.z - j * sh.blocks) * ROWS;
-    first = sh.slot0 + j * sh.T + t0, count = min(ROWS, sh.T - t0), x0 = gather != nullptr ? t0 : first;
+    first = sh.slot0 + j * sh.T + t0, M = min(ROWS, sh.T - t0), x0 = gather != nullptr ? t0 : first;
     wt = sh.W + (j * sh.expert + tile * sh.stride + kb) * 512;
   }
-  if (count <= 0) return;
+  if (M <= 0) return;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wt), (short)0, nb * 1024, 0x00020000);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X + kb * 32), (short)0,
                                                                       ((xrows - 1) * ldx + K - kb * 32) * 2, 0x00020000);
   if constexpr (F32) Yv = reinterpret_cast<float*>(Yv) + blockIdx.y * ysplit;
-  for (int r0 = 0; r0 < count; r0 += ROWS) {
-    const int M = min(ROWS, count - r0);
-    const size_t yo = (size_t)(first + r0) * ldy;
-    void* y = F32 ? (void*)(reinterpret_cast<float*>(Yv) + yo) : (void*)(reinterpret_cast<uint16_t*>(Yv) + yo);
-    const int* rows = gather != nullptr && e >= 0 ? gather + first + r0 : nullptr;
-    const int n0 = blockIdx.x * TW * 16;
-    if (M <= 16) group_rows<1, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
-    else if (M <= 32) group_rows<2, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
-    else if (M <= 48) group_rows<3, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
-    else group_rows<4, EPI, F32>(smem, wr, xr, rows, x0 + r0, ldx, nb, M, y, ldy, n0, epi_arg);
-    __syncthreads();  // the next block's rows overwrite what this one reads
-  }
+  const size_t yo = (size_t)first * ldy;
+  void* y = F32 ? (void*)(reinterpret_cast<float*>(Yv) + yo) : (void*)(reinterpret_cast<uint16_t*>(Yv) + yo);
+  const int* rows = gather != nullptr && e >= 0 ? gather + first : nullptr;
+  const int n0 = blockIdx.x * TW * 16;
+  if (M <= 16) group_rows<1, EPI, F32>(smem, wr, xr, rows, x0, ldx, nb, M, y, ldy, n0, epi_arg);
+  else if (M <= 32) group_rows<2, EPI, F32>(smem, wr, xr, rows, x0, ldx, nb, M, y, ldy, n0, epi_arg);
+  else if (M <= 48) group_rows<3, EPI, F32>(smem, wr, xr, rows, x0, ldx, nb, M, y, ldy, n0, epi_arg);
+  else group_rows<4, EPI, F32>(smem, wr, xr, rows, x0, ldx, nb, M, y, ldy, n0, epi_arg);
 }
 
 }  // namespace
@@ -217,9 +243,11 @@ int launch_gemm_group(const uint16_t* X, int ldx, int xrows, const uint16_t* W, 
   if (epi != EPI_NONE && (out_f32 || (epi != EPI_SILU && epi != EPI_CLAMP_GLU))) return -1;
   const long kbl = K / 32;
   const Shared sh{Wsh, nsh, max_rows, (max_rows + ROWS - 1) / ROWS, slot0, sh_cols ? kbl : N / 16 * kbl, sh_cols ? nsh * kbl : kbl};
-  const dim3 grid(N / 128, S, E + nsh * sh.blocks);
+  const int more = max_rows > ROWS ? slot0 / ROWS : 0;  // (each has 64 rows of its expert before it)
+  if (E + (int64_t)nsh * sh.blocks + more > 65535) return -1;
+  const dim3 grid(N / 128, S, E + nsh * sh.blocks + more);
   auto go = [&](auto kern) {
-    kern<<<grid, 64 * TW, 2 * HALF, st>>>(X, ldx, xrows, W, Y, ldy, off, gather, N, K, S > 1 ? ysplit : 0L, epi_arg, sh);
+    kern<<<grid, 64 * TW, 2 * HALF, st>>>(X, ldx, xrows, W, Y, ldy, off, gather, E, N, K, S > 1 ? ysplit : 0L, epi_arg, sh);
   };
   if (epi == EPI_SILU) go(gemm_group_kernel<EPI_SILU, false>);
   else if (epi == EPI_CLAMP_GLU) go(gemm_group_kernel<EPI_CLAMP_GLU, false>);
