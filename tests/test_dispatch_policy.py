@@ -61,6 +61,8 @@ def test_tuner_offers_two_phase_ping_pong(monkeypatch):
   # short row tiles: the two-phase 192-row tile is offered and preferred like the 256-row one
   assert ("big", 1922256, 1) in L.GemmPolicy._big_cands(384, 8192, 8192)
   assert L._tie_break({("big", 1920256, 2): 0.50, ("big", 1922256, 2): 0.51}) == ("big", 1922256, 2)
+  t = {("big", 128, 4): 55.0, ("big", 2256, 6): 59.6}  # across K splits half of that between 512 and the tall rows
+  assert [L._tie_break(t, M)[1] for M in (512, 513, 911, L.W4_PREF_M - 1)] == [2256, 128, 128, 128]
   monkeypatch.setattr(L, "TIE_X", 0.0)
   assert L._tie_break({("big", 128, 2): 0.843, ("big", 2256, 4): 0.85}) == ("big", 128, 2)
   monkeypatch.setattr(L, "PP2", False)

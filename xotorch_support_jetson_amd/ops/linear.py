@@ -551,7 +551,9 @@ TIE = float(os.environ.get("XOT_GEMM_TIE", "0.05"))
 # ... and across K splits, the two-phase tile within TIE_X of the fastest: the isolated timing runs below the power
 # cap, where a sparser MFMA schedule gains most from the higher clock.  Llama-3-70B o-proj at 512 rows: timed
 # 256 x 128 S 2 84.3 us vs two-phase S 4 92.7 us, but in the step the two-phase pick is 0.5 ms faster (78.30 vs
-# 78.82 / 78.86 ms, profiles/r4/tuner/oproj/)
+# 78.82 / 78.86 ms, profiles/r4/tuner/oproj/).  From 513 rows to the tall ones half of it: picks beyond lose there (1B prompts, the
+# down product of 911 rows 256 x 128 S 4 55.0 us, two-phase S 6 59.6; the prompt 2633 us with the first, 2763 with the second; of 600
+# rows 2412 and 2467, of 900 2971 and 3088; 512 rows of Llama-3-8B 2689 and 2699)
 TIE_X = float(os.environ.get("XOT_GEMM_TIE_X", "0.10"))
 TUNE_LOG = os.environ.get("XOT_GEMM_TUNE_LOG", "0") == "1"  # print every shuffled-weight tuning's timings
 _BIG_PREF = {2256: 0, 4256: 1, 1256: 2, 256: 3, 224: 4, 128: 5}
@@ -565,9 +567,10 @@ def _tie_break(times: Dict, M: int = 0) -> Tuple:
     return best
   pref = _BIG_PREF_TALL if M >= W4_PREF_M else _BIG_PREF
   top = min(pref, key=pref.get)
+  wide = TIE_X / 2 if 512 < M < W4_PREF_M else TIE_X
   close = [c for c, t in times.items()
            if c[0] == "big" and code(c) in pref and ((c[2] == best[2] and t <= times[best] * (1 + TIE))
-                                                     or (code(c) == top and t <= times[best] * (1 + TIE_X)))]
+                                                     or (code(c) == top and t <= times[best] * (1 + wide)))]
   return min(close, key=lambda c: (pref[code(c)], times[c]))
 
 
