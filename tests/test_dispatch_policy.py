@@ -144,6 +144,43 @@ def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
   assert splits(L.GemmPolicy(), 2048, 4096, 28672) == 1
 
 
+def test_qkv_projection_is_timed_with_what_follows_it(monkeypatch):
+  """linear_rope_kv's choice: the rotation and the KV write behind a whole product, one launch behind slabs, are part of the time, so
+  a whole product that is the faster one by itself does not win."""
+  M, H, Hkv, Dh, D = 300, 4, 2, 64, 512
+  N, ran = (H + 2 * Hkv) * Dh, []
+  x, w = (torch.empty(*s, dtype=torch.bfloat16, device="meta") for s in ((M, D), (N, D)))
+  kc, vc = torch.empty(8, Hkv, 64, Dh, dtype=torch.bfloat16, device="meta"), torch.empty(8, Hkv, Dh, 64, dtype=torch.bfloat16, device="meta")
+  took = {"whole": 10.0, "slabs": 10.1, "write": 9.0, "rotate": 9.0 - 5.0}
+  clock = [0.0]
+
+  def step(name, got=None):
+    return lambda *a, **k: (ran.append(name), clock.__setitem__(0, clock[0] + took[name]), got)[2]
+
+  def timed(fn):
+    clock[0] = 0.0
+    fn()
+    return clock[0]
+
+  class Lib:
+    splitk_rope_kv_write = staticmethod(step("rotate"))
+  pol = L.GemmPolicy()
+  pol._path_resolved = True
+  for name, value in (("_no_tuning", lambda self: False), ("_time", staticmethod(timed)),
+                      ("_big_cands", staticmethod(lambda *a: [("big", 128, 1), ("big", 128, 2)])), ("_stream_cands", staticmethod(lambda *a: []))):
+    monkeypatch.setattr(L.GemmPolicy, name, value)
+  monkeypatch.setattr(L, "policy", pol)
+  monkeypatch.setattr(L.scratch, "splitk", lambda dev, n, slot=0: torch.empty(n, device="meta"))
+  monkeypatch.setattr(L, "_shuffled_call", step("whole"))
+  monkeypatch.setattr(L, "_slab_call", step("slabs"))
+  monkeypatch.setattr(L.K, "rope_kv_write", step("write"))
+  monkeypatch.setattr(L, "require", lambda: Lib)
+  monkeypatch.setattr(L, "layout_of", lambda w: "stream")
+  monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+  L.linear_rope_kv(x, w, None, None, None, None, kc, vc, H, Hkv)
+  assert list(pol.table.values()) == [("big", 128, 2)] and ran[-2:] == ["slabs", "rotate"] and ran.count("whole") == ran.count("write") == 1
+
+
 def test_untuned_choice_without_stream_candidates(monkeypatch):
   """The GELU pair epilogue is built for the tall tiles alone: a choice without a timing pass takes one of them at any row count."""
   monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: True)

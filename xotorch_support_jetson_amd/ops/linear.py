@@ -447,11 +447,12 @@ class GemmPolicy:
     top = sorted(busiest, key=lambda nt: (busiest[nt], -nt))[:3]
     return [("wave", nt, 1) for nt in top if busiest[nt] * 256 <= 1.4 * tiles]
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", slabs: bool = False) -> Tuple:
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", slabs: bool = False, run=None) -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
     reduce, timed with them, stands for the launch that does it there).  slabs: the caller's consumer reads split-K slabs
-    itself, so a split is timed without their reduce (2048 x 5632 at 6 rows: 9.1 us whole, 6.4 in 11 slabs, 10.2 with the reduce)."""
+    itself, so a split is timed without their reduce (2048 x 5632 at 6 rows: 9.1 us whole, 6.4 in 11 slabs, 10.2 with the reduce).
+    run(cfg): what the caller does with a choice, where launches of its own that depend on it follow; timed in the GEMM's place."""
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WIDE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
@@ -506,7 +507,7 @@ class GemmPolicy:
     for cfg in cands:
       try:
         call = _slab_call if slabs and cfg[2] > 1 else _shuffled_call
-        times[cfg] = self._time(lambda: call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
+        times[cfg] = self._time(lambda: run(cfg) if run else call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
       except RuntimeError:
         pass
     got = _tie_break(times, 0 if kept and M <= 128 else M) if times else cands[0]
@@ -902,22 +903,23 @@ def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, 
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
-    cfg = policy.shuffled_cfg(x, w, bias, None, "none", x.dtype, wave=wave)
-    if cfg[0] == "wave":
-      q, kw = rope(M)
-      require().gemm_wave(x, w, None, bias, None, K.EPI["none"], cfg[1], **kw)
-      return q
-    if cfg[0] in ("stream", "big") and cfg[2] > 1:
-      S = cfg[2]
-      ws = scratch.splitk(x.device, S * M * N)
-      y = torch.empty(M, N, dtype=x.dtype, device=x.device)  # shape carrier only: the slabs are not reduced
-      C = require()
-      if cfg[0] == "stream":
-        C.gemm_stream(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, True, False)
-      else:
-        C.gemm_big(x, w, y, None, None, ws, K.EPI["none"], cfg[1], S, False)
+
+    def run(cfg):
+      if cfg[0] == "wave":
+        q, kw = rope(M)
+        require().gemm_wave(x, w, None, bias, None, K.EPI["none"], cfg[1], **kw)
+        return q
+      y = torch.empty(M, N, dtype=x.dtype, device=x.device)  # (split over K a shape carrier only: the slabs are not reduced)
+      if cfg[2] == 1:
+        qkv = linear(x, w, bias=bias, out=y) if M <= WIDE_MAX_M else _shuffled_call(x, w, bias, None, "none", y, cfg)
+        return K.rope_kv_write(qkv, pos, cos_sin, slots, k_cache, v_cache, H, Hkv)
+      ws = _slab_call(x, w, None, None, "none", y, cfg)
       q = torch.empty(M, H, Dh, dtype=x.dtype, device=x.device)
-      C.splitk_rope_kv_write(ws, S, bias, pos, cos_sin, slots, q, k_cache, v_cache, int(H), int(Hkv))
+      require().splitk_rope_kv_write(ws, cfg[2], bias, pos, cos_sin, slots, q, k_cache, v_cache, int(H), int(Hkv))
       return q
+    # (more than 64 rows: timed as a whole, for behind one product stand a rotation and a tiled V write, behind slabs one launch.  512 rows
+    # of Llama-3.2-1B, 3072 x 2048: products of S 1 and S 2 take 27.4 and 27.6 us with the latter's reduce, the whole 42.4 and 35.2;
+    # which of them a process drew decided between 2.6 and 2.4 ms for the step)
+    return run(policy.shuffled_cfg(x, w, bias, None, "none", x.dtype, wave=wave, run=run if M > WIDE_MAX_M else None))
   qkv = linear(x, w, bias=bias)
   return K.rope_kv_write(qkv, pos, cos_sin, slots, k_cache, v_cache, H, Hkv)
