@@ -1,5 +1,5 @@
-"""The two-phase ping-pong schedule of csrc/gemm_big.hip (tile codes 2256 / 2192 / 2128): its order of LDS reads and refills, on a
-model of the workgroup's barriers, and its products at few k stages."""
+"""The ping-pong schedules of csrc/gemm_big.hip, two-phase (tile codes 2256 / 2192 / 2128) and four-phase (1256): their order of LDS reads
+and refills, on a model of the workgroup's barriers, and the former's products at few k stages."""
 import pytest
 import torch
 
@@ -26,6 +26,14 @@ def two_phase(t, T):
   if t + 2 < T:
     yield from (("issue", "A0", t + 2), ("issue", "B", t + 2))
   yield from (("landed", "A0", t + 1), ("landed", "B", t + 1), "bar", "lgkm", "bar")
+
+
+def four_phase(t, T):
+  """A stage of the four-phase schedule (B's halves apart): everything is refilled in the last phase."""
+  yield from (("read", "A0"), ("read", "B"), "bar", "lgkm", "bar", ("read", "B"), "bar", "lgkm", "bar", ("read", "A1"), "bar", "lgkm", "bar")
+  if t + 2 < T:
+    yield from (("issue", "A0", t + 2), ("issue", "B", t + 2), ("issue", "A1", t + 2))
+  yield from (("landed", "A0", t + 1), ("landed", "B", t + 1), ("landed", "A1", t + 1), "bar", "bar")
 
 
 def accesses(stage, T, half, wave):
@@ -71,7 +79,7 @@ def unordered(stage, T):
 
 def test_every_refill_is_a_barrier_away_from_its_readers():
   for T in range(1, 7):
-    assert not unordered(two_phase, T), T
+    assert not unordered(two_phase, T) and not unordered(four_phase, T), T
   found = {(r[5][1], r[0] // 2 == w[0] // 2) for r, w in unordered(former, 5)}
   assert found == {("A1", True), ("B", False)}  # a half's own second rows; the other half's reads of W
 

@@ -67,7 +67,7 @@ def test_exact(gpu, code, M, N, Kd, S):
       torch.testing.assert_close(a.cpu().double(), want, rtol=2 ** -7, atol=1e-6)
 
 
-def test_routed_models_keep_their_sums(monkeypatch):
+def test_routed_models_keep_their_candidates(monkeypatch):
   """Attention weights of models with routed experts: the candidates of 17 to 256 rows are those without the tiles above, under keys
   of their own."""
   seen = {}

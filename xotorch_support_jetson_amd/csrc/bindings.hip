@@ -670,8 +670,8 @@ void gemm_moe(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const at:
                                   (long)(slots * y.size(1)), (int)big_bm, (float)epi_arg, cur_stream());
   } else {
     // many small experts, or more tokens than the streaming kernel's 64-row tile: gemm_group, which works through the rows an
-    // expert has.  gate/up + down, us, gemm_stream / gemm_group: 64 experts of 1408 x 2048 at 4 tokens 41 + 31 / 40 + 26, 37
-    // 133 + 59 / 123 + 58, 130 213 + 117 / 130 + 66; 8 of 14336 x 4096 at 64 tokens 311 + 143 / 316 + 148, at 90 365 + 156 / 318 + 151
+    // expert has.  gate/up + down, us, gemm_stream / gemm_group: 64 experts of 1408 x 2048 at 4 tokens 41 + 31 / 34 + 23, 37
+    // 133 + 59 / 124 + 56, 130 213 + 117 / 128 + 62; 8 of 14336 x 4096 at 64 tokens 311 + 143 / 313 + 143, at 90 365 + 156 / 311 + 149
     rc = -1;
     if (wshuf && (E > 16 || max_rows > 64 || nsh > 0))
       rc = xot::launch_gemm_group(bf(x), (int)x.stride(0), (int)x.size(0), bf(w), y.data_ptr(), (int)y.stride(0), f32, (int)epi,

@@ -32,8 +32,8 @@ struct Stage {
   s16x8 w[U];
 };
 
-// One block of M <= 16 MT rows (its registers: one and two row tiles fit the 128 of four waves a SIMD, three spill a dozen, four a
-// hundred, 116 to 140 bytes a lane).  wr: the wave's tile and K slice; xr: X from the slice's first column on, to
+// One block of M <= 16 MT rows.  (Of the 128 registers that four waves a SIMD leave, one and two row tiles take 104 to 125; three
+// spill 8 to 16, four 73 to 112, up to 116 bytes a lane.)  wr: the wave's tile and K slice; xr: X from the slice's first column on, to
 // the end of its last row; rows: gather entries of the block's slots, or null with the slots' rows from row0 on.
 template <int MT, int EPI, bool F32>
 __device__ __forceinline__ void group_rows(char* smem, __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t xr, const int* rows, int row0,

@@ -57,10 +57,11 @@ def moe_tiles(T: int, k: int, E: int) -> Tuple[int, int, int]:
   gemm_big tiles, or (0, 0, 0): the weight-streaming kernels (csrc/gemm_group.hip, gemm.hip), which are bound by the expert weights
   as long as few rows meet them.  Tile code = row tile, + 1000 with a deeper LDS pipeline, + 2000 on the two-phase ping-pong
   schedule.  gate/up + down, us, at rows = T k / E; all of them sum in the same order.  Many small experts (64 of 1408 x 2048):
-  24 rows 133 + 71 streamed, 136 + 72 (2128), 182 + 85 (2256); 48 rows 150 + 81, 139 + 76, 170 + 86; 94 rows 296 + 155, 152 + 88,
-  186 + 92; 192 rows 292 + 171 (2128), 209 + 118 (2256).  Few large ones (8 of 14336 x 4096): 16 rows (up to 64 tokens) 311 + 143
-  streamed, 22 rows 365 + 156 streamed, 330 + 142 (1128); 64 rows 343 + 148 (1128), 419 + 184 (2256), 375 + 157 (2192); 128 rows
-  485 + 248, 448 + 190, 404 + 172."""
+  24 rows 131 + 68 streamed, 140 + 71 (2128), 173 + 82 (2256); 32 rows 131 + 68, 132 + 72, 169 + 79, rows in a Zipf spread 162 +
+  86, 157 + 90; 48 rows 136 + 76, 143 + 76, 173 + 88, Zipf 184 + 97, 165 + 95; 94 rows 263 + 152, 151 + 89, 195 + 92; 192 rows 295 +
+  172 (2128), 208 + 121 (2256).  Few large ones (8 of 14336 x 4096): 16 rows (up to 64 tokens) 313 + 143 streamed, 340 + 142
+  (1128); 22 rows 311 + 149, 337 + 142; 64 rows 343 + 148 (1128), 419 + 184 (2256), 375 + 157 (2192); 128 rows 485 + 248, 448 + 190,
+  404 + 172."""
   rows = T * k / E
   if rows < MOE_TILE_ROWS[1 if E > 16 else 2 if T <= 64 else 0]:
     return 0, 0, 0

@@ -96,9 +96,10 @@ def layout_of(w: torch.Tensor) -> str:
 
 
 def keep_order(w: Optional[torch.Tensor]) -> None:
-  """Products of w at 17 to 256 rows choose among the kernels they always had, so their K splits, and with them the order of their
-  sums, stay: the attention of models with routed experts.  A token whose experts are almost tied turns on the last bits, and its
-  whole row with it (64 sequences of Mixtral: rel 0.021, single logits 0.7 of their size, either way round)."""
+  """Products of w at 17 to 256 rows choose among the stream GEMM and gemm_big's older tiles alone: the attention of models with routed
+  experts.  A token whose experts are almost tied turns on the last bits, and its whole row with it (64 sequences of Mixtral: rel
+  0.021, single logits 0.7 of their size, either way round, nearer to float64 by chance), so kernels with another order of
+  K stay out.  It is the set that is kept: which of it is taken, and its K split, is what the timing says, process by process."""
   if isinstance(w, torch.Tensor):
     w.xot_keep_order = True
 
