@@ -331,8 +331,8 @@ __device__ __forceinline__ void decode_wave_unit(
         st[t][r] = v;
         mx = fmaxf(mx, v);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = xor_max<16>(mx);
+    mx = xor_max<32>(mx);
     const float mn = fmaxf(m, mx);
     const float alpha = exp2f(m - mn);
     m = mn;
@@ -393,8 +393,8 @@ __device__ __forceinline__ void decode_wave_unit(
   }
 
   // lane (g, c): head c, d rows 16dt + 4g + r
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = xor_sum<16>(l);
+  l = xor_sum<32>(l);
   const int h = kvh * G + c;
   if constexpr (NW > 1) {
     constexpr int LD = DH + 4;
@@ -890,8 +890,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2_kernel(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[blk][j][r]);
-      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      mt = xor_max<16>(mt);
+      mt = xor_max<32>(mt);
       const float mn = fmaxf(m[blk], mt * scale_log2);
       alpha[blk] = __builtin_amdgcn_exp2f(m[blk] - mn);
       m[blk] = mn;
@@ -974,8 +974,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2_kernel(
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
     float L = l[blk];
-    L += __shfl_xor(L, 16, 64);
-    L += __shfl_xor(L, 32, 64);
+    L = xor_sum<16>(L);
+    L = xor_sum<32>(L);
     const int row = row0 + 32 * wave + 16 * blk + c;
     if (row < nrows) {
       const int ti = row / G, hi = row % G;

@@ -369,8 +369,8 @@ __global__ __launch_bounds__(512, 1) void attn_train_fwd_v2_kernel(const uint16_
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[blk][j][r]);
-      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      mt = xor_max<16>(mt);
+      mt = xor_max<32>(mt);
       const float mn = fmaxf(m[blk], mt * sl);
       alpha[blk] = __builtin_amdgcn_exp2f(m[blk] - mn);
       m[blk] = mn;
@@ -448,8 +448,8 @@ __global__ __launch_bounds__(512, 1) void attn_train_fwd_v2_kernel(const uint16_
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
     float ls = l[blk];
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = xor_sum<16>(ls);
+    ls = xor_sum<32>(ls);
     const int row = row0 + 32 * wave + 16 * blk + c;
     if (row < nrows) {
       const int ti = row / G, h = kvh * G + row % G;
@@ -717,8 +717,8 @@ __global__ __launch_bounds__(256) void attn_train_dq_v2_kernel(const uint16_t* _
       for (int e = 0; e < 8; ++e) dsum += bf2f(df[s][e]) * bf2f(ov[e]);
     }
   }
-  dsum += __shfl_xor(dsum, 16, 64);  // delta of query c, in every lane group
-  dsum += __shfl_xor(dsum, 32, 64);
+  dsum = xor_sum<16>(dsum);  // delta of query c, in every lane group
+  dsum = xor_sum<32>(dsum);
   if (g == 0 && qi < L) delta[((long)b * H + h) * L + qi] = dsum;
   const float lse = lse2[((long)b * H + h) * L + min(qi, L - 1)];
   f32x4 dqT[NDT];  // [dim 16 dt + 4 g + r][query c]

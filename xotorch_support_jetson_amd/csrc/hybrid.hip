@@ -646,8 +646,8 @@ __global__ __launch_bounds__(256) void attn_window_pool_mfma_k(
             s[kt][qt][r] = t;
             mx = fmaxf(mx, t);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = xor_max<16>(mx);
+        mx = xor_max<32>(mx);
         const float mn = fmaxf(m[qt], mx);
         const float ms = mn == -INFINITY ? 0.0f : mn;  // (nothing seen yet: every weight below is exp2(-inf) = 0)
         const float corr = __builtin_amdgcn_exp2f(m[qt] - ms);
@@ -749,8 +749,8 @@ __global__ __launch_bounds__(256) void attn_window_pool_mfma_k(
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     float ls = lsum[qt];
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = xor_sum<16>(ls);
+    ls = xor_sum<32>(ls);
     if (qt * 16 + c >= nq) continue;
     const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
     OT* op = out + (int64_t)(t0 + q0 + qt * 16 + c) * ldo + h * dv + 4 * g4;

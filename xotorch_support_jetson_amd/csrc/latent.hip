@@ -474,8 +474,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_k(
         mx = fmaxf(mx, S[sub][r]);
       }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = xor_max<16>(mx);
+    mx = xor_max<32>(mx);
     const float mn = fmaxf(m, mx);
     const float corr = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
     m = mn;
@@ -512,8 +512,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_k(
     __syncthreads();  // the next page is written, this one's readers are done
   }
   if (DEC && wave != 0) return;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = xor_sum<16>(l);
+  l = xor_sum<32>(l);
   if (!valid) return;
   if (DEC && nsplit > 1) {
     float* pr = part + (((int64_t)tok * H + head) * nsplit + blockIdx.x) * (2 + R);

@@ -152,8 +152,7 @@ __global__ __launch_bounds__(256) void gated_norm_half_k(const float* __restrict
 #pragma unroll
   for (int r = 0; r < TOK; ++r) {
     float ss = in ? (v[r][0] * v[r][0] + v[r][1] * v[r][1]) + (v[r][2] * v[r][2] + v[r][3] * v[r][3]) : 0.0f;
-#pragma unroll
-    for (int m = 16; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    ss = group16_sum(xor_sum<16>(ss));
     const float k = scale / sqrtf(ss / (float)dv + eps);
     if (!in || t0 + r >= T) continue;
     f32x4 y;

@@ -354,8 +354,8 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
       st[r] = key0 + r < nkeys ? st[r] * scale_log2 : -INFINITY;
       mt = fmaxf(mt, st[r]);
     }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = xor_max<16>(mt);
+    mt = xor_max<32>(mt);
     if (g == 0) red[wave * 16 + c] = mt;
     lds_barrier();
     const float mp = fmaxf(fmaxf(red[c], red[16 + c]), fmaxf(red[32 + c], red[48 + c]));
@@ -376,8 +376,8 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) ls += bf2f(pf[kk][e]);
     }
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = xor_sum<16>(ls);
+    ls = xor_sum<32>(ls);
     l = l * alpha + ls;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
@@ -552,8 +552,8 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
         st[j][r] = key < nkeys ? st[j][r] * scale_log2 : -INFINITY;
         mt = fmaxf(mt, st[j][r]);
       }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = xor_max<16>(mt);
+    mt = xor_max<32>(mt);
     const float mn = fmaxf(m, mt);
     const float alpha = exp2f(m - mn);
     m = mn;
@@ -567,8 +567,8 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
         pf[kk][e] = (short)pb;
         ls += bf2f(pb);
       }
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = xor_sum<16>(ls);
+    ls = xor_sum<32>(ls);
     l = l * alpha + ls;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) {

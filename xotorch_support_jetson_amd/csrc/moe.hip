@@ -158,15 +158,7 @@ __global__ __launch_bounds__(256) void moe_topk_ds_kernel(const float* __restric
       for (int j = 0; j < topk_group; ++j) {  // wave argmax over the groups (ties: lower group id)
         float v = (lane < n_group && !(keep >> lane & 1u)) ? gsc : -INFINITY;
         int id = lane;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          const float ov = __shfl_xor(v, o, 64);
-          const int oi = __shfl_xor(id, o, 64);
-          if (ov > v || (ov == v && oi < id)) {
-            v = ov;
-            id = oi;
-          }
-        }
+        wave_argmax(v, id);
         keep |= 1u << id;
       }
     }
@@ -188,15 +180,7 @@ __global__ __launch_bounds__(256) void moe_topk_ds_kernel(const float* __restric
           id = e;
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o, 64);
-        const int oi = __shfl_xor(id, o, 64);
-        if (ov > v || (ov == v && oi < id)) {
-          v = ov;
-          id = oi;
-        }
-      }
+      wave_argmax(v, id);
       // (scores that are not numbers -- rows of a padded batch may hold anything -- leave no winner: take expert j,
       // so that every index written below is an expert)
       if (id >= E) id = j;
@@ -521,9 +505,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint16_t* __re
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    float v = acc[e];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    const float v = wave_sum(acc[e]);
     if ((tid & 63) == 0) red[tid >> 6][e] = v;
   }
   __syncthreads();

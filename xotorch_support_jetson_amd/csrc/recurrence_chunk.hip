@@ -130,10 +130,10 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
             dq += qr * kh[j][r];
             if (DELTA) dk += kr * kh[j][r];
           }
-        dq += __shfl_xor(dq, 16);
-        dq += __shfl_xor(dq, 32);
-        dk += __shfl_xor(dk, 16);
-        dk += __shfl_xor(dk, 32);
+        dq = xor_sum<16>(dq);
+        dq = xor_sum<32>(dq);
+        dk = xor_sum<16>(dk);
+        dk = xor_sum<32>(dk);
         if ((row >> 2) == g) {
           qs[0][0] = (row & 3) == 0 ? dq : qs[0][0], ks[0][0] = (row & 3) == 0 ? dk : ks[0][0];
           qs[0][1] = (row & 3) == 1 ? dq : qs[0][1], ks[0][1] = (row & 3) == 1 ? dk : ks[0][1];

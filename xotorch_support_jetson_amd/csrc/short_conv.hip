@@ -214,9 +214,7 @@ __device__ __forceinline__ void conv_body(const ConvArgs& A, int bx, int by) {
         for (int e = 0; e < VW; ++e) s[i] += ok[i] && in[e] ? y[i][e] * y[i][e] : 0.0f;
       }
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int i = 0; i < NT; ++i) s[i] += __shfl_xor(s[i], o, 64);
+      for (int i = 0; i < NT; ++i) s[i] = wave_sum(s[i]);
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         const float k = kind & CONV_RMS ? 1.0f / sqrtf(s[i] / (float)n + eps)
@@ -385,8 +383,7 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
   }
 #pragma unroll
   for (int i = 0; i < GTOK; ++i) {
-    z[i] += __shfl_xor(z[i], 1, 64);
-    z[i] += __shfl_xor(z[i], 2, 64);
+    z[i] = quad_sum(z[i]);
   }
   if (c >= nc) return;
 #pragma unroll

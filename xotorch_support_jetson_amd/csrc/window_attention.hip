@@ -199,8 +199,8 @@ __global__ __launch_bounds__(512, 1) void window_prefill_k(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[blk][j][r]);
-      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      mt = xor_max<16>(mt);
+      mt = xor_max<32>(mt);
       const float mn = fmaxf(m[blk], mt);
       alpha[blk] = __builtin_amdgcn_exp2f(m[blk] - mn);
       m[blk] = mn;
@@ -276,8 +276,8 @@ __global__ __launch_bounds__(512, 1) void window_prefill_k(
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {  // o[blk][dt][r] = O[row c of the block][dim 16 dt + 4 g + r]
     float L = l[blk];
-    L += __shfl_xor(L, 16, 64);
-    L += __shfl_xor(L, 32, 64);
+    L = xor_sum<16>(L);
+    L = xor_sum<32>(L);
     const int row = row0 + 32 * wave + 16 * blk + c;
     if (row < nrows) {
       OT* op = out + (int64_t)(q0 + row / rep) * ldo + (kvh * rep + row % rep) * DV + 4 * g;
@@ -382,8 +382,8 @@ __global__ __launch_bounds__(64 * WDW, 1) void window_decode_k(
         st[j][r] = seen(key, pos, lo, keep) ? t : -INFINITY;
         mt = fmaxf(mt, st[j][r]);
       }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = xor_max<16>(mt);
+    mt = xor_max<32>(mt);
     const float mn = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
     float ls = 0.f;
@@ -409,8 +409,8 @@ __global__ __launch_bounds__(64 * WDW, 1) void window_decode_k(
       for (int kk = 0; kk < 2; ++kk) o[dt] = mfma16(vf[dt][kk], pf[kk], o[dt]);
     }
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = xor_sum<16>(l);
+  l = xor_sum<32>(l);
   if (c < rep) {
     float* mine = sm + (wave * rep + c) * ms;
     if (g == 0) {
