@@ -43,7 +43,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx_lens,
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int H, int Hkv,
-    int pages_per_part, int nparts, float scale_log2, int num_pages, int* __restrict__ tickets) {
+    int pages_per_part, int nparts, float scale_log2, int num_pages) {
   constexpr int KS = DH / 32;   // MFMA k-steps over the head dim
   constexpr int NDT = DH / 16;  // 16-wide d tiles of the output
   constexpr int PLD = PAGE + 8;
@@ -230,25 +230,53 @@ __global__ __launch_bounds__(DH) void attn_decode_reduce_kernel(const float* __r
 // NT: K / V pages loaded non-temporal (read once per step; algo 3 / 6 / 8; the workgroup form of algo 2 / 3 follows)
 // NW > 1 (PF 2): the NW waves of a workgroup share the unit, wave w takes pages w, w + NW, ..., and they meet in LDS (sm:
 //       [NW][G][DH + 4] partial sums, then [NW][G][2] maxima and sums)
-template <int DH, int PF, bool NT, int NW = 1>
+// AGENT (NW > 1): partial results are read by another workgroup of the same launch: stored past this XCD's L2
+struct DecodeUnit {
+  int b, kvh, first, last;  // pages first .. last of the sequence
+  bool whole;               // all of them: the result goes to out
+  int prow, pstride;        // row of the partial results of the group's first head, rows from head to head
+};
+
+// pairs of floats that workgroups of one launch hand over: relaxed 64-bit accesses at agent scope, past the L2 of an XCD
+__device__ __forceinline__ void agent_store2(float* p, float a, float b) {
+  const uint64_t v = (uint64_t)__float_as_uint(b) << 32 | __float_as_uint(a);
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store4(float* p, const f32x4& v) {
+  agent_store2(p, v[0], v[1]);
+  agent_store2(p + 2, v[2], v[3]);
+}
+__device__ __forceinline__ f32x2_t agent_load2(const float* p) {
+  const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return {__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32))};
+}
+__device__ __forceinline__ f32x4 agent_load4(const float* p) {
+  const f32x2_t a = agent_load2(p), b = agent_load2(p + 2);
+  return {a[0], a[1], b[0], b[1]};
+}
+// four results o / l in bf16 (a row without keys: zeros)
+__device__ __forceinline__ void st_bf16x4(uint16_t* p, const f32x4& o, float l) {
+  s16x4 y;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) y[r] = (short)f2bf(l > 0.f ? o[r] / l : 0.f);
+  *reinterpret_cast<s16x4*>(p) = y;
+}
+
+template <int DH, int PF, bool NT, int NW = 1, bool AGENT = false>
 __device__ __forceinline__ void decode_wave_unit(
-    const int unit, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
-    const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx_lens,
-    uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int B, int H, int Hkv,
-    int pages_per_part, int nparts, float scale_log2, int num_pages, int* __restrict__ tickets, bool vtail,
-    float* sm = nullptr) {
+    const DecodeUnit un, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int32_t* __restrict__ block_tables, int max_blocks, const int ctx,
+    uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int H, int Hkv,
+    float scale_log2, int num_pages, bool vtail, float* sm = nullptr) {
   static_assert(NW == 1 || PF == 2, "waves that share a unit run the single-set pipeline");
   constexpr int KS = DH / 32;   // k-steps of S^T over the head dim
   constexpr int NDT = DH / 16;  // 16-row d tiles of O^T
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
-  const int part = unit % nparts, kvh = (unit / nparts) % Hkv, b = unit / (nparts * Hkv);
+  const int kvh = un.kvh, b = un.b;
   const int G = H / Hkv;
-  const int ctx = min(max(ctx_lens[b], 0), max_blocks * PAGE);
-  const int npages = (ctx + PAGE - 1) / PAGE;
   const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int p_begin = part * pages_per_part + wave;
-  const int p_end = min(npages, part * pages_per_part + pages_per_part);
+  const int p_begin = un.first + wave, p_end = un.last;
 
   // Q^T (B operand): column c = query head kvh*G + c; k-step s, lane group g: d 32s + 8g .. +8
   // (natural MFMA order, so each K load instruction below reads 64 contiguous bytes of 16 rows).
@@ -409,32 +437,36 @@ __device__ __forceinline__ void decode_wave_unit(
       }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < G * DH; e += NW * 64) {
+    for (int e = 4 * threadIdx.x; e < G * DH; e += 4 * NW * 64) {
       const int hq = e / DH, d = e - hq * DH;
       float M = NEG_BIG;
 #pragma unroll
       for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[(w * G + hq) * 2]);
-      float L = 0.f, O = 0.f;
+      float L = 0.f;
+      f32x4 O = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < NW; ++w) {  // (a wave without pages: m = NEG_BIG, l = 0, o = 0)
         const float f = exp2f(ml[(w * G + hq) * 2] - M);
         L += ml[(w * G + hq) * 2 + 1] * f;
-        O += sm[(w * G + hq) * LD + d] * f;
+        O += *reinterpret_cast<const f32x4*>(sm + (w * G + hq) * LD + d) * f;
       }
-      const size_t row = (size_t)b * H + kvh * G + hq;
-      if (nparts == 1) {
-        out[row * DH + d] = f2bf(L > 0.f ? O / L : 0.f);
+      const size_t pr = (size_t)un.prow + (size_t)hq * un.pstride;
+      if (un.whole) {
+        st_bf16x4(out + ((size_t)b * H + kvh * G + hq) * DH + d, O, L);
+      } else if constexpr (AGENT) {
+        agent_store4(ws_o + pr * DH + d, O);
+        if (d == 0) agent_store2(ws_ml + pr * 2, M, L);
       } else {
-        ws_o[(row * nparts + part) * DH + d] = O;
+        *reinterpret_cast<f32x4*>(ws_o + pr * DH + d) = O;
         if (d == 0) {
-          ws_ml[(row * nparts + part) * 2] = M;
-          ws_ml[(row * nparts + part) * 2 + 1] = L;
+          ws_ml[pr * 2] = M;
+          ws_ml[pr * 2 + 1] = L;
         }
       }
     }
     return;
   }
-  if (nparts == 1) {
+  if (un.whole) {
     if (c >= G) return;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint16_t* op = out + ((size_t)b * H + h) * DH + 4 * g;
@@ -448,7 +480,7 @@ __device__ __forceinline__ void decode_wave_unit(
     return;
   }
   if (c < G) {
-    const size_t idx = ((size_t)b * H + h) * nparts + part;
+    const size_t idx = (size_t)un.prow + (size_t)c * un.pstride;
     float* wo = ws_o + idx * DH + 4 * g;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4*>(wo + 16 * dt) = o[dt];
@@ -460,6 +492,13 @@ __device__ __forceinline__ void decode_wave_unit(
 }
 
 
+// unit -> (sequence, KV head, partition of pages_per_part pages), partitions fastest
+__device__ __forceinline__ DecodeUnit fixed_unit(int unit, int nparts, int pages_per_part, int H, int Hkv, int ctx) {
+  const int part = unit % nparts, kvh = (unit / nparts) % Hkv, b = unit / (nparts * Hkv);
+  const int npages = (ctx + PAGE - 1) / PAGE, first = part * pages_per_part;
+  return {b, kvh, first, min(npages, first + pages_per_part), nparts == 1, (b * H + kvh * (H / Hkv)) * nparts + part, nparts};
+}
+
 // Wave-uniform unit id in an SGPR: page indices and block-table reads stay scalar (s_load, counted by lgkmcnt),
 // so they never force a vmcnt(0) drain of the K / V prefetch.  (A strided persistent grid on a subset of the CUs,
 // to leave whole CUs to concurrent GEMMs, was measured and dropped: profiles/r4/overlap/.)
@@ -468,11 +507,12 @@ __global__ __launch_bounds__(PF == 2 ? 512 : 256, PF == 2 ? 2 : 1) void attn_dec
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ ctx_lens,
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int B, int H, int Hkv,
-    int pages_per_part, int nparts, float scale_log2, int num_pages, int* __restrict__ tickets, int vtail) {
+    int pages_per_part, int nparts, float scale_log2, int num_pages, int vtail) {
   const int unit = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
   if (unit >= B * Hkv * nparts) return;  // whole wave
-  decode_wave_unit<DH, PF, NT>(unit, q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, ws_ml, B, H, Hkv,
-                               pages_per_part, nparts, scale_log2, num_pages, tickets, vtail != 0);
+  const int ctx = min(max(ctx_lens[unit / (nparts * Hkv)], 0), max_blocks * PAGE);
+  decode_wave_unit<DH, PF, NT>(fixed_unit(unit, nparts, pages_per_part, H, Hkv, ctx), q, kc, vc, block_tables, max_blocks, ctx,
+                               out, ws_o, ws_ml, H, Hkv, scale_log2, num_pages, vtail != 0);
 }
 
 // The NW waves of a workgroup share one (sequence, KV head, partition): a short context's pages are in flight together and the
@@ -495,18 +535,185 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_group_kernel(
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int B, int H, int Hkv,
     int pages_per_part, int nparts, float scale_log2, int num_pages) {
   extern __shared__ __attribute__((aligned(16))) float gsm[];
-  decode_wave_unit<DH, 2, NT, NW>(blockIdx.x, q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, ws_ml, B, H, Hkv,
-                                  pages_per_part, nparts, scale_log2, num_pages, nullptr, true, gsm);
+  const int ctx = min(max(ctx_lens[blockIdx.x / (nparts * Hkv)], 0), max_blocks * PAGE);
+  decode_wave_unit<DH, 2, NT, NW>(fixed_unit(blockIdx.x, nparts, pages_per_part, H, Hkv, ctx), q, kc, vc, block_tables, max_blocks,
+                                  ctx, out, ws_o, ws_ml, H, Hkv, scale_log2, num_pages, true, gsm);
+}
+
+// The same over units that a plan lists (decode_plan_kernel): partitions cut by the contexts the step has, whatever the width of the
+// block tables, so that no CU (about 50 GB/s) has much more than its share of the pages.  The last workgroup of a (sequence, KV head)
+// to arrive merges its partitions (tickets [B][Hkv], zero between launches), in their order whoever it is.  The partial results pass
+// the XCD's L2 both ways (relaxed agent-scope accesses, waited for before the ticket): a release fence would write that L2 back, one
+// workgroup after another, and cost more than the merge launch (24 sequences of 74 .. 1407 tokens 50 us, 16 without).  The merge
+// is about 3 us behind a unit's pages, a launch for it 4.7.  Times beside ops.kernels.plan_pays.
+template <int DH, bool NT>
+__global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+    const int32_t* __restrict__ block_tables, int max_blocks, const DecodePart* __restrict__ plan,
+    uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int H, int Hkv,
+    float scale_log2, int num_pages, int* __restrict__ tickets) {
+  extern __shared__ __attribute__((aligned(16))) float gsm[];
+  __shared__ int last_sm;
+  const int part = blockIdx.x / Hkv, kvh = blockIdx.x - part * Hkv, G = H / Hkv;
+  const DecodePart d = plan[part];
+  if (d.parts == 0) return;  // uniform over the workgroup: a place no part takes
+  decode_wave_unit<DH, 2, NT, 4, true>({d.b, kvh, d.first, d.last, d.parts == 1, (int)blockIdx.x * G, 1}, q, kc, vc, block_tables,
+                                       max_blocks, d.ctx, out, ws_o, ws_ml, H, Hkv, scale_log2, num_pages, true, gsm);
+  if (d.parts == 1) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial results have left (agent stores), no L2 write-back needed
+  __syncthreads();
+  int* t = tickets + d.b * Hkv + kvh;
+  if (threadIdx.x == 0) last_sm = __hip_atomic_fetch_add(t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == d.parts - 1;
+  __syncthreads();
+  if (!last_sm) return;
+  if (threadIdx.x == 0) __hip_atomic_store(t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const size_t row0 = ((size_t)d.place * Hkv + kvh) * G, step = (size_t)Hkv * G;
+  for (int e = 4 * threadIdx.x; e < G * DH; e += 1024) {
+    const int hq = e / DH, dim = e - hq * DH;
+    float M = NEG_BIG, L = 0.f;
+    f32x4 O = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < d.parts; s0 += 8) {
+      f32x2_t ml[8];
+      f32x4 o[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const size_t r = row0 + hq + min(s0 + i, d.parts - 1) * step;
+        ml[i] = agent_load2(ws_ml + r * 2);
+        o[i] = agent_load4(ws_o + r * DH + dim);
+      }
+      float mx = M;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, ml[i][0]);
+      const float f0 = exp2f(M - mx);
+      L *= f0;
+      O *= f0;
+      M = mx;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (s0 + i < d.parts) {
+          const float f = exp2f(ml[i][0] - M);
+          L += ml[i][1] * f;
+          O += o[i] * f;
+        }
+    }
+    st_bf16x4(out + ((size_t)d.b * H + kvh * G + hq) * DH + dim, O, L);
+  }
+}
+
+// The units of a decode step: every sequence's pages in equal parts of at most ppp pages; an empty sequence is one part (which writes
+// zeros).  ppp is the candidate with the least estimated time, in pages a CU reads one behind the other: its longest part, and an
+// average one beside it where there are more units than CUs (two workgroups a CU run at once), or, past two a CU, its share of all
+// pages and a part that starts last.  One workgroup, a wave per candidate.
+__global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restrict__ ctx_lens, int B, unsigned Hkv, int max_blocks,
+                                                          int places, DecodePart* __restrict__ plan) {
+  __shared__ int red[8], ctx_sm[512], first_sm[513];
+  __shared__ float est_sm[8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int mine = tid < B ? min(max(ctx_lens[tid], 0), max_blocks * PAGE) : 0;
+  auto ctx_of = [&](int b) { return b < 512 ? ctx_sm[b] : min(max(ctx_lens[b], 0), max_blocks * PAGE); };
+  auto pages_of = [](int ctx) { return (unsigned)(ctx + PAGE - 1) / PAGE; };
+  ctx_sm[tid] = mine;
+  __syncthreads();
+  unsigned total = 0, most = 0;  // (each wave by itself)
+  for (int b = lane; b < B; b += 64) {
+    const unsigned n = pages_of(ctx_of(b));
+    total += n;
+    most = max(most, n);
+  }
+  total = wave_sum_u(total);
+  most = wave_max_u(most);
+  const unsigned all = total * Hkv;
+  // candidate 0: the longest sequence whole; c: 64 (c + 1) units, DECODE_UNITS at most
+  auto ppp_of = [&](int c) {
+    const unsigned u = 64 * (c + 1);
+    return max((unsigned)DECODE_MIN_PAGES, c == 0 ? most : (all + u - 1) / u);
+  };
+  {
+    const unsigned ppp = ppp_of(wave);
+    unsigned units = 0, big = 0;
+    for (int b = lane; b < B; b += 64) {
+      const unsigned pages = pages_of(ctx_of(b)), parts = max(1u, (pages + ppp - 1) / ppp);
+      units += parts;
+      big = max(big, (pages + parts - 1) / parts);
+    }
+    units = wave_sum_u(units);
+    big = wave_max_u(big);
+    const float u = (float)units * Hkv, work = (float)all, share = work / 256.f;
+    if (lane == 0) est_sm[wave] = u <= 256.f ? big : u <= 512.f ? fmaxf(big + work / u, share) + 1.f : share + big + 1.f;
+  }
+  __syncthreads();
+  int best = 0;
+#pragma unroll
+  for (int c = 1; c < 8; ++c)
+    if (est_sm[c] < est_sm[best]) best = c;
+  const unsigned ppp = ppp_of(best);
+  int base = 0;
+  for (int b0 = 0; b0 < B; b0 += 512) {
+    const int n = min(512, B - b0), parts = tid < n ? (int)max(1u, (pages_of(ctx_of(b0 + tid)) + ppp - 1) / ppp) : 0;
+    int end = parts;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int v = __shfl_up(end, s, 64);
+      if (lane >= s) end += v;
+    }
+    __syncthreads();
+    if (lane == 63) red[wave] = end;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) end += red[w];
+    if (tid < n) first_sm[tid] = base + end - parts;
+    if (tid == n - 1) first_sm[n] = base + end;
+    __syncthreads();
+    const int stop = first_sm[n];
+    for (int i = base + tid; i < min(stop, places); i += 512) {
+      int lo = 0, hi = n;  // the last of the n sequences whose first place is at most i
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (first_sm[mid] <= i) lo = mid;
+        else hi = mid;
+      }
+      const int first = first_sm[lo], np = first_sm[lo + 1] - first, ctx = ctx_of(b0 + lo);
+      const unsigned pages = pages_of(ctx), q = pages / np, r = pages - q * np, k = i - first;  // (the first r parts: a page more)
+      const int p0 = (int)(k * q + min(k, r));
+      plan[i] = {b0 + lo, p0, p0 + (int)(q + (k < r)), np, first, ctx, 0, 0};
+    }
+    base = stop;
+  }
+  for (int i = base + tid; i < places; i += 512) plan[i] = {0, 0, 0, 0, 0, 0, 0, 0};
+}
+
+int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, DecodePart* plan, hipStream_t s) {
+  if (B <= 0) return 0;
+  decode_plan_kernel<<<1, 512, 0, s>>>(ctx_lens, B, Hkv, max_blocks, decode_split_places(B, Hkv, max_blocks), plan);
+  return 0;
+}
+
+int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables, int max_blocks,
+                             const DecodePart* plan, int places, int* tickets, uint16_t* out, float* ws_o, float* ws_ml, int H,
+                             int Hkv, int Dh, float scale, int num_pages, bool nt, hipStream_t s) {
+  if (places <= 0) return 0;
+  if (H % Hkv != 0 || H / Hkv > 16) return -1;
+  const size_t lds = (size_t)4 * (H / Hkv) * (Dh + 6) * sizeof(float);  // at most 34 KB
+#define XOT_SPLIT(DHV, NTV)                                                                                                \
+  attn_decode_split_kernel<DHV, NTV><<<places * Hkv, 256, lds, s>>>(q, kc, vc, block_tables, max_blocks, plan, out, ws_o, ws_ml, \
+                                                                    H, Hkv, scale * LOG2E, num_pages, tickets)
+  if (Dh == 128) {
+    if (nt) XOT_SPLIT(128, true);
+    else XOT_SPLIT(128, false);
+  } else if (Dh == 64) {
+    if (nt) XOT_SPLIT(64, true);
+    else XOT_SPLIT(64, false);
+  } else {
+    return -1;
+  }
+#undef XOT_SPLIT
+  return 0;
 }
 
 int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                        int max_blocks, const int32_t* ctx_lens, uint16_t* out, float* ws_o, float* ws_ml, int B,
                        int H, int Hkv, int Dh, int pages_per_part, int nparts, float scale, int num_pages, int algo,
                        hipStream_t s, bool merge) {
-  // (an in-kernel merge by the last-arriving partition measured slower than the reduce launch in every
-  // configuration, profiles/bench_attn_small_r1.json, and was removed in round 6.)  merge = false: the
-  // partitions are left in ws_o / ws_ml for the consumer (launch_gemm_stream_merge's prologue at batch 1).
-  int* tickets = nullptr;
+  // merge = false: the partitions are left in ws_o / ws_ml for the consumer (launch_gemm_stream_merge's prologue at batch 1).
   const bool reduce = nparts > 1 && merge;
   if (B <= 0) return 0;
   if (H % Hkv != 0 || H / Hkv > 16) return -1;
@@ -540,7 +747,7 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
     const int wgs = (units + wpg - 1) / wpg;
 #define XOT_WAVE(DHV, PFV, NTV)                                                                                  \
   attn_decode_wave_kernel<DHV, PFV, NTV><<<wgs, 64 * wpg, 0, s>>>(q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, \
-                                                        ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages, tickets, 1)
+                                                        ws_ml, B, H, Hkv, pages_per_part, nparts, sl, num_pages, 1)
     // algo 1: no prefetch; 5 / 6: one register set refilled per half (6: nt loads); 7 / 8: two register sets (8: nt loads)
     if (Dh == 128) {
       if (algo == 5) XOT_WAVE(128, 2, false); else if (algo == 6) XOT_WAVE(128, 2, true);
@@ -558,11 +765,11 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
   }
   if (Dh == 128) {
     attn_decode_kernel<128><<<grid, 256, 0, s>>>(q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, ws_ml,
-                                                 H, Hkv, pages_per_part, nparts, sl, num_pages, tickets);
+                                                 H, Hkv, pages_per_part, nparts, sl, num_pages);
     if (reduce) attn_decode_reduce_kernel<128><<<B * H, 128, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
   } else if (Dh == 64) {
     attn_decode_kernel<64><<<grid, 256, 0, s>>>(q, kc, vc, block_tables, max_blocks, ctx_lens, out, ws_o, ws_ml, H,
-                                                Hkv, pages_per_part, nparts, sl, num_pages, tickets);
+                                                Hkv, pages_per_part, nparts, sl, num_pages);
     if (reduce) attn_decode_reduce_kernel<64><<<B * H, 64, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
   } else {
     return -1;

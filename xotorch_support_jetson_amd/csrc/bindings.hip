@@ -896,6 +896,50 @@ void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tenso
   XCHECK(rc == 0, "attn_decode: unsupported H=", H, " Hkv=", Hkv, " Dh=", Dh);
 }
 
+// the plan of attn_decode_split: int32 [places, 8] (see kernels.h DecodePart), written by one launch
+at::Tensor decode_plan(const at::Tensor& ctx_lens, int64_t B, int64_t Hkv, int64_t max_blocks) {
+  CHECK_DT(ctx_lens, at::kInt);
+  XCHECK(all_contig_gpu(ctx_lens) && B >= 1 && ctx_lens.numel() >= B, "decode_plan: ctx_lens");
+  XCHECK(Hkv >= 1 && max_blocks >= 1 && B <= (1 << 20) && max_blocks <= (1 << 24), "decode_plan: sizes");
+  at::Tensor plan = at::empty({xot::decode_split_places((int)B, (int)Hkv, (int)max_blocks), 8}, ctx_lens.options());
+  XCHECK(reinterpret_cast<uintptr_t>(plan.data_ptr()) % 32 == 0, "decode_plan: alignment");
+  xot::launch_decode_plan(ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hkv, (int)max_blocks,
+                          reinterpret_cast<xot::DecodePart*>(plan.data_ptr<int32_t>()), cur_stream());
+  return plan;
+}
+
+void attn_decode_split(const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache, const at::Tensor& block_tables,
+                       const at::Tensor& plan, at::Tensor& tickets, at::Tensor& out, at::Tensor& ws_o, at::Tensor& ws_ml,
+                       double scale, bool nt) {
+  CHECK_BF16(q);
+  CHECK_BF16(k_cache);
+  CHECK_BF16(v_cache);
+  CHECK_BF16(out);
+  CHECK_DT(block_tables, at::kInt);
+  CHECK_DT(plan, at::kInt);
+  CHECK_DT(tickets, at::kInt);
+  CHECK_DT(ws_o, at::kFloat);
+  CHECK_DT(ws_ml, at::kFloat);
+  XCHECK(all_contig_gpu(q, k_cache, v_cache, block_tables, plan, tickets, out, ws_o, ws_ml),
+         "attn_decode_split: all tensors must be contiguous GPU tensors");
+  XCHECK(q.dim() == 3 && k_cache.dim() == 4 && v_cache.dim() == 4, "attn_decode_split: q [B,H,Dh], caches 4-D");
+  const int64_t B = q.size(0), H = q.size(1), Dh = q.size(2), Hkv = k_cache.size(1), nb = k_cache.size(0);
+  XCHECK(k_cache.size(2) == 64 && k_cache.size(3) == Dh && v_cache.size(2) == Dh && v_cache.size(3) == 64 &&
+             v_cache.size(0) == nb && v_cache.size(1) == Hkv,
+         "attn_decode_split: cache layout K[nb,Hkv,64,Dh] V[nb,Hkv,Dh,64]");
+  XCHECK(block_tables.dim() == 2 && block_tables.size(0) >= B, "attn_decode_split: tables");
+  XCHECK(out.numel() == B * H * Dh, "attn_decode_split: out shape");
+  XCHECK(plan.dim() == 2 && plan.size(1) == 8 && reinterpret_cast<uintptr_t>(plan.data_ptr()) % 32 == 0, "attn_decode_split: plan");
+  const int64_t places = plan.size(0);
+  XCHECK(tickets.numel() >= B * Hkv && ws_o.numel() >= places * H * Dh && ws_ml.numel() >= places * H * 2,
+         "attn_decode_split: workspace small");
+  const int rc = xot::launch_attn_decode_split(
+      bf(q), bf(k_cache), bf(v_cache), block_tables.data_ptr<int32_t>(), (int)block_tables.size(1),
+      reinterpret_cast<const xot::DecodePart*>(plan.data_ptr<int32_t>()), (int)places, tickets.data_ptr<int32_t>(), bf(out),
+      ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), (int)H, (int)Hkv, (int)Dh, (float)scale, (int)nb, nt, cur_stream());
+  XCHECK(rc == 0, "attn_decode_split: unsupported H=", H, " Hkv=", Hkv, " Dh=", Dh);
+}
+
 // the partition merge attn_decode(merge = false) left out: out [B, H, Dh] from ws_o / ws_ml
 void attn_decode_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, const at::Tensor& ctx_lens, at::Tensor& out,
                        int64_t pages_per_part, int64_t nparts) {
@@ -1219,6 +1263,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
         py::arg("nparts"), py::arg("scale"), py::arg("algo") = 2, py::arg("merge") = true);
+  m.def("decode_plan", &decode_plan, py::arg("ctx_lens"), py::arg("B"), py::arg("Hkv"), py::arg("max_blocks"));
+  m.def("attn_decode_split", &attn_decode_split, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
+        py::arg("plan"), py::arg("tickets"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("scale"), py::arg("nt"));
   m.def("attn_decode_merge", &attn_decode_merge, py::arg("ws_o"), py::arg("ws_ml"), py::arg("ctx_lens"), py::arg("out"),
         py::arg("pages_per_part"), py::arg("nparts"));
   m.def("gemm_stream_merge", &gemm_stream_merge, py::arg("w"), py::arg("ws"), py::arg("ntw"), py::arg("splits"),

@@ -108,6 +108,23 @@ __device__ __forceinline__ void wave_argmax(float& v, int& id) {
   take(row_turn<1>(__float_as_uint(v)), row_turn<1>((uint32_t)id));
 }
 
+__device__ __forceinline__ uint32_t wave_sum_u(uint32_t v) {
+  auto add = [](uint32_t a, uint32_t b) { return a + b; };
+  v = lane_xor<16>(lane_xor<32>(v, add), add);
+  v += row_turn<8>(v);
+  v += row_turn<4>(v);
+  v += row_turn<2>(v);
+  return v + row_turn<1>(v);
+}
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
+  auto most = [](uint32_t a, uint32_t b) { return max(a, b); };
+  v = lane_xor<16>(lane_xor<32>(v, most), most);
+  v = max(v, row_turn<8>(v));
+  v = max(v, row_turn<4>(v));
+  v = max(v, row_turn<2>(v));
+  return max(v, row_turn<1>(v));
+}
+
 __device__ __forceinline__ s16x8 ld16(const void* p) { return *reinterpret_cast<const s16x8*>(p); }
 // non-temporal 16-B load (global_load_dwordx4 ... nt): bytes read once per kernel (KV pages in decode)
 __device__ __forceinline__ s16x8 ld16nt(const void* p) {

@@ -157,6 +157,25 @@ int launch_gemm_tiled(const uint16_t* X, int ldx, const uint16_t* W, int ldw, co
                       const uint16_t* R, int ldr, void* Y, int ldy, bool out_f32, int epi, int M, int N, int K,
                       hipStream_t s);
 
+// one unit of a decode step's attention for every KV head: pages first .. last of sequence b, one of its `parts` parts (0: none), the
+// first of which has place `place`
+struct __attribute__((aligned(32))) DecodePart {
+  int b, first, last, parts, place, ctx, pad0, pad1;
+};
+// Parts of a sequence have at least MIN_PAGES pages (a page for each of a unit's four waves), and there are about UNITS of them over
+// all KV heads at most (two workgroups on each of 256 CUs).
+constexpr int DECODE_MIN_PAGES = 4, DECODE_UNITS = 512;
+// places of a plan: sum over the sequences of max(1, ceil(pages / ppp)) < B + total / ppp + 1, and ppp >= total Hkv / UNITS
+inline int decode_split_places(int B, int Hkv, int max_blocks) {
+  const int64_t wide = (int64_t)B * ((max_blocks + DECODE_MIN_PAGES - 1) / DECODE_MIN_PAGES);
+  const int64_t n = (int64_t)B + DECODE_UNITS / Hkv;
+  return (int)(n < wide ? n : wide);
+}
+int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, DecodePart* plan, hipStream_t s);
+// ws_o [places][H][Dh], ws_ml [places][H][2], tickets [B][Hkv] (zero before and after)
+int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables, int max_blocks,
+                             const DecodePart* plan, int places, int* tickets, uint16_t* out, float* ws_o, float* ws_ml, int H,
+                             int Hkv, int Dh, float scale, int num_pages, bool nt, hipStream_t s);
 int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                        int max_blocks, const int32_t* ctx_lens, uint16_t* out, float* ws_o, float* ws_ml, int B,
                        int H, int Hkv, int Dh, int pages_per_part, int nparts, float scale, int num_pages, int algo,

@@ -275,11 +275,11 @@ class ShardModel:
     return range(start + o, start + n + o)
 
   # ------------------------------------------------------------------ helpers
-  def _attention(self, q: torch.Tensor, li: int, inp: StepInputs, ws=None, defer_merge: bool = False):
+  def _attention(self, q: torch.Tensor, li: int, inp: StepInputs, ws=None, defer_merge: bool = False, plan=None):
     kc, vc = self.kv.k[li], self.kv.v[li]
     if inp.decode:
       return K.attn_decode(q, kc, vc, inp.block_tables, inp.ctx_lens, self.scale, ws or self.ws,
-                           defer_merge=defer_merge)
+                           defer_merge=defer_merge, plan=plan)
     return K.attn_prefill(q, kc, vc, inp.block_tables, inp.cu_q, inp.ctx_lens, inp.max_qlen, self.scale)
 
   def _mla(self, xn: torch.Tensor, lw, li: int, inp: StepInputs) -> torch.Tensor:
@@ -1154,6 +1154,9 @@ class ShardModel:
     fuse = FUSE_NORM and h.is_cuda and h.shape[0] == 1 and not c.is_mla and n > 0
     hb = (h, torch.empty_like(h)) if fuse else None
     other = (lambda t: hb[1] if t is hb[0] else hb[0]) if fuse else (lambda t: None)
+    plan = None  # of the step's attention, for all layers
+    if inp.decode and n and self.ws is not None and not c.is_mla:
+      plan = self.ws.plan(inp.block_tables, inp.ctx_lens, c.num_kv_heads)
     for j, li in enumerate(self.layer_ids):
       lw = w.layers[li]
       if c.is_mla:
@@ -1164,7 +1167,7 @@ class ShardModel:
                            self.kv.v[j], c.num_heads, c.num_kv_heads, wide=not c.num_experts)
         if isinstance(xn, PendingNorm):
           h = xn.dst
-        a = self._attention(q, j, inp, defer_merge=fuse and FUSE_MERGE and lw.router is None)
+        a = self._attention(q, j, inp, defer_merge=fuse and FUSE_MERGE and lw.router is None, plan=plan)
         if not isinstance(a, K.PendingMerge):  # (a pending merge is finished inside o_proj's prologue)
           a = a.view(h.shape[0], c.num_heads * c.head_dim)
       # o_proj + residual + post-attention norm (one fused pass when the projection runs split-K)

@@ -208,6 +208,20 @@ def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None =
   return -(-pages // nparts)
 
 
+SPLIT_MIN_PAGES = 8  # widest block table whose contexts are not worth cutting
+
+
+def plan_pays(batch: int, Hkv: int, width_pages: int) -> bool:
+  """Whether a decode step cuts its contexts by their lengths (one small launch of 4.5 us a step, then every layer gains).  Up to 8 pages
+  a context is two rounds of a unit's four waves and best left whole (20 sequences x 8 heads up to 469 tokens 9.9 us either way).  Beyond,
+  the longest context ends the launch unless the pairs fill the chip several times over.  us a layer, uncut (or cut by the table's
+  width) / by the lengths: 24 sequences x 8 heads of 128, 74 .. 1407 tokens 21.1 / 15.2 (table of 128 pages 26.4 / 15.8), 8 of 125 .. 3176
+  33.5 / 12.8, 32 of 315 .. 7412 114 / 62, 48 of 31 .. 1059 24.4 / 19.8, 128 of 30 .. 1869 68 / 53; even ones 24 of 520 14.0 / 14.1, 64 of
+  1000 47.1 / 47.0, 12 of 900 15.3 / 15.0.  More pairs: 256 of 30 .. 1884 107 / 107, 130 of 10 .. 590 26.7 / 26.1."""
+  pairs = batch * Hkv
+  return width_pages > SPLIT_MIN_PAGES and pairs < 64 * min(width_pages, 32) and pairs * width_pages < 1 << 30
+
+
 class DecodeWorkspace:
   """Split-KV scratch for attn_decode, sized for every batch up to max_batch at this context bound.
   The partitioning is chosen per call from the actual batch (static per captured graph).  routed: the model has routed
@@ -231,7 +245,12 @@ class DecodeWorkspace:
           continue
         ppp = pages_per_part or choose_pages_per_part(b, hkv, max_ctx, kind)
         worst = max(worst, b * -(-pages // ppp))
+    # rows of split-KV partials: batch * nparts, or the places of a plan (a KV head has at most 16 query heads)
+    self.max_batch = max_batch
     self.units = worst  # max over batch of batch * nparts
+    if pages > SPLIT_MIN_PAGES and not routed:
+      worst = max(worst, max_batch + 512 // max(1, -(-H // 16)))
+    self.tickets = torch.zeros(max_batch * H, dtype=torch.int32, device=device)
     self.o = torch.empty(worst * H * Dh, dtype=torch.float32, device=device)
     self.ml = torch.empty(worst * H * 2, dtype=torch.float32, device=device)
 
@@ -243,6 +262,16 @@ class DecodeWorkspace:
     if batch * nparts > self.units:
       raise RuntimeError(f"decode workspace sized for {self.units} units, need {batch * nparts}")
     return ppp, nparts, algo
+
+
+  def plan(self, block_tables: torch.Tensor, ctx_lens: torch.Tensor, Hkv: int) -> torch.Tensor | None:
+    """The units of a decode step's attention (csrc/attention.hip decode_plan_kernel), one launch for all layers of the step; None
+    where attn_decode goes by itself."""
+    B, width = ctx_lens.shape[0], block_tables.shape[1]
+    if (not block_tables.is_cuda or self.fixed_ppp or B > self.max_batch or not plan_pays(B, Hkv, width) or self.Dh not in (64, 128)
+        or resolve_decode_algo(B, Hkv, self.algo, routed=self.routed) not in (2, 3)):
+      return None
+    return require().decode_plan(ctx_lens, B, Hkv, width)
 
 
 class PendingMerge:
@@ -261,8 +290,8 @@ class PendingMerge:
 
 
 def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, ws: DecodeWorkspace | None = None,
-                out: torch.Tensor | None = None, defer_merge: bool = False):
-  """defer_merge (one sequence): return a PendingMerge when the context is split over partitions."""
+                out: torch.Tensor | None = None, defer_merge: bool = False, plan: torch.Tensor | None = None):
+  """defer_merge (one sequence): return a PendingMerge when the context is split over partitions.  plan: ws.plan of the same step."""
   if not _gpu(q):
     y = ref.attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale)
     if out is not None:
@@ -273,8 +302,12 @@ def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, ws: D
   width = block_tables.shape[1]
   if ws is None:
     ws = DecodeWorkspace(B, H, Dh, width * PAGE, q.device)
-  ppp, nparts, algo = ws.partition(B, k_cache.shape[1], width)
   out = torch.empty_like(q) if out is None else out
+  if plan is not None:
+    nt = B * k_cache.shape[1] * width * PAGE * Dh * 4 >= NT_MIN_KV_BYTES
+    require().attn_decode_split(q, k_cache, v_cache, block_tables, plan, ws.tickets, out, ws.o, ws.ml, float(scale), nt)
+    return out
+  ppp, nparts, algo = ws.partition(B, k_cache.shape[1], width)
   defer = defer_merge and B == 1 and nparts > 1
   require().attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, ws.o, ws.ml, ppp, nparts, float(scale),
                         algo, not defer)
