@@ -58,7 +58,7 @@ def test_split_kernel(H, Hkv, Dh, lens):
   runs = []
   for nt in (False, True, False):
     out = torch.full_like(q, float("nan"))
-    C.attn_decode_split(q, kc, vc, bt, plan, ws.tickets, out, ws.o, ws.ml, Dh ** -0.5, nt)
+    C.attn_decode_split(q, kc, vc, bt, plan, cl, ws.tickets, out, ws.o, ws.ml, Dh ** -0.5, nt)
     assert int(ws.tickets.abs().max()) == 0
     runs.append(out)
   assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])  # whoever merges, in the order of the parts
@@ -96,3 +96,22 @@ def test_plan_follows_the_contexts_under_a_graph():
     assert torch.equal(got, step())
     whole = K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, K.DecodeWorkspace(len(lens), H, Dh, width * 64, q.device, pages_per_part=width, algo=2))
     assert float((got.float() - whole.float()).abs().max()) < 2e-2 * float(whole.float().abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Hkv,Dh", [(32, 8, 64), (16, 1, 128), (14, 2, 64), (32, 32, 128)])
+def test_lone_sequence_needs_no_plan(H, Hkv, Dh):
+  for width in (1, 8, 40, 128):
+    ws = None
+    for n in sorted({1, 64, 65, 255, 257, 321, width * 64 - 1, width * 64, 0} & set(range(width * 64 + 1))):
+      q, kc, vc, bt, cl = _step([n], width, H, Hkv, Dh)
+      ws = ws or K.DecodeWorkspace(1, H, Dh, width * 64, q.device)
+      assert ws.plan(bt, cl, Hkv) is K.LONE
+      out = K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, ws, plan=K.LONE)
+      assert torch.equal(out, K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, ws, plan=K.LONE)) and int(ws.tickets.abs().max()) == 0
+      if n == 0:
+        assert float(out.abs().max()) == 0.0
+        continue
+      want = R.attn_decode(q, kc, vc, bt, cl, 1 / math.sqrt(Dh)).float()
+      # (as above)
+      assert float((out.float() - want).abs().max()) < 2e-2 * float(want.abs().max()), (width, n)

@@ -546,20 +546,30 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_decode_group_kernel(
 // the XCD's L2 both ways (relaxed agent-scope accesses, waited for before the ticket): a release fence would write that L2 back, one
 // workgroup after another, and cost more than the merge launch (24 sequences of 74 .. 1407 tokens 50 us, 16 without).  The merge
 // is about 3 us behind a unit's pages, a launch for it 4.7.  Times beside ops.kernels.plan_pays.
+// plan none: one sequence; defer: its parts are left for o_proj's GEMM to merge (csrc/gemm_wave.hip)
+__device__ __forceinline__ DecodePart lone_part(int part, int ctx, int Hkv) {
+  const int pages = (ctx + PAGE - 1) / PAGE;
+  const int ppp = decode_lone_pages(pages, Hkv);
+  const int parts = max(1, (pages + ppp - 1) / ppp);
+  if (part >= parts) return {0, 0, 0, 0, 0, 0, 0, 0};
+  const int q = pages / parts, r = pages - q * parts, first = part * q + min(part, r);
+  return {0, first, first + q + (part < r), parts, 0, ctx, 0, 0};
+}
+
 template <int DH, bool NT>
 __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
-    const int32_t* __restrict__ block_tables, int max_blocks, const DecodePart* __restrict__ plan,
+    const int32_t* __restrict__ block_tables, int max_blocks, const DecodePart* __restrict__ plan, const int32_t* __restrict__ ctx_lens,
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int H, int Hkv,
-    float scale_log2, int num_pages, int* __restrict__ tickets) {
+    float scale_log2, int num_pages, int* __restrict__ tickets, bool defer) {
   extern __shared__ __attribute__((aligned(16))) float gsm[];
   __shared__ int last_sm;
   const int part = blockIdx.x / Hkv, kvh = blockIdx.x - part * Hkv, G = H / Hkv;
-  const DecodePart d = plan[part];
+  const DecodePart d = plan != nullptr ? plan[part] : lone_part(part, min(max(ctx_lens[0], 0), max_blocks * PAGE), Hkv);
   if (d.parts == 0) return;  // uniform over the workgroup: a place no part takes
-  decode_wave_unit<DH, 2, NT, 4, true>({d.b, kvh, d.first, d.last, d.parts == 1, (int)blockIdx.x * G, 1}, q, kc, vc, block_tables,
+  decode_wave_unit<DH, 2, NT, 4, true>({d.b, kvh, d.first, d.last, d.parts == 1 && !defer, (int)blockIdx.x * G, 1}, q, kc, vc, block_tables,
                                        max_blocks, d.ctx, out, ws_o, ws_ml, H, Hkv, scale_log2, num_pages, true, gsm);
-  if (d.parts == 1) return;
+  if (d.parts == 1 || defer) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial results have left (agent stores), no L2 write-back needed
   __syncthreads();
   int* t = tickets + d.b * Hkv + kvh;
@@ -603,7 +613,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
 // The units of a decode step: every sequence's pages in equal parts of at most ppp pages; an empty sequence is one part (which writes
 // zeros).  ppp is the candidate with the least estimated time, in pages a CU reads one behind the other: its longest part, and an
 // average one beside it where there are more units than CUs (two workgroups a CU run at once), or, past two a CU, its share of all
-// pages and a part that starts last.  One workgroup, a wave per candidate.
+// pages and a part that starts last; and the merge of its parts.  One workgroup, a wave per candidate.
 __global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restrict__ ctx_lens, int B, unsigned Hkv, int max_blocks,
                                                           int places, DecodePart* __restrict__ plan) {
   __shared__ int red[8], ctx_sm[512], first_sm[513];
@@ -639,7 +649,8 @@ __global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restr
     units = wave_sum_u(units);
     big = wave_max_u(big);
     const float u = (float)units * Hkv, work = (float)all, share = work / 256.f;
-    if (lane == 0) est_sm[wave] = u <= 256.f ? big : u <= 512.f ? fmaxf(big + work / u, share) + 1.f : share + big + 1.f;
+    const float merge = 0.4f * (float)((most + ppp - 1) / ppp);  // the longest sequence's parts, behind its last one
+    if (lane == 0) est_sm[wave] = (u <= 256.f ? big : u <= 512.f ? fmaxf(big + work / u, share) + 1.f : share + big + 1.f) + merge;
   }
   __syncthreads();
   int best = 0;
@@ -688,14 +699,14 @@ int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, 
 }
 
 int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables, int max_blocks,
-                             const DecodePart* plan, int places, int* tickets, uint16_t* out, float* ws_o, float* ws_ml, int H,
-                             int Hkv, int Dh, float scale, int num_pages, bool nt, hipStream_t s) {
+                             const DecodePart* plan, int places, const int32_t* ctx_lens, int* tickets, uint16_t* out, float* ws_o, float* ws_ml, int H,
+                             int Hkv, int Dh, float scale, int num_pages, bool nt, bool defer, hipStream_t s) {
   if (places <= 0) return 0;
   if (H % Hkv != 0 || H / Hkv > 16) return -1;
   const size_t lds = (size_t)4 * (H / Hkv) * (Dh + 6) * sizeof(float);  // at most 34 KB
 #define XOT_SPLIT(DHV, NTV)                                                                                                \
-  attn_decode_split_kernel<DHV, NTV><<<places * Hkv, 256, lds, s>>>(q, kc, vc, block_tables, max_blocks, plan, out, ws_o, ws_ml, \
-                                                                    H, Hkv, scale * LOG2E, num_pages, tickets)
+  attn_decode_split_kernel<DHV, NTV><<<places * Hkv, 256, lds, s>>>(q, kc, vc, block_tables, max_blocks, plan, ctx_lens, out, ws_o, ws_ml, \
+                                                                    H, Hkv, scale * LOG2E, num_pages, tickets, defer)
   if (Dh == 128) {
     if (nt) XOT_SPLIT(128, true);
     else XOT_SPLIT(128, false);
@@ -712,9 +723,8 @@ int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16
 int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                        int max_blocks, const int32_t* ctx_lens, uint16_t* out, float* ws_o, float* ws_ml, int B,
                        int H, int Hkv, int Dh, int pages_per_part, int nparts, float scale, int num_pages, int algo,
-                       hipStream_t s, bool merge) {
-  // merge = false: the partitions are left in ws_o / ws_ml for the consumer (launch_gemm_stream_merge's prologue at batch 1).
-  const bool reduce = nparts > 1 && merge;
+                       hipStream_t s) {
+  const bool reduce = nparts > 1;
   if (B <= 0) return 0;
   if (H % Hkv != 0 || H / Hkv > 16) return -1;
   dim3 grid(nparts, Hkv, B);
@@ -775,15 +785,6 @@ int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc
     return -1;
   }
   return 0;
-}
-
-void launch_attn_decode_merge(const float* ws_o, const float* ws_ml, const int32_t* ctx_lens, uint16_t* out, int B,
-                              int H, int Dh, int nparts, int pages_per_part, hipStream_t s) {
-  if (B <= 0) return;
-  if (Dh == 128)
-    attn_decode_reduce_kernel<128><<<B * H, 128, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
-  else if (Dh == 64)
-    attn_decode_reduce_kernel<64><<<B * H, 64, 0, s>>>(ws_o, ws_ml, ctx_lens, out, H, nparts, pages_per_part);
 }
 
 // ============================================================================ prefill

@@ -866,8 +866,7 @@ void moe_combine_norm(const at::Tensor& y, const at::Tensor& slot_of, const at::
 
 void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                  const at::Tensor& block_tables, const at::Tensor& ctx_lens, at::Tensor& out, at::Tensor& ws_o,
-                 at::Tensor& ws_ml, int64_t pages_per_part, int64_t nparts, double scale, int64_t algo,
-                 bool merge) {
+                 at::Tensor& ws_ml, int64_t pages_per_part, int64_t nparts, double scale, int64_t algo) {
   CHECK_BF16(q);
   CHECK_BF16(k_cache);
   CHECK_BF16(v_cache);
@@ -892,7 +891,7 @@ void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tenso
                                          (int)block_tables.size(1), ctx_lens.data_ptr<int32_t>(), bf(out),
                                          ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), (int)B, (int)H, (int)Hkv,
                                          (int)Dh, (int)pages_per_part, (int)nparts, (float)scale, (int)nb, (int)algo,
-                                         cur_stream(), merge);
+                                         cur_stream());
   XCHECK(rc == 0, "attn_decode: unsupported H=", H, " Hkv=", Hkv, " Dh=", Dh);
 }
 
@@ -909,18 +908,18 @@ at::Tensor decode_plan(const at::Tensor& ctx_lens, int64_t B, int64_t Hkv, int64
 }
 
 void attn_decode_split(const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache, const at::Tensor& block_tables,
-                       const at::Tensor& plan, at::Tensor& tickets, at::Tensor& out, at::Tensor& ws_o, at::Tensor& ws_ml,
-                       double scale, bool nt) {
+                       const c10::optional<at::Tensor>& plan, const at::Tensor& ctx_lens, at::Tensor& tickets, at::Tensor& out, at::Tensor& ws_o, at::Tensor& ws_ml,
+                       double scale, bool nt, bool defer) {
   CHECK_BF16(q);
   CHECK_BF16(k_cache);
   CHECK_BF16(v_cache);
   CHECK_BF16(out);
   CHECK_DT(block_tables, at::kInt);
-  CHECK_DT(plan, at::kInt);
+  CHECK_DT(ctx_lens, at::kInt);
   CHECK_DT(tickets, at::kInt);
   CHECK_DT(ws_o, at::kFloat);
   CHECK_DT(ws_ml, at::kFloat);
-  XCHECK(all_contig_gpu(q, k_cache, v_cache, block_tables, plan, tickets, out, ws_o, ws_ml),
+  XCHECK(all_contig_gpu(q, k_cache, v_cache, block_tables, ctx_lens, tickets, out, ws_o, ws_ml),
          "attn_decode_split: all tensors must be contiguous GPU tensors");
   XCHECK(q.dim() == 3 && k_cache.dim() == 4 && v_cache.dim() == 4, "attn_decode_split: q [B,H,Dh], caches 4-D");
   const int64_t B = q.size(0), H = q.size(1), Dh = q.size(2), Hkv = k_cache.size(1), nb = k_cache.size(0);
@@ -929,57 +928,58 @@ void attn_decode_split(const at::Tensor& q, const at::Tensor& k_cache, const at:
          "attn_decode_split: cache layout K[nb,Hkv,64,Dh] V[nb,Hkv,Dh,64]");
   XCHECK(block_tables.dim() == 2 && block_tables.size(0) >= B, "attn_decode_split: tables");
   XCHECK(out.numel() == B * H * Dh, "attn_decode_split: out shape");
-  XCHECK(plan.dim() == 2 && plan.size(1) == 8 && reinterpret_cast<uintptr_t>(plan.data_ptr()) % 32 == 0, "attn_decode_split: plan");
-  const int64_t places = plan.size(0);
+  XCHECK(!defer || !plan.has_value(), "attn_decode_split: only a lone sequence's parts can be left unmerged");
+  int64_t places = 0;
+  const xot::DecodePart* parts = nullptr;
+  if (plan.has_value()) {
+    CHECK_DT((*plan), at::kInt);
+    XCHECK(all_contig_gpu(*plan) && plan->dim() == 2 && plan->size(1) == 8 && reinterpret_cast<uintptr_t>(plan->data_ptr()) % 32 == 0,
+           "attn_decode_split: plan");
+    places = plan->size(0);
+    parts = reinterpret_cast<const xot::DecodePart*>(plan->data_ptr<int32_t>());
+  } else {
+    XCHECK(B == 1 && ctx_lens.numel() >= 1, "attn_decode_split: several sequences need a plan");
+    places = xot::decode_split_places(1, (int)Hkv, (int)block_tables.size(1));
+  }
   XCHECK(tickets.numel() >= B * Hkv && ws_o.numel() >= places * H * Dh && ws_ml.numel() >= places * H * 2,
          "attn_decode_split: workspace small");
   const int rc = xot::launch_attn_decode_split(
       bf(q), bf(k_cache), bf(v_cache), block_tables.data_ptr<int32_t>(), (int)block_tables.size(1),
-      reinterpret_cast<const xot::DecodePart*>(plan.data_ptr<int32_t>()), (int)places, tickets.data_ptr<int32_t>(), bf(out),
-      ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), (int)H, (int)Hkv, (int)Dh, (float)scale, (int)nb, nt, cur_stream());
+      parts, (int)places, ctx_lens.data_ptr<int32_t>(), tickets.data_ptr<int32_t>(), bf(out),
+      ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), (int)H, (int)Hkv, (int)Dh, (float)scale, (int)nb, nt, defer, cur_stream());
   XCHECK(rc == 0, "attn_decode_split: unsupported H=", H, " Hkv=", Hkv, " Dh=", Dh);
 }
 
-// the partition merge attn_decode(merge = false) left out: out [B, H, Dh] from ws_o / ws_ml
-void attn_decode_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, const at::Tensor& ctx_lens, at::Tensor& out,
-                       int64_t pages_per_part, int64_t nparts) {
-  CHECK_BF16(out);
-  CHECK_DT(ws_o, at::kFloat);
-  CHECK_DT(ws_ml, at::kFloat);
-  CHECK_DT(ctx_lens, at::kInt);
-  XCHECK(all_contig_gpu(ws_o, ws_ml, ctx_lens, out) && out.dim() == 3, "attn_decode_merge: contiguous GPU, out [B,H,Dh]");
-  const int64_t B = out.size(0), H = out.size(1), Dh = out.size(2);
-  XCHECK(Dh == 128 || Dh == 64, "attn_decode_merge: Dh");
-  XCHECK(ws_o.numel() >= B * H * nparts * Dh && ws_ml.numel() >= B * H * nparts * 2 && ctx_lens.numel() >= B,
-         "attn_decode_merge: workspace");
-  xot::launch_attn_decode_merge(ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), ctx_lens.data_ptr<int32_t>(), bf(out),
-                                (int)B, (int)H, (int)Dh, (int)nparts, (int)pages_per_part, cur_stream());
-}
-
-// o_proj of a batch-1 decode step on the pre-shuffled weight w [N, H*Dh], its input row merged from the attention's
-// partitions (ws_o / ws_ml, row 0) in the prologue; writes `splits` fp32 slabs into ws (no reduce)
-void gemm_stream_merge(const at::Tensor& w, at::Tensor& ws, int64_t ntw, int64_t splits, const at::Tensor& ws_o,
-                       const at::Tensor& ws_ml, const at::Tensor& ctx_lens, int64_t pages_per_part, int64_t nparts,
-                       int64_t Dh) {
+// o_proj of a lone sequence on the pre-shuffled weight w [N, H * Dh]: h [1, N] += (its attention's parts merged) . w^T (+ bias)
+void gemm_solo_merge(const at::Tensor& w, at::Tensor& h, const c10::optional<at::Tensor>& bias, const at::Tensor& ws_o,
+                     const at::Tensor& ws_ml, const at::Tensor& ctx_lens, int64_t max_blocks, int64_t Hkv, int64_t Dh) {
   CHECK_BF16(w);
-  CHECK_DT(ws, at::kFloat);
+  CHECK_BF16(h);
   CHECK_DT(ws_o, at::kFloat);
   CHECK_DT(ws_ml, at::kFloat);
   CHECK_DT(ctx_lens, at::kInt);
-  XCHECK(all_contig_gpu(w, ws, ws_o, ws_ml, ctx_lens) && w.dim() == 2, "gemm_stream_merge: contiguous GPU tensors");
   const int64_t N = w.size(0), K = w.size(1);
-  XCHECK(Dh > 0 && K % Dh == 0 && ws_o.numel() >= (K / Dh) * nparts * Dh && ws_ml.numel() >= (K / Dh) * nparts * 2,
-         "gemm_stream_merge: attention workspace");
-  xot::NormPro np{};
-  np.mo = ws_o.data_ptr<float>();
-  np.ml = ws_ml.data_ptr<float>();
-  np.ctx = ctx_lens.data_ptr<int32_t>();
-  np.nparts = (int)nparts;
-  np.ppp = (int)pages_per_part;
-  np.dh = (int)Dh;
-  const int rc = xot::launch_gemm_stream_merge(bf(w), ws.data_ptr<float>(), ws.numel(), (int)N, (int)K, (int)ntw,
-                                               (int)splits, np, cur_stream());
-  XCHECK(rc == 0, "gemm_stream_merge: unsupported N=", N, " K=", K, " ntw=", ntw, " splits=", splits);
+  XCHECK(all_contig_gpu(w, h, ws_o, ws_ml, ctx_lens) && w.dim() == 2 && h.numel() == N && ctx_lens.numel() >= 1,
+         "gemm_solo_merge: contiguous GPU tensors, h [1, N]");
+  XCHECK((Dh == 64 || Dh == 128) && K % Dh == 0 && Hkv >= 1 && (K / Dh) % Hkv == 0 && max_blocks >= 1, "gemm_solo_merge: heads");
+  const int64_t parts = xot::decode_split_places(1, (int)Hkv, (int)max_blocks);
+  XCHECK(ws_o.numel() >= parts * K && ws_ml.numel() >= parts * (K / Dh) * 2, "gemm_solo_merge: workspace");
+  xot::WaveGemm a{};
+  a.W = bf(w);
+  a.Y = h.data_ptr();
+  a.R = bf(h);
+  a.ldy = a.ldr = (int)N;
+  a.M = 1;
+  a.N = (int)N;
+  a.K = (int)K;
+  if (bias.has_value()) {
+    CHECK_BF16((*bias));
+    XCHECK(bias->numel() == N && bias->is_contiguous(), "gemm_solo_merge: bias");
+    a.bias = bf(*bias);
+  }
+  a.mg = xot::LoneMerge{ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), ctx_lens.data_ptr<int32_t>(), (int)max_blocks, (int)Hkv, (int)Dh, (int)parts};
+  const int rc = xot::launch_gemm_wave(a, false, 1, 0, cur_stream());
+  XCHECK(rc == 0, "gemm_solo_merge: unsupported N=", N, " K=", K, " pages=", max_blocks);
 }
 
 // training attention: 2-D token-major views ([B*L, n*Dh] rows, unit inner stride; row strides may differ,
@@ -1262,15 +1262,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("splits") = 1, py::arg("n_shared") = 0);
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
-        py::arg("nparts"), py::arg("scale"), py::arg("algo") = 2, py::arg("merge") = true);
+        py::arg("nparts"), py::arg("scale"), py::arg("algo") = 2);
   m.def("decode_plan", &decode_plan, py::arg("ctx_lens"), py::arg("B"), py::arg("Hkv"), py::arg("max_blocks"));
   m.def("attn_decode_split", &attn_decode_split, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
-        py::arg("plan"), py::arg("tickets"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("scale"), py::arg("nt"));
-  m.def("attn_decode_merge", &attn_decode_merge, py::arg("ws_o"), py::arg("ws_ml"), py::arg("ctx_lens"), py::arg("out"),
-        py::arg("pages_per_part"), py::arg("nparts"));
-  m.def("gemm_stream_merge", &gemm_stream_merge, py::arg("w"), py::arg("ws"), py::arg("ntw"), py::arg("splits"),
-        py::arg("ws_o"), py::arg("ws_ml"), py::arg("ctx_lens"), py::arg("pages_per_part"), py::arg("nparts"),
-        py::arg("Dh"));
+        py::arg("plan"), py::arg("ctx_lens"), py::arg("tickets"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("scale"), py::arg("nt"),
+        py::arg("defer") = false);
+  m.def("gemm_solo_merge", &gemm_solo_merge, py::arg("w"), py::arg("h"), py::arg("bias"), py::arg("ws_o"), py::arg("ws_ml"),
+        py::arg("ctx_lens"), py::arg("max_blocks"), py::arg("Hkv"), py::arg("Dh"));
   m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("cu_q"), py::arg("ctx_lens"), py::arg("out"), py::arg("max_qlen"), py::arg("scale"), py::arg("algo") = 2);
   m.def("router_logits", &router_logits);

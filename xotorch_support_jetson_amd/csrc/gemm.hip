@@ -206,7 +206,7 @@ int launch_gemm_skinny(const uint16_t* X, int ldx, const uint16_t* W, int ldw, c
 // the bytes of the bf16 layout.  v_cvt_scalef32_pk_bf16_fp8 widens each fragment just before its MFMAs;
 // the row scale is applied to the fp32 accumulators (so split-K slabs are already scaled).
 template <int MT, int NTW, int KS, int EPI, bool OUT_F32, bool SPLIT, bool WSHUF, int OCC, int MOE, bool W8 = false,
-          int NORM = 0, bool MERGE = false>
+          int NORM = 0>
 __global__ __launch_bounds__(256, OCC) void gemm_stream_kernel(const uint16_t* __restrict__ X, int ldx,
                                                              const uint16_t* __restrict__ W, int ldw,
                                                              const uint16_t* __restrict__ bias,
@@ -362,63 +362,12 @@ __global__ __launch_bounds__(256, OCC) void gemm_stream_kernel(const uint16_t* _
   // loads stay unconditional) and finishes with a single-chunk tail.
   const int last = nch - 1;
   s16x8 wa[NTW][KS], wb[NTW][KS];
-  if constexpr (NORM > 0 || MERGE) {
+  if constexpr (NORM > 0) {
   static_assert(MT == 1 && MOE == 0 && !W8 && WSHUF, "row prologue: one row, pre-shuffled bf16 weights");
   uint16_t* x1 = xs_raw;  // this workgroup's K slice of the input row, [kper] bf16
   wload(wa, 0);
   wload(wb, min(1, last));
-  if constexpr (MERGE) {
-    // split-KV decode attention merge (attn_decode_reduce_kernel's arithmetic, in its order) for the heads of
-    // this workgroup's K slice: o = sum_p 2^(m_p - M) o_p / sum_p 2^(m_p - M) l_p over the row's partitions
-    const int npages = (max(np.ctx[0], 0) + 63) / 64;
-    int npart = (npages + np.ppp - 1) / np.ppp;
-    npart = npart < 1 ? 1 : (npart > np.nparts ? np.nparts : npart);
-    constexpr int NPM = 8;  // partitions whose loads are all requested before use (more: a second, per-element loop)
-    for (int e0 = 4 * tid; e0 < kper; e0 += 4 * NTH) {  // 4 consecutive elements of one head per thread
-      const int k = kb + e0, hd = k / np.dh, d = k - hd * np.dh;
-      const size_t base = (size_t)hd * np.nparts;
-      float o4[4];
-      if (npart <= NPM) {
-        f32x2_t mv[NPM];
-        f32x4 ov[NPM];
-#pragma unroll
-        for (int q = 0; q < NPM; ++q)
-          if (q < npart) {
-            mv[q] = *reinterpret_cast<const f32x2_t*>(np.ml + (base + q) * 2);
-            ov[q] = *reinterpret_cast<const f32x4*>(np.mo + (base + q) * np.dh + d);
-          }
-        float M = -1e30f;
-#pragma unroll
-        for (int q = 0; q < NPM; ++q)
-          if (q < npart) M = fmaxf(M, mv[q][0]);
-        float L = 0.f, O[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < NPM; ++q)
-          if (q < npart) {
-            const float f = exp2f(mv[q][0] - M);
-            L += mv[q][1] * f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) O[j] += ov[q][j] * f;
-          }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o4[j] = L > 0.f ? O[j] / L : 0.f;
-      } else {
-        float M = -1e30f;
-        for (int q = 0; q < npart; ++q) M = fmaxf(M, np.ml[(base + q) * 2]);
-        float L = 0.f, O[4] = {0.f, 0.f, 0.f, 0.f};
-        for (int q = 0; q < npart; ++q) {
-          const float f = exp2f(np.ml[(base + q) * 2] - M);
-          L += np.ml[(base + q) * 2 + 1] * f;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) O[j] += np.mo[(base + q) * np.dh + d + j] * f;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o4[j] = L > 0.f ? O[j] / L : 0.f;
-      }
-      *reinterpret_cast<s16x4*>(x1 + e0) =
-          s16x4{(short)f2bf(o4[0]), (short)f2bf(o4[1]), (short)f2bf(o4[2]), (short)f2bf(o4[3])};
-    }
-  } else {
+  {
     // RMSNorm prologue (one input row; NORM = 16-B chunks of the row per thread): the first two weight chunks,
     // then every residual / bias / norm-weight load and the first SMAX slabs are requested before any is used,
     // so the chain is one L2 round trip per SMAX slabs (the producer just wrote them), one wave reduction and two
@@ -897,30 +846,6 @@ static void stream_norm_launch(const uint16_t* W, const uint16_t* bias, void* Y,
   if (!reduce) return;
   const int ncol = EPI == EPI_SILU ? N / 2 : N;
   splitk_reduce_kernel<EPI, false><<<(ncol / 8 + 255) / 256, 256, 0, st>>>(ws, S, 1, N, bias, nullptr, 0, Y, ldy);
-}
-
-// o_proj of a batch-1 decode step with the attention's partition merge in its prologue: split-K slabs only (the
-// consumer -- splitk_resid_rmsnorm or the next GEMM's norm prologue -- adds them to the residual)
-int launch_gemm_stream_merge(const uint16_t* W, float* ws, long ws_elems, int N, int K, int ntw, int S,
-                             const NormPro& np, hipStream_t s) {
-  if (ntw == 4) ntw = 2;
-  if (ntw != 1 && ntw != 2) return -1;
-  if (S < 2 || N % (64 * ntw) != 0 || K % (S * 128) != 0 || (long)(K / S) * 2 > 65536) return -1;
-  if (ws == nullptr || ws_elems < (long)S * N || np.mo == nullptr || np.ml == nullptr || np.ctx == nullptr ||
-      np.nparts < 1 || np.ppp < 1 || np.dh <= 0 || np.dh % 4 != 0 || K % np.dh != 0)
-    return -1;
-  const int kper = K / S;
-  const dim3 grid(N / (64 * ntw), S);
-  const size_t smem = (size_t)kper * 2;
-  if (ntw == 1)
-    gemm_stream_kernel<1, 1, 4, EPI_NONE, false, true, true, 2, 0, false, 0, true><<<grid, 256, smem, s>>>(
-        nullptr, 0, W, K, nullptr, nullptr, 0, nullptr, N, ws, 1, N, kper, 1, nullptr, nullptr, nullptr, 0L, nullptr,
-        0L, 0L, np, 0.f);
-  else
-    gemm_stream_kernel<1, 2, 4, EPI_NONE, false, true, true, 2, 0, false, 0, true><<<grid, 256, smem, s>>>(
-        nullptr, 0, W, K, nullptr, nullptr, 0, nullptr, N, ws, 1, N, kper, 1, nullptr, nullptr, nullptr, 0L, nullptr,
-        0L, 0L, np, 0.f);
-  return 0;
 }
 
 int launch_gemm_stream_norm(const uint16_t* W, const uint16_t* bias, void* Y, int ldy, int epi, float* ws,

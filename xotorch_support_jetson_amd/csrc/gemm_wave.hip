@@ -439,23 +439,223 @@ int normed(const WaveGemm& a, int epi, int nt, hipStream_t st) {
                          : one_row_tile<EPI_NONE, false, NORM, SM, false>(a, nt, st);
 }
 
+// Up to 16 rows, one column tile a workgroup (HALF: half of one, its eight columns), the eight waves a part of K each: a wave copies
+// the rows of X that its own blocks need through LDS of its own, so no wave waits for another before the partial tiles meet.
+// HALF: a load takes the tile half's 128-byte runs of two k blocks, the first in columns 0 .. 7 of the MFMA operand, the second in
+// 8 .. 15; each block's rows of X multiply it all and the sums of the other block's columns are not used.
+// Bound by the weight stream: 2048 columns by whole tiles keep half of the CUs, which take 50 GB/s each at most (2048 x 8192 at one
+// row 9.4 us by tiles, 7.9 by halves; x 5632 7.4 and 6.2, 8.7 with four waves a tile that meet at barriers); from 9 rows on slabs are the
+// faster, for every workgroup copies all of X (2048 x 5632 at 16 rows 9.1 / 6.9).
+// NP (one row): X is the merge of a lone sequence's attention parts, NP at most, in attn_decode_split_kernel's arithmetic: a wave merges
+// what its own blocks multiply, while its weights are on their way.
+template <bool HALF, int XL, int EPI, bool F32, int NP = 0>
+__global__ __launch_bounds__(512, 2) void gemm_solo_kernel(const uint16_t* __restrict__ X, int ldx, const uint16_t* __restrict__ W,
+                                                           const uint16_t* __restrict__ bias, const uint16_t* __restrict__ R, int ldr,
+                                                           void* __restrict__ Yv, int ldy, int M, int N, int K, LoneMerge mg) {
+  static_assert(NP == 0 || XL == 1, "merged parts are one row");
+  constexpr int KW = 8, CB = U * KW, SL = U * 4;   // waves, k blocks of a chunk, 16-byte slots of a row's part of it
+  constexpr int RL = 64 / SL, ROWS = XL * RL;      // rows of a 1 KB piece of X; rows in LDS (MFMA rows past them repeat them)
+  constexpr int NI = HALF ? U / 2 : U;             // weight loads of a stage
+  __shared__ __attribute__((aligned(16))) char smem[KW * XL * 1024 > KW * 1024 ? KW * XL * 1024 : KW * 1024];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = HALF ? blockIdx.x >> 1 : blockIdx.x, col0 = HALF ? (blockIdx.x & 1) * 8 : 0;
+  const int nb = K >> 5, nch = (nb + CB - 1) / CB;
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W + (size_t)tile * nb * 512), (short)0, nb * 1024, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X), (short)0, NP ? 0 : ((M - 1) * ldx + K) * 2, 0x00020000);
+  char* xs = smem + p * (XL * 1024);
+  struct Stage {
+    s16x8 w[NI];
+  };
+  const unsigned woff = HALF ? (c >> 3) * 1024u + (g * 16 + col0 + (c & 7)) * 16u : lane * 16u;
+  auto load = [&](Stage& s, int ch) {  // the wave's blocks of chunk ch (past K: zeros, not used)
+#pragma unroll
+    for (int u = 0; u < NI; ++u) s.w[u] = buf16(wr, woff + (ch * CB + p * U + u * (U / NI)) * 1024u, true);
+  };
+  const int prow = lane / SL, pslot = lane % SL;
+  auto xload = [&](s16x8 (&x)[XL], int ch) {  // (past K: the next row's numbers or zeros, not used)
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      x[i] = buf16(xr, min(i * RL + prow, M - 1) * ldx * 2u + pslot * 16u + (ch * CB + p * U) * 64u, false);
+  };
+  auto xstore = [&](const s16x8 (&x)[XL]) {
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int row = i * RL + prow;
+      *reinterpret_cast<s16x8*>(xs + (row * SL + (pslot ^ (row & 15))) * 16) = x[i];
+    }
+  };
+  const int row0 = c & (ROWS - 1);
+  int fo[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) fo[j] = (row0 * SL + ((4 * j + g) ^ row0)) * 16;
+  f32x4 acc[HALF ? 2 : 1];
+#pragma unroll
+  for (int i = 0; i < (HALF ? 2 : 1); ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const Stage& s, int ch) {
+    const int left = nb - ch * CB - p * U;  // blocks of K from the wave's part on (a multiple of four)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < left) {
+        const s16x8 a = *reinterpret_cast<const s16x8*>(xs + fo[u & 3] + (u >> 2) * 256);
+        f32x4& t = acc[HALF ? u & 1 : 0];
+        t = mfma16(a, s.w[HALF ? u >> 1 : u], t);
+      }
+  };
+  Stage sa, sb;
+  s16x8 xa[XL], xb[XL];
+  if constexpr (NP > 0) {  // (at most two chunks: xa and xb are all of X)
+    const int pages = (min(max(mg.ctx[0], 0), mg.max_blocks * 64) + 63) / 64, ppp = decode_lone_pages(pages, mg.Hkv);
+    const int np = min(max(1, (pages + ppp - 1) / ppp), NP);
+    struct Part {
+      f32x2_t ml;
+      f32x4 o[2];
+    };
+    auto parts = [&](Part (&t)[NP], int ch) {
+      const int k = min((ch * CB + p * U) * 32 + pslot * 8, K - 8);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {  // (past the last: the last again, not used)
+        const int at = min(q, np - 1) * K + k, sh = mg.Dh == 128 ? 7 : 6;
+        t[q].ml = *reinterpret_cast<const f32x2_t*>(mg.ml + (at >> sh) * 2);
+        t[q].o[0] = *reinterpret_cast<const f32x4*>(mg.o + at);
+        t[q].o[1] = *reinterpret_cast<const f32x4*>(mg.o + at + 4);
+      }
+    };
+    auto merge = [&](const Part (&t)[NP]) {
+      float M = -1e30f, L = 0.f;
+#pragma unroll
+      for (int q = 0; q < NP; ++q) M = fmaxf(M, t[q].ml[0]);
+      f32x4 o[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int q = 0; q < NP; ++q)
+        if (q < np) {
+          const float f = exp2f(t[q].ml[0] - M);
+          L += t[q].ml[1] * f;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) o[i] += t[q].o[i] * f;
+        }
+      s16x8 x;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (short)f2bf(L > 0.f ? o[e >> 2][e & 3] / L : 0.f);
+      return x;
+    };
+    Part ta[NP], tb[NP];
+    parts(ta, 0);
+    if (nch > 1) parts(tb, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load(sa, 0);
+    load(sb, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    xa[0] = merge(ta);
+    if (nch > 1) xb[0] = merge(tb);
+  } else {
+    xload(xa, 0);
+    load(sa, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    xload(xb, 1);
+    load(sb, 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  for (int ch = 0; ch < nch; ch += 2) {  // (a wave's LDS accesses keep their order: no wait between a chunk's reads and the next writes)
+    xstore(xa);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NP == 0) xload(xa, ch + 2);
+    compute(sa, ch);
+    __builtin_amdgcn_sched_barrier(0);
+    load(sa, ch + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    if (ch + 1 >= nch) break;
+    xstore(xb);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NP == 0) xload(xb, ch + 3);
+    compute(sb, ch + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load(sb, ch + 3);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  f32x4 v = acc[0];
+  if constexpr (HALF) {  // columns c and c ^ 8 are one, over the even and the odd blocks
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float t = c < 8 ? acc[0][r] : acc[1][r];
+      v[r] = t + __uint_as_float(row_turn<8>(__float_as_uint(t)));
+    }
+  }
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(smem);  // [KW][64]
+  red[p * 64 + lane] = v;
+  __syncthreads();
+  if (p != 0 || (HALF && c >= 8)) return;
+#pragma unroll
+  for (int q = 1; q < KW; ++q) v += red[q * 64 + lane];
+  const int n = tile * 16 + col0 + c;
+  if (bias != nullptr) v += bf2f(bias[n]);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {  // lane (g, c): token 4 g + r
+    const int m = 4 * g + r;
+    if (m >= M) continue;
+    float y = v[r];
+    if constexpr (EPI == EPI_RESID) y += bf2f(R[(size_t)m * ldr + n]);
+    if constexpr (F32) reinterpret_cast<float*>(Yv)[(size_t)m * ldy + n] = y;
+    else reinterpret_cast<uint16_t*>(Yv)[(size_t)m * ldy + n] = f2bf(y);
+  }
+}
+
+template <bool HALF, int EPI, bool F32>
+int solo_rows(const WaveGemm& a, hipStream_t st) {
+  const int grid = HALF ? a.N / 8 : a.N / 16;
+#define XOT_SOLO(XLV) \
+  gemm_solo_kernel<HALF, XLV, EPI, F32><<<grid, 512, 0, st>>>(a.X, a.ldx, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy, a.M, a.N, a.K, a.mg)
+  if (a.M <= 2) XOT_SOLO(1);
+  else if (a.M <= 4) XOT_SOLO(2);
+  else if (a.M <= 8) XOT_SOLO(4);
+  else XOT_SOLO(8);
+#undef XOT_SOLO
+  return 0;
+}
+
+constexpr int MERGE_PARTS = 4;
+template <bool HALF>
+int solo_merge(const WaveGemm& a, hipStream_t st) {
+  gemm_solo_kernel<HALF, 1, EPI_RESID, false, MERGE_PARTS><<<HALF ? a.N / 8 : a.N / 16, 512, 0, st>>>(
+      nullptr, 0, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy, 1, a.N, a.K, a.mg);
+  return 0;
+}
+
+template <int EPI, bool F32>
+int solo(const WaveGemm& a, hipStream_t st) {
+  return a.N <= 2048 ? solo_rows<true, EPI, F32>(a, st) : solo_rows<false, EPI, F32>(a, st);
+}
+
 }  // namespace
 
 int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream_t st) {
   if (a.M <= 0) return 0;
   const bool rope = a.ro.q != nullptr, norm = a.np.h != nullptr;
-  if (a.M > 64 || a.K % 128 != 0 || a.K <= 0 || nt < 1 || nt > 8 || a.N % 16 != 0) return -1;
+  if (a.M > 64 || a.K % 128 != 0 || a.K <= 0 || nt < 0 || nt > 8 || a.N % 16 != 0) return -1;
   if ((int64_t)a.K * 32 >= (int64_t(1) << 31)) return -1;  // (32-bit byte offsets into a tile)
   if (!norm && (a.ldx % 8 != 0 || (int64_t)a.M * a.ldx * 2 >= (int64_t(1) << 31))) return -1;
   if ((rope || epi_is_glu(epi)) && (nt % 2 != 0 || a.N % 32 != 0)) return -1;
   if (rope && (epi != EPI_NONE || out_f32 || a.ro.Dh % 32 != 0 || a.N != (a.ro.H + 2 * a.ro.Hkv) * a.ro.Dh || a.ro.max_pos < 1)) return -1;
   if (norm) {
-    if (a.M != 1 || out_f32 || (epi != EPI_NONE && epi != EPI_SILU) || a.np.D != a.K || a.K > 8192 || a.np.S < 0 ||
+    if (nt == 0 || a.M != 1 || out_f32 || (epi != EPI_NONE && epi != EPI_SILU) || a.np.D != a.K || a.K > 8192 || a.np.S < 0 ||
         a.np.lnw == nullptr || a.np.hout == nullptr || (a.np.S > 0 && (a.np.ws == nullptr || a.np.sstride < a.K)))
       return -1;
     // (slabs of the first round trip: 8 where the row is short, or they would keep a second workgroup off the CU)
     if (a.K <= 2048) return a.np.S > 4 ? normed<1, 8>(a, epi, nt, st) : normed<1, 4>(a, epi, nt, st);
     return a.K <= 4096 ? normed<2, 4>(a, epi, nt, st) : normed<4, 2>(a, epi, nt, st);
+  }
+  if (a.mg.o != nullptr) {  // (two chunks of K)
+    if (nt != 0 || a.M != 1 || out_f32 || epi != EPI_RESID || rope || norm || a.K > 2 * 2048 || a.mg.max_parts > MERGE_PARTS || a.K % a.mg.Dh != 0) return -1;
+    return a.N <= 2048 ? solo_merge<true>(a, st) : solo_merge<false>(a, st);
+  }
+  if (nt == 0) {
+    if (rope || norm || a.M > 16) return -1;
+    if (epi == EPI_RESID) return out_f32 ? -1 : solo<EPI_RESID, false>(a, st);
+    if (epi != EPI_NONE) return -1;
+    return out_f32 ? solo<EPI_NONE, true>(a, st) : solo<EPI_NONE, false>(a, st);
   }
   if (rope) return by_rows<EPI_NONE, false, true>(a, nt, st);
   switch (epi) {

@@ -38,9 +38,6 @@ int launch_gemm_stream(const uint16_t* X, int ldx, const uint16_t* W, int ldw, c
 // reduce + norm launch); workgroup (0, 0) stores the summed residual row to hout (never h itself: the other
 // workgroups are still reading h).  Pre-shuffled bf16 weights, epi none / silu, split-K into ws (a different
 // buffer from np.ws).
-// The same kernel's other row prologue (launch_gemm_stream_merge): the row is the merge of a batch-1 split-KV
-// decode attention's partitions (mo [H][nparts][dh], ml [H][nparts][2], ctx_lens[0]), so the o_proj GEMM replaces
-// the attention's merge launch.
 struct NormPro {
   const uint16_t* h;
   const float* ws;
@@ -51,15 +48,7 @@ struct NormPro {
   uint16_t* hout;
   float eps;
   int D;
-  const float* mo;
-  const float* ml;
-  const int32_t* ctx;
-  int nparts, ppp, dh;
 };
-int launch_gemm_stream_merge(const uint16_t* W, float* ws, long ws_elems, int N, int K, int ntw, int S,
-                             const NormPro& np, hipStream_t s);
-void launch_attn_decode_merge(const float* ws_o, const float* ws_ml, const int32_t* ctx_lens, uint16_t* out, int B,
-                              int H, int Dh, int nparts, int pages_per_part, hipStream_t s);
 int launch_gemm_stream_norm(const uint16_t* W, const uint16_t* bias, void* Y, int ldy, int epi, float* ws,
                             long ws_elems, int N, int K, int ntw, int S, bool reduce, const NormPro& np,
                             hipStream_t s);
@@ -74,6 +63,13 @@ struct RopeOut {
   int H, Hkv, Dh, BS, max_pos;
   int64_t nslots;
 };
+// a lone sequence's attention left in parts (attn_decode_split_kernel, defer): o [parts][K], ml [parts][K / Dh][2], at most max_parts,
+// cut by decode_lone_pages of ctx[0] tokens (max_blocks pages at most) over Hkv heads; o_proj's GEMM merges them (X none)
+struct LoneMerge {
+  const float *o, *ml;
+  const int32_t* ctx;
+  int max_blocks, Hkv, Dh, max_parts;
+};
 struct WaveGemm {
   const uint16_t* X;
   int ldx;
@@ -84,6 +80,7 @@ struct WaveGemm {
   float epi_arg;
   NormPro np;
   RopeOut ro;
+  LoneMerge mg;
 };
 int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream_t st);
 // decode GEMM with weight-only FP8 (e4m3 pre-shuffled tiles + per-row fp32 scale), bf16 activations
@@ -171,15 +168,22 @@ inline int decode_split_places(int B, int Hkv, int max_blocks) {
   const int64_t n = (int64_t)B + DECODE_UNITS / Hkv;
   return (int)(n < wide ? n : wide);
 }
+// Pages of a part of a lone sequence, which every workgroup cuts by itself: 0.63 sqrt(pages), for a page costs 0.75 us and a further part
+// to merge about 0.3 (8000 tokens in parts of 4 / 6 / 8 pages 19.1 / 16.9 / 16.0 us).
+__device__ __forceinline__ int decode_lone_pages(int pages, int Hkv) {
+  const int p = max(DECODE_MIN_PAGES, (int)(0.63f * sqrtf((float)pages) + 0.5f));
+  return max(p, (pages * Hkv + DECODE_UNITS - 1) / DECODE_UNITS);
+}
 int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, DecodePart* plan, hipStream_t s);
-// ws_o [places][H][Dh], ws_ml [places][H][2], tickets [B][Hkv] (zero before and after)
+// ws_o [places][H][Dh], ws_ml [places][H][2], tickets [B][Hkv] (zero before and after); plan none: one sequence of ctx_lens[0] tokens,
+// whose parts stay in ws_o / ws_ml with defer
 int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables, int max_blocks,
-                             const DecodePart* plan, int places, int* tickets, uint16_t* out, float* ws_o, float* ws_ml, int H,
-                             int Hkv, int Dh, float scale, int num_pages, bool nt, hipStream_t s);
+                             const DecodePart* plan, int places, const int32_t* ctx_lens, int* tickets, uint16_t* out, float* ws_o,
+                             float* ws_ml, int H, int Hkv, int Dh, float scale, int num_pages, bool nt, bool defer, hipStream_t s);
 int launch_attn_decode(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                        int max_blocks, const int32_t* ctx_lens, uint16_t* out, float* ws_o, float* ws_ml, int B,
                        int H, int Hkv, int Dh, int pages_per_part, int nparts, float scale, int num_pages, int algo,
-                       hipStream_t s, bool merge = true);
+                       hipStream_t s);
 int launch_attn_prefill(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables,
                         int max_blocks, const int32_t* cu_q, const int32_t* ctx_lens, uint16_t* out, int B,
                         int max_qlen, int H, int Hkv, int Dh, float scale, int num_pages, int algo, hipStream_t s);

@@ -28,7 +28,7 @@ import torch
 from ..inference.shard import Shard
 from ..ops import kernels as K
 from ..ops._ext import require
-from ..ops.linear import (FUSE_MERGE, FUSE_NORM, PendingNorm, keep_order, layout_of, linear, linear_resid_norm, linear_rope_kv,
+from ..ops.linear import (FUSE_MERGE, FUSE_NORM, PendingNorm, keep_order, layout_of, linear, linear_resid_norm, linear_rope_kv, merge_fits,
                           linear_slabs, scratch, stream_rows)
 from ..ops.rope import longrope_window, rope_shift, rope_table
 from .config import ModelConfig
@@ -1167,7 +1167,7 @@ class ShardModel:
                            self.kv.v[j], c.num_heads, c.num_kv_heads, wide=not c.num_experts)
         if isinstance(xn, PendingNorm):
           h = xn.dst
-        a = self._attention(q, j, inp, defer_merge=fuse and FUSE_MERGE and lw.router is None, plan=plan)
+        a = self._attention(q, j, inp, defer_merge=fuse and FUSE_MERGE and merge_fits(lw.o_w), plan=plan)
         if not isinstance(a, K.PendingMerge):  # (a pending merge is finished inside o_proj's prologue)
           a = a.view(h.shape[0], c.num_heads * c.head_dim)
       # o_proj + residual + post-attention norm (one fused pass when the projection runs split-K)

@@ -208,6 +208,7 @@ def choose_pages_per_part(batch: int, Hkv: int, max_ctx: int, algo: int | None =
   return -(-pages // nparts)
 
 
+LONE = object()  # the plan of one sequence
 SPLIT_MIN_PAGES = 8  # widest block table whose contexts are not worth cutting
 
 
@@ -248,8 +249,8 @@ class DecodeWorkspace:
     # rows of split-KV partials: batch * nparts, or the places of a plan (a KV head has at most 16 query heads)
     self.max_batch = max_batch
     self.units = worst  # max over batch of batch * nparts
-    if pages > SPLIT_MIN_PAGES and not routed:
-      worst = max(worst, max_batch + 512 // max(1, -(-H // 16)))
+    if not routed:
+      worst = max(worst, min(max_batch + 512 // max(1, -(-H // 16)), max_batch * -(-pages // 4)))
     self.tickets = torch.zeros(max_batch * H, dtype=torch.int32, device=device)
     self.o = torch.empty(worst * H * Dh, dtype=torch.float32, device=device)
     self.ml = torch.empty(worst * H * 2, dtype=torch.float32, device=device)
@@ -264,34 +265,39 @@ class DecodeWorkspace:
     return ppp, nparts, algo
 
 
-  def plan(self, block_tables: torch.Tensor, ctx_lens: torch.Tensor, Hkv: int) -> torch.Tensor | None:
-    """The units of a decode step's attention (csrc/attention.hip decode_plan_kernel), one launch for all layers of the step; None
-    where attn_decode goes by itself."""
+  def plan(self, block_tables: torch.Tensor, ctx_lens: torch.Tensor, Hkv: int):
+    """The units of a decode step's attention (csrc/attention.hip decode_plan_kernel), one launch for all layers of the step; LONE for
+    one sequence, which needs none; None where attn_decode goes by itself."""
     B, width = ctx_lens.shape[0], block_tables.shape[1]
-    if (not block_tables.is_cuda or self.fixed_ppp or B > self.max_batch or not plan_pays(B, Hkv, width) or self.Dh not in (64, 128)
-        or resolve_decode_algo(B, Hkv, self.algo, routed=self.routed) not in (2, 3)):
+    if not block_tables.is_cuda or self.fixed_ppp or self.routed or B > self.max_batch or self.Dh not in (64, 128):
+      return None
+    if B == 1 and self.algo == -1 and width * Hkv < 1 << 30:
+      return LONE
+    if not plan_pays(B, Hkv, width) or resolve_decode_algo(B, Hkv, self.algo) not in (2, 3):
       return None
     return require().decode_plan(ctx_lens, B, Hkv, width)
 
 
 class PendingMerge:
-  """A batch-1 split-KV decode attention whose partition merge was left to its consumer: o_proj merges the
-  partitions of its K slice in its GEMM prologue (linear_resid_norm -> gemm_stream_merge), one launch less per
-  layer.  materialize() runs the merge kernel into `out` instead."""
+  """A lone sequence's decode attention in parts whose merge was left to its consumer: o_proj merges what its workgroups multiply in
+  its prologue (linear_resid_norm -> gemm_solo_merge), instead of the last workgroup of the attention."""
 
-  __slots__ = ("o", "ml", "ctx_lens", "ppp", "nparts", "out")
+  __slots__ = ("o", "ml", "ctx_lens", "width", "Hkv", "Dh")
 
-  def __init__(self, o, ml, ctx_lens, ppp, nparts, out):
-    self.o, self.ml, self.ctx_lens, self.ppp, self.nparts, self.out = o, ml, ctx_lens, ppp, nparts, out
+  def __init__(self, o, ml, ctx_lens, width, Hkv, Dh):
+    self.o, self.ml, self.ctx_lens, self.width, self.Hkv, self.Dh = o, ml, ctx_lens, width, Hkv, Dh
 
-  def materialize(self) -> torch.Tensor:
-    require().attn_decode_merge(self.o, self.ml, self.ctx_lens, self.out, self.ppp, self.nparts)
-    return self.out
+
+# Block tables whose parts (2 to 4) the output projection merges: in its prologue they cost it 0.5 us, or 1 us of 8 layers of 4096
+# columns, whatever the context; the attention's last workgroup takes 2 to 3 us, but only where there is more than one part.  us a step
+# of Llama-3.2-1B / Llama-3-8B (8 layers), left / merged there: 60 tokens 644 / 636 and 835 / 828, 400 664 / 677 and 856 / 862 (8 pages
+# both), 600 678 / 687 and 864 / 866, 2000 695 / 699 and 881 / 872
+MERGE_PAGES = (9, 16)
 
 
 def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, ws: DecodeWorkspace | None = None,
-                out: torch.Tensor | None = None, defer_merge: bool = False, plan: torch.Tensor | None = None):
-  """defer_merge (one sequence): return a PendingMerge when the context is split over partitions.  plan: ws.plan of the same step."""
+                out: torch.Tensor | None = None, defer_merge: bool = False, plan=None):
+  """plan: ws.plan of the same step.  defer_merge (plan LONE, MERGE_PAGES wide): return a PendingMerge."""
   if not _gpu(q):
     y = ref.attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale)
     if out is not None:
@@ -305,13 +311,14 @@ def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale: float, ws: D
   out = torch.empty_like(q) if out is None else out
   if plan is not None:
     nt = B * k_cache.shape[1] * width * PAGE * Dh * 4 >= NT_MIN_KV_BYTES
-    require().attn_decode_split(q, k_cache, v_cache, block_tables, plan, ws.tickets, out, ws.o, ws.ml, float(scale), nt)
-    return out
+    lone = plan is LONE
+    defer = defer_merge and lone and MERGE_PAGES[0] <= width <= MERGE_PAGES[1]
+    require().attn_decode_split(q, k_cache, v_cache, block_tables, None if lone else plan, ctx_lens, ws.tickets, out, ws.o, ws.ml,
+                                float(scale), nt, defer)
+    return PendingMerge(ws.o, ws.ml, ctx_lens, width, k_cache.shape[1], Dh) if defer else out
   ppp, nparts, algo = ws.partition(B, k_cache.shape[1], width)
-  defer = defer_merge and B == 1 and nparts > 1
-  require().attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, ws.o, ws.ml, ppp, nparts, float(scale),
-                        algo, not defer)
-  return PendingMerge(ws.o, ws.ml, ctx_lens, ppp, nparts, out) if defer else out
+  require().attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, ws.o, ws.ml, ppp, nparts, float(scale), algo)
+  return out
 
 
 # XOT_PREFILL_ATTN: 2 = 256-row workgroups, LDS-DMA page ring, in-register softmax (default); 1 = the

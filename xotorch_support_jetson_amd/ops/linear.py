@@ -59,6 +59,9 @@ STREAM_MAX_M = int(os.environ.get("XOT_STREAM_MAX_M", "512"))
 WAVE_MAX_M = 16
 # ... and at all (its row tiles; a chunk of X for more would not fit beside a second workgroup's)
 WIDE_MAX_M = 64
+# largest M for which the whole-K GEMM of single column tiles (csrc/gemm_wave.hip gemm_solo_kernel, code ("wave", 0, 1)) is a candidate:
+# us in slabs / whole, with the norm behind them, of 2048 x 5632 at 2 rows 10.3 / 8.6, 4 10.7 / 9.7, 6 10.8 / 10.3, 9 10.9 / 11.2
+SOLO_MAX_M = 8
 # smallest M for which gemm_big is a candidate, and for which its 64-row tiles are (XOT_BIG_MIN_M: no gemm_big below that)
 BIG_MIN_M, ROWS64_MIN_M = (int(os.environ.get("XOT_BIG_MIN_M", m)) for m in ("65", "17"))
 
@@ -89,6 +92,11 @@ def tile_width(code: int) -> int:
 
 def tile_rows(code: int) -> int:
   return code // 10000 or 256
+
+
+def solo_fits(M: int, N: int, Kd: int) -> bool:
+  """Shapes of the whole-K GEMM of single column tiles that leave no CU with more than a tile (two column halves of 2048 and fewer)."""
+  return M <= SOLO_MAX_M and N % 16 == 0 and N <= 4096 and Kd % 128 == 0
 
 
 def layout_of(w: torch.Tensor) -> str:
@@ -453,13 +461,14 @@ class GemmPolicy:
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
     reduce, timed with them, stands for the launch that does it there).  slabs: the caller's consumer reads split-K slabs
     itself, so a split is timed without their reduce (2048 x 5632 at 6 rows: 9.1 us whole, 6.4 in 11 slabs, 10.2 with the reduce).
-    run(cfg): what the caller does with a choice, where launches of its own that depend on it follow; timed in the GEMM's place."""
+    run(cfg): what the caller does with a choice, where launches of its own that depend on it follow; timed in the GEMM's place.
+    wave "solo": the caller takes the whole-K GEMM of single column tiles too."""
     M, Kd = x.shape
     N = w.shape[0]
     wave = wave if M <= WIDE_MAX_M and (out_dtype == torch.bfloat16 or epi == "none") else ""
     # (a residual product's plain entry belongs to linear_resid_norm, which sums the slabs itself; a caller that does not
     # take the whole-K GEMM passes over such an entry)
-    kind = "sl" if slabs else "sh" + wave if wave == "rope" or epi == "resid" else "sh"
+    kind = "sl" if slabs else "sh" + wave if wave in ("rope", "solo") or epi == "resid" else "sh"
     kept = getattr(w, "xot_keep_order", False)
     if kept and WAVE_MAX_M < M <= 256:
       kind += "o"
@@ -491,6 +500,8 @@ class GemmPolicy:
     cands = []
     if M <= STREAM_MAX_M and epi != "gelu_glu":
       cands += [("stream",) + c for c in self._stream_cands(M, N, Kd, epi)]
+    if (wave == "solo" or slabs and N >= 1024) and solo_fits(M, N, Kd):  # (fewer columns keep fewer than half of the CUs; slabs, all)
+      cands.append(("wave", 0, 1))
     if wave and epi != "gelu_glu" and not (kept and M > WAVE_MAX_M):
       cands += self._wave_cands(M, N, Kd, epi, wave == "rope") or self._wide_cands(M, N, Kd, epi, wave == "rope")
     if epi not in ("clamp_glu", "relu2", "gelu_glu") and Kd % 128 == 0 and not kept:
@@ -509,6 +520,8 @@ class GemmPolicy:
       try:
         call = _slab_call if slabs and cfg[2] > 1 else _shuffled_call
         times[cfg] = self._time(lambda: run(cfg) if run else call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
+        if slabs and cfg[2] > 1 and M <= SOLO_MAX_M:
+          times[cfg] += 1e-4 * cfg[2]  # a row's reader waits about 0.1 us for each slab more (11 of 2048 columns 1.0 us, of 6 rows 1.5)
       except RuntimeError:
         pass
     got = _tie_break(times, 0 if kept and M <= 128 else M) if times else cands[0]
@@ -697,23 +710,23 @@ def _blas(x, w, bias, residual, epi, out, out_dtype):
   return y
 
 
-# XOT_FUSE_NORM=0: batch-1 decode keeps the separate split-K reduce + residual + RMSNorm launch after o_proj /
-# down_proj (fused: the next GEMM recomputes the norm of the pending slabs in its prologue, csrc/gemm.hip NORM)
+# XOT_FUSE_NORM=0: batch-1 decode keeps the RMSNorm launch after o_proj / down_proj (fused: the next GEMM computes the norm
+# in its prologue)
 FUSE_NORM = os.environ.get("XOT_FUSE_NORM", "1") != "0"
-# XOT_FUSE_MERGE=0: batch-1 decode keeps the attention's partition-merge launch (fused: o_proj merges the partitions
-# of its K slice in its prologue, csrc/gemm.hip MERGE; only together with the deferred norm above)
+# XOT_FUSE_MERGE=0: batch-1 decode merges the attention's parts in its own launch (fused: o_proj merges what its workgroups multiply
+# in their prologue; only together with the deferred norm above)
 FUSE_MERGE = os.environ.get("XOT_FUSE_MERGE", "1") != "0"
-# widest residual row whose norm is deferred: every consumer workgroup re-reads the row and all its slabs, which paid
+# widest residual row whose norm is deferred: every consumer workgroup re-reads the row, which paid
 # at 4096 (Llama-3-8B 3.50 -> 3.33 ms/token) but not at 8192 (Llama-3-70B 23.97 vs 24.07 ms, profiles/r6/headline/b1/)
 DEFER_MAX_D = 4096
 
 
 class PendingNorm:
-  """rmsnorm(bf16(src + bias + sum of the S fp32 slabs in ws)) * ln_w, not computed yet.
+  """rmsnorm(bf16(src + bias + sum of the S fp32 slabs in ws)) * ln_w, not computed yet (S 0: rmsnorm(src) * ln_w).
 
-  A residual projection of a batch-1 decode step (linear_resid_norm with defer_to) leaves its split-K slabs; the
-  next GEMM (linear with epi none / silu, linear_rope_kv) folds the slab sum, the residual add and the RMSNorm into
-  its prologue (gemm_stream_norm) and stores the summed residual row into dst -- a buffer distinct from src, since
+  A residual projection of a batch-1 decode step (linear_resid_norm with defer_to) leaves its norm; the
+  next GEMM (linear with epi none / silu, linear_rope_kv) folds the RMSNorm, and the sum of slabs if there are any, into
+  its prologue (gemm_wave, gemm_stream_norm) and stores the summed residual row into dst -- a buffer distinct from src, since
   every workgroup of that GEMM reads src.  Any other consumer calls materialize(), the unfused kernel, which
   leaves the same residual in dst.  After either, dst is the residual stream."""
 
@@ -727,6 +740,9 @@ class PendingNorm:
     return self.src.shape
 
   def materialize(self) -> torch.Tensor:
+    if self.S == 0:  # (the product summed by itself)
+      self.dst.copy_(self.src)
+      return K.rmsnorm(self.dst, self.ln_w, self.eps)[0]
     if self.dst.data_ptr() != self.src.data_ptr():
       self.dst.copy_(self.src)
     out = torch.empty_like(self.dst)
@@ -811,6 +827,18 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0, once: bool = T
 
 
 
+def merge_fits(w: torch.Tensor) -> bool:
+  """Whether o_proj (its weight w) merges a lone sequence's attention parts itself: two chunks of K, single column tiles."""
+  return layout_of(w) == "stream" and w.dtype == torch.bfloat16 and solo_fits(1, *w.shape) and w.shape[1] <= 4096
+
+
+def _solo_norm(h, ln_w, eps, defer_to):
+  """The norm behind a whole-K residual product of one row: left to the next GEMM (its residual stream in defer_to), or run."""
+  if defer_to is not None and FUSE_NORM and h.shape[1] <= DEFER_MAX_D:
+    return PendingNorm(h, defer_to, None, 0, None, ln_w, eps)
+  return K.rmsnorm(h, ln_w, eps)[0]
+
+
 def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: torch.Tensor, eps: float,
                       bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
                       defer_to: torch.Tensor | None = None):
@@ -818,39 +846,46 @@ def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: t
 
   When the projection runs split-K on the pre-shuffled layout, the GEMM leaves its fp32 slabs and one
   kernel does the slab reduce, the residual add and the RMSNorm (instead of reduce + norm kernels).
-  defer_to (a second residual buffer, one row): return a PendingNorm instead -- the slabs stay for the next
-  GEMM's prologue, and the residual stream continues in defer_to (h is left as it was).
-  x may be a kernels.PendingMerge (batch-1 decode attention): with defer_to, the projection merges the attention's
-  partitions in its own prologue (gemm_stream_merge); otherwise the merge kernel runs first."""
+  defer_to (a second residual buffer, one row): return a PendingNorm instead -- the norm is left to the next
+  GEMM's prologue, and the residual stream continues in defer_to (a copy of the summed h).
+  x may be a kernels.PendingMerge (a lone sequence's decode attention), where merge_fits(w): the projection merges the
+  attention's parts in its own prologue."""
   if isinstance(x, K.PendingMerge):
-    xm = x.out.view(x.out.shape[0], -1)  # [1, H * Dh]; the stand-in operand of the configuration choice
-    if defer_to is not None and FUSE_NORM and layout_of(w) == "stream" and xm.shape[0] == 1:
-      N, Kd = w.shape
-      cfg = policy.shuffled_cfg(xm, w, bias, h, "resid", h.dtype)
-      if (cfg[0] == "stream" and 1 < cfg[2] <= 8 and Kd % (cfg[2] * 128) == 0 and (Kd // cfg[2]) * 2 <= 65536
-          and h.is_contiguous() and h.dtype == torch.bfloat16):
-        S = cfg[2]
-        if N <= DEFER_MAX_D and out is None:  # merge here, norm in the next GEMM's prologue
-          ws = scratch.splitk(h.device, S * N, slot=1)
-          require().gemm_stream_merge(w, ws, cfg[1], S, x.o, x.ml, x.ctx_lens, x.ppp, x.nparts, x.out.shape[-1])
-          return PendingNorm(h, defer_to, ws, S, bias, ln_w, eps)
-        ws = scratch.splitk(h.device, S * N)  # merge here, then the usual slab reduce + residual + norm
-        require().gemm_stream_merge(w, ws, cfg[1], S, x.o, x.ml, x.ctx_lens, x.ppp, x.nparts, x.out.shape[-1])
-        out = torch.empty_like(h) if out is None else out
-        require().splitk_resid_rmsnorm(ws, S, bias, h, ln_w, out, float(eps))
-        return out
-    x = x.materialize().view(xm.shape)
+    if not (merge_fits(w) and out is None and h.is_contiguous()):
+      raise RuntimeError("a pending merge is for output projections that merge_fits")
+    require().gemm_solo_merge(w, h, bias, x.o, x.ml, x.ctx_lens, x.width, x.Hkv, x.Dh)
+    return _solo_norm(h, ln_w, eps, defer_to)
   if x.is_cuda and layout_of(w) == "stream":
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     M, N = x.shape[0], w.shape[0]
+    inner = out is None and h.is_contiguous() and h.dtype == x.dtype == torch.bfloat16
+    if M == 1 and inner and solo_fits(M, N, w.shape[1]):
+      # one row: the whole sum in one launch.  Every workgroup of the next GEMM would read the slabs in its prologue, which costs
+      # it 1.3 to 2.4 us for 8 of 2048 columns; product in 8 slabs / whole, us: 2048 x 2048 3.75 / 3.84, 2048 x 8192 8.5 / 7.9,
+      # 4096 x 4096 8.2 / 8.1, 4096 x 14336 20.7 / 20.6
+      require().gemm_wave(x, w, h, bias, h, K.EPI["resid"], 0)
+      return _solo_norm(h, ln_w, eps, defer_to)
+
+    def run(cfg, h):
+      if cfg[2] > 1:
+        ws = scratch.splitk(x.device, cfg[2] * M * N)
+        (require().gemm_stream(x, w, h, None, h, ws, K.EPI["resid"], cfg[1], cfg[2], True, False) if cfg[0] == "stream" else
+         require().gemm_big(x, w, h, None, h, ws, K.EPI["resid"], cfg[1], cfg[2], False))
+        y = torch.empty_like(h) if out is None else out
+        require().splitk_resid_rmsnorm(ws, cfg[2], bias, h, ln_w, y, float(eps))
+        return y
+      _shuffled_call(x, w, bias, h, "resid", h, cfg)
+      return K.rmsnorm(h, ln_w, eps, out=out)[0]
+    if inner and M <= SOLO_MAX_M and solo_fits(M, N, w.shape[1]):
+      # a handful of rows: timed with the norm that follows (of 4 rows us in 11 slabs / whole: 2048 x 5632 6.8 + 3.9 / 6.8 + 2.9)
+      tmp = []
+
+      def timed(cfg):
+        tmp or tmp.append(h.clone())
+        return run(cfg, tmp[0])
+      return run(policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype, wave="solo", run=timed), h)
     cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype)
-    if (defer_to is not None and FUSE_NORM and M == 1 and cfg[0] == "stream" and 1 < cfg[2] <= 8 and N <= DEFER_MAX_D
-        and out is None and h.is_contiguous() and h.dtype == torch.bfloat16):
-      S = cfg[2]
-      ws = scratch.splitk(x.device, S * M * N, slot=1)
-      require().gemm_stream(x, w, h, None, h, ws, K.EPI["resid"], cfg[1], S, True, False)
-      return PendingNorm(h, defer_to, ws, S, bias, ln_w, eps)
     if cfg[0] in ("stream", "big") and cfg[2] > 1 and (M < W4_PREF_M or h.is_contiguous()):
       S = cfg[2]
       ws = scratch.splitk(x.device, S * M * N)
