@@ -265,9 +265,15 @@ __global__ void conv_tail_k(const float* __restrict__ P, int ldp, int S, int64_t
 
 // ------------------------------------------------------------------ gates
 // Workgroup = (GTOK tokens, job): job 0 the step sizes beta, then blocks of 64 decay channels, then blocks of 64 output-gate
-// channels.  The tokens' rank rows lie in LDS; four neighbouring lanes share a channel, each sums a quarter of its weight row
-// (in pieces of eight) for all the tokens.
-constexpr int GTOK = 8;
+// channels.  The tokens' rank rows lie in LDS; a wave multiplies them with the weight rows of 16 channels on the fp32 matrix unit
+// (ranks of whole eights; else four neighbouring lanes share a channel, each sums a quarter of its weight row).  Bound by
+// latencies: launch, the rank rows' way through LDS, the products.  With a channel's products on the vector unit, every lane reading
+// all tokens' rows out of LDS again, 6 tokens, two 2048 x 128 products: 10.0 us, 7.0 here; with the convolutions in one launch 9.0, 6.5.
+constexpr int GTOK = 16;
+constexpr int DTOK = 8;  // tokens a thread of channel_decay_k
+// the rank rows in LDS: whole 32s; consecutive tokens four banks apart (but for the longest, which 64 KB just hold)
+__host__ __device__ inline int gate_row(int rank) { return (rank + 31) & ~31; }
+__host__ __device__ inline int gate_ld(int rank) { return gate_row(rank) + (rank > 992 ? 0 : 4); }
 
 struct GateArgs {
   const float* P;
@@ -288,7 +294,7 @@ struct GateArgs {
 };
 
 template <typename WT>
-__device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, float* ys) {  // ys: LDS [GTOK][rank]
+__device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, float* ys) {  // ys: LDS [GTOK][gate_ld(rank)]
   const float* __restrict__ P = A.P;
   const WT* __restrict__ a2 = (const WT*)A.a2;
   const WT* __restrict__ g2 = (const WT*)A.g2;
@@ -311,86 +317,93 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
   }
   --job;
   const bool dec = job < nab;
-  const int part = threadIdx.x & 3, c = (dec ? job : job - nab) * 64 + (threadIdx.x >> 2), nc = dec ? HD : ng;
-  const int rank = dec ? ra : rg, off = dec ? a1_off : g1_off;
+  const int rank = dec ? ra : rg, off = dec ? a1_off : g1_off, ld = gate_ld(rank), nc = dec ? HD : ng, c0 = (dec ? job : job - nab) * 64;
+  const bool whole = (rank & 7) == 0;
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  const int part = threadIdx.x & 3, c = c0 + (whole ? (threadIdx.x >> 6) * 16 + (lane & 15) : threadIdx.x >> 2);
   const WT* w = (dec ? a2 : g2) + (int64_t)min(c, nc - 1) * rank;
   const float rate = dec ? expf(A_log[min(c, nc - 1) / d]) : 0.0f, bias = dec ? dt_bias[min(c, nc - 1)] : 0.0f;
   // the first four pieces of the lane's weight row are on their way while the rank rows are summed
-  const bool pieces = (rank & 7) == 0;
   float wv[4][8];
-  if (pieces) {
+  if (whole) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ld8(w + min(8 * part + 32 * k, rank - 8), wv[k]);
+    for (int k = 0; k < 4; ++k) ld8(w + min(8 * g + 32 * k, rank - 8), wv[k]);
   }
-  // the rank rows: four elements a thread and eight slabs in flight at a time, without branches around the loads
-  const int ne = GTOK * rank;
-  for (int e0 = 0; e0 < ne; e0 += 1024) {
-    const float* p[4];
-    float v[4];
+  // the rank rows (zeros up to whole 32s): four elements a thread and eight slabs in flight at a time, without branches around the loads
+  const int rows = nt <= 8 ? 8 : GTOK, row = gate_row(rank);
+  for (int i0 = 0; i0 < rows; i0 += 8) {  // 32 lanes a token
+    const int i = i0 + (threadIdx.x >> 5);
+    const float* p = P + (int64_t)(t0 + min(i, nt - 1)) * ldp + off;
+    for (int r0 = threadIdx.x & 31; r0 < row; r0 += 128) {
+      float v[4];
+      int r[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = min(e0 + (int)threadIdx.x + 256 * j, ne - 1), i = e / rank;
-      p[j] = P + (int64_t)(t0 + min(i, nt - 1)) * ldp + off + e - i * rank;
-      v[j] = 0.0f;
-    }
-    if (S == 1) {
+      for (int j = 0; j < 4; ++j) {
+        r[j] = min(r0 + 32 * j, rank - 1);
+        v[j] = 0.0f;
+      }
+      if (S == 1) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = *p[j];
-    }
-    for (int k0 = 0; S > 1 && k0 < S; k0 += 8) {
-      float a[8][4];
+        for (int j = 0; j < 4; ++j) v[j] = p[r[j]];
+      }
+      for (int k0 = 0; S > 1 && k0 < S; k0 += 8) {
+        float a[8][4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < 8; ++k)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a[k][j] = p[j][min(k0 + k, S - 1) * ss];
+          for (int j = 0; j < 4; ++j) a[k][j] = p[min(k0 + k, S - 1) * ss + r[j]];
 #pragma unroll
-      for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < 8; ++k)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += k0 + k < S ? a[k][j] : 0.0f;
-    }
+          for (int j = 0; j < 4; ++j) v[j] += k0 + k < S ? a[k][j] : 0.0f;
+      }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = e0 + threadIdx.x + 256 * j;
-      if (e < ne) ys[e] = v[j];
+      for (int j = 0; j < 4; ++j)
+        if (r0 + 32 * j < row) ys[i * ld + r0 + 32 * j] = r0 + 32 * j < rank ? v[j] : 0.0f;
     }
   }
   __syncthreads();
-  float z[GTOK];
+  auto put = [&](int i, float z) {  // token t0 + i of channel c
+    if (c >= nc || i >= nt) return;
+    if (dec) decay[(int64_t)(t0 + i) * HD + c] = expf(-rate * softplusf_(z + bias));
+    else gate[(int64_t)(t0 + i) * ng + c] = z;
+  };
+  if (whole) {
+    // k runs as the lanes' pieces lie: step e of a block of 32 multiplies k = 8 g + e of lane group g
+    f32x4 z[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const float* yr = ys + (lane & (rows - 1)) * ld + 8 * g;  // (MFMA rows past the tokens repeat them)
+    auto add = [&](const float* v, int r) {  // r: the block's first k
+      const f32x4 a = *reinterpret_cast<const f32x4*>(yr + r), b = *reinterpret_cast<const f32x4*>(yr + r + 4);
+      const bool in = r + 8 * g < rank;
 #pragma unroll
-  for (int i = 0; i < GTOK; ++i) z[i] = 0.0f;
-  if (pieces) {
-    auto add = [&](const float* v, int r) {
-#pragma unroll
-      for (int i = 0; i < GTOK; ++i) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(ys + i * rank + r), b = *reinterpret_cast<const f32x4*>(ys + i * rank + r + 4);
-        z[i] += v[0] * a[0] + v[1] * a[1] + v[2] * a[2] + v[3] * a[3] + v[4] * b[0] + v[5] * b[1] + v[6] * b[2] + v[7] * b[3];
-      }
+      for (int e = 0; e < 8; ++e)
+        z[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(e < 4 ? a[e & 3] : b[e & 3], in ? v[e] : 0.0f, z[e & 1], 0, 0, 0);
     };
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-      if (8 * part + 32 * k < rank) add(wv[k], 8 * part + 32 * k);
-    for (int r = 8 * part + 128; r < rank; r += 32) {
+      if (32 * k < rank) add(wv[k], 32 * k);
+    for (int r = 128; r < rank; r += 32) {
       float v[8];
-      ld8(w + r, v);
+      ld8(w + min(r + 8 * g, rank - 8), v);
       add(v, r);
     }
-  } else {
-    for (int r = part; r < rank; r += 4) {
-      const float v = ldf(w + r);
+    const f32x4 t = z[0] + z[1];  // lane (g, channel): tokens 4 g + r
 #pragma unroll
-      for (int i = 0; i < GTOK; ++i) z[i] += v * ys[i * rank + r];
-    }
+    for (int r = 0; r < 4; ++r) put(4 * g + r, t[r]);
+    return;
+  }
+  float z[GTOK];
+#pragma unroll
+  for (int i = 0; i < GTOK; ++i) z[i] = 0.0f;
+  for (int r = part; r < rank; r += 4) {
+    const float v = ldf(w + r);
+#pragma unroll
+    for (int i = 0; i < GTOK; ++i) z[i] += v * ys[(i & (rows - 1)) * ld + r];
   }
 #pragma unroll
   for (int i = 0; i < GTOK; ++i) {
     z[i] = quad_sum(z[i]);
-  }
-  if (c >= nc) return;
-#pragma unroll
-  for (int i = 0; i < GTOK; ++i) {
-    if (i >= nt || (i & 3) != part) continue;  // (the four lanes of a channel share the writes)
-    if (dec) decay[(int64_t)(t0 + i) * HD + c] = expf(-rate * softplusf_(z[i] + bias));
-    else gate[(int64_t)(t0 + i) * ng + c] = z[i];
+    if ((i & 3) == part) put(i, z[i]);  // (the four lanes of a channel share the writes)
   }
 }
 
@@ -406,7 +419,7 @@ __global__ __launch_bounds__(256) void channel_decay_k(const float* __restrict__
                                                        float* __restrict__ beta, int H, const float* __restrict__ za, int ldz,
                                                        const float* __restrict__ dt_bias, const float* __restrict__ A_log, int d,
                                                        float* __restrict__ decay) {
-  const int t0 = blockIdx.x * GTOK, nt = min(GTOK, T - t0), HD = H * d;
+  const int t0 = blockIdx.x * DTOK, nt = min(DTOK, T - t0), HD = H * d;
   if (blockIdx.y == 0) {
     for (int e = threadIdx.x; e < nt * H; e += 256) {
       const int t = t0 + e / H, h = e % H;
@@ -416,20 +429,20 @@ __global__ __launch_bounds__(256) void channel_decay_k(const float* __restrict__
   }
   const int c = ((blockIdx.y - 1) * 256 + threadIdx.x) * W;
   if (c >= HD) return;  // (W > 1: HD is a multiple of W)
-  float rate[W], bias[W], z[GTOK][W];
+  float rate[W], bias[W], z[DTOK][W];
 #pragma unroll
   for (int e = 0; e < W; ++e) {
     rate[e] = -expf(A_log[(c + e) / d]);
     bias[e] = dt_bias[c + e];
   }
 #pragma unroll
-  for (int i = 0; i < GTOK; ++i) {
+  for (int i = 0; i < DTOK; ++i) {
     const float* p = za + (int64_t)(t0 + min(i, nt - 1)) * ldz + c;
     if constexpr (W == 4) *reinterpret_cast<f32x4*>(z[i]) = *reinterpret_cast<const f32x4*>(p);
     else z[i][0] = *p;
   }
 #pragma unroll
-  for (int i = 0; i < GTOK; ++i) {
+  for (int i = 0; i < DTOK; ++i) {
     if (i >= nt) continue;
 #pragma unroll
     for (int e = 0; e < W; ++e) z[i][e] = expf(rate[e] * softplusf_(z[i][e] + bias[e]));
@@ -579,7 +592,7 @@ GateArgs gate_args(const Slabs& p, int64_t b_off, at::Tensor& beta, int64_t a1_o
   return a;
 }
 inline unsigned gate_jobs(const GateArgs& a) { return (unsigned)(1 + (a.H * a.d + 63) / 64 + (a.ng + 63) / 64); }
-inline size_t gate_lds(const GateArgs& a) { return (size_t)GTOK * std::max(a.ra, a.rg) * sizeof(float); }
+inline size_t gate_lds(const GateArgs& a) { return (size_t)GTOK * gate_ld(std::max(a.ra, a.rg)) * sizeof(float); }
 
 StepArgs step_args(const Slabs& p, int64_t dt_off, const at::Tensor& dt_bias, const at::Tensor& A_log, at::Tensor& dt, at::Tensor& decay,
                    int64_t b_off = -1) {
@@ -706,7 +719,7 @@ void recurrence_gates(const at::Tensor& P, int64_t b_off, at::Tensor& beta, int6
     const bool vec = HD % 4 == 0 && ldz % 4 == 0 && (reinterpret_cast<uintptr_t>(za->data_ptr()) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(decay.data_ptr()) & 15) == 0;
     const int64_t per = vec ? 1024 : 256;
-    const dim3 grid((unsigned)((T + GTOK - 1) / GTOK), (unsigned)(1 + (HD + per - 1) / per));
+    const dim3 grid((unsigned)((T + DTOK - 1) / DTOK), (unsigned)(1 + (HD + per - 1) / per));
 #define CD_GO(W)                                                                                                             \
   channel_decay_k<W><<<grid, 256, 0, stream()>>>(p.p, p.ld, p.S, p.ss, (int)T, (int)b_off, beta.data_ptr<float>(), (int)H,   \
                                                  za->data_ptr<float>(), ldz, dt_bias.data_ptr<float>(),                      \
