@@ -397,6 +397,124 @@ __global__ void attn_split_sum_k(const float* __restrict__ part, int KS, int T, 
   stf(out + (int64_t)t * ldo + i, o * out_scale);
 }
 
+// Steps of single tokens (bf16, d = 32 NK, at most 16 query heads a kv head): workgroup = (sequence, kv head), its waves take the pages
+// of the token's chunk in turn and meet in LDS.  Scores as S^T = K Q^T, so a lane's accumulators are four consecutive keys of one
+// query head; the weights, fp32 as they are, enter O^T += V^T P^T as three bf16 terms that sum to them exactly (8 bits of the
+// mantissa each), so a product costs three MFMA steps and keeps what fp32 had.  Bound by latencies (table, pages, merge).  On the vector
+// unit, in up to eight key splits and with a launch that added them, 48 tokens x 4 kv heads of 128, contexts of 60 to 110: 9.5 + 4.7
+// us, 6.4 here; 1000 tokens each 42.1 / 24.9, 200 tokens of contexts 30 to 160 29.2 / 16.0, one of 40 10.1 / 5.2, one of 1000 18.7 both.
+template <int NK, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void attn_gated_step_k(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    const int* __restrict__ block_tables, int width, const int* __restrict__ ctx_lens, const float* __restrict__ pb, float scale, int chunk,
+    float out_scale, uint16_t* __restrict__ out, int ldo, int H, int G) {
+  constexpr int D = NK * 32, ND = NK * 2, LD = D + 4;
+  extern __shared__ __attribute__((aligned(16))) float sm[];  // [NW][hpg][LD]
+  const int b = blockIdx.x, kvh = blockIdx.y, hpg = H / G;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const int ctx = ctx_lens[b];
+  if (ctx <= 0) return;  // padding row of a captured decode batch
+  const int pos = ctx - 1, lo = pos / chunk * chunk, last = pos / PAGE_TOK;
+  const int* bt = block_tables + (int64_t)b * width;
+  const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int hq = kvh * hpg + min(c, hpg - 1);
+  s16x8 qf[NK], kf[4][NK];
+  auto load_k = [&](int p) {
+    const uint16_t* kb = k_cache + ((int64_t)bt[p] * G + kvh) * PAGE_TOK * D + 8 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // row c of score tile j: key 32 (j / 2) + 8 (c / 4) + 4 (j % 2) + c % 4
+      const int r = 32 * (j >> 1) + 8 * (c >> 2) + 4 * (j & 1) + (c & 3);
+#pragma unroll
+      for (int s = 0; s < NK; ++s) kf[j][s] = ld16(kb + r * D + 32 * s);
+    }
+  };
+  int p = lo / PAGE_TOK + wave;
+  if (p <= last) load_k(p);
+#pragma unroll
+  for (int s = 0; s < NK; ++s) {
+    const s16x8 v = ld16(q + ((int64_t)b * H + hq) * D + 8 * g + 32 * s);
+    qf[s] = c < hpg ? v : zero;
+  }
+  const float bias = pb[hq];
+  f32x4 o[ND];
+#pragma unroll
+  for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (; p <= last; p += NW) {
+    const uint16_t* vb = v_cache + ((int64_t)bt[p] * G + kvh) * PAGE_TOK * D + 8 * g;
+    s16x8 vf[ND][2];
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) vf[dt][kk] = ld16(vb + (16 * dt + c) * PAGE_TOK + 32 * kk);
+    f32x4 st[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      st[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < NK; ++s) st[j] = mfma16(kf[j][s], qf[s], st[j]);
+    }
+    if (p + NW <= last) load_k(p + NW);
+    const int key0 = p * PAGE_TOK + 8 * g;
+    s16x8 pf[2][3];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      u32x4 t[3];
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        uint32_t u[2][3];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const int key = key0 + 32 * kk + e + x;
+          const float v = key >= lo && key <= pos ? sigmoidf_(st[2 * kk + (e >> 2)][(e + x) & 3] * scale + bias) : 0.0f;
+          const float r1 = v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
+          const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+          u[x][0] = __float_as_uint(v);
+          u[x][1] = __float_as_uint(r1);
+          u[x][2] = __float_as_uint(r2);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) t[i][e >> 1] = __builtin_amdgcn_perm(u[1][i], u[0][i], 0x07060302u);  // the upper halves
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) pf[kk][i] = __builtin_bit_cast(s16x8, t[i]);
+    }
+    if (p == last) {  // slots past the token may hold anything: zeros
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const int left = pos + 1 - (key0 + 32 * kk);  // keys of the lane's eight that are there
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e >= left) {
+#pragma unroll
+            for (int dt = 0; dt < ND; ++dt) vf[dt][kk][e] = 0;
+          }
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 2; i >= 0; --i)
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) o[dt] = mfma16(vf[dt][kk], pf[kk][i], o[dt]);
+  }
+  if (c < hpg) {
+    float* mine = sm + (wave * hpg + c) * LD + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) *reinterpret_cast<f32x4*>(mine + 16 * dt) = o[dt];
+  }
+  __syncthreads();
+  for (int e = 4 * threadIdx.x; e < hpg * D; e += 4 * 64 * NW) {
+    const int h = e / D, i = e - h * D;
+    f32x4 v = *reinterpret_cast<const f32x4*>(sm + h * LD + i);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const f32x4*>(sm + (w * hpg + h) * LD + i);
+    s16x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = (short)f2bf(v[r] * out_scale);
+    *reinterpret_cast<s16x4*>(out + (int64_t)b * ldo + (kvh * hpg + h) * D + i) = y;
+  }
+}
+
 // MFMA kernel (bf16, d = 32 NK): a workgroup owns 128 consecutive queries of one (sequence, head), 32 per wave, and
 // walks the keys of their chunk(s) a tile of KT keys at a time: the K rows and V^T runs of the tile are staged in LDS
 // with whole-line loads and shared by the four waves.  Scores are computed transposed, S^T = K Q^T (keys x queries),
@@ -1006,6 +1124,28 @@ void attn_gated_chunk(const at::Tensor& q, const at::Tensor& k_cache, const at::
       ATT_CASE(1) ATT_CASE(2) ATT_CASE(3) ATT_CASE(4) ATT_CASE(5) ATT_CASE(6) ATT_CASE(7) ATT_CASE(8)
     }
 #undef ATT_CASE
+    return;
+  }
+  if (bf && max_qlen == 1 && T == B && d % 32 == 0 && d <= 128 && H / G <= 16 && ldo % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 &&
+      ((reinterpret_cast<uintptr_t>(q.data_ptr()) | reinterpret_cast<uintptr_t>(k_cache.data_ptr()) | reinterpret_cast<uintptr_t>(v_cache.data_ptr())) & 15) == 0) {
+    // eight waves where the (sequence, kv head) pairs leave CUs idle: half as many rounds of a long chunk
+    const dim3 grid((unsigned)B, (unsigned)G);
+    const int hpg = (int)(H / G);
+#define ATS_GO(N, W)                                                                                                                  \
+  attn_gated_step_k<N, W><<<grid, 64 * W, (size_t)W * hpg * (32 * N + 4) * sizeof(float), stream()>>>(                                \
+      (const uint16_t*)q.data_ptr(), (const uint16_t*)k_cache.data_ptr(), (const uint16_t*)v_cache.data_ptr(),                        \
+      block_tables.data_ptr<int>(), (int)block_tables.size(1), ctx_lens.data_ptr<int>(), pb.data_ptr<float>(), (float)scale, (int)chunk, \
+      (float)out_scale, (uint16_t*)out.data_ptr(), ldo, (int)H, (int)G)
+#define ATS_CASE(N)                       \
+  case N:                                 \
+    if (wide) ATS_GO(N, 8);               \
+    else ATS_GO(N, 4);                    \
+    break;
+    const bool wide = B * G < 256 && hpg <= 8;  // (LDS: at most 34 KB)
+    switch (d / 32) { ATS_CASE(1) ATS_CASE(2) ATS_CASE(3) ATS_CASE(4) }
+#undef ATS_CASE
+#undef ATS_GO
     return;
   }
   if (H / G <= ATG_HEADS) {
