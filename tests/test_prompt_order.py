@@ -1,0 +1,56 @@
+"""Prompts of unlike lengths in one step: every workgroup of the launch finds its sequence, head and rows, whatever the batch."""
+import pytest
+import torch
+
+from xotorch_support_jetson_amd.ops import kernels as K
+from xotorch_support_jetson_amd.ops import reference as R
+
+# (new tokens, cached tokens) per sequence: one, two equal ones, a pair count that is no multiple of 8, the sorted range's end and past it
+BATCHES = {"one": [(300, 0)], "equal": [(64, 0)] * 2, "decode and prompt": [(1, 700), (500, 0), (1, 30)], "nine": [(7 + 67 * (4 * i % 9), 31 * i) for i in range(9)],
+           "32": [(1 + 37 * i % 211, 0) for i in range(32)], "33": [(1 + 37 * i % 211, 0) for i in range(33)]}
+
+
+def _step(batch, G, d):
+  g = torch.Generator(device="cuda").manual_seed(len(batch) + G)
+  ctx = [n + m for n, m in batch]
+  width, pages = max(-(-c // 64) for c in ctx), sum(-(-c // 64) for c in ctx)
+  kc = torch.randn(pages, G, 64, d, generator=g, device="cuda").bfloat16()
+  vc = torch.randn(pages, G, d, 64, generator=g, device="cuda").bfloat16()
+  perm, bt, at = torch.randperm(pages, generator=g, device="cuda").int().cpu(), torch.zeros(len(ctx), width, dtype=torch.int32), 0
+  for b, c in enumerate(ctx):
+    bt[b, :-(-c // 64)] = perm[at:at - (-c // 64)]
+    at += -(-c // 64)
+  cu = torch.tensor([0] + [n for n, _ in batch]).cumsum(0).int().cuda()
+  return kc, vc, bt.cuda(), cu, torch.tensor(ctx, dtype=torch.int32, device="cuda"), g
+
+
+# bf16 probabilities (2^-9 each, independent) and a bf16 result (2^-9): well within 2^-6 of the largest value
+def _near(y, ref):
+  assert (y.float() - ref.float()).abs().max() <= 2**-6 * ref.float().abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G", [(32, 8), (6, 3), (4, 4)])
+@pytest.mark.parametrize("batch", BATCHES)
+def test_causal(batch, H, G):
+  batch = BATCHES[batch]
+  kc, vc, bt, cu, cl, g = _step(batch, G, 128)
+  q = torch.randn(sum(n for n, _ in batch), H, 128, generator=g, device="cuda").bfloat16()
+  args = (q, kc, vc, bt, cu, cl)
+  out = torch.full_like(q, float("nan"))
+  K.attn_prefill(*args, max(n for n, _ in batch), 128**-0.5, out=out)
+  _near(out, R.attn_prefill(*args, 128**-0.5))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G", [(16, 4), (6, 3), (8, 8)])
+@pytest.mark.parametrize("batch", BATCHES)
+def test_window(batch, H, G):
+  batch = BATCHES[batch]
+  kc, vc, bt, cu, cl, g = _step(batch, G, 128)
+  q = torch.randn(sum(n for n, _ in batch), H, 128, generator=g, device="cuda").bfloat16()
+  args, longest = (q, kc, vc, None, None, bt, cu, cl), max(n for n, _ in batch)
+  out, ref = torch.full((len(q), H * 128), float("nan"), device="cuda"), torch.zeros(len(q), H * 128)
+  K.attn_window_pool(*args, None, 128**-0.5, 200, 0, out, longest, 0, 4)
+  R.attn_window_pool(*(x if x is None else x.cpu() for x in args), None, 128**-0.5, 200, 0, ref, longest, 0, 4)
+  _near(out.cpu(), ref)

@@ -949,8 +949,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(
 // K and V^T pages (16 KB each at Dh 128) arrive by LDS-DMA into a 2-deep ring, XOR-swizzled per row
 // through the per-lane source address (swizzles found by exhaustive search against the ds_read_b128 lane
 // groups: every fragment read is conflict-free).  Waves skip the math of pages past their last row's
-// position (causal); workgroups are dispatched heaviest tile first, the tiles of one (sequence, KV head)
-// kept on one XCD.
+// position (causal).  Where a workgroup's work lies in the launch: prompt_work.  With contiguous runs of workgroups per XCD, as
+// before, one XCD had most of a long prompt among short ones (32 heads on 8, us, before -> now: 9 prompts of 21 .. 872 tokens
+// 61.3 -> 39.7, 24 of 33 .. 2700 663 -> 329, 64 of 31 .. 970 320 -> 220, 7000 beside 20 624 -> 324; one of 3000 on 4 KV heads
+// 152 -> 108; even batches as they were).
 template <int DH>
 __device__ __forceinline__ int pf_kswz(int r) {
   return DH == 128 ? (3 * (r & 1)) | (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 3)
@@ -971,17 +973,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_v2_kernel(
   constexpr int CPW = NCH / 8;
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];  // [3][K page | V^T page]
 
-  int tile, kvh, b;
-  {
-    const int nwg = gridDim.x * gridDim.y * gridDim.z;
-    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = lin & 7, qq = nwg >> 3, rr = nwg & 7;
-    lin = (xcd < rr ? xcd * (qq + 1) : rr * (qq + 1) + (xcd - rr) * qq) + (lin >> 3);
-    tile = gridDim.x - 1 - lin % gridDim.x;  // heaviest (latest rows) first
-    lin /= gridDim.x;
-    kvh = lin % gridDim.y;
-    b = lin / gridDim.y;
-  }
+  const PromptWork work = prompt_work(ctx_lens);
+  const int tile = work.tile, kvh = work.head, b = work.seq;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int G = H / Hkv;

@@ -125,6 +125,46 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
   return max(v, row_turn<1>(v));
 }
 
+// The sequence at place p of B when the longest come first (len(b); equal ones as they are given).  Each wave finds it for
+// itself: a sequence a lane, B compares, under 1 us with the loads.  Above 32 sequences the given order stays: there are then
+// several rounds of workgroups, and a long sequence met late costs the launch a small part.
+template <typename F>
+__device__ __forceinline__ int nth_longest(int B, int p, F len) {
+  if (B <= 1 || B > 32) return p;
+  const int lane = threadIdx.x & 63, n = lane < B ? len(lane) : 0;
+  int rank = 0;
+  for (int j = 0; j < B; ++j) {
+    const int m = __builtin_amdgcn_readlane(n, j);
+    rank += m > n || (m == n && j < lane) ? 1 : 0;
+  }
+  return __builtin_ctzll(__ballot(lane < B && rank == p));
+}
+
+// Work of a prompt attention workgroup, of a grid (tiles, kv heads, sequences).  Consecutive workgroups go to the 8 XCDs in
+// turn.  Where the (sequence, kv head) pairs are a multiple of 8 they are dealt to the XCDs in turn, longest context first,
+// and an XCD takes a pair's tiles one after the other, the last rows (most keys) first: the pair's pages come from one L2,
+// and every XCD has its share of the long sequences.  Otherwise the pairs run fastest: all pairs' heaviest tiles first, a
+// pair over several XCDs.
+struct PromptWork {
+  int tile, head, seq;
+};
+__device__ __forceinline__ PromptWork prompt_work(const int* ctx_lens) {
+  const uint32_t tiles = gridDim.x, heads = gridDim.y, pairs = heads * gridDim.z;
+  const uint32_t lin = blockIdx.x + tiles * (blockIdx.y + heads * blockIdx.z);
+  uint32_t pair, turn;
+  if ((pairs & 7) == 0) {
+    const uint32_t j = lin >> 3, r = j / tiles;
+    pair = r * 8 + (lin & 7);
+    turn = j - r * tiles;
+  } else {
+    turn = lin / pairs;
+    pair = lin - turn * pairs;
+  }
+  const uint32_t p = pair / heads;
+  const int seq = nth_longest((int)gridDim.z, (int)p, [&](int b) { return ctx_lens[b]; });
+  return {(int)(tiles - 1 - turn), (int)(pair - p * heads), seq};
+}
+
 __device__ __forceinline__ s16x8 ld16(const void* p) { return *reinterpret_cast<const s16x8*>(p); }
 // non-temporal 16-B load (global_load_dwordx4 ... nt): bytes read once per kernel (KV pages in decode)
 __device__ __forceinline__ s16x8 ld16nt(const void* p) {

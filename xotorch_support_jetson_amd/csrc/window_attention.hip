@@ -2,7 +2,8 @@
 // (K [pages, G, 64, d], V^T [pages, Gv, dv, 64], bf16): the kernels behind attn_window_pool for steps without pooled blocks.
 //
 //   window_prefill_k   prompt portions: a workgroup owns 256 (token, head of the group) rows of one (sequence, kv head), so
-//                      a page is read once for all query heads of the group
+//                      a page is read once for all query heads of the group (work dealt to the XCDs by prompt_work: 5
+//                      prompts of 364 .. 1728 tokens, 16 heads on 4: 98 us before, 66 now)
 //   window_decode_k    single tokens: a workgroup owns one (sequence, kv head, share of the pages), its waves deal the
 //                      pages among themselves and merge through LDS; window_merge_k adds up the shares
 //
@@ -61,17 +62,8 @@ __global__ __launch_bounds__(512, 1) void window_prefill_k(
   static_assert(NCH % 8 == 0 && DK % 32 == 0 && DV % 16 == 0, "chunks split over 8 waves");
   constexpr int CPW = NCH / 8;
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];  // [3][K page | V^T page]
-  int tile, kvh, b;
-  {
-    const int nwg = gridDim.x * gridDim.y * gridDim.z;
-    int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = lin & 7, qq = nwg >> 3, rr = nwg & 7;
-    lin = (xcd < rr ? xcd * (qq + 1) : rr * (qq + 1) + (xcd - rr) * qq) + (lin >> 3);
-    tile = gridDim.x - 1 - lin % gridDim.x;
-    lin /= gridDim.x;
-    kvh = lin % gridDim.y;
-    b = lin / gridDim.y;
-  }
+  const PromptWork work = prompt_work(ctx_lens);
+  const int tile = work.tile, kvh = work.head, b = work.seq;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int rep = H / G, gv = kvh / (G / Gv);
