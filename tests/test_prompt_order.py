@@ -54,3 +54,40 @@ def test_window(batch, H, G):
   K.attn_window_pool(*args, None, 128**-0.5, 200, 0, out, longest, 0, 4)
   R.attn_window_pool(*(x if x is None else x.cpu() for x in args), None, 128**-0.5, 200, 0, ref, longest, 0, 4)
   _near(out.cpu(), ref)
+
+
+# a workgroup's arithmetic does not know the batch: each sequence as it comes alone (which other tests hold against float64)
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [2, 5, 7, 8, 9, 32, 33])  # 64 workgroups a sequence: up to 256, up to 512, and more; sorted and as given
+def test_scan_alone(B):
+  H, G, d, dv = 16, 4, 64, 128
+  lens = [64 + 53 * (5 * i % B) % 190 for i in range(B)]
+  g = torch.Generator(device="cuda").manual_seed(B)
+  rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+  T, cu = sum(lens), torch.tensor([0] + lens).cumsum(0).int().cuda()
+  q, k, v = rn(T, G * d) / 8, rn(T, G * d) / 8, rn(T, H * dv)
+  decay, beta, state = torch.sigmoid(rn(T, H) + 3), torch.sigmoid(rn(T, H)), rn(B, H, dv, d)
+  slots, S, out = torch.randperm(B, generator=g, device="cuda").int(), state.clone(), torch.full((T, H * dv), float("nan"), device="cuda")
+  K.linear_recurrence(q, k, v, decay, beta, 0.5, S, slots, cu, out, False, max(lens))
+  for b, n in enumerate(lens):
+    rows, one = slice(int(cu[b]), int(cu[b]) + n), torch.empty(n, H * dv, device="cuda")
+    K.linear_recurrence(q[rows], k[rows], v[rows], decay[rows], beta[rows], 0.5, state, slots[b:b + 1], torch.tensor([0, n]).int().cuda(), one,
+                        False, max(lens))
+    assert torch.equal(one, out[rows]), b
+  assert torch.equal(state, S)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G", [(16, 4), (6, 3)])
+@pytest.mark.parametrize("batch", BATCHES)
+def test_gated_alone(batch, H, G):
+  batch = BATCHES[batch]
+  kc, vc, bt, cu, cl, g = _step(batch, G, 64)
+  q, pb = torch.randn(int(cu[-1]), H, 64, generator=g, device="cuda").bfloat16(), torch.randn(H, generator=g, device="cuda")
+  out = torch.full((len(q), H * 64), float("nan"), device="cuda", dtype=torch.bfloat16)
+  K.attn_gated_chunk(q, kc, vc, bt, cu, cl, pb, 0.125, 256, 0.5, out, max(n for n, _ in batch))
+  for b, (n, _) in enumerate(batch):
+    rows = slice(int(cu[b]), int(cu[b]) + n)
+    one = torch.empty(n, H * 64, device="cuda", dtype=torch.bfloat16)
+    K.attn_gated_chunk(q[rows], kc, vc, bt[b:b + 1], torch.tensor([0, n]).int().cuda(), cl[b:b + 1], pb, 0.125, 256, 0.5, one, max(n, 2))
+    assert torch.equal(one, out[rows]), b

@@ -520,20 +520,26 @@ __global__ __launch_bounds__(64 * NW, 1) void attn_gated_step_k(
 // with whole-line loads and shared by the four waves.  Scores are computed transposed, S^T = K Q^T (keys x queries),
 // so a lane's four accumulator rows are four consecutive keys of ONE query: after the sigmoid they are, as they lie,
 // the B operand of O^T += V^T P^T, whose k slots (g, j) are read as keys {4g .. 4g+3, 16+4g .. 16+4g+3} on both
-// operands.  LDS rows are padded by 16 B so the fragment reads of 16 rows hit distinct banks.
+// operands.  LDS rows are padded by 16 B so the fragment reads of 16 rows hit distinct banks.  The heads of a tile are
+// neighbours in the launch, so every XCD has its share of every sequence, and the longest sequences start first (with the
+// sequence as the fastest index eight of them had an XCD each: 8 of 961 .. 2433 tokens, 16 heads of 128 in chunks of 1024,
+// 189 us before, 124 now, 32 of 53 .. 1422 307 and 106).
 template <int NK>
 __global__ __launch_bounds__(256) void attn_gated_chunk_mfma_k(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int* __restrict__ block_tables, int width, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
-    const float* __restrict__ pb, float scale, int chunk, float out_scale, uint16_t* __restrict__ out, int ldo, int H, int G) {
+    const float* __restrict__ pb, float scale, int chunk, float out_scale, uint16_t* __restrict__ out, int ldo, int H, int G, int B,
+    int tiles) {
   constexpr int D = NK * 32, ND = NK * 2, QT = 2;
   constexpr int KT = D > 192 ? 32 : 64;  // keys per tile (a page holds a whole number of tiles)
   constexpr int KP = D + 8, VP = KT + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sK[KT][KP], sV[D][VP];
-  const int b = blockIdx.x, h = blockIdx.z;
+  const uint32_t place = blockIdx.x / (uint32_t)H, turn = place / (uint32_t)tiles;
+  const int h = (int)(blockIdx.x - place * H);
+  const int b = nth_longest(B, (int)turn, [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g4 = l >> 4;
   const int t0 = cu_q[b], qlen = cu_q[b + 1] - t0, ctx = ctx_lens[b];
-  const int wq0 = blockIdx.y * 128;
+  const int wq0 = (int)(place - turn * tiles) * 128;
   if (ctx <= 0 || wq0 >= qlen) return;
   const int q0 = wq0 + wave * 32;
   const bool active = q0 < qlen;
@@ -1080,13 +1086,13 @@ void gelu_gather_mul(const at::Tensor& P, int64_t off, const at::Tensor& table, 
 }
 
 template <int NK>
-void launch_attn_mfma(dim3 grid, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
+void launch_attn_mfma(int B, int tiles, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                       const at::Tensor& block_tables, const at::Tensor& cu_q, const at::Tensor& ctx_lens, const at::Tensor& pb,
                       float scale, int chunk, float out_scale, at::Tensor& out, int ldo, int H, int G) {
-  attn_gated_chunk_mfma_k<NK><<<grid, 256, 0, stream()>>>(
+  attn_gated_chunk_mfma_k<NK><<<(unsigned)(B * H) * tiles, 256, 0, stream()>>>(
       (const uint16_t*)q.data_ptr(), (const uint16_t*)k_cache.data_ptr(), (const uint16_t*)v_cache.data_ptr(),
       block_tables.data_ptr<int>(), (int)block_tables.size(1), cu_q.data_ptr<int>(), ctx_lens.data_ptr<int>(),
-      pb.data_ptr<float>(), scale, chunk, out_scale, (uint16_t*)out.data_ptr(), ldo, H, G);
+      pb.data_ptr<float>(), scale, chunk, out_scale, (uint16_t*)out.data_ptr(), ldo, H, G, B, tiles);
 }
 
 // max_qlen: the longest run of new tokens of one sequence in this step (1: single decoded tokens -> the wave-per-token
@@ -1114,10 +1120,10 @@ void attn_gated_chunk(const at::Tensor& q, const at::Tensor& k_cache, const at::
   MCHECK(out.scalar_type() == q.scalar_type(), "out must have q's dtype");
   const bool bf = q.scalar_type() == at::kBFloat16;
   if (bf && max_qlen > 1 && d % 32 == 0 && ldo % 4 == 0 && reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0) {
-    const dim3 grid((unsigned)B, (unsigned)((max_qlen + 127) / 128), (unsigned)H);
+    const int tiles = (int)((max_qlen + 127) / 128);
 #define ATT_CASE(N)                                                                                                         \
   case N:                                                                                                                   \
-    launch_attn_mfma<N>(grid, q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, (float)scale, (int)chunk, (float)out_scale, \
+    launch_attn_mfma<N>((int)B, tiles, q, k_cache, v_cache, block_tables, cu_q, ctx_lens, pb, (float)scale, (int)chunk, (float)out_scale, \
                         out, ldo, (int)H, (int)G);                                                                          \
     break;
     switch (d / 32) {
@@ -1284,8 +1290,8 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
   // Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
   // its 1.4 us a chunk (2.2 with channel decays) beat 0.2 us a token, whatever the other sequences of the step do.  us before / after,
-  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 196, 8 of 961 .. 2431 1018 / 425, 30 single tokens and one
-  // prompt of 500 131 / 95, one of 33 11 / 15; channel decays 498 / 308, 1124 / 574, 229 / 132, 14 / 20.
+  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 196, 8 of 961 .. 2431 1018 / 316, 30 single tokens and one
+  // prompt of 500 131 / 95, one of 33 11 / 15; channel decays 498 / 308, 1124 / 477, 229 / 132, 14 / 20.
   // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
   const int64_t widest = std::max(std::max<int64_t>(ldq, ldk), std::max<int64_t>(std::max<int64_t>(ldv, H * dv), H * d));
   if ((d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && on16(q, ldq) &&

@@ -11,14 +11,14 @@
 //   * chunk_scan_k, the chain: a workgroup per (sequence, head, 32 value channels), a wave per 16 of them and half of the key
 //     dims: the partial products are exchanged through LDS, and from 512 workgroups on a SIMD has two waves, one's products
 //     under the other's waits (a wave with all key dims and 64 channels a workgroup: 294 us instead of 191 for one prompt of 2000,
-//     427 / 419 for eight).  The state stays in MFMA accumulators: tile t, register r, lane group g holds key row
+//     427 / 419 for eight then).  The state stays in MFMA accumulators: tile t, register r, lane group g holds key row
 //     16 t + 4 g + r of value channel lane % 16, and as a B operand the same register is rows 4 g + r of the tile for g = 0 .. 3
 //     -- the A operands only have to name their k dims in that order, four consecutive floats a lane.  So the state never
 //     moves, U and M, N meet the same way, and a chunk is 3 D / 8 + 8 MFMAs a wave (plain write: D / 4 + 4); q, k and the decays
 //     pass LDS once per workgroup, two chunks ahead in registers.
 // Bound by that chain: about 1.4 us a chunk at D 128 where 56 MFMAs of 32 cycles are 0.75 (the rest: two barriers, LDS
 // reads and the four-step products with M and N between them).  Tarepel-design prompts (8 of 961 .. 2431 tokens, 16 heads
-// of 128 x 128): 1018 -> 425 us, delta rule with channel decays 1124 -> 574.
+// of 128 x 128): 1018 -> 316 us, delta rule with channel decays 1124 -> 477.
 // v_mfma_f32_16x16x4_f32 multiplies and accumulates in fp32 as the vector units do; no operand is rounded.
 //
 // Decays per key channel: where a prefix product P leaves 2^-100 .. 2^100 (a decay of 0, or a value that is no number, among
@@ -204,11 +204,23 @@ __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, int off) {
   return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
 
+// The scan's sequences in the order of their workgroups (0: the longest), `per` workgroups a sequence.  Two workgroups share a
+// CU at about twice the time a chunk, so the long sequences are spread over the XCDs (heads fastest) and start first: with
+// the sequences fastest an XCD had one of eight to itself.  Delta rule, 16 heads of 128 x 128, us before and so: 8 of 961 ..
+// 2433 tokens 385 and 333, 16 of 110 .. 1820 536 and 244, 64 of 51 .. 1460 1433 and 708.  Where the launch is between one and
+// two workgroups a CU, the second ones, which take the CUs in the order of the first, are the shortest, beside the shortest
+// of the first that have a neighbour at all: 8 of 961 .. 2433 333 -> 316, 5 of 364 .. 1728 197 -> 183.
+__device__ __forceinline__ int scan_order(int turn, int B, int per) {
+  const int first = 256 / per, second = B - first;
+  if (second <= 0 || second > first) return turn;
+  return turn >= first ? B - 1 - (turn - first) : turn < second ? first - second + turn : turn - second;
+}
+
 template <int D, bool CHAN, bool DELTA>
 __global__ __launch_bounds__(256, 2) void chunk_scan_k(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ decay, const float* __restrict__ inscale, float q_scale, float* __restrict__ state,
-    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int H, int G, int dv, int dvin,
+    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin,
     const float* __restrict__ ws, float* __restrict__ out) {
   constexpr int LD = D + 4;                       // LDS row: consecutive tokens four banks apart
   constexpr int NF = CT * D / 1024;               // float4s of k (and of q) a thread
@@ -218,13 +230,15 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
   __shared__ __attribute__((aligned(16))) float sp[2][CHAN ? D : 4];
   __shared__ f32x4 sx[4][DELTA ? 2 : 1][64];      // the waves' partial products, for the wave with the other key dims
   constexpr int TILES = D / 32;                   // 16-row state tiles of a wave: half of the key dims
-  const int b = blockIdx.x, h = blockIdx.y;
+  const uint32_t cols = (uint32_t)(dv + 31) / 32, place = blockIdx.x / (uint32_t)H, turn = place / cols;
+  const int h = (int)(blockIdx.x - place * H);
+  const int b = nth_longest(B, scan_order((int)turn, B, H * (int)cols), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
   const int t0 = cu_q[b], n = cu_q[b + 1] - t0;
   if (slot < 0 || n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 1;
-  const int col = blockIdx.z * 32 + (wave & 1) * 16 + i;
+  const int col = (int)(place - turn * cols) * 32 + (wave & 1) * 16 + i;
   const bool live = col < dv;
   const int hk = h / (H / G);
   const int d0 = half * (D / 2);                  // the wave's first key dim
@@ -458,11 +472,11 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
 template <int D, bool CHAN, bool DELTA>
 void go(const ChunkRecurrence& a) {
   const int slots = a.T / CT + a.B;
-  const dim3 pg((unsigned)slots, (unsigned)a.H), sg((unsigned)a.B, (unsigned)a.H, (unsigned)((a.dv + 31) / 32));
+  const dim3 pg((unsigned)slots, (unsigned)a.H), sg((unsigned)(a.B * a.H * ((a.dv + 31) / 32)));
   chunk_prep_k<D, CHAN, DELTA><<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale,
                                                         a.state_slots, a.cu_q, a.B, a.H, a.G, a.ws);
   chunk_scan_k<D, CHAN, DELTA><<<sg, 256, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, a.decay, DELTA ? nullptr : a.beta,
-                                                         a.q_scale, a.state, a.state_slots, a.cu_q, a.H, a.G, a.dv, a.dvin,
+                                                         a.q_scale, a.state, a.state_slots, a.cu_q, a.B, a.H, a.G, a.dv, a.dvin,
                                                          a.ws, a.out);
 }
 
