@@ -251,6 +251,19 @@ int launch_mla_prep_slabs(const float* P, int S, long ss, int N, int nope, const
 }
 
 // ------------------------------------------------------------------------------------------ attention
+// sequence of query token t: the largest b with cu_q[b] <= t.  In a step of single tokens it is t itself, one load instead
+// of a chain of them.
+__device__ __forceinline__ int seq_of_query(const int32_t* cu_q, int B, int T, int t) {
+  if (T == B && cu_q[t] <= t && cu_q[t + 1] > t) return t;
+  int lo = 0, hi = B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (cu_q[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 template <int DL>
 __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
     const uint16_t* __restrict__ q_lat, const uint16_t* __restrict__ q_pe, long ldqpe,
@@ -271,39 +284,79 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
   uint16_t* pbuf = smem + 2 * PAGE * ROW;        // [16 heads][PLD] bf16
   float* red = reinterpret_cast<float*>(pbuf + 16 * PLD);  // [4 waves][16 heads]
 
-  // XCD-aware order: the head blocks of one (token, partition) read the same latent pages, so they get
-  // consecutive logical ids that round-robin dispatch places on ONE XCD (one HBM read, the rest from
-  // that XCD's L2) instead of spreading them over all 8 L2s (measured 8x the cache bytes from HBM).
+  // Consecutive workgroups go to the 8 XCDs in turn.  The head blocks of one (token, partition) read the same latent pages:
+  // they are 8 apart, on ONE XCD (one HBM read, the rest from that XCD's L2; spread over all 8 they read 8x the bytes from
+  // HBM).  The tokens follow each other over the XCDs, the last first (in a prompt they have the most keys), and a token's
+  // partitions, of which a short context fills only the first, are on different ones.  (In contiguous runs per XCD one had a
+  // prompt's longest rows: 1500 tokens, 16 heads 250 us, 146 now.)
   int part, hb, t;
   {
-    const int nwg = gridDim.x * gridDim.y * gridDim.z;
-    int b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = b & 7, q = nwg >> 3, r = nwg & 7;
-    b = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (b >> 3);
-    hb = b % gridDim.y;
-    b /= gridDim.y;
-    part = b % gridDim.x;
-    t = b / gridDim.x;
+    const uint32_t hbs = gridDim.y, units = gridDim.x * T, whole = units & ~7u;
+    const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + hbs * blockIdx.z);
+    uint32_t unit;
+    if (lin < whole * hbs) {
+      const uint32_t k = lin >> 3, r = k / hbs;
+      unit = r * 8 + (lin & 7);
+      hb = (int)(k - r * hbs);
+    } else {
+      const uint32_t k = lin - whole * hbs, r = k / hbs;
+      unit = whole + r;
+      hb = (int)(k - r * hbs);
+    }
+    part = (int)(unit / (uint32_t)T);
+    t = (int)(unit - (uint32_t)part * T) + part % T;
+    t = T - 1 - (t >= T ? t - T : t);
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c = lane & 15;
   const int h = hb * 16 + c;
   const bool hv = h < H;
 
-  // sequence of query token t: largest b with cu_q[b] <= t
-  int lo = 0, hi = B - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cu_q[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  const int b = lo;
+  const int b = seq_of_query(cu_q, B, T, t);
   const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
   const int npages = nkeys > 0 ? (nkeys + PAGE - 1) / PAGE : 0;
   const int p_begin = part * pages_per_part;
   const int p_end = min(npages, p_begin + pages_per_part);
   const int np = max(0, p_end - p_begin);
+  if (np == 0 && nparts > 1) return;  // (the merge reads the parts that have pages)
 
+  float m = NEG_BIG, l = 0.f;  // running max / sum of head c (replicated over the 4 lane groups and waves)
+  f32x4 o[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int32_t* bt = block_tables + (size_t)b * max_blocks;
+  // LDS image of a page and its conflict-free reads: as the many-head kernel's below (the plain layout took 16 LDS cycles a K
+  // row read and 8 a transposed V read instead of 4 and 2); the wave's 16 keys are tile j = wave of that order.  37 sequences
+  // of 60 .. 900 tokens, 16 heads, with the merge: 20.3 us so far; these reads, the first page asked for before the queries
+  // and empty partitions that write nothing 15.2, in partitions of two pages instead of three 14.1.
+  auto swz = [](int r) { return (((r >> 1) & 1) << 1) | (((r >> 3) & 1) << 2); };
+  constexpr int GPR = ROW / 8;  // granules per row
+  int from[CPW];                // the lane's source granule of each of the wave's chunks, in elements
+#pragma unroll
+  for (int i = 0; i < CPW; ++i) {
+    const int P = (wave * CPW + i) * 64 + lane, r = P / GPR, j = (P - r * GPR) ^ swz(r);
+    from[i] = (r * GPR + j) * 8;
+  }
+  auto issue = [&](int pi, int buf) {
+    const long page = min(max(bt[p_begin + pi], 0), num_pages - 1);
+    const uint16_t* src = cache + (size_t)page * PAGE * ROW;
+    uint16_t* dst = smem + buf * PAGE * ROW;
+#pragma unroll
+    for (int i = 0; i < CPW; ++i) glds16(src + from[i], dst + (wave * CPW + i) * 512);
+  };
+  int kb[2], vb[4];
+  const int q4 = c >> 2, p4 = c & 3;
+  {
+    const int r = 32 * (wave >> 1) + 8 * q4 + 4 * (wave & 1) + p4, x = g ^ swz(r), xb = x >> 2, xl = x & 3;
+    kb[0] = r * ROW + 8 * xl + 32 * xb;  // even s: s ^ xb = s + xb
+    kb[1] = r * ROW + 8 * xl - 32 * xb;  // odd s: s ^ xb = s - xb
+    const int rv = 8 * g + q4, y = (p4 >> 1) ^ swz(rv), y1 = y >> 1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) vb[v] = rv * ROW + 16 * (v ^ y1) + 8 * (y & 1) + 4 * (p4 & 1) + wave * DW;
+  }
+
+  if (np > 0) issue(0, 0);
   // Q^T fragments (B operand of S^T: k = dims, n = heads): lane (c, g) holds dims 32s + 8g .. +8 of head h
   s16x8 qf[KS];
 #pragma unroll
@@ -314,24 +367,6 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
     qf[s] = x;
   }
 
-  float m = NEG_BIG, l = 0.f;  // running max / sum of head c (replicated over the 4 lane groups and waves)
-  f32x4 o[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int32_t* bt = block_tables + (size_t)b * max_blocks;
-  auto issue = [&](int pi, int buf) {
-    const long page = min(max(bt[p_begin + pi], 0), num_pages - 1);
-    const uint16_t* src = cache + (size_t)page * PAGE * ROW;
-    uint16_t* dst = smem + buf * PAGE * ROW;
-#pragma unroll
-    for (int i = 0; i < CPW; ++i) {
-      const int ch = wave * CPW + i;
-      glds16(src + ch * 512 + lane * 8, dst + ch * 512);
-    }
-  };
-
-  if (np > 0) issue(0, 0);
   for (int pi = 0; pi < np; ++pi) {
     const int buf = pi & 1;
     if (pi + 1 < np) {
@@ -343,11 +378,11 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
     lds_barrier();  // page pi landed for every wave
     const uint16_t* Ks = smem + buf * PAGE * ROW;
 
-    // S^T for this wave's 16 keys: st[r] = S[head c][key 16 wave + 4g + r]
+    // S^T for this wave's 16 keys: st[r] = S[head c][key 32 (wave / 2) + 8 g + 4 (wave % 2) + r]
     f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s) st = mfma16(ld16(Ks + (16 * wave + c) * ROW + 32 * s + 8 * g), qf[s], st);
-    const int key0 = (p_begin + pi) * PAGE + 16 * wave + 4 * g;
+    for (int s = 0; s < KS; ++s) st = mfma16(ld16(Ks + kb[s & 1] + 32 * s), qf[s], st);
+    const int own = 32 * (wave >> 1) + 8 * g + 4 * (wave & 1), key0 = (p_begin + pi) * PAGE + own;
     float mt = NEG_BIG;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -360,12 +395,12 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
     lds_barrier();
     const float mp = fmaxf(fmaxf(red[c], red[16 + c]), fmaxf(red[32 + c], red[48 + c]));
     const float mn = fmaxf(m, mp);
-    const float alpha = exp2f(m - mn);
+    const float alpha = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
     s16x4 pw;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pw[r] = (short)f2bf(exp2f(st[r] - m));
-    *reinterpret_cast<s16x4*>(pbuf + c * PLD + 16 * wave + 4 * g) = pw;
+    for (int r = 0; r < 4; ++r) pw[r] = (short)f2bf(__builtin_amdgcn_exp2f(st[r] - m));
+    *reinterpret_cast<s16x4*>(pbuf + c * PLD + own) = pw;
     lds_barrier();
     // P^T fragments (B operand of O^T: k = keys, n = heads) and the page's row sum of head c
     s16x8 pf[2];
@@ -385,13 +420,11 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
       for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
     // V^T fragments by transposed LDS reads: lane 4q+p of group g addresses key 32kk + 8g (+4) + q,
     // dims d0 + 4p .. +3; lane c receives dim d0 + c of those 4 keys
-    const int q4 = c >> 2, p4 = c & 3;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) {
-      const int d0 = wave * DW + 16 * dt;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        const uint16_t* base = Ks + (32 * kk + 8 * g + q4) * ROW + d0 + 4 * p4;
+        const uint16_t* base = Ks + vb[dt & 3] + 32 * kk * ROW + 64 * (dt >> 2);
         const s16x4 lo4 = tr_read(base), hi4 = tr_read(base + 4 * ROW);
         const s16x8 vf = s16x8{lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
         o[dt] = mfma16(vf, pf[kk], o[dt]);
@@ -462,18 +495,13 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
   const int h = (hg * nw + wave) * 16 + c;
   const bool hv = h < H;
 
-  int lo = 0, hi = B - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cu_q[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  const int b = lo;
+  const int b = seq_of_query(cu_q, B, T, t);
   const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
   const int npages = nkeys > 0 ? (nkeys + PAGE - 1) / PAGE : 0;
   const int p_begin = part * pages_per_part;
   const int p_end = min(npages, p_begin + pages_per_part);
   const int np = max(0, p_end - p_begin);
+  if (np == 0 && nparts > 1) return;
 
   s16x8 qf[KS];
 #pragma unroll
@@ -555,7 +583,7 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
     mt = xor_max<16>(mt);
     mt = xor_max<32>(mt);
     const float mn = fmaxf(m, mt);
-    const float alpha = exp2f(m - mn);
+    const float alpha = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
     s16x8 pf[2];
     float ls = 0.f;
@@ -563,7 +591,7 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint16_t pb = f2bf(exp2f(st[2 * kk + (e >> 2)][e & 3] - m));
+        const uint16_t pb = f2bf(__builtin_amdgcn_exp2f(st[2 * kk + (e >> 2)][e & 3] - m));
         pf[kk][e] = (short)pb;
         ls += bf2f(pb);
       }
@@ -608,21 +636,49 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
   }
 }
 
-// merge the split-KV partials of (token, head): out[h][t][:] = sum_p O_p 2^(m_p - M) / sum_p l_p 2^(m_p - M)
+// merge the split-KV partials of (token, head) that have pages: out[h][t][:] = sum_p O_p 2^(m_p - M) / sum_p l_p 2^(m_p - M).
+// A part a lane for the maxima and sums, four parts' rows in flight at a time, two dims a thread.
 __global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
-                                                          uint16_t* __restrict__ out, int T, int H, int DL, int nparts) {
-  const int th = blockIdx.x, t = th / H, h = th % H;
+                                                          uint16_t* __restrict__ out, const int32_t* __restrict__ cu_q,
+                                                          const int32_t* __restrict__ ctx_lens, int B, int T, int H, int DL,
+                                                          int max_blocks, int pages_per_part, int nparts) {
+  const int th = blockIdx.x, t = th / H, h = th - t * H, lane = threadIdx.x & 63;
+  const int b = seq_of_query(cu_q, B, T, t);
+  const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
+  const int n = nkeys > 0 ? min(nparts, ((nkeys + PAGE - 1) / PAGE + pages_per_part - 1) / pages_per_part) : 0;
   const size_t base = (size_t)th * nparts;
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + base;
+  const int d = 2 * threadIdx.x;
+  const bool live = d < DL;
+  const float* src = ws_o + base * DL + (live ? d : 0);
   float M = NEG_BIG;
-  for (int p = 0; p < nparts; ++p) M = fmaxf(M, ws_ml[(base + p) * 2]);
-  float L = 0.f;
-  for (int p = 0; p < nparts; ++p) L += ws_ml[(base + p) * 2 + 1] * exp2f(ws_ml[(base + p) * 2] - M);
-  const float il = L > 0.f ? 1.f / L : 0.f;
-  for (int d = threadIdx.x; d < DL; d += 256) {
-    float acc = 0.f;
-    for (int p = 0; p < nparts; ++p) acc += ws_o[(base + p) * DL + d] * exp2f(ws_ml[(base + p) * 2] - M);
-    out[((size_t)h * T + t) * DL + d] = f2bf(acc * il);
+  for (int p = lane; p < n; p += 64) M = fmaxf(M, ml[p].x);
+  M = wave_max(M);
+  float L = 0.f, a0 = 0.f, a1 = 0.f;
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    const int m = min(64, n - c0);
+    float w = 0.f;
+    if (lane < m) {
+      const float2 x = ml[c0 + lane];
+      w = __builtin_amdgcn_exp2f(x.x - M);
+      L += w * x.y;
+    }
+    for (int p = 0; p < m; p += 4) {
+      float2 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float2*>(src + (size_t)(c0 + min(p + j, m - 1)) * DL);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (p + j < m) {
+          const float wj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), p + j));
+          a0 += v[j].x * wj;
+          a1 += v[j].y * wj;
+        }
+    }
   }
+  L = wave_sum(L);
+  const float il = L > 0.f ? 1.f / L : 0.f;
+  if (live) *reinterpret_cast<uint32_t*>(out + ((size_t)h * T + t) * DL + d) = (uint32_t)f2bf(a0 * il) | (uint32_t)f2bf(a1 * il) << 16;
 }
 
 template <int DL>
@@ -654,7 +710,8 @@ static void mla_launch(const uint16_t* q_lat, const uint16_t* q_pe, long ldqpe, 
     kern<<<grid, 256, SMEM, s>>>(q_lat, q_pe, ldqpe, cache, bt, max_blocks, cu_q, ctx, B, T, H, out, ws_o, ws_ml, ppp,
                                  nparts, scale * LOG2E, num_pages);
   }
-  if (nparts > 1) mla_combine_kernel<<<T * H, 256, 0, s>>>(ws_o, ws_ml, out, T, H, DL, nparts);
+  static_assert(DL <= 512, "two dims a thread");
+  if (nparts > 1) mla_combine_kernel<<<T * H, 256, 0, s>>>(ws_o, ws_ml, out, cu_q, ctx, B, T, H, DL, max_blocks, ppp, nparts);
 }
 
 int launch_mla_attn(const uint16_t* q_lat, const uint16_t* q_pe, long ldqpe, const uint16_t* cache,

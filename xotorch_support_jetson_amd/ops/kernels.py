@@ -423,7 +423,7 @@ class MLAWorkspace:
   def __init__(self, max_tokens: int, H: int, DL: int, max_ctx: int, device):
     self.max_tokens, self.H, self.DL = max_tokens, H, DL
     self.pages = max(1, -(-max_ctx // PAGE))
-    self.max_parts = max(self.partition(1, self.pages)[1], self.partition(8, self.pages)[1])
+    self.max_parts = max(self.partition(T, w)[1] for T in (1, 8) for w in (self.pages, min(self.pages, 16)))
     units = max(max_tokens * self.max_parts, 1)
     self.o = torch.empty(units * H * DL, dtype=torch.float32, device=device)
     self.ml = torch.empty(units * H * 2, dtype=torch.float32, device=device)
@@ -438,13 +438,19 @@ class MLAWorkspace:
     return self.H >= 64 and T >= 8
 
   def partition(self, T: int, width_pages: int):
-    """(pages per partition, partitions, wide): enough workgroups for 256 CUs (one per CU: the kernels
-    hold two 73 KB pages in LDS); narrow-kernel partitions of at least 2 pages."""
+    """(pages per partition, partitions, wide).  A CU holds one workgroup (two 73 KB pages in LDS).  Many heads: enough
+    workgroups for 256 CUs.  Narrow kernel: one and a half a CU at most, since the partitions past a sequence's end cost
+    next to nothing, of at least two pages; of one for a handful of workgroups on a short table.  us in partitions of 1 / 2 /
+    3 / 4 pages, 16 heads, attention and merge: one of 900 tokens 9.9 / 11.3 / 13.1 / 14.8, one of 2000 13.5 / 13.1 / 14.5 /
+    15.4; 16 of 65 .. 830 12.5 / 12.4 / 14.1 / 15.1; 37 18.5 / 14.1 / 15.1 / 16.2; 64 25.2 / 23.2 / 16.8 / 17.7; 200 of
+    up to 400 41 / 29 / 30 / 28, whole 20.7."""
     nhb = -(-self.H // 16)
     wide = self.wide(T)
-    units = T * -(-nhb // 8) if wide else T * nhb
-    want = max(1, -(-256 // max(units, 1)))
-    cap = width_pages if wide else (width_pages // 2 if width_pages >= 2 else 1)
+    units = max(1, T * -(-nhb // 8) if wide else T * nhb)
+    if wide:
+      want, cap = -(-256 // units), width_pages
+    else:
+      want, cap = 384 // units, width_pages if width_pages <= 16 and units * width_pages <= 128 else max(1, width_pages // 2)
     nparts = max(1, min(want, cap))
     ppp = -(-width_pages // nparts)
     return ppp, -(-width_pages // ppp), wide
