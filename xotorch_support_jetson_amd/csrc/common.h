@@ -78,6 +78,28 @@ __device__ __forceinline__ float group16_max(float v) {
   return v;
 }
 __device__ __forceinline__ float wave_sum(float v) { return group16_sum(xor_sum<16>(xor_sum<32>(v))); }
+// The wave's sums of eight values at once, 18 operations instead of eight times eight: each of the first three steps adds two
+// values' halves, so that lane wave_sum8_lane(i), and the seven behind it, end with the sum of v[i].
+__device__ __forceinline__ float wave_sum8(const float (&v)[8]) {
+  float u[4], w[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[2 * j]), __float_as_uint(v[2 * j + 1]), false, false);
+    u[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(u[2 * j]), __float_as_uint(u[2 * j + 1]), false, false);
+    w[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) w[j] += __uint_as_float(row_turn<8>(__float_as_uint(w[j])));
+  float s = threadIdx.x & 8 ? w[1] : w[0];
+  s += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(s), 0x141, 0xf, 0xf, false));  // the eight lanes mirrored
+  s += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(s), 0x4e, 0xf, 0xf, false));   // lane ^ 2
+  return s + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(s), 0xb1, 0xf, 0xf, false));  // lane ^ 1
+}
+__device__ __forceinline__ constexpr int wave_sum8_lane(int i) { return 32 * (i & 1) + 16 * ((i >> 1) & 1) + 8 * (i >> 2); }
 __device__ __forceinline__ float wave_max(float v) { return group16_max(xor_max<16>(xor_max<32>(v))); }
 // sum of a quad of lanes: v + its neighbour's (lane ^ 1), then that + the other pair's
 __device__ __forceinline__ float quad_sum(float v) {
