@@ -22,7 +22,7 @@ constexpr int CTB = 8;  // tokens whose inputs are in flight together (runs of t
 // writes the state (else conv_tail_k does, after every token has read it).
 // Runs are bound by the vector unit nearly as much as by memory: SiLU in half the operations, the eight tokens' sums of squares
 // reduced together and their factors computed a token a lane, us before and after: 4593 tokens x 6144 channels in heads of
-// 128 63 -> 51 (226 MB: 47 at a copy's rate), 12807 x 4096 136 -> 123 (420 MB: 87), 4593 x 1024 in heads of 64 35 -> 21.
+// 128 63 -> 53 (226 MB: 47 at a copy's rate), 12807 x 4096 136 -> 124 (420 MB: 87), 4593 x 1024 in heads of 64 35 -> 21.
 struct ConvArgs {
   const float* P;  // [S][T][ldp], slabs ss apart
   int ldp, S;
@@ -41,12 +41,14 @@ struct ConvArgs {
   float* out;
 };
 
-// x / (1 + e^-x) in half the operations: e^-x from the base-2 exponential of the hardware, its argument in two parts, and the quotient from its reciprocal, corrected by the remainder (no number there is an infinite x's: dropped)
+// x / (1 + e^-x) in half the operations: e^-x from the base-2 exponential of the hardware (its argument reduced with log2 e in
+// two parts) and the quotient from its reciprocal, corrected by the remainder (which is no number for an infinite x: dropped).
+// Error against float64 over -80 .. 20: 3.9e-8 rms, 1.7e-7 at most, as with expf and a division.
 __device__ __forceinline__ float silu_n(float x) {
   const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
-  const float p = c * -1.44269502e0f;
-  const float lo = fmaf(c, -1.92596299e-8f, fmaf(c, -1.44269502e0f, -p)), n = rintf(p);
-  const float e = ldexpf(__builtin_amdgcn_exp2f((p - n) + lo), (int)n);
+  const float n = rintf(c * -1.44269502f);  // -x log2 e = n + a, log2 e in two parts
+  const float a = fmaf(c, -1.92596299e-8f, fmaf(c, -1.44269502f, -n));
+  const float e = ldexpf(__builtin_amdgcn_exp2f(a), (int)n);
   const float d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), y = x * r;
   return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, y, x), -1e35f, 1e35f), r, y);
 }
