@@ -56,3 +56,43 @@ def test_gated_step(H, G, d, chunk, rep):
   assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5)[live].all())
   assert float((buf[:, :4] - 3).abs().max()) == 0 and float((buf[:, -4:] - 3).abs().max()) == 0
   assert float((out[~live] - 3).abs().max()) == 0  # padding rows are not written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,d", [(16, 4, 128), (16, 1, 64), (32, 4, 32), (12, 1, 96)])
+@pytest.mark.parametrize("chunk,n", [(96, 130), (7, 60), (96, 100), (1024, 400)])
+def test_values_that_are_no_numbers(H, G, d, chunk, n):
+  """Values before the chunk that are no numbers or infinite, and those of keys whose weight underflowed, are left out; infinite ones
+  of the chunk reach the sums of their channel with their sign, beside the terms of a weight that are 0."""
+  g = torch.Generator(device="cuda").manual_seed(H + d + n)
+  width, lo = -(-n // 64), (n - 1) // chunk * chunk
+  kc = torch.randn(width, G, 64, d, generator=g, device="cuda").bfloat16()
+  vc = torch.randn(width, G, d, 64, generator=g, device="cuda").bfloat16()
+  q = torch.randn(1, H, d, generator=g, device="cuda").bfloat16()
+  bt = torch.arange(width, dtype=torch.int32, device="cuda")[None].contiguous()
+  cu, cl = torch.tensor([0, 1], dtype=torch.int32, device="cuda"), torch.tensor([n], dtype=torch.int32, device="cuda")
+
+  def run(kc, vc, pb, max_qlen):
+    out = torch.zeros(1, H * d, dtype=torch.bfloat16, device="cuda")
+    K.attn_gated_chunk(q, kc, vc, bt, cu, cl, pb, d ** -0.5, chunk, 1.5, out, max_qlen=max_qlen)
+    return out
+  pb = torch.randn(H, generator=g, device="cuda") - 2
+  plain = _exact(q, kc, vc, bt, [n], pb, d ** -0.5, chunk, 1.5)
+  near = lambda got, want: bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())  # noqa: E731 - (as above)
+  if lo % 64:
+    for bad in (float("nan"), float("-inf")):
+      v = vc.clone()
+      v[lo // 64, :, :, :lo % 64] = bad
+      assert near(run(kc, v, pb, 1), plain), bad
+  v = vc.clone()
+  at = n - 1 - (n - 1 - lo) // 3  # a key of the chunk
+  v[at // 64, :, 1, at % 64], v[at // 64, :, 5, at % 64], v[at // 64, :, 9, at % 64] = float("inf"), float("-inf"), float("nan")
+  want = plain.view(1, H, d).clone()
+  want[:, :, 1], want[:, :, 5], want[:, :, 9] = float("inf"), float("-inf"), float("nan")
+  for max_qlen in (1, 0):  # (0: the kernel of any head size)
+    got = run(kc, v, pb, max_qlen).double()
+    same = ((got - want.view(1, -1)).abs() <= 2.0 ** -8 * want.view(1, -1).abs() + 1e-5) | (got == want.view(1, -1)) | (got.isnan() & want.view(1, -1).isnan())
+    assert bool(same.all()), max_qlen
+  off = torch.full_like(pb, -200.0)  # (every weight 0)
+  for max_qlen in (1, 0):
+    assert float(run(kc, v, off, max_qlen).abs().max()) == 0, max_qlen

@@ -403,6 +403,9 @@ __global__ void attn_split_sum_k(const float* __restrict__ part, int KS, int T, 
 // mantissa each), so a product costs three MFMA steps and keeps what fp32 had.  Bound by latencies (table, pages, merge).  On the vector
 // unit, in up to eight key splits and with a launch that added them, 48 tokens x 4 kv heads of 128, contexts of 60 to 110: 9.5 + 4.7
 // us, 6.4 here; 1000 tokens each 42.1 / 24.9, 200 tokens of contexts 30 to 160 29.2 / 16.0, one of 40 10.1 / 5.2, one of 1000 18.7 both.
+// A product with a weight, or a term of one, that is 0 would carry over values that are no numbers or infinite: of keys before the chunk,
+// of a weight that underflowed, of a term that is 0 beside an infinite value.  They leave a sum that is no number, so a wave with
+// a result that is not finite adds the chunk again for its results, on the vector unit and without the products of a weight of 0.
 template <int NK, int NW>
 __global__ __launch_bounds__(64 * NW, 1) void attn_gated_step_k(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
@@ -503,6 +506,7 @@ __global__ __launch_bounds__(64 * NW, 1) void attn_gated_step_k(
     for (int dt = 0; dt < ND; ++dt) *reinterpret_cast<f32x4*>(mine + 16 * dt) = o[dt];
   }
   __syncthreads();
+  bool finite = true;
   for (int e = 4 * threadIdx.x; e < hpg * D; e += 4 * 64 * NW) {
     const int h = e / D, i = e - h * D;
     f32x4 v = *reinterpret_cast<const f32x4*>(sm + h * LD + i);
@@ -510,8 +514,46 @@ __global__ __launch_bounds__(64 * NW, 1) void attn_gated_step_k(
     for (int w = 1; w < NW; ++w) v += *reinterpret_cast<const f32x4*>(sm + (w * hpg + h) * LD + i);
     s16x4 y;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) y[r] = (short)f2bf(v[r] * out_scale);
+    for (int r = 0; r < 4; ++r) {
+      y[r] = (short)f2bf(v[r] * out_scale);
+      finite &= fabsf(v[r]) < INFINITY;
+    }
     *reinterpret_cast<s16x4*>(out + (int64_t)b * ldo + (kvh * hpg + h) * D + i) = y;
+  }
+  if (__builtin_expect(__ballot(!finite) == 0, 1)) return;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // (the results above are there before those below)
+  for (int h = 0; h < hpg; ++h) {
+    const int head = kvh * hpg + h;
+    const uint16_t* qr = q + ((int64_t)b * H + head) * D;
+    float acc[(D + 63) / 64] = {};  // of dims lane, lane + 64
+    for (p = lo / PAGE_TOK; p <= last; ++p) {  // a key a lane
+      const int64_t page = (int64_t)bt[p] * G + kvh;
+      const uint16_t* kr = k_cache + (page * PAGE_TOK + lane) * D;
+      float s = 0.0f;
+      for (int i = 0; i < D; i += 8) {
+        const s16x8 kv = ld16(kr + i), qv = ld16(qr + i);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += bf2f(qv[e]) * bf2f(kv[e]);
+      }
+      const int key = p * PAGE_TOK + lane;
+      const float w = key >= lo && key <= pos ? sigmoidf_(s * scale + pb[head]) : 0.0f;
+      for (int k = 0; k < PAGE_TOK; k += 8)
+#pragma unroll
+        for (int j = 0; j < (D + 63) / 64; ++j) {
+          const s16x8 v = ld16(v_cache + (page * D + min(lane + 64 * j, D - 1)) * PAGE_TOK + k);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float we = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), k + e));
+            acc[j] += we != 0.0f ? we * bf2f(v[e]) : 0.0f;
+          }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < (D + 63) / 64; ++j) {
+      const int i = lane + 64 * j, e = h * D + i;
+      if (i < D && (e >> 8) % NW == wave)  // (else another wave's result)
+        out[(int64_t)b * ldo + kvh * hpg * D + e] = f2bf(acc[j] * out_scale);
+    }
   }
 }
 
