@@ -32,3 +32,31 @@ def test_units(head, lens):
         err = f * (err + u.abs() * f * (err.norm(dim=-1, keepdim=True) if not kind & R.CONV_UNIT_SCALED else err.norm(dim=-1, keepdim=True) * head**0.5)) + 2**-20 * (u * f).abs()
         u = u * f
       assert ((out[cu[b]:cu[b + 1], at].cpu().double() - u).abs() <= err + 1e-30).all(), (b, i)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs", [True, False])
+def test_silu_of_any_input(runs):
+  """SiLU where e^-x leaves the range of a float: -0 or 0 for finite inputs, however large, and infinities and no numbers as a
+  quotient has them."""
+  inf, nan = float("inf"), float("nan")
+  v = [-inf, -3e38, -1e35, -1e30, -1e4, -129.0, -128.0, -100.0, -89.0, -88.0, -87.5, -87.0, -80.0, -1.0, -1e-30, 0.0, 1e-30, 1.0, 80.0, 87.0, 100.0, 1e35, 3e38, inf, nan]
+  x = torch.tensor([v, v[::-1], v], dtype=torch.float32, device="cuda")
+  T, C = x.shape
+  units, width = R.conv_units([(C, R.CONV_SILU)], C)
+  out, slots = torch.zeros_like(x), torch.arange(1 if runs else T, dtype=torch.int32, device="cuda")
+  cu = torch.tensor([0, T] if runs else list(range(T + 1)), dtype=torch.int32, device="cuda")
+  K.conv_prep(x, 0, torch.ones(C, 1, device="cuda"), None, units.cuda(), None, torch.zeros(len(slots), 0, C, device="cuda"), slots, cu, 1e-5, out,
+              T if runs else 1, width)
+  got, x = out.double().cpu(), x.double().cpu()
+  want = x / (1 + torch.exp(-x))
+  want[(x < -700) & (x > -inf)] = 0.0  # (e^-x past float64)
+  assert torch.equal(got.isnan(), want.isnan())
+  ok = ~want.isnan()
+  got, want, x = got[ok], want[ok], x[ok]
+  assert torch.equal(got.isinf(), want.isinf()) and bool((got[got.isinf()] > 0).all())
+  fin = ~want.isinf()
+  got, want, x = got[fin], want[fin], x[fin]
+  # 2^-22 of the value (twice the 1.7e-7 of ordinary ones); between -88.8 and -87.3 the reciprocal may be 0, below it is
+  assert bool(((got - want).abs() <= 2.0 ** -22 * want.abs() + torch.where(x < -87.3, 1.2e-36, 0.0)).all())
+  assert bool((got[x < -88.8] == 0).all())

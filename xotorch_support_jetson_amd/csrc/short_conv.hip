@@ -43,9 +43,11 @@ struct ConvArgs {
 
 // x / (1 + e^-x) in half the operations: e^-x from the base-2 exponential of the hardware (its argument reduced with log2 e in
 // two parts) and the quotient from its reciprocal, corrected by the remainder (which is no number for an infinite x: dropped).
-// Error against float64 over -80 .. 20: 3.9e-8 rms, 1.7e-7 at most, as with expf and a division.
+// Error against float64 over -80 .. 20: 3.9e-8 rms, 1.7e-7 at most, as with expf and a division.  Below -87.3, where the
+// reciprocal leaves the normal numbers and the true value is at most 1.1e-36, the result is 0, from -88.8 on because e^-x is infinite;
+// the argument is limited to keep the whole number of its base-2 logarithm small (-inf, like no number, gives no number).
 __device__ __forceinline__ float silu_n(float x) {
-  const float c = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
+  const float c = __builtin_amdgcn_fmed3f(x, -128.0f, 87.0f);
   const float n = rintf(c * -1.44269502f);  // -x log2 e = n + a, log2 e in two parts
   const float a = fmaf(c, -1.92596299e-8f, fmaf(c, -1.44269502f, -n));
   const float e = ldexpf(__builtin_amdgcn_exp2f(a), (int)n);
