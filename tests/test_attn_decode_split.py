@@ -115,3 +115,20 @@ def test_lone_sequence_needs_no_plan(H, Hkv, Dh):
       want = R.attn_decode(q, kc, vc, bt, cl, 1 / math.sqrt(Dh)).float()
       # (as above)
       assert float((out.float() - want).abs().max()) < 2e-2 * float(want.abs().max()), (width, n)
+
+
+@pytest.mark.gpu
+def test_steps_too_large_to_count_are_refused():
+  """Pages over all KV heads are counted in 32 bits, and a plan belongs to the batch and the tables it was made for."""
+  C = K.require()
+  cl = torch.ones(1 << 20, dtype=torch.int32, device="cuda")
+  for B, Hkv, width in ((1, 1 << 10, 1 << 20), (1 << 20, 1 << 10, 1), (1 << 15, 1 << 5, 1 << 10), (1 << 10, 1 << 20, 1 << 24), (1, 1, (1 << 24) + 1), (0, 8, 9), (2, 0, 9)):
+    with pytest.raises(RuntimeError):
+      C.decode_plan(cl, B, Hkv, width)
+  q, kc, vc, bt, cl = _step([600] * 6, 10, 16, 4, 64)
+  ws = K.DecodeWorkspace(64, 16, 64, 64 * 64, q.device, algo=2)
+  for B, width in ((5, 10), (7, 10), (64, 64)):  # (no plan of these has as many places)
+    plan = C.decode_plan(torch.full((B,), 600, dtype=torch.int32, device="cuda"), B, 4, width)
+    with pytest.raises(RuntimeError):
+      C.attn_decode_split(q, kc, vc, bt, plan, cl, ws.tickets, torch.empty_like(q), ws.o, ws.ml, 0.125, False)
+  assert int(ws.tickets.abs().max()) == 0

@@ -895,11 +895,18 @@ void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tenso
   XCHECK(rc == 0, "attn_decode: unsupported H=", H, " Hkv=", Hkv, " Dh=", Dh);
 }
 
+// A decode step whose contexts are cut by their lengths counts its pages over all KV heads in 32 bits.  Past that a part would be too
+// short, the parts more than the places, and a sequence without all of its parts never merged.
+static bool decode_sizes_ok(int64_t B, int64_t Hkv, int64_t max_blocks) {
+  return B >= 1 && B <= (1 << 20) && Hkv >= 1 && Hkv <= (1 << 20) && max_blocks >= 1 && max_blocks <= (1 << 24) &&
+         B * Hkv < (int64_t(1) << 30) && B * Hkv * max_blocks < (int64_t(1) << 30);
+}
+
 // the plan of attn_decode_split: int32 [places, 8] (see kernels.h DecodePart), written by one launch
 at::Tensor decode_plan(const at::Tensor& ctx_lens, int64_t B, int64_t Hkv, int64_t max_blocks) {
   CHECK_DT(ctx_lens, at::kInt);
   XCHECK(all_contig_gpu(ctx_lens) && B >= 1 && ctx_lens.numel() >= B, "decode_plan: ctx_lens");
-  XCHECK(Hkv >= 1 && max_blocks >= 1 && B <= (1 << 20) && max_blocks <= (1 << 24), "decode_plan: sizes");
+  XCHECK(decode_sizes_ok(B, Hkv, max_blocks), "decode_plan: sizes");
   at::Tensor plan = at::empty({xot::decode_split_places((int)B, (int)Hkv, (int)max_blocks), 8}, ctx_lens.options());
   XCHECK(reinterpret_cast<uintptr_t>(plan.data_ptr()) % 32 == 0, "decode_plan: alignment");
   xot::launch_decode_plan(ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hkv, (int)max_blocks,
@@ -927,6 +934,7 @@ void attn_decode_split(const at::Tensor& q, const at::Tensor& k_cache, const at:
              v_cache.size(0) == nb && v_cache.size(1) == Hkv,
          "attn_decode_split: cache layout K[nb,Hkv,64,Dh] V[nb,Hkv,Dh,64]");
   XCHECK(block_tables.dim() == 2 && block_tables.size(0) >= B, "attn_decode_split: tables");
+  XCHECK(decode_sizes_ok(B, Hkv, block_tables.size(1)), "attn_decode_split: sizes");
   XCHECK(out.numel() == B * H * Dh, "attn_decode_split: out shape");
   XCHECK(!defer || !plan.has_value(), "attn_decode_split: only a lone sequence's parts can be left unmerged");
   int64_t places = 0;
@@ -936,6 +944,7 @@ void attn_decode_split(const at::Tensor& q, const at::Tensor& k_cache, const at:
     XCHECK(all_contig_gpu(*plan) && plan->dim() == 2 && plan->size(1) == 8 && reinterpret_cast<uintptr_t>(plan->data_ptr()) % 32 == 0,
            "attn_decode_split: plan");
     places = plan->size(0);
+    XCHECK(places == xot::decode_split_places((int)B, (int)Hkv, (int)block_tables.size(1)), "attn_decode_split: another step's plan");
     parts = reinterpret_cast<const xot::DecodePart*>(plan->data_ptr<int32_t>());
   } else {
     XCHECK(B == 1 && ctx_lens.numel() >= 1, "attn_decode_split: several sequences need a plan");
