@@ -132,3 +132,25 @@ def test_steps_too_large_to_count_are_refused():
     with pytest.raises(RuntimeError):
       C.attn_decode_split(q, kc, vc, bt, plan, cl, ws.tickets, torch.empty_like(q), ws.o, ws.ml, 0.125, False)
   assert int(ws.tickets.abs().max()) == 0
+
+
+def test_places_of_the_rule():
+  """Every plan of a workspace's own batches and widths fits it (a KV head has at most 16 query heads)."""
+  for max_batch, H, max_ctx in ((1, 32, 300), (4, 64, 2048), (32, 32, 512), (300, 14, 9000)):
+    ws = K.DecodeWorkspace(max_batch, H, 128, max_ctx, torch.device("cpu"))
+    for Hkv in (n for n in range(1, H + 1) if H % n == 0 and H // n <= 16):
+      assert all(K.split_places(B, Hkv, w) <= ws.places for B in {1, max_batch // 2 or 1, max_batch} for w in range(1, -(-max_ctx // 64) + 1))
+
+
+@pytest.mark.gpu
+def test_tables_wider_than_the_workspace():
+  """A workspace of a shorter context bound serves wide tables as it can: whole contexts, no plan."""
+  B, H, Hkv, Dh, width = 32, 16, 8, 128, 32
+  q, kc, vc, bt, cl = _step([40 + (53 * i) % 1100 for i in range(B)], width, H, Hkv, Dh)
+  ws = K.DecodeWorkspace(B, H, Dh, 512, q.device)
+  plan = ws.plan(bt, cl, Hkv)
+  out = K.attn_decode(q, kc, vc, bt, cl, Dh ** -0.5, ws, plan=plan)
+  want = R.attn_decode(q, kc, vc, bt, cl, 1 / math.sqrt(Dh)).float()
+  assert float((out.float() - want).abs().max()) < 2e-2 * float(want.abs().max())  # (as above)
+  assert plan is None and K.DecodeWorkspace(B, H, Dh, width * 64, q.device).plan(bt, cl, Hkv) is not None
+  assert K.split_places(7, Hkv, 33) == K.require().decode_plan(cl.new_ones(7), 7, Hkv, 33).shape[0]

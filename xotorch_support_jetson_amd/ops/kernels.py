@@ -223,6 +223,11 @@ def plan_pays(batch: int, Hkv: int, width_pages: int) -> bool:
   return width_pages > SPLIT_MIN_PAGES and pairs < 64 * min(width_pages, 32) and pairs * width_pages < 1 << 30
 
 
+def split_places(batch: int, Hkv: int, width_pages: int) -> int:
+  """Places of a plan (csrc/kernels.h decode_split_places), each with a row of partials per query head."""
+  return min(batch + 512 // Hkv, batch * -(-width_pages // 4))
+
+
 class DecodeWorkspace:
   """Split-KV scratch for attn_decode, sized for every batch up to max_batch at this context bound.
   The partitioning is chosen per call from the actual batch (static per captured graph).  routed: the model has routed
@@ -250,7 +255,8 @@ class DecodeWorkspace:
     self.max_batch = max_batch
     self.units = worst  # max over batch of batch * nparts
     if not routed:
-      worst = max(worst, min(max_batch + 512 // max(1, -(-H // 16)), max_batch * -(-pages // 4)))
+      worst = max(worst, split_places(max_batch, max(1, -(-H // 16)), pages))
+    self.places = worst
     self.tickets = torch.zeros(max_batch * H, dtype=torch.int32, device=device)
     self.o = torch.empty(worst * H * Dh, dtype=torch.float32, device=device)
     self.ml = torch.empty(worst * H * 2, dtype=torch.float32, device=device)
@@ -270,6 +276,8 @@ class DecodeWorkspace:
     one sequence, which needs none; None where attn_decode goes by itself."""
     B, width = ctx_lens.shape[0], block_tables.shape[1]
     if not block_tables.is_cuda or self.fixed_ppp or self.routed or B > self.max_batch or self.Dh not in (64, 128):
+      return None
+    if split_places(B, Hkv, width) > self.places:  # (tables wider than this workspace's context bound)
       return None
     if B == 1 and self.algo == -1 and width * Hkv < 1 << 30:
       return LONE
