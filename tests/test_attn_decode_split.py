@@ -122,7 +122,7 @@ def test_steps_too_large_to_count_are_refused():
   """Pages over all KV heads are counted in 32 bits, and a plan belongs to the batch and the tables it was made for."""
   C = K.require()
   cl = torch.ones(1 << 20, dtype=torch.int32, device="cuda")
-  for B, Hkv, width in ((1, 1 << 10, 1 << 20), (1 << 20, 1 << 10, 1), (1 << 15, 1 << 5, 1 << 10), (1 << 10, 1 << 20, 1 << 24), (1, 1, (1 << 24) + 1), (0, 8, 9), (2, 0, 9)):
+  for B, Hkv, width in ((1, 1 << 10, 1 << 20), (1 << 20, 1 << 10, 1), (1 << 20, 1 << 4, 1), (1 << 15, 1 << 5, 1 << 10), (1 << 10, 1 << 20, 1 << 24), (1, 1, (1 << 24) + 1), (0, 8, 9), (2, 0, 9)):
     with pytest.raises(RuntimeError):
       C.decode_plan(cl, B, Hkv, width)
   q, kc, vc, bt, cl = _step([600] * 6, 10, 16, 4, 64)

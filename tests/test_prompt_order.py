@@ -91,3 +91,27 @@ def test_gated_alone(batch, H, G):
     one = torch.empty(n, H * 64, device="cuda", dtype=torch.bfloat16)
     K.attn_gated_chunk(q[rows], kc, vc, bt[b:b + 1], torch.tensor([0, n]).int().cuda(), cl[b:b + 1], pb, 0.125, 256, 0.5, one, max(n, 2))
     assert torch.equal(one, out[rows]), b
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,longest", [(5, 52, 65535 * 128), (66000, 2, 2)])
+def test_gated_chunk_of_many_workgroups(B, H, longest):
+  """More workgroups than one launch dimension holds work items for, most of them without rows (the longest run is a bound), and a
+  large batch: what the launch is told does not change the rows."""
+  d, T = 32, B + 4
+  g = torch.Generator(device="cuda").manual_seed(H)
+  kc, vc = (torch.randn(1, 1, *s, generator=g, device="cuda").bfloat16() for s in ((64, d), (d, 64)))
+  q = torch.randn(T, H, d, generator=g, device="cuda").bfloat16()
+  pb, cu = torch.randn(H, generator=g, device="cuda"), torch.arange(B + 1, dtype=torch.int32, device="cuda")
+  cu[-1] = T  # the last sequence has five tokens, the others one
+  cl = torch.ones(B, dtype=torch.int32, device="cuda")
+  cl[-1] = 5
+  bt = torch.zeros(B, 1, dtype=torch.int32, device="cuda")
+  out = torch.full((T, H * d), float("nan"), device="cuda", dtype=torch.bfloat16)
+  K.attn_gated_chunk(q, kc, vc, bt, cu, cl, pb, d**-0.5, 1024, 1.0, out, longest)
+  torch.cuda.synchronize()
+  k, v = kc[0, 0, :5].double(), vc[0, 0, :, :5].t().double()
+  w = torch.sigmoid(q.double() @ k.t() * d**-0.5 + pb.double()[:, None])
+  pos = torch.cat([torch.zeros(B - 1, dtype=torch.long), torch.arange(5)]).cuda()
+  w = w * (torch.arange(5, device="cuda") <= pos[:, None])[:, None]
+  _near(out, (w @ v).reshape(T, H * d))

@@ -896,10 +896,11 @@ void attn_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tenso
 }
 
 // A decode step whose contexts are cut by their lengths counts its pages over all KV heads in 32 bits.  Past that a part would be too
-// short, the parts more than the places, and a sequence without all of its parts never merged.
+// short, the parts more than the places, and a sequence without all of its parts never merged.  Its pairs are workgroups of 256 in one
+// dimension of a launch, which holds 2^32 work items.
 static bool decode_sizes_ok(int64_t B, int64_t Hkv, int64_t max_blocks) {
   return B >= 1 && B <= (1 << 20) && Hkv >= 1 && Hkv <= (1 << 20) && max_blocks >= 1 && max_blocks <= (1 << 24) &&
-         B * Hkv < (int64_t(1) << 30) && B * Hkv * max_blocks < (int64_t(1) << 30);
+         B * Hkv <= (1 << 23) && B * Hkv * max_blocks < (int64_t(1) << 30);
 }
 
 // the plan of attn_decode_split: int32 [places, 8] (see kernels.h DecodePart), written by one launch

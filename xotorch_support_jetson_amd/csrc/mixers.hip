@@ -570,18 +570,16 @@ template <int NK>
 __global__ __launch_bounds__(256) void attn_gated_chunk_mfma_k(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int* __restrict__ block_tables, int width, const int* __restrict__ cu_q, const int* __restrict__ ctx_lens,
-    const float* __restrict__ pb, float scale, int chunk, float out_scale, uint16_t* __restrict__ out, int ldo, int H, int G, int B,
-    int tiles) {
+    const float* __restrict__ pb, float scale, int chunk, float out_scale, uint16_t* __restrict__ out, int ldo, int H, int G, int B) {
   constexpr int D = NK * 32, ND = NK * 2, QT = 2;
   constexpr int KT = D > 192 ? 32 : 64;  // keys per tile (a page holds a whole number of tiles)
   constexpr int KP = D + 8, VP = KT + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sK[KT][KP], sV[D][VP];
-  const uint32_t place = blockIdx.x / (uint32_t)H, turn = place / (uint32_t)tiles;
-  const int h = (int)(blockIdx.x - place * H);
-  const int b = nth_longest(B, (int)turn, [&](int j) { return cu_q[j + 1] - cu_q[j]; });
+  const int h = blockIdx.x;
+  const int b = nth_longest(B, (int)blockIdx.z, [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, g4 = l >> 4;
   const int t0 = cu_q[b], qlen = cu_q[b + 1] - t0, ctx = ctx_lens[b];
-  const int wq0 = (int)(place - turn * tiles) * 128;
+  const int wq0 = blockIdx.y * 128;
   if (ctx <= 0 || wq0 >= qlen) return;
   const int q0 = wq0 + wave * 32;
   const bool active = q0 < qlen;
@@ -1131,10 +1129,10 @@ template <int NK>
 void launch_attn_mfma(int B, int tiles, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                       const at::Tensor& block_tables, const at::Tensor& cu_q, const at::Tensor& ctx_lens, const at::Tensor& pb,
                       float scale, int chunk, float out_scale, at::Tensor& out, int ldo, int H, int G) {
-  attn_gated_chunk_mfma_k<NK><<<(unsigned)(B * H) * tiles, 256, 0, stream()>>>(
+  attn_gated_chunk_mfma_k<NK><<<dim3((unsigned)H, (unsigned)tiles, (unsigned)B), 256, 0, stream()>>>(
       (const uint16_t*)q.data_ptr(), (const uint16_t*)k_cache.data_ptr(), (const uint16_t*)v_cache.data_ptr(),
       block_tables.data_ptr<int>(), (int)block_tables.size(1), cu_q.data_ptr<int>(), ctx_lens.data_ptr<int>(),
-      pb.data_ptr<float>(), scale, chunk, out_scale, (uint16_t*)out.data_ptr(), ldo, H, G, B, tiles);
+      pb.data_ptr<float>(), scale, chunk, out_scale, (uint16_t*)out.data_ptr(), ldo, H, G, B);
 }
 
 // max_qlen: the longest run of new tokens of one sequence in this step (1: single decoded tokens -> the wave-per-token
