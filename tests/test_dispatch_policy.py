@@ -1,5 +1,6 @@
 """Host-side dispatch policy (CPU): decode-attention partitioning per batch / block-table width, and the
 GEMM tuner's split-K slab charge.  The kernels these choices select are covered in tests/test_kernels_gpu.py."""
+import pytest
 import torch
 
 from xotorch_support_jetson_amd.ops import kernels as K
@@ -179,6 +180,24 @@ def test_qkv_projection_is_timed_with_what_follows_it(monkeypatch):
   monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
   L.linear_rope_kv(x, w, None, None, None, None, kc, vc, H, Hkv)
   assert list(pol.table.values()) == [("big", 128, 2)] and ran[-2:] == ["slabs", "rotate"] and ran.count("whole") == ran.count("write") == 1
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_a_timed_run_is_not_charged_for_its_slabs_again(monkeypatch, whole):
+  """Where the caller's whole step is timed, the read of the slabs lies in the timing; a product alone is charged for it."""
+  M, N, Kd = 512, 3072, 2048
+  read = L._slab_read_ms(("big", 128, 4), M, N)
+  took = {("big", 128, 1): 1.0, ("big", 128, 4): 1.0 - read / 2}
+  pol, now = L.GemmPolicy(), []
+  pol._path_resolved = True
+  for name, value in (("_no_tuning", lambda self: False), ("_time", staticmethod(lambda fn: (fn(), took[now[-1]])[1])),
+                      ("_big_cands", staticmethod(lambda *a: list(took))), ("_stream_cands", staticmethod(lambda *a: []))):
+    monkeypatch.setattr(L.GemmPolicy, name, value)
+  monkeypatch.setattr(L, "_shuffled_call", lambda x, w, b, r, e, y, cfg: now.append(cfg))
+  monkeypatch.setattr(L.scratch, "splitk", lambda dev, n, slot=0: None)
+  x, w = (torch.empty(*s, dtype=torch.bfloat16, device="meta") for s in ((M, Kd), (N, Kd)))
+  got = pol.shuffled_cfg(x, w, None, None, "none", torch.bfloat16, run=now.append if whole else None)
+  assert got == ("big", 128, 4 if whole else 1)
 
 
 def test_untuned_choice_without_stream_candidates(monkeypatch):

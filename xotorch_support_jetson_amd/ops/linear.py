@@ -519,7 +519,8 @@ class GemmPolicy:
     for cfg in cands:
       try:
         call = _slab_call if slabs and cfg[2] > 1 else _shuffled_call
-        times[cfg] = self._time(lambda: run(cfg) if run else call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
+        # (a run reads its slabs itself; for the others the read is charged)
+        times[cfg] = self._time(lambda: run(cfg)) if run else self._time(lambda: call(x, w, bias, residual, epi, y, cfg)) + _slab_read_ms(cfg, M, N)
         if slabs and cfg[2] > 1 and M <= SOLO_MAX_M:
           times[cfg] += 1e-4 * cfg[2]  # a row's reader waits about 0.1 us for each slab more (11 of 2048 columns 1.0 us, of 6 rows 1.5)
       except RuntimeError:
