@@ -96,7 +96,7 @@ def test_rope_and_cache_write(gpu, M, H, Hkv, Dh, bias):
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,S", [(128, 1), (2048, 3), (2176, 8), (4096, 4), (8192, 5)])
 def test_norm_prologue_is_the_unfused_row(gpu, D, S):
-  """One row whose residual add and RMS norm run in the prologue: the residual and the product bit for bit those of the slab
+  """One row whose RMS norm runs in the prologue: the residual and the product bit for bit those of the slab
   reduce followed by the plain kernel, with and without the gated epilogue and the rotation."""
   from xotorch_support_jetson_amd.ops._ext import require
   g = torch.Generator(device=gpu).manual_seed(D)
@@ -106,17 +106,16 @@ def test_norm_prologue_is_the_unfused_row(gpu, D, S):
   N = (H + 2 * Hkv) * Dh
   w = shuffle_for_stream((rn(N, D) / D ** 0.5).to(torch.bfloat16))
   w.xot_layout = "stream"
-  p = L.PendingNorm(h, torch.zeros_like(h), slabs, S, None, lnw, 1e-5)
-  xn = L.PendingNorm(h, torch.zeros_like(h), slabs, S, None, lnw, 1e-5).materialize()
-  C = require()
+  C, m, xn = require(), h.clone(), torch.empty_like(h)
+  C.splitk_resid_rmsnorm(slabs, S, None, m, lnw, xn, 1e-5)  # the sum of the slabs: the row the prologue reads
+  p = L.PendingNorm(m.clone(), torch.zeros_like(h), lnw, 1e-5)
+  assert torch.equal(L.PendingNorm(m.clone(), torch.zeros_like(h), lnw, 1e-5).materialize(), xn)
   for epi, nt, n in (("none", 1, N), ("none", 4, N), ("silu", 2, N // 2)):
     y, z = (torch.zeros(1, n, dtype=torch.bfloat16, device=gpu) for _ in range(2))
     p.run_wave(w, y, None, epi, nt)
     C.gemm_wave(xn, w, z, None, None, K.EPI[epi], nt)
     assert torch.equal(y, z), (epi, nt)
-  m = h.clone()
-  C.splitk_resid_rmsnorm(slabs, S, None, m, lnw, torch.empty_like(m), 1e-5)
-  assert torch.equal(p.dst, m)
+  assert torch.equal(p.dst, m) and torch.equal(p.src, m)
   tab, pos, slots = rn(16, Dh), torch.tensor([5], dtype=torch.int32, device=gpu), torch.tensor([9], device=gpu)
   got = []
   for fused in (True, False):

@@ -286,13 +286,12 @@ void gemm_stream(const at::Tensor& x, const at::Tensor& w, at::Tensor& y, const 
          " splits=", splits);
 }
 
-// Batch-1 decode GEMM on pre-shuffled weights whose input row is rmsnorm(bf16(h + bias_in + sum of the S_in slabs of
-// ws_in)) * lnw, computed in the GEMM's prologue; the summed residual row is stored to hout (!= h).  y = [1, N] (epi 0)
-// or [1, N / 2] (epi 2, SiLU * up); splits > 1 writes fp32 slabs into ws (!= ws_in), reduced unless reduce = false.
+// Batch-1 decode GEMM on pre-shuffled weights whose input row is rmsnorm(h) * lnw, computed in the GEMM's prologue; h is
+// stored to hout (!= h) too.  y = [1, N] (epi 0) or [1, N / 2] (epi 2, SiLU * up); splits > 1 writes fp32 slabs into ws,
+// reduced unless reduce = false.
 void gemm_stream_norm(const at::Tensor& w, at::Tensor& y, const c10::optional<at::Tensor>& bias,
                       const c10::optional<at::Tensor>& ws, int64_t epi, int64_t ntw, int64_t splits, bool reduce,
-                      const at::Tensor& h, const c10::optional<at::Tensor>& ws_in, int64_t s_in,
-                      const c10::optional<at::Tensor>& bias_in, const at::Tensor& lnw, at::Tensor& hout, double eps) {
+                      const at::Tensor& h, const at::Tensor& lnw, at::Tensor& hout, double eps) {
   CHECK_BF16(w);
   CHECK_BF16(h);
   CHECK_BF16(lnw);
@@ -311,10 +310,6 @@ void gemm_stream_norm(const at::Tensor& w, at::Tensor& y, const c10::optional<at
     CHECK_BF16((*bias));
     XCHECK(bias->numel() == N && bias->is_contiguous(), "gemm_stream_norm: bias");
   }
-  if (bias_in.has_value()) {
-    CHECK_BF16((*bias_in));
-    XCHECK(bias_in->numel() == K && bias_in->is_contiguous(), "gemm_stream_norm: bias_in");
-  }
   float* wsp = nullptr;
   long ws_elems = 0;
   if (ws.has_value()) {
@@ -324,28 +319,18 @@ void gemm_stream_norm(const at::Tensor& w, at::Tensor& y, const c10::optional<at
     wsp = ws->data_ptr<float>();
     ws_elems = ws->numel();
   }
-  xot::NormPro np{bf(h), nullptr, K, (int)s_in, bf_opt(bias_in), bf(lnw), bf(hout), (float)eps, (int)K};
-  if (s_in > 0) {
-    XCHECK(ws_in.has_value(), "gemm_stream_norm: ws_in");
-    CHECK_GPU((*ws_in));
-    CHECK_DT((*ws_in), at::kFloat);
-    XCHECK(ws_in->is_contiguous() && ws_in->numel() >= s_in * K, "gemm_stream_norm: ws_in holds s_in slabs of K");
-    np.ws = ws_in->data_ptr<float>();
-  }
+  const xot::NormPro np{bf(h), bf(lnw), bf(hout), (float)eps, (int)K};
   const int rc = xot::launch_gemm_stream_norm(bf(w), bf_opt(bias), y.data_ptr(), (int)y.stride(0), (int)epi, wsp,
                                               ws_elems, (int)N, (int)K, (int)ntw, (int)splits, reduce, np,
                                               cur_stream());
-  XCHECK(rc == 0, "gemm_stream_norm: unsupported N=", N, " K=", K, " epi=", epi, " ntw=", ntw, " splits=", splits,
-         " s_in=", s_in);
+  XCHECK(rc == 0, "gemm_stream_norm: unsupported N=", N, " K=", K, " epi=", epi, " ntw=", ntw, " splits=", splits);
 }
 
 // Decode GEMM on whole K sums (gemm_wave.hip).  x [M, K], or (norm row) none and h .. eps as in gemm_stream_norm; y as in
 // gemm_stream, or (rope) none and pos .. Hkv as in splitk_rope_kv_write.
 void gemm_wave(const c10::optional<at::Tensor>& x, const at::Tensor& w, const c10::optional<at::Tensor>& y,
                const c10::optional<at::Tensor>& bias, const c10::optional<at::Tensor>& res, int64_t epi, int64_t nt, double epi_arg,
-               const c10::optional<at::Tensor>& h, const c10::optional<at::Tensor>& ws_in, int64_t s_in,
-               const c10::optional<at::Tensor>& bias_in, const c10::optional<at::Tensor>& lnw, const c10::optional<at::Tensor>& hout,
-               double eps, const c10::optional<at::Tensor>& pos, const c10::optional<at::Tensor>& cos_sin,
+               const c10::optional<at::Tensor>& h, const c10::optional<at::Tensor>& lnw, const c10::optional<at::Tensor>& hout, double eps, const c10::optional<at::Tensor>& pos, const c10::optional<at::Tensor>& cos_sin,
                const c10::optional<at::Tensor>& slots, const c10::optional<at::Tensor>& q_out, const c10::optional<at::Tensor>& k_cache,
                const c10::optional<at::Tensor>& v_cache, int64_t H, int64_t Hkv) {
   CHECK_BF16(w);
@@ -374,18 +359,7 @@ void gemm_wave(const c10::optional<at::Tensor>& x, const at::Tensor& w, const c1
     XCHECK(h->dim() == 2 && h->size(0) == 1 && h->size(1) == K && h->is_contiguous() && hout->sizes() == h->sizes() &&
                hout->is_contiguous() && hout->data_ptr() != h->data_ptr() && lnw->numel() == K && lnw->is_contiguous(),
            "gemm_wave: h, hout must be distinct [1, K] rows, lnw [K]");
-    if (bias_in.has_value()) {
-      CHECK_BF16((*bias_in));
-      XCHECK(bias_in->numel() == K && bias_in->is_contiguous(), "gemm_wave: bias_in");
-    }
-    a.np = xot::NormPro{bf(*h), nullptr, (long)K, (int)s_in, bf_opt(bias_in), bf(*lnw), bf(*hout), (float)eps, (int)K};
-    if (s_in > 0) {
-      XCHECK(ws_in.has_value(), "gemm_wave: ws_in");
-      CHECK_GPU((*ws_in));
-      CHECK_DT((*ws_in), at::kFloat);
-      XCHECK(ws_in->is_contiguous() && ws_in->numel() >= s_in * K, "gemm_wave: ws_in holds s_in slabs of K");
-      a.np.ws = ws_in->data_ptr<float>();
-    }
+    a.np = xot::NormPro{bf(*h), bf(*lnw), bf(*hout), (float)eps, (int)K};
     a.M = 1;
   }
   if (bias.has_value()) {
@@ -428,7 +402,7 @@ void gemm_wave(const c10::optional<at::Tensor>& x, const at::Tensor& w, const c1
                         slots->data_ptr<int64_t>(), (int)H, (int)Hkv, (int)Dh, (int)BS, (int)cos_sin->size(0), nb * BS};
   }
   const int rc = xot::launch_gemm_wave(a, f32, (int)epi, (int)nt, cur_stream());
-  XCHECK(rc == 0, "gemm_wave: unsupported M=", a.M, " N=", N, " K=", K, " epi=", epi, " nt=", nt, " s_in=", s_in);
+  XCHECK(rc == 0, "gemm_wave: unsupported M=", a.M, " N=", N, " K=", K, " epi=", epi, " nt=", nt);
 }
 
 // Decode GEMM on FP8 (e4m3) pre-shuffled weights w8 [N, K] uint8 with per-row fp32 scales (y = x . (w8 * s)^T).
@@ -1240,8 +1214,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("ws"), py::arg("epi"), py::arg("ntw"), py::arg("splits"), py::arg("wshuf"),
         py::arg("reduce") = true, py::arg("epi_arg") = 0.0);
   m.def("gemm_stream_norm", &gemm_stream_norm, py::arg("w"), py::arg("y"), py::arg("bias"), py::arg("ws"),
-        py::arg("epi"), py::arg("ntw"), py::arg("splits"), py::arg("reduce"), py::arg("h"), py::arg("ws_in"),
-        py::arg("s_in"), py::arg("bias_in"), py::arg("lnw"), py::arg("hout"), py::arg("eps"));
+        py::arg("epi"), py::arg("ntw"), py::arg("splits"), py::arg("reduce"), py::arg("h"), py::arg("lnw"),
+        py::arg("hout"), py::arg("eps"));
   m.def("gemm_stream8", &gemm_stream8, py::arg("x"), py::arg("w8"), py::arg("wscale"), py::arg("y"), py::arg("bias"),
         py::arg("res"), py::arg("ws"), py::arg("epi"), py::arg("ntw"), py::arg("splits"), py::arg("reduce") = true);
   m.def("relayout", &relayout, py::arg("src"), py::arg("dst"), py::arg("mode"));
@@ -1250,8 +1224,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_batched", &gemm_batched, py::arg("x"), py::arg("xbat"), py::arg("K"), py::arg("w"), py::arg("y"),
         py::arg("ybat"), py::arg("ldy"), py::arg("M"));
   m.def("gemm_wave", &gemm_wave, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("bias"), py::arg("res"), py::arg("epi"),
-        py::arg("nt"), py::arg("epi_arg") = 0.0, py::arg("h") = py::none(), py::arg("ws_in") = py::none(), py::arg("s_in") = 0,
-        py::arg("bias_in") = py::none(), py::arg("lnw") = py::none(), py::arg("hout") = py::none(), py::arg("eps") = 0.0,
+        py::arg("nt"), py::arg("epi_arg") = 0.0, py::arg("h") = py::none(), py::arg("lnw") = py::none(), py::arg("hout") = py::none(),
+        py::arg("eps") = 0.0,
         py::arg("pos") = py::none(), py::arg("cos_sin") = py::none(), py::arg("slots") = py::none(), py::arg("q_out") = py::none(),
         py::arg("k_cache") = py::none(), py::arg("v_cache") = py::none(), py::arg("H") = 0, py::arg("Hkv") = 0);
   m.def("gemm_big", &gemm_big, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("bias"), py::arg("res"),

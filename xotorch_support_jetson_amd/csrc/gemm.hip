@@ -368,66 +368,22 @@ __global__ __launch_bounds__(256, OCC) void gemm_stream_kernel(const uint16_t* _
   wload(wa, 0);
   wload(wb, min(1, last));
   {
-    // RMSNorm prologue (one input row; NORM = 16-B chunks of the row per thread): the first two weight chunks,
-    // then every residual / bias / norm-weight load and the first SMAX slabs are requested before any is used,
-    // so the chain is one L2 round trip per SMAX slabs (the producer just wrote them), one wave reduction and two
-    // barriers, under the weight stream's own HBM latency.  Same arithmetic and reduction order as
+    // RMSNorm prologue (one input row; NORM = 16-B chunks of the row per thread): the first two weight chunks, then the
+    // row and the norm weight are requested, so the chain is one L2 round trip, one wave reduction and two barriers,
+    // under the weight stream's own HBM latency.  Same arithmetic and reduction order as
     // splitk_resid_rmsnorm_kernel<*, *, 256>: the row is bitwise the one the unfused pair gives.
-    constexpr int PM = NORM, SMAX = NORM >= 4 ? 2 : 8;  // slabs per round trip (registers: PM x SMAX x 8)
+    constexpr int PM = NORM;
     __shared__ float nred[NTH / 64];
     const int nchunk = np.D >> 3, c0 = kb >> 3, c1 = (kb + kper) >> 3;
     const bool wg0 = blockIdx.x == 0 && blockIdx.y == 0;
-    s16x8 ha[PM], ba[PM], la[PM];
-    f32x4 p[PM][SMAX][2];
-    // slabs s0 .. s0 + SMAX - 1 of this thread's chunks (all requested before any is added)
-    auto slabs = [&](int s0) {
-#pragma unroll
-      for (int i = 0; i < PM; ++i) {
-        const int cc = tid + NTH * i;
-        if (cc < nchunk) {
-#pragma unroll
-          for (int sl = 0; sl < SMAX; ++sl)
-            if (s0 + sl < np.S) {
-              const float* sp = np.ws + (s0 + sl) * np.sstride + cc * 8;
-              p[i][sl][0] = *reinterpret_cast<const f32x4*>(sp);
-              p[i][sl][1] = *reinterpret_cast<const f32x4*>(sp + 4);
-            }
-        }
-      }
-    };
+    s16x8 ha[PM], la[PM];
 #pragma unroll
     for (int i = 0; i < PM; ++i) {
       const int cc = tid + NTH * i;
       if (cc < nchunk) {
         ha[i] = ld16(np.h + cc * 8);
-        if (np.bias != nullptr) ba[i] = ld16(np.bias + cc * 8);
         if (cc >= c0 && cc < c1) la[i] = ld16(np.lnw + cc * 8);
       }
-    }
-    slabs(0);
-    float v[PM][8];
-#pragma unroll
-    for (int i = 0; i < PM; ++i) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = bf2f(ha[i][j]);
-      if (np.bias != nullptr) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] += bf2f(ba[i][j]);
-      }
-    }
-    for (int s0 = 0; s0 < np.S; s0 += SMAX) {  // one L2 round trip per SMAX slabs
-      if (s0 > 0) slabs(s0);
-#pragma unroll
-      for (int i = 0; i < PM; ++i)
-#pragma unroll
-        for (int sl = 0; sl < SMAX; ++sl)
-          if (s0 + sl < np.S) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              v[i][j] += p[i][sl][0][j];
-              v[i][4 + j] += p[i][sl][1][j];
-            }
-          }
     }
     float ss = 0.f;
 #pragma unroll
@@ -436,7 +392,6 @@ __global__ __launch_bounds__(256, OCC) void gemm_stream_kernel(const uint16_t* _
       if (cc < nchunk) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          ha[i][j] = (short)f2bf(v[i][j]);
           const float r = bf2f(ha[i][j]);
           ss += r * r;
         }
@@ -854,11 +809,9 @@ int launch_gemm_stream_norm(const uint16_t* W, const uint16_t* bias, void* Y, in
   if (epi != EPI_NONE && epi != EPI_SILU) return -1;
   if (epi == EPI_SILU || ntw == 4) ntw = 2;  // one row: NTW 4 is never picked (stream_dispatch)
   if (ntw != 1 && ntw != 2) return -1;
-  if (np.D != K || K % 8 != 0 || K > 8 * 256 * 4 || np.S < 0 || np.S > 8 || np.h == nullptr || np.lnw == nullptr || np.hout == nullptr)
-    return -1;
-  if (np.S > 0 && (np.ws == nullptr || np.sstride < K)) return -1;
+  if (np.D != K || K % 8 != 0 || K > 8 * 256 * 4 || np.h == nullptr || np.lnw == nullptr || np.hout == nullptr) return -1;
   if (S < 1 || N % (64 * ntw) != 0 || K % (S * 128) != 0 || (long)(K / S) * 2 > 65536) return -1;
-  if (S > 1 && (ws == nullptr || ws == np.ws || ws_elems < (long)S * N)) return -1;
+  if (S > 1 && (ws == nullptr || ws_elems < (long)S * N)) return -1;
   const int pm = (K / 8 + 255) / 256;  // 16-B chunks of the row per thread
   auto go = [&](auto pmc) {
     constexpr int PM = decltype(pmc)::value;

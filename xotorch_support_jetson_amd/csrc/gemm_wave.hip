@@ -13,8 +13,8 @@
 // 16384 x 2048 SiLU 15.8 / 12.3 (a plain read: 12.6), 6 rows 11264 x 2048 clamped 13.9 / 10.9, 6144 x 2048 8.4 / 7.0, 12 rows
 // 128256 x 2048 94 (gemm_stream) / 86.  Beyond 16 rows, gemm_stream / here: 48 x 20224 x 2048 23.3 / 19.6, 37 x 21888 x 2048 SiLU
 // 25.9 / 20.6, 24 x 28672 x 4096 SiLU 47.2 / 45.2, 24 x 6144 x 4096 with RoPE 16.3 / 15.2.
-// NORM (batch-1 decode): the input row is rmsnorm(residual + the previous projection's slabs), computed by the first four waves
-// in splitk_resid_rmsnorm's order while all have their first weight blocks in flight.
+// NORM (batch-1 decode): the input row is rmsnorm(residual), computed by the first four waves in splitk_resid_rmsnorm's order while all
+// have their first weight blocks in flight.
 #include <algorithm>
 
 #include "common.h"
@@ -35,8 +35,8 @@ __device__ __forceinline__ s16x8 buf16(__amdgpu_buffer_rsrc_t r, unsigned off, b
 
 // MT: 16-row tiles of X.  XL: X pieces (1 KB) a wave copies per chunk.  rw: rows of X kept in LDS (a power of two >= M up to 16,
 // whole tiles beyond; MFMA rows past it repeat them)
-template <int MT, int KW, int XL, int EPI, bool F32, int NORM, int SM, bool ROPE>
-__global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE ? 4 : 2) void gemm_wave_kernel(const uint16_t* __restrict__ X, int ldx, const uint16_t* __restrict__ W,
+template <int MT, int KW, int XL, int EPI, bool F32, int NORM, bool ROPE>
+__global__ __launch_bounds__(512, MT == 1 && XL <= 4 && !ROPE ? 4 : 2) void gemm_wave_kernel(const uint16_t* __restrict__ X, int ldx, const uint16_t* __restrict__ W,
                                                         const uint16_t* __restrict__ bias, const uint16_t* __restrict__ R,
                                                         int ldr, void* __restrict__ Yv, int ldy, int M, int N, int K, int rw,
                                                         float epi_arg, NormPro np, RopeOut ro) {
@@ -165,19 +165,7 @@ __global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE 
   Stage sa, sb;
   if constexpr (NORM > 0) {
     s16x8 ha[NORM], la[NORM];
-    f32x4 pv[NORM][SM][2];
     const int nchunk = np.D >> 3;
-    // SM slabs from s0 on of the thread's chunks (past the last: the last again, not added)
-    auto slabs = [&](int s0) {
-#pragma unroll
-      for (int i = 0; i < NORM; ++i)
-#pragma unroll
-        for (int sl = 0; sl < SM; ++sl) {
-          const float* sp = np.ws + min(s0 + sl, np.S - 1) * np.sstride + min((tid & 255) + 256 * i, nchunk - 1) * 8;
-          pv[i][sl][0] = *reinterpret_cast<const f32x4*>(sp);
-          pv[i][sl][1] = *reinterpret_cast<const f32x4*>(sp + 4);
-        }
-    };
     // (asked for before the weights: loads return in order, and the row's chain is the longer one)
 #pragma unroll
     for (int i = 0; i < NORM; ++i) {
@@ -185,50 +173,23 @@ __global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE 
       ha[i] = ld16(np.h + cc * 8);
       la[i] = ld16(np.lnw + cc * 8);
     }
-    if (np.S > 0) slabs(0);
     __builtin_amdgcn_sched_barrier(0);
     load(sa, 0);
     load(sb, 1);
     __builtin_amdgcn_sched_barrier(0);
     if (rope_here) rope_table(wave);
     __builtin_amdgcn_sched_barrier(0);
-    // one row: residual + bias + slabs -> bf16 residual (stored by workgroup 0), its RMS norm times the weight -> LDS.  256
-    // threads, 8 consecutive elements each per round, in the order of splitk_resid_rmsnorm_kernel<*, *, 256>
+    // one row: the residual (stored again by workgroup 0), its RMS norm times the weight -> LDS.  256 threads, 8 consecutive elements
+    // each per round, in the order of splitk_resid_rmsnorm_kernel<*, *, 256>
     __shared__ float nred[4];
     if (wave < 4) {
-      float v[NORM][8], ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < NORM; ++i) {
-        const int cc = tid + 256 * i;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[i][e] = bf2f(ha[i][e]);
-        if (np.bias != nullptr && cc < nchunk) {
-          const s16x8 ba = ld16(np.bias + cc * 8);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[i][e] += bf2f(ba[e]);
-        }
-      }
-      for (int s0 = 0; s0 < np.S; s0 += SM) {
-        if (s0 > 0) slabs(s0);
-#pragma unroll
-        for (int i = 0; i < NORM; ++i)
-#pragma unroll
-          for (int sl = 0; sl < SM; ++sl)
-            if (s0 + sl < np.S) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                v[i][e] += pv[i][sl][0][e];
-                v[i][4 + e] += pv[i][sl][1][e];
-              }
-            }
-      }
+      float ss = 0.f;
 #pragma unroll
       for (int i = 0; i < NORM; ++i) {
         const int cc = tid + 256 * i;
         if (cc >= nchunk) continue;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          ha[i][e] = (short)f2bf(v[i][e]);
           const float r = bf2f(ha[i][e]);
           ss += r * r;
         }
@@ -392,7 +353,7 @@ __global__ __launch_bounds__(512, MT == 1 && XL <= 4 && NORM * SM <= 4 && !ROPE 
   }
 }
 
-template <int MT, int KW, int XL, int EPI, bool F32, int NORM, int SM, bool ROPE>
+template <int MT, int KW, int XL, int EPI, bool F32, int NORM, bool ROPE>
 int go(const WaveGemm& a, int nt, hipStream_t st) {
   constexpr int CB = U * KW;
   int rw = 16 * MT;
@@ -401,7 +362,7 @@ int go(const WaveGemm& a, int nt, hipStream_t st) {
   const int nw = nt * KW, nb = a.K / 32;
   const size_t xbytes = NORM ? (size_t)(nb + CB - 1) / CB * CB * 64 : (size_t)2 * rw * CB * 64;
   const size_t smem = std::max(xbytes, KW > 1 || ROPE || epi_is_glu(EPI) ? (size_t)nw * MT * 1024 : 0);
-  auto kern = gemm_wave_kernel<MT, KW, XL, EPI, F32, NORM, SM, ROPE>;
+  auto kern = gemm_wave_kernel<MT, KW, XL, EPI, F32, NORM, ROPE>;
   static_assert(2 * 16 * MT * CB * 64 <= 65536 && 8 * MT * 1024 <= 65536, "LDS a launch takes without asking");
   kern<<<(a.N / 16 + nt - 1) / nt, 64 * nw, smem, st>>>(a.X, a.ldx, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy, a.M, a.N, a.K, rw, a.epi_arg,
                                                         a.np, a.ro);
@@ -412,34 +373,34 @@ int go(const WaveGemm& a, int nt, hipStream_t st) {
 // 1 row by single tiles, 4 / 8 waves 5.0 / 5.2, 6144 x 2048 at 6 rows 8.0 / 10.2; 11264 x 2048 by fours, 1 / 2 waves 12.2 / 10.9.
 // More rows: the chunk's X takes the LDS that more parts would need, and the waves' stages are enough in flight: 20224 x 2048 at
 // 48 rows by threes, 1 / 2 waves 20.8 / 24.1; two only beside a lone pair (6144 x 4096 at 24 rows 16.4 / 14.7).
-template <int EPI, bool F32, int NORM, int SM, bool ROPE>
+template <int EPI, bool F32, int NORM, bool ROPE>
 int one_row_tile(const WaveGemm& a, int nt, hipStream_t st) {
   constexpr bool LONE = !ROPE && !epi_is_glu(EPI);
   if (nt == 1) {
-    if constexpr (LONE) return go<1, 4, NORM ? 4 : 8, EPI, F32, NORM, SM, ROPE>(a, nt, st);  // (half the waves copy X)
+    if constexpr (LONE) return go<1, 4, NORM ? 4 : 8, EPI, F32, NORM, ROPE>(a, nt, st);  // (half the waves copy X)
     else return -1;
   }
-  if (nt == 2) return go<1, 4, 4, EPI, F32, NORM, SM, ROPE>(a, nt, st);
-  return nt <= 4 ? go<1, 2, 4, EPI, F32, NORM, SM, ROPE>(a, nt, st) : -1;
+  if (nt == 2) return go<1, 4, 4, EPI, F32, NORM, ROPE>(a, nt, st);
+  return nt <= 4 ? go<1, 2, 4, EPI, F32, NORM, ROPE>(a, nt, st) : -1;
 }
 
 template <int EPI, bool F32, bool ROPE>
 int by_rows(const WaveGemm& a, int nt, hipStream_t st) {
   const int mt = (a.M + 15) / 16;
-  if (mt == 1) return one_row_tile<EPI, F32, 0, 1, ROPE>(a, nt, st);
+  if (mt == 1) return one_row_tile<EPI, F32, 0, ROPE>(a, nt, st);
   if (nt < mt) return -1;  // (a wave copies at most eight pieces of a chunk)
-  if (mt == 2) return nt == 2 ? go<2, 2, 8, EPI, F32, 0, 1, ROPE>(a, nt, st) : go<2, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st);
-  return mt == 3 ? go<3, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st) : go<4, 1, 8, EPI, F32, 0, 1, ROPE>(a, nt, st);
+  if (mt == 2) return nt == 2 ? go<2, 2, 8, EPI, F32, 0, ROPE>(a, nt, st) : go<2, 1, 8, EPI, F32, 0, ROPE>(a, nt, st);
+  return mt == 3 ? go<3, 1, 8, EPI, F32, 0, ROPE>(a, nt, st) : go<4, 1, 8, EPI, F32, 0, ROPE>(a, nt, st);
 }
 
-template <int NORM, int SM>
+template <int NORM>
 int normed(const WaveGemm& a, int epi, int nt, hipStream_t st) {
-  if (a.ro.q != nullptr) return one_row_tile<EPI_NONE, false, NORM, SM, true>(a, nt, st);
-  return epi == EPI_SILU ? one_row_tile<EPI_SILU, false, NORM, SM, false>(a, nt, st)
-                         : one_row_tile<EPI_NONE, false, NORM, SM, false>(a, nt, st);
+  if (a.ro.q != nullptr) return one_row_tile<EPI_NONE, false, NORM, true>(a, nt, st);
+  return epi == EPI_SILU ? one_row_tile<EPI_SILU, false, NORM, false>(a, nt, st)
+                         : one_row_tile<EPI_NONE, false, NORM, false>(a, nt, st);
 }
 
-// Up to 16 rows, one column tile a workgroup (HALF: half of one, its eight columns), the eight waves a part of K each: a wave copies
+// Up to 8 rows, one column tile a workgroup (HALF: half of one, its eight columns), the eight waves a part of K each: a wave copies
 // the rows of X that its own blocks need through LDS of its own, so no wave waits for another before the partial tiles meet.
 // HALF: a load takes the tile half's 128-byte runs of two k blocks, the first in columns 0 .. 7 of the MFMA operand, the second in
 // 8 .. 15; each block's rows of X multiply it all and the sums of the other block's columns are not used.
@@ -610,8 +571,7 @@ int solo_rows(const WaveGemm& a, hipStream_t st) {
   gemm_solo_kernel<HALF, XLV, EPI, F32><<<grid, 512, 0, st>>>(a.X, a.ldx, a.W, a.bias, a.R, a.ldr, a.Y, a.ldy, a.M, a.N, a.K, a.mg)
   if (a.M <= 2) XOT_SOLO(1);
   else if (a.M <= 4) XOT_SOLO(2);
-  else if (a.M <= 8) XOT_SOLO(4);
-  else XOT_SOLO(8);
+  else XOT_SOLO(4);
 #undef XOT_SOLO
   return 0;
 }
@@ -640,19 +600,17 @@ int launch_gemm_wave(const WaveGemm& a, bool out_f32, int epi, int nt, hipStream
   if ((rope || epi_is_glu(epi)) && (nt % 2 != 0 || a.N % 32 != 0)) return -1;
   if (rope && (epi != EPI_NONE || out_f32 || a.ro.Dh % 32 != 0 || a.N != (a.ro.H + 2 * a.ro.Hkv) * a.ro.Dh || a.ro.max_pos < 1)) return -1;
   if (norm) {
-    if (nt == 0 || a.M != 1 || out_f32 || (epi != EPI_NONE && epi != EPI_SILU) || a.np.D != a.K || a.K > 8192 || a.np.S < 0 ||
-        a.np.lnw == nullptr || a.np.hout == nullptr || (a.np.S > 0 && (a.np.ws == nullptr || a.np.sstride < a.K)))
+    if (nt == 0 || a.M != 1 || out_f32 || (epi != EPI_NONE && epi != EPI_SILU) || a.np.D != a.K || a.K > 8192 || a.np.lnw == nullptr ||
+        a.np.hout == nullptr)
       return -1;
-    // (slabs of the first round trip: 8 where the row is short, or they would keep a second workgroup off the CU)
-    if (a.K <= 2048) return a.np.S > 4 ? normed<1, 8>(a, epi, nt, st) : normed<1, 4>(a, epi, nt, st);
-    return a.K <= 4096 ? normed<2, 4>(a, epi, nt, st) : normed<4, 2>(a, epi, nt, st);
+    return a.K <= 2048 ? normed<1>(a, epi, nt, st) : a.K <= 4096 ? normed<2>(a, epi, nt, st) : normed<4>(a, epi, nt, st);
   }
   if (a.mg.o != nullptr) {  // (two chunks of K)
     if (nt != 0 || a.M != 1 || out_f32 || epi != EPI_RESID || rope || norm || a.K > 2 * 2048 || a.mg.max_parts > MERGE_PARTS || a.K % a.mg.Dh != 0) return -1;
     return a.N <= 2048 ? solo_merge<true>(a, st) : solo_merge<false>(a, st);
   }
   if (nt == 0) {
-    if (rope || norm || a.M > 16) return -1;
+    if (rope || norm || a.M > 8) return -1;
     if (epi == EPI_RESID) return out_f32 ? -1 : solo<EPI_RESID, false>(a, st);
     if (epi != EPI_NONE) return -1;
     return out_f32 ? solo<EPI_NONE, true>(a, st) : solo<EPI_NONE, false>(a, st);

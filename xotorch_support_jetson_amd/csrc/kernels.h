@@ -33,17 +33,11 @@ int launch_gemm_skinny(const uint16_t* X, int ldx, const uint16_t* W, int ldw, c
 int launch_gemm_stream(const uint16_t* X, int ldx, const uint16_t* W, int ldw, const uint16_t* bias,
                        const uint16_t* R, int ldr, void* Y, int ldy, bool out_f32, int epi, float* ws, long ws_elems,
                        int M, int N, int K, int ntw, int S, bool wshuf, bool reduce, float epi_arg, hipStream_t s);
-// Batch-1 decode GEMM whose input row is the RMSNorm of a residual projection's pending split-K sum:
-// x = rmsnorm(bf16(h + bias + sum_s ws[s])) * lnw, recomputed by every workgroup from the slabs (no separate
-// reduce + norm launch); workgroup (0, 0) stores the summed residual row to hout (never h itself: the other
-// workgroups are still reading h).  Pre-shuffled bf16 weights, epi none / silu, split-K into ws (a different
-// buffer from np.ws).
+// Batch-1 decode GEMM whose input row is the residual row's RMSNorm, x = rmsnorm(h) * lnw, recomputed by every workgroup
+// (no norm launch); workgroup (0, 0) stores the row to hout too (never h itself: the other workgroups are still reading
+// h).  Pre-shuffled bf16 weights, epi none / silu, split-K into ws.
 struct NormPro {
   const uint16_t* h;
-  const float* ws;
-  long sstride;
-  int S;
-  const uint16_t* bias;
   const uint16_t* lnw;
   uint16_t* hout;
   float eps;

@@ -1149,8 +1149,8 @@ class ShardModel:
     last = self.shard.is_last_layer()
     n = len(self.layer_ids)
     xn, _ = K.rmsnorm(h, w.layers[self.layer_ids[0]].ln1, c.rms_norm_eps) if n else (None, None)
-    # batch-1 decode: the split-K reduce + residual + RMSNorm after o_proj / down_proj is deferred into the next
-    # GEMM's prologue (ops.linear.PendingNorm); the residual stream then alternates between two row buffers
+    # batch-1 decode: the RMSNorm after o_proj / down_proj is deferred into the next GEMM's prologue
+    # (ops.linear.PendingNorm); the residual stream then alternates between two row buffers
     fuse = FUSE_NORM and h.is_cuda and h.shape[0] == 1 and not c.is_mla and n > 0
     hb = (h, torch.empty_like(h)) if fuse else None
     other = (lambda t: hb[1] if t is hb[0] else hb[0]) if fuse else (lambda t: None)

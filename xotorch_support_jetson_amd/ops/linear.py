@@ -175,9 +175,7 @@ class _Scratch:
       self._own.name = old
 
   def splitk(self, device, n: int, slot: int = 0) -> torch.Tensor:
-    """slot 1 holds the slabs of a residual projection whose reduce is deferred into the next GEMM (PendingNorm),
-    which writes its own slabs to slot 0 while it still reads slot 1, or those of the second of two projections whose
-    slabs one kernel sums."""
+    """slot 1 holds the slabs of the second of two projections whose slabs one kernel sums."""
     key = (device.index or 0, slot, self._own.name)
     t = self.ws.get(key)
     if t is None or t.numel() < n:
@@ -723,36 +721,29 @@ DEFER_MAX_D = 4096
 
 
 class PendingNorm:
-  """rmsnorm(bf16(src + bias + sum of the S fp32 slabs in ws)) * ln_w, not computed yet (S 0: rmsnorm(src) * ln_w).
+  """rmsnorm(src) * ln_w, not computed yet.
 
   A residual projection of a batch-1 decode step (linear_resid_norm with defer_to) leaves its norm; the
-  next GEMM (linear with epi none / silu, linear_rope_kv) folds the RMSNorm, and the sum of slabs if there are any, into
-  its prologue (gemm_wave, gemm_stream_norm) and stores the summed residual row into dst -- a buffer distinct from src, since
-  every workgroup of that GEMM reads src.  Any other consumer calls materialize(), the unfused kernel, which
-  leaves the same residual in dst.  After either, dst is the residual stream."""
+  next GEMM (linear with epi none / silu, linear_rope_kv) folds the RMSNorm into its prologue (gemm_wave,
+  gemm_stream_norm) and stores the residual row into dst -- a buffer distinct from src, since every workgroup of that
+  GEMM reads src.  Any other consumer calls materialize(), the unfused kernel, which leaves the same residual in dst.
+  After either, dst is the residual stream."""
 
-  __slots__ = ("src", "dst", "ws", "S", "bias", "ln_w", "eps")
+  __slots__ = ("src", "dst", "ln_w", "eps")
 
-  def __init__(self, src, dst, ws, S, bias, ln_w, eps):
-    self.src, self.dst, self.ws, self.S, self.bias, self.ln_w, self.eps = src, dst, ws, S, bias, ln_w, float(eps)
+  def __init__(self, src, dst, ln_w, eps):
+    self.src, self.dst, self.ln_w, self.eps = src, dst, ln_w, float(eps)
 
   @property
   def shape(self):
     return self.src.shape
 
   def materialize(self) -> torch.Tensor:
-    if self.S == 0:  # (the product summed by itself)
-      self.dst.copy_(self.src)
-      return K.rmsnorm(self.dst, self.ln_w, self.eps)[0]
-    if self.dst.data_ptr() != self.src.data_ptr():
-      self.dst.copy_(self.src)
-    out = torch.empty_like(self.dst)
-    require().splitk_resid_rmsnorm(self.ws, self.S, self.bias, self.dst, self.ln_w, out, self.eps)
-    return out
+    self.dst.copy_(self.src)
+    return K.rmsnorm(self.dst, self.ln_w, self.eps)[0]
 
   def run_wave(self, w: torch.Tensor, y, bias, epi: str, nt: int, **rope) -> None:
-    require().gemm_wave(None, w, y, bias, None, K.EPI[epi], nt, 0.0, self.src, self.ws, self.S, self.bias, self.ln_w, self.dst,
-                        self.eps, **rope)
+    require().gemm_wave(None, w, y, bias, None, K.EPI[epi], nt, 0.0, self.src, self.ln_w, self.dst, self.eps, **rope)
 
   def run(self, w: torch.Tensor, y, bias, epi: str, cfg: Tuple, reduce: bool = True, **rope) -> None:
     """The consumer GEMM in the configuration _pending_cfg gave (rope: outputs of the whole-K form that rotates and writes)."""
@@ -760,8 +751,7 @@ class PendingNorm:
       return self.run_wave(w, y, bias, epi, cfg[1], **rope)
     _, ntw, S = cfg
     ws = scratch.splitk(y.device, S * w.shape[0]) if S > 1 else None
-    require().gemm_stream_norm(w, y, bias, ws, K.EPI[epi], ntw, S, reduce, self.src, self.ws, self.S, self.bias,
-                               self.ln_w, self.dst, self.eps)
+    require().gemm_stream_norm(w, y, bias, ws, K.EPI[epi], ntw, S, reduce, self.src, self.ln_w, self.dst, self.eps)
 
 
 def _pending_cfg(p: PendingNorm, w: torch.Tensor, bias, epi: str, wave: str = "y"):
@@ -836,7 +826,7 @@ def merge_fits(w: torch.Tensor) -> bool:
 def _solo_norm(h, ln_w, eps, defer_to):
   """The norm behind a whole-K residual product of one row: left to the next GEMM (its residual stream in defer_to), or run."""
   if defer_to is not None and FUSE_NORM and h.shape[1] <= DEFER_MAX_D:
-    return PendingNorm(h, defer_to, None, 0, None, ln_w, eps)
+    return PendingNorm(h, defer_to, ln_w, eps)
   return K.rmsnorm(h, ln_w, eps)[0]
 
 
