@@ -491,7 +491,7 @@ def test_decode_tick_issues_no_host_sync(gpu):
 @pytest.mark.parametrize("name,defer_max_d", [("llama-3-8b", 4096), ("llama-3-8b", 0), ("tiny-qwen", 4096),
                                               ("tiny-phi3", 4096), ("tiny-mixtral", 4096)])
 def test_batch1_fused_norm_decode_matches_unfused(gpu, monkeypatch, name, defer_max_d):
-  """Batch-1 decode with the split-K reduce + residual + RMSNorm deferred into the next GEMM's prologue
+  """Batch-1 decode with the RMSNorm behind a residual product deferred into the next GEMM's prologue
   (ops.linear.PendingNorm) and the attention's partition merge done in o_proj's prologue (kernels.PendingMerge),
   the defaults, against the unfused kernels on the same weights: two Llama-3-8B layers, a 600-token context (split
   over attention partitions), eager and HIP-graph decode, bitwise-equal logits, and both fused paths really ran."""
@@ -515,7 +515,7 @@ def test_batch1_fused_norm_decode_matches_unfused(gpu, monkeypatch, name, defer_
 
   monkeypatch.setattr(L.PendingNorm, "run", counted)
   monkeypatch.setattr(KK, "attn_decode", attn)
-  monkeypatch.setattr(L, "DEFER_MAX_D", defer_max_d)  # 0: the merge-only form the 8192-wide models take
+  monkeypatch.setattr(L, "DEFER_MAX_D", defer_max_d)  # 0: the merge alone, as with rows too wide for a deferred norm
   P = 600
   ids = torch.randint(0, c.vocab_size, (P,), generator=torch.Generator().manual_seed(1), dtype=torch.int32)
 
@@ -535,7 +535,7 @@ def test_batch1_fused_norm_decode_matches_unfused(gpu, monkeypatch, name, defer_
   assert runs == {"norm": 0, "merge": 0}
   for graphs in (False, True):
     got = decode(True, graphs)
-    if name == "llama-3-8b":  # (the tiny presets' projections may not split K: then nothing is deferred)
+    if name == "llama-3-8b":  # (the tiny presets' projections may fit neither: then nothing is deferred)
       assert (runs["norm"] > 0) == (defer_max_d > 0) and runs["merge"] > 0, runs
     for a, b in zip(ref, got):
       assert torch.equal(a, b), (a.float() - b.float()).abs().max().item()

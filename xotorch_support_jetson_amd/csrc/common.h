@@ -149,7 +149,9 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
 
 // The sequence at place p of B when the longest come first (len(b); equal ones as they are given).  Each wave finds it for
 // itself: a sequence a lane, B compares, under 1 us with the loads.  Above 32 sequences the given order stays: there are then
-// several rounds of workgroups, and a long sequence met late costs the launch a small part.
+// several rounds of workgroups.  What a long sequence met late costs them, us with 4000 tokens first / last among 39 prompts of 60
+// to 360: prompt attention of 32 heads 260 / 262, chunk-local attention 79 / 91, delta-rule scans of 16 heads 464 / 635; among 99
+// 417 / 420, 139 / 151, 605 / 981.
 template <typename F>
 __device__ __forceinline__ int nth_longest(int B, int p, F len) {
   if (B <= 1 || B > 32) return p;

@@ -153,8 +153,9 @@ int launch_gemm_tiled(const uint16_t* X, int ldx, const uint16_t* W, int ldw, co
 struct __attribute__((aligned(32))) DecodePart {
   int b, first, last, parts, place, ctx, pad0, pad1;
 };
-// Parts of a sequence have at least MIN_PAGES pages (a page for each of a unit's four waves), and there are about UNITS of them over
-// all KV heads at most (two workgroups on each of 256 CUs).
+// A part holds at most ppp pages, ppp at least MIN_PAGES (a page for each of a unit's four waves); the parts of a sequence are equal to a
+// page, so they have at least half of that (5 pages: 3 + 2).  Over all KV heads there are at most B Hkv + UNITS units: one a sequence,
+// and what cutting adds (two workgroups on each of 256 CUs).
 constexpr int DECODE_MIN_PAGES = 4, DECODE_UNITS = 512;
 // places of a plan: sum over the sequences of max(1, ceil(pages / ppp)) < B + total / ppp + 1, and ppp >= total Hkv / UNITS
 inline int decode_split_places(int B, int Hkv, int max_blocks) {

@@ -22,7 +22,8 @@ constexpr int CTB = 8;  // tokens whose inputs are in flight together (runs of t
 // writes the state (else conv_tail_k does, after every token has read it).
 // Runs are bound by the vector unit nearly as much as by memory: SiLU in half the operations, the eight tokens' sums of squares
 // reduced together and their factors computed a token a lane, us before and after: 4593 tokens x 6144 channels in heads of
-// 128 63 -> 53 (226 MB: 47 at a copy's rate), 12807 x 4096 136 -> 124 (420 MB: 87), 4593 x 1024 in heads of 64 35 -> 21.
+// 128 63 -> 53 (226 MB: 47 at a copy's rate), 12807 x 4096 136 -> 124 (420 MB: 87), 4593 x 1024 in heads of 64 35 -> 21, one launch
+// behind the other.  In a step, behind other kernels, 90 -> 83 and 146 -> 131.
 struct ConvArgs {
   const float* P;  // [S][T][ldp], slabs ss apart
   int ldp, S;

@@ -152,10 +152,11 @@ def rope_apply(x: torch.Tensor, pos: torch.Tensor, cos_sin: torch.Tensor, nh: in
 #    loads under the current one (6: non-temporal)
 # 2 / 3: four waves per (sequence, KV head, partition), each as in 5, meeting in LDS (one over short tables at large batches); 3
 #    with non-temporal K / V loads
-# -1 (default): 0 below 16 (sequence, KV head) pairs, where the partitions of a single sequence are merged by the output
-#    projection's prologue; else 3 once a layer's K / V pages (batch x block-table width) outgrow the 256 MB last-level cache
-#    (256 sequences of 1900 tokens: 301 us, 331 with plain loads), 2 below (24 up to 1407 tokens: 21.3 us, 23.5 with nt).
-#    From 16 pairs on 2 also leads 0: 2 sequences x 8 heads of 130 tokens 6.3 us / 9.1, of 8000 21.0 / 29.8; 6 of 2000 15.0 / 18.8
+# -1 (default): 0 below 16 (sequence, KV head) pairs; else 3 once a layer's K / V pages (batch x block-table width) outgrow the
+#    256 MB last-level cache (256 sequences of 1900 tokens: 301 us, 331 with plain loads), 2 below (24 up to 1407 tokens: 21.3
+#    us, 23.5 with nt).  From 16 pairs on 2 also leads 0: 2 sequences x 8 heads of 130 tokens 6.3 us / 9.1, of 8000 21.0 / 29.8;
+#    6 of 2000 15.0 / 18.8.  Beside it, without routed experts: a lone sequence is always cut by its length (LONE), and from 16
+#    pairs on ragged contexts by theirs (plan_pays), in units of four waves as in 2 / 3
 # 7 / 8: as 5 / 6 with two register sets, one wave a SIMD.  With routed experts (DecodeWorkspace.routed) -1 is 0 below 64 pairs
 #    and 7 or 8 above: those sum a partition page by page and merge the partitions in order.  2 / 3 deal a context's pages to
 #    waves, sums in another order, no less exact; but a token whose experts are almost tied turns on the last bits, and its whole
