@@ -6,10 +6,13 @@ import torch
 from xotorch_support_jetson_amd.ops import kernels as K
 from xotorch_support_jetson_amd.ops import reference as R
 
+# ranks of whole eights and others: inside a block of 32, across the four blocks that are asked for first and past them
+RANKS = [(128, 128), (8, 40), (136, 16), (12, 128), (1024, 1000), (3, 5), (100, 31), (129, 255)]
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 7, 8, 9, 16, 17, 48])
-@pytest.mark.parametrize("ra,rg", [(128, 128), (8, 40), (136, 16), (12, 128), (1024, 1000), (3, 5)])
+@pytest.mark.parametrize("ra,rg", RANKS)
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("S", [1, 3, 9])
 def test_gates(T, ra, rg, dt, S):

@@ -101,11 +101,6 @@ __device__ __forceinline__ float wave_sum8(const float (&v)[8]) {
 }
 __device__ __forceinline__ constexpr int wave_sum8_lane(int i) { return 32 * (i & 1) + 16 * ((i >> 1) & 1) + 8 * (i >> 2); }
 __device__ __forceinline__ float wave_max(float v) { return group16_max(xor_max<16>(xor_max<32>(v))); }
-// sum of a quad of lanes: v + its neighbour's (lane ^ 1), then that + the other pair's
-__device__ __forceinline__ float quad_sum(float v) {
-  v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0xB1, 0xf, 0xf, false));
-  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x4E, 0xf, 0xf, false));
-}
 // the largest v of the wave with its id, the lowest id among equals
 __device__ __forceinline__ void wave_argmax(float& v, int& id) {
   auto take = [&](uint32_t ov, uint32_t oi) {

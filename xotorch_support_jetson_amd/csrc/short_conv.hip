@@ -295,9 +295,10 @@ __global__ void conv_tail_k(const float* __restrict__ P, int ldp, int S, int64_t
 // ------------------------------------------------------------------ gates
 // Workgroup = (GTOK tokens, job): job 0 the step sizes beta, then blocks of 64 decay channels, then blocks of 64 output-gate
 // channels.  The tokens' rank rows lie in LDS; a wave multiplies them with the weight rows of 16 channels on the fp32 matrix unit
-// (ranks of whole eights; else four neighbouring lanes share a channel, each sums a quarter of its weight row).  Bound by
+// (weights in pieces of eight, one by one where the rank is no whole number of eights).  Bound by
 // latencies: launch, the rank rows' way through LDS, the products.  With a channel's products on the vector unit, every lane reading
-// all tokens' rows out of LDS again, 6 tokens, two 2048 x 128 products: 10.0 us, 7.0 here; with the convolutions in one launch 9.0, 6.5.
+// all tokens' rows out of LDS again, 6 tokens, two 2048 x 128 products: 10.0 us, 7.0 here; with the convolutions in one launch 9.0, 6.5;
+// of rank 100, whose weights come one by one, 48 tokens 9.5, 7.6, one 6.1, 5.5.
 constexpr int GTOK = 16;
 constexpr int DTOK = 8;  // tokens a thread of channel_decay_k
 // the rank rows in LDS: whole 32s; consecutive tokens four banks apart (but for the longest, which 64 KB just hold)
@@ -349,14 +350,22 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
   const int rank = dec ? ra : rg, off = dec ? a1_off : g1_off, ld = gate_ld(rank), nc = dec ? HD : ng, c0 = (dec ? job : job - nab) * 64;
   const bool whole = (rank & 7) == 0;
   const int lane = threadIdx.x & 63, g = lane >> 4;
-  const int part = threadIdx.x & 3, c = c0 + (whole ? (threadIdx.x >> 6) * 16 + (lane & 15) : threadIdx.x >> 2);
+  const int c = c0 + (threadIdx.x >> 6) * 16 + (lane & 15);
   const WT* w = (dec ? a2 : g2) + (int64_t)min(c, nc - 1) * rank;
   const float rate = dec ? expf(A_log[min(c, nc - 1) / d]) : 0.0f, bias = dec ? dt_bias[min(c, nc - 1)] : 0.0f;
-  // the first four pieces of the lane's weight row are on their way while the rank rows are summed
+  auto piece = [&](float (&v)[8], int r) {  // eight of the lane's weight row from r on (past the rank its last ones, not used)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = ldf(w + min(r + e, rank - 1));
+  };
+  // the first four pieces are on their way while the rank rows are summed
   float wv[4][8];
   if (whole) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) ld8(w + min(8 * g + 32 * k, rank - 8), wv[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (32 * k < rank) piece(wv[k], 8 * g + 32 * k);
   }
   // the rank rows (zeros up to whole 32s): four elements a thread and eight slabs in flight at a time, without branches around the loads
   const int rows = nt <= 8 ? 8 : GTOK, row = gate_row(rank);
@@ -397,43 +406,33 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
     if (dec) decay[(int64_t)(t0 + i) * HD + c] = expf(-rate * softplusf_(z + bias));
     else gate[(int64_t)(t0 + i) * ng + c] = z;
   };
-  if (whole) {
-    // k runs as the lanes' pieces lie: step e of a block of 32 multiplies k = 8 g + e of lane group g
-    f32x4 z[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    const float* yr = ys + (lane & (rows - 1)) * ld + 8 * g;  // (MFMA rows past the tokens repeat them)
+  // k runs as the lanes' pieces lie: step e of a block of 32 multiplies k = 8 g + e of lane group g
+  f32x4 z[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  const float* yr = ys + (lane & (rows - 1)) * ld + 8 * g;  // (MFMA rows past the tokens repeat them)
+  auto products = [&](auto eights) {
+    constexpr bool W8 = decltype(eights)::value;
     auto add = [&](const float* v, int r) {  // r: the block's first k
       const f32x4 a = *reinterpret_cast<const f32x4*>(yr + r), b = *reinterpret_cast<const f32x4*>(yr + r + 4);
       const bool in = r + 8 * g < rank;
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        z[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(e < 4 ? a[e & 3] : b[e & 3], in ? v[e] : 0.0f, z[e & 1], 0, 0, 0);
+        z[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(e < 4 ? a[e & 3] : b[e & 3], (W8 ? in : r + 8 * g + e < rank) ? v[e] : 0.0f, z[e & 1], 0, 0, 0);
     };
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       if (32 * k < rank) add(wv[k], 32 * k);
     for (int r = 128; r < rank; r += 32) {
       float v[8];
-      ld8(w + min(r + 8 * g, rank - 8), v);
+      if constexpr (W8) ld8(w + min(r + 8 * g, rank - 8), v);
+      else piece(v, r + 8 * g);
       add(v, r);
     }
-    const f32x4 t = z[0] + z[1];  // lane (g, channel): tokens 4 g + r
+  };
+  if (whole) products(std::true_type());
+  else products(std::false_type());
+  const f32x4 t = z[0] + z[1];  // lane (g, channel): tokens 4 g + r
 #pragma unroll
-    for (int r = 0; r < 4; ++r) put(4 * g + r, t[r]);
-    return;
-  }
-  float z[GTOK];
-#pragma unroll
-  for (int i = 0; i < GTOK; ++i) z[i] = 0.0f;
-  for (int r = part; r < rank; r += 4) {
-    const float v = ldf(w + r);
-#pragma unroll
-    for (int i = 0; i < GTOK; ++i) z[i] += v * ys[(i & (rows - 1)) * ld + r];
-  }
-#pragma unroll
-  for (int i = 0; i < GTOK; ++i) {
-    z[i] = quad_sum(z[i]);
-    if ((i & 3) == part) put(i, z[i]);  // (the four lanes of a channel share the writes)
-  }
+  for (int r = 0; r < 4; ++r) put(4 * g + r, t[r]);
 }
 
 template <typename WT>
