@@ -6,14 +6,15 @@ from xotorch_support_jetson_amd.ops import kernels as K
 from xotorch_support_jetson_amd.ops import reference as R
 
 
-@pytest.mark.parametrize("max_tokens,H,max_ctx", [(1, 16, 17 * 64), (1, 16, 4096), (37, 16, 2048), (512, 16, 4096), (8, 128, 8192), (3, 200, 1100)])
+@pytest.mark.parametrize("max_tokens,H,max_ctx", [(1, 16, 17 * 64), (1, 16, 4096), (37, 16, 2048), (512, 16, 4096), (8, 128, 8192), (3, 200, 1100), (1, 128, 8192),
+                                                  (1, 16, 64000)])
 def test_workspace_holds_every_table(max_tokens, H, max_ctx):
   ws = K.MLAWorkspace(max_tokens, H, 256, max_ctx, torch.device("cpu"))
-  for width in range(1, ws.pages + 1):
-    for T in {1, 2, 3, 7, 8, 9, max_tokens}:
+  for width in [*range(1, ws.pages + 1), 2 * ws.pages, 100 * ws.pages]:
+    for T in {1, 2, 3, 7, 8, 9, 100, 129, 255, 256, 300, max_tokens}:
       ppp, nparts, _ = ws.partition(T, width)
       assert ppp * nparts >= width > ppp * (nparts - 1)
-      assert T > max_tokens or T * nparts <= max_tokens * ws.max_parts
+      assert nparts == 1 or ws.o.numel() >= T * nparts * H * 256 and ws.ml.numel() >= T * nparts * H * 2
 
 
 # (contexts, new tokens, pages a part)

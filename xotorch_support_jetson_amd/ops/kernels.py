@@ -427,15 +427,16 @@ def mla_prep(ckv, kv_ln, q, qpe_off: int, H: int, pos, cos_sin, slots, cache, ep
 
 
 class MLAWorkspace:
-  """Split-KV scratch of the MLA attention kernel."""
+  """Split-KV scratch of the MLA attention kernel: ROWS rows of partials a head, which hold the partitions of every step, whatever its
+  tokens and its tables' width (128 heads, 512 tokens of up to 32768: 0.13 GB; a bound on the tokens times one on the partitions 6.3)."""
+
+  ROWS = 512  # partition(): tokens x partitions is at most 384 over the blocks of 16 heads, with many heads below 256 + 255
 
   def __init__(self, max_tokens: int, H: int, DL: int, max_ctx: int, device):
     self.max_tokens, self.H, self.DL = max_tokens, H, DL
     self.pages = max(1, -(-max_ctx // PAGE))
-    self.max_parts = max(self.partition(T, w)[1] for T in (1, 8) for w in (self.pages, min(self.pages, 16)))
-    units = max(max_tokens * self.max_parts, 1)
-    self.o = torch.empty(units * H * DL, dtype=torch.float32, device=device)
-    self.ml = torch.empty(units * H * 2, dtype=torch.float32, device=device)
+    self.o = torch.empty(self.ROWS * H * DL, dtype=torch.float32, device=device)
+    self.ml = torch.empty(self.ROWS * H * 2, dtype=torch.float32, device=device)
 
   def wide(self, T: int) -> bool:
     """Many-head kernel (one workgroup covers up to 128 heads, each page loaded once for all of them) for
@@ -479,8 +480,6 @@ def mla_attn(q_lat, q_pe, cache, block_tables, cu_q, ctx_lens, scale: float, ws:
   if ws is None:
     ws = MLAWorkspace(T, H, DL, width * PAGE, q_lat.device)
   ppp, nparts, wide = ws.partition(T, width)
-  if T * nparts > ws.max_tokens * ws.max_parts:
-    ppp, nparts = width, 1
   out = torch.empty_like(q_lat) if out is None else out
   require().mla_attn(q_lat, q_pe, cache, block_tables, cu_q, ctx_lens, out, ws.o, ws.ml, int(ppp), int(nparts),
                      float(scale), int(wide))
