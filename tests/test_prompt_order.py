@@ -78,6 +78,22 @@ def test_scan_alone(B):
 
 
 @pytest.mark.gpu
+def test_scan_of_many_workgroups():
+  """More workgroups than one launch dimension holds work items for, all but two sequences' without tokens: the last one runs too."""
+  B, H, d, dv, n = 32769, 16, 64, 1024, 97  # x 32 column blocks: 2^24 + 512
+  g = torch.Generator(device="cuda").manual_seed(3)
+  rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+  q, k, v = rn(2 * n, H * d) / 8, rn(2 * n, H * d) / 8, rn(2 * n, H * dv)
+  decay, beta, state = torch.sigmoid(rn(2 * n, H) + 3), torch.sigmoid(rn(2 * n, H)), rn(2, H, dv, d)
+  cu, slots = torch.full((B + 1,), n, dtype=torch.int32), torch.full((B,), -1, dtype=torch.int32)
+  cu[0], cu[-1], slots[0], slots[-1] = 0, 2 * n, 0, 1
+  S, out, one = state.clone(), torch.full((2 * n, H * dv), float("nan"), device="cuda"), torch.empty(2 * n, H * dv, device="cuda")
+  K.linear_recurrence(q, k, v, decay, beta, 0.5, S, slots.cuda(), cu.cuda(), out, False, n)
+  K.linear_recurrence(q, k, v, decay, beta, 0.5, state, torch.tensor([0, 1]).int().cuda(), torch.tensor([0, n, 2 * n]).int().cuda(), one, False, n)
+  assert torch.equal(out, one) and torch.equal(S, state)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G", [(16, 4), (6, 3)])
 @pytest.mark.parametrize("batch", BATCHES)
 def test_gated_alone(batch, H, G):

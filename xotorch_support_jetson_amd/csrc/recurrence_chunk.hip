@@ -230,15 +230,14 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
   __shared__ __attribute__((aligned(16))) float sp[2][CHAN ? D : 4];
   __shared__ f32x4 sx[4][DELTA ? 2 : 1][64];      // the waves' partial products, for the wave with the other key dims
   constexpr int TILES = D / 32;                   // 16-row state tiles of a wave: half of the key dims
-  const uint32_t cols = (uint32_t)(dv + 31) / 32, place = blockIdx.x / (uint32_t)H, turn = place / cols;
-  const int h = (int)(blockIdx.x - place * H);
-  const int b = nth_longest(B, scan_order((int)turn, B, H * (int)cols), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
+  const int h = blockIdx.x;
+  const int b = nth_longest(B, scan_order((int)blockIdx.z, B, H * (int)gridDim.y), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
   const int t0 = cu_q[b], n = cu_q[b + 1] - t0;
   if (slot < 0 || n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 1;
-  const int col = (int)(place - turn * cols) * 32 + (wave & 1) * 16 + i;
+  const int col = (int)blockIdx.y * 32 + (wave & 1) * 16 + i;
   const bool live = col < dv;
   const int hk = h / (H / G);
   const int d0 = half * (D / 2);                  // the wave's first key dim
@@ -472,7 +471,7 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
 template <int D, bool CHAN, bool DELTA>
 void go(const ChunkRecurrence& a) {
   const int slots = a.T / CT + a.B;
-  const dim3 pg((unsigned)slots, (unsigned)a.H), sg((unsigned)(a.B * a.H * ((a.dv + 31) / 32)));
+  const dim3 pg((unsigned)slots, (unsigned)a.H), sg((unsigned)a.H, (unsigned)((a.dv + 31) / 32), (unsigned)a.B);
   chunk_prep_k<D, CHAN, DELTA><<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale,
                                                         a.state_slots, a.cu_q, a.B, a.H, a.G, a.ws);
   chunk_scan_k<D, CHAN, DELTA><<<sg, 256, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, a.decay, DELTA ? nullptr : a.beta,
