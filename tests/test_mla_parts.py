@@ -17,6 +17,19 @@ def test_workspace_holds_every_table(max_tokens, H, max_ctx):
       assert nparts == 1 or ws.o.numel() >= T * nparts * H * 256 and ws.ml.numel() >= T * nparts * H * 2
 
 
+@pytest.mark.parametrize("H", [16, 32, 128])
+def test_contexts_alike_are_one_round(H):
+  """A part a CU, and one round of them where the CUs are enough; short tables and a prompt's rows that fill the chip stay whole."""
+  ws = K.MLAWorkspace(64, H, 256, 4096, torch.device("cpu"))
+  for T in range(1, 400):
+    units = T * -(-H // 128) if ws.wide(T) else T * H // 16
+    for width in (1, 2, 3, 4, 8, 16, 17, 40, 64):
+      nparts = ws.partition(T, width)[1]
+      assert nparts == 1 or units * nparts < 256 + units
+      assert nparts == 1 or units <= 128 or width > 16 and T <= 64
+      assert nparts == 1 or width > 3 or ws.wide(T)
+
+
 # (contexts, new tokens, pages a part)
 STEPS = {"ragged": ([1, 64, 65, 300, 0, 129, 700, 2], None, 1), "70 parts": ([70 * 64, 100, 65 * 64], None, 1), "37": ([20 + 41 * i % 500 for i in range(37)], None, 2),
          "prompts": ([130, 5, 200], [130, 1, 77], 2), "whole": ([130, 90], [130, 20], 8)}

@@ -430,7 +430,7 @@ class MLAWorkspace:
   """Split-KV scratch of the MLA attention kernel: ROWS rows of partials a head, which hold the partitions of every step, whatever its
   tokens and its tables' width (128 heads, 512 tokens of up to 32768: 0.13 GB; a bound on the tokens times one on the partitions 6.3)."""
 
-  ROWS = 512  # partition(): tokens x partitions is at most 384 over the blocks of 16 heads, with many heads below 256 + 255
+  ROWS = 512  # partition(): tokens x partitions of more than one is below 256 + 255
 
   def __init__(self, max_tokens: int, H: int, DL: int, max_ctx: int, device):
     self.max_tokens, self.H, self.DL = max_tokens, H, DL
@@ -448,19 +448,18 @@ class MLAWorkspace:
     return self.H >= 64 and T >= 8
 
   def partition(self, T: int, width_pages: int):
-    """(pages per partition, partitions, wide).  A CU holds one workgroup (two 73 KB pages in LDS).  Many heads: enough
-    workgroups for 256 CUs.  Narrow kernel: one and a half a CU at most, since the partitions past a sequence's end cost
-    next to nothing, of at least two pages; of one for a handful of workgroups on a short table.  us in partitions of 1 / 2 /
-    3 / 4 pages, 16 heads, attention and merge: one of 900 tokens 9.9 / 11.3 / 13.1 / 14.8, one of 2000 13.5 / 13.1 / 14.5 /
-    15.4; 16 of 65 .. 830 12.5 / 12.4 / 14.1 / 15.1; 37 18.5 / 14.1 / 15.1 / 16.2; 64 25.2 / 23.2 / 16.8 / 17.7; 200 of
-    up to 400 41 / 29 / 30 / 28, whole 20.7."""
+    """(pages per partition, partitions, wide).  A CU holds one workgroup (two 73 KB pages in LDS): enough for 256 CUs, and not many
+    more, since contexts alike fill them all (16 heads, 64 of 900 in tables of 16 pages, us in 4 / 6 parts 25.4 / 31.4, of 65 .. 830
+    17.7 / 16.8; 37 of 900 in 6 / 8 22.7 / 25.9, of 62 .. 867 15.4 / 14.5).  Narrow kernel: parts of at least two pages; of one for a
+    handful of workgroups on a short table (us in parts of 1 / 2 / 3 / 4 pages, attention and merge: one of 900 9.9 / 11.3 / 13.1 /
+    14.8, one of 2000 13.5 / 13.1 / 14.5 / 15.4), but for tables of three and fewer (64 of 100 13.3 in two parts, 10.3 whole).
+    More than 128 workgroups on a short table, and those of a prompt's rows (their contexts are alike), stay whole: 16 heads, 200 of up
+    to 400 28 in parts of 4 pages, 20.7; 128 heads, 200 new tokens 88 in two parts, 38, behind 2000 243, 199."""
     nhb = -(-self.H // 16)
     wide = self.wide(T)
     units = max(1, T * -(-nhb // 8) if wide else T * nhb)
-    if wide:
-      want, cap = -(-256 // units), width_pages
-    else:
-      want, cap = 384 // units, width_pages if width_pages <= 16 and units * width_pages <= 128 else max(1, width_pages // 2)
+    want = 1 if units > 128 and (width_pages <= 16 or T > self.max_tokens) else -(-256 // units)
+    cap = width_pages if wide or 3 < width_pages <= 16 and units * width_pages <= 128 else width_pages // 2 if width_pages > 3 else 1
     nparts = max(1, min(want, cap))
     ppp = -(-width_pages // nparts)
     return ppp, -(-width_pages // ppp), wide
