@@ -1172,10 +1172,18 @@ void attn_gated_chunk(const at::Tensor& q, const at::Tensor& k_cache, const at::
 #undef ATT_CASE
     return;
   }
-  if (bf && max_qlen == 1 && T == B && d % 32 == 0 && d <= 128 && H / G <= 16 && ldo % 4 == 0 &&
+  // Single tokens: the step kernel, whose work is a page's and not a head's.  With few pairs, a long chunk and less than 8 heads a kv
+  // head the vector kernel's key splits keep more CUs busy, us step kernel / splits: one sequence at the end of a chunk of 1024, 16 heads
+  // of 128 on 16 20.5 / 14.3, on 8 20.3 / 14.9, on 4 20.2 / 19.9 (of 4096 60.4 / 50.7), on 2 of 8192 115 / 141; 12 sequences of up to 4000,
+  // 16 on 16, chunks of 4096 62.5 / 53.4.  Many pairs with chunks of parts of pages: 300 sequences of 130, chunks of 100, 16 on 4 19.7 / 16.9.
+  const int64_t pairs = B * G, pages = std::min((chunk + 63) / 64, block_tables.size(1));
+  const bool splits = H / G < 8 && (pairs < 256 ? pages * d > (pairs < 128 ? 512 : 2048) * (H / G) : pairs >= 1024 && chunk < 128);
+  if (bf && max_qlen == 1 && T == B && d % 32 == 0 && d <= 128 && H / G <= 16 && ldo % 4 == 0 && !splits &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0 &&
       ((reinterpret_cast<uintptr_t>(q.data_ptr()) | reinterpret_cast<uintptr_t>(k_cache.data_ptr()) | reinterpret_cast<uintptr_t>(v_cache.data_ptr())) & 15) == 0) {
-    // eight waves where the (sequence, kv head) pairs leave CUs idle: half as many rounds of a long chunk
+    // eight waves where the (sequence, kv head) pairs leave CUs idle: half as many rounds of a long chunk; two where the pairs fill
+    // them several times over: a short context has no page for the others, which only keep the next workgroup waiting (300 sequences of
+    // 20, 16 heads of 128 on 16 44.3 us with four waves, 30.1 with two, on 4 17.5 and 13.8)
     const dim3 grid((unsigned)B, (unsigned)G);
     const int hpg = (int)(H / G);
 #define ATS_GO(N, W)                                                                                                                  \
@@ -1186,9 +1194,10 @@ void attn_gated_chunk(const at::Tensor& q, const at::Tensor& k_cache, const at::
 #define ATS_CASE(N)                       \
   case N:                                 \
     if (wide) ATS_GO(N, 8);               \
-    else ATS_GO(N, 4);                    \
+    else if (pairs < 1024) ATS_GO(N, 4);  \
+    else ATS_GO(N, 2);                    \
     break;
-    const bool wide = B * G < 256 && hpg <= 8;  // (LDS: at most 34 KB)
+    const bool wide = pairs < 256 && hpg <= 8;  // (LDS: at most 34 KB)
     switch (d / 32) { ATS_CASE(1) ATS_CASE(2) ATS_CASE(3) ATS_CASE(4) }
 #undef ATS_CASE
 #undef ATS_GO
