@@ -118,6 +118,15 @@ def test_lone_sequence_needs_no_plan(H, Hkv, Dh):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,Hkv,whole", [([600] * 40, 8, True), ([300] * 150, 2, True), ([1000] * 100, 16, True), ([1600] + [100] * 23, 8, False), ([3000] * 4, 8, False)])
+def test_contexts_that_fill_the_chip_stay_whole(lens, Hkv, whole):
+  """A merge costs about four pages, which a cut has to bring in."""
+  cl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+  parts = K.require().decode_plan(cl, len(lens), Hkv, 64)[:, 3].max().item()
+  assert (parts == 1) == whole
+
+
+@pytest.mark.gpu
 def test_steps_too_large_to_count_are_refused():
   """Pages over all KV heads are counted in 32 bits, and a plan belongs to the batch and the tables it was made for."""
   C = K.require()
