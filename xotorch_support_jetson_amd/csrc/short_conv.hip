@@ -321,10 +321,11 @@ struct GateArgs {
   const void* g2;
   int rg, ng;
   float* gate;
+  int tok;  // tokens of a workgroup: GTOK, or 8
 };
 
 template <typename WT>
-__device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, float* ys) {  // ys: LDS [GTOK][gate_ld(rank)]
+__device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, float* ys) {  // ys: LDS [tok][gate_ld(rank)]
   const float* __restrict__ P = A.P;
   const WT* __restrict__ a2 = (const WT*)A.a2;
   const WT* __restrict__ g2 = (const WT*)A.g2;
@@ -336,7 +337,7 @@ __device__ __forceinline__ void gates_body(const GateArgs& A, int bx, int by, fl
   const int ldp = A.ldp, S = A.S, T = A.T, b_off = A.b_off, H = A.H, a1_off = A.a1_off, ra = A.ra, d = A.d, g1_off = A.g1_off,
             rg = A.rg, ng = A.ng;
   const int64_t ss = A.ss;
-  const int t0 = bx * GTOK, nt = min(GTOK, T - t0), HD = H * d, nab = (HD + 63) / 64;
+  const int t0 = bx * A.tok, nt = min(A.tok, T - t0), HD = H * d, nab = (HD + 63) / 64;
   int job = by;
   if (job == 0) {
     for (int e = threadIdx.x; e < nt * H; e += 256) {
@@ -617,10 +618,12 @@ GateArgs gate_args(const Slabs& p, int64_t b_off, at::Tensor& beta, int64_t a1_o
     a.g2 = g2->data_ptr();
     a.gate = gate->data_ptr<float>();
   }
+  // slabs of long rank rows are what a workgroup spends its time on
+  a.tok = a.S > 1 && std::max(a.ra, a.rg) > 512 ? 8 : GTOK;
   return a;
 }
 inline unsigned gate_jobs(const GateArgs& a) { return (unsigned)(1 + (a.H * a.d + 63) / 64 + (a.ng + 63) / 64); }
-inline size_t gate_lds(const GateArgs& a) { return (size_t)GTOK * gate_ld(std::max(a.ra, a.rg)) * sizeof(float); }
+inline size_t gate_lds(const GateArgs& a) { return (size_t)a.tok * gate_ld(std::max(a.ra, a.rg)) * sizeof(float); }
 
 StepArgs step_args(const Slabs& p, int64_t dt_off, const at::Tensor& dt_bias, const at::Tensor& A_log, at::Tensor& dt, at::Tensor& decay,
                    int64_t b_off = -1) {
@@ -708,7 +711,7 @@ void conv_prep_gates(const at::Tensor& P, int64_t x_off, const at::Tensor& conv_
   } else if (beta.has_value()) {
     at::Tensor bt = *beta;
     g = gate_args(p, b_off, bt, a1_off, a2, dt_bias, A_log, decay, g1_off, g2, gate, &bf);
-    gate_x = (a.T + GTOK - 1) / GTOK;
+    gate_x = (a.T + g.tok - 1) / g.tok;
     n_gate = gate_x * (int)gate_jobs(g);
     lds = gate_lds(g);
   } else {
@@ -759,7 +762,7 @@ void recurrence_gates(const at::Tensor& P, int64_t b_off, at::Tensor& beta, int6
   }
   bool bf = false;
   const GateArgs a = gate_args(p, b_off, beta, a1_off, a2, dt_bias, A_log, decay, g1_off, g2, gate, &bf);
-  const dim3 grid((unsigned)((T + GTOK - 1) / GTOK), gate_jobs(a));
+  const dim3 grid((unsigned)((T + a.tok - 1) / a.tok), gate_jobs(a));
   if (bf) recurrence_gates_k<uint16_t><<<grid, 256, gate_lds(a), stream()>>>(a);
   else recurrence_gates_k<float><<<grid, 256, gate_lds(a), stream()>>>(a);
 }
