@@ -618,7 +618,7 @@ GateArgs gate_args(const Slabs& p, int64_t b_off, at::Tensor& beta, int64_t a1_o
     a.g2 = g2->data_ptr();
     a.gate = gate->data_ptr<float>();
   }
-  // slabs of long rank rows are what a workgroup spends its time on
+  // slabs of long rank rows are what a workgroup spends its time on (rank 1024 in 8, 16 tokens 26.1 us with all 16, 20.2 with 8)
   a.tok = a.S > 1 && std::max(a.ra, a.rg) > 512 ? 8 : GTOK;
   return a;
 }

@@ -449,12 +449,12 @@ class MLAWorkspace:
 
   def partition(self, T: int, width_pages: int):
     """(pages per partition, partitions, wide).  A CU holds one workgroup (two 73 KB pages in LDS): enough for 256 CUs, and not many
-    more, since contexts alike fill them all (16 heads, 64 of 900 in tables of 16 pages, us in 4 / 6 parts 25.4 / 31.4, of 65 .. 830
-    17.7 / 16.8; 37 of 900 in 6 / 8 22.7 / 25.9, of 62 .. 867 15.4 / 14.5).  Narrow kernel: parts of at least two pages; of one for a
+    more, since contexts alike fill them all (16 heads, 64 of 900 in tables of 16 pages, us in 4 / 6 parts 24.2 / 31.4, of 65 .. 830
+    17.5 / 15.9; 37 of 900 in 6 / 8 20.5 / 25.9, of 62 .. 867 15.8 / 14.5).  Narrow kernel: parts of at least two pages; of one for a
     handful of workgroups on a short table (us in parts of 1 / 2 / 3 / 4 pages, attention and merge: one of 900 9.9 / 11.3 / 13.1 /
-    14.8, one of 2000 13.5 / 13.1 / 14.5 / 15.4), but for tables of three and fewer (64 of 100 13.3 in two parts, 10.3 whole).
+    14.8, one of 2000 13.5 / 13.1 / 14.5 / 15.4), but for tables of three and fewer (64 of 100 13.3 in two parts, 9.4 whole).
     More than 128 workgroups on a short table, and those of a prompt's rows (their contexts are alike), stay whole: 16 heads, 200 of up
-    to 400 28 in parts of 4 pages, 20.7; 128 heads, 200 new tokens 88 in two parts, 38, behind 2000 243, 199."""
+    to 400 28 in parts of 4 pages, 20.7; 128 heads, 200 new tokens 88 in two parts, 40, behind 2000 243, 199."""
     nhb = -(-self.H // 16)
     wide = self.wide(T)
     units = max(1, T * -(-nhb // 8) if wide else T * nhb)
