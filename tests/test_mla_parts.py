@@ -55,3 +55,27 @@ def test_parts(step, H, DL, wide, monkeypatch):
   # bf16 probabilities and results, 2^-9 each of a row's values
   assert (out - ref)[:, rows].abs().max() <= 2**-6 * ref[:, rows].abs().max()
   assert not out[:, [t for t in range(T) if t not in rows]].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [16, 40])
+@pytest.mark.parametrize("lens", ["alike", "ragged", "64", "edge"])
+def test_parts_by_the_contexts(H, lens):
+  """Parts of two lengths, of which the step's contexts take one: both against the reference, whatever the batch leaves of a wave."""
+  lens = {"alike": [900] * 37, "ragged": [62 + 22 * i for i in range(36)] + [0], "64": [(97 * i) % 1024 + 1 for i in range(64)],
+          "edge": [1024] * 32}[lens]
+  B, DL, width = len(lens), 256, 16
+  g = torch.Generator().manual_seed(B + H)
+  rn = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+  q_lat, q_pe, cache = rn(H, B, DL), rn(B, H * 64), rn(B * width, 64, DL + 64)
+  bt = torch.randperm(B * width, generator=g).int().view(B, width)
+  args = (q_lat, q_pe, cache, bt, torch.arange(B + 1).int(), torch.tensor(lens).int())
+  ws = K.MLAWorkspace(B, H, DL, width * 64, torch.device("cuda"))
+  ref = R.mla_attn(*args, 0.04).float()
+  ws.o.fill_(float("nan"))
+  ws.ml.fill_(float("nan"))
+  out = K.mla_attn(*(x.cuda() for x in args), 0.04, ws).float().cpu()
+  live = [b for b in range(B) if lens[b]]
+  # bf16 probabilities and results, 2^-9 each of a row's values
+  assert (out - ref)[:, live].abs().max() <= 2**-6 * ref[:, live].abs().max()
+  assert not out[:, [b for b in range(B) if not lens[b]]].any()

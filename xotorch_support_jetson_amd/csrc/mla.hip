@@ -264,13 +264,24 @@ __device__ __forceinline__ int seq_of_query(const int32_t* cu_q, int B, int T, i
   return lo;
 }
 
+// Pages of a part: `even` (0: none; more than ppp) where parts of ppp pages would be more than a workgroup for each of 256 CUs.  Single tokens
+// of at most 64 sequences, a lane each; nhb: workgroups of a part.  (The quotients are a reciprocal's: all workgroups, the merge's
+// among them, only have to agree.)
+__device__ __forceinline__ int pages_of_parts(const int32_t* ctx_lens, int B, int max_blocks, int nhb, int ppp, int even) {
+  if (even == 0) return ppp;
+  const int lane = threadIdx.x & 63;
+  const int n = lane < B ? min(max(ctx_lens[lane], 0), max_blocks * PAGE) : 0;
+  const uint32_t parts = wave_sum_u((uint32_t)((float)((n + PAGE - 1) / PAGE + ppp - 1) * __builtin_amdgcn_rcpf((float)ppp) + 0.01f));
+  return __builtin_amdgcn_readfirstlane((int)parts) * nhb > 256 ? even : ppp;
+}
+
 template <int DL>
 __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
     const uint16_t* __restrict__ q_lat, const uint16_t* __restrict__ q_pe, long ldqpe,
     const uint16_t* __restrict__ cache, const int32_t* __restrict__ block_tables, int max_blocks,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ ctx_lens, int B, int T, int H,
     uint16_t* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, int pages_per_part, int nparts,
-    float scale_log2, int num_pages) {
+    float scale_log2, int num_pages, int even) {
   constexpr int DR = 64;
   constexpr int ROW = DL + DR;                   // elements per cached token
   constexpr int KS = ROW / 32;                   // MFMA k-steps of S^T
@@ -284,6 +295,7 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
   uint16_t* pbuf = smem + 2 * PAGE * ROW;        // [16 heads][PLD] bf16
   float* red = reinterpret_cast<float*>(pbuf + 16 * PLD);  // [4 waves][16 heads]
 
+  const int ppp = pages_of_parts(ctx_lens, B, max_blocks, gridDim.y, pages_per_part, even);
   // Consecutive workgroups go to the 8 XCDs in turn.  The head blocks of one (token, partition) read the same latent pages:
   // they are 8 apart, on ONE XCD (one HBM read, the rest from that XCD's L2; spread over all 8 they read 8x the bytes from
   // HBM).  The tokens follow each other over the XCDs, the last first (in a prompt they have the most keys), and a token's
@@ -315,8 +327,8 @@ __global__ __launch_bounds__(256, 1) void mla_attn_kernel(
   const int b = seq_of_query(cu_q, B, T, t);
   const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
   const int npages = nkeys > 0 ? (nkeys + PAGE - 1) / PAGE : 0;
-  const int p_begin = part * pages_per_part;
-  const int p_end = min(npages, p_begin + pages_per_part);
+  const int p_begin = part * ppp;
+  const int p_end = min(npages, p_begin + ppp);
   const int np = max(0, p_end - p_begin);
   if (np == 0 && nparts > 1) return;  // (the merge reads the parts that have pages)
 
@@ -641,32 +653,40 @@ __global__ __launch_bounds__(512, 1) void mla_attn_wide_kernel(
 __global__ __launch_bounds__(256) void mla_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                           uint16_t* __restrict__ out, const int32_t* __restrict__ cu_q,
                                                           const int32_t* __restrict__ ctx_lens, int B, int T, int H, int DL,
-                                                          int max_blocks, int pages_per_part, int nparts) {
+                                                          int max_blocks, int pages_per_part, int nparts, int even) {
   const int th = blockIdx.x, t = th / H, h = th - t * H, lane = threadIdx.x & 63;
-  const int b = seq_of_query(cu_q, B, T, t);
-  const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
-  const int n = nkeys > 0 ? min(nparts, ((nkeys + PAGE - 1) / PAGE + pages_per_part - 1) / pages_per_part) : 0;
   const size_t base = (size_t)th * nparts;
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + base;
   const int d = 2 * threadIdx.x;
   const bool live = d < DL;
   const float* src = ws_o + base * DL + (live ? d : 0);
-  float M = NEG_BIG;
-  for (int p = lane; p < n; p += 64) M = fmaxf(M, ml[p].x);
+  auto row = [&](int p) { return *reinterpret_cast<const float2*>(src + (size_t)p * DL); };
+  // the first parts, on their way while they are counted (of a part without pages whatever lies there, not used)
+  const float2 x0 = ml[min(lane, nparts - 1)];
+  float2 v0[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v0[j] = row(min(j, nparts - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  const int ppp = pages_of_parts(ctx_lens, B, max_blocks, (H + 15) / 16, pages_per_part, even);
+  const int b = seq_of_query(cu_q, B, T, t);
+  const int nkeys = min(ctx_lens[b] - (cu_q[b + 1] - 1 - t), max_blocks * PAGE);
+  const int n = nkeys > 0 ? min(nparts, ((nkeys + PAGE - 1) / PAGE + ppp - 1) / ppp) : 0;
+  float M = lane < n ? x0.x : NEG_BIG;
+  for (int p = lane + 64; p < n; p += 64) M = fmaxf(M, ml[p].x);
   M = wave_max(M);
   float L = 0.f, a0 = 0.f, a1 = 0.f;
   for (int c0 = 0; c0 < n; c0 += 64) {
     const int m = min(64, n - c0);
     float w = 0.f;
     if (lane < m) {
-      const float2 x = ml[c0 + lane];
+      const float2 x = c0 == 0 ? x0 : ml[c0 + lane];
       w = __builtin_amdgcn_exp2f(x.x - M);
       L += w * x.y;
     }
     for (int p = 0; p < m; p += 4) {
       float2 v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float2*>(src + (size_t)(c0 + min(p + j, m - 1)) * DL);
+      for (int j = 0; j < 4; ++j) v[j] = c0 + p == 0 ? v0[j] : row(c0 + min(p + j, m - 1));
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (p + j < m) {
@@ -685,7 +705,7 @@ template <int DL>
 static void mla_launch(const uint16_t* q_lat, const uint16_t* q_pe, long ldqpe, const uint16_t* cache,
                        const int32_t* bt, int max_blocks, const int32_t* cu_q, const int32_t* ctx, int B, int T, int H,
                        uint16_t* out, float* ws_o, float* ws_ml, int ppp, int nparts, float scale, int num_pages,
-                       int wide, hipStream_t s) {
+                       int wide, int even, hipStream_t s) {
   constexpr int ROW = DL + 64;
   const int nhb = (H + 15) / 16;
   if (wide) {
@@ -708,24 +728,25 @@ static void mla_launch(const uint16_t* q_lat, const uint16_t* q_pe, long ldqpe, 
     (void)attr;
     const dim3 grid(nparts, nhb, T);
     kern<<<grid, 256, SMEM, s>>>(q_lat, q_pe, ldqpe, cache, bt, max_blocks, cu_q, ctx, B, T, H, out, ws_o, ws_ml, ppp,
-                                 nparts, scale * LOG2E, num_pages);
+                                 nparts, scale * LOG2E, num_pages, even);
   }
   static_assert(DL <= 512, "two dims a thread");
-  if (nparts > 1) mla_combine_kernel<<<T * H, 256, 0, s>>>(ws_o, ws_ml, out, cu_q, ctx, B, T, H, DL, max_blocks, ppp, nparts);
+  if (nparts > 1) mla_combine_kernel<<<T * H, 256, 0, s>>>(ws_o, ws_ml, out, cu_q, ctx, B, T, H, DL, max_blocks, ppp, nparts, even);
 }
 
 int launch_mla_attn(const uint16_t* q_lat, const uint16_t* q_pe, long ldqpe, const uint16_t* cache,
                     const int32_t* block_tables, int max_blocks, const int32_t* cu_q, const int32_t* ctx_lens, int B,
                     int T, int H, int DL, int DR, uint16_t* out, float* ws_o, float* ws_ml, int pages_per_part,
-                    int nparts, float scale, int num_pages, int wide, hipStream_t s) {
+                    int nparts, float scale, int num_pages, int wide, int even, hipStream_t s) {
   if (T <= 0) return 0;
   if (DR != 64 || B < 1 || pages_per_part < 1 || nparts < 1) return -1;
   if (nparts > 1 && (ws_o == nullptr || ws_ml == nullptr)) return -1;
+  if (even != 0 && (wide || T != B || B > 64 || even <= pages_per_part)) return -1;
   switch (DL) {
     case 512: mla_launch<512>(q_lat, q_pe, ldqpe, cache, block_tables, max_blocks, cu_q, ctx_lens, B, T, H, out, ws_o,
-                              ws_ml, pages_per_part, nparts, scale, num_pages, wide, s); return 0;
+                              ws_ml, pages_per_part, nparts, scale, num_pages, wide, even, s); return 0;
     case 256: mla_launch<256>(q_lat, q_pe, ldqpe, cache, block_tables, max_blocks, cu_q, ctx_lens, B, T, H, out, ws_o,
-                              ws_ml, pages_per_part, nparts, scale, num_pages, wide, s); return 0;
+                              ws_ml, pages_per_part, nparts, scale, num_pages, wide, even, s); return 0;
     default: return -1;
   }
 }

@@ -449,8 +449,8 @@ class MLAWorkspace:
 
   def partition(self, T: int, width_pages: int):
     """(pages per partition, partitions, wide).  A CU holds one workgroup (two 73 KB pages in LDS): enough for 256 CUs, and not many
-    more, since contexts alike fill them all (16 heads, 64 of 900 in tables of 16 pages, us in 4 / 6 parts 24.2 / 31.4, of 65 .. 830
-    17.5 / 15.9; 37 of 900 in 6 / 8 20.5 / 25.9, of 62 .. 867 15.8 / 14.5).  Narrow kernel: parts of at least two pages; of one for a
+    more, since contexts alike fill them all (16 heads, 64 of 900 in tables of 16 pages, us in 4 / 6 parts 24.2 / 31.4, 37 of 900 in 6 / 8
+    20.5 / 25.9; but ragged_pages).  Narrow kernel: parts of at least two pages; of one for a
     handful of workgroups on a short table (us in parts of 1 / 2 / 3 / 4 pages, attention and merge: one of 900 9.9 / 11.3 / 13.1 /
     14.8, one of 2000 13.5 / 13.1 / 14.5 / 15.4), but for tables of three and fewer (64 of 100 13.3 in two parts, 9.4 whole).
     More than 128 workgroups on a short table, and those of a prompt's rows (their contexts are alike), stay whole: 16 heads, 200 of up
@@ -463,6 +463,13 @@ class MLAWorkspace:
     nparts = max(1, min(want, cap))
     ppp = -(-width_pages // nparts)
     return ppp, -(-width_pages // ppp), wide
+
+  def ragged_pages(self, T: int, width_pages: int) -> int:
+    """Pages per partition of the narrow kernel for contexts that leave many partitions empty: one and a half workgroups a CU (16 heads,
+    37 sequences of 62 .. 867 tokens 15.8 us in partition()'s parts, 14.5 in these, 64 of 65 .. 830 17.5 and 15.9).  Which of the two a
+    step of single tokens takes is counted on the device: csrc/mla.hip pages_of_parts."""
+    units = T * -(-self.H // 16)
+    return -(-width_pages // max(1, min(384 // units, width_pages // 2)))
 
 
 def mla_attn(q_lat, q_pe, cache, block_tables, cu_q, ctx_lens, scale: float, ws: MLAWorkspace | None = None,
@@ -479,9 +486,14 @@ def mla_attn(q_lat, q_pe, cache, block_tables, cu_q, ctx_lens, scale: float, ws:
   if ws is None:
     ws = MLAWorkspace(T, H, DL, width * PAGE, q_lat.device)
   ppp, nparts, wide = ws.partition(T, width)
+  even = 0
+  if nparts > 1 and not wide and T == ctx_lens.shape[0] <= 64:
+    fine = ws.ragged_pages(T, width)
+    if fine < ppp:
+      even, ppp, nparts = ppp, fine, -(-width // fine)
   out = torch.empty_like(q_lat) if out is None else out
   require().mla_attn(q_lat, q_pe, cache, block_tables, cu_q, ctx_lens, out, ws.o, ws.ml, int(ppp), int(nparts),
-                     float(scale), int(wide))
+                     float(scale), int(wide), int(even))
   return out
 
 
