@@ -118,11 +118,12 @@ def test_lone_sequence_needs_no_plan(H, Hkv, Dh):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("lens,Hkv,whole", [([600] * 40, 8, True), ([300] * 150, 2, True), ([1000] * 100, 16, True), ([1600] + [100] * 23, 8, False), ([3000] * 4, 8, False)])
-def test_contexts_that_fill_the_chip_stay_whole(lens, Hkv, whole):
-  """A merge costs about four pages, which a cut has to bring in."""
+@pytest.mark.parametrize("lens,Hkv,Dh,whole", [([600] * 40, 8, 128, True), ([300] * 150, 2, 64, True), ([1000] * 100, 16, 128, True), ([1600] + [100] * 23, 8, 128, False),
+                                               ([3000] * 4, 8, 64, False), ([17 * (i + 1) for i in range(40)], 8, 64, True)])
+def test_contexts_that_fill_the_chip_stay_whole(lens, Hkv, Dh, whole):
+  """A merge costs about four pages, of heads of 64 seven, which a cut has to bring in."""
   cl = torch.tensor(lens, dtype=torch.int32, device="cuda")
-  parts = K.require().decode_plan(cl, len(lens), Hkv, 64)[:, 3].max().item()
+  parts = K.require().decode_plan(cl, len(lens), Hkv, 64, Dh)[:, 3].max().item()
   assert (parts == 1) == whole
 
 

@@ -613,12 +613,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_split_kernel(
 // The units of a decode step: every sequence's pages in equal parts of at most ppp pages; an empty sequence is one part (which writes
 // zeros).  ppp is the candidate with the least estimated time, in pages a CU reads one behind the other: its longest part, and an
 // average one beside it where there are more units than CUs (two workgroups a CU run at once), or, past two a CU, its share of all
-// pages and a part that starts last; and the merge of its parts, about four pages.  The weights are those with which 973 steps (16 to 1200
-// pairs, 7 head layouts, 300 to 8000 tokens alike, ragged or all but one short) come nearest to their best candidate: 1.2 % on average, 12 of
-// them more than 5 % behind the uncut contexts.  (With 0.4 a part as the merge's whole cost 2.3 % and 45: 40 sequences x 8 heads of 600
-// tokens 20.8 us uncut, 25.8 in the two parts it took.)  One workgroup, a wave per candidate.
+// pages and a part that starts last; and the merge of its parts, about four pages, or seven of heads of 64, which are read in half the
+// time.  The weights are those with which 973 steps (16 to 1200 pairs, 7 head layouts, 300 to 8000 tokens alike, ragged or all but one
+// short) come nearest to their best candidate: 1.0 % on average, 8 of them more than 5 % behind the uncut contexts.  (With 0.4 a part as the
+// merge's whole cost 2.3 % and 45: 40 sequences x 8 heads of 600 tokens 20.8 us uncut, 25.8 in the two parts it took.)
+// One workgroup, a wave per candidate.
 __global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restrict__ ctx_lens, int B, unsigned Hkv, int max_blocks,
-                                                          int places, DecodePart* __restrict__ plan) {
+                                                          float merge_pages, int places, DecodePart* __restrict__ plan) {
   __shared__ int red[8], ctx_sm[512], first_sm[513];
   __shared__ float est_sm[8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -653,7 +654,7 @@ __global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restr
     big = wave_max_u(big);
     const float u = (float)units * Hkv, work = (float)all, share = work / 256.f;
     const unsigned parts = (most + ppp - 1) / ppp;  // of the longest sequence, merged behind its last one
-    const float merge = parts > 1 ? 4.f + 0.3f * (float)parts : 0.f;
+    const float merge = parts > 1 ? merge_pages + 0.3f * (float)parts : 0.f;
     if (lane == 0)
       est_sm[wave] = (u <= 256.f ? big : u <= 512.f ? fmaxf(big + work / u, 1.3f * share) + 1.f : share + 0.8f * big + 1.f) + merge;
   }
@@ -697,9 +698,9 @@ __global__ __launch_bounds__(512) void decode_plan_kernel(const int32_t* __restr
   for (int i = base + tid; i < places; i += 512) plan[i] = {0, 0, 0, 0, 0, 0, 0, 0};
 }
 
-int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, DecodePart* plan, hipStream_t s) {
+int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int Dh, int max_blocks, DecodePart* plan, hipStream_t s) {
   if (B <= 0) return 0;
-  decode_plan_kernel<<<1, 512, 0, s>>>(ctx_lens, B, Hkv, max_blocks, decode_split_places(B, Hkv, max_blocks), plan);
+  decode_plan_kernel<<<1, 512, 0, s>>>(ctx_lens, B, Hkv, max_blocks, Dh <= 64 ? 7.f : 4.f, decode_split_places(B, Hkv, max_blocks), plan);
   return 0;
 }
 

@@ -878,13 +878,13 @@ static bool decode_sizes_ok(int64_t B, int64_t Hkv, int64_t max_blocks) {
 }
 
 // the plan of attn_decode_split: int32 [places, 8] (see kernels.h DecodePart), written by one launch
-at::Tensor decode_plan(const at::Tensor& ctx_lens, int64_t B, int64_t Hkv, int64_t max_blocks) {
+at::Tensor decode_plan(const at::Tensor& ctx_lens, int64_t B, int64_t Hkv, int64_t max_blocks, int64_t Dh) {
   CHECK_DT(ctx_lens, at::kInt);
   XCHECK(all_contig_gpu(ctx_lens) && B >= 1 && ctx_lens.numel() >= B, "decode_plan: ctx_lens");
   XCHECK(decode_sizes_ok(B, Hkv, max_blocks), "decode_plan: sizes");
   at::Tensor plan = at::empty({xot::decode_split_places((int)B, (int)Hkv, (int)max_blocks), 8}, ctx_lens.options());
   XCHECK(reinterpret_cast<uintptr_t>(plan.data_ptr()) % 32 == 0, "decode_plan: alignment");
-  xot::launch_decode_plan(ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hkv, (int)max_blocks,
+  xot::launch_decode_plan(ctx_lens.data_ptr<int32_t>(), (int)B, (int)Hkv, (int)Dh, (int)max_blocks,
                           reinterpret_cast<xot::DecodePart*>(plan.data_ptr<int32_t>()), cur_stream());
   return plan;
 }
@@ -1247,7 +1247,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_decode", &attn_decode, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("ctx_lens"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("pages_per_part"),
         py::arg("nparts"), py::arg("scale"), py::arg("algo") = 2);
-  m.def("decode_plan", &decode_plan, py::arg("ctx_lens"), py::arg("B"), py::arg("Hkv"), py::arg("max_blocks"));
+  m.def("decode_plan", &decode_plan, py::arg("ctx_lens"), py::arg("B"), py::arg("Hkv"), py::arg("max_blocks"),
+        py::arg("Dh") = 128);
   m.def("attn_decode_split", &attn_decode_split, py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
         py::arg("plan"), py::arg("ctx_lens"), py::arg("tickets"), py::arg("out"), py::arg("ws_o"), py::arg("ws_ml"), py::arg("scale"), py::arg("nt"),
         py::arg("defer") = false);

@@ -169,7 +169,7 @@ __device__ __forceinline__ int decode_lone_pages(int pages, int Hkv) {
   const int p = max(DECODE_MIN_PAGES, (int)(0.63f * sqrtf((float)pages) + 0.5f));
   return max(p, (pages * Hkv + DECODE_UNITS - 1) / DECODE_UNITS);
 }
-int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int max_blocks, DecodePart* plan, hipStream_t s);
+int launch_decode_plan(const int32_t* ctx_lens, int B, int Hkv, int Dh, int max_blocks, DecodePart* plan, hipStream_t s);
 // ws_o [places][H][Dh], ws_ml [places][H][2], tickets [B][Hkv] (zero before and after); plan none: one sequence of ctx_lens[0] tokens,
 // whose parts stay in ws_o / ws_ml with defer
 int launch_attn_decode_split(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* block_tables, int max_blocks,

@@ -284,7 +284,7 @@ class DecodeWorkspace:
       return LONE
     if not plan_pays(B, Hkv, width) or resolve_decode_algo(B, Hkv, self.algo) not in (2, 3):
       return None
-    return require().decode_plan(ctx_lens, B, Hkv, width)
+    return require().decode_plan(ctx_lens, B, Hkv, width, self.Dh)
 
 
 class PendingMerge:
