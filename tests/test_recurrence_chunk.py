@@ -79,6 +79,45 @@ def test_chunks_match_token_by_token(gpu, rule, d, dv, G, decays):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rule", list(RULES))
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("lens", [(100, 97, 96, 1, 112, 95, 81, 60), (97, 33, 16) * 6], ids=["halves", "many"])
+def test_forms_of_the_scan(gpu, rule, d, lens):
+  """Steps bound by all their chunks (csrc/recurrence_chunk.hip go()): waves of half of the key dims, with two chunks and, the delta rule's
+  of more than 512 workgroups, with one in flight; the other tests' steps are bound by their longest sequence."""
+  channel, delta, scaled, norm = RULES[rule]
+  H, dv, q_scale = 16, 64 - norm, 0.7
+  G = H if channel and not delta else 4
+  T, B, dvs = sum(lens), len(lens), dv + norm
+  assert T * H * 2 >= 180 * max(lens) and (B * H * 2 > 512) == (B > 16)
+  g = torch.Generator().manual_seed(d + B)
+  rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+  q, k, v, a = rn(T, G, d), rn(T, G, d), rn(T, H, dv), torch.sigmoid(3 + rn(T, H, d if channel else 1)) ** (1 / 16)
+  q, k = q / q.norm(dim=-1, keepdim=True), k / k.norm(dim=-1, keepdim=True)
+  beta = torch.sigmoid(rn(T, H)) if delta or scaled else None
+  state, cu = rn(B, H, dvs, d), torch.tensor((0, *lens)).cumsum(0).to(torch.int32)
+
+  def run(v):
+    S, out = state.to(gpu), torch.full((T, H * dvs), 7.0, device=gpu)
+    K.linear_recurrence(*(x.reshape(T, -1).to(gpu) for x in (q, k, v, a)), None if beta is None else beta.to(gpu), q_scale, S,
+                        torch.arange(B, dtype=torch.int32, device=gpu), cu.to(gpu), out, plain=scaled and not norm, max_qlen=max(lens))
+    return S.cpu(), out.cpu().view(T, H, dvs)
+  S, out = run(v)
+  for b in range(min(B, 7)):
+    t0, t1 = int(cu[b]), int(cu[b + 1])
+    want, last = token_by_token(q[t0:t1], k[t0:t1], v[t0:t1], a[t0:t1], None if beta is None else beta[t0:t1], q_scale,
+                                state[b].to(F64), rule, H)
+    for got, ref in ((out[t0:t1], want), (S[b], last)):  # (the bound of test_chunks_match_token_by_token)
+      assert ((got.to(F64) - ref).norm() / ref.norm()) < 1e-6, (b, lens[b])
+  v[44, 3, 5] = float("nan")  # (a token of the first sequence: what is not behind it, and other heads, as without it)
+  S2, out2 = run(v)
+  other = [h for h in range(H) if h != 3]
+  torch.testing.assert_close(out2[:44], out[:44], rtol=0, atol=float(2e-6 * out[:44].abs().max()))
+  assert out2[44, 3, 5].isnan() and torch.equal(out2[:, other], out[:, other]) and torch.equal(out2[lens[0]:], out[lens[0]:])
+  assert torch.equal(S2[1:], S[1:]) and torch.equal(S2[0, other], S[0, other])
+
+
+@pytest.mark.gpu
 def test_chunk_rule_keeps_what_it_cannot_take(gpu):
   """Rows off 16 bytes, key dims it has no tiles for and short steps run token by token, with the same results."""
   g = torch.Generator(device=gpu).manual_seed(3)

@@ -1338,17 +1338,17 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   auto on16 = [](const at::Tensor& t, int ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
   // Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
-  // its 1.4 us a chunk (2.2 with channel decays) beat 0.2 us a token, whatever the other sequences of the step do.  us before / after,
-  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 196, 8 of 961 .. 2431 1018 / 316, 30 single tokens and one
-  // prompt of 500 131 / 95, one of 33 11 / 15; channel decays 498 / 308, 1124 / 477, 229 / 132, 14 / 20.
+  // its 1.0 us a chunk beat 0.2 us a token, whatever the other sequences of the step do.  us token by token / in chunks,
+  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 130, 8 of 961 .. 2433 1018 / 298, 30 single tokens and one
+  // prompt of 500 131 / 58, one of 33 11 / 15; channel decays 498 / 138, 1124 / 400, 229 / 65, 14 / 20.
   // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
   const int64_t widest = std::max(std::max<int64_t>(ldq, ldk), std::max<int64_t>(std::max<int64_t>(ldv, H * dv), H * d));
   if ((d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && on16(q, ldq) &&
       on16(k, ldk) && on16(state, 0) && (!per_channel || on16(decay, 0))) {
-    auto ws = at::empty({chunk_recurrence_ws(T, B, H)}, q.options());
+    auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta)}, q.options());
     chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, ldk, ldv,
                       fixed ? 0 : (int)H, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(),
-                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, per_channel, delta, ws.data_ptr<float>(),
+                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? max_qlen : T / B), per_channel, delta, ws.data_ptr<float>(),
                       out.data_ptr<float>()});
     return;
   }

@@ -10,13 +10,13 @@ struct ChunkRecurrence {
   float q_scale;
   float* state;
   const int *state_slots, *cu_q;
-  int T, B, H, G, d, dv, dvin;
+  int T, B, H, G, d, dv, dvin, longest;  // longest: tokens of the longest sequence, or what is taken for it
   bool chan, delta;  // a decay per key channel; the delta rule
   float *ws, *out;
 };
 
 // takes d 64 or 128, rows of q, k, the decays (chan) and the state on 16-byte boundaries
 void chunk_recurrence(const ChunkRecurrence& a);
-int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H);  // floats
+int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta);  // floats
 
 }  // namespace xot

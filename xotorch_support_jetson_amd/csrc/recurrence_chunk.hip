@@ -7,18 +7,23 @@
 //   delta rule   U = M (V - (P K) S),  M = (I + tril(b_i G_ij k_i.k_j, -1))^-1 diag(b)      plain write   U = b V
 //   O = (P Q) S + N U,  N = tril(G_ij q_i.k_j)            S <- P_16 S + (G_16,j K)^T U
 //   * chunk_prep_k, a wave per (chunk, head), all of them in parallel: q.k and k.k products, the decays, the triangular
-//     inverse by forward substitution -> M, N (16 x 16) and the scalar decays into a workspace, 2.1 KB per chunk and head.
-//   * chunk_scan_k, the chain: a workgroup per (sequence, head, 32 value channels), a wave per 16 of them and half of the key
-//     dims: the partial products are exchanged through LDS, and from 512 workgroups on a SIMD has two waves, one's products
-//     under the other's waits (a wave with all key dims and 64 channels a workgroup: 294 us instead of 191 for one prompt of 2000,
-//     427 / 419 for eight then).  The state stays in MFMA accumulators: tile t, register r, lane group g holds key row
+//     inverse by forward substitution -> M, N (16 x 16) and the scalar decays into a workspace, 2.1 KB per chunk and head.  With channel
+//     decays the scan's operands P Q, P K and (G K)^T follow them, up to 24 KB: what it costs to write them (16 heads of 128 x 128,
+//     4593 tokens: 42 us without, 69 with) every workgroup of the scan was paying again, 16 products a thread and chunk on the chain.
+//   * chunk_scan_k, the chain: a workgroup per (sequence, head, 16 or 32 value channels), a wave per 16 of them and a quarter or half
+//     of the key dims.  The state stays in MFMA accumulators: tile t, register r, lane group g holds key row
 //     16 t + 4 g + r of value channel lane % 16, and as a B operand the same register is rows 4 g + r of the tile for g = 0 .. 3
 //     -- the A operands only have to name their k dims in that order, four consecutive floats a lane.  So the state never
-//     moves, U and M, N meet the same way, and a chunk is 3 D / 8 + 8 MFMAs a wave (plain write: D / 4 + 4); q, k and the decays
-//     pass LDS once per workgroup, two chunks ahead in registers.
-// Bound by that chain: about 1.4 us a chunk at D 128 where 56 MFMAs of 32 cycles are 0.75 (the rest: two barriers, LDS
-// reads and the four-step products with M and N between them).  Tarepel-design prompts (8 of 961 .. 2431 tokens, 16 heads
-// of 128 x 128): 1018 -> 316 us, delta rule with channel decays 1124 -> 477.
+//     moves, U and M, N meet the same way, and q and k come from memory as the operands they are, one to three chunks ahead in
+//     registers: nothing is staged for a workgroup, and a chunk has one barrier, behind which the partial products k S of the
+//     other key dims are read (those of q S a chunk later, they are not on the chain).
+// What bounds it: with few sequences the chain, k S -> exchange -> M -> write, 1.0 us a chunk at D 128 (1.5 with q, k and decays through
+// LDS, all waves' products of half of the key dims and two barriers; a wave issues one instruction at a time, and loads,
+// addresses and selections between the MFMAs were as many as them).  With many the matrix unit: 54 MFMAs of 32 cycles a wave of
+// half of the key dims, at 55 % of its rate.  One prompt of 2000 tokens, both kernels, us before and now: delta rule 16 heads of 128 x 128
+// 196 and 130, with channel decays 310 and 138, per-channel decays 16 heads of 64 x 128 157 and 79, plain write 32 heads of 128 x 64 160 and
+// 98; 5 of 364 .. 1728: 187, 294, 142, 152 and 152, 180, 84, 100; 8 of 961 .. 2433: 312, 490, 220, 254 and 298, 400, 205, 223; 32 of
+// 51 .. 1460: 302, 458, 203, 270 and 308, 411, 194, 230.
 // v_mfma_f32_16x16x4_f32 multiplies and accumulates in fp32 as the vector units do; no operand is rounded.
 //
 // Decays per key channel: where a prefix product P leaves 2^-100 .. 2^100 (a decay of 0, or a value that is no number, among
@@ -33,7 +38,9 @@ using namespace mix;
 constexpr int CT = 16;                          // tokens a chunk
 constexpr int MN = 2 * CT * CT + 2 * CT;        // workspace floats per (chunk, head): M, N, P_i, G_16,j
 constexpr float FAR = 1.2676506e30f;            // 2^100
-constexpr int RING = 2;                         // chunks in flight from memory (even: the LDS buffer alternates)
+// workspace floats of a (chunk, head): with channel decays the scan's operands follow, the decay over the chunk (D), then P Q, (G K)^T
+// and (delta rule) P K by state tile and lane
+constexpr int rec_floats(int D, bool chan, bool delta) { return MN + (chan ? D + (delta ? 3 : 2) * CT * D : 0); }
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -50,6 +57,15 @@ __device__ __forceinline__ float row_scan(float v) {
   return row_mul<0x118>(v);
 }
 
+// exclusive product of the lanes behind, in the same row
+__device__ __forceinline__ float row_after(float v) {
+  v = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(1.0f), __float_as_int(v), 0x101, 0xf, 0xf, false));  // row_shl 1
+  v = row_mul<0x101>(v);
+  v = row_mul<0x102>(v);
+  v = row_mul<0x104>(v);
+  return row_mul<0x108>(v);
+}
+
 // chunk slots of a step: sequence b's chunks start at cu[b] / 16 + b (at least ceil(n / 16) slots before the next one's)
 __device__ __forceinline__ int slot_base(const int* cu, int b) { return cu[b] / CT + b; }
 
@@ -58,9 +74,10 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
                                                    const float* __restrict__ decay, int dstride,
                                                    const float* __restrict__ beta, float q_scale,
                                                    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B,
-                                                   int H, int G, float* __restrict__ ws) {
+                                                   int H, int G, int heads, float* __restrict__ ws) {
   __shared__ float sA[CT][CT + 1];
-  const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, i = lane & 15, g = lane >> 4;
+  constexpr bool SHARE = !CHAN && !DELTA;
+  const int s = blockIdx.x, h = blockIdx.y * (SHARE ? heads : 1), lane = threadIdx.x, i = lane & 15, g = lane >> 4;
   int lo = 0, hi = B - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -79,7 +96,7 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
     kf[j] = *reinterpret_cast<const f32x4*>(k + t * ldk + hk * D + 16 * j + 4 * g);
     if (CHAN) af[CHAN ? j : 0] = *reinterpret_cast<const f32x4*>(decay + (t * H + h) * D + 16 * j + 4 * g);
   }
-  const float gi = CHAN || !valid ? 1.0f : decay[t * dstride + h];
+  float gi = CHAN || !valid ? 1.0f : decay[t * dstride + h];
   const float bi = DELTA && valid ? beta[t * H + h] : 0.0f;
   if (!valid) {
 #pragma unroll
@@ -88,7 +105,7 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
       if (CHAN) af[CHAN ? j : 0] = f32x4{1.f, 1.f, 1.f, 1.f};
     }
   }
-  float* M = ws + ((int64_t)s * H + h) * MN;
+  float* M = ws + ((int64_t)s * H + h) * rec_floats(D, CHAN, DELTA);
   // accumulators: row 4 g + r (token i), column lane % 16 (token j)
   f32x4 qs[8], ks[8];
 #pragma unroll
@@ -104,6 +121,17 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
         P[j][r] = row_scan(af[CHAN ? j : 0][r]);
         near = near && P[j][r] >= 1.0f / FAR && P[j][r] <= FAR;
       }
+    // the scan's operands: P Q and P K as they are here, (decays after a token) K with tokens and dims exchanged
+    float* op = M + MN;
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) {
+      if (i == CT - 1) *reinterpret_cast<f32x4*>(op + 16 * j + 4 * g) = P[j];
+      *reinterpret_cast<f32x4*>(op + D + j * 256 + lane * 4) = qf[j] * P[j] * q_scale;
+      if (DELTA) *reinterpret_cast<f32x4*>(op + D + 2 * CT * D + j * 256 + lane * 4) = kf[j] * P[j];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        op[D + CT * D + j * 256 + ((i >> 2) * 16 + 4 * g + r) * 4 + (i & 3)] = kf[j][r] * row_after(af[CHAN ? j : 0][r]);
+    }
     if (__all(near)) {
 #pragma unroll
       for (int j = 0; j < D / 16; ++j)
@@ -150,47 +178,57 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
         qs[r + 4 * (j & 1)] = mfma4(qf[j][r], kf[j][r], qs[r + 4 * (j & 1)]);
         if (DELTA) ks[r + 4 * (j & 1)] = mfma4(kf[j][r], kf[j][r], ks[r + 4 * (j & 1)]);
       }
-    // G_ij: the decays after j up to i, multiplied on token by token (no quotient)
-    float p = 1.0f, all = 1.0f, after = 1.0f;
-#pragma unroll
-    for (int row = 0; row < CT; ++row) {
-      const float d = __shfl(gi, row);
-      p = row > i ? p * d : 1.0f;
-      all *= d;
-      if (row > i) after *= d;
-      if ((row >> 2) == g) {
-        if ((row & 3) == 0) gam[0] = p; else if ((row & 3) == 1) gam[1] = p; else if ((row & 3) == 2) gam[2] = p; else gam[3] = p;
-      }
-      if (row == lane) M[2 * CT * CT + lane] = all;
-    }
-    if (lane < CT) M[2 * CT * CT + CT + lane] = after;
   }
   const f32x4 qk = ((qs[0] + qs[1]) + (qs[2] + qs[3])) + ((qs[4] + qs[5]) + (qs[6] + qs[7]));
   const f32x4 kk = ((ks[0] + ks[1]) + (ks[2] + ks[3])) + ((ks[4] + ks[5]) + (ks[6] + ks[7]));
+  for (int e = 0;; ++e) {
+    float gn = 1.0f;  // (the next head's, in flight under this one's)
+    if (SHARE && e + 1 < heads) gn = valid ? decay[t * dstride + h + e + 1] : 1.0f;
+    if (!CHAN) {
+      // G_ij: the decays after j up to i, multiplied on token by token (no quotient)
+      float p = 1.0f, all = 1.0f, after = 1.0f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = 4 * g + r;
-    const float br = __shfl(bi, row);
-    M[CT * CT + row * CT + i] = row >= i ? qk[r] * gam[r] * q_scale : 0.0f;
-    if (DELTA) sA[row][i] = row > i ? kk[r] * gam[r] * br : 0.0f;
-  }
-  if (!DELTA) return;
-  __syncthreads();
-  // column i of (I + A)^-1 by forward substitution, 16 lanes (the other groups repeat it)
-  float x[CT];
-#pragma unroll
-  for (int row = 0; row < CT; ++row) {
-    float a0 = row == i ? 1.0f : 0.0f, a1 = 0.0f;
-#pragma unroll
-    for (int m = 0; m < row; ++m) {
-      if (m & 1) a1 -= sA[row][m] * x[m];
-      else a0 -= sA[row][m] * x[m];
+      for (int row = 0; row < CT; ++row) {
+        const float d = __shfl(gi, row);
+        p = row > i ? p * d : 1.0f;
+        all *= d;
+        if (row > i) after *= d;
+        if ((row >> 2) == g) {
+          if ((row & 3) == 0) gam[0] = p; else if ((row & 3) == 1) gam[1] = p; else if ((row & 3) == 2) gam[2] = p; else gam[3] = p;
+        }
+        if (row == lane) M[2 * CT * CT + lane] = all;
+      }
+      if (lane < CT) M[2 * CT * CT + CT + lane] = after;
     }
-    x[row] = a0 + a1;
-  }
 #pragma unroll
-  for (int row = 0; row < CT; ++row)
-    if ((row >> 2) == g) M[row * CT + i] = row >= i ? x[row] * bi : 0.0f;  // (selected: bi may be no number)
+    for (int r = 0; r < 4; ++r) {
+      const int row = 4 * g + r;
+      const float br = __shfl(bi, row);
+      M[CT * CT + row * CT + i] = row >= i ? qk[r] * gam[r] * q_scale : 0.0f;
+      if (DELTA) sA[row][i] = row > i ? kk[r] * gam[r] * br : 0.0f;
+    }
+    if (DELTA) {
+      __syncthreads();
+      // column i of (I + A)^-1 by forward substitution, 16 lanes (the other groups repeat it)
+      float x[CT];
+#pragma unroll
+      for (int row = 0; row < CT; ++row) {
+        float a0 = row == i ? 1.0f : 0.0f, a1 = 0.0f;
+#pragma unroll
+        for (int m = 0; m < row; ++m) {
+          if (m & 1) a1 -= sA[row][m] * x[m];
+          else a0 -= sA[row][m] * x[m];
+        }
+        x[row] = a0 + a1;
+      }
+#pragma unroll
+      for (int row = 0; row < CT; ++row)
+        if ((row >> 2) == g) M[row * CT + i] = row >= i ? x[row] * bi : 0.0f;  // (selected: bi may be no number)
+    }
+    if (!SHARE || e + 1 >= heads) return;
+    M += rec_floats(D, CHAN, DELTA);
+    gi = gn;
+  }
 }
 
 // buffer over `bytes` from p on: loads past the end give 0, stores past it are dropped
@@ -216,135 +254,132 @@ __device__ __forceinline__ int scan_order(int turn, int B, int per) {
   return turn >= first ? B - 1 - (turn - first) : turn < second ? first - second + turn : turn - second;
 }
 
-template <int D, bool CHAN, bool DELTA>
-__global__ __launch_bounds__(256, 2) void chunk_scan_k(
+// CG groups of 16 value channels a workgroup, KP waves each: wave (kp, cg) has key dims kp D / KP .. of group cg.
+template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
+__global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
-    const float* __restrict__ decay, const float* __restrict__ inscale, float q_scale, float* __restrict__ state,
-    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin,
-    const float* __restrict__ ws, float* __restrict__ out) {
-  constexpr int LD = D + 4;                       // LDS row: consecutive tokens four banks apart
-  constexpr int NF = CT * D / 1024;               // float4s of k (and of q) a thread
-  constexpr int HALVES = 128 / D, TH = CT / HALVES;  // channel decays: threads per (channel, operand), tokens of each
-  constexpr bool KD = DELTA || !CHAN;             // k (channel decays: k P) rows, and the decayed k of the state update
-  __shared__ __attribute__((aligned(16))) float sq[2][CT][LD], sk[KD ? 2 : 1][KD ? CT : 1][LD], sb[CHAN ? 2 : 1][CHAN ? CT : 1][LD];
-  __shared__ __attribute__((aligned(16))) float sp[2][CHAN ? D : 4];
-  __shared__ f32x4 sx[4][DELTA ? 2 : 1][64];      // the waves' partial products, for the wave with the other key dims
-  constexpr int TILES = D / 32;                   // 16-row state tiles of a wave: half of the key dims
+    const float* __restrict__ inscale, float q_scale, float* __restrict__ state, const int* __restrict__ state_slots,
+    const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, const float* __restrict__ ws, float* __restrict__ out) {
+  constexpr int TILES = D / 16 / KP;              // 16-row state tiles of a wave
+  constexpr int REC = rec_floats(D, CHAN, DELTA);
+  // the write's operand, k with tokens and dims exchanged: from the workspace (channel decays), from the rows of k that the delta
+  // rule's product has through LDS, or element by element (16 heads of 128 x 128, 8 of 961 .. 2433 tokens: delta rule 312 us
+  // element by element and 298 through LDS; plain write 247 and 304, where those rows are no operand otherwise)
+  constexpr bool TURN = DELTA && !CHAN, SINGLE = !DELTA && !CHAN;
+  constexpr int LT = D / KP + 4;                  // LDS row of a wave's k: consecutive tokens four banks apart
+  __shared__ __attribute__((aligned(16))) float sk[TURN ? KP * CG : 1][TURN ? CT * LT : 1];
+  __shared__ f32x4 sx[DELTA && KP > 1 ? 2 : 1][CG][DELTA && KP > 1 ? KP : 1][64];  // partial products of the waves of a group
+  __shared__ f32x4 sy[KP > 1 ? 2 : 1][CG][KP > 1 ? KP : 1][64];
   const int h = blockIdx.x;
   const int b = nth_longest(B, scan_order((int)blockIdx.z, B, H * (int)gridDim.y), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
   const int t0 = cu_q[b], n = cu_q[b + 1] - t0;
   if (slot < 0 || n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave >> 1;
-  const int col = (int)blockIdx.y * 32 + (wave & 1) * 16 + i;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cg = wave % CG, kp = wave / CG;
+  const int col = ((int)blockIdx.y * CG + cg) * 16 + i;
   const bool live = col < dv;
   const int hk = h / (H / G);
-  const int d0 = half * (D / 2);                  // the wave's first key dim
+  const int d0 = kp * (D / KP);                   // the wave's first key dim
   float* St = state + (((int64_t)slot * H + h) * dv + (live ? col : 0)) * D + d0 + 4 * g;
   f32x4 S[TILES];
 #pragma unroll
   for (int j = 0; j < TILES; ++j) S[j] = *reinterpret_cast<const f32x4*>(St + 16 * j);
-  const float* W = ws + ((int64_t)slot_base(cu_q, b) * H + h) * MN;
-  const int64_t wstep = (int64_t)H * MN;
+  const float* W = ws + ((int64_t)slot_base(cu_q, b) * H + h) * REC;
+  const int64_t wstep = (int64_t)H * REC;
 
-  // Every load of a chunk goes through a buffer that ends with the sequence: its base moves in scalar registers and a
-  // lane's offset never changes, so a chunk's loads cost the vector unit nothing (64-bit addresses and clamped rows were
-  // 2700 of 6500 cycles a chunk, 4600 with channel decays).  RING chunks ahead, in registers: the thread's share of q, k and
-  // the decays; the wave's value rows; M, N, decays.  Nothing is computed from what is loaded until it is used.
-  struct Share {
-    f32x4 q[CHAN ? 1 : NF], k[CHAN ? 1 : NF];
-    float a[CHAN ? CT : 1], x[CHAN ? TH : 1];
-  };
-  struct Wave {
+  // What a chunk is made of, two chunks ahead in registers: q, k (channel decays: P Q, P K from the workspace) as A operands of the
+  // products with the state, (channel decays) (G K)^T for the write, and value rows, M, N and decays.
+  // Every load goes through a buffer that ends with the sequence: its base moves in scalar registers and a lane's offset never
+  // changes, so a chunk's loads cost the vector unit nothing; rows past the end give zeros, which leave the state as it is.
+  struct Ops {
+    f32x4 q[TILES], k[DELTA ? TILES : 1], t[TURN ? 1 : TILES], d[CHAN ? TILES : 1];
     f32x4 v, m, nn, p, e;
     float all;
   };
   const int chunks = (n + CT - 1) / CT;
-  const int ch = tid % D, part = tid / D, first = CHAN ? (part % HALVES) * TH : 0;
-  const bool is_q = __builtin_amdgcn_readfirstlane(part >= HALVES);  // (whole waves)
-  const float *q0 = q + (int64_t)t0 * ldq + hk * D, *k0 = k + (int64_t)t0 * ldk + hk * D, *v0 = v + (int64_t)t0 * ldv + h * dvin;
-  const float *a0 = decay + ((int64_t)t0 * H + h) * D, *b0 = inscale + (int64_t)t0 * H + h;
-  const float* x0 = is_q ? q0 : k0;
-  const int ldx = is_q ? ldq : ldk;
+  // A lane's place in the rows moves on by a chunk with every load; the windows end with the sequence, its state records with its chunks
+  const __amdgpu_buffer_rsrc_t rq = window(q + (int64_t)t0 * ldq + hk * D, ((int64_t)(n - 1) * ldq + D) * 4),
+                               rk = window(k + (int64_t)t0 * ldk + hk * D, ((int64_t)(n - 1) * ldk + D) * 4),
+                               rv = window(v + (int64_t)t0 * ldv + h * dvin, ((int64_t)(n - 1) * ldv + dvin) * 4),
+                               rb = window(inscale + (int64_t)t0 * H + h, inscale ? ((int64_t)(n - 1) * H + 1) * 4 : 0),
+                               ro = window(out + ((int64_t)t0 * H + h) * dv, ((int64_t)(n - 1) * H * dv + dv) * 4);
   const int vcol = min(col, dvin - 1);
-  auto fetch = [&](int cc, Share& s) {  // (past the end: the last chunk again, not used)
-    const int c = min(cc, chunks - 1), left = n - c * CT;  // rows from here to the end
+  uint32_t oq = (i * ldq + d0 + 4 * g) * 4, ok = (i * ldk + d0 + 4 * g) * 4, ot[4], ov[4], ob[4], oo[4];
+  uint32_t om = (i * CT + 4 * g) * 4, od = (CHAN ? MN + d0 + 4 * g : 2 * CT * CT + 4 * g) * 4;
+  uint32_t oc = (MN + D + kp * TILES * 256 + lane * 4) * 4;  // channel decays: P Q; (G K)^T and P K follow
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    ot[r] = ((4 * g + r) * ldk + d0 + i) * 4;
+    ov[r] = ((4 * g + r) * ldv + vcol) * 4;
+    ob[r] = (4 * g + r) * H * 4;
+    // (KP > 1: a chunk's rows are stored in the next one's turn.  What is before the first chunk, channels past the end and the waves
+    // that do not have the sum: past every window)
+    oo[r] = live && kp == 0 ? (uint32_t)(((4 * g + r - (KP > 1 ? CT : 0)) * H * dv + col) * 4) : 0x80000000u;
+    asm volatile("" : "+v"(ot[r]), "+v"(ov[r]), "+v"(oo[r]));
+  }
+  asm volatile("" : "+v"(oq), "+v"(ok), "+v"(om), "+v"(od), "+v"(oc));  // (constants added to them are then the loads' own)
+  const uint32_t ostep = live && kp == 0 ? CT * H * dv * 4 : 0;  // (the places past every window stay there)
+  const float *Wq = W, *Wr = W;  // the records of the next loads
+  int cq = 0, cr = 0;            // their chunks
+  auto record = [&](const float* w, int c) { return window(w, c < chunks ? REC * 4 : 0); };
+  // load s of a chunk's operands of the products with the state, then a step to the next chunk
+  auto load_q = [&](__amdgpu_buffer_rsrc_t w, Ops& o, int j) {
+    if (j < TILES) o.q[j] = CHAN ? load4(w, oc + 1024 * j) : load4(rq, oq + 64 * j);
+  };
+  auto load_k = [&](__amdgpu_buffer_rsrc_t w, Ops& o, int j) {
+    if (DELTA && j < TILES) o.k[DELTA ? j : 0] = CHAN ? load4(w, oc + (8 * CT * D + 1024 * j)) : load4(rk, ok + 64 * j);
+  };
+  auto next_state = [&]() {
+    ++cq;
     if (CHAN) {
-      const __amdgpu_buffer_rsrc_t ra = window(a0 + (int64_t)c * CT * H * D, ((int64_t)(left - 1) * H + 1) * D * 4);
-      const __amdgpu_buffer_rsrc_t rx = window(x0 + (int64_t)c * CT * ldx, ((int64_t)(left - 1) * ldx + D) * 4);
-#pragma unroll
-      for (int j = 0; j < CT; ++j) s.a[CHAN ? j : 0] = load1(ra, (j * H * D + ch) * 4);
-#pragma unroll
-      for (int j = 0; j < TH; ++j) s.x[CHAN ? j : 0] = load1(rx, ((first + j) * ldx + ch) * 4);
+      Wq += wstep;
     } else {
-      const __amdgpu_buffer_rsrc_t rq = window(q0 + (int64_t)c * CT * ldq, ((int64_t)(left - 1) * ldq + D) * 4);
-      const __amdgpu_buffer_rsrc_t rk = window(k0 + (int64_t)c * CT * ldk, ((int64_t)(left - 1) * ldk + D) * 4);
-#pragma unroll
-      for (int j = 0; j < NF; ++j) {
-        const int e = tid + 256 * j, tt = e / (D / 4), f = e % (D / 4);
-        s.q[CHAN ? 0 : j] = load4(rq, (tt * ldq + 4 * f) * 4);
-        s.k[CHAN ? 0 : j] = load4(rk, (tt * ldk + 4 * f) * 4);
+      oq += CT * ldq * 4;
+      ok += CT * ldk * 4;
+    }
+  };
+  // the rest of a chunk, NR loads
+  constexpr int NF = CHAN ? 2 * TILES : SINGLE ? 3 + 4 * TILES : 3, NR = NF + 1 + 4 + (DELTA ? 1 : 4);
+  auto load_rest = [&](__amdgpu_buffer_rsrc_t w, Ops& o, int s) {
+    if (s < 4) {
+      o.v[s & 3] = load1(rv, ov[s & 3]);
+    } else if (s == 4) {
+      o.nn = load4(w, om + CT * CT * 4);
+    } else if (DELTA && s == 5) {
+      o.m = load4(w, om);
+    } else if (!DELTA && s < 9) {
+      o.m[(s - 5) & 3] = load1(rb, ob[(s - 5) & 3]);
+    } else if (s < NR) {
+      const int f = s - (NR - NF);
+      if constexpr (CHAN) {
+        if (f < TILES) o.d[CHAN ? f : 0] = load4(w, od + 64 * f);
+        else o.t[f % TILES] = load4(w, oc + (4 * CT * D + 1024 * (f % TILES)));
+      } else {
+        if (f == 0) o.all = load1(w, (2 * CT * CT + CT - 1) * 4);
+        else if (f == 1) o.p = load4(w, od);
+        else if (f == 2) o.e = load4(w, od + CT * 4);
+        else if constexpr (SINGLE) o.t[(f - 3) % TILES][(f - 3) / TILES] = load1(rk, ot[(f - 3) / TILES] + 64 * ((f - 3) % TILES));
       }
     }
   };
-  auto fetch_wave = [&](int cc, Wave& w) {
-    const int c = min(cc, chunks - 1), left = n - c * CT;
-    const __amdgpu_buffer_rsrc_t rm = window(W + c * wstep, MN * 4);
-    w.nn = load4(rm, (CT * CT + i * CT + 4 * g) * 4);
-    if (DELTA) w.m = load4(rm, (i * CT + 4 * g) * 4);
-    if (!CHAN) {
-      w.p = load4(rm, (2 * CT * CT + 4 * g) * 4);
-      w.e = load4(rm, (2 * CT * CT + CT + 4 * g) * 4);
-      w.all = load1(rm, (2 * CT * CT + CT - 1) * 4);
-    }
-    const __amdgpu_buffer_rsrc_t rv = window(v0 + (int64_t)c * CT * ldv, ((int64_t)(left - 1) * ldv + dvin) * 4);
+  auto next_rest = [&]() {
+    ++cr;
+    Wr += wstep;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) w.v[r] = load1(rv, ((4 * g + r) * ldv + vcol) * 4);
-    if (!DELTA && inscale) {
-      const __amdgpu_buffer_rsrc_t rb = window(b0 + (int64_t)c * CT * H, ((int64_t)(left - 1) * H + 1) * 4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) w.m[r] = load1(rb, (4 * g + r) * H * 4);
+    for (int r = 0; r < 4; ++r) {
+      ov[r] += CT * ldv * 4;
+      if (SINGLE) ot[r] += CT * ldk * 4;
+      if (!DELTA) ob[r] += CT * H * 4;
     }
   };
-  auto stage = [&](int c, int buf, const Share& s) {  // tokens past the end: k = q = 0 and a decay of 1 leave the state as it is
-    if (CHAN) {
-      float a[CT], pre[CT], suf[CT];
-      float x = 1.0f;
+  auto store = [&](f32x4 Y) {
 #pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        a[j] = c * CT + j < n ? s.a[CHAN ? j : 0] : 1.0f;
-        x *= a[j];
-        pre[j] = x;
-      }
-      if (part == 0) sp[buf][CHAN ? ch : 0] = x;
-      x = 1.0f;
-#pragma unroll
-      for (int j = CT - 1; j >= 0; --j) {
-        suf[j] = x;
-        x *= a[j];
-      }
-      // (compile-time register indices: each of the halves' tokens selected, not addressed)
-#pragma unroll
-      for (int j = 0; j < TH; ++j) {
-        const bool up = HALVES > 1 && first != 0;
-        const float p = up ? pre[j + CT - TH] : pre[j], e = up ? suf[j + CT - TH] : suf[j];
-        // (q and k threads write different rows by address, without a branch)
-        float* row = is_q ? &sq[buf][0][0] : &sb[CHAN ? buf : 0][0][0];
-        row[(first + j) * LD + ch] = s.x[CHAN ? j : 0] * (is_q ? p * q_scale : e);
-        if (KD && !is_q) sk[KD ? buf : 0][KD ? first + j : 0][ch] = s.x[CHAN ? j : 0] * p;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < NF; ++j) {
-        const int e = tid + 256 * j, tt = e / (D / 4), f = e % (D / 4);
-        *reinterpret_cast<f32x4*>(&sq[buf][tt][4 * f]) = s.q[CHAN ? 0 : j] * q_scale;
-        *reinterpret_cast<f32x4*>(&sk[KD ? buf : 0][KD ? tt : 0][4 * f]) = s.k[CHAN ? 0 : j];
-      }
+    for (int r = 0; r < 4; ++r) {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Y[r]), ro, oo[r], 0, 0);
+      oo[r] += ostep;
     }
   };
-  const int64_t ldo = (int64_t)H * dv;
-  float* o0 = out + (int64_t)t0 * ldo + h * dv;
   // barrier that leaves loads and stores to memory in flight (LDS writes done): the prefetch lives across it
   auto bar = [&]() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -355,133 +390,210 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_k(
   // above its diagonal would carry an infinity or a NaN of b back to earlier tokens: such a chunk sums what is below alone
   // (all lanes of the wave; no memory operation, so that the loads in flight are waited for as without it).
   auto lower = [&](f32x4 l, f32x4 b, f32x4 c) {
-    uint32_t top = 0;
+    float odd = 0.0f * b[0];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) top = max(top, __float_as_uint(b[r]) & 0x7fffffffu);
-    if (__builtin_expect(__any(top >= 0x7f800000u), 0)) {
+    for (int r = 1; r < 4; ++r) odd = __builtin_fmaf(0.0f, b[r], odd);
+    if (__builtin_expect(__any(odd != odd), 0)) {
+      int at = lane;
+      asm volatile("" : "+v"(at));  // (or its addresses are kept in registers through the whole scan)
+      const int ai = at & 15, ag = 4 * (at >> 4);
+      for (int mm = 0; mm < CT; mm += 4)
 #pragma unroll
-      for (int m = 0; m < CT; ++m) {
-        const float bm = __shfl(b[m & 3], (m >> 2) * 16 + i);
+        for (int m = 0; m < 4; ++m) {
+          const float bm = __shfl(b[m], mm * 4 + ai);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float lm = __shfl(l[m & 3], (m >> 2) * 16 + 4 * g + r);
-          c[r] = m <= 4 * g + r ? c[r] + lm * bm : c[r];
+          for (int r = 0; r < 4; ++r) {
+            const float lm = __shfl(l[m], mm * 4 + ag + r);
+            c[r] = mm + m <= ag + r ? c[r] + lm * bm : c[r];
+          }
         }
-      }
       return c;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) c = mfma4(l[r], b[r], c);
     return c;
   };
-  Share sh[RING];
-  Wave wv[RING];
+  Ops ops[RING];
 #pragma unroll
   for (int u = 0; u < RING; ++u) {
-    fetch(u, sh[u]);
-    fetch_wave(u, wv[u]);
-  }
-  stage(0, 0, sh[0]);
-  bar();
-  auto chunk = [&](int c, int buf, Share& mine, Share& ahead, Wave& cur) {
-    fetch(c + RING, mine);
-    // (four partial sums each: shorter chains, and sums of D / 4 terms instead of D)
-    f32x4 xs[4], ys[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) xs[r] = ys[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __amdgpu_buffer_rsrc_t wq = record(Wq, cq), wr = record(Wr, cr);
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
-      const f32x4 qa = *reinterpret_cast<const f32x4*>(&sq[buf][i][d0 + 16 * j + 4 * g]);
-      f32x4 ka;
-      if (DELTA) ka = *reinterpret_cast<const f32x4*>(&sk[KD ? buf : 0][KD ? i : 0][d0 + 16 * j + 4 * g]);
+      load_k(wq, ops[u], j);
+      load_q(wq, ops[u], j);
+    }
+    next_state();
+    if (u == RING - 1) break;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) load_rest(wr, ops[u], j);
+    next_rest();
+  }
+  f32x4 last = {0.f, 0.f, 0.f, 0.f};  // KP > 1: the chunk before, of which the other waves' parts are in LDS
+  auto parts = [&](int buf) {
+    f32x4 y = last;
+#pragma unroll
+    for (int w = 1; w < KP; ++w) y += sy[KP > 1 ? buf : 0][cg][KP > 1 ? w : 0][lane];
+    return y;
+  };
+  // Loads and stores between the MFMAs, which hold the matrix unit 32 cycles each: behind them they were on the chain
+  auto pin = [&]() { __builtin_amdgcn_sched_barrier(0x86); };  // (vector, scalar and LDS operations may pass)
+  auto chunk = [&](int c, int buf, Ops& o, Ops& before) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    // (partial sums: shorter chains, and sums of fewer terms)
+    f32x4 xs[2] = {zero, zero}, ys[2] = {zero, zero};
+    const __amdgpu_buffer_rsrc_t wq = record(Wq, cq), wr = record(Wr, cr);
+    int s = 0;
+    float* kt = &sk[TURN ? wave : 0][0];
+    if constexpr (TURN) {  // (the wave's own: no barrier)
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) *reinterpret_cast<f32x4*>(kt + i * LT + 16 * j + 4 * g) = o.k[DELTA ? j : 0];
+    }
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          xs[r & 1] = mfma4(o.k[DELTA ? j : 0][r], S[j][r], xs[r & 1]);
+          load_rest(wr, before, s++);
+          load_rest(wr, before, s++);
+          pin();
+        }
+    }
+    f32x4 X = xs[0] + xs[1];
+    if constexpr (KP > 1) {
+      if constexpr (DELTA) sx[DELTA ? buf : 0][cg][DELTA ? kp : 0][lane] = X;
+      bar();
+    }
+    f32x4 xo[KP > 1 ? KP - 1 : 1];
+    if constexpr (DELTA && KP > 1) {
+#pragma unroll
+      for (int w = 1; w < KP; ++w) xo[w - 1] = sx[DELTA ? buf : 0][cg][DELTA ? (kp + w) % KP : 0][lane];
+    }
+    f32x4 y = last;
+    if constexpr (KP > 1) y = parts(buf ^ 1);
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        if (DELTA) xs[r] = mfma4(ka[r], S[j][r], xs[r]);
-        ys[r] = mfma4(qa[r], S[j][r], ys[r]);
+        ys[r & 1] = mfma4(o.q[j][r], S[j][r], ys[r & 1]);
+        if (r == 0) load_k(wq, o, j);
+        if constexpr (DELTA) {
+          load_rest(wr, before, s++);
+        } else {
+          load_rest(wr, before, s++);
+          load_rest(wr, before, s++);
+        }
+        pin();
       }
-    }
+#pragma unroll
+    for (; s < NR; ++s) load_rest(wr, before, s);
+    next_rest();
+    if constexpr (KP > 1) store(y);
     // the decayed state meets the chunk's write after the products that read it
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
-      const f32x4 p = CHAN ? *reinterpret_cast<const f32x4*>(&sp[buf][CHAN ? d0 + 16 * j + 4 * g : 0]) : f32x4{cur.all, cur.all, cur.all, cur.all};
+      const f32x4 p = CHAN ? o.d[CHAN ? j : 0] : f32x4{o.all, o.all, o.all, o.all};
 #pragma unroll
       for (int r = 0; r < 4; ++r) S[j][r] *= p[r];
     }
-    f32x4 X = (xs[0] + xs[1]) + (xs[2] + xs[3]);
-    f32x4 Y = (ys[0] + ys[1]) + (ys[2] + ys[3]);
-    if (DELTA) sx[wave][DELTA ? 1 : 0][lane] = X;
-    if (half == 1) sx[wave][0][lane] = Y;
-    bar();
-    if (DELTA) X += sx[wave ^ 2][DELTA ? 1 : 0][lane];
-    Y += sx[wave | 2][0][lane];  // (used by the waves of the first half)
-    f32x4 U;  // the value rows (0 past the end); the normaliser's channel is fed with ones
+    f32x4 U;  // the value rows; the normaliser's channel is fed with ones (past the end k is 0: no such row reaches anything)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      U[r] = col < dvin ? cur.v[r] : col < dv && c * CT + 4 * g + r < n ? 1.0f : 0.0f;
-      if (!DELTA && inscale) U[r] *= cur.m[r];
+      U[r] = DELTA || col < dvin ? o.v[r] : 1.0f;
+      if (!DELTA) U[r] *= inscale ? o.m[r] : 1.0f;
     }
-    if (DELTA) {
+    if constexpr (DELTA) {
+      if constexpr (KP > 1) {
+#pragma unroll
+        for (int w = 1; w < KP; ++w) X += xo[w - 1];
+      }
       f32x4 R;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) R[r] = U[r] - (CHAN ? X[r] : cur.p[r] * X[r]);
-      U = lower(cur.m, R, f32x4{0.f, 0.f, 0.f, 0.f});
+      for (int r = 0; r < 4; ++r) R[r] = U[r] - (CHAN ? X[r] : o.p[r] * X[r]);
+      U = lower(o.m, R, zero);
     }
-    if (!CHAN) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Y[r] *= cur.p[r];
-    }
-    Y = lower(cur.nn, U, Y);
     f32x4 E = U;
     if (!CHAN) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) E[r] *= cur.e[r];
+      for (int r = 0; r < 4; ++r) E[r] *= o.e[r];
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int j = 0; j < TILES; ++j) {
-        const int e = d0 + 16 * j + i;
-        const float ka = CHAN ? sb[CHAN ? buf : 0][CHAN ? 4 * g + r : 0][e] : sk[KD ? buf : 0][KD ? 4 * g + r : 0][e];
-        S[j] = mfma4(ka, E[r], S[j]);
+        S[j] = mfma4(TURN ? kt[(4 * g + r) * LT + 16 * j + i] : o.t[TURN ? 0 : j][r], E[r], S[j]);
+        if (r == 0) load_q(wq, o, j);
+        pin();
       }
-    const __amdgpu_buffer_rsrc_t ro = window(o0 + (int64_t)c * CT * ldo, ((int64_t)(n - c * CT - 1) * ldo + dv) * 4);
+    next_state();
+    f32x4 Y = ys[0] + ys[1];
+    if (!CHAN) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)  // (channels past the end and the second half's waves: an offset no window reaches)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Y[r]), ro, live && half == 0 ? (int)(((4 * g + r) * ldo + col) * 4) : -16, 0, 0);
-    fetch_wave(c + RING, cur);
-    stage(c + 1, buf ^ 1, ahead);  // (its last readers passed the barrier that ended the previous chunk)
-    bar();
+      for (int r = 0; r < 4; ++r) Y[r] *= o.p[r] * q_scale;
+    }
+    if (KP == 1 || kp == 0) Y = lower(o.nn, U, Y);
+    if constexpr (KP > 1) {
+      sy[KP > 1 ? buf : 0][cg][KP > 1 ? kp : 0][lane] = Y;
+      last = Y;
+    } else {
+      store(Y);
+    }
   };
-  // whole rings without a branch between the chunks (at a join the compiler waits for every load that one of the paths may
-  // have issued last), then the rest
-  int c = 0;
-  for (; c + RING <= chunks; c += RING) {
+  // (ends left where the chunks end, none joined again: at a join the compiler waits for every load that one of the paths may have
+  // issued last, and a copy of the loop's body for the rest keeps a second set of operands in registers)
+  for (int c = 0;; c += RING) {
+    bool end = false;
 #pragma unroll
-    for (int u = 0; u < RING; ++u) chunk(c + u, u & 1, sh[u], sh[(u + 1) % RING], wv[u]);
+    for (int u = 0; u < RING; ++u) {
+      chunk(c + u, (c + u) & 1, ops[u], ops[(u + RING - 1) % RING]);
+      end = c + u + 1 >= chunks;
+      if (end) break;
+    }
+    if (end) break;
   }
-#pragma unroll
-  for (int u = 0; u < RING - 1; ++u)
-    if (c + u < chunks) chunk(c + u, u & 1, sh[u], sh[u + 1], wv[u]);
+  if constexpr (KP > 1) {
+    bar();
+    store(parts((chunks - 1) & 1));
+  }
   if (live) {
 #pragma unroll
     for (int j = 0; j < TILES; ++j) *reinterpret_cast<f32x4*>(St + 16 * j) = S[j];
   }
 }
 
+template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
+void scan(const ChunkRecurrence& a) {
+  const dim3 grid((unsigned)a.H, (unsigned)((a.dv + 16 * CG - 1) / (16 * CG)), (unsigned)a.B);
+  chunk_scan_k<D, CHAN, DELTA, KP, CG, WPE, RING><<<grid, 64 * KP * CG, 0, stream()>>>(
+      a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, DELTA ? nullptr : a.beta, a.q_scale, a.state, a.state_slots, a.cu_q, a.B, a.H, a.G, a.dv,
+      a.dvin, a.ws, a.out);
+}
+
 template <int D, bool CHAN, bool DELTA>
 void go(const ChunkRecurrence& a) {
   const int slots = a.T / CT + a.B;
-  const dim3 pg((unsigned)slots, (unsigned)a.H), sg((unsigned)a.H, (unsigned)((a.dv + 31) / 32), (unsigned)a.B);
+  // plain write, a decay per head: the heads of a q / k head share its products where that leaves enough waves (32 heads on 8, with the
+  // scan: 5 of 364 .. 1728 tokens 110 -> 100 us, 8 of 961 .. 2433 247 -> 223; three of 1000 not; two heads under the delta rule gave nothing)
+  const int heads = !CHAN && !DELTA && (int64_t)slots * a.G >= 2048 ? a.H / a.G : 1;
+  const dim3 pg((unsigned)slots, (unsigned)(a.H / heads));
   chunk_prep_k<D, CHAN, DELTA><<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale,
-                                                        a.state_slots, a.cu_q, a.B, a.H, a.G, a.ws);
-  chunk_scan_k<D, CHAN, DELTA><<<sg, 256, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, a.decay, DELTA ? nullptr : a.beta,
-                                                         a.q_scale, a.state, a.state_slots, a.cu_q, a.B, a.H, a.G, a.dv, a.dvin,
-                                                         a.ws, a.out);
+                                                        a.state_slots, a.cu_q, a.B, a.H, a.G, heads, a.ws);
+  // Steps whose longest sequence takes longer than the CUs' share of all chunks are bound by its chain: four waves of a quarter of the
+  // key dims each, 16 channels a workgroup, three chunks ahead.  Others by the matrix unit: two halves and 32 channels, which
+  // repeat the products with M and N less.  The line by T (tokens) x workgroups of 32 channels a sequence / (256 x the longest), us
+  // quarters / halves, delta rule 16 heads of 128 x 128: 0.25 (one of 2000) 130 / 167, 0.5 77 / 93, 0.66 (5 of 364 .. 1728) 149 / 164,
+  // 0.75 (three of 1000) 111 / 98, 1.3 (8 of 961 .. 2433) 332 / 298.
+  const int64_t per = (int64_t)a.H * ((a.dv + 31) / 32);
+  if (a.T * per < 180 * (int64_t)a.longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a);
+  else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a);
+  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a);  // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us)
 }
 
 }  // namespace
 
-int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H) { return (T / CT + B) * H * MN; }
+int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta) {
+  return (T / CT + B) * H * rec_floats((int)d, chan, delta);
+}
 
 void chunk_recurrence(const ChunkRecurrence& a) {
 #define XOT_CHUNK(D)                                              \
