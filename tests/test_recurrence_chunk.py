@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from xotorch_support_jetson_amd.ops import kernels as K
+from xotorch_support_jetson_amd.ops._ext import require
 
 F64 = torch.float64
 # rule -> (decay per key channel, delta rule, input scale, normaliser channel)
@@ -115,6 +116,55 @@ def test_forms_of_the_scan(gpu, rule, d, lens):
   torch.testing.assert_close(out2[:44], out[:44], rtol=0, atol=float(2e-6 * out[:44].abs().max()))
   assert out2[44, 3, 5].isnan() and torch.equal(out2[:, other], out[:, other]) and torch.equal(out2[lens[0]:], out[lens[0]:])
   assert torch.equal(S2[1:], S[1:]) and torch.equal(S2[0, other], S[0, other])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rank", [16, 48, 24])
+def test_decays_from_a_low_rank_product(gpu, d, rank):
+  """linear_recurrence_made without A_log: decays of gla_prep, made by the chunks; a rank of no whole 16 is left to the two launches."""
+  H, dv, tau, lens = 2, 33, 16.0, [101, 16, 1, 47]
+  T, B, off = sum(lens), len(lens), 8
+  g = torch.Generator().manual_seed(d + rank)
+  rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+  P, a2, a2_b = rn(T, off + rank + 4), rn(H * d, rank) / rank ** 0.5, rn(H * d) + 3
+  q, k, v, state = rn(T, H * d) / d ** 0.5, rn(T, H * d) / d ** 0.5, rn(T, H * dv), rn(B, H, dv, d)
+  cu, slots = torch.tensor([0] + lens).cumsum(0).to(torch.int32), torch.arange(B, dtype=torch.int32)
+  S, out = state.to(gpu), torch.full((T, H * dv), 7.0, device=gpu)
+  took = require().linear_recurrence_made(q.to(gpu), k.to(gpu), v.to(gpu), P.to(gpu), off, a2.to(gpu), a2_b.to(gpu), tau, None, 0.7, S,
+                                          slots.to(gpu), cu.to(gpu), out, max(lens))
+  assert took == (rank % 16 == 0)
+  if not took:
+    assert (out == 7.0).all() and torch.equal(S.cpu(), state)
+    return
+  a = torch.exp(torch.nn.functional.logsigmoid(P[:, off:off + rank].to(F64) @ a2.to(F64).T + a2_b.to(F64)) / tau).view(T, H, d)
+  S, out = S.cpu(), out.cpu().view(T, H, dv)
+  for b in range(B):
+    t0, t1 = int(cu[b]), int(cu[b + 1])
+    want, last = token_by_token(*(x[t0:t1].view(t1 - t0, H, -1) for x in (q, k, v)), a[t0:t1], None, 0.7, state[b].to(F64), "channel", H)
+    # fp32 sums of up to 48 products: some 3e-7 of |z| < 7, a sixteenth of it in a decay's logarithm, over the about 60 tokens that a decay
+    # of 0.98 remembers: below 1e-5, the rest as in test_chunks_match_token_by_token
+    for got, ref in ((out[t0:t1], want), (S[b], last)):
+      assert ((got.to(F64) - ref).norm() / ref.norm()) < 1e-5, (b, lens[b])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,G", [(64, 2), (128, 4)])
+def test_decays_and_write_strengths_from_finished_products(gpu, d, G):
+  """linear_recurrence_made with A_log: exactly what recurrence_gates' decays and write strengths give, which are the same arithmetic."""
+  H, dv, lens = 4, 40, [97, 33, 100, 1]
+  T, B = sum(lens), len(lens)
+  g = torch.Generator(device=gpu).manual_seed(d)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  P, za, dt_bias, A_log = rn(T, H + 3), rn(T, H * d + 8), rn(H * d), rn(H) * 0.4 - 1.2
+  q, k, v, state = rn(T, G * d) / d ** 0.5, rn(T, G * d) / d ** 0.5, rn(T, H * dv), rn(B, H, dv, d)
+  cu, slots = torch.tensor([0] + lens, device=gpu).cumsum(0).to(torch.int32), torch.arange(B, dtype=torch.int32, device=gpu)
+  beta, decay = torch.empty(T, H, device=gpu), torch.empty(T, H * d, device=gpu)
+  K.recurrence_gates(P, 2, beta, 0, None, dt_bias, A_log, decay, 0, None, None, za=za)
+  one, two = (state.clone(), torch.empty(T, H * dv, device=gpu)), (state.clone(), torch.empty(T, H * dv, device=gpu))
+  K.linear_recurrence(q, k, v, decay, beta, 0.7, one[0], slots, cu, one[1], max_qlen=100)
+  assert require().linear_recurrence_made(q, k, v, P, 2, za, dt_bias, 1.0, A_log, 0.7, two[0], slots, cu, two[1], 100)
+  assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
 
 
 @pytest.mark.gpu

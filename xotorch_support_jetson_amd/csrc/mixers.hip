@@ -1298,6 +1298,21 @@ void launch_rec(int KR, dim3 grid, const float* q, int ldq, const float* k, int 
 #undef REC_CASE
 }
 
+bool rows16(const at::Tensor& t, int64_t ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+// Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
+// its 1.0 us a chunk beat 0.2 us a token, whatever the other sequences of the step do.  us token by token / in chunks,
+// 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 130, 8 of 961 .. 2433 1018 / 298, 30 single tokens and one
+// prompt of 500 131 / 58, one of 33 11 / 15; channel decays 498 / 138, 1124 / 400, 229 / 65, 14 / 20.
+// (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
+bool chunks_take(const at::Tensor& q, int64_t ldq, const at::Tensor& k, int64_t ldk, int64_t ldv, const at::Tensor& state, int64_t T,
+                 int64_t B, int64_t H, int64_t max_qlen) {
+  const int64_t dv = state.size(2), d = state.size(3);
+  const int64_t widest = std::max(std::max(ldq, ldk), std::max(std::max(ldv, H * dv), H * d));
+  return (d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && rows16(q, ldq) &&
+         rows16(k, ldk) && rows16(state, 0);
+}
+
 // q / k [T, G d], v [T, H dv]: fp32 rows of unit inner stride (column slices allowed).  decay [T, H] (delta rule, or
 // without beta: one decay per head and a plain outer-product write; a 1-D [H]: the same decay at every token) or [T, H d]
 // (per key channel; with beta: the delta rule on such a decay); beta [T, H] (delta
@@ -1335,21 +1350,13 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool fixed = !beta.has_value() && decay.dim() == 1 && decay.numel() == H;
   const bool scalar = !beta.has_value() && (fixed || decay.numel() == T * H);
   const float* bp = beta.has_value() ? beta->data_ptr<float>() : nullptr;
-  auto on16 = [](const at::Tensor& t, int ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; };
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
-  // Prompts go 16 tokens at a time (recurrence_chunk.hip): from about 100 tokens of the longest sequence its two launches and
-  // its 1.0 us a chunk beat 0.2 us a token, whatever the other sequences of the step do.  us token by token / in chunks,
-  // 16 heads: delta rule 128 x 128, one prompt of 2000 415 / 130, 8 of 961 .. 2433 1018 / 298, 30 single tokens and one
-  // prompt of 500 131 / 58, one of 33 11 / 15; channel decays 498 / 138, 1124 / 400, 229 / 65, 14 / 20.
-  // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
-  const int64_t widest = std::max(std::max<int64_t>(ldq, ldk), std::max<int64_t>(std::max<int64_t>(ldv, H * dv), H * d));
-  if ((d == 64 || d == 128) && (max_qlen > 0 ? max_qlen : T / B) >= 96 && T * widest * 4 < (int64_t(1) << 31) && on16(q, ldq) &&
-      on16(k, ldk) && on16(state, 0) && (!per_channel || on16(decay, 0))) {
+  if (chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, max_qlen) && (!per_channel || rows16(decay, 0))) {
     auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta)}, q.options());
     chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, ldk, ldv,
                       fixed ? 0 : (int)H, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(),
-                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? max_qlen : T / B), per_channel, delta, ws.data_ptr<float>(),
-                      out.data_ptr<float>()});
+                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? max_qlen : T / B),
+                      per_channel, delta, ws.data_ptr<float>(), out.data_ptr<float>(), DecaySource{}});
     return;
   }
   int DP = 16;
@@ -1376,6 +1383,47 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   else if (scalar) REC_GO(16, 2, 1);
   else REC_GO(16, 0, 1);
 #undef REC_GO
+}
+
+// linear_recurrence of a prompt whose decays per key channel are made on the way (recurrence_chunk.h DecaySource): the plain write's from
+// P's columns p_off .. + rank and w [H d, rank], b [H d]; with A_log the delta rule's from finished products w [T, >= H d] and b
+// [H d], its write strengths from P's columns p_off .. + H.  False where the chunks do not take it (nothing is done then).
+bool linear_recurrence_made(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& P, int64_t p_off,
+                            const at::Tensor& w, const at::Tensor& b, double tau, const c10::optional<at::Tensor>& A_log,
+                            double q_scale, at::Tensor& state, const at::Tensor& state_slots, const at::Tensor& cu_q, at::Tensor& out,
+                            int64_t max_qlen) {
+  const int ldq = ld_of(q, "q"), ldk = ld_of(k, "k"), ldv = ld_of(v, "v"), ldp = ld_of(P, "P"), ldw = ld_of(w, "w");
+  f32c(b, "b");
+  f32c(state, "state");
+  f32c(out, "out");
+  i32c(state_slots, "state_slots");
+  i32c(cu_q, "cu_q");
+  MCHECK(state.dim() == 4, "state must be [slots, H, dv, d]");
+  const int64_t T = q.size(0), H = state.size(1), dv = state.size(2), d = state.size(3), B = state_slots.numel();
+  if (T == 0 || B == 0) return true;
+  const bool delta = A_log.has_value();
+  MCHECK(q.size(1) % d == 0 && q.size(1) == k.size(1), "q / k must be [T, G d]");
+  const int64_t G = q.size(1) / d;
+  MCHECK(G > 0 && H % G == 0 && (delta || G == H) && k.size(0) == T && v.size(0) == T && v.size(1) == H * dv && out.numel() == T * H * dv &&
+             cu_q.numel() == B + 1 && P.size(0) == T && b.numel() == H * d && tau > 0,
+         "linear_recurrence_made: shape mismatch");
+  if (delta) {
+    f32c(*A_log, "A_log");
+    MCHECK(A_log->numel() == H && w.size(0) == T && w.size(1) >= H * d, "products must be [T, >= H d], A_log [H]");
+    cols_ok(P, p_off, H, "step sizes");
+  } else {
+    MCHECK(w.size(0) == H * d && w.is_contiguous(), "w must be [H d, rank]");
+    cols_ok(P, p_off, w.size(1), "decay projection");
+    if (w.size(1) % 16 != 0 || !rows16(P, ldp) || p_off % 4 != 0) return false;
+  }
+  if (!chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, max_qlen) || !rows16(w, ldw) || !rows16(b, 0)) return false;
+  auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, true, delta)}, q.options());
+  chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), nullptr, nullptr, ldq, ldk, ldv, 0, (float)q_scale,
+                    state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(), (int)T, (int)B, (int)H, (int)G, (int)d,
+                    (int)dv, (int)dv, (int)(max_qlen > 0 ? max_qlen : T / B), true, delta, ws.data_ptr<float>(), out.data_ptr<float>(),
+                    {P.data_ptr<float>(), ldp, (int)p_off, w.data_ptr<float>(), b.data_ptr<float>(), ldw, (float)(1.0 / tau),
+                     delta ? A_log->data_ptr<float>() : nullptr}});
+  return true;
 }
 
 void gated_rmsnorm(const at::Tensor& o, const at::Tensor& w, const at::Tensor& P, int64_t g_off, double eps, double out_scale,
@@ -1433,6 +1481,7 @@ void bind_mixers(pybind11::module& m) {
   m.def("attn_gated_chunk", &attn_gated_chunk);
   m.def("gla_prep", &gla_prep);
   m.def("linear_recurrence", &linear_recurrence);
+  m.def("linear_recurrence_made", &linear_recurrence_made);
   m.def("gated_rmsnorm", &gated_rmsnorm);
 }
 

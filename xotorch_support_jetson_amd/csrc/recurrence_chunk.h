@@ -4,6 +4,18 @@
 
 namespace xot {
 
+// Decays per key channel that chunk_prep_k makes itself: the plain write's from a low-rank product, sigmoid(P[:, p_off : +rank] w^T + b)
+// to the power of 1 / tau (w [H d, rank], A_log null), or the delta rule's exp(-exp(A_log) softplus(w + b)) of finished products w
+// [T, >= H d], with sigmoid(P[:, p_off : +H]) as the write strengths.
+struct DecaySource {
+  const float* P;
+  int ldp, p_off;
+  const float *w, *b;
+  int ldw;  // rank, or the row stride of the finished products
+  float inv_tau;
+  const float* A_log;
+};
+
 struct ChunkRecurrence {
   const float *q, *k, *v, *decay, *beta;  // beta: the delta rule's write strength, or (not delta) an input scale, may be null
   int ldq, ldk, ldv, dstride;             // dstride: decays of consecutive tokens (0: one fixed decay per head)
@@ -13,6 +25,7 @@ struct ChunkRecurrence {
   int T, B, H, G, d, dv, dvin, longest;  // longest: tokens of the longest sequence, or what is taken for it
   bool chan, delta;  // a decay per key channel; the delta rule
   float *ws, *out;
+  DecaySource src;  // (P null: decay and beta hold them)
 };
 
 // takes d 64 or 128, rows of q, k, the decays (chan) and the state on 16-byte boundaries

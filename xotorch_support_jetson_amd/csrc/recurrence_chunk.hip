@@ -9,7 +9,7 @@
 //   * chunk_prep_k, a wave per (chunk, head), all of them in parallel: q.k and k.k products, the decays, the triangular
 //     inverse by forward substitution -> M, N (16 x 16) and the scalar decays into a workspace, 2.1 KB per chunk and head.  With channel
 //     decays the scan's operands P Q, P K and (G K)^T follow them, up to 24 KB: what it costs to write them (16 heads of 128 x 128,
-//     4593 tokens: 42 us without, 69 with) every workgroup of the scan was paying again, 16 products a thread and chunk on the chain.
+//     4593 tokens: 45 us without, 64 with) every workgroup of the scan was paying again, 16 products a thread and chunk on the chain.
 //   * chunk_scan_k, the chain: a workgroup per (sequence, head, 16 or 32 value channels), a wave per 16 of them and a quarter or half
 //     of the key dims.  The state stays in MFMA accumulators: tile t, register r, lane group g holds key row
 //     16 t + 4 g + r of value channel lane % 16, and as a B operand the same register is rows 4 g + r of the tile for g = 0 .. 3
@@ -69,13 +69,19 @@ __device__ __forceinline__ float row_after(float v) {
 // chunk slots of a step: sequence b's chunks start at cu[b] / 16 + b (at least ceil(n / 16) slots before the next one's)
 __device__ __forceinline__ int slot_base(const int* cu, int b) { return cu[b] / CT + b; }
 
-template <int D, bool CHAN, bool DELTA>
-__global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk,
+// Bound by the bytes, what it reads and the operands it writes, and by registers, of which three waves a SIMD leave 168: tile by tile in a
+// chunk with channel decays, and once more from memory where a prefix product left the range (all tiles held: one wave a SIMD, 69 us).
+// MADE: the decays (and the delta rule's write strengths) come from src, in the vector unit's time.  A pass of its own that wrote them cost,
+// behind the kernels that write its inputs, 48 us for 12807 tokens of 16 heads of 64 (rank 16) and 40 for 4593 of 16 of 128, of
+// which the exponentials here take 29 (58 -> 87) and 25 (64 -> 89).
+template <int D, bool CHAN, bool DELTA, bool MADE>
+__global__ __launch_bounds__(64, CHAN ? 3 : 2) void chunk_prep_k(const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk,
                                                    const float* __restrict__ decay, int dstride,
                                                    const float* __restrict__ beta, float q_scale,
                                                    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B,
-                                                   int H, int G, int heads, float* __restrict__ ws) {
+                                                   int H, int G, int heads, DecaySource src, float* __restrict__ ws) {
   __shared__ float sA[CT][CT + 1];
+  __shared__ __attribute__((aligned(16))) float sT[CHAN ? 2 : 1][CHAN ? CT : 1][CT + 4];  // a tile's way from dims to tokens
   constexpr bool SHARE = !CHAN && !DELTA;
   const int s = blockIdx.x, h = blockIdx.y * (SHARE ? heads : 1), lane = threadIdx.x, i = lane & 15, g = lane >> 4;
   int lo = 0, hi = B - 1;
@@ -89,84 +95,116 @@ __global__ __launch_bounds__(64) void chunk_prep_k(const float* __restrict__ q, 
   const bool valid = tok < n;
   const int64_t t = t0 + min(tok, n - 1);
   const int hk = h / (H / G);
-  f32x4 qf[D / 16], kf[D / 16], af[CHAN ? D / 16 : 1];
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  // tile j of the tokens' q, k (past the end: 0) and what their decays come from
+  auto load_q = [&](int j) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(q + t * ldq + hk * D + 16 * j + 4 * g);
+    return valid ? x : zero4;
+  };
+  auto load_k = [&](int j) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(k + t * ldk + hk * D + 16 * j + 4 * g);
+    return valid ? x : zero4;
+  };
+  auto load_a = [&](int j) {
+    if constexpr (!CHAN || (MADE && !DELTA)) return zero4;
+    else if constexpr (MADE) return *reinterpret_cast<const f32x4*>(src.w + t * src.ldw + h * D + 16 * j + 4 * g);
+    else return *reinterpret_cast<const f32x4*>(decay + (t * H + h) * D + 16 * j + 4 * g);
+  };
+  f32x4 qf[D / 16], kf[D / 16], af[D / 16];
 #pragma unroll
   for (int j = 0; j < D / 16; ++j) {
-    qf[j] = *reinterpret_cast<const f32x4*>(q + t * ldq + hk * D + 16 * j + 4 * g);
-    kf[j] = *reinterpret_cast<const f32x4*>(k + t * ldk + hk * D + 16 * j + 4 * g);
-    if (CHAN) af[CHAN ? j : 0] = *reinterpret_cast<const f32x4*>(decay + (t * H + h) * D + 16 * j + 4 * g);
+    qf[j] = load_q(j);
+    kf[j] = load_k(j);
+    af[j] = load_a(j);
   }
-  float gi = CHAN || !valid ? 1.0f : decay[t * dstride + h];
-  const float bi = DELTA && valid ? beta[t * H + h] : 0.0f;
-  if (!valid) {
+  const float rate = MADE && DELTA ? -expf(src.A_log[h]) : 0.0f;
+  auto decays = [&](int j, f32x4 a) {  // tile j of the decays (past the end: 1)
+    if constexpr (MADE) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(src.b + h * D + 16 * j + 4 * g);
+      if constexpr (!DELTA) {
+        // (the product, dims by tokens, has them where the loads have theirs: row 4 g + r is dim 16 j + 4 g + r, column i the token; of
+        // each 16 of the rank a lane brings 4 g .. 4 g + 3)
+        for (int k0 = 0; k0 < src.ldw; k0 += 16) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(src.P + t * src.ldp + src.p_off + k0 + 4 * g);
+          const f32x4 w = *reinterpret_cast<const f32x4*>(src.w + (int64_t)(h * D + 16 * j + i) * src.ldw + k0 + 4 * g);
 #pragma unroll
-    for (int j = 0; j < D / 16; ++j) {
-      qf[j] = kf[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (CHAN) af[CHAN ? j : 0] = f32x4{1.f, 1.f, 1.f, 1.f};
+          for (int r = 0; r < 4; ++r) a = mfma4(w[r], x[r], a);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        a[r] = DELTA ? expf(rate * softplusf_(a[r] + b[r])) : expf(logsigmoidf_(a[r] + b[r]) * src.inv_tau);
     }
-  }
+    return valid ? a : f32x4{1.f, 1.f, 1.f, 1.f};
+  };
+  float gi = CHAN || !valid ? 1.0f : decay[t * dstride + h];
+  const float bi = !DELTA || !valid ? 0.0f : MADE ? sigmoidf_(src.P[t * src.ldp + src.p_off + h]) : beta[t * H + h];
   float* M = ws + ((int64_t)s * H + h) * rec_floats(D, CHAN, DELTA);
   // accumulators: row 4 g + r (token i), column lane % 16 (token j)
   f32x4 qs[8], ks[8];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) qs[r] = ks[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < 8; ++r) qs[r] = ks[r] = zero4;
   f32x4 gam = {1.f, 1.f, 1.f, 1.f};
   if (CHAN) {
+    // Tile by tile, so that what is loaded is what takes registers: the scan's operands P Q and P K as they are here and (decays after a
+    // token) K with tokens and dims exchanged, and the products for chunks whose prefix products all stay near one
     bool near = true;
-    f32x4 P[D / 16];
-#pragma unroll
-    for (int j = 0; j < D / 16; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        P[j][r] = row_scan(af[CHAN ? j : 0][r]);
-        near = near && P[j][r] >= 1.0f / FAR && P[j][r] <= FAR;
-      }
-    // the scan's operands: P Q and P K as they are here, (decays after a token) K with tokens and dims exchanged
     float* op = M + MN;
 #pragma unroll
     for (int j = 0; j < D / 16; ++j) {
-      if (i == CT - 1) *reinterpret_cast<f32x4*>(op + 16 * j + 4 * g) = P[j];
-      *reinterpret_cast<f32x4*>(op + D + j * 256 + lane * 4) = qf[j] * P[j] * q_scale;
-      if (DELTA) *reinterpret_cast<f32x4*>(op + D + 2 * CT * D + j * 256 + lane * 4) = kf[j] * P[j];
+      const f32x4 a = decays(j, af[j]);
+      f32x4 P, ki;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        op[D + CT * D + j * 256 + ((i >> 2) * 16 + 4 * g + r) * 4 + (i & 3)] = kf[j][r] * row_after(af[CHAN ? j : 0][r]);
+      for (int r = 0; r < 4; ++r) {
+        P[r] = row_scan(a[r]);
+        near = near && P[r] >= 1.0f / FAR && P[r] <= FAR;
+        ki[r] = kf[j][r] / P[r];
+      }
+      if (i == CT - 1) *reinterpret_cast<f32x4*>(op + 16 * j + 4 * g) = P;
+      const f32x4 pq = qf[j] * P, pk = kf[j] * P;
+      *reinterpret_cast<f32x4*>(op + D + j * 256 + lane * 4) = pq * q_scale;
+      if (DELTA) *reinterpret_cast<f32x4*>(op + D + 2 * CT * D + j * 256 + lane * 4) = pk;
+      f32x4 gk;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gk[r] = kf[j][r] * row_after(a[r]);
+      *reinterpret_cast<f32x4*>(&sT[CHAN ? j & 1 : 0][CHAN ? i : 0][4 * g]) = gk;  // (one wave: its LDS accesses keep their order)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        qs[r + 4 * (j & 1)] = mfma4(pq[r], ki[r], qs[r + 4 * (j & 1)]);
+        if (DELTA) ks[r + 4 * (j & 1)] = mfma4(pk[r], ki[r], ks[r + 4 * (j & 1)]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gk[r] = sT[CHAN ? j & 1 : 0][CHAN ? 4 * g + r : 0][i];
+      *reinterpret_cast<f32x4*>(op + D + CT * D + j * 256 + lane * 4) = gk;
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (__all(near)) {
+    if (!__all(near)) {
+      // row by row: kh_j = k_j times the decays after j, multiplied on token by token (from memory again)
 #pragma unroll
-      for (int j = 0; j < D / 16; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float ki = kf[j][r] / P[j][r];
-          qs[r + 4 * (j & 1)] = mfma4(qf[j][r] * P[j][r], ki, qs[r + 4 * (j & 1)]);
-          if (DELTA) ks[r + 4 * (j & 1)] = mfma4(kf[j][r] * P[j][r], ki, ks[r + 4 * (j & 1)]);
-        }
-    } else {
-      // row by row: kh_j = k_j times the decays after j, multiplied on token by token
-      f32x4 kh[D / 16];
-#pragma unroll
-      for (int j = 0; j < D / 16; ++j) kh[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int row = 0; row < CT; ++row) {
-        const int src = (lane & 48) + row;
-        float dq = 0.0f, dk = 0.0f;
-#pragma unroll
-        for (int j = 0; j < D / 16; ++j)
+      for (int r = 0; r < 8; ++r) qs[r] = ks[r] = zero4;
+      for (int j = 0; j < D / 16; ++j) {
+        const f32x4 qj = load_q(j), kj = load_k(j), a = decays(j, load_a(j));
+        f32x4 kh = zero4;
+        for (int row = 0; row < CT; ++row) {
+          const int from = (lane & 48) + row;
+          float dq = 0.0f, dk = 0.0f;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float ar = __shfl(af[CHAN ? j : 0][r], src), qr = __shfl(qf[j][r], src), kr = __shfl(kf[j][r], src);
-            kh[j][r] = i == row ? kf[j][r] : i < row ? kh[j][r] * ar : 0.0f;
-            dq += qr * kh[j][r];
-            if (DELTA) dk += kr * kh[j][r];
+            const float ar = __shfl(a[r], from), qr = __shfl(qj[r], from), kr = __shfl(kj[r], from);
+            kh[r] = i == row ? kj[r] : i < row ? kh[r] * ar : 0.0f;
+            dq += qr * kh[r];
+            if (DELTA) dk += kr * kh[r];
           }
-        dq = xor_sum<16>(dq);
-        dq = xor_sum<32>(dq);
-        dk = xor_sum<16>(dk);
-        dk = xor_sum<32>(dk);
-        if ((row >> 2) == g) {
-          qs[0][0] = (row & 3) == 0 ? dq : qs[0][0], ks[0][0] = (row & 3) == 0 ? dk : ks[0][0];
-          qs[0][1] = (row & 3) == 1 ? dq : qs[0][1], ks[0][1] = (row & 3) == 1 ? dk : ks[0][1];
-          qs[0][2] = (row & 3) == 2 ? dq : qs[0][2], ks[0][2] = (row & 3) == 2 ? dk : ks[0][2];
-          qs[0][3] = (row & 3) == 3 ? dq : qs[0][3], ks[0][3] = (row & 3) == 3 ? dk : ks[0][3];
+          dq = xor_sum<16>(dq);
+          dq = xor_sum<32>(dq);
+          dk = xor_sum<16>(dk);
+          dk = xor_sum<32>(dk);
+          if ((row >> 2) == g) {
+            qs[0][0] += (row & 3) == 0 ? dq : 0.0f, ks[0][0] += (row & 3) == 0 ? dk : 0.0f;
+            qs[0][1] += (row & 3) == 1 ? dq : 0.0f, ks[0][1] += (row & 3) == 1 ? dk : 0.0f;
+            qs[0][2] += (row & 3) == 2 ? dq : 0.0f, ks[0][2] += (row & 3) == 2 ? dk : 0.0f;
+            qs[0][3] += (row & 3) == 3 ? dq : 0.0f, ks[0][3] += (row & 3) == 3 ? dk : 0.0f;
+          }
         }
       }
     }
@@ -576,8 +614,16 @@ void go(const ChunkRecurrence& a) {
   // scan: 5 of 364 .. 1728 tokens 110 -> 100 us, 8 of 961 .. 2433 247 -> 223; three of 1000 not; two heads under the delta rule gave nothing)
   const int heads = !CHAN && !DELTA && (int64_t)slots * a.G >= 2048 ? a.H / a.G : 1;
   const dim3 pg((unsigned)slots, (unsigned)(a.H / heads));
-  chunk_prep_k<D, CHAN, DELTA><<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale,
-                                                        a.state_slots, a.cu_q, a.B, a.H, a.G, heads, a.ws);
+  auto prep = [&](auto kern) {
+    kern<<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale, a.state_slots, a.cu_q, a.B, a.H, a.G,
+                                  heads, a.src, a.ws);
+  };
+  if constexpr (CHAN) {
+    if (a.src.P != nullptr) prep(chunk_prep_k<D, CHAN, DELTA, true>);
+    else prep(chunk_prep_k<D, CHAN, DELTA, false>);
+  } else {
+    prep(chunk_prep_k<D, CHAN, DELTA, false>);
+  }
   // Steps whose longest sequence takes longer than the CUs' share of all chunks are bound by its chain: four waves of a quarter of the
   // key dims each, 16 channels a workgroup, three chunks ahead.  Others by the matrix unit: two halves and 32 channels, which
   // repeat the products with M and N less.  The line by T (tokens) x workgroups of 32 channels a sequence / (256 x the longest), us

@@ -744,30 +744,35 @@ class ShardModel:
                 self.c.rms_norm_eps, out, max_qlen=inp.max_qlen, width=lw.conv_width, **gates)
     return out
 
-  def _low_rank(self, P: torch.Tensor, off: int, n: int, w: torch.Tensor) -> torch.Tensor:
-    """Second projection of a low-rank pair on the GEMM kernels: w (padded) times the operand copy of P[:, off : +n]."""
-    x = torch.zeros(P.shape[0], w.shape[1], dtype=w.dtype, device=P.device)
-    x[:, :n] = P[:, off:off + n].to(w.dtype)
-    return self._proj(x, w)
+  def _low_rank(self, P: torch.Tensor, a, b) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Second projections of two low-rank pairs on the GEMM kernels: for each of a, b = (first column, rank, w) w (its columns padded)
+    times the operand copy of P[:, first : + rank]; of ranks that need no padding, side by side in P, one copy."""
+    (a0, an, aw), (b0, bn, bw) = a, b
+    if b0 == a0 + an and an == aw.shape[1] and bn == bw.shape[1]:
+      x = P[:, a0:b0 + bn].to(aw.dtype)
+      return self._proj(x[:, :an], aw), self._proj(x[:, an:], bw)
+    pad = torch.nn.functional.pad
+    return tuple(self._proj(pad(P[:, o:o + n].to(w.dtype), (0, w.shape[1] - n)), w) for o, n, w in (a, b))
 
   def _channel_delta(self, P: torch.Tensor, lw, j: int, inp: StepInputs, mix: torch.Tensor) -> None:
     """Delta rule with a decay per key channel on the state slots: convolutions + SiLU + unit norms, step sizes and low-rank
     decays and output gates (prompts: their second projections are GEMMs), the recurrence, the per-head gated norm."""
     r, st, dev = lw.spec.rec, self.state, P.device
     T, H, nk, nv = mix.shape[0], r.heads, r.kv_heads * r.dim, r.heads * r.vdim
-    beta = torch.empty(T, H, dtype=torch.float32, device=dev)
-    decay = torch.empty(T, H * r.dim, dtype=torch.float32, device=dev)
     (a0, an), (g0, gn) = lw.cols["ra1"], lw.cols["rg1"]
+    beta = decay = chan = None
     if P.is_cuda and P.dim() == 2 and lw.a2_p is not None and T >= LOW_RANK_GEMM_ROWS:
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp)
-      za, gate = self._low_rank(P, a0, an, lw.a2_p), self._low_rank(P, g0, gn, lw.g2_p)
-      K.recurrence_gates(P, lw.cols["rb"][0], beta, 0, None, lw.dt_bias, lw.A_log, decay, 0, None, None, za=za)
+      za, gate = self._low_rank(P, (a0, an, lw.a2_p), (g0, gn, lw.g2_p))
+      chan = (P, lw.cols["rb"][0], za, lw.dt_bias, lw.A_log)
     else:
+      beta = torch.empty(T, H, dtype=torch.float32, device=dev)
+      decay = torch.empty(T, H * r.dim, dtype=torch.float32, device=dev)
       gate = torch.empty(T, nv, dtype=torch.float32, device=dev)
       qkv = self._conv(P, lw.cols["rq"][0], lw, j, inp,
                        gates=(lw.cols["rb"][0], beta, a0, lw.a2_w, lw.dt_bias, lw.A_log, decay, g0, lw.g2_w, gate))
     K.recurrence_norm(qkv[:, :nk], qkv[:, nk:2 * nk], qkv[:, 2 * nk:], decay, beta, 1.0, st.S[j], inp.state_slots, inp.cu_q,
-                      lw.rec_norm, gate, True, self.c.rms_norm_eps, 1.0, mix, max_qlen=inp.max_qlen)
+                      lw.rec_norm, gate, True, self.c.rms_norm_eps, 1.0, mix, max_qlen=inp.max_qlen, chan=chan)
 
   def _ssd_conv(self, P: torch.Tensor, x: torch.Tensor, dt: torch.Tensor, decay: torch.Tensor, lw, j: int, inp: StepInputs,
                 mix: torch.Tensor) -> None:

@@ -665,11 +665,21 @@ def gated_rmsnorm(o, w, P, g_off: int, eps: float, out_scale: float, out) -> Non
 
 
 def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu_q, w, gate, sigmoid: bool, eps: float, scale: float,
-                    out, gla=None, max_qlen: int = 0, gelu=None) -> None:
+                    out, gla=None, max_qlen: int = 0, gelu=None, chan=None) -> None:
   """linear_recurrence, then each head's RMS norm times w ([dv], or one per head [H dv]), gate [T, H dv]'s silu (or its logistic
   function) and scale -> out [T, >= H dv].  gla: (P, first column, a2, a2_b, tau) of gla_prep, which then makes the decays.  gelu:
-  arguments of a gelu_mul that is done along with it.  A step of single tokens is one launch on the GPU (csrc/recurrence_step.hip)
-  where that covers the sizes."""
+  arguments of a gelu_mul that is done along with it.  chan: (P, column of the step sizes, za, dt_bias, A_log) of recurrence_gates, which
+  then makes decays and write strengths.  A step of single tokens is one launch on the GPU (csrc/recurrence_step.hip)
+  where that covers the sizes; prompts' decays are made inside the recurrence (csrc/recurrence_chunk.hip) where it takes them."""
+  def made_gates():
+    P, b_off, za, dt_bias, A_log = chan
+    beta = torch.empty(q.shape[0], A_log.numel(), dtype=torch.float32, device=q.device)
+    decay = torch.empty(q.shape[0], dt_bias.numel(), dtype=torch.float32, device=q.device)
+    recurrence_gates(P, b_off, beta, 0, None, dt_bias, A_log, decay, 0, None, None, za=za)
+    return decay, beta
+  if chan is not None and (max_qlen == 1 or not _gpu(q)):
+    decay, beta = made_gates()
+    chan = None
   if max_qlen == 1 and _gpu(q):
     a1, a2, a2_b, tau = (gla[0][:, gla[1]:gla[1] + gla[2].shape[1]], *gla[2:]) if gla is not None else (None, None, None, 0.0)
     for g in ((gelu, None) if gelu is not None else (None,)):  # (an activation it cannot take along has a launch of its own)
@@ -681,11 +691,22 @@ def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu
   if gelu is not None:
     gelu_mul(*gelu)
   T, H, dv, d = q.shape[0], state.shape[1], state.shape[2], state.shape[3]
-  if gla is not None:
-    decay = torch.empty(T, H * d, dtype=torch.float32, device=q.device)
-    gla_prep(*gla, decay)
   o = torch.empty(T, H * dv, dtype=torch.float32, device=q.device)
-  linear_recurrence(q, k, v, decay, beta, q_scale, state, state_slots, cu_q, o, max_qlen=max_qlen)
+  done = False
+  if chan is not None:
+    P, b_off, za, dt_bias, A_log = chan
+    done = require().linear_recurrence_made(q, k, v, P, int(b_off), za, dt_bias, 1.0, A_log, float(q_scale), state, state_slots, cu_q, o, int(max_qlen))
+    if not done:
+      decay, beta = made_gates()
+  elif gla is not None:
+    if _gpu(q) and beta is None and gla[0].dim() == 2:
+      P, a1_off, a2, a2_b, tau = gla
+      done = require().linear_recurrence_made(q, k, v, P, int(a1_off), a2, a2_b, float(tau), None, float(q_scale), state, state_slots, cu_q, o, int(max_qlen))
+    if not done:
+      decay = torch.empty(T, H * d, dtype=torch.float32, device=q.device)
+      gla_prep(*gla, decay)
+  if not done:
+    linear_recurrence(q, k, v, decay, beta, q_scale, state, state_slots, cu_q, o, max_qlen=max_qlen)
   if sigmoid:  # (that pass has a weight per head and no scale)
     wh = w if w.numel() == H * dv else w.repeat(H)
     gated_group_norm(o, None, wh if scale == 1.0 else wh * scale, gate, 0, H, eps, out)
