@@ -21,9 +21,9 @@
 // LDS, all waves' products of half of the key dims and two barriers; a wave issues one instruction at a time, and loads,
 // addresses and selections between the MFMAs were as many as them).  With many the matrix unit: 54 MFMAs of 32 cycles a wave of
 // half of the key dims, at 55 % of its rate.  One prompt of 2000 tokens, both kernels, us before and now: delta rule 16 heads of 128 x 128
-// 196 and 130, with channel decays 310 and 138, per-channel decays 16 heads of 64 x 128 157 and 79, plain write 32 heads of 128 x 64 160 and
-// 98; 5 of 364 .. 1728: 187, 294, 142, 152 and 152, 180, 84, 100; 8 of 961 .. 2433: 312, 490, 220, 254 and 298, 400, 205, 223; 32 of
-// 51 .. 1460: 302, 458, 203, 270 and 308, 411, 194, 230.
+// 197 and 129, with channel decays 306 and 136, per-channel decays 16 heads of 64 x 128 153 and 81, plain write 32 heads of 128 x 64 156 and
+// 103; 5 of 364 .. 1728: 185, 293, 141, 150 and 143, 181, 87, 104; 8 of 961 .. 2433: 307, 488, 219, 253 and 292, 402, 197, 223; 32 of
+// 50 .. 1515: 314, 476, 211, 283 and 317, 439, 202, 243.
 // v_mfma_f32_16x16x4_f32 multiplies and accumulates in fp32 as the vector units do; no operand is rounded.
 //
 // Decays per key channel: where a prefix product P leaves 2^-100 .. 2^100 (a decay of 0, or a value that is no number, among
@@ -43,6 +43,12 @@ constexpr float FAR = 1.2676506e30f;            // 2^100
 constexpr int rec_floats(int D, bool chan, bool delta) { return MN + (chan ? D + (delta ? 3 : 2) * CT * D : 0); }
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// a b, rounded before anything is added to it
+__device__ __forceinline__ f32x4 times(f32x4 a, f32x4 b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
 
 // inclusive product over the 16 lanes of a DPP row, in lane order (lanes without a source keep their value: x * 1)
 template <int CTRL>
@@ -298,7 +304,9 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ inscale, float q_scale, float* __restrict__ state, const int* __restrict__ state_slots,
     const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, const float* __restrict__ ws, float* __restrict__ out) {
+  static_assert(KP == 2 || KP == 4, "the order of the sums is that of quarters of the key dims");
   constexpr int TILES = D / 16 / KP;              // 16-row state tiles of a wave
+  constexpr int QW = 4 / KP, QT = TILES / QW;     // quarters of the key dims in a wave, tiles of each
   constexpr int REC = rec_floats(D, CHAN, DELTA);
   // the write's operand, k with tokens and dims exchanged: from the workspace (channel decays), from the rows of k that the delta
   // rule's product has through LDS, or element by element (16 heads of 128 x 128, 8 of 961 .. 2433 tokens: delta rule 312 us
@@ -306,8 +314,8 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
   constexpr bool TURN = DELTA && !CHAN, SINGLE = !DELTA && !CHAN;
   constexpr int LT = D / KP + 4;                  // LDS row of a wave's k: consecutive tokens four banks apart
   __shared__ __attribute__((aligned(16))) float sk[TURN ? KP * CG : 1][TURN ? CT * LT : 1];
-  __shared__ f32x4 sx[DELTA && KP > 1 ? 2 : 1][CG][DELTA && KP > 1 ? KP : 1][64];  // partial products of the waves of a group
-  __shared__ f32x4 sy[KP > 1 ? 2 : 1][CG][KP > 1 ? KP : 1][64];
+  __shared__ f32x4 sx[DELTA ? 2 : 1][CG][DELTA ? KP : 1][64];  // partial products of the waves of a group
+  __shared__ f32x4 sy[2][CG][KP][64];
   const int h = blockIdx.x;
   const int b = nth_longest(B, scan_order((int)blockIdx.z, B, H * (int)gridDim.y), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
@@ -351,9 +359,9 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     ot[r] = ((4 * g + r) * ldk + d0 + i) * 4;
     ov[r] = ((4 * g + r) * ldv + vcol) * 4;
     ob[r] = (4 * g + r) * H * 4;
-    // (KP > 1: a chunk's rows are stored in the next one's turn.  What is before the first chunk, channels past the end and the waves
-    // that do not have the sum: past every window)
-    oo[r] = live && kp == 0 ? (uint32_t)(((4 * g + r - (KP > 1 ? CT : 0)) * H * dv + col) * 4) : 0x80000000u;
+    // (a chunk's rows are stored in the next one's turn.  What is before the first chunk, channels past the end and the waves that do
+    // not have the sum: past every window)
+    oo[r] = live && kp == 0 ? (uint32_t)(((4 * g + r - CT) * H * dv + col) * 4) : 0x80000000u;
     asm volatile("" : "+v"(ot[r]), "+v"(ov[r]), "+v"(oo[r]));
   }
   asm volatile("" : "+v"(oq), "+v"(ok), "+v"(om), "+v"(od), "+v"(oc));  // (constants added to them are then the loads' own)
@@ -466,19 +474,24 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     for (int j = 0; j < NR; ++j) load_rest(wr, ops[u], j);
     next_rest();
   }
-  f32x4 last = {0.f, 0.f, 0.f, 0.f};  // KP > 1: the chunk before, of which the other waves' parts are in LDS
+  // Products with the state are summed by quarters of the key dims, these in pairs, whichever waves hold them: a sequence's numbers do
+  // not depend on the form of the scan, which the step's other sequences have a part in, and are the same in all waves of a group.
+  auto pairs = [&](f32x4 mine, const f32x4 (&other)[KP - 1]) {
+    if constexpr (KP == 2) return mine + other[0];
+    else return (mine + other[0]) + (other[1] + other[2]);
+  };
+  f32x4 last = {0.f, 0.f, 0.f, 0.f};  // the chunk before: N U (kp 0); the waves' parts of P Q S are in LDS
   auto parts = [&](int buf) {
-    f32x4 y = last;
+    f32x4 other[KP - 1];
 #pragma unroll
-    for (int w = 1; w < KP; ++w) y += sy[KP > 1 ? buf : 0][cg][KP > 1 ? w : 0][lane];
-    return y;
+    for (int w = 1; w < KP; ++w) other[w - 1] = sy[buf][cg][kp ^ w][lane];
+    return last + pairs(sy[buf][cg][kp][lane], other);
   };
   // Loads and stores between the MFMAs, which hold the matrix unit 32 cycles each: behind them they were on the chain
   auto pin = [&]() { __builtin_amdgcn_sched_barrier(0x86); };  // (vector, scalar and LDS operations may pass)
   auto chunk = [&](int c, int buf, Ops& o, Ops& before) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    // (partial sums: shorter chains, and sums of fewer terms)
-    f32x4 xs[2] = {zero, zero}, ys[2] = {zero, zero};
+    f32x4 xs[2], ys[2], X, mine;  // (partial sums: shorter chains, and sums of fewer terms)
     const __amdgpu_buffer_rsrc_t wq = record(Wq, cq), wr = record(Wr, cr);
     int s = 0;
     float* kt = &sk[TURN ? wave : 0][0];
@@ -491,29 +504,26 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
       for (int j = 0; j < TILES; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          xs[r & 1] = mfma4(o.k[DELTA ? j : 0][r], S[j][r], xs[r & 1]);
+          xs[r & 1] = mfma4(o.k[DELTA ? j : 0][r], S[j][r], r < 2 && j % QT == 0 ? zero : xs[r & 1]);
           load_rest(wr, before, s++);
           load_rest(wr, before, s++);
           pin();
+          if (r == 3 && j % QT == QT - 1) X = j < QT ? xs[0] + xs[1] : X + (xs[0] + xs[1]);
         }
+      sx[DELTA ? buf : 0][cg][DELTA ? kp : 0][lane] = X;
     }
-    f32x4 X = xs[0] + xs[1];
-    if constexpr (KP > 1) {
-      if constexpr (DELTA) sx[DELTA ? buf : 0][cg][DELTA ? kp : 0][lane] = X;
-      bar();
-    }
-    f32x4 xo[KP > 1 ? KP - 1 : 1];
-    if constexpr (DELTA && KP > 1) {
+    bar();
+    f32x4 xo[KP - 1];
+    if constexpr (DELTA) {
 #pragma unroll
-      for (int w = 1; w < KP; ++w) xo[w - 1] = sx[DELTA ? buf : 0][cg][DELTA ? (kp + w) % KP : 0][lane];
+      for (int w = 1; w < KP; ++w) xo[w - 1] = sx[DELTA ? buf : 0][cg][DELTA ? kp ^ w : 0][lane];
     }
-    f32x4 y = last;
-    if constexpr (KP > 1) y = parts(buf ^ 1);
+    const f32x4 y = parts(buf ^ 1);
 #pragma unroll
     for (int j = 0; j < TILES; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        ys[r & 1] = mfma4(o.q[j][r], S[j][r], ys[r & 1]);
+        ys[r & 1] = mfma4(o.q[j][r], S[j][r], r < 2 && j % QT == 0 ? zero : ys[r & 1]);
         if (r == 0) load_k(wq, o, j);
         if constexpr (DELTA) {
           load_rest(wr, before, s++);
@@ -522,11 +532,16 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
           load_rest(wr, before, s++);
         }
         pin();
+        if (r == 3 && j % QT == QT - 1) {
+          f32x4 part = ys[0] + ys[1];
+          if (!CHAN) part = times(part, o.p * q_scale);
+          mine = j < QT ? part : mine + part;
+        }
       }
 #pragma unroll
     for (; s < NR; ++s) load_rest(wr, before, s);
     next_rest();
-    if constexpr (KP > 1) store(y);
+    store(y);
     // the decayed state meets the chunk's write after the products that read it
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
@@ -541,10 +556,7 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
       if (!DELTA) U[r] *= inscale ? o.m[r] : 1.0f;
     }
     if constexpr (DELTA) {
-      if constexpr (KP > 1) {
-#pragma unroll
-        for (int w = 1; w < KP; ++w) X += xo[w - 1];
-      }
+      X = pairs(X, xo);
       f32x4 R;
 #pragma unroll
       for (int r = 0; r < 4; ++r) R[r] = U[r] - (CHAN ? X[r] : o.p[r] * X[r]);
@@ -564,18 +576,8 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
         pin();
       }
     next_state();
-    f32x4 Y = ys[0] + ys[1];
-    if (!CHAN) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Y[r] *= o.p[r] * q_scale;
-    }
-    if (KP == 1 || kp == 0) Y = lower(o.nn, U, Y);
-    if constexpr (KP > 1) {
-      sy[KP > 1 ? buf : 0][cg][KP > 1 ? kp : 0][lane] = Y;
-      last = Y;
-    } else {
-      store(Y);
-    }
+    sy[buf][cg][kp][lane] = mine;
+    if (kp == 0) last = lower(o.nn, U, zero);
   };
   // (ends left where the chunks end, none joined again: at a join the compiler waits for every load that one of the paths may have
   // issued last, and a copy of the loop's body for the rest keeps a second set of operands in registers)
@@ -589,10 +591,8 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     }
     if (end) break;
   }
-  if constexpr (KP > 1) {
-    bar();
-    store(parts((chunks - 1) & 1));
-  }
+  bar();
+  store(parts((chunks - 1) & 1));
   if (live) {
 #pragma unroll
     for (int j = 0; j < TILES; ++j) *reinterpret_cast<f32x4*>(St + 16 * j) = S[j];
