@@ -168,6 +168,27 @@ def test_decays_and_write_strengths_from_finished_products(gpu, d, G):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rule", ["delta", "channel_delta", "channel", "scaled"])
+@pytest.mark.parametrize("B,dv,longest", [(1, 64, 47), (1, 64, 48), (3, 64, 63), (3, 64, 64), (32, 128, 31), (32, 128, 32), (31, 128, 32)])
+def test_both_sides_of_the_chunk_rule(gpu, rule, B, dv, longest):
+  """The lengths from which steps go by chunks (mixers.hip chunks_take), against the same step token by token (longest taken as 1)."""
+  channel, delta, scaled, _ = RULES[rule]
+  H, d, lens = 16, 64, [max(1, longest - 5 * b % longest) for b in range(B)]
+  T, g = sum(lens), torch.Generator(device=gpu).manual_seed(B + longest)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  q, k, v, a = rn(T, H * d) / 8, rn(T, H * d) / 8, rn(T, H * dv), torch.sigmoid(3 + rn(T, H * (d if channel else 1)))
+  beta, state = torch.sigmoid(rn(T, H)) if delta or scaled else None, rn(B, H, dv, d)
+  slots, cu, got = torch.arange(B, dtype=torch.int32, device=gpu), torch.tensor([0] + lens).cumsum(0).int().to(gpu), []
+  for said in (1, longest):
+    S, out = state.clone(), torch.empty(T, H * dv, device=gpu)
+    K.linear_recurrence(q, k, v, a, beta, 0.7, S, slots, cu, out, plain=scaled, max_qlen=said)
+    got.append((out, S))
+  for one, other in zip(*got):  # (both are within 1e-6 of float64, test_chunks_match_token_by_token; a single value within some times that)
+    assert ((one - other).norm() / one.norm()) < 2e-6
+    torch.testing.assert_close(one, other, rtol=0, atol=float(4e-6 * one.abs().max()))
+
+
+@pytest.mark.gpu
 def test_chunk_rule_keeps_what_it_cannot_take(gpu):
   """Rows off 16 bytes, key dims it has no tiles for and short steps run token by token, with the same results."""
   g = torch.Generator(device=gpu).manual_seed(3)
