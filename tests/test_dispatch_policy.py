@@ -145,6 +145,24 @@ def test_tall_k_halves_follow_the_rows_of_the_call(monkeypatch):
   assert splits(L.GemmPolicy(), 2048, 4096, 28672) == 1
 
 
+@pytest.mark.parametrize("M,N,Kd,parts", [(1024, 2048, 2048, 3), (1280, 2048, 5632, 3), (1281, 2048, 5632, 2), (1663, 2048, 4096, 2),
+                                          (2048, 2048, 2048, 2), (2049, 2048, 2048, 1), (1663, 2048, 1920, 1), (4096, 1024, 2048, 2),
+                                          (1024, 4096, 2048, 2), (1025, 4096, 2048, 1), (1664, 2048, 24576, 2)])
+def test_tall_parts_that_the_next_pass_sums(monkeypatch, M, N, Kd, parts):
+  """A product whose slabs the pass behind it sums is cut where 128-row tiles fill at most half the CUs, into no more than one round."""
+  monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: False)
+  sized = []
+  monkeypatch.setattr(L.scratch, "splitk", lambda dev, n, slot=0: sized.append(n))
+  x, w = (torch.empty(r, Kd, dtype=torch.bfloat16, device="meta") for r in (M, N))
+  for epi, dt in (("none", torch.float32), ("resid", torch.bfloat16)):
+    assert L.GemmPolicy().shuffled_cfg(x, w, None, None, epi, dt, summed=True) == ("big", 4256, parts)
+    whole = L.GemmPolicy().shuffled_cfg(x, w, None, None, epi, dt)
+    assert whole == ("big", 4256, 2 if Kd == 24576 else 1)
+  assert sized == ([parts * M * N] * len(sized)) and (parts == 1) == (not sized)
+  monkeypatch.setattr(L.GemmPolicy, "_no_tuning", lambda self: True)
+  assert L.GemmPolicy().shuffled_cfg(x, w, None, None, "none", torch.float32, summed=True) == ("big", 4256, 1)
+
+
 def test_qkv_projection_is_timed_with_what_follows_it(monkeypatch):
   """linear_rope_kv's choice: the rotation and the KV write behind a whole product, one launch behind slabs, are part of the time, so
   a whole product that is the faster one by itself does not win."""

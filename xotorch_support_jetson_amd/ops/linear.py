@@ -454,12 +454,14 @@ class GemmPolicy:
     top = sorted(busiest, key=lambda nt: (busiest[nt], -nt))[:3]
     return [("wave", nt, 1) for nt in top if busiest[nt] * 256 <= 1.4 * tiles]
 
-  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", slabs: bool = False, run=None) -> Tuple:
+  def shuffled_cfg(self, x, w, bias, residual, epi, out_dtype, wave: str = "", slabs: bool = False, run=None,
+                   summed: bool = False) -> Tuple:
     """(kernel, ntw | bn, split-K) for a pre-shuffled weight at this M bucket.  wave: the caller also takes the whole-K decode
     GEMM ("y": plain output; "rope": the QKV projection, whose rotation and KV write it does itself -- the others' slab
     reduce, timed with them, stands for the launch that does it there).  slabs: the caller's consumer reads split-K slabs
     itself, so a split is timed without their reduce (2048 x 5632 at 6 rows: 9.1 us whole, 6.4 in 11 slabs, 10.2 with the reduce).
     run(cfg): what the caller does with a choice, where launches of its own that depend on it follow; timed in the GEMM's place.
+    summed: the pass over rows that follows reads slabs in place of the result, at any number of rows.
     wave "solo": the caller takes the whole-K GEMM of single column tiles too."""
     M, Kd = x.shape
     N = w.shape[0]
@@ -489,11 +491,18 @@ class GemmPolicy:
       # halves summed by the norm: 1024 x 4096 x 8192 124 / 89 / 129 / 82, x 14336 185 / 121 / 190 / 122; 1500 x 4096 x 14336
       # 186 / 150 / 193 / 150; 2048 x 4096 x 8192 131 / 116 / 138 / 118, x 11008 144 / 149 / 156 / 149, x 14336 204 / 202 / 210
       # / 199; K 4096: 58 / 74.  Plain ones from K ~ 24576 (2048 x 4096 x 28672 427 / 369).
-      # Not stored: the halves follow this M, a table entry would answer for its whole bucket.
-      half = -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576)
-      if half and not self._no_tuning():  # (the slabs are sized outside a capture)
-        scratch.splitk(x.device, 2 * M * N)
-        return ("big", 4256, 2)
+      # Where even 128-row tiles leave half the CUs idle and the pass that follows sums the slabs, two parts, or three where they fit one
+      # round, from K 2048 on; us in one, two and three parts with that pass, 2048 columns, fp32 result and scaled residual sum:
+      # 1663 rows x 2048 39 / 33 / 36, x 4096 61 / 45 / 46, x 5632 75 / 53 / 53; 1200 x 4096 58 / 41 / 37; 2048 x 2048 41 / 36 /
+      # 42; bf16 residual and norm 1663 x 2048 33 / 30 / 33, x 4096 55 / 42 / 43, 1200 x 4096 53 / 39 / 35; x 1024 lost.
+      # Not stored: the parts follow this M, a table entry would answer for its whole bucket.
+      parts = 2 if -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576) else 1
+      tiles = -(-M // 128) * (N // 256)
+      if summed and tiles <= 128 and Kd >= 2048:
+        parts = min(256 // tiles, 3)
+      if parts > 1 and not self._no_tuning():  # (the slabs are sized outside a capture)
+        scratch.splitk(x.device, parts * M * N)
+        return ("big", 4256, parts)
       return ("big", 4256, 1)
     cands = []
     if M <= STREAM_MAX_M and epi != "gelu_glu":
@@ -811,7 +820,7 @@ def linear_slabs(x: torch.Tensor, w: torch.Tensor, slot: int = 0, once: bool = T
     if x.stride(1) != 1 or x.stride(0) % 8:
       x = x.contiguous()
     y = torch.empty(x.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
-    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y", slabs=once and x.shape[0] <= WIDE_MAX_M)
+    cfg = policy.shuffled_cfg(x, w, None, None, "none", torch.float32, wave="y", slabs=once and x.shape[0] <= WIDE_MAX_M, summed=once)
     return _slab_call(x, w, None, None, "none", y, cfg, slot) if cfg[2] > 1 else _shuffled_call(x, w, None, None, "none", y, cfg)
   return linear(x, w, out_dtype=torch.float32)
 
@@ -876,7 +885,7 @@ def linear_resid_norm(x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ln_w: t
         tmp or tmp.append(h.clone())
         return run(cfg, tmp[0])
       return run(policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype, wave="solo", run=timed), h)
-    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype)
+    cfg = policy.shuffled_cfg(x, w, bias, h, "resid", h.dtype, summed=h.is_contiguous())
     if cfg[0] in ("stream", "big") and cfg[2] > 1 and (M < W4_PREF_M or h.is_contiguous()):
       S = cfg[2]
       ws = scratch.splitk(x.device, S * M * N)
