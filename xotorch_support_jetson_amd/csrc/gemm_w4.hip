@@ -95,7 +95,7 @@ template <int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {  // f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
   static_for_<0, N>(f);
 }
-constexpr int BN = 256, BK = 64;
+constexpr int BN = 256, BK = 64, CUS = 256;
 constexpr int least(int a, int b) { return a < b ? a : b; }
 constexpr int smem_bytes(int mi) { return 2 * (32 * mi + BN) * BK * 2; }  // two stage buffers (MI = 8: 128 KB)
 }  // namespace w4
@@ -128,19 +128,20 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   const int g = lane >> 4, c = lane & 15;
   const int wm = wave >> 1, wn = wave & 1;
 
-  // ---- tile: bijective XCD remap, split-major, tall grids rastered in groups of group_m row tiles (gemm_big)
+  // ---- tiles of this workgroup: blockIdx.x, + gridDim.x .. (one unless the grid is smaller than the tiles).  Bijective XCD remap,
+  // split-major, tall grids rastered in groups of group_m row tiles (gemm_big)
   const int mtiles = (M + BM - 1) / BM, ntiles = N / BN;
   const int nwg = mtiles * ntiles * S;
-  int b = blockIdx.x;
-  {
+  const int T_all = K / BK;
+  struct Tile {
+    int m0, n0, split, t_beg, T;
+  };
+  auto place = [&](int b) {
     const int xcd = b & 7, q = nwg >> 3, r = nwg & 7;
     b = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (b >> 3);
-  }
-  int mt, nt, split;
-  {
     const int tiles = mtiles * ntiles;
-    split = b / tiles;
-    const int bt = b - split * tiles;
+    const int split = b / tiles, bt = b - split * tiles;
+    int mt, nt;
     if (group_m > 1 && mtiles >= 2 * group_m) {
       const int per = group_m * ntiles, grp = bt / per, first = grp * group_m;
       const int gm = min(mtiles - first, group_m), rr = bt - grp * per;
@@ -150,28 +151,34 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
       mt = bt % mtiles;
       nt = bt / mtiles;
     }
-  }
-  const int m0 = mt * BM, n0 = nt * BN;
-  const int T_all = K / BK;
-  const int t_beg = (int)((long)split * T_all / S), t_end = (int)((long)(split + 1) * T_all / S);
-  const int T = t_end - t_beg;
+    const int t_beg = (int)((long)split * T_all / S);
+    return Tile{mt * BM, nt * BN, split, t_beg, (int)((long)(split + 1) * T_all / S) - t_beg};
+  };
 
   // ---- LDS-DMA: buffer loads with the whole address in scalar registers but for constant per-lane byte offsets
   // (9 VGPRs): the k stage goes in soffset, the LDS destination in M0 (SALU), so issuing a refill
   // costs the MFMA stream no VALU work.  (Per-issue 64-bit address arithmetic + readfirstlane for M0 -- ~70 VALU
   // per stage -- cost 20 % of the k loop: profiles/r5/gemm_w4/lab_ablation.log.)  Byte offsets are 32-bit: the
-  // launcher requires X and this tile's weight rows below 4 GB.
+  // launcher requires X and this tile's weight rows below 4 GB.  A tile's place is in the buffers' bases alone, so the lanes' offsets
+  // serve every tile of the workgroup.
   //   X image: 256 rows x 128 B, 16-B slot (lane % 8) of row r holds logical slot (lane % 8) ^ ((r >> 1) & 7) (gemm_big's
   //   BK = 64 map); instruction d < MI copies rows 8 (MI wave + d) .. +7, so the swizzle of lane's row is
-  //   ((lane >> 4) + 4 ((MI wave + d) & 1)) & 7.  Rows past M re-read the last; their outputs are masked.
+  //   ((lane >> 4) + 4 ((MI wave + d) & 1)) & 7.  Rows past M are past the buffer's end; their outputs are masked.
   //   W image: (16-row group, k32 block) 1-KB blocks in order (group * 2 + block); instruction MI + i copies block
   //   i & 1 of group 4 wave + i / 2.  PERM: lane l of a block loads granule (kq = l >> 4, row (l & 15) ^ 4 (kq & 1)).
   auto aswz = [](int row) -> int { return (row >> 1) & 7; };
   const int swave = __builtin_amdgcn_readfirstlane(wave);
-  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void*)X, (short)0, -1, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(W + (size_t)((n0 >> 4) + 4 * swave) * (K / 128) * 2048), (short)0, -1, 0x00020000);
-  int xvo[8], wvo;  // per-lane byte offsets: X per instruction (row clamp), W one for all (the rest is scalar)
+  struct Source {
+    const uint16_t *x, *w;
+    int xbytes;
+  };
+  auto source = [&](const Tile& o) {
+    if constexpr (TN) return Source{X + o.m0, W + o.n0, -1};
+    else return Source{X + (size_t)o.m0 * ldx, W + (size_t)((o.n0 >> 4) + 4 * swave) * (K / 128) * 2048, (int)((unsigned)(M - o.m0) * (unsigned)ldx * 2u)};
+  };
+  auto xbuf = [&](const Source& o) { return __builtin_amdgcn_make_buffer_rsrc((void*)o.x, (short)0, o.xbytes, 0x00020000); };
+  auto wbuf = [&](const Source& o) { return __builtin_amdgcn_make_buffer_rsrc((void*)o.w, (short)0, -1, 0x00020000); };
+  int xvo[8], wvo;  // per-lane byte offsets: X per instruction, W one for all (the rest is scalar)
   int tvo[8];       // TN: the W operand's per-instruction offsets
   // TN: instruction q = 8 wave + d of either operand copies k rows 2q, 2q + 1 of the stage (512 B each): lane l ->
   // k row 2q + l / 32, physical granule l % 32 holding logical granule (l % 32) ^ tn_swz(k row).  tn_swz puts the
@@ -181,8 +188,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
       const int kr = 2 * (8 * wave + d) + (lane >> 5), lg = (lane & 31) ^ tn_swz(kr);
-      xvo[d] = (int)(((unsigned)kr * (unsigned)ldx + (unsigned)(m0 + 8 * lg)) * 2u);
-      tvo[d] = (int)(((unsigned)kr * (unsigned)ldw + (unsigned)(n0 + 8 * lg)) * 2u);
+      xvo[d] = (int)(((unsigned)kr * (unsigned)ldx + (unsigned)(8 * lg)) * 2u);
+      tvo[d] = (int)(((unsigned)kr * (unsigned)ldw + (unsigned)(8 * lg)) * 2u);
     }
     wvo = 0;
   } else {
@@ -190,14 +197,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
 #pragma unroll
     for (int d = 0; d < MI; ++d) {
       const int slot = ((lane & 7) ^ (((lane >> 4) + 4 * ((MI * wave + d) & 1)) & 7)) * 8;
-      xvo[d] = (int)(((unsigned)min(m0 + xr0 + 8 * d, M - 1) * (unsigned)ldx + slot) * 2u);
+      xvo[d] = (int)(((unsigned)(xr0 + 8 * d) * (unsigned)ldx + slot) * 2u);
     }
     wvo = (PERM ? (((lane >> 4) * 16 + ((lane & 15) ^ (4 * ((lane >> 4) & 1)))) * 8) : lane * 8) * 2;
 #pragma unroll
     for (int d = 0; d < 8; ++d) tvo[d] = 0;
   }
-  const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc((void*)W, (short)0, -1, 0x00020000);
-  auto issue = [&](int t, int buf, int d) {  // LDS-DMA instruction d (0 .. NR - 1) of this wave for k stage t
+  // LDS-DMA instruction d (0 .. NR - 1) of this wave for k stage t of the tile whose operands xrs and wrs begin with
+  auto issue = [&](__amdgpu_buffer_rsrc_t xrs, __amdgpu_buffer_rsrc_t wrs, int t, int buf, int d) {
     typedef __attribute__((address_space(3))) void* lds_t;
     uint16_t* As = smem + buf * STAGE;
     if constexpr (TN) {
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (lds_t)(As + (8 * swave + d) * 512), 16, xvo[d], t * (BK * 2) * ldx,
                                                  0, W4_XAUX);
       else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(trs, (lds_t)(As + A_EL + (8 * swave + d - 8) * 512), 16, tvo[d - 8],
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (lds_t)(As + A_EL + (8 * swave + d - 8) * 512), 16, tvo[d - 8],
                                                  t * (BK * 2) * ldw, 0, W4_WAUX);
       return;
     }
@@ -243,10 +250,6 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   }
 
   f32x4 acc[MI][8];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   s16x8 wf[2][8], xf[2][MI];
 
   // The k loop's waits as the s_waitcnt builtin, not inline asm: the compiler's wait-count model then sees them.
@@ -372,11 +375,14 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     }
   };
 
+  Tile at = place(blockIdx.x);
+  Source src = source(at);
   {  // T >= 1 (S <= K / 64).  Prologue without branches: stage 1 (stage 0 again when T == 1) into buffer 1
+    const __amdgpu_buffer_rsrc_t xr = xbuf(src), wr = wbuf(src);
 #pragma unroll
-    for (int d = 0; d < NR; ++d) issue(t_beg, 0, d);
+    for (int d = 0; d < NR; ++d) issue(xr, wr, at.t_beg, 0, d);
 #pragma unroll
-    for (int d = 0; d < NR; ++d) issue(t_beg + min(1, T - 1), 1, d);
+    for (int d = 0; d < NR; ++d) issue(xr, wr, at.t_beg + min(1, at.T - 1), 1, d);
     wait_vm<NR>();
     bar();
 #pragma unroll
@@ -384,9 +390,24 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
       rd(0, 0, f);
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  // Tile after tile without a pause: the last two stages of one refill their buffers with the first two of the next, whose first
+  // fragments are in registers while the epilogue stores.
+  int stage = 0;  // stages behind: a buffer is a stage's parity
+  for (int b = blockIdx.x;; b += gridDim.x) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) asm volatile("v_accvgpr_write_b32 %0, 0" : "=a"(acc[i][j][r]));
+    const bool more = b + (int)gridDim.x < nwg;
+    const Tile then = more ? place(b + gridDim.x) : at;  // (nothing follows: its own stages again, which nobody reads)
+    const Source next = source(then);
+    const int T = at.T;
 
-    // one 64-deep stage.  Every stage refills and reads ahead unconditionally -- past the end stage T - 1 again,
-    // into a buffer no later stage reads -- so the k loop is straight-line code: a branch inside it made the
+    // one 64-deep stage.  Every stage refills and reads ahead unconditionally -- past the end stages of the tile that follows --
+    // so the k loop is straight-line code: a branch inside it made the
     // register allocator shuffle the 256 accumulators between AGPR quads at the join.
     // Global MFMA index v = 0 .. 2 H - 1 of a stage (half v / H, MFMA v % H).  Half 1's NR fragment reads go under the
     // first NR; after MFMA B1 - 1 every wave has them (lgkmcnt(0) + barrier) and this buffer is free; the NR refill
@@ -399,8 +420,11 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
     static_assert(B1 >= NR && B1 <= H && B2 >= 4 && B2 <= 48, "schedule positions");
     static_assert(!W4_ASMRD || RSP == 1, "the explicit read waits assume one read per MFMA");
     auto body = [&](int t) {
-      const int buf = t & 1;
-      const int tr = t_beg + min(t + 2, T - 1);
+      const int buf = (stage + t) & 1;
+      const bool own = t + 2 < T;
+      const int tr = own ? at.t_beg + t + 2 : then.t_beg + min(t + 2 - T, T - 1);
+      const Source from = own ? src : next;
+      const __amdgpu_buffer_rsrc_t xr = xbuf(from), wr = wbuf(from);
       W4_MARK(0);
       static_for<2 * H>([&](auto vc) {  // compile-time v: every condition below folds away
         constexpr int v = decltype(vc)::value;
@@ -430,7 +454,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
         if constexpr (!(W4_ABL & 1) && v >= B1 && v < H + B2) {
           static_for<NR>([&](auto kc) {  // refill DMA k after MFMA B1 + ((k + 1) SPAN) / NR - 1
             constexpr int k = decltype(kc)::value;
-            if constexpr ((DGAP ? B1 + DGAP * k : B1 + ((k + 1) * SPAN) / NR - 1) == v) issue(tr, buf, k);
+            if constexpr ((DGAP ? B1 + DGAP * k : B1 + ((k + 1) * SPAN) / NR - 1) == v) issue(xr, wr, tr, buf, k);
           });
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -453,152 +477,170 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
       __builtin_amdgcn_sched_barrier(0);
       W4_MARK(3);
     };
-    // One loop body for every stage, the last included (its read-ahead reads a re-loaded stage nobody uses): a
+    // One loop body for every stage, the last included: a
     // peeled last body got its own accumulator allocation, and the AGPR shuffle the allocator put between the loop
     // and it raced the inline-asm MFMAs it cannot see.
-    for (int t = 0; t < T; ++t) body(t);
-    wait_vm<0>();  // the last refills (re-loads of stage T - 1 nobody reads) land before the wave ends
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // ... and the last read-ahead, before registers are reused
-  }
+    // (the zeros are in their registers before the first MFMA, which the hazard recognizer does not see)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 7" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    int t = 0;
+    do body(t);
+    while (++t < T);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last read-ahead, before registers are moved or reused
 
-  // the last MFMAs (inline asm: the hazard recognizer does not see them) retire before the epilogue reads their
-  // accumulators; the scheduling barrier keeps those reads (no dependence on the nops) from moving above them
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 7\n s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
+    // the last MFMAs (inline asm: the hazard recognizer does not see them) retire before the epilogue reads their
+    // accumulators; the scheduling barrier keeps those reads (no dependence on the nops) from moving above them
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 7\n s_nop 7\n s_nop 7\n s_nop 7" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 
-  // ---- epilogue.  Lane (g, c): token row trow(i) = m0 + 16 MI wm + 16 i + c; PERM: columns 32 J + 8 g .. +8 of the
-  // wave's 128 from tiles (2J, 2J + 1); SiLU: output columns 16 J + 4 g .. +4 (gate tile 2J, up tile 2J + 1).
-  const int rbase = m0 + wm * (16 * MI) + c;
-  const int cbase = n0 + wn * 128;
-  if constexpr (SPLIT) {  // raw fp32 partial slabs, in the natural or permuted column order of the lane
-    float* slab = ws + (size_t)split * M * N;
+    // (accumulators leave their AGPRs where they are stored: left to the compiler they moved all at once, into registers that the
+    // next tile's fragments hold, and on to scratch)
+    auto sum_of = [&](int i, int j) {
+      f32x4 v;
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int m = rbase + 16 * i;
-      if (m >= M) continue;
-      float* row = slab + (size_t)m * N + cbase;
+      for (int r = 0; r < 4; ++r) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[i][j][r]));
+      return v;
+    };
+    // ---- epilogue.  Lane (g, c): token row trow(i) = m0 + 16 MI wm + 16 i + c; PERM: columns 32 J + 8 g .. +8 of the
+    // wave's 128 from tiles (2J, 2J + 1); SiLU: output columns 16 J + 4 g .. +4 (gate tile 2J, up tile 2J + 1).
+    const int rbase = at.m0 + wm * (16 * MI) + c;
+    const int cbase = at.n0 + wn * 128;
+    if constexpr (SPLIT) {  // raw fp32 partial slabs, in the natural or permuted column order of the lane
+      float* slab = ws + (size_t)at.split * M * N;
 #pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        if constexpr (PERM) {
-          *reinterpret_cast<f32x4*>(row + 32 * J + 8 * g) = acc[i][2 * J];
-          *reinterpret_cast<f32x4*>(row + 32 * J + 8 * g + 4) = acc[i][2 * J + 1];
-        } else {
-          *reinterpret_cast<f32x4*>(row + 32 * J + 4 * g) = acc[i][2 * J];
-          *reinterpret_cast<f32x4*>(row + 32 * J + 16 + 4 * g) = acc[i][2 * J + 1];
-        }
-      }
-    }
-  } else if constexpr (TN) {  // natural column order: lane (g, c) holds columns cbase + 16 j + 4 g .. +4 of token row
-    typedef short s16x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int m = rbase + 16 * i;
-      if (m >= M) continue;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int col = cbase + 16 * j + 4 * g;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r];
-        if constexpr (EPI == EPI_RESID) {
-          const s16x4_t rv = *reinterpret_cast<const s16x4_t*>(R + (size_t)m * ldr + col);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] += bf2f(rv[r]);
-        }
-        if constexpr (OUT_F32) {
-          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-          s16x4_t o;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(v[r]);
-          *reinterpret_cast<s16x4_t*>(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col) = o;
-        }
-      }
-    }
-  } else if constexpr (PERM) {
-    s16x8 bv[4];
-    if (bias != nullptr) {
-#pragma unroll
-      for (int J = 0; J < 4; ++J) bv[J] = ld16(bias + cbase + 32 * J + 8 * g);
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int m = rbase + 16 * i;
-      s16x8 rv[4];
-      if constexpr (EPI == EPI_RESID) {
-        const int mr = min(m, M - 1);
-#pragma unroll
-        for (int J = 0; J < 4; ++J) rv[J] = ld16(R + (size_t)mr * ldr + cbase + 32 * J + 8 * g);
-      }
-      if (m < M) {
+      for (int i = 0; i < MI; ++i) {
+        const int m = rbase + 16 * i;
+        if (m >= M) continue;
+        float* row = slab + (size_t)m * N + cbase;
 #pragma unroll
         for (int J = 0; J < 4; ++J) {
-          float v[8];
+          if constexpr (PERM) {
+            *reinterpret_cast<f32x4*>(row + 32 * J + 8 * g) = sum_of(i, 2 * J);
+            *reinterpret_cast<f32x4*>(row + 32 * J + 8 * g + 4) = sum_of(i, 2 * J + 1);
+          } else {
+            *reinterpret_cast<f32x4*>(row + 32 * J + 4 * g) = sum_of(i, 2 * J);
+            *reinterpret_cast<f32x4*>(row + 32 * J + 16 + 4 * g) = sum_of(i, 2 * J + 1);
+          }
+        }
+      }
+    } else if constexpr (TN) {  // natural column order: lane (g, c) holds columns cbase + 16 j + 4 g .. +4 of token row
+      typedef short s16x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int m = rbase + 16 * i;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int col = cbase + 16 * j + 4 * g;
+          f32x4 v = sum_of(i, j);
+          if constexpr (EPI == EPI_RESID) {
+            const s16x4_t rv = *reinterpret_cast<const s16x4_t*>(R + (size_t)m * ldr + col);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += bf2f(rv[r]);
+          }
+          if constexpr (OUT_F32) {
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col) = v;
+          } else {
+            s16x4_t o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(v[r]);
+            *reinterpret_cast<s16x4_t*>(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col) = o;
+          }
+        }
+      }
+    } else if constexpr (PERM) {
+      s16x8 bv[4];
+      if (bias != nullptr) {
+#pragma unroll
+        for (int J = 0; J < 4; ++J) bv[J] = ld16(bias + cbase + 32 * J + 8 * g);
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int m = rbase + 16 * i;
+        s16x8 rv[4];
+        if constexpr (EPI == EPI_RESID) {
+          const int mr = min(m, M - 1);
+#pragma unroll
+          for (int J = 0; J < 4; ++J) rv[J] = ld16(R + (size_t)mr * ldr + cbase + 32 * J + 8 * g);
+        }
+        if (m < M) {
+#pragma unroll
+          for (int J = 0; J < 4; ++J) {
+            const f32x4 lo = sum_of(i, 2 * J), hi = sum_of(i, 2 * J + 1);
+            float v[8];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              v[r] = lo[r];
+              v[4 + r] = hi[r];
+            }
+            const int col = cbase + 32 * J + 8 * g;
+            {
+              if (bias != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += bf2f(bv[J][e]);
+              }
+              if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += bf2f(rv[J][e]);
+              }
+#pragma unroll
+              for (int e = 0; e < 8; ++e) v[e] = epi_elem<EPI>(v[e]);
+              if constexpr (OUT_F32) {
+                float* p = reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col;
+                *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+                *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+              } else {
+                s16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(v[e]);
+                st16(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col, o);
+              }
+            }
+          }
+        }
+      }
+    } else {  // SiLU: natural rows, gate tile 2J / up tile 2J + 1 -> 4 output columns per lane
+      const int obase = cbase / 2;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const int m = rbase + 16 * i;
+        if (m >= M) continue;
+#pragma unroll
+        for (int J = 0; J < 4; ++J) {
+          const int gcol = cbase + 32 * J + 4 * g;  // gate rows of this lane (16-row interleaved gate / up groups)
+          const f32x4 gate = sum_of(i, 2 * J), up = sum_of(i, 2 * J + 1);
+          float o4[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            v[r] = acc[i][2 * J][r];
-            v[4 + r] = acc[i][2 * J + 1][r];
-          }
-          const int col = cbase + 32 * J + 8 * g;
-          {
+            float gv = gate[r], uv = up[r];
             if (bias != nullptr) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) v[e] += bf2f(bv[J][e]);
+              gv += bf2f(bias[gcol + r]);
+              uv += bf2f(bias[gcol + 16 + r]);
             }
-            if constexpr (EPI == EPI_RESID) {
+            o4[r] = glu_pair<EPI>(gv, uv, epi_arg);
+          }
+          const int col = obase + 16 * J + 4 * g;
+          if constexpr (OUT_F32) {
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col) =
+                f32x4{o4[0], o4[1], o4[2], o4[3]};
+          } else {
+            typedef short s16x4_t __attribute__((ext_vector_type(4)));
+            s16x4_t o;
 #pragma unroll
-              for (int e = 0; e < 8; ++e) v[e] += bf2f(rv[J][e]);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = epi_elem<EPI>(v[e]);
-            if constexpr (OUT_F32) {
-              float* p = reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col;
-              *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
-              *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
-            } else {
-              s16x8 o;
-#pragma unroll
-              for (int e = 0; e < 8; ++e) o[e] = (short)f2bf(v[e]);
-              st16(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col, o);
-            }
+            for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(o4[r]);
+            *reinterpret_cast<s16x4_t*>(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col) = o;
           }
         }
       }
     }
-  } else {  // SiLU: natural rows, gate tile 2J / up tile 2J + 1 -> 4 output columns per lane
-    const int obase = cbase / 2;
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int m = rbase + 16 * i;
-      if (m >= M) continue;
-#pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        const int gcol = cbase + 32 * J + 4 * g;  // gate rows of this lane (16-row interleaved gate / up groups)
-        float o4[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float gv = acc[i][2 * J][r], uv = acc[i][2 * J + 1][r];
-          if (bias != nullptr) {
-            gv += bf2f(bias[gcol + r]);
-            uv += bf2f(bias[gcol + 16 + r]);
-          }
-          o4[r] = glu_pair<EPI>(gv, uv, epi_arg);
-        }
-        const int col = obase + 16 * J + 4 * g;
-        if constexpr (OUT_F32) {
-          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Yv) + (size_t)m * ldy + col) =
-              f32x4{o4[0], o4[1], o4[2], o4[3]};
-        } else {
-          typedef short s16x4_t __attribute__((ext_vector_type(4)));
-          s16x4_t o;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = (short)f2bf(o4[r]);
-          *reinterpret_cast<s16x4_t*>(reinterpret_cast<uint16_t*>(Yv) + (size_t)m * ldy + col) = o;
-        }
-      }
-    }
+    if (!more) break;
+    stage += T;
+    at = then;
+    src = next;
   }
+  wait_vm<0>();  // the last refills land before the wave ends
 }
 
 template <int EPI, bool F32, bool SPLIT, int MI>
@@ -611,7 +653,11 @@ static void w4_launch_rows(const uint16_t* X, int ldx, const uint16_t* W, const 
       hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) == hipSuccess;
   (void)attr;
   const int nwg = ((M + 32 * MI - 1) / (32 * MI)) * (N / 256) * S;
-  kern<<<nwg, 256, SMEM, st>>>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, 0, epi_arg);
+  // From three rounds of tiles a CU on, one workgroup a CU takes tile after tile: a tile's first stages arrive under the last ones and the
+  // epilogue of the one before (SiLU gate / up of 28672 x 4096, 2313 rows 456 -> 446 us, 1999 rows 369 -> 361; bit for bit the same).
+  // With fewer rounds the dispatcher's order is kept: it lets a weight gradient on a side stream have the CUs between tiles (a training
+  // step with 448 tiles in turn too 26.1 -> 26.4 ms).
+  kern<<<SPLIT || nwg < 3 * w4::CUS ? nwg : w4::CUS, 256, SMEM, st>>>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, 0, epi_arg);
 }
 
 template <int EPI, bool F32, bool SPLIT>
