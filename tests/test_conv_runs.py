@@ -35,6 +35,25 @@ def test_units(head, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("head", [1, 7, 64, 66, 126, 128, 130, 256])
+@pytest.mark.parametrize("off", [0, 1, 2])
+@pytest.mark.parametrize("taps,lens", [(4, [5, 1, 37]), (2, [1030, 0, 9]), (1, [33])])
+def test_whole_rows_as_two_slabs(head, off, taps, lens):
+  """Rows loaded without a branch (whole vectors, unsplit) and any others: the same numbers as the sum of the rows and of nothing."""
+  C, T, B = 3 * head, sum(lens), len(lens)
+  units, width = R.conv_units([(head, R.CONV_SILU | R.CONV_UNIT), (head, R.CONV_SILU), (head, 0)], C)
+  g = torch.Generator(device="cuda").manual_seed(head + off)
+  rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+  P, w, state = rn(T, C + 4), rn(C, taps), rn(B, taps - 1, C)
+  cu, slots, got = torch.tensor([0] + lens).cumsum(0).int().cuda(), torch.arange(B, dtype=torch.int32, device="cuda"), []
+  for rows in (P, torch.stack([P, torch.zeros_like(P)])):
+    S, out = state.clone(), torch.full((T, C), float("nan"), device="cuda")
+    K.conv_prep(rows, off, w, None, units.cuda(), None, S, slots, cu, 1e-5, out, max(lens), width)
+    got.append((out, S))
+  assert all(torch.equal(a, b) for a, b in zip(*got)) and not got[0][0].isnan().any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("runs", [True, False])
 def test_silu_of_any_input(runs):
   """SiLU where e^-x leaves the range of a float: -0 or 0 for finite inputs, however large, and infinities and no numbers as a
