@@ -5,6 +5,7 @@ import torch
 from xotorch_support_jetson_amd.ops import kernels as K
 from xotorch_support_jetson_amd.ops import linear as L
 from xotorch_support_jetson_amd.ops._ext import require
+from xotorch_support_jetson_amd.train import autograd_ops as A
 
 
 def product(x, w, epi, dtype, bias=None, residual=None, arg=0.0):
@@ -37,3 +38,22 @@ def test_rows_of_many_tiles_as_rows_of_few(gpu, epi, dtype, tall, Kd, pad):
     want = x[-70:].float() @ w.float().T + (bias.float() if bias is not None else res[-70:].float())
     tol = 2 ** -8 if dtype == torch.bfloat16 else 1e-5  # the result's rounding; sums of up to 384 products of size one in fp32
     torch.testing.assert_close(out[-70:].float(), want, rtol=tol, atol=1e-5 * Kd ** 0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [64, 128, 192, 320])  # one stage a tile (a workgroup each), two, and odd numbers: the buffers change places
+@pytest.mark.parametrize("M,N", [(8192, 6400), (7680, 6656)])  # 800 and 780 tiles
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_weight_gradients_of_many_tiles(gpu, tokens, M, N, accumulate):
+  g = torch.Generator(device=gpu).manual_seed(tokens + M)
+  dy, x = (torch.randn(tokens, n, device=gpu, generator=g).to(torch.bfloat16) for n in (M, N))
+  start = torch.randn(M, N, device=gpu, generator=g).to(torch.bfloat16)
+  for _ in range(2):
+    out = start.clone()
+    assert A.dw_tn(dy, x, out, accumulate)
+    for a in range(0, M, 1536):  # (fewer tiles: a workgroup each)
+      b = min(M, a + 1536)
+      part = start[a:b].clone()
+      assert A.dw_tn(dy[:, a:b], x, part, accumulate) and torch.equal(out[a:b], part), a
+  want = dy[:, -300:].float().T @ x.float() + (start[-300:].float() if accumulate else 0)
+  torch.testing.assert_close(out[-300:].float(), want, rtol=2 ** -8, atol=1e-5 * tokens ** 0.5)  # (the result's rounding; fp32 sums)
