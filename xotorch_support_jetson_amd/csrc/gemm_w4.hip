@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   // serve every tile of the workgroup.
   //   X image: 256 rows x 128 B, 16-B slot (lane % 8) of row r holds logical slot (lane % 8) ^ ((r >> 1) & 7) (gemm_big's
   //   BK = 64 map); instruction d < MI copies rows 8 (MI wave + d) .. +7, so the swizzle of lane's row is
-  //   ((lane >> 4) + 4 ((MI wave + d) & 1)) & 7.  Rows past M are past the buffer's end; their outputs are masked.
+  //   ((lane >> 4) + 4 ((MI wave + d) & 1)) & 7.  The buffer ends with the last element of row M - 1, whatever the row stride
+  //   (rows may repeat, ldx 0, or overlap); rows past M give zeros, or what such rows hold, and their outputs are masked.
   //   W image: (16-row group, k32 block) 1-KB blocks in order (group * 2 + block); instruction MI + i copies block
   //   i & 1 of group 4 wave + i / 2.  PERM: lane l of a block loads granule (kq = l >> 4, row (l & 15) ^ 4 (kq & 1)).
   auto aswz = [](int row) -> int { return (row >> 1) & 7; };
@@ -174,7 +175,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w4_kernel(const uint16_t* __restr
   };
   auto source = [&](const Tile& o) {
     if constexpr (TN) return Source{X + o.m0, W + o.n0, -1};
-    else return Source{X + (size_t)o.m0 * ldx, W + (size_t)((o.n0 >> 4) + 4 * swave) * (K / 128) * 2048, (int)((unsigned)(M - o.m0) * (unsigned)ldx * 2u)};
+    else return Source{X + (size_t)o.m0 * ldx, W + (size_t)((o.n0 >> 4) + 4 * swave) * (K / 128) * 2048,
+                       (int)(((unsigned)(M - 1 - o.m0) * (unsigned)ldx + (unsigned)K) * 2u)};
   };
   auto xbuf = [&](const Source& o) { return __builtin_amdgcn_make_buffer_rsrc((void*)o.x, (short)0, o.xbytes, 0x00020000); };
   auto wbuf = [&](const Source& o) { return __builtin_amdgcn_make_buffer_rsrc((void*)o.w, (short)0, -1, 0x00020000); };
@@ -737,7 +739,7 @@ int launch_gemm_w4(const uint16_t* X, int ldx, const uint16_t* W, const uint16_t
                    float epi_arg, hipStream_t st) {
   if (M <= 0) return 0;
   if (N % 256 != 0 || K % 128 != 0 || S < 1 || S > K / 64) return -1;
-  if ((size_t)M * ldx * 2 >= (1ull << 32)) return -1;  // 32-bit byte offsets of the LDS-DMA buffer loads
+  if (((size_t)(M - 1) * ldx + (ldx > K ? ldx : K)) * 2 >= (1ull << 32)) return -1;  // 32-bit byte offsets of the LDS-DMA buffer loads
   if (rows != 0 && (rows % 32 != 0 || rows < 128 || rows > 256)) return -1;
   const int mi = rows ? rows / 32 : gemm_w4_mi(M, N, S);
   if (S > 1) {
