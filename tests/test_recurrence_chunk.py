@@ -245,3 +245,42 @@ def test_a_value_that_is_no_number_reaches_no_earlier_token(gpu, rule, value, wh
   diff = torch.where(number, got[:lens[0]].to(F64) - want, torch.zeros((), dtype=F64)).abs().max()
   assert diff < 1e-5 * want[number].abs().max()
   assert not torch.isfinite(got[:lens[0]][~number]).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule,d,H,G,dv,lens", [("channel_delta", 128, 16, 16, 40, (9000, 3, 40, 7001, 4001)),  # 27 KB a chunk and head
+                                               ("channel", 64, 32, 32, 33, (1, 9, 12100, 12001, 0, 3000)),
+                                               ("delta", 64, 64, 2, 8, (31, 50000, 800, 17, 14003)), ("head", 64, 64, 1, 8, (70001,))])
+def test_long_steps_go_in_portions_of_the_workspace(gpu, rule, d, H, G, dv, lens):
+  """A step whose chunks' records are more than 512 MB, in portions of every sequence and (delta; the longest not known) of the slots: no
+  more memory than that, and bit for bit the numbers of its sequences alone, token by token within the forms' bound."""
+  channel, delta, _, _ = RULES[rule]
+  T, B = sum(lens), len(lens)
+  g = torch.Generator(device=gpu).manual_seed(T)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  q, k, v = rn(T, G * d) / d ** 0.5, rn(T, G * d) / d ** 0.5, rn(T, H * dv)
+  a, beta = torch.sigmoid(3 + rn(T, H * (d if channel else 1))), torch.sigmoid(rn(T, H)) if delta else None
+  state, starts = rn(B, H, dv, d), torch.tensor([0, *lens]).cumsum(0).tolist()
+
+  def run(b0, b1, longest):
+    t0, t1 = starts[b0], starts[b1]
+    S, out = state[b0:b1].clone(), torch.full((t1 - t0, H * dv), 7.0, device=gpu)
+    cu = torch.tensor([x - t0 for x in starts[b0:b1 + 1]], dtype=torch.int32, device=gpu)
+    slots = torch.arange(b1 - b0, dtype=torch.int32, device=gpu)
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    K.linear_recurrence(q[t0:t1], k[t0:t1], v[t0:t1], a[t0:t1], None if beta is None else beta[t0:t1], 0.7, S, slots, cu, out, max_qlen=longest)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - held <= (512 << 20) + (2 << 20)  # (blocks of 2 MB)
+    return out, S
+  out, S = run(0, B, max(lens))
+  assert not out.isnan().any()
+  for said in (0, T + 1):
+    assert all(torch.equal(x, y) for x, y in zip((out, S), run(0, B, said)))
+  for b in range(B):
+    if lens[b] >= 96:  # (shorter ones alone go token by token)
+      one, last = run(b, b + 1, lens[b])
+      assert torch.equal(out[starts[b]:starts[b + 1]], one) and torch.equal(S[b], last[0]), lens[b]
+  for got, want in zip((out, S), run(0, B, 1)):  # (both within 1e-6 of float64, test_chunks_match_token_by_token)
+    assert ((got - want).norm() / want.norm()) < 2e-6

@@ -1356,11 +1356,11 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const float* bp = beta.has_value() ? beta->data_ptr<float>() : nullptr;
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
   if (chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, per_channel, max_qlen) && (!per_channel || rows16(decay, 0))) {
-    auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta)}, q.options());
+    auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta, std::min(max_qlen, T))}, q.options());
     chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, ldk, ldv,
                       fixed ? 0 : (int)H, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(),
-                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? max_qlen : T / B),
-                      per_channel, delta, ws.data_ptr<float>(), out.data_ptr<float>(), DecaySource{}});
+                      (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? std::min(max_qlen, T) : T / B),
+                      max_qlen > 0, per_channel, delta, ws.data_ptr<float>(), out.data_ptr<float>(), DecaySource{}});
     return;
   }
   int DP = 16;
@@ -1421,10 +1421,10 @@ bool linear_recurrence_made(const at::Tensor& q, const at::Tensor& k, const at::
     if (w.size(1) % 16 != 0 || !rows16(P, ldp) || p_off % 4 != 0) return false;
   }
   if (!chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, true, max_qlen) || !rows16(w, ldw) || !rows16(b, 0)) return false;
-  auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, true, delta)}, q.options());
+  auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, true, delta, std::min(max_qlen, T))}, q.options());
   chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), nullptr, nullptr, ldq, ldk, ldv, 0, (float)q_scale,
                     state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(), (int)T, (int)B, (int)H, (int)G, (int)d,
-                    (int)dv, (int)dv, (int)(max_qlen > 0 ? max_qlen : T / B), true, delta, ws.data_ptr<float>(), out.data_ptr<float>(),
+                    (int)dv, (int)dv, (int)(max_qlen > 0 ? std::min(max_qlen, T) : T / B), max_qlen > 0, true, delta, ws.data_ptr<float>(), out.data_ptr<float>(),
                     {P.data_ptr<float>(), ldp, (int)p_off, w.data_ptr<float>(), b.data_ptr<float>(), ldw, (float)(1.0 / tau),
                      delta ? A_log->data_ptr<float>() : nullptr}});
   return true;

@@ -22,7 +22,8 @@ struct ChunkRecurrence {
   float q_scale;
   float* state;
   const int *state_slots, *cu_q;
-  int T, B, H, G, d, dv, dvin, longest;  // longest: tokens of the longest sequence, or what is taken for it
+  int T, B, H, G, d, dv, dvin, longest;  // longest: tokens of the longest sequence, or (not known) what is taken for it
+  bool known;
   bool chan, delta;  // a decay per key channel; the delta rule
   float *ws, *out;
   DecaySource src;  // (P null: decay and beta hold them)
@@ -30,6 +31,6 @@ struct ChunkRecurrence {
 
 // takes d 64 or 128, rows of q, k, the decays (chan) and the state on 16-byte boundaries
 void chunk_recurrence(const ChunkRecurrence& a);
-int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta);  // floats
+int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta, int64_t max_qlen);  // floats, at most 128 M
 
 }  // namespace xot

@@ -41,6 +41,26 @@ constexpr float FAR = 1.2676506e30f;            // 2^100
 // workspace floats of a (chunk, head): with channel decays the scan's operands follow, the decay over the chunk (D), then P Q, (G K)^T
 // and (delta rule) P K by state tile and lane
 constexpr int rec_floats(int D, bool chan, bool delta) { return MN + (chan ? D + (delta ? 3 : 2) * CT * D : 0); }
+constexpr int64_t WS_MOST = 128 << 20;          // workspace floats (Portions)
+
+// A record is 2.2 KB a chunk and head, with channel decays up to 27 KB (key dims of 128 under the delta rule: 3.3 times the decays that
+// it replaces).  Steps whose records fit 512 MB (19.7 thousand tokens of 16 such heads) go at once, longer ones in portions, each with as
+// many chunks of every sequence, so that the sequences go on side by side.  Where the lengths are unlike enough to double the portions,
+// a portion would be fewer than 64 chunks of each or the longest is not known, portions are slots as they come.  The same heads, us at once
+// / in portions / as slots come: three of 9000 tokens 977 / 1008 / 1415, of 20000 2145 / 2222 / 3475, six of 8000 1556 / 1619 / 2054;
+// 64 of 512, which go as slots come, 904 / - / 950.
+struct Portions {
+  int count, slots, each;  // slots of the workspace; each: chunks of a sequence in a portion, or 0
+};
+Portions portions(int64_t T, int64_t B, int64_t H, int rec, int64_t longest) {
+  const int64_t slots = T / CT + B, most = std::max<int64_t>(WS_MOST / (H * rec), 1), parts = (slots + most - 1) / most;
+  const int64_t each = most / B, chunks = (longest + CT - 1) / CT;
+  if (parts > 1 && longest > 0 && each >= 64 && chunks <= 2 * parts * each) {
+    const int64_t turns = (chunks + each - 1) / each, even = (chunks + turns - 1) / turns;
+    return {(int)turns, (int)(B * even), (int)even};
+  }
+  return {(int)parts, (int)((slots + parts - 1) / parts), 0};
+}
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -85,19 +105,26 @@ __global__ __launch_bounds__(64, CHAN ? 3 : 2) void chunk_prep_k(const float* __
                                                    const float* __restrict__ decay, int dstride,
                                                    const float* __restrict__ beta, float q_scale,
                                                    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B,
-                                                   int H, int G, int heads, DecaySource src, float* __restrict__ ws) {
+                                                   int H, int G, int heads, DecaySource src, int from, int each,
+                                                   float* __restrict__ ws) {
   __shared__ float sA[CT][CT + 1];
   __shared__ __attribute__((aligned(16))) float sT[CHAN ? 2 : 1][CHAN ? CT : 1][CT + 4];  // a tile's way from dims to tokens
   constexpr bool SHARE = !CHAN && !DELTA;
   const int per = SHARE ? H / heads : H;  // workgroups a chunk, neighbours: they read and write whole rows together (channel
                                          // decays made, 4593 tokens x 16 heads of 128 100 -> 91 us; delta rule, 12807 48 -> 44)
-  const int s = blockIdx.x / per, h = blockIdx.x % per * (SHARE ? heads : 1), lane = threadIdx.x, i = lane & 15, g = lane >> 4;
-  int lo = 0, hi = B - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (slot_base(cu_q, mid) <= s) lo = mid; else hi = mid - 1;
+  const int s = (int)(blockIdx.x / per), h = blockIdx.x % per * (SHARE ? heads : 1), lane = threadIdx.x, i = lane & 15, g = lane >> 4;
+  int lo = 0, hi = B - 1, c;
+  if (each) {
+    lo = s / each;
+    c = from + s % each;
+  } else {
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (slot_base(cu_q, mid) <= from + s) lo = mid; else hi = mid - 1;
+    }
+    c = from + s - slot_base(cu_q, lo);
   }
-  const int t0 = cu_q[lo], n = cu_q[lo + 1] - t0, c = s - slot_base(cu_q, lo);
+  const int t0 = cu_q[lo], n = cu_q[lo + 1] - t0;
   if (state_slots[lo] < 0 || c * CT >= n) return;
   const int tok = c * CT + i;
   const bool valid = tok < n;
@@ -300,12 +327,15 @@ __device__ __forceinline__ int scan_order(int turn, int B, int per) {
   return turn >= first ? B - 1 - (turn - first) : turn < second ? first - second + turn : turn - second;
 }
 
-// CG groups of 16 value channels a workgroup, KP waves each: wave (kp, cg) has key dims kp D / KP .. of group cg.
+// CG groups of 16 value channels a workgroup, KP waves each: wave (kp, cg) has key dims kp D / KP .. of group cg.  Of every sequence
+// the chunks whose records the workspace holds (Portions): `each` from its chunk `from` on, or those in `slots` slots from slot `from` of
+// the step; between portions the state is in its place in memory.
 template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
 __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ inscale, float q_scale, float* __restrict__ state, const int* __restrict__ state_slots,
-    const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, const float* __restrict__ ws, float* __restrict__ out) {
+    const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, int from, int slots, int each, const float* __restrict__ ws,
+    float* __restrict__ out) {
   static_assert(KP == 2 || KP == 4, "the order of the sums is that of quarters of the key dims");
   constexpr int TILES = D / 16 / KP;              // 16-row state tiles of a wave
   constexpr int QW = 4 / KP, QT = TILES / QW;     // quarters of the key dims in a wave, tiles of each
@@ -321,7 +351,9 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
   const int h = blockIdx.x;
   const int b = nth_longest(B, scan_order((int)blockIdx.z, B, H * (int)gridDim.y), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
-  const int t0 = cu_q[b], n = cu_q[b + 1] - t0;
+  const int base = slot_base(cu_q, b) - from;  // the sequence's first slot in the portion, or (negative) before it
+  const int c0 = each ? from : max(-base, 0), first = each ? b * each : base + c0;
+  const int t0 = cu_q[b] + CT * c0, n = min(cu_q[b + 1] - t0, CT * (each ? each : slots - first));
   if (slot < 0 || n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cg = wave % CG, kp = wave / CG;
@@ -333,7 +365,7 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
   f32x4 S[TILES];
 #pragma unroll
   for (int j = 0; j < TILES; ++j) S[j] = *reinterpret_cast<const f32x4*>(St + 16 * j);
-  const float* W = ws + ((int64_t)slot_base(cu_q, b) * H + h) * REC;
+  const float* W = ws + ((int64_t)first * H + h) * REC;
   const int64_t wstep = (int64_t)H * REC;
 
   // What a chunk is made of, two chunks ahead in registers: q, k (channel decays: P Q, P K from the workspace) as A operands of the
@@ -602,23 +634,23 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
 }
 
 template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
-void scan(const ChunkRecurrence& a) {
+void scan(const ChunkRecurrence& a, int from, int slots, int each) {
   const dim3 grid((unsigned)a.H, (unsigned)((a.dv + 16 * CG - 1) / (16 * CG)), (unsigned)a.B);
   chunk_scan_k<D, CHAN, DELTA, KP, CG, WPE, RING><<<grid, 64 * KP * CG, 0, stream()>>>(
       a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, DELTA ? nullptr : a.beta, a.q_scale, a.state, a.state_slots, a.cu_q, a.B, a.H, a.G, a.dv,
-      a.dvin, a.ws, a.out);
+      a.dvin, from, slots, each, a.ws, a.out);
 }
 
+// a portion
 template <int D, bool CHAN, bool DELTA>
-void go(const ChunkRecurrence& a) {
-  const int slots = a.T / CT + a.B;
+void go(const ChunkRecurrence& a, int from, int slots, int each) {
   // plain write, a decay per head: the heads of a q / k head share its products where that leaves enough waves (32 heads on 8, with the
   // scan: 5 of 364 .. 1728 tokens 110 -> 100 us, 8 of 961 .. 2433 247 -> 223; three of 1000 not; two heads under the delta rule gave nothing)
   const int heads = !CHAN && !DELTA && (int64_t)slots * a.G >= 2048 ? a.H / a.G : 1;
   const unsigned pg = (unsigned)slots * (unsigned)(a.H / heads);
   auto prep = [&](auto kern) {
     kern<<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale, a.state_slots, a.cu_q, a.B, a.H, a.G,
-                                  heads, a.src, a.ws);
+                                  heads, a.src, from, each, a.ws);
   };
   if constexpr (CHAN) {
     if (a.src.P != nullptr) prep(chunk_prep_k<D, CHAN, DELTA, true>);
@@ -632,15 +664,23 @@ void go(const ChunkRecurrence& a) {
   // quarters / halves, delta rule 16 heads of 128 x 128: 0.25 (one of 2000) 130 / 167, 0.5 77 / 93, 0.66 (5 of 364 .. 1728) 149 / 164,
   // 0.75 (three of 1000) 111 / 98, 1.3 (8 of 961 .. 2433) 332 / 298.
   const int64_t per = (int64_t)a.H * ((a.dv + 31) / 32);
-  if (a.T * per < 180 * (int64_t)a.longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a);
-  else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a);
-  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a);  // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us)
+  const int64_t tokens = std::min<int64_t>(a.T, (int64_t)CT * slots), longest = std::min<int64_t>(a.longest, (int64_t)CT * (each ? each : slots));
+  if (tokens * per < 180 * longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a, from, slots, each);
+  else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a, from, slots, each);
+  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a, from, slots, each);  // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us)
+}
+
+template <int D, bool CHAN, bool DELTA>
+void go(const ChunkRecurrence& a) {
+  const Portions p = portions(a.T, a.B, a.H, rec_floats(D, CHAN, DELTA), a.known ? a.longest : 0);
+  for (int turn = 0; turn < p.count; ++turn) go<D, CHAN, DELTA>(a, turn * (p.each ? p.each : p.slots), p.slots, p.each);
 }
 
 }  // namespace
 
-int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta) {
-  return (T / CT + B) * H * rec_floats((int)d, chan, delta);
+int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta, int64_t max_qlen) {
+  const int rec = rec_floats((int)d, chan, delta);
+  return portions(T, B, H, rec, max_qlen).slots * H * rec;
 }
 
 void chunk_recurrence(const ChunkRecurrence& a) {
