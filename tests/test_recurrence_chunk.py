@@ -167,13 +167,22 @@ def test_decays_and_write_strengths_from_finished_products(gpu, d, G):
   assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
 
 
+ALL, SCALAR, DELTA, NONE = {"delta", "channel_delta", "channel", "scaled"}, {"delta", "scaled"}, {"delta"}, set()
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("rule", ["delta", "channel_delta", "channel", "scaled"])
-@pytest.mark.parametrize("B,dv,longest", [(1, 64, 47), (1, 64, 48), (3, 64, 63), (3, 64, 64), (32, 128, 31), (32, 128, 32), (31, 128, 32)])
-def test_both_sides_of_the_chunk_rule(gpu, rule, B, dv, longest):
-  """The lengths from which steps go by chunks (mixers.hip chunks_take), against the same step token by token (longest taken as 1)."""
+@pytest.mark.parametrize("rule", sorted(ALL))
+@pytest.mark.parametrize("B,dv,longest,chunks", [
+  (1, 64, 47, NONE), (1, 64, 48, SCALAR), (3, 64, 63, SCALAR), (3, 64, 64, ALL),  # few sequences
+  (32, 128, 31, NONE), (32, 128, 32, ALL), (31, 128, 32, NONE), (64, 128, -32, ALL),  # the CUs filled twice over, four times
+  (65, 128, -32, DELTA), (65, 128, -47, DELTA), (65, 128, -48, ALL), (128, 128, -48, ALL),  # (minus: behind single tokens)
+  (129, 128, -48, DELTA), (129, 128, -95, DELTA), (129, 128, -96, ALL), (129, 128, 35, ALL), (129, 128, 31, NONE)])
+def test_both_sides_of_the_chunk_rule(gpu, rule, B, dv, longest, chunks):
+  """The lengths from which steps go by chunks (mixers.hip chunks_take), against the same step token by token (longest taken as 1): the
+  same numbers to the bit where the rule leaves it at that, sums in another order where it does not."""
   channel, delta, scaled, _ = RULES[rule]
-  H, d, lens = 16, 64, [max(1, longest - 5 * b % longest) for b in range(B)]
+  lens = [1] * (B - 1) + [-longest] if longest < 0 else [max(1, longest - 5 * b % longest) for b in range(B)]
+  H, d, longest = 16, 64, max(lens)
   T, g = sum(lens), torch.Generator(device=gpu).manual_seed(B + longest)
   rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
   q, k, v, a = rn(T, H * d) / 8, rn(T, H * d) / 8, rn(T, H * dv), torch.sigmoid(3 + rn(T, H * (d if channel else 1)))
@@ -184,7 +193,7 @@ def test_both_sides_of_the_chunk_rule(gpu, rule, B, dv, longest):
     K.linear_recurrence(q, k, v, a, beta, 0.7, S, slots, cu, out, plain=scaled, max_qlen=said)
     got.append((out, S))
   for one, other in zip(*got):  # (both are within 1e-6 of float64, test_chunks_match_token_by_token; a single value within some times that)
-    assert ((one - other).norm() / one.norm()) < 2e-6
+    assert ((one - other).norm() / one.norm()) < 2e-6 and torch.equal(one, other) == (rule not in chunks)
     torch.testing.assert_close(one, other, rtol=0, atol=float(4e-6 * one.abs().max()))
 
 
