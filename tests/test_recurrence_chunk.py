@@ -293,3 +293,24 @@ def test_long_steps_go_in_portions_of_the_workspace(gpu, rule, d, H, G, dv, lens
       assert torch.equal(out[starts[b]:starts[b + 1]], one) and torch.equal(S[b], last[0]), lens[b]
   for got, want in zip((out, S), run(0, B, 1)):  # (both within 1e-6 of float64, test_chunks_match_token_by_token)
     assert ((got - want).norm() / want.norm()) < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule", list(RULES))
+@pytest.mark.parametrize("ld", [0, 4, 64])  # one row for all tokens, rows that overlap, rows whose heads lie in the next ones
+def test_rows_that_repeat_or_overlap(gpu, rule, ld):
+  """q, k and v of fewer floats a token than their heads hold: as the same rows one behind the other."""
+  channel, delta, scaled, norm = RULES[rule]
+  H, d, dv, lens = 4, 64, 40, [101, 17, 50]
+  T, B = sum(lens), len(lens)
+  g = torch.Generator(device=gpu).manual_seed(ld)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  q, k, v = ((rn(T * ld + H * n) / n ** 0.5).as_strided((T, H * n), (ld, 1)) for n in (d, d, dv))
+  a, beta = torch.sigmoid(3 + rn(T, H * (d if channel else 1))), torch.sigmoid(rn(T, H)) if delta or scaled else None
+  state, cu = rn(B, H, dv + norm, d), torch.tensor([0, *lens]).cumsum(0).int().to(gpu)
+  slots, got = torch.arange(B, dtype=torch.int32, device=gpu), []
+  for x in ((q, k, v), tuple(t.contiguous() for t in (q, k, v))):
+    S, out = state.clone(), torch.full((T, H * (dv + norm)), 7.0, device=gpu)
+    K.linear_recurrence(*x, a, beta, 0.7, S, slots, cu, out, plain=scaled and not norm, max_qlen=max(lens))
+    got.append((out, S))
+  assert all(torch.equal(one, other) for one, other in zip(*got))

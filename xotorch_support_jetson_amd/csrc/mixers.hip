@@ -1363,7 +1363,9 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
   if (chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, delta, per_channel, max_qlen) && (!per_channel || rows16(decay, 0))) {
     auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta, std::min(max_qlen, T))}, q.options());
-    chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, ldk, ldv,
+    // (rows past a sequence's end are zeros because they are behind its last one: rows of k closer than a head is wide are not)
+    const at::Tensor kr = ldk < d ? k.contiguous() : k;
+    chunk_recurrence({q.data_ptr<float>(), kr.data_ptr<float>(), v.data_ptr<float>(), decay.data_ptr<float>(), bp, ldq, (int)kr.stride(0), ldv,
                       fixed ? 0 : (int)H, (float)q_scale, state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(),
                       (int)T, (int)B, (int)H, (int)G, (int)d, (int)dv, (int)dvin, (int)(max_qlen > 0 ? std::min(max_qlen, T) : T / B),
                       max_qlen > 0, per_channel, delta, ws.data_ptr<float>(), out.data_ptr<float>(), DecaySource{}});
