@@ -41,7 +41,8 @@ def test_rows_of_many_tiles_as_rows_of_few(gpu, epi, dtype, tall, Kd, pad):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [64, 128, 192, 320])  # one stage a tile (a workgroup each), two, and odd numbers: the buffers change places
+@pytest.mark.parametrize("tokens", [64, 128, 192, 320, 2560, 2624])  # one stage a tile (a workgroup each), two, and odd numbers: the
+# buffers change places; the most of tile after tile, and more
 @pytest.mark.parametrize("M,N", [(8192, 6400), (7680, 6656)])  # 800 and 780 tiles
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_weight_gradients_of_many_tiles(gpu, tokens, M, N, accumulate):

@@ -656,7 +656,8 @@ static void w4_launch_rows(const uint16_t* X, int ldx, const uint16_t* W, const 
   (void)attr;
   const int nwg = ((M + 32 * MI - 1) / (32 * MI)) * (N / 256) * S;
   // From three rounds of tiles a CU on, one workgroup a CU takes tile after tile: a tile's first stages arrive under the last ones and the
-  // epilogue of the one before (SiLU gate / up of 28672 x 4096, 2313 rows 456 -> 446 us, 1999 rows 369 -> 361; bit for bit the same).
+  // epilogue of the one before (SiLU gate / up of 28672 x 4096, 2313 rows 456 -> 446 us, 1999 rows 369 -> 361, 8192 rows 1361 -> 1348, 12807 x
+  // 22528 x 2048 959 -> 932; of K 8192 and more within 1 % either way; bit for bit the same).
   // With fewer rounds the dispatcher's order is kept: it lets a weight gradient on a side stream have the CUs between tiles (a training
   // step with 448 tiles in turn too 26.1 -> 26.4 ms).
   kern<<<SPLIT || nwg < 3 * w4::CUS ? nwg : w4::CUS, 256, SMEM, st>>>(X, ldx, W, bias, R, ldr, Y, ldy, ws, M, N, K, S, group_m, 0, epi_arg);
@@ -685,11 +686,14 @@ static void w4_tn_launch(const uint16_t* Xt, int ldx, const uint16_t* Wt, int ld
   static bool attr =
       hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, w4::smem_bytes(8)) == hipSuccess;
   (void)attr;
-  // Tile after tile as above, from two stages a tile on (a tile's last two refills are the next one's first two).  A training step of
-  // 2 x 1024 tokens, whose weight gradients run beside the input gradients: 1.003, 1.008 and 1.002 x the rate of a workgroup a tile, 0.998 x
-  // with the input gradients' side alone.
+  // Tile after tile as above, from two stages a tile on (a tile's last two refills are the next one's first two) up to 2560 tokens, beyond
+  // which a tile's fixed cost is small and the workgroups, no longer dealt out as they end, drift apart.  us a workgroup a tile /
+  // so: 28672 x 4096 of 256 tokens 118 / 102, 512 158 / 146, 1024 237 / 227, 2048 396 / 390, 2560 489 / 474, 3072 578 / 580, 4096 745 / 760,
+  // 8192 1476 / 1520; 57344 x 8192 of 512 655 / 578, 2048 1611 / 1615, 4096 2960 / 3140; 4096 x 14336 of 2048 221 / 216; 128256 x 4096 of 2048
+  // 1883 / 1823.  A training step of 2 x 1024 tokens, whose weight gradients run beside the input gradients, 25.1 / 24.7 ms (1.010 to 1.021 x
+  // in four measurements, of which each side's own runs differ by 2 to 5 %).
   const int nwg = (M / 256) * (N / 256);
-  kern<<<nwg < 3 * w4::CUS || K < 128 ? nwg : w4::CUS, 256, w4::smem_bytes(8), st>>>(Xt, ldx, Wt, nullptr, R, ldr, Y, ldy, nullptr, M, N, K, 1,
+  kern<<<nwg < 3 * w4::CUS || K < 128 || K > 2560 ? nwg : w4::CUS, 256, w4::smem_bytes(8), st>>>(Xt, ldx, Wt, nullptr, R, ldr, Y, ldy, nullptr, M, N, K, 1,
                                                        group_m, ldw, 0.f);
 }
 
