@@ -97,6 +97,8 @@ __device__ __forceinline__ int slot_base(const int* cu, int b) { return cu[b] / 
 
 // Bound by the bytes, what it reads and the operands it writes, and by registers, of which three waves a SIMD leave 168: tile by tile in a
 // chunk with channel decays, and once more from memory where a prefix product left the range (all tiles held: one wave a SIMD, 69 us).
+// What the tiles are made of is loaded ahead of them all, 96 registers at key dims of 128, and under the delta rule with channel decays 17 of
+// them (22 where the decays are made) are in scratch memory meanwhile, 68 (92) bytes a lane.
 // MADE: the decays (and the delta rule's write strengths) come from src, in the vector unit's time.  A pass of its own that wrote them cost,
 // behind the kernels that write its inputs, 48 us for 12807 tokens of 16 heads of 64 (rank 16) and 40 for 4593 of 16 of 128, of
 // which the exponentials here take 29 (58 -> 87) and 25 (64 -> 89).
@@ -667,7 +669,8 @@ void go(const ChunkRecurrence& a, int from, int slots, int each) {
   const int64_t tokens = std::min<int64_t>(a.T, (int64_t)CT * slots), longest = std::min<int64_t>(a.longest, (int64_t)CT * (each ? each : slots));
   if (tokens * per < 180 * longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a, from, slots, each);
   else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a, from, slots, each);
-  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a, from, slots, each);  // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us)
+  // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us; with channel decays at key dims of 128 four registers are in scratch memory)
+  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a, from, slots, each);
 }
 
 template <int D, bool CHAN, bool DELTA>

@@ -494,7 +494,11 @@ class GemmPolicy:
       # Where even 128-row tiles leave half the CUs idle and the pass that follows sums the slabs, two parts, or three where they fit one
       # round, from K 2048 on; us in one, two and three parts with that pass, 2048 columns, fp32 result and scaled residual sum:
       # 1663 rows x 2048 39 / 33 / 36, x 4096 61 / 45 / 46, x 5632 75 / 53 / 53; 1200 x 4096 58 / 41 / 37; 2048 x 2048 41 / 36 /
-      # 42; bf16 residual and norm 1663 x 2048 33 / 30 / 33, x 4096 55 / 42 / 43, 1200 x 4096 53 / 39 / 35; x 1024 lost.
+      # 42; bf16 residual and norm 1663 x 2048 33 / 30 / 33, x 4096 55 / 42 / 43, 1200 x 4096 53 / 39 / 35; x 1024 lost.  Whole / so at
+      # other widths, fp32 result and scaled residual sum: 512 columns 1024 x 2048 31 / 21, 8192 x 2048 45 / 39 (bf16 residual and norm
+      # 36 / 35), 8192 x 8192 105 / 75; 1024 columns 2400 x 2048 38 / 29, 4096 x 4096 64 / 49; 3072 columns 1280 x 2048 42 / 37; 4096 columns
+      # 1024 x 2048 42 / 36, x 8192 103 / 83: nothing lost.  A row's sums so depend on how many rows its step has (three, two or one
+      # part), as they do below 1024 rows; all of them in fp32.
       # Not stored: the parts follow this M, a table entry would answer for its whole bucket.
       parts = 2 if -(-M // 256) * (N // 256) <= 128 and Kd >= (8192 if epi == "resid" else 24576) else 1
       tiles = -(-M // 128) * (N // 256)
