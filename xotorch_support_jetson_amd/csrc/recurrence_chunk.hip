@@ -662,11 +662,14 @@ void go(const ChunkRecurrence& a, int from, int slots, int each) {
   }
   // Steps whose longest sequence takes longer than the CUs' share of all chunks are bound by its chain: four waves of a quarter of the
   // key dims each, 16 channels a workgroup, three chunks ahead.  Others by the matrix unit: two halves and 32 channels, which
-  // repeat the products with M and N less.  The line by T (tokens) x workgroups of 32 channels a sequence / (256 x the longest), us
+  // repeat the products with M and N less.  The line by tokens x workgroups of 32 channels a sequence / (256 x the longest), us
   // quarters / halves, delta rule 16 heads of 128 x 128: 0.25 (one of 2000) 130 / 167, 0.5 77 / 93, 0.66 (5 of 364 .. 1728) 149 / 164,
-  // 0.75 (three of 1000) 111 / 98, 1.3 (8 of 961 .. 2433) 332 / 298.
+  // 0.75 (three of 1000) 111 / 98, 1.3 (8 of 961 .. 2433) 332 / 298.  A sequence's state, first loads and end cost its workgroups
+  // what 40 tokens do: one of 570 behind 64 single tokens 102 / 84 (0.4 by its tokens alone), behind 8 49 / 60, 16 heads of 64 x 128 with one
+  // decay each behind 233 190 / 99.
   const int64_t per = (int64_t)a.H * ((a.dv + 31) / 32);
-  const int64_t tokens = std::min<int64_t>(a.T, (int64_t)CT * slots), longest = std::min<int64_t>(a.longest, (int64_t)CT * (each ? each : slots));
+  const int64_t tokens = std::min<int64_t>(a.T, (int64_t)CT * slots) + 40 * (int64_t)a.B;
+  const int64_t longest = std::min<int64_t>(a.longest, (int64_t)CT * (each ? each : slots));
   if (tokens * per < 180 * longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a, from, slots, each);
   else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a, from, slots, each);
   // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us; with channel decays at key dims of 128 four registers are in scratch memory)
