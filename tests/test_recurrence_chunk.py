@@ -167,16 +167,17 @@ def test_decays_and_write_strengths_from_finished_products(gpu, d, G):
   assert torch.equal(one[0], two[0]) and torch.equal(one[1], two[1])
 
 
-ALL, SCALAR, DELTA, NONE = {"delta", "channel_delta", "channel", "scaled"}, {"delta", "scaled"}, {"delta"}, set()
+ALL, SCALAR, NONE = {"delta", "channel_delta", "channel", "scaled"}, {"delta", "scaled"}, set()
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rule", sorted(ALL))
 @pytest.mark.parametrize("B,dv,longest,chunks", [
-  (1, 64, 47, NONE), (1, 64, 48, SCALAR), (3, 64, 63, SCALAR), (3, 64, 64, ALL),  # few sequences
-  (32, 128, 31, NONE), (32, 128, 32, ALL), (31, 128, 32, NONE), (64, 128, -32, ALL),  # the CUs filled twice over, four times
-  (65, 128, -32, DELTA), (65, 128, -47, DELTA), (65, 128, -48, ALL), (128, 128, -48, ALL),  # (minus: behind single tokens)
-  (129, 128, -48, DELTA), (129, 128, -95, DELTA), (129, 128, -96, ALL), (129, 128, 35, ALL), (129, 128, 31, NONE)])
+  (1, 64, 55, NONE), (1, 64, 56, SCALAR), (3, 64, 63, SCALAR), (3, 64, 64, ALL), (4, 16, 64, ALL), (5, 32, 95, NONE), (5, 32, 96, ALL),  # prompts
+  (32, 128, 31, NONE), (32, 128, 32, ALL), (31, 128, 32, NONE), (129, 128, 35, ALL), (129, 128, 31, NONE),  # that fill the CUs twice over, or nearly
+  (16, 64, -55, NONE), (16, 64, -56, SCALAR), (17, 128, -95, NONE), (17, 128, -96, ALL), (32, 64, -64, ALL),  # (minus: behind single tokens)
+  (64, 128, -47, NONE), (64, 128, -48, ALL), (56, 64, -95, NONE), (128, 128, -63, NONE), (128, 128, -64, ALL), (129, 128, -95, NONE),
+  (136, 128, -95, NONE), (136, 128, -96, ALL)])
 def test_both_sides_of_the_chunk_rule(gpu, rule, B, dv, longest, chunks):
   """The lengths from which steps go by chunks (mixers.hip chunks_take), against the same step token by token (longest taken as 1): the
   same numbers to the bit where the rule leaves it at that, sums in another order where it does not."""

@@ -1300,25 +1300,31 @@ void launch_rec(int KR, dim3 grid, const float* q, int ldq, const float* k, int 
 
 bool rows16(const at::Tensor& t, int64_t ld) { return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 
-// Prompts go 16 tokens at a time (recurrence_chunk.hip) where that beats 0.2 us a token of the longest sequence: few sequences from 48
-// tokens on, 64 with channel decays, whose chunks write operands.  us token by token / in chunks, 16 heads of 128 x 128 delta rule, the
-// same with channel decays, 16 of 64 x 128 per-channel decays, 32 of 128 x 64 input scales: one of 48 tokens 12.4 / 12.7, 14.5 / 17.3,
-// 8.7 / 9.0, 11.0 / 10.5, of 64 15.9 / 13.7, 18.4 / 18.5, 10.7 / 10.8, 13.7 / 11.3.  Where the sequences' (value channel, key row) lanes
-// fill the CUs twice over, every sequence's tokens count token by token, and in chunks a single token costs what sixteen do.  Rate
-// of chunks by that of tokens, one to 16 prompts behind single tokens: 64 sequences (four fills) 1.3 .. 1.5, 1.3, 1.1, 1.1 .. 1.2 with
-// prompts of 32, 128 of 32 1.1, 1.0, 0.9, 0.9 and of 48 1.4, 1.2 .. 1.3, 1.1, 1.1, 256 of 64 1.2, 1.0, 1.0, 0.95, 512 of 32 1.0, 0.7, 0.75,
-// 0.8, of 95 1.2, 0.9, 0.9, 1.0: from 32 tokens on for the delta rule and up to four fills, from 48 up to eight, from 96 for more.
-// And from 32 where the mean sequence fills a chunk: 256 of 1 .. 32 1.5, 1.0, 1.1, 1.0, 128 of 32 among as many single ones 1.6, 1.1,
-// 1.2, 1.1, behind them 1.3, 0.9, 1.0, 0.9.
+// Prompts go 16 tokens at a time (recurrence_chunk.hip): from 96 tokens of the longest on whatever the other sequences are, and from fewer
+// where that beats 0.2 us a token.  The rate of chunks by that of tokens over 3900 random steps of all rules with a longest of 32 .. 95
+// (geometric mean, lowest and highest tenth):
+//   * prompts, 8 tokens and more in the mean: from 56 tokens on (64 with channel decays, whose chunks write operands) 1.28 (1.06 .. 1.57),
+//     below 0.95.  From 32 where their (value channel, key row) lanes fill the CUs twice over, so that token by token every token counts: 1.25
+//     (0.99 .. 1.67).  Not heads of fewer than 48 value channels, which leave a workgroup's waves idle: 1.05 (0.76 .. 1.30); of up to four
+//     sequences 1.20 (1.02 .. 1.44).
+//   * prompts behind or among single tokens, which cost a chunk each: the same for up to 16 sequences, 1.61 (1.04 .. 2.60); of more 0.86
+//     (0.69 .. 1.07), unless the sequences are a whole number of eights: token by token a prompt's workgroups then share one XCD.
+//     Up to 32 of those 1.41 (1.00 .. 2.53), from 48 tokens and two fills of the CUs up to 64 1.60 (1.21 .. 2.55), from 64 up to 128 1.33 (0.95 ..
+//     1.98), beyond 0.92.
 // (max_qlen 0: not known, the mean stands in.)  Key dims of two MFMA tile pairs or four, rows on 16 bytes, 32-bit offsets.
 bool chunks_take(const at::Tensor& q, int64_t ldq, const at::Tensor& k, int64_t ldk, int64_t ldv, const at::Tensor& state, int64_t T,
-                 int64_t B, int64_t H, bool delta, bool per_channel, int64_t max_qlen) {
-  const int64_t dv = state.size(2), d = state.size(3), longest = max_qlen > 0 ? max_qlen : T / B, lanes = B * H * dv;
+                 int64_t B, int64_t H, bool per_channel, int64_t max_qlen) {
+  const int64_t dv = state.size(2), d = state.size(3), longest = max_qlen > 0 ? max_qlen : T / B, few = per_channel ? 64 : 56;
   const int64_t widest = std::max(std::max(ldq, ldk), std::max(std::max(ldv, H * dv), H * d));
-  const int64_t from = lanes < 65536                                               ? (per_channel ? 64 : 48)
-                       : lanes <= 131072 || (delta && !per_channel) || T >= 16 * B ? 32
-                       : lanes <= 262144                                           ? 48
-                                                                                   : 96;
+  const bool full = B * H * dv >= 65536;
+  int64_t from = 96;
+  if (T >= 8 * B) {
+    if (dv >= 48 || B <= 4) from = full ? 32 : few;
+  } else if (B <= 16 || (B <= 32 && B % 8 == 0)) {
+    from = few;
+  } else if (B <= 128 && B % 8 == 0 && full) {
+    from = B <= 64 ? 48 : 64;
+  }
   return (d == 64 || d == 128) && longest >= from && T * widest * 4 < (int64_t(1) << 31) && rows16(q, ldq) && rows16(k, ldk) &&
          rows16(state, 0);
 }
@@ -1361,7 +1367,7 @@ void linear_recurrence(const at::Tensor& q, const at::Tensor& k, const at::Tenso
   const bool scalar = !beta.has_value() && (fixed || decay.numel() == T * H);
   const float* bp = beta.has_value() ? beta->data_ptr<float>() : nullptr;
   const bool per_channel = chan || (!delta && !inscale && !normch && !scalar);
-  if (chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, delta, per_channel, max_qlen) && (!per_channel || rows16(decay, 0))) {
+  if (chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, per_channel, max_qlen) && (!per_channel || rows16(decay, 0))) {
     auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, per_channel, delta, std::min(max_qlen, T))}, q.options());
     // (rows past a sequence's end are zeros because they are behind its last one: rows of k closer than a head is wide are not)
     const at::Tensor kr = ldk < d ? k.contiguous() : k;
@@ -1428,7 +1434,7 @@ bool linear_recurrence_made(const at::Tensor& q, const at::Tensor& k, const at::
     cols_ok(P, p_off, w.size(1), "decay projection");
     if (w.size(1) % 16 != 0 || !rows16(P, ldp) || p_off % 4 != 0) return false;
   }
-  if (!chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, delta, true, max_qlen) || !rows16(w, ldw) || !rows16(b, 0)) return false;
+  if (!chunks_take(q, ldq, k, ldk, ldv, state, T, B, H, true, max_qlen) || !rows16(w, ldw) || !rows16(b, 0)) return false;
   auto ws = at::empty({chunk_recurrence_ws(T, B, H, d, true, delta, std::min(max_qlen, T))}, q.options());
   chunk_recurrence({q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), nullptr, nullptr, ldq, ldk, ldv, 0, (float)q_scale,
                     state.data_ptr<float>(), state_slots.data_ptr<int>(), cu_q.data_ptr<int>(), (int)T, (int)B, (int)H, (int)G, (int)d,
