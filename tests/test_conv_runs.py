@@ -37,7 +37,7 @@ def test_units(head, lens):
 @pytest.mark.gpu
 @pytest.mark.parametrize("head", [1, 7, 64, 66, 126, 128, 130, 256])
 @pytest.mark.parametrize("off", [0, 1, 2])
-@pytest.mark.parametrize("taps,lens", [(4, [5, 1, 37]), (2, [1030, 0, 9]), (1, [33])])
+@pytest.mark.parametrize("taps,lens", [(4, [5, 1, 37]), (2, [1030, 0, 9]), (1, [33]), (6, [70, 3])])  # (runs or units as neighbours)
 def test_whole_rows_as_two_slabs(head, off, taps, lens):
   """Rows loaded without a branch (whole vectors, unsplit) and any others: the same numbers as the sum of the rows and of nothing."""
   C, T, B = 3 * head, sum(lens), len(lens)

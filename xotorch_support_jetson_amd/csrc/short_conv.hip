@@ -37,7 +37,7 @@ struct ConvArgs {
   int norm_n;
   float* conv_state;
   const int *state_slots, *cu;
-  int B, T, run;
+  int B, T, run, runs;  // runs: workgroups of a unit, where these are the neighbours (0: those of a run are)
   float eps;
   float* out;
 };
@@ -71,7 +71,8 @@ __device__ __forceinline__ void conv_body(const ConvArgs& A, int bx, int by) {
   constexpr int NT = SINGLE ? 1 : CTB;  // tokens whose inputs are in flight together
   const int64_t ss = A.ss;
   const float eps = A.eps;
-  const int unit = by * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // (filters of any length: in a scalar register 7200 tokens of 6400 channels and six taps took 1190 us, 1058 so)
+  const int unit = by * 4 + (TAPS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   if (unit >= NU) return;  // (wave-uniform; no workgroup barrier below)
   const int taps = TAPS ? TAPS : taps_rt;
   const int c0 = min(max(units[4 * unit], 0), C), n = min(min(max(units[4 * unit + 1], 0), 64 * VW), C - c0);
@@ -153,9 +154,10 @@ __device__ __forceinline__ void conv_body(const ConvArgs& A, int bx, int by) {
 
   // A run's tokens of whole vectors, unsplit, with no branch between their loads (lanes past the unit read its first channels): a
   // branch each, whose two ways load into the same registers, had the compiler wait for every load before the next.  Prompts,
-  // us before / so: 4593 tokens of 6144 channels 77 / 57, 12807 of 4096 125 / 85, 1663 of 4096 37 / 30.
+  // us before / so: 4593 tokens of 6144 channels 77 / 57, 12807 of 4096 125 / 85, 1663 of 4096 37 / 30.  (Filters of any length read
+  // their inputs again for every token: nothing to gain.)
   typedef float vecw __attribute__((ext_vector_type(VW)));
-  const bool flat = !SINGLE && S == 1 && (VW == 1 || vec);
+  const bool flat = TAPS && !SINGLE && S == 1 && (VW == 1 || vec);
   const float* rows = P + x_off + c0 + (in[0] ? l0 : 0);
 
   const int t0 = bx * run, t1 = min(T, t0 + run);
@@ -289,11 +291,13 @@ __device__ __forceinline__ void conv_body(const ConvArgs& A, int bx, int by) {
   }
 }
 
-// (units fastest: neighbours read and write whole rows together, 6144 channels of 4593 tokens 81 -> 77 us)
+// Neighbours are the units of a run, which read and write whole rows together (4096 channels of 12807 tokens 127 -> 110 us, 6144 of 4593
+// 81 -> 77), where rows are whole vectors; else (loads a channel each) the runs of a unit, us / so: 1536 channels of 9389 tokens, rows off
+// 8 bytes 63 / 58, 4096 of 8000 104 / 93, 6400 of 7200 with six taps 1223 / 1184.
 template <int TAPS, int VW, bool SINGLE>
 __global__ __launch_bounds__(256) void conv_prep_k(ConvArgs a) {
   const int groups = (a.NU + 3) / 4;
-  conv_body<TAPS, VW, SINGLE>(a, blockIdx.x / groups, blockIdx.x % groups);
+  conv_body<TAPS, VW, SINGLE>(a, a.runs ? blockIdx.x % a.runs : blockIdx.x / groups, a.runs ? blockIdx.x / a.runs : blockIdx.x % groups);
 }
 
 // the last taps - 1 inputs of every sequence -> its state slot
@@ -691,7 +695,10 @@ void conv_prep(const at::Tensor& P, int64_t x_off, const at::Tensor& conv_w, con
   if (a.T == 0 || a.B == 0 || a.NU == 0) return;
   const bool single = max_qlen == 1 && a.T == a.B;
   a.run = single ? 1 : a.T >= 1024 ? 32 : CTB;
-  const int64_t grid = ((int64_t)a.T + a.run - 1) / a.run * ((a.NU + 3) / 4);
+  const int64_t runs = ((int64_t)a.T + a.run - 1) / a.run, grid = runs * ((a.NU + 3) / 4);
+  const int vw = width <= 64 ? 1 : width <= 128 ? 2 : 4;
+  const bool whole = a.taps <= 4 && a.ldp % vw == 0 && a.ss % vw == 0 && a.x_off % vw == 0 && a.C % vw == 0;
+  a.runs = whole ? 0 : (int)runs;
   MCHECK(grid < (int64_t(1) << 31), "conv_prep: too many rows");
 #define CP_GO(TAPS, VW)                                                      \
   do {                                                                       \
