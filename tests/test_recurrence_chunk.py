@@ -315,3 +315,36 @@ def test_rows_that_repeat_or_overlap(gpu, rule, ld):
     K.linear_recurrence(*x, a, beta, 0.7, S, slots, cu, out, plain=scaled and not norm, max_qlen=max(lens))
     got.append((out, S))
   assert all(torch.equal(one, other) for one, other in zip(*got))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,H,lens,made", [(64, 16, (200, 31, 1), True), (64, 15, (200, 31, 1), False), (128, 32, (450, 31), True), (128, 32, (400, 31), False),
+                                          (64, 64, (31, 31, 31), False), (64, 16, (20,) * 32, False)])
+def test_low_rank_decays_by_the_chunks_or_apart(gpu, d, H, lens, made, monkeypatch):
+  """recurrence_norm with a low-rank decay: made by the chunks where these are many enough (16 chunk slots of 16 heads at key dims of 64,
+  32 of 32 at 128) and a prompt is long enough for them, else in a launch of its own; the same numbers."""
+  T, B, dv, rank, tau = sum(lens), len(lens), 32, 16, 16.0
+  g = torch.Generator(device=gpu).manual_seed(T)
+  rn = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+  P, a2, a2_b, qkv = rn(T, rank + 16), rn(H * d, rank) / rank ** 0.5, rn(H * d) + 3, rn(T, H * (2 * d + dv)) / d ** 0.5
+  q, k, v = qkv[:, :H * d], qkv[:, H * d:2 * H * d], qkv[:, 2 * H * d:]
+  state, w, gate, slots = rn(B, H, dv, d), rn(dv), rn(T, H * dv), torch.arange(B, dtype=torch.int32, device=gpu)
+  cu, calls, C = torch.tensor([0, *lens], device=gpu).cumsum(0).int(), [], require()
+
+  class Seen:
+    def __getattr__(self, name):
+      calls.append(name)
+      return getattr(C, name)
+  monkeypatch.setattr(K, "require", Seen)
+  decay, got = torch.empty(T, H * d, device=gpu), []
+  K.gla_prep(P, 8, a2, a2_b, tau, decay)
+  for kw in (dict(gla=(P, 8, a2, a2_b, tau)), {}):
+    calls.clear()
+    S, out = state.clone(), torch.empty(T, H * dv, device=gpu)
+    K.recurrence_norm(q, k, v, None if kw else decay, None, 0.7, S, slots, cu, w, gate, False, 1e-5, 1.0, out, max_qlen=max(lens), **kw)
+    got.append((out, S))
+    assert ("linear_recurrence_made" in calls) == (made and bool(kw)) and ("linear_recurrence" in calls) == (not made or not kw)
+  # (the same to the bit apart; made by the chunks the low-rank sums are in another order: some 1e-7 of |z| < 7, a sixteenth of it in a decay's
+  # logarithm, over the tokens that a decay remembers)
+  for one, other in zip(*got):
+    assert torch.equal(one, other) if not made else ((one - other).norm() / other.norm()) < 1e-5

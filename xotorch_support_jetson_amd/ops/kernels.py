@@ -677,7 +677,8 @@ def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu
     decay = torch.empty(q.shape[0], dt_bias.numel(), dtype=torch.float32, device=q.device)
     recurrence_gates(P, b_off, beta, 0, None, dt_bias, A_log, decay, 0, None, None, za=za)
     return decay, beta
-  if chan is not None and (max_qlen == 1 or not _gpu(q)):
+  apart = 0 < max_qlen < 32 or not _gpu(q)  # (never by chunks: 1.2 us less of the host's time than asking)
+  if chan is not None and apart:
     decay, beta = made_gates()
     chan = None
   if max_qlen == 1 and _gpu(q):
@@ -699,7 +700,11 @@ def recurrence_norm(q, k, v, decay, beta, q_scale: float, state, state_slots, cu
     if not done:
       decay, beta = made_gates()
   elif gla is not None:
-    if _gpu(q) and beta is None and gla[0].dim() == 2:
+    # A chunk's low-rank product is a chain of its own, tile by tile, which pays from a quarter of a (chunk, head) a SIMD on, at key
+    # dims of 128 from one; us a launch of its own / made by the chunks, rank 16: 4 heads of 64, one of 300 tokens 21.8 / 23.7, of 1000 49.1 /
+    # 48.2, 16 heads of 1000 53 / 50, 12 of 1000 206 / 187; 16 heads of 128, one of 300 29.6 / 34.3, of 1000 65.4 / 63.6, 12 of 1000 346 / 325.
+    waves = (T // 16 + state_slots.numel()) * H
+    if not apart and beta is None and gla[0].dim() == 2 and waves >= (256 if d == 64 else 1024):
       P, a1_off, a2, a2_b, tau = gla
       done = require().linear_recurrence_made(q, k, v, P, int(a1_off), a2, a2_b, float(tau), None, float(q_scale), state, state_slots, cu_q, o, int(max_qlen))
     if not done:
