@@ -47,8 +47,9 @@ constexpr int64_t WS_MOST = 128 << 20;          // workspace floats (Portions)
 // it replaces).  Steps whose records fit 512 MB (19.7 thousand tokens of 16 such heads) go at once, longer ones in portions, each with as
 // many chunks of every sequence, so that the sequences go on side by side.  Where the lengths are unlike enough to double the portions,
 // a portion would be fewer than 64 chunks of each or the longest is not known, portions are slots as they come.  The same heads, us at once
-// / in portions / as slots come: three of 9000 tokens 977 / 1008 / 1415, of 20000 2145 / 2222 / 3475, six of 8000 1556 / 1619 / 2054;
-// 64 of 512, which go as slots come, 904 / - / 950.
+// / in portions / as slots come: three of 9000 tokens 980 / 1024 / 1415, of 20000 2147 / 2254 / 3475, six of 8000 1556 / 1640 / 2054;
+// 64 of 512, which go as slots come, 907 / - / 952.  (16 to 32 us of the portions are the launches for what the longest, if it was
+// understated, would leave.)
 struct Portions {
   int count, slots, each;  // slots of the workspace; each: chunks of a sequence in a portion, or 0
 };
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(64, CHAN ? 3 : 2) void chunk_prep_k(const float* __
                                                    const float* __restrict__ decay, int dstride,
                                                    const float* __restrict__ beta, float q_scale,
                                                    const int* __restrict__ state_slots, const int* __restrict__ cu_q, int B,
-                                                   int H, int G, int heads, DecaySource src, int from, int each,
+                                                   int H, int G, int heads, DecaySource src, int from, int each, int done,
                                                    float* __restrict__ ws) {
   __shared__ float sA[CT][CT + 1];
   __shared__ __attribute__((aligned(16))) float sT[CHAN ? 2 : 1][CHAN ? CT : 1][CT + 4];  // a tile's way from dims to tokens
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(64, CHAN ? 3 : 2) void chunk_prep_k(const float* __
     c = from + s - slot_base(cu_q, lo);
   }
   const int t0 = cu_q[lo], n = cu_q[lo + 1] - t0;
-  if (state_slots[lo] < 0 || c * CT >= n) return;
+  if (state_slots[lo] < 0 || c < done || c * CT >= n) return;
   const int tok = c * CT + i;
   const bool valid = tok < n;
   const int64_t t = t0 + min(tok, n - 1);
@@ -331,13 +332,13 @@ __device__ __forceinline__ int scan_order(int turn, int B, int per) {
 
 // CG groups of 16 value channels a workgroup, KP waves each: wave (kp, cg) has key dims kp D / KP .. of group cg.  Of every sequence
 // the chunks whose records the workspace holds (Portions): `each` from its chunk `from` on, or those in `slots` slots from slot `from` of
-// the step; between portions the state is in its place in memory.
+// the step, but the first `done` of each; between portions the state is in its place in memory.
 template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
 __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ v, int ldv,
     const float* __restrict__ inscale, float q_scale, float* __restrict__ state, const int* __restrict__ state_slots,
-    const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, int from, int slots, int each, const float* __restrict__ ws,
-    float* __restrict__ out) {
+    const int* __restrict__ cu_q, int B, int H, int G, int dv, int dvin, int from, int slots, int each, int done,
+    const float* __restrict__ ws, float* __restrict__ out) {
   static_assert(KP == 2 || KP == 4, "the order of the sums is that of quarters of the key dims");
   constexpr int TILES = D / 16 / KP;              // 16-row state tiles of a wave
   constexpr int QW = 4 / KP, QT = TILES / QW;     // quarters of the key dims in a wave, tiles of each
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
   const int b = nth_longest(B, scan_order((int)blockIdx.z, B, H * (int)gridDim.y), [&](int j) { return cu_q[j + 1] - cu_q[j]; });
   const int slot = state_slots[b];
   const int base = slot_base(cu_q, b) - from;  // the sequence's first slot in the portion, or (negative) before it
-  const int c0 = each ? from : max(-base, 0), first = each ? b * each : base + c0;
+  const int c0 = each ? from : max(-base, done), first = each ? b * each : base + c0;
   const int t0 = cu_q[b] + CT * c0, n = min(cu_q[b + 1] - t0, CT * (each ? each : slots - first));
   if (slot < 0 || n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
@@ -636,23 +637,23 @@ __global__ __launch_bounds__(64 * KP * CG, WPE) void chunk_scan_k(
 }
 
 template <int D, bool CHAN, bool DELTA, int KP, int CG, int WPE, int RING>
-void scan(const ChunkRecurrence& a, int from, int slots, int each) {
+void scan(const ChunkRecurrence& a, int from, int slots, int each, int done) {
   const dim3 grid((unsigned)a.H, (unsigned)((a.dv + 16 * CG - 1) / (16 * CG)), (unsigned)a.B);
   chunk_scan_k<D, CHAN, DELTA, KP, CG, WPE, RING><<<grid, 64 * KP * CG, 0, stream()>>>(
       a.q, a.ldq, a.k, a.ldk, a.v, a.ldv, DELTA ? nullptr : a.beta, a.q_scale, a.state, a.state_slots, a.cu_q, a.B, a.H, a.G, a.dv,
-      a.dvin, from, slots, each, a.ws, a.out);
+      a.dvin, from, slots, each, done, a.ws, a.out);
 }
 
 // a portion
 template <int D, bool CHAN, bool DELTA>
-void go(const ChunkRecurrence& a, int from, int slots, int each) {
+void go(const ChunkRecurrence& a, int from, int slots, int each, int done) {
   // plain write, a decay per head: the heads of a q / k head share its products where that leaves enough waves (32 heads on 8, with the
   // scan: 5 of 364 .. 1728 tokens 110 -> 100 us, 8 of 961 .. 2433 247 -> 223; three of 1000 not; two heads under the delta rule gave nothing)
   const int heads = !CHAN && !DELTA && (int64_t)slots * a.G >= 2048 ? a.H / a.G : 1;
   const unsigned pg = (unsigned)slots * (unsigned)(a.H / heads);
   auto prep = [&](auto kern) {
     kern<<<pg, 64, 0, stream()>>>(a.q, a.ldq, a.k, a.ldk, a.decay, a.dstride, a.beta, a.q_scale, a.state_slots, a.cu_q, a.B, a.H, a.G,
-                                  heads, a.src, from, each, a.ws);
+                                  heads, a.src, from, each, done, a.ws);
   };
   if constexpr (CHAN) {
     if (a.src.P != nullptr) prep(chunk_prep_k<D, CHAN, DELTA, true>);
@@ -670,23 +671,29 @@ void go(const ChunkRecurrence& a, int from, int slots, int each) {
   const int64_t per = (int64_t)a.H * ((a.dv + 31) / 32);
   const int64_t tokens = std::min<int64_t>(a.T, (int64_t)CT * slots) + 40 * (int64_t)a.B;
   const int64_t longest = std::min<int64_t>(a.longest, (int64_t)CT * (each ? each : slots));
-  if (tokens * per < 180 * longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a, from, slots, each);
-  else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a, from, slots, each);
+  if (tokens * per < 180 * longest) scan<D, CHAN, DELTA, 4, 1, 2, 3>(a, from, slots, each, done);
+  else if (a.B * per <= 512 || !DELTA) scan<D, CHAN, DELTA, 2, 2, 2, 2>(a, from, slots, each, done);
   // (four waves a SIMD: 12 of 130 tokens 51.7 -> 49.1 us; with channel decays at key dims of 128 four registers are in scratch memory)
-  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a, from, slots, each);
+  else if constexpr (DELTA) scan<D, CHAN, DELTA, 2, 2, 4, 1>(a, from, slots, each, done);
 }
 
 template <int D, bool CHAN, bool DELTA>
 void go(const ChunkRecurrence& a) {
   const Portions p = portions(a.T, a.B, a.H, rec_floats(D, CHAN, DELTA), a.known ? a.longest : 0);
-  for (int turn = 0; turn < p.count; ++turn) go<D, CHAN, DELTA>(a, turn * (p.each ? p.each : p.slots), p.slots, p.each);
+  for (int turn = 0; turn < p.count; ++turn) go<D, CHAN, DELTA>(a, turn * (p.each ? p.each : p.slots), p.slots, p.each, 0);
+  const int done = p.count * p.each;  // chunks of every sequence
+  if (done == 0 || (int64_t)CT * done >= a.T) return;
+  // what is left of sequences longer than the longest was said to be, as slots come (nothing: workgroups that end at once)
+  const Portions rest = portions(a.T, a.B, a.H, rec_floats(D, CHAN, DELTA), 0);
+  for (int turn = 0; turn < rest.count; ++turn) go<D, CHAN, DELTA>(a, turn * rest.slots, rest.slots, 0, done);
 }
 
 }  // namespace
 
 int64_t chunk_recurrence_ws(int64_t T, int64_t B, int64_t H, int64_t d, bool chan, bool delta, int64_t max_qlen) {
   const int rec = rec_floats((int)d, chan, delta);
-  return portions(T, B, H, rec, max_qlen).slots * H * rec;
+  const Portions p = portions(T, B, H, rec, max_qlen), rest = p.each ? portions(T, B, H, rec, 0) : p;
+  return std::max(p.slots, rest.slots) * H * rec;
 }
 
 void chunk_recurrence(const ChunkRecurrence& a) {

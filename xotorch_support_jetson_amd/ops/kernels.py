@@ -652,7 +652,7 @@ def linear_recurrence(q, k, v, decay, beta, q_scale: float, state, state_slots, 
   q is scaled by q_scale.
   A state with one value channel more than v has (decay [T, H], beta [T, H] an input scale): S = g S + k (beta [v | 1])^T,
   the last channel being a normaliser n = g n + beta k; out [T, H (dv + 1)] then ends each head with n . q.
-  max_qlen: tokens of the step's longest sequence, no fewer (0: not known); long ones run in chunks of 16 tokens on the GPU."""
+  max_qlen: tokens of the step's longest sequence (0: not known); long ones run in chunks of 16 tokens on the GPU."""
   if _gpu(q):
     require().linear_recurrence(q, k, v, decay, beta, float(q_scale), state, state_slots, cu_q, out, bool(plain), int(max_qlen))
   else:
